@@ -175,6 +175,19 @@ int lact_layer_post_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H,
                              float eps, const void* o, const float* norm_weight, const void* gate_raw,
                              const void* dy, void* d_o, void* dgate_raw, float* dw_part, void* stream);
 
+/* Causal attention inside a sliding window (query i sees keys i - window + 1 .. i; window >= L: plain causal), bf16, head
+ * size D = 64 or 128, softmax scale 1/sqrt(D): flash_attn_func(causal=True, window_size=(window-1, 0)) of
+ * causal_lact_with_sliding_window_attn.py:371-375.  q, k, v, dout: [B, L, H, D] with token stride *_ld and batch stride *_bs
+ * (elements, multiples of 8; heads contiguous inside a token).  out, dq, dk, dv: [B, L, H, D] contiguous; lse and delta:
+ * [B, H, L] fp32, lse kept from the forward for the backward, delta a work buffer of the backward. */
+int lact_window_attention_forward(int32_t B, int32_t L, int32_t H, int32_t D, int32_t window, const void* q, int32_t q_ld,
+                                  int64_t q_bs, const void* k, int32_t k_ld, int64_t k_bs, const void* v, int32_t v_ld,
+                                  int64_t v_bs, void* out, float* lse, void* stream);
+int lact_window_attention_backward(int32_t B, int32_t L, int32_t H, int32_t D, int32_t window, const void* q, int32_t q_ld,
+                                   int64_t q_bs, const void* k, int32_t k_ld, int64_t k_bs, const void* v, int32_t v_ld,
+                                   int64_t v_bs, const void* out, const float* lse, const void* dout, int32_t do_ld,
+                                   int64_t do_bs, float* delta, void* dq, void* dk, void* dv, void* stream);
+
 /* Execution options (process-wide; no counterpart in the reference, where PyTorch enqueues the whole layer on one
  * stream as separate kernels).  The switches are on by default and change no result bit.
  *   LACT_OPT_STREAM_OVERLAP: the apply steps of a program do not depend on the update chain that runs beside

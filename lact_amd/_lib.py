@@ -40,7 +40,8 @@ EXPORTS = ("lact_last_error", "lact_version", "lact_query_sizes", "lact_forward"
            "lact_newton_schulz_static", "lact_newton_schulz_backward_workspace_bytes", "lact_newton_schulz_backward",
            "lact_check_async_error", "lact_mfma_calibration", "lact_set_option", "lact_profile_enable",
            "lact_profile_report", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward",
-           "lact_layer_lr_backward", "lact_layer_post_forward", "lact_layer_post_dw_rows", "lact_layer_post_backward")
+           "lact_layer_lr_backward", "lact_layer_post_forward", "lact_layer_post_dw_rows", "lact_layer_post_backward",
+           "lact_window_attention_forward", "lact_window_attention_backward")
 
 _lib = None
 
@@ -91,7 +92,9 @@ def lib():
     L.lact_layer_post_forward.argtypes = [i32] * 6 + [f32] + [vp] * 5
     L.lact_layer_post_dw_rows.argtypes = [i32] * 3
     L.lact_layer_post_backward.argtypes = [i32] * 6 + [f32] + [vp] * 8
-    for fn in ("lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward", "lact_layer_lr_backward",
+    L.lact_window_attention_forward.argtypes = [i32] * 5 + [vp, i32, c_int64] * 3 + [vp] * 3
+    L.lact_window_attention_backward.argtypes = [i32] * 5 + [vp, i32, c_int64] * 3 + [vp, vp] + [vp, i32, c_int64] + [vp] * 5
+    for fn in ("lact_window_attention_forward", "lact_window_attention_backward", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward", "lact_layer_lr_backward",
                "lact_layer_post_forward", "lact_layer_post_dw_rows", "lact_layer_post_backward"):
         getattr(L, fn).restype = c_int32
     L.lact_profile_enable.argtypes = [c_int32]

@@ -20,6 +20,7 @@
 #include "gemm_kernels.h"
 #include "state_kernels.h"
 #include "layer_kernels.h"
+#include "window_attention.h"
 
 using namespace lact;
 
@@ -1948,6 +1949,81 @@ int lact_layer_pre_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, 
   if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_pre_bwd", "layer_pre_bwd", 0.0, (k_layer_pre<uint16_t, true>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
   else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_pre_bwd", "layer_pre_bwd", 0.0, (k_layer_pre<float, true>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
   else return fail("act_dtype must be LACT_BF16 or LACT_F32");
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+// ---- sliding-window attention of the causal layer
+}  // extern "C"
+namespace {
+int window_attn_params(int B, int L, int H, int D, int window, WindowAttnParams* p) {
+  memset(p, 0, sizeof(*p));
+  if (B <= 0 || L <= 0 || H <= 0 || window <= 0) return fail("B, L, H and window must be positive");
+  if (D != 64 && D != 128) return fail("window attention: head size must be 64 or 128");
+  if ((long long)B * H > (1 << 20) || (long long)L * H * D > (1LL << 31)) return fail("window attention: sequence or batch too large");
+  p->B = B; p->L = L; p->H = H; p->window = std::min(window, L);
+  p->scale = 1.0f / sqrtf((float)D);
+  return 0;
+}
+int attn_rows(const void* ptr, int ld, long long bs, int H, int D, const uint16_t** out_ptr, int* out_ld, long long* out_bs) {
+  if (!ptr) return fail("null pointer: window attention tensors");
+  if (ld % 8 || bs % 8 || ld < H * D || (reinterpret_cast<uintptr_t>(ptr) & 15)) return fail("window attention: rows must be 16-byte aligned and hold H * D elements");
+  if (ld > (1 << 24)) return fail("window attention: row stride too large");
+  *out_ptr = static_cast<const uint16_t*>(ptr); *out_ld = ld; *out_bs = bs;
+  return 0;
+}
+// Waves per block: 8 (256 rows, two waves per SIMD) once that gives every compute unit a block, else 4.
+template <int D, int NW>
+void launch_window_attn(int which, WindowAttnParams p, hipStream_t s) {
+  p.map = make_tile_map(ceil_div(p.L, 32 * NW), 1, p.B * p.H);
+  const dim3 grid(p.map.grid()), block(64 * NW);
+  constexpr int SM = attn_lds_bytes<D, NW>(false), SMS = attn_lds_bytes<D, NW>(true);
+  LACT_BIG_LDS((k_window_attn_fwd<D, NW>), SM);
+  LACT_BIG_LDS((k_window_attn_dq<D, NW>), SM);
+  LACT_BIG_LDS((k_window_attn_dkv<D, NW>), SMS);
+  const double w = p.window, pairs = (double)p.L * w - w * (w - 1) / 2, f = 2.0 * pairs * D * p.B * p.H;
+  if (which == 0) LACT_LAUNCH_SMEM("k_window_attn_fwd", "window_attn", 2 * f, (k_window_attn_fwd<D, NW>), grid, block, SM, s, p);
+  if (which == 1) {
+    LACT_LAUNCH_SMEM("k_window_attn_dq", "window_attn_bwd", 3 * f, (k_window_attn_dq<D, NW>), grid, block, SM, s, p);
+    LACT_LAUNCH_SMEM("k_window_attn_dkv", "window_attn_bwd", 4 * f, (k_window_attn_dkv<D, NW>), grid, block, SMS, s, p);
+  }
+}
+void launch_window_attn(int which, int D, const WindowAttnParams& p, hipStream_t s) {
+  const bool wide = (long long)ceil_div(p.L, 256) * p.B * p.H >= 256;
+  if (D == 128) wide ? launch_window_attn<128, 8>(which, p, s) : launch_window_attn<128, 4>(which, p, s);
+  else wide ? launch_window_attn<64, 8>(which, p, s) : launch_window_attn<64, 4>(which, p, s);
+}
+}  // namespace
+extern "C" {
+
+int lact_window_attention_forward(int32_t B, int32_t L, int32_t H, int32_t D, int32_t window, const void* q, int32_t q_ld, int64_t q_bs,
+                                  const void* k, int32_t k_ld, int64_t k_bs, const void* v, int32_t v_ld, int64_t v_bs, void* out,
+                                  float* lse, void* stream) {
+  WindowAttnParams p;
+  if (window_attn_params(B, L, H, D, window, &p)) return -1;
+  if (attn_rows(q, q_ld, q_bs, H, D, &p.q, &p.ldq, &p.bsq) || attn_rows(k, k_ld, k_bs, H, D, &p.k, &p.ldk, &p.bsk) ||
+      attn_rows(v, v_ld, v_bs, H, D, &p.v, &p.ldv, &p.bsv))
+    return -1;
+  if (check_ptrs({out, lse}, "window attention outputs")) return -1;
+  p.out = static_cast<uint16_t*>(out); p.lse = lse;
+  launch_window_attn(0, D, p, reinterpret_cast<hipStream_t>(stream));
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+int lact_window_attention_backward(int32_t B, int32_t L, int32_t H, int32_t D, int32_t window, const void* q, int32_t q_ld, int64_t q_bs,
+                                   const void* k, int32_t k_ld, int64_t k_bs, const void* v, int32_t v_ld, int64_t v_bs, const void* out,
+                                   const float* lse, const void* dout, int32_t do_ld, int64_t do_bs, float* delta, void* dq, void* dk,
+                                   void* dv, void* stream) {
+  WindowAttnParams p;
+  if (window_attn_params(B, L, H, D, window, &p)) return -1;
+  if (attn_rows(q, q_ld, q_bs, H, D, &p.q, &p.ldq, &p.bsq) || attn_rows(k, k_ld, k_bs, H, D, &p.k, &p.ldk, &p.bsk) ||
+      attn_rows(v, v_ld, v_bs, H, D, &p.v, &p.ldv, &p.bsv) || attn_rows(dout, do_ld, do_bs, H, D, &p.dout, &p.lddo, &p.bsdo))
+    return -1;
+  if (check_ptrs({out, lse, delta, dq, dk, dv}, "window attention backward tensors")) return -1;
+  p.o = static_cast<const uint16_t*>(out); p.lse = const_cast<float*>(lse); p.delta = delta;
+  p.dq = static_cast<uint16_t*>(dq); p.dk = static_cast<uint16_t*>(dk); p.dv = static_cast<uint16_t*>(dv);
+  launch_window_attn(1, D, p, reinterpret_cast<hipStream_t>(stream));
   LACT_CHECK_LAUNCH();
   return 0;
 }

@@ -193,11 +193,52 @@ class BidirectionalLaCTSwiGLU(nn.Module):
         return self.o_proj(_PostFn.apply(o, weight, None, B, self.num_heads, use_norm, eps))
 
 
+def _head_rows(t: torch.Tensor) -> torch.Tensor:
+    """[b, l, h, d] whose heads lie next to each other inside a token, 16-byte aligned."""
+    ok = (t.stride(3) == 1 and t.stride(2) == t.shape[3] and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
+          and t.stride(1) >= t.shape[2] * t.shape[3] and t.data_ptr() % 16 == 0)
+    return t if ok else t.contiguous()
+
+
+class _WindowAttentionFn(torch.autograd.Function):
+    """bf16 sliding-window attention on [b, l, h, d], d = 64 or 128 (csrc/window_attention.h)."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, window):
+        q, k, v = _head_rows(q), _head_rows(k), _head_rows(v)
+        B, L, H, D = q.shape
+        out = torch.empty((B, L, H, D), dtype=q.dtype, device=q.device)
+        lse = torch.empty((B, H, L), dtype=torch.float32, device=q.device)
+        with torch.cuda.device(q.device):
+            _lib.check(_lib.lib().lact_window_attention_forward(
+                B, L, H, D, window, _ptr(q), q.stride(1), q.stride(0), _ptr(k), k.stride(1), k.stride(0), _ptr(v), v.stride(1), v.stride(0),
+                _ptr(out), _ptr(lse), _stream(q)))
+        ctx.save_for_backward(q, k, v, out, lse)
+        ctx.window = window
+        return out
+
+    @staticmethod
+    def backward(ctx, g):
+        q, k, v, out, lse = ctx.saved_tensors
+        B, L, H, D = q.shape
+        g = _head_rows(g.to(q.dtype))
+        dq, dk, dv = (torch.empty((B, L, H, D), dtype=q.dtype, device=q.device) for _ in range(3))
+        delta = torch.empty_like(lse)
+        with torch.cuda.device(q.device):
+            _lib.check(_lib.lib().lact_window_attention_backward(
+                B, L, H, D, ctx.window, _ptr(q), q.stride(1), q.stride(0), _ptr(k), k.stride(1), k.stride(0), _ptr(v), v.stride(1), v.stride(0),
+                _ptr(out), _ptr(lse), _ptr(g), g.stride(1), g.stride(0), _ptr(delta), _ptr(dq), _ptr(dk), _ptr(dv), _stream(q)))
+        return dq, dk, dv, None
+
+
 def sliding_window_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window: Optional[int]) -> torch.Tensor:
     """q, k, v: [b, l, h, d].  Causal attention where query i sees keys i-(window-1) .. i -- what the reference asks
     of flash_attn_func(causal=True, window_size=(window-1, 0)) (causal_lact_with_sliding_window_attn.py:371-375).
-    Query blocks of `window` rows attend to their own and the previous block under a band mask."""
+    bf16 with heads of 64 or 128 runs in this library's kernels; other types and head sizes through torch's attention, where
+    query blocks of `window` rows attend to their own and the previous block under a band mask."""
     b, l, h, d = q.shape
+    if q.is_cuda and d in (64, 128) and b * l > 0 and q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype == torch.bfloat16:
+        return _WindowAttentionFn.apply(q, k, v, l if window is None else min(window, l))
     q, k, v = (t.transpose(1, 2) for t in (q, k, v))              # [b, h, l, d]
     if window is None or window >= l:
         return F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2)

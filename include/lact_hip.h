@@ -153,6 +153,18 @@ int lact_layer_pre_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, i
 int lact_layer_pre_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm,
                             const void* qkv, const void* dq, const void* dk, const void* dv, void* dqkv,
                             void* stream);
+/* The same with what the causal layer's attention reads of the projection, [B, L, H*hd] each: aq = q * qk_scale[:, 0] +
+ *      qk_offset[:, 0], ak likewise with column 1 (parameters fp32 [H*hd, 2]; round_product: they have the activations' type
+ *      in the layer, so the product is rounded to it), av = v (causal_lact_with_sliding_window_attn.py:314-316,362-366).
+ *      The backward adds both branches' gradients into dqkv; part: lact_layer_pre_attn_part_rows(B, L, H) * 4 * H*hd floats. */
+int lact_layer_pre_attn_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm,
+                                int32_t round_product, const void* qkv, const float* qk_scale, const float* qk_offset, void* q,
+                                void* k, void* v, void* aq, void* ak, void* av, void* stream);
+int32_t lact_layer_pre_attn_part_rows(int32_t B, int32_t L, int32_t H);
+int lact_layer_pre_attn_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm,
+                                 const void* qkv, const float* qk_scale, const void* dq, const void* dk, const void* dv,
+                                 const void* daq, const void* dak, const void* dav, void* dqkv, float* part, float* dqk_scale,
+                                 float* dqk_offset, void* stream);
 /* lr: lr_raw fp32 (output of lr_proj) -> lr0, lr1, lr2 [(B H), L] = softplus(raw + base_lr_inv); lr_raw is
  *     [B, L, H, 3] ('b l (h lrs d)') when rates_major == 0 and [B, L, 3, H] ('b l (lrs h d)', lact_ttt.py:213-216) else;
  *     momentum_raw [B, L, H] fp32 (nullable; output of the linear map of momentum_proj) -> sigmoid, [(B H), L]
@@ -164,12 +176,16 @@ int lact_layer_lr_backward(int32_t B, int32_t L, int32_t H, int32_t rates_major,
                            const float* momentum_raw, const float* dmomentum, float* dmomentum_raw, void* stream);
 /* post: o [(B H), L, hd] (output of the operation) -> y [B, L, H*hd]: RMSNorm over the head dim with weight
  *      norm_weight [hd] fp32 (nullable = ones) when use_norm, times silu(gate_raw [B, L, H]) when gate_raw is
- *      given, head layout (bidirectional_lact_layer.py:268-270; causal_lact_with_sliding_window_attn.py:351-357).
+ *      given, head layout, and in the _add form plus add
+ *      [B, L, H*hd] (nullable; its gradient is dy) (bidirectional_lact_layer.py:268-270; causal_lact_with_sliding_window_attn.py:351-357).
  *      The backward writes lact_layer_post_dw_rows(B, L, H) partial rows of the weight gradient into
  *      dw_part [rows][hd] fp32 (the caller sums them), d_o and dgate_raw. */
 int lact_layer_post_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm,
                             float eps, const void* o, const float* norm_weight, const void* gate_raw, void* y,
                             void* stream);
+int lact_layer_post_add_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm,
+                                float eps, const void* o, const float* norm_weight, const void* gate_raw, const void* add,
+                                void* y, void* stream);
 int32_t lact_layer_post_dw_rows(int32_t B, int32_t L, int32_t H);
 int lact_layer_post_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm,
                              float eps, const void* o, const float* norm_weight, const void* gate_raw,

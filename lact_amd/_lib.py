@@ -41,7 +41,8 @@ EXPORTS = ("lact_last_error", "lact_version", "lact_query_sizes", "lact_forward"
            "lact_check_async_error", "lact_mfma_calibration", "lact_set_option", "lact_profile_enable",
            "lact_profile_report", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward",
            "lact_layer_lr_backward", "lact_layer_post_forward", "lact_layer_post_dw_rows", "lact_layer_post_backward",
-           "lact_window_attention_forward", "lact_window_attention_backward")
+           "lact_window_attention_forward", "lact_window_attention_backward", "lact_layer_pre_attn_forward",
+           "lact_layer_pre_attn_part_rows", "lact_layer_pre_attn_backward", "lact_layer_post_add_forward")
 
 _lib = None
 
@@ -90,11 +91,15 @@ def lib():
     L.lact_layer_lr_forward.argtypes = [i32] * 4 + [f32] + [vp] * 7
     L.lact_layer_lr_backward.argtypes = [i32] * 4 + [f32] + [vp] * 9
     L.lact_layer_post_forward.argtypes = [i32] * 6 + [f32] + [vp] * 5
+    L.lact_layer_post_add_forward.argtypes = [i32] * 6 + [f32] + [vp] * 6
     L.lact_layer_post_dw_rows.argtypes = [i32] * 3
     L.lact_layer_post_backward.argtypes = [i32] * 6 + [f32] + [vp] * 8
     L.lact_window_attention_forward.argtypes = [i32] * 5 + [vp, i32, c_int64] * 3 + [vp] * 3
     L.lact_window_attention_backward.argtypes = [i32] * 5 + [vp, i32, c_int64] * 3 + [vp, vp] + [vp, i32, c_int64] + [vp] * 5
-    for fn in ("lact_window_attention_forward", "lact_window_attention_backward", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward", "lact_layer_lr_backward",
+    L.lact_layer_pre_attn_forward.argtypes = [i32] * 7 + [vp] * 10
+    L.lact_layer_pre_attn_part_rows.argtypes = [i32] * 3
+    L.lact_layer_pre_attn_backward.argtypes = [i32] * 6 + [vp] * 13
+    for fn in ("lact_layer_post_add_forward", "lact_layer_pre_attn_forward", "lact_layer_pre_attn_part_rows", "lact_layer_pre_attn_backward", "lact_window_attention_forward", "lact_window_attention_backward", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward", "lact_layer_lr_backward",
                "lact_layer_post_forward", "lact_layer_post_dw_rows", "lact_layer_post_backward"):
         getattr(L, fn).restype = c_int32
     L.lact_profile_enable.argtypes = [c_int32]

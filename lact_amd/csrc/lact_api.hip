@@ -1923,6 +1923,39 @@ unsigned layer_row_blocks(const LayerGeom& g) { return (unsigned)(((long long)g.
 unsigned layer_post_bwd_blocks(const LayerGeom& g) { return std::min(layer_row_blocks(g), 2048u); }
 }  // namespace
 
+}  // extern "C"
+namespace {
+template <typename T, bool BWD, bool ATT>
+void launch_layer_pre_t(const char* name, const char* site, const LayerPreParams& p, int blocks_per_head, hipStream_t s) {
+  const dim3 grid((unsigned)(blocks_per_head * p.g.H)), block(256);
+  if (p.g.hd <= 256) LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, 1>), grid, block, s, p);
+  else if (p.g.hd <= 512) LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, 2>), grid, block, s, p);
+  else LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, LAYER_VEC_MAX>), grid, block, s, p);
+}
+template <bool BWD>
+int launch_layer_pre(int act_dtype, LayerPreParams& p, int blocks_per_head, hipStream_t s) {
+  const bool att = p.att[0] || p.datt[0];
+  p.tokens_per_pass = 4 * blocks_per_head;
+  const char* name = BWD ? "k_layer_pre_bwd" : "k_layer_pre";
+  const char* site = BWD ? "layer_pre_bwd" : "layer_pre";
+  if (act_dtype == LACT_BF16) {
+    if (att) launch_layer_pre_t<uint16_t, BWD, true>(name, site, p, blocks_per_head, s);
+    else launch_layer_pre_t<uint16_t, BWD, false>(name, site, p, blocks_per_head, s);
+  } else if (act_dtype == LACT_F32) {
+    if (att) launch_layer_pre_t<float, BWD, true>(name, site, p, blocks_per_head, s);
+    else launch_layer_pre_t<float, BWD, false>(name, site, p, blocks_per_head, s);
+  } else {
+    return fail("act_dtype must be LACT_BF16 or LACT_F32");
+  }
+  return 0;
+}
+int layer_token_blocks(const LayerGeom& g) { return (int)(((long long)g.B * g.L + 3) / 4); }   // one token per wave
+// blocks per head of the backward with parameter gradients: enough waves to hide the memory latency (16 per compute
+// unit), few enough that the partial sums stay small beside the activations
+int layer_pre_attn_blocks(const LayerGeom& g) { return std::max(1, std::min(layer_token_blocks(g), 1024 / g.H)); }
+}  // namespace
+extern "C" {
+
 int lact_layer_pre_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm, const void* qkv,
                            void* q, void* k, void* v, void* stream) {
   LayerPreParams p;
@@ -1930,10 +1963,7 @@ int lact_layer_pre_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, i
   if (layer_geom(B, L, H, hd, &p.g)) return -1;
   if (check_ptrs({qkv, q, k, v}, "layer pre tensors")) return -1;
   p.l2norm = l2norm; p.qkv = qkv; p.out[0] = q; p.out[1] = k; p.out[2] = v;
-  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_pre", "layer_pre", 0.0, (k_layer_pre<uint16_t, false>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
-  else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_pre", "layer_pre", 0.0, (k_layer_pre<float, false>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
-  else return fail("act_dtype must be LACT_BF16 or LACT_F32");
+  if (launch_layer_pre<false>(act_dtype, p, layer_token_blocks(p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
   LACT_CHECK_LAUNCH();
   return 0;
 }
@@ -1945,10 +1975,44 @@ int lact_layer_pre_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, 
   if (layer_geom(B, L, H, hd, &p.g)) return -1;
   if (check_ptrs({qkv, dq, dk, dv, dqkv}, "layer pre backward tensors")) return -1;
   p.l2norm = l2norm; p.qkv = qkv; p.dout[0] = dq; p.dout[1] = dk; p.dout[2] = dv; p.dqkv = dqkv;
+  if (launch_layer_pre<true>(act_dtype, p, layer_token_blocks(p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+int lact_layer_pre_attn_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm, int32_t round_product,
+                                const void* qkv, const float* qk_scale, const float* qk_offset, void* q, void* k, void* v, void* aq,
+                                void* ak, void* av, void* stream) {
+  LayerPreParams p;
+  memset(&p, 0, sizeof(p));
+  if (layer_geom(B, L, H, hd, &p.g)) return -1;
+  if (check_ptrs({qkv, qk_scale, qk_offset, q, k, v, aq, ak, av}, "layer pre tensors")) return -1;
+  p.l2norm = l2norm; p.qkv = qkv; p.out[0] = q; p.out[1] = k; p.out[2] = v;
+  p.att[0] = aq; p.att[1] = ak; p.att[2] = av; p.qk_scale = qk_scale; p.qk_offset = qk_offset; p.round_product = round_product;
+  if (launch_layer_pre<false>(act_dtype, p, layer_token_blocks(p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+int32_t lact_layer_pre_attn_part_rows(int32_t B, int32_t L, int32_t H) {
+  LayerGeom g;
+  if (layer_geom(B, L, H, 4, &g)) return -1;
+  return layer_pre_attn_blocks(g);
+}
+
+int lact_layer_pre_attn_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm, const void* qkv,
+                                 const float* qk_scale, const void* dq, const void* dk, const void* dv, const void* daq, const void* dak,
+                                 const void* dav, void* dqkv, float* part, float* dqk_scale, float* dqk_offset, void* stream) {
+  LayerPreParams p;
+  memset(&p, 0, sizeof(p));
+  if (layer_geom(B, L, H, hd, &p.g)) return -1;
+  if (check_ptrs({qkv, qk_scale, dq, dk, dv, daq, dak, dav, dqkv, part, dqk_scale, dqk_offset}, "layer pre backward tensors")) return -1;
+  p.l2norm = l2norm; p.qkv = qkv; p.dout[0] = dq; p.dout[1] = dk; p.dout[2] = dv; p.dqkv = dqkv;
+  p.datt[0] = daq; p.datt[1] = dak; p.datt[2] = dav; p.qk_scale = qk_scale; p.part = part;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_pre_bwd", "layer_pre_bwd", 0.0, (k_layer_pre<uint16_t, true>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
-  else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_pre_bwd", "layer_pre_bwd", 0.0, (k_layer_pre<float, true>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
-  else return fail("act_dtype must be LACT_BF16 or LACT_F32");
+  const int rows = layer_pre_attn_blocks(p.g), dim = H * hd;
+  if (launch_layer_pre<true>(act_dtype, p, rows, s)) return -1;
+  LACT_LAUNCH("k_layer_qk_reduce", "layer_pre_bwd", 0.0, k_layer_qk_reduce, dim3((dim + 63) / 64, 4), dim3(256), s, part, rows, dim, dqk_scale, dqk_offset);
   LACT_CHECK_LAUNCH();
   return 0;
 }
@@ -2063,19 +2127,24 @@ int lact_layer_lr_backward(int32_t B, int32_t L, int32_t H, int32_t rates_major,
   return 0;
 }
 
-int lact_layer_post_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm, float eps,
-                            const void* o, const float* norm_weight, const void* gate_raw, void* y, void* stream) {
+int lact_layer_post_add_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm, float eps,
+                            const void* o, const float* norm_weight, const void* gate_raw, const void* add, void* y, void* stream) {
   LayerPostParams p;
   memset(&p, 0, sizeof(p));
   if (layer_geom(B, L, H, hd, &p.g)) return -1;
   if (check_ptrs({o, y}, "layer post tensors")) return -1;
-  p.eps = eps; p.use_norm = use_norm; p.o = o; p.w = norm_weight; p.gate_raw = gate_raw; p.y = y;
+  p.eps = eps; p.use_norm = use_norm; p.o = o; p.w = norm_weight; p.gate_raw = gate_raw; p.add = add; p.y = y;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_post", "layer_post", 0.0, (k_layer_post<uint16_t, false>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
   else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_post", "layer_post", 0.0, (k_layer_post<float, false>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
   else return fail("act_dtype must be LACT_BF16 or LACT_F32");
   LACT_CHECK_LAUNCH();
   return 0;
+}
+
+int lact_layer_post_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm, float eps,
+                            const void* o, const float* norm_weight, const void* gate_raw, void* y, void* stream) {
+  return lact_layer_post_add_forward(act_dtype, B, L, H, hd, use_norm, eps, o, norm_weight, gate_raw, nullptr, y, stream);
 }
 
 int32_t lact_layer_post_dw_rows(int32_t B, int32_t L, int32_t H) {

@@ -2,11 +2,12 @@
 //
 //   pre :  qkv [B, L, 3, H, hd]  ->  q, k, v [(B H), L, hd]     silu, per-head L2 norm of q and k, head layout
 //          (bidirectional_lact_layer.py:231-244, causal_lact_with_sliding_window_attn.py:313-322)
+//          and, for the causal layer, the attention's q and k (rescaled per channel) and v in token layout
 //   lr  :  raw [B, L, H, 3] -> lr0, lr1, lr2 [(B H), L]          softplus(raw + inverse-softplus(base lr))
 //          momentum raw [B, L, H] -> [(B H), L]                  sigmoid
 //          (bidirectional_lact_layer.py:248-256, causal_...:326-345)
 //   post:  o [(B H), L, hd] -> y [B, L, H*hd]                    per-head RMSNorm (affine), optional silu gate per
-//          token and head, head layout  (bidirectional_lact_layer.py:268-270, causal_...:351-357)
+//          token and head, head layout, optionally plus the attention branch  (bidirectional_lact_layer.py:268-270, causal_...:351-357)
 //
 // and their backward passes.  One wave per (token, head) row of hd elements; 16 bytes per lane.
 // Element type T = uint16_t (bf16) or float; all statistics in fp32.
@@ -34,83 +35,172 @@ struct LayerPreParams {
   int l2norm;                 // L2-normalise q and k
   const void* qkv;            // [B, L, 3, H, hd]
   void* out[3];               // q, k, v  [(B H), L, hd]
+  // ATT: what the causal layer's attention reads of the same projection, [B, L, H * hd] each: q and k rescaled per channel
+  // (x * qk_scale + qk_offset), v as it is
+  void* att[3];
+  const float* qk_scale;      // [H * hd][2] (q, k), as is qk_offset
+  const float* qk_offset;
+  int round_product;          // the rescaling parameters have type T: so has the product in front of the sum
   // backward
   const void* dout[3];
+  const void* datt[3];
   void* dqkv;
+  float* part;                // ATT: [gridDim.x / H][4][H * hd] partial sums of the gradients of scale q, offset q, scale k, offset k
+  int tokens_per_pass;        // tokens between two of a wave
 };
 
-// Grid: ceil(rows / 4) blocks of 256 threads, one wave per (b, l, h); the wave handles q, k and v of its row.
-template <typename T, bool BWD>
+// Grid: H * m blocks of 256 threads; a wave handles q, k and v of one head and the tokens wave, wave + tokens_per_pass, ...
+// NV: chunks of 256 elements that cover hd.
+// HBM bound: one read of qkv and of the gradients, one write of every output; all loads of a token are issued before the
+// first of them is used (the norms otherwise put three round trips in line).  The attention's inputs ride along because
+// the projection's output is in registers here: as tensor operations of their own (slices, rescaling, and in the backward
+// three zero-padded slice gradients to add up) they took 0.9 ms of a training step at 16384 tokens of 1536 channels.
+template <typename T, bool BWD, bool ATT, int NV>
 __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
-  const long long row = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
-  const int lane = threadIdx.x & 63;
-  if (row >= p.g.rows()) return;
-  const int h = (int)(row % p.g.H);
-  const long long bl = row / p.g.H;            // b*L + l
-  const int l = (int)(bl % p.g.L);
-  const long long b = bl / p.g.L;
-  const int hd = p.g.hd;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int hd = p.g.hd, h = blockIdx.x % p.g.H;
+  const size_t dim = (size_t)p.g.H * hd;
+  float sc[2][NV][4], off[2][NV][4];           // ATT: this lane's channels of the rescaling
+  float acc[4][NV][4];                         // ATT && BWD: this wave's share of the parameter gradients
+  if (ATT) {
 #pragma unroll
-  for (int which = 0; which < 3; ++which) {
-    const size_t si = ((size_t)(bl * 3 + which) * p.g.H + h) * hd;
-    const size_t oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd;
-    const T* src = reinterpret_cast<const T*>(p.qkv) + si;
-    const bool norm = p.l2norm && which < 2;
-    float x[LAYER_VEC_MAX][4], y[LAYER_VEC_MAX][4];
-    float ss = 0.f;
+    for (int i = 0; i < NV; ++i) {
+      const int c = min(lane * 4 + i * 256, hd - 4);
+      const float* ps = p.qk_scale + ((size_t)h * hd + c) * 2;
+      const float4 s0 = *reinterpret_cast<const float4*>(ps), s1 = *reinterpret_cast<const float4*>(ps + 4);
+      sc[0][i][0] = s0.x; sc[1][i][0] = s0.y; sc[0][i][1] = s0.z; sc[1][i][1] = s0.w;
+      sc[0][i][2] = s1.x; sc[1][i][2] = s1.y; sc[0][i][3] = s1.z; sc[1][i][3] = s1.w;
+      if (!BWD) {
+        const float* po = p.qk_offset + ((size_t)h * hd + c) * 2;
+        const float4 o0 = *reinterpret_cast<const float4*>(po), o1 = *reinterpret_cast<const float4*>(po + 4);
+        off[0][i][0] = o0.x; off[1][i][0] = o0.y; off[0][i][1] = o0.z; off[1][i][1] = o0.w;
+        off[0][i][2] = o1.x; off[1][i][2] = o1.y; off[0][i][3] = o1.z; off[1][i][3] = o1.w;
+      } else {
 #pragma unroll
-    for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-      const int c = lane * 4 + i * 256;
-      if (c < hd) {
-        Elem<T>::load4(src + c, x[i]);
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[a][i][j] = 0.f;
+      }
+    }
+  }
+  for (long long bl = (long long)(blockIdx.x / p.g.H) * 4 + wave; bl < (long long)p.g.B * p.g.L; bl += p.tokens_per_pass) {
+    const int l = (int)(bl % p.g.L);
+    const long long b = bl / p.g.L;
+    const size_t oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd, ai = (size_t)bl * dim + (size_t)h * hd;
+    float xs[3][NV][4], gs[3][NV][4], as[3][NV][4];
+#pragma unroll
+    for (int which = 0; which < 3; ++which)
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        const int c = lane * 4 + i * 256;
+        if (c < hd) {
+          Elem<T>::load4(reinterpret_cast<const T*>(p.qkv) + ((size_t)(bl * 3 + which) * p.g.H + h) * hd + c, xs[which][i]);
+          if (BWD) Elem<T>::load4(reinterpret_cast<const T*>(p.dout[which]) + oi + c, gs[which][i]);
+          if (BWD && ATT) Elem<T>::load4(reinterpret_cast<const T*>(p.datt[which]) + ai + c, as[which][i]);
+        } else {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) xs[which][i][j] = gs[which][i][j] = as[which][i][j] = 0.f;
+        }
+      }
+#pragma unroll
+    for (int which = 0; which < 3; ++which) {
+      const bool norm = p.l2norm && which < 2;
+      float (&x)[NV][4] = xs[which];
+      float (&g)[NV][4] = gs[which];
+      float y[NV][4];
+      float ss = 0.f, dot = 0.f;
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
           y[i][j] = Elem<T>::rnd(silu_f(x[i][j]));       // silu output is a tensor of type T in the reference
           ss += y[i][j] * y[i][j];
+          if (BWD) dot += g[i][j] * y[i][j];
         }
-      }
-    }
-    float n = 0.f;
-    if (norm) n = sqrtf(wave_sum(ss));
-    const float inv = norm ? 1.f / (n + 1e-5f) : 1.f;
-    if (!BWD) {
-      T* dst = reinterpret_cast<T*>(p.out[which]) + oi;
-#pragma unroll
-      for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-        const int c = lane * 4 + i * 256;
-        if (c < hd) Elem<T>::store4(dst + c, y[i][0] * inv, y[i][1] * inv, y[i][2] * inv, y[i][3] * inv);
-      }
-    } else {
-      // z = y / (n + eps):  dy = dz / (n + eps) - y <dz, y> / (n (n + eps)^2);  dx = dy silu'(x)
-      const T* dz = reinterpret_cast<const T*>(p.dout[which]) + oi;
-      float g[LAYER_VEC_MAX][4];
-      float dot = 0.f;
-#pragma unroll
-      for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-        const int c = lane * 4 + i * 256;
-        if (c < hd) {
-          Elem<T>::load4(dz + c, g[i]);
-#pragma unroll
-          for (int j = 0; j < 4; ++j) dot += g[i][j] * y[i][j];
-        }
-      }
+      float n = 0.f;
+      if (norm) n = sqrtf(wave_sum(ss));
+      const float inv = norm ? 1.f / (n + 1e-5f) : 1.f;
       float c1 = 0.f;
-      if (norm) {
+      if (BWD && norm) {
+        // z = y / (n + eps):  dy = dz / (n + eps) - y <dz, y> / (n (n + eps)^2);  dx = dy silu'(x)
         dot = wave_sum(dot);
         c1 = n > 0.f ? dot / (n * (n + 1e-5f) * (n + 1e-5f)) : 0.f;
       }
-      T* dx = reinterpret_cast<T*>(p.dqkv) + si;
 #pragma unroll
-      for (int i = 0; i < LAYER_VEC_MAX; ++i) {
+      for (int i = 0; i < NV; ++i) {
         const int c = lane * 4 + i * 256;
-        if (c < hd) {
+        if (c >= hd) continue;
+        if (!BWD) {
+          Elem<T>::store4(reinterpret_cast<T*>(p.out[which]) + oi + c, y[i][0] * inv, y[i][1] * inv, y[i][2] * inv, y[i][3] * inv);
+          if (ATT) {
+            float a[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              a[j] = x[i][j];
+              if (which < 2) {
+                a[j] = __fmul_rn(a[j], sc[which & 1][i][j]);
+                if (p.round_product) a[j] = Elem<T>::rnd(a[j]);
+                a[j] = __fadd_rn(a[j], off[which & 1][i][j]);
+              }
+            }
+            Elem<T>::store4(reinterpret_cast<T*>(p.att[which]) + ai + c, a[0], a[1], a[2], a[3]);
+          }
+        } else {
           float o[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) o[j] = (g[i][j] * inv - y[i][j] * c1) * silu_grad_f(x[i][j]);
-          Elem<T>::store4(dx + c, o[0], o[1], o[2], o[3]);
+          for (int j = 0; j < 4; ++j) {
+            o[j] = (g[i][j] * inv - y[i][j] * c1) * silu_grad_f(x[i][j]);
+            if (ATT) {
+              const float a = as[which][i][j];
+              if (which < 2) {
+                acc[2 * (which & 1)][i][j] += a * x[i][j];
+                acc[2 * (which & 1) + 1][i][j] += a;
+                o[j] += a * sc[which & 1][i][j];
+              } else {
+                o[j] += a;
+              }
+            }
+          }
+          Elem<T>::store4(reinterpret_cast<T*>(p.dqkv) + ((size_t)(bl * 3 + which) * p.g.H + h) * hd + c, o[0], o[1], o[2], o[3]);
         }
       }
     }
+  }
+  if (ATT && BWD) {      // the four waves' shares, in a fixed order
+    __shared__ float red[4][NV * 256];
+    for (int w = 0; w < 4; ++w) {
+      if (wave == w) {
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+#pragma unroll
+          for (int i = 0; i < NV; ++i)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+              float* r = &red[a][lane * 4 + i * 256 + j];
+              *r = w == 0 ? acc[a][i][j] : *r + acc[a][i][j];
+            }
+      }
+      __syncthreads();
+    }
+    for (int a = 0; a < 4; ++a)
+      for (int c = threadIdx.x; c < hd; c += 256) p.part[((size_t)(blockIdx.x / p.g.H) * 4 + a) * dim + (size_t)h * hd + c] = red[a][c];
+  }
+}
+
+// Sums the partial rows of k_layer_pre's parameter gradients into dscale, doffset [dim][2].  Grid ceil(dim / 64) x 4 blocks
+// of 256 threads: 64 columns, four groups of rows.
+__global__ __launch_bounds__(256) void k_layer_qk_reduce(const float* part, int rows, int dim, float* dscale, float* doffset) {
+  __shared__ float red[4][64];
+  const int c = blockIdx.x * 64 + (threadIdx.x & 63), a = blockIdx.y, grp = threadIdx.x >> 6;
+  float s = 0.f;
+  if (c < dim)
+#pragma unroll 8
+    for (int r = grp; r < rows; r += 4) s += part[((size_t)r * 4 + a) * dim + c];
+  red[grp][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (grp == 0 && c < dim) {
+    const int i = threadIdx.x & 63;
+    (a & 1 ? doffset : dscale)[(size_t)c * 2 + a / 2] = red[0][i] + red[1][i] + red[2][i] + red[3][i];
   }
 }
 
@@ -158,6 +248,7 @@ struct LayerPostParams {
   const void* o;              // [(B H), L, hd]
   const float* w;             // [hd] RMSNorm weight (null = ones)
   const void* gate_raw;       // [B, L, H] type T, or null: y *= silu(gate_raw)
+  const void* add;            // [B, L, H*hd] type T, or null: y += add (the layer's attention branch)
   void* y;                    // [B, L, H*hd]
   // backward
   const void* dy; void* d_o; void* dgate_raw;
@@ -217,6 +308,12 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
             float t = x[i][j] * rstd;
             if (p.use_norm) t = Elem<T>::rnd(t * wv[i][j]);     // the normalised tensor has type T in the reference
             o[j] = t * gate;
+          }
+          if (p.add) {
+            float a[4];
+            Elem<T>::load4(reinterpret_cast<const T*>(p.add) + yi + c, a);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) o[j] = a[j] + Elem<T>::rnd(o[j]);
           }
           Elem<T>::store4(dst + c, o[0], o[1], o[2], o[3]);
         }

@@ -74,6 +74,40 @@ class _PreFn(torch.autograd.Function):
         return dqkv, None, None, None
 
 
+class _PreAttnFn(torch.autograd.Function):
+    """qkv [B, L, 3*H*hd], qk_scale, qk_offset [H*hd, 2] -> q, k, v [(B H), L, hd] as _PreFn, and the attention's rescaled q and
+    k and its v, [B, L, H*hd] each."""
+
+    @staticmethod
+    def forward(ctx, qkv, qk_scale, qk_offset, H, hd, l2norm):
+        qkv = qkv.contiguous()
+        B, L, _ = qkv.shape
+        scale, offset = qk_scale.detach().float().contiguous(), qk_offset.detach().float().contiguous()
+        outs = [torch.empty((B * H, L, hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3)]
+        att = [torch.empty((B, L, H * hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3)]
+        with torch.cuda.device(qkv.device):
+            _lib.check(_lib.lib().lact_layer_pre_attn_forward(
+                _act(qkv), B, L, H, hd, int(l2norm), int(qk_scale.dtype == qkv.dtype), _ptr(qkv), _ptr(scale), _ptr(offset),
+                *[_ptr(t) for t in outs], *[_ptr(t) for t in att], _stream(qkv)))
+        ctx.save_for_backward(qkv, scale)
+        ctx.dims, ctx.dtypes = (B, L, H, hd, int(l2norm)), (qk_scale.dtype, qk_offset.dtype)
+        return (*outs, *att)
+
+    @staticmethod
+    def backward(ctx, *grads):
+        qkv, scale = ctx.saved_tensors
+        B, L, H, hd, l2norm = ctx.dims
+        shapes = [(B * H, L, hd)] * 3 + [(B, L, H * hd)] * 3
+        grads = [torch.zeros(s, dtype=qkv.dtype, device=qkv.device) if g is None else g.to(qkv.dtype).contiguous() for g, s in zip(grads, shapes)]
+        lib = _lib.lib()
+        dqkv, dscale, doffset = torch.empty_like(qkv), torch.empty_like(scale), torch.empty_like(scale)
+        part = torch.empty(lib.lact_layer_pre_attn_part_rows(B, L, H) * 4 * H * hd, dtype=torch.float32, device=qkv.device)
+        with torch.cuda.device(qkv.device):
+            _lib.check(lib.lact_layer_pre_attn_backward(_act(qkv), B, L, H, hd, l2norm, _ptr(qkv), _ptr(scale), *[_ptr(g) for g in grads],
+                                                        _ptr(dqkv), _ptr(part), _ptr(dscale), _ptr(doffset), _stream(qkv)))
+        return dqkv, dscale.to(ctx.dtypes[0]), doffset.to(ctx.dtypes[1]), None, None, None
+
+
 class _LrFn(torch.autograd.Function):
     """lr_raw [B, L, 3*H] (head-major with three rates per head, or rate-major when rates_major), momentum_raw
     [B, L, H] or None -> lr0, lr1, lr2, momentum [(B H), L, 1] fp32."""
@@ -113,19 +147,21 @@ class _LrFn(torch.autograd.Function):
 
 class _PostFn(torch.autograd.Function):
     """o [(B H), L, hd] -> y [B, L, H*hd]: RMSNorm(weight) per head if weight is given or use_norm, times
-    silu(gate_raw [B, L, H]) if given."""
+    silu(gate_raw [B, L, H]) if given, plus add [B, L, H*hd] if given."""
 
     @staticmethod
-    def forward(ctx, o, weight, gate_raw, B, H, use_norm, eps):
+    def forward(ctx, o, weight, gate_raw, B, H, use_norm, eps, add=None):
         o = o.contiguous()
         _, L, hd = o.shape
         w = None if weight is None else weight.float().contiguous()
         g = None if gate_raw is None else gate_raw.to(o.dtype).contiguous()
+        add_c = None if add is None else add.to(o.dtype).contiguous()
         y = torch.empty((B, L, H * hd), dtype=o.dtype, device=o.device)
         with torch.cuda.device(o.device):
-            _lib.check(_lib.lib().lact_layer_post_forward(_act(o), B, L, H, hd, int(use_norm), float(eps), _ptr(o), _ptr(w),
-                                                          _ptr(g), _ptr(y), _stream(o)))
+            _lib.check(_lib.lib().lact_layer_post_add_forward(_act(o), B, L, H, hd, int(use_norm), float(eps), _ptr(o), _ptr(w),
+                                                          _ptr(g), _ptr(add_c), _ptr(y), _stream(o)))
         ctx.save_for_backward(o, w, g)
+        ctx.add_dtype = None if add is None else add.dtype
         ctx.dims = (B, L, H, hd, int(use_norm), float(eps))
         ctx.dtypes = (None if weight is None else weight.dtype, None if gate_raw is None else gate_raw.dtype)
         return y
@@ -145,7 +181,7 @@ class _PostFn(torch.autograd.Function):
                                                     _ptr(d_o), _ptr(dg), _ptr(dw_part), _stream(o)))
         wd, gd = ctx.dtypes
         dw = None if dw_part is None else dw_part.sum(dim=0).to(wd)
-        return d_o, dw, (None if dg is None else dg.to(gd)), None, None, None, None
+        return d_o, dw, (None if dg is None else dg.to(gd)), None, None, None, None, (None if ctx.add_dtype is None else dy.to(ctx.add_dtype))
 
 
 def _fast_weights(layer, B):
@@ -282,18 +318,11 @@ class CausalLaCTSwiGLUWithSlidingWindowAttn(nn.Module):
         # the reference creates this only when ttt_scale_before_sum, and its forward always uses it (:348)
         self.ttt_scale_proj = nn.Linear(dim, self.num_ttt_heads)
 
-    def _rescale_qk(self, q, k):
-        dt = q.dtype
-        q = q * self.qk_scale[:, 0] + self.qk_offset[:, 0]
-        k = k * self.qk_scale[:, 1] + self.qk_offset[:, 1]
-        return q.to(dt), k.to(dt)
-
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x: [b, l, d] -> [b, l, d]"""
         B, L, _ = x.shape
         H = self.num_ttt_heads
-        attn_qkv = self.to_qkv(x)
-        q, k, v = _PreFn.apply(attn_qkv, H, self.head_dim, True)
+        q, k, v, aq, ak, av = _PreAttnFn.apply(self.to_qkv(x), self.qk_scale, self.qk_offset, H, self.head_dim, True)
         with torch.autocast(device_type="cuda", enabled=False):
             lr_raw = self.lr_proj(x)
         mom_raw = self.momentum_proj[0](x) if self.use_momentum else None      # the Sigmoid of the Sequential is in the kernel
@@ -303,13 +332,10 @@ class CausalLaCTSwiGLUWithSlidingWindowAttn(nn.Module):
         w0, w1, w2 = _fast_weights(self, B)
         o = block_causal_lact_swiglu(w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, self.use_muon,
                                      chunk_size=self.lact_chunk_size)
-        weight, use_norm, eps = _norm_args(self.o_norm)
-        ttt = _PostFn.apply(o, weight, self.ttt_scale_proj(x), B, H, use_norm, eps)
-        aq, ak, av = attn_qkv.chunk(3, dim=-1)
-        aq, ak = self._rescale_qk(aq, ak)
         sh = lambda t: t.reshape(B, L, self.num_attn_heads, self.attn_head_dim)
         attn = sliding_window_attention(sh(aq), sh(ak), sh(av), self.window_size).reshape(B, L, -1)
-        return self.o_proj(attn + ttt)
+        weight, use_norm, eps = _norm_args(self.o_norm)
+        return self.o_proj(_PostFn.apply(o, weight, self.ttt_scale_proj(x), B, H, use_norm, eps, attn))
 
 
 class FastWeightGluMLPMultihead(nn.Module):

@@ -27,3 +27,30 @@ def test_window_attention_against_oracle(b, l, h, d, window):
     assert out.dtype == torch.bfloat16 and rel_l2(out, ref) < 5e-3
     for i, (a, r) in enumerate(zip(gx.chunk(3, dim=-1), gr.chunk(3, dim=-1))):
         assert rel_l2(a, r) < 1e-2, i
+
+
+@pytest.mark.parametrize("dtype,B,L,H,hd", [(torch.float32, 2, 37, 3, 16), (torch.float32, 1, 5, 2, 520), (torch.bfloat16, 1, 4099, 2, 384)])
+def test_pre_attention_kernel_against_torch(dtype, B, L, H, hd):
+    """The layer's pre-processing with the attention's inputs: outputs, and the gradients of the projection and of the rescaling."""
+    print("[gpu-test] layer pre with attention", dtype, B, L, H, hd, flush=True)
+    from lact_amd import layers as HL
+    g = torch.Generator().manual_seed(7)
+    qkv = torch.randn(B, L, 3 * H * hd, generator=g).to(dtype)
+    scale, offset = torch.rand(H * hd, 2, generator=g) + 0.5, torch.randn(H * hd, 2, generator=g)
+    gos = [torch.randn(B * H, L, hd, generator=g).to(dtype) for _ in range(3)] + [torch.randn(B, L, H * hd, generator=g).to(dtype) for _ in range(3)]
+
+    def reference(t, s, o):
+        raw = t.chunk(3, dim=-1)
+        heads = [torch.nn.functional.silu(r).reshape(B, L, H, hd).transpose(1, 2).reshape(B * H, L, hd) for r in raw]
+        norm = lambda x: x / (x.norm(dim=-1, keepdim=True) + 1e-5)
+        return [norm(heads[0]), norm(heads[1]), heads[2], raw[0] * s[:, 0] + o[:, 0], raw[1] * s[:, 1] + o[:, 1], raw[2]]
+
+    ref_in = [t.double().requires_grad_(True) for t in (qkv, scale, offset)]
+    ref = reference(*ref_in)
+    ref_grads = torch.autograd.grad(ref, ref_in, [t.double() for t in gos])
+    dev_in = [t.to("cuda").requires_grad_(True) for t in (qkv, scale, offset)]
+    out = HL._PreAttnFn.apply(*dev_in, H, hd, True)
+    grads = torch.autograd.grad(out, dev_in, [t.to("cuda") for t in gos])
+    tol = 1e-5 if dtype == torch.float32 else 6e-3
+    for a, r in zip(list(out) + list(grads), list(ref) + list(ref_grads)):
+        assert a.shape == r.shape and rel_l2(a, r) < tol

@@ -44,7 +44,25 @@ EXPORTS = ("lact_last_error", "lact_version", "lact_query_sizes", "lact_forward"
            "lact_window_attention_forward", "lact_window_attention_backward", "lact_layer_pre_attn_forward",
            "lact_layer_pre_attn_part_rows", "lact_layer_pre_attn_backward", "lact_layer_post_add_forward")
 
+HOST_PATH = os.path.join(HERE, "lib", "_lact_host.so")
+
 _lib = None
+_host = None
+
+
+def host():
+    """The native host module over the library (csrc/torch_host.cpp)."""
+    global _host
+    if _host is None:
+        lib()
+        import importlib.util
+        import torch  # noqa: F401  (its libraries have to be loaded first)
+        if not os.path.exists(HOST_PATH):
+            raise RuntimeError(f"{HOST_PATH} is missing: build it with `python -m lact_amd.build`. lact_amd has no CPU or PyTorch fallback.")
+        spec = importlib.util.spec_from_file_location("_lact_host", HOST_PATH)
+        _host = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(_host)
+    return _host
 
 
 def lib():

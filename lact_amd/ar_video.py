@@ -1,6 +1,7 @@
 """Drop-ins for the operations of lact_ar_video/minVid/models/blocks/ar_lact_swa_repeat{,_sp}.py."""
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -32,6 +33,18 @@ def _ar_steps(seq_len, q_len, mini_batch_size, update_length, update_every, num_
     return tuple(steps)
 
 
+@lru_cache(maxsize=256)
+def _interleaved_program(kv_len, q_len, mini_batch_size, update_length, update_every, num_repeat, iters, weight_norm, ns_mode):
+    return Program(steps=_ar_steps(kv_len, q_len, mini_batch_size, update_length, update_every, num_repeat), out_len=q_len,
+                   ns_coeffs=None if iters is None else (NS_CLASSIC,) * iters, weight_norm=weight_norm, ns_mode=ns_mode)
+
+
+@lru_cache(maxsize=256)
+def _inference_program(mini_batch, updates, q_len, iters, weight_norm, ns_mode):
+    return Program(steps=((LACT_UPDATE, 0, mini_batch, 0),) * updates + ((LACT_APPLY, 0, q_len, 0),), out_len=q_len,
+                   ns_coeffs=None if iters is None else (NS_CLASSIC,) * iters, weight_norm=weight_norm, ns_mode=ns_mode)
+
+
 def _scaled(lr, w_scale: float):
     """The reference forms (k * lr) * w_scale, left to right (ar_lact_swa_repeat.py:134-138); the kernels take one
     per-token factor, so lr * w_scale is folded first.  The two agree bit for bit when w_scale is a power of two --
@@ -45,9 +58,8 @@ def ar_fast_weight_swish_glu_weight_norm_mini_batch_with_momentum(
         update_length: int = -1, update_every: int = -1, use_moun: bool = False, num_moun_iters: int = 3,
         weight_norm: bool = True, fw_momentum: Optional[torch.Tensor] = None, use_momentum: bool = False):
     """ar_lact_swa_repeat_sp.py:28-193.  Returns (output, w0, w1, w2)."""
-    prog = Program(steps=_ar_steps(k.shape[1], q.shape[1], mini_batch_size, update_length, update_every, num_repeat),
-                   out_len=q.shape[1], ns_coeffs=(NS_CLASSIC,) * num_moun_iters if use_moun else None,
-                   weight_norm=weight_norm, ns_mode=ops._ns_mode(q))
+    prog = _interleaved_program(k.shape[1], q.shape[1], mini_batch_size, update_length, update_every, num_repeat,
+                                num_moun_iters if use_moun else None, bool(weight_norm), ops._ns_mode(q))
     out, ws, _ = run_program(prog, w0, w1, w2, q, k, v, _scaled(lr0, w_scale), _scaled(lr1, w_scale), _scaled(lr2, w_scale),
                              fw_momentum if use_momentum else None)
     return (out,) + tuple(ws)
@@ -68,10 +80,8 @@ def ar_fast_weight_swish_glu_weight_norm_mini_batch_inference(
         do_update: bool = False, use_moun: bool = False, num_moun_iters: int = 3, weight_norm: bool = True):
     """ar_lact_swa_repeat.py:172-296: optional repeated update on the first mini-batch, then apply on all q."""
     mb = k.shape[1] if mini_batch_size == -1 else min(mini_batch_size, k.shape[1])
-    steps = [(LACT_UPDATE, 0, mb, 0)] * (num_repeat if do_update else 0) + [(LACT_APPLY, 0, q.shape[1], 0)]
-    prog = Program(steps=tuple(steps), out_len=q.shape[1],
-                   ns_coeffs=(NS_CLASSIC,) * num_moun_iters if use_moun else None,
-                   weight_norm=weight_norm, ns_mode=ops._ns_mode(q))
+    prog = _inference_program(mb, num_repeat if do_update else 0, q.shape[1], num_moun_iters if use_moun else None, bool(weight_norm),
+                              ops._ns_mode(q))
     out, ws, _ = run_program(prog, w0, w1, w2, q, k, v, _scaled(lr0, w_scale), _scaled(lr1, w_scale), _scaled(lr2, w_scale), None)
     return (out,) + tuple(ws)
 
@@ -86,10 +96,7 @@ def ar_fast_weight_swish_glu_weight_norm_mini_batch_inference_with_momentum(
     come out, so that the caller can keep them between denoising steps.  Inference only (torch.no_grad)."""
     mb = k.shape[1] if mini_batch_size == -1 else min(mini_batch_size, k.shape[1])
     updates = num_repeat if do_update else 0
-    steps = [(LACT_UPDATE, 0, mb, 0)] * updates + [(LACT_APPLY, 0, q.shape[1], 0)]
-    prog = Program(steps=tuple(steps), out_len=q.shape[1],
-                   ns_coeffs=(NS_CLASSIC,) * num_moun_iters if use_moun else None,
-                   weight_norm=weight_norm, ns_mode=ops._ns_mode(q))
+    prog = _inference_program(mb, updates, q.shape[1], num_moun_iters if use_moun else None, bool(weight_norm), ops._ns_mode(q))
     state = (dw0_momentum, dw1_momentum, dw2_momentum) if (use_momentum and dw0_momentum is not None) else None
     out, ws, ms = run_program(prog, w0, w1, w2, q, k, v, _scaled(lr0, w_scale), _scaled(lr1, w_scale), _scaled(lr2, w_scale),
                               fw_momentum if use_momentum else None, momentum_state=state if updates else None)

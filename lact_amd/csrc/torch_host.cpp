@@ -1,0 +1,303 @@
+// PyTorch side of the operation's calls: checks and converts the tensors, allocates outputs and buffers with torch's
+// allocator, enqueues liblact_hip.so on torch's current stream and carries the autograd boundary.  Native because a small
+// call (one view rendered, one short sequence) is bound by this code: the same steps in Python cost 65 us of host time per
+// forward call and made the GPU wait.  All arithmetic stays behind the C ABI (include/lact_hip.h).
+#include <torch/extension.h>
+#include <torch/csrc/autograd/functions/basic_ops.h>
+#include <ATen/autocast_mode.h>
+#include <c10/hip/HIPGuard.h>
+#include <c10/hip/HIPStream.h>
+
+#include <algorithm>
+#include <memory>
+#include <optional>
+#include <string>
+#include <utility>
+#include <vector>
+
+#include "../../include/lact_hip.h"
+
+namespace {
+
+using at::Tensor;
+using OptTensor = std::optional<Tensor>;
+using torch::autograd::AutogradContext;
+using torch::autograd::variable_list;
+
+// A test-time-training schedule (ops.Program) in the C ABI's terms.
+struct Schedule : torch::CustomClassHolder {
+  std::vector<lact_step_t> steps;
+  std::vector<float> coeffs;
+  lact_desc_t flags{};          // everything of a descriptor that does not depend on the tensors
+  int64_t out_len = 0;
+  bool has_update = false, return_state = true, covers = false;
+
+  Schedule(const std::vector<std::vector<int>>& steps_, int64_t out_len_, const std::optional<std::vector<float>>& coeffs_, bool prenorm,
+           bool weight_norm, bool detach_norms, bool muon_replaces_weight, int ns_mode, bool muon_stacked, bool renorm_eps_in_sqrt,
+           bool return_state_)
+      : out_len(out_len_), return_state(return_state_) {
+    std::vector<std::pair<int, int>> rows;
+    for (const auto& s : steps_) {
+      steps.push_back(lact_step_t{s.at(0), s.at(1), s.at(2), s.at(3)});
+      if (s[0] == LACT_UPDATE) has_update = true;
+      else rows.emplace_back(s[3], s[3] + s[2] - s[1]);
+    }
+    if (coeffs_) coeffs = *coeffs_;
+    flags.n_steps = (int)steps.size();
+    flags.out_len = (int)out_len;
+    flags.ns_steps = coeffs_ ? (int)coeffs.size() / 3 : -1;
+    flags.prenorm = prenorm; flags.weight_norm = weight_norm; flags.detach_norms = detach_norms;
+    flags.muon_replaces_weight = muon_replaces_weight; flags.ns_mode = ns_mode;
+    flags.muon_stacked = muon_stacked; flags.renorm_eps_in_sqrt = renorm_eps_in_sqrt;
+    // do the apply steps write every output row?
+    std::sort(rows.begin(), rows.end());
+    int pos = 0;
+    covers = true;
+    for (auto& r : rows) {
+      if (r.first > pos) covers = false;
+      pos = std::max(pos, r.second);
+    }
+    covers = covers && pos >= out_len;
+  }
+};
+
+void check(int rc) {
+  if (rc != 0) throw std::runtime_error(std::string("liblact_hip: ") + lact_last_error());
+}
+
+// [b, L, d] whose rows the kernels can read with 16-byte vectors
+Tensor rows_view(Tensor t, at::ScalarType dtype) {
+  if (t.scalar_type() != dtype) t = t.to(dtype);
+  const int64_t align = 16 / t.element_size();
+  const bool ok = t.dim() == 3 && t.stride(2) == 1 && t.stride(1) % align == 0 && t.stride(0) % align == 0 && t.stride(1) >= t.size(2) &&
+                  reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+  return ok ? t : t.contiguous();
+}
+
+Tensor plain_f32(const Tensor& t) {
+  return t.scalar_type() == at::kFloat ? t.contiguous() : t.to(at::kFloat).contiguous();
+}
+
+Tensor per_token(const Tensor& t, int64_t b, int64_t L, const char* name) {
+  if (t.numel() != b * L) {
+    std::string s = "(";
+    for (auto v : t.sizes()) s += std::to_string(v) + ", ";
+    throw std::invalid_argument(std::string(name) + " must hold one value per head and token ([b, l, 1]); got " + s + ")");
+  }
+  return plain_f32(t.reshape({b, L}));
+}
+
+void* ptr(const Tensor& t) { return t.defined() ? t.data_ptr() : nullptr; }
+template <typename T = float>
+T* fptr(const Tensor& t) { return static_cast<T*>(ptr(t)); }
+
+lact_desc_t describe(const Schedule& sc, int64_t b, int64_t d, int64_t dh, const Tensor& q, const Tensor& k, const Tensor& v, const Tensor& out) {
+  lact_desc_t D = sc.flags;
+  D.b = (int)b; D.d = (int)d; D.dh = (int)dh;
+  D.q_len = (int)q.size(1); D.kv_len = k.defined() ? (int)k.size(1) : 0;
+  D.act_dtype = q.scalar_type() == at::kBFloat16 ? LACT_BF16 : LACT_F32;
+  D.steps = sc.steps.data();
+  D.ns_coeffs = sc.coeffs.empty() ? nullptr : sc.coeffs.data();
+  D.q_bs = q.stride(0); D.q_ld = (int)q.stride(1);
+  if (k.defined()) {
+    D.k_bs = k.stride(0); D.k_ld = (int)k.stride(1); D.v_bs = v.stride(0); D.v_ld = (int)v.stride(1);
+  } else {
+    D.k_ld = D.v_ld = (int)d;
+  }
+  D.o_bs = D.do_bs = out.stride(0); D.o_ld = D.do_ld = (int)out.stride(1);
+  return D;
+}
+
+struct Operands {      // what a forward call hands to its backward
+  Tensor q, k, v, lr0, lr1, lr2, momentum, saved;
+  int64_t b = 0, d = 0, dh = 0;
+};
+
+// Returns the output, the three final weights (when the schedule returns its state) and the three momentum states (when it
+// does and there is momentum).
+std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& w1, const Tensor& w2, const Tensor& q, const OptTensor& k,
+                            const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1, const OptTensor& lr2, const OptTensor& momentum,
+                            const std::vector<Tensor>& m_state, bool needs_backward, Operands* keep) {
+  if (!q.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)");
+  const c10::hip::HIPGuard guard(q.device().index());
+  const int64_t b = w0.size(0), dh = w0.size(1), d = w0.size(2);
+  if (w1.sizes() != at::IntArrayRef({b, d, dh}) || w2.sizes() != at::IntArrayRef({b, dh, d}))
+    throw std::invalid_argument("expected w0, w2: [b, dh, d] and w1: [b, d, dh] with equal key and value dims");
+  auto act = (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) ? at::kBFloat16 : at::kFloat;
+  if (at::autocast::is_autocast_enabled(at::kCUDA)) act = at::kBFloat16;
+  Operands o;
+  o.b = b; o.d = d; o.dh = dh;
+  o.q = rows_view(q, act);
+  if (sc.has_update) {
+    if (!k || !v || !lr0 || !lr1 || !lr2) throw std::invalid_argument("a schedule with an update needs k, v and the three learning rates");
+    o.k = rows_view(*k, act);
+    o.v = rows_view(*v, act);
+    const int64_t L = o.k.size(1);
+    o.lr0 = per_token(*lr0, b, L, "lr");
+    o.lr1 = per_token(*lr1, b, L, "lr");
+    o.lr2 = per_token(*lr2, b, L, "lr");
+    if (momentum) o.momentum = per_token(*momentum, b, L, "momentum");
+  }
+  const Tensor w[3] = {plain_f32(w0), plain_f32(w1), plain_f32(w2)};
+  const auto act_opt = o.q.options();
+  Tensor out = sc.covers ? at::empty({b, sc.out_len, d}, act_opt) : at::zeros({b, sc.out_len, d}, act_opt);
+  lact_desc_t D = describe(sc, b, d, dh, o.q, o.k, o.v, out);
+  D.use_momentum = o.momentum.defined();
+  D.forward_only = !needs_backward;
+  Tensor m_in[3];
+  const bool carried = !m_state.empty() && o.momentum.defined();
+  if (carried) {
+    if (needs_backward) throw std::runtime_error("a carried momentum state is an inference feature: call under torch.no_grad()");
+    for (int i = 0; i < 3; ++i) {
+      m_in[i] = plain_f32(m_state.at(i));
+      if (m_in[i].sizes() != w[i].sizes()) throw std::invalid_argument("momentum states must have the shapes of w0, w1, w2");
+    }
+    D.momentum_state_in = 1;
+  }
+  size_t saved_bytes = 0, scratch_bytes = 0;
+  check(lact_query_sizes(&D, &saved_bytes, &scratch_bytes));
+  const auto bytes = act_opt.dtype(at::kByte);
+  o.saved = at::empty({(int64_t)saved_bytes}, bytes);
+  const Tensor scratch = at::empty({(int64_t)scratch_bytes}, bytes);
+  std::vector<Tensor> res{out};
+  float* w_out[3] = {nullptr, nullptr, nullptr};
+  float* m_out[3] = {nullptr, nullptr, nullptr};
+  if (sc.return_state) {
+    for (int i = 0; i < 3; ++i) res.push_back(at::empty_like(w[i]));
+    if (o.momentum.defined())
+      for (int i = 0; i < 3; ++i) res.push_back(at::empty_like(w[i]));
+    for (int i = 0; i < 3; ++i) w_out[i] = fptr(res[1 + i]);
+    if (o.momentum.defined())
+      for (int i = 0; i < 3; ++i) m_out[i] = fptr(res[4 + i]);
+  }
+  const float* m_ptr[3] = {fptr(m_in[0]), fptr(m_in[1]), fptr(m_in[2])};
+  check(lact_forward_from_state(&D, fptr(w[0]), fptr(w[1]), fptr(w[2]), ptr(o.q), ptr(o.k), ptr(o.v), fptr(o.lr0), fptr(o.lr1), fptr(o.lr2),
+                                fptr(o.momentum), carried ? m_ptr : nullptr, ptr(out), w_out, m_out, ptr(o.saved), ptr(scratch),
+                                c10::hip::getCurrentHIPStream().stream()));
+  auto out_dtype = (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kFloat) ? q.scalar_type() : act;
+  if (v && v->scalar_type() == at::kFloat && act == at::kBFloat16) out_dtype = at::kFloat;   // zeros_like(v) receives the bf16 products
+  if (out_dtype != act) res[0] = out.to(out_dtype);
+  if (keep) *keep = std::move(o);
+  return res;
+}
+
+Tensor cast(const Tensor& t, at::ScalarType dtype) { return !t.defined() || t.scalar_type() == dtype ? t : t.to(dtype); }
+
+// What the backward of one call needs beside the saved tensors.
+struct CallRecord : torch::CustomClassHolder {
+  c10::intrusive_ptr<Schedule> sc;
+  int64_t b = 0, d = 0, dh = 0;
+  at::ScalarType dtype[8];                 // of w0, w1, w2, q, k, v, the rates, momentum
+  std::vector<int64_t> lr_shape, m_shape;
+};
+
+struct ProgramFn : torch::autograd::Function<ProgramFn> {
+  static variable_list forward(AutogradContext* ctx, c10::intrusive_ptr<Schedule> sc, const Tensor& w0, const Tensor& w1, const Tensor& w2,
+                               const Tensor& q, const OptTensor& k, const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1,
+                               const OptTensor& lr2, const OptTensor& momentum) {
+    Operands o;
+    auto res = ::forward(*sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, {}, true, &o);
+    auto rec = c10::make_intrusive<CallRecord>();
+    rec->sc = sc;
+    rec->b = o.b; rec->d = o.d; rec->dh = o.dh;
+    auto type = [](const OptTensor& t) { return t ? t->scalar_type() : at::kFloat; };
+    const at::ScalarType types[8] = {type(w0), type(w1), type(w2), type(q), type(k), type(v), type(lr0), type(momentum)};
+    std::copy(types, types + 8, rec->dtype);
+    if (lr0) rec->lr_shape = lr0->sizes().vec();
+    if (momentum) rec->m_shape = momentum->sizes().vec();
+    ctx->save_for_backward({o.q, o.k, o.v, o.lr0, o.lr1, o.lr2, o.momentum, o.saved});
+    ctx->saved_data["call"] = c10::IValue::make_capsule(std::move(rec));
+    if (res.size() == 7) ctx->mark_non_differentiable({res[4], res[5], res[6]});
+    ctx->set_materialize_grads(false);   // unused outputs arrive undefined in backward, not as zero tensors
+    return res;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool twice = at::GradMode::is_enabled() &&
+                       std::any_of(grads.begin(), grads.end(), [](const Tensor& g) { return g.defined() && g.requires_grad(); });
+    const at::AutoGradMode off(false);
+    auto t = ctx->get_saved_variables();
+    const Tensor &q = t[0], &k = t[1], &v = t[2], &momentum = t[6], &saved = t[7];
+    const auto capsule = ctx->saved_data["call"].toCapsule();
+    const auto& rec = static_cast<const CallRecord&>(*capsule);
+    const Schedule& sc = *rec.sc;
+    const int64_t b = rec.b, d = rec.d, dh = rec.dh;
+    const c10::hip::HIPGuard guard(q.device().index());
+    const auto act_opt = q.options(), f32 = act_opt.dtype(at::kFloat);
+    Tensor g_out = grads[0].defined() ? rows_view(grads[0], q.scalar_type()) : at::zeros({b, sc.out_len, d}, act_opt);
+    Tensor gw[3];
+    const float* gwp[3] = {nullptr, nullptr, nullptr};
+    for (size_t i = 0; i < 3 && i + 1 < grads.size(); ++i)
+      if (grads[i + 1].defined()) {
+        gw[i] = plain_f32(grads[i + 1]);
+        gwp[i] = fptr(gw[i]);
+      }
+    lact_desc_t D = describe(sc, b, d, dh, q, k, v, g_out);
+    D.use_momentum = momentum.defined();
+    size_t saved_bytes = 0, scratch_bytes = 0;
+    check(lact_query_sizes(&D, &saved_bytes, &scratch_bytes));
+    const Tensor scratch = at::empty({(int64_t)scratch_bytes}, act_opt.dtype(at::kByte));
+    // lact_backward writes every element of its outputs (rows no step touches are zeroed by the library)
+    const Tensor dw[3] = {at::empty({b, dh, d}, f32), at::empty({b, d, dh}, f32), at::empty({b, dh, d}, f32)};
+    const Tensor dq = at::empty({b, q.size(1), d}, act_opt);
+    Tensor dk, dv, dlr[3], dm;
+    if (sc.has_update) {
+      dk = at::empty({b, k.size(1), d}, act_opt);
+      dv = at::empty({b, k.size(1), d}, act_opt);
+      for (auto& x : dlr) x = at::empty({b, k.size(1)}, f32);
+      if (momentum.defined()) dm = at::empty({b, k.size(1)}, f32);
+    }
+    check(lact_backward(&D, ptr(q), ptr(k), ptr(v), fptr(t[3]), fptr(t[4]), fptr(t[5]), fptr(momentum), ptr(g_out), gwp, ptr(saved),
+                        ptr(scratch), fptr(dw[0]), fptr(dw[1]), fptr(dw[2]), ptr(dq), ptr(dk), ptr(dv), fptr(dlr[0]), fptr(dlr[1]), fptr(dlr[2]),
+                        fptr(dm), c10::hip::getCurrentHIPStream().stream()));
+    auto type = [&](int i) { return rec.dtype[i]; };
+    variable_list res{Tensor(), cast(dw[0], type(0)), cast(dw[1], type(1)), cast(dw[2], type(2)), cast(dq, type(3)), cast(dk, type(4)), cast(dv, type(5))};
+    for (auto& x : dlr) res.push_back(x.defined() ? cast(x.reshape(rec.lr_shape), type(6)) : x);
+    res.push_back(dm.defined() ? cast(dm.reshape(rec.m_shape), type(7)) : dm);
+    if (twice) {   // the gradients have no backward of their own: an attempt at one is an error, not a silent zero
+      auto err = std::make_shared<torch::autograd::DelayedError>(
+          "trying to differentiate twice a function that was marked with @once_differentiable", (int64_t)res.size());
+      for (auto& x : res)
+        if (x.defined()) x = x.detach().set_requires_grad(true);
+      const at::AutoGradMode on(true);
+      res = (*err)(std::move(res));
+    }
+    return res;
+  }
+};
+
+bool wants_grad(const OptTensor& t) { return t && t->requires_grad(); }
+
+// (out, w0, w1, w2, m0, m1, m2), None where there is nothing to return
+py::tuple run_program(const c10::intrusive_ptr<Schedule>& sc, const Tensor& w0, const Tensor& w1, const Tensor& w2, const Tensor& q,
+                      const OptTensor& k, const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1, const OptTensor& lr2,
+                      const OptTensor& momentum, const OptTensor& m0, const OptTensor& m1, const OptTensor& m2) {
+  const bool needs_backward = at::GradMode::is_enabled() &&
+                              (w0.requires_grad() || w1.requires_grad() || w2.requires_grad() || q.requires_grad() || wants_grad(k) ||
+                               wants_grad(v) || wants_grad(lr0) || wants_grad(lr1) || wants_grad(lr2) || wants_grad(momentum));
+  std::vector<Tensor> m_state;
+  if (m0 && m1 && m2) m_state = {*m0, *m1, *m2};
+  if (needs_backward && !m_state.empty() && momentum && sc->has_update)
+    throw std::runtime_error("a carried momentum state is an inference feature: call under torch.no_grad()");
+  variable_list res;
+  {
+    const py::gil_scoped_release nogil;
+    if (needs_backward) {
+      res = ProgramFn::apply(sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum);
+    } else {
+      const at::AutoGradMode off(false);
+      res = forward(*sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m_state, false, nullptr);
+    }
+  }
+  py::tuple out(7);
+  for (size_t i = 0; i < 7; ++i) out[i] = i < res.size() ? py::cast(res[i]) : py::none();
+  return out;
+}
+
+}  // namespace
+
+PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
+  py::class_<Schedule, c10::intrusive_ptr<Schedule>>(m, "Schedule")
+      .def(py::init<const std::vector<std::vector<int>>&, int64_t, const std::optional<std::vector<float>>&, bool, bool, bool, bool, int, bool,
+                    bool, bool>());
+  m.def("run_program", &run_program);
+}

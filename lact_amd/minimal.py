@@ -2,6 +2,7 @@
 from __future__ import annotations
 
 import math
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -25,14 +26,17 @@ def block_causal_lact_swiglu(w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum: Optio
     return _block_causal(w0, w1, w2, q, k, v, lr0, lr1, lr2, chunk_size, use_muon, momentum, False)
 
 
+@lru_cache(maxsize=256)
+def _bidirectional_program(kv_len, q_len, use_muon, replaces, ns_mode):
+    return Program(steps=((LACT_UPDATE, 0, kv_len, 0), (LACT_APPLY, 0, q_len, 0)), out_len=q_len, return_state=False,
+                   ns_coeffs=NS5_COEFFS if use_muon else None, muon_replaces_weight=replaces, ns_mode=ns_mode)
+
+
 def bidirectional_lact_swiglu(w0, w1, w2, q, k, v, lr0, lr1, lr2, use_muon: bool = True,
                               muon_mode: str = "reference") -> torch.Tensor:
     """bidirectional_lact_layer.py:74-160: one update on every token, then apply to every query.
     muon_mode="reference" reproduces :139-146 (the orthogonalised gradient replaces the weight and the
     raw gradient is added); "intended" adds the orthogonalised gradient to the weight."""
-    prog = Program(steps=((LACT_UPDATE, 0, k.shape[1], 0), (LACT_APPLY, 0, q.shape[1], 0)), out_len=q.shape[1], return_state=False,
-                   ns_coeffs=NS5_COEFFS if use_muon else None,
-                   muon_replaces_weight=(use_muon and muon_mode == "reference"),
-                   ns_mode=ops._ns_mode(q))
+    prog = _bidirectional_program(k.shape[1], q.shape[1], bool(use_muon), bool(use_muon and muon_mode == "reference"), ops._ns_mode(q))
     out, _, _ = run_program(prog, w0, w1, w2, q, k, v, lr0, lr1, lr2, None)
     return out

@@ -2,6 +2,7 @@
 defaults; the arithmetic runs in liblact_hip.so."""
 from __future__ import annotations
 
+from functools import lru_cache
 from typing import Optional
 
 import torch
@@ -26,12 +27,16 @@ def zeropower_via_newtonschulz5(G: torch.Tensor) -> torch.Tensor:
     return ops.newton_schulz(G, NS5_COEFFS, ns_mode=ops.NS_AUTOCAST if torch.is_autocast_enabled() else ops.NS_PLAIN_BF16)
 
 
+@lru_cache(maxsize=256)
+def _block_causal_program(kv_len, q_len, chunk_size, use_muon, prenorm, ns_mode, muon_stacked, renorm_eps_in_sqrt):
+    return Program(steps=block_causal_steps(kv_len, chunk_size), out_len=q_len, return_state=False,
+                   ns_coeffs=NS5_COEFFS if use_muon else None, prenorm=prenorm, ns_mode=ns_mode,
+                   muon_stacked=muon_stacked and use_muon, renorm_eps_in_sqrt=renorm_eps_in_sqrt)
+
+
 def _block_causal(w0, w1, w2, q, k, v, lr0, lr1, lr2, chunk_size, use_muon, momentum, prenorm,
                   muon_stacked=False, renorm_eps_in_sqrt=False):
-    prog = Program(steps=block_causal_steps(k.shape[1], chunk_size), out_len=q.shape[1], return_state=False,
-                   ns_coeffs=NS5_COEFFS if use_muon else None, prenorm=prenorm,
-                   ns_mode=ops._ns_mode(q), muon_stacked=muon_stacked and use_muon,
-                   renorm_eps_in_sqrt=renorm_eps_in_sqrt)
+    prog = _block_causal_program(k.shape[1], q.shape[1], int(chunk_size), bool(use_muon), prenorm, ops._ns_mode(q), muon_stacked, renorm_eps_in_sqrt)
     out, _, _ = run_program(prog, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum)
     return out
 

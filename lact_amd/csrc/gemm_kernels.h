@@ -1,10 +1,11 @@
-// GEMM-shaped kernels of the TTT operation, all built on gemm_mainloop().
+// GEMM-shaped kernels of the TTT operation on the asynchronous pipeline of gemm_async.h: fp32, and the bf16 shapes that the
+// dedicated-loader kernels (gemm_dma_kernels.h) do not take.
 //
 // Row layout throughout: activations are [tokens, feature] with the feature dimension contiguous;
 // fast weights w0,w2 are [dh, d], w1 is [d, dh] (the reference's LLM layout,
 // lact_llm/lact_model/ttt_operation.py:71-105).
 #pragma once
-#include "gemm_core.h"
+#include "gemm_async.h"
 
 namespace lact {
 
@@ -57,18 +58,23 @@ __device__ __forceinline__ float dual_blend(float prod, float ax, int plain_bf16
   return plain_bf16 ? round_bf16(round_bf16(prod) + round_bf16(ax)) : __fadd_rn(ax, prod);
 }
 
-template <typename T, class TS, bool B_KC, int NT, int EPI>
-__global__ __launch_bounds__(TS::THREADS) void k_row_gemm(const RowGemmParams<NT> p) {
-  __shared__ __attribute__((aligned(16))) char smem[GemmSmem<T, TS>::BYTES];
+template <typename T, bool B_KC, int NT, int EPI>
+__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_row_gemm(const RowGemmParams<NT> p) {
+  using TS = typename AsyncTile<T>::TS;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   f32x16 acc[TS::TM][TS::TN];
   zero_acc<TS>(acc);
+  AsyncPipe<T, NT> pipe(smem);
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const T* A = reinterpret_cast<const T*>(p.t[t].A) + z * p.t[t].bsA + (size_t)m0 * p.t[t].lda;
     const T* B = reinterpret_cast<const T*>(p.t[t].B) + z * p.t[t].bsB + (B_KC ? (size_t)n0 * p.t[t].ldb : (size_t)n0);
-    gemm_mainloop<T, TS, true, B_KC>(acc, A, p.t[t].lda, p.M - m0, B, p.t[t].ldb, p.N - n0, p.t[t].K, smem);
+    pipe.phase(t, A, p.t[t].lda, p.M - m0, false, B, p.t[t].ldb, p.N - n0, !B_KC, p.t[t].K);
   }
+  pipe.start();
+#pragma unroll
+  for (int t = 0; t < NT; ++t) pipe.template accumulate<false, !B_KC>(t, acc);
   LACT_FOR_QUADS(TS) {
     const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
     if (m >= p.M || n >= p.N) continue;
@@ -139,9 +145,10 @@ struct HiddenParams {
 };
 
 // apply forward:  O0 = silu(X W0^T) * (X W2^T)                       (ttt_operation.py:141-143)
-template <typename T, class TS>
-__global__ __launch_bounds__(TS::THREADS) void k_apply_hidden(const HiddenParams p) {
-  __shared__ __attribute__((aligned(16))) char smem[GemmSmem<T, TS>::BYTES];
+template <typename T>
+__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_hidden(const HiddenParams p) {
+  using TS = typename AsyncTile<T>::TS;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
   const T* W0 = reinterpret_cast<const T*>(p.W0) + z * p.bsw + (size_t)n0 * p.d;
@@ -149,8 +156,12 @@ __global__ __launch_bounds__(TS::THREADS) void k_apply_hidden(const HiddenParams
   f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN];
   zero_acc<TS>(a0);
   zero_acc<TS>(a2);
-  gemm_mainloop<T, TS, true, true>(a0, X, p.ldx, p.T - m0, W0, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, true>(a2, X, p.ldx, p.T - m0, W2, p.d, p.dh - n0, p.d, smem);
+  AsyncPipe<T, 2> pipe(smem);
+  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
+  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
+  pipe.start();
+  pipe.template accumulate<false, false>(0, a0);
+  pipe.template accumulate<false, false>(1, a2);
   LACT_FOR_QUADS(TS) {
     const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
     if (m >= p.T || n >= p.dh) continue;
@@ -185,9 +196,10 @@ __device__ __forceinline__ UpdatePointwise update_pointwise(float g, float h2, f
 
 // update forward:  O0 = dgate_before_act, O1 = hidden * lr1, O2 = dhidden_before_mul
 // (ttt_operation.py:147-168: lr1 scales the hidden-side operand of dw1, lr0 and lr2 scale k -- see k_lr_scale_rows).
-template <typename T, class TS>
-__global__ __launch_bounds__(TS::THREADS) void k_update_hidden(const HiddenParams p) {
-  __shared__ __attribute__((aligned(16))) char smem[GemmSmem<T, TS>::BYTES];
+template <typename T>
+__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_hidden(const HiddenParams p) {
+  using TS = typename AsyncTile<T>::TS;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
   const T* Y = reinterpret_cast<const T*>(p.Y) + z * p.bsy + (size_t)m0 * p.ldy;
@@ -198,9 +210,14 @@ __global__ __launch_bounds__(TS::THREADS) void k_update_hidden(const HiddenParam
   zero_acc<TS>(a0);
   zero_acc<TS>(a2);
   zero_acc<TS>(a1);
-  gemm_mainloop<T, TS, true, true>(a0, X, p.ldx, p.T - m0, W0, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, true>(a2, X, p.ldx, p.T - m0, W2, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, false>(a1, Y, p.ldy, p.T - m0, W1, p.dh, p.dh - n0, p.d, smem);
+  AsyncPipe<T, 3> pipe(smem);
+  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
+  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
+  pipe.phase(2, Y, p.ldy, p.T - m0, false, W1, p.dh, p.dh - n0, true, p.d);
+  pipe.start();
+  pipe.template accumulate<false, false>(0, a0);
+  pipe.template accumulate<false, false>(1, a2);
+  pipe.template accumulate<false, true>(2, a1);
   LACT_FOR_QUADS(TS) {
     const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
     if (m >= p.T || n >= p.dh) continue;
@@ -253,9 +270,10 @@ __device__ __forceinline__ void store_row_partials(const HiddenParams& p, int wh
 
 // apply backward, hidden stage:  O0 = hidden (recomputed), O1 = d/d(X W0^T), O2 = d/d(X W2^T)
 // with Y = upstream gradient of the apply output  (lact_triton_kernels/lact_swiglu_ffn.py:57-65).
-template <typename T, class TS>
-__global__ __launch_bounds__(TS::THREADS) void k_apply_bwd_hidden(const HiddenParams p) {
-  __shared__ __attribute__((aligned(16))) char smem[GemmSmem<T, TS>::BYTES];
+template <typename T>
+__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_bwd_hidden(const HiddenParams p) {
+  using TS = typename AsyncTile<T>::TS;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
   const T* Y = reinterpret_cast<const T*>(p.Y) + z * p.bsy + (size_t)m0 * p.ldy;
@@ -266,9 +284,14 @@ __global__ __launch_bounds__(TS::THREADS) void k_apply_bwd_hidden(const HiddenPa
   zero_acc<TS>(a0);
   zero_acc<TS>(a2);
   zero_acc<TS>(a1);
-  gemm_mainloop<T, TS, true, true>(a0, X, p.ldx, p.T - m0, W0, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, true>(a2, X, p.ldx, p.T - m0, W2, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, false>(a1, Y, p.ldy, p.T - m0, W1, p.dh, p.dh - n0, p.d, smem);
+  AsyncPipe<T, 3> pipe(smem);
+  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
+  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
+  pipe.phase(2, Y, p.ldy, p.T - m0, false, W1, p.dh, p.dh - n0, true, p.d);
+  pipe.start();
+  pipe.template accumulate<false, false>(0, a0);
+  pipe.template accumulate<false, false>(1, a2);
+  pipe.template accumulate<false, true>(2, a1);
   LACT_FOR_QUADS(TS) {
     const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
     if (m >= p.T || n >= p.dh) continue;
@@ -296,9 +319,10 @@ __global__ __launch_bounds__(TS::THREADS) void k_apply_bwd_hidden(const HiddenPa
 //   O0 = d/d gate_before_act, O1 = d/d dhidden, O2 = d/d hidden_before_mul,
 //   O3 = dgate_before_act*lr0, O4 = hidden*lr1, O5 = dhidden_before_mul*lr2 (recomputed operands)
 // plus per-token partial sums of the lr gradients.
-template <typename T, class TS>
-__global__ __launch_bounds__(TS::THREADS) void k_update_bwd_hidden(const HiddenParams p) {
-  __shared__ __attribute__((aligned(16))) char smem[GemmSmem<T, TS>::BYTES];
+template <typename T>
+__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_bwd_hidden(const HiddenParams p) {
+  using TS = typename AsyncTile<T>::TS;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
   const T* Y = reinterpret_cast<const T*>(p.Y) + z * p.bsy + (size_t)m0 * p.ldy;
@@ -312,12 +336,20 @@ __global__ __launch_bounds__(TS::THREADS) void k_update_bwd_hidden(const HiddenP
   f32x16 b0[TS::TM][TS::TN], b2[TS::TM][TS::TN], b1[TS::TM][TS::TN];
   zero_acc<TS>(a0); zero_acc<TS>(a2); zero_acc<TS>(a1);
   zero_acc<TS>(b0); zero_acc<TS>(b2); zero_acc<TS>(b1);
-  gemm_mainloop<T, TS, true, true>(a0, X, p.ldx, p.T - m0, W0, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, true>(a2, X, p.ldx, p.T - m0, W2, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, true>(b0, X, p.ldx, p.T - m0, G0, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, true>(b2, X, p.ldx, p.T - m0, G2, p.d, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, false>(a1, Y, p.ldy, p.T - m0, W1, p.dh, p.dh - n0, p.d, smem);
-  gemm_mainloop<T, TS, true, false>(b1, Y, p.ldy, p.T - m0, G1, p.dh, p.dh - n0, p.d, smem);
+  AsyncPipe<T, 6> pipe(smem);
+  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
+  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
+  pipe.phase(2, X, p.ldx, p.T - m0, false, G0, p.d, p.dh - n0, false, p.d);
+  pipe.phase(3, X, p.ldx, p.T - m0, false, G2, p.d, p.dh - n0, false, p.d);
+  pipe.phase(4, Y, p.ldy, p.T - m0, false, W1, p.dh, p.dh - n0, true, p.d);
+  pipe.phase(5, Y, p.ldy, p.T - m0, false, G1, p.dh, p.dh - n0, true, p.d);
+  pipe.start();
+  pipe.template accumulate<false, false>(0, a0);
+  pipe.template accumulate<false, false>(1, a2);
+  pipe.template accumulate<false, false>(2, b0);
+  pipe.template accumulate<false, false>(3, b2);
+  pipe.template accumulate<false, true>(4, a1);
+  pipe.template accumulate<false, true>(5, b1);
 #pragma unroll
   for (int tm = 0; tm < TS::TM; ++tm) {
     const int m = m0 + quad_m<TS>(tm);
@@ -382,7 +414,7 @@ struct TokenReduceParams {
   TokenReduceJob job[3];
   int nb, tokens, split_len;   // split_len: tokens per split (multiple of 32)
   float* partial; long long mat_elems;
-  // single split only (asynchronous-copy kernel): out = coeff*add_in + result written here instead of a partial
+  // single split only: out = coeff*add_in + result written here instead of a partial
   float* add_out; const float* add_in; float coeff;
   // single split only, forward update: what k_momentum_prep would do with the result, done by the epilogue --
   // d_out = round_bf16(result) + m_prev * mbar[batch] (fp32 momentum state), its bf16 copy g16 in the same
@@ -393,9 +425,10 @@ struct TokenReduceParams {
   ClearWords prep_clear;   // barrier lines of the fused Newton-Schulz kernel that follows (cleared by the first block)
 };
 
-template <typename T, class TS>
-__global__ __launch_bounds__(TS::THREADS) void k_token_reduce(const TokenReduceParams p) {
-  __shared__ __attribute__((aligned(16))) char smem[GemmSmem<T, TS>::BYTES];
+template <typename T>
+__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_token_reduce(const TokenReduceParams p) {
+  using TS = typename AsyncTile<T>::TS;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
   const int j = blockIdx.z / p.nb, ib = blockIdx.z % p.nb;
   const TokenReduceJob& job = p.job[j];
   const int tiles_n = (job.N + TS::BN - 1) / TS::BN;
@@ -405,15 +438,28 @@ __global__ __launch_bounds__(TS::THREADS) void k_token_reduce(const TokenReduceP
   const int klen = min(p.split_len, p.tokens - k_begin);
   f32x16 acc[TS::TM][TS::TN];
   zero_acc<TS>(acc);
-  for (int t = 0; t < job.nterms; ++t) {
-    const T* A = reinterpret_cast<const T*>(job.t[t].A) + ib * job.t[t].bsA + (size_t)k_begin * job.t[t].lda + m0;
-    const T* B = reinterpret_cast<const T*>(job.t[t].B) + ib * job.t[t].bsB + (size_t)k_begin * job.t[t].ldb + n0;
-    gemm_mainloop<T, TS, false, false>(acc, A, job.t[t].lda, job.M - m0, B, job.t[t].ldb, job.N - n0, klen, smem);
+  AsyncPipe<T, 2> pipe(smem);
+#pragma unroll
+  for (int t = 0; t < 2; ++t) {
+    const TokenReduceTerm& tt = job.t[t < job.nterms ? t : 0];
+    const T* A = reinterpret_cast<const T*>(tt.A) + ib * tt.bsA + (size_t)k_begin * tt.lda + m0;
+    const T* B = reinterpret_cast<const T*>(tt.B) + ib * tt.bsB + (size_t)k_begin * tt.ldb + n0;
+    pipe.phase(t, A, tt.lda, job.M - m0, true, B, tt.ldb, job.N - n0, true, t < job.nterms ? klen : 0);
   }
-  float* out = p.partial + ((size_t)blockIdx.y * gridDim.z + blockIdx.z) * p.mat_elems;
+  pipe.start();
+  pipe.template accumulate<true, true>(0, acc);
+  pipe.template accumulate<true, true>(1, acc);
+  const size_t slot = (size_t)blockIdx.z * p.mat_elems;
+  float* out = p.add_out ? p.add_out + slot : p.partial + (size_t)blockIdx.y * gridDim.z * p.mat_elems + slot;
   LACT_FOR_QUADS(TS) {
     const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
     if (m >= job.M || n >= job.N) continue;
+    if (p.add_out && p.add_in) {
+      float in[4];
+      Elem<float>::load4(p.add_in + slot + (size_t)m * job.N + n, in);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[tm][tn][4 * g + j] += p.coeff * in[j];
+    }
     Elem<float>::store4(out + (size_t)m * job.N + n, acc[tm][tn][4 * g], acc[tm][tn][4 * g + 1], acc[tm][tn][4 * g + 2],
                         acc[tm][tn][4 * g + 3]);
   }

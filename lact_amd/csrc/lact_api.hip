@@ -187,8 +187,7 @@ SideCtx* side_ctx() {
   return &c;
 }
 
-using TSA = TileShape<128, 128, 2, 2>;  // two or three accumulators
-using TSB = TileShape<64, 128, 2, 2>;   // six accumulators (update backward)
+template <typename T> using TSG = typename AsyncTile<T>::TS;   // tile of the kernels in gemm_kernels.h
 
 struct Bump {
   size_t off = 0;
@@ -214,6 +213,20 @@ Split choose_split(int tokens, int tiles_total, int max_n) {
   ns = std::min(std::min(ns, std::max(1, max_n)), std::max(1, tokens / 1536));
   int len = ceil_div(ceil_div(tokens, ns), 64) * 64;
   return Split{ceil_div(tokens, len), len};
+}
+
+// The same for the kernel of gemm_kernels.h, whose tiles are small: two rounds of blocks at most, each over at least 128
+// tokens where the consumer adds the partial sums up anyway (the momentum step of a forward update), over 1024 where a
+// launch of its own has to (`own_launch`; 5 us against 0.014 us per token of a split saved).
+Split choose_split_async(int tokens, int tiles_total, int max_n, bool own_launch) {
+  int ns = std::max(1, 512 / std::max(1, tiles_total));
+  ns = std::min(std::min(ns, std::max(1, max_n)), std::max(1, tokens / (own_launch ? 1024 : 128)));
+  int len = ceil_div(ceil_div(tokens, ns), 64) * 64;
+  return Split{ceil_div(tokens, len), len};
+}
+template <typename T>
+int token_reduce_tiles(int d, int dh) {
+  return std::max(ceil_div(dh, TSG<T>::BM) * ceil_div(d, TSG<T>::BN), ceil_div(d, TSG<T>::BM) * ceil_div(dh, TSG<T>::BN));
 }
 
 // output tiles per matrix of the asynchronous-copy token reduction
@@ -347,11 +360,10 @@ struct Plan {
     }
     nblk = std::max(1, std::min(256, (int)((g.elems + 2047) / 2048)));
     lr_slots = ceil_div(d.dh, 128) * 4;   // (hidden tiles) x (wave columns) of the widest update-backward tiling
-    tiles = ceil_div(d.dh, TSA::BM) * ceil_div(d.d, TSA::BN);
-    tiles = std::max(tiles, ceil_div(d.d, TSA::BM) * ceil_div(d.dh, TSA::BN));
+    tiles = bf16 ? token_reduce_tiles<uint16_t>(d.d, d.dh) : token_reduce_tiles<float>(d.d, d.dh);
     // partial-sum slots: the larger split count of the two token-reduction kernels at the longest chunk (the
-    // count grows with the tokens) + the slot of a ragged tail
-    nsplit_max = std::max(choose_split(Tcap, tiles * 3 * d.b, 16).n, choose_split(Tcap, token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b, 16).n) + 1;
+    // count grows with the tokens)
+    nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, 16, false).n, choose_split(Tcap, token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b, 16).n);
 
     Bump sv;
     s_n0 = sv.take((size_t)3 * d.b * g.maxrows() * 4);
@@ -463,11 +475,14 @@ void launch_row_gemm(const char* site, const RowGemmParams<NT>& p, int batch, hi
       return;
     }
   }
-  dim3 grid(ceil_div(p.M, TSA::BM), ceil_div(p.N, TSA::BN), batch);
+  using TS = TSG<T>;
+  constexpr int SM = AsyncPipe<T, NT>::BYTES;
+  dim3 grid(ceil_div(p.M, TS::BM), ceil_div(p.N, TS::BN), batch);
   double ksum = 0;
   for (int t = 0; t < NT; ++t) ksum += p.t[t].K;
-  LACT_LAUNCH((row_gemm_name<T, B_KC, NT, EPI>()), site, 2.0 * p.M * p.N * ksum * batch,
-              (k_row_gemm<T, TSA, B_KC, NT, EPI>), grid, dim3(TSA::THREADS), s, p);
+  LACT_BIG_LDS((k_row_gemm<T, B_KC, NT, EPI>), SM);
+  LACT_LAUNCH_SMEM((row_gemm_name<T, B_KC, NT, EPI>()), site, 2.0 * p.M * p.N * ksum * batch,
+                   (k_row_gemm<T, B_KC, NT, EPI>), grid, dim3(TS::THREADS), SM, s, p);
 }
 
 template <int NT>
@@ -695,7 +710,7 @@ struct Runner {
   bool dma_hidden() const { return kBf16 && d.d % 64 == 0; }
   // row-partial slots the update-backward hidden kernel in use writes: (hidden tiles) x (wave columns)
   int lr_parts() const {
-    if (!dma_hidden()) return ceil_div(d.dh, TSB::BN) * TSB::WAVES_N;
+    if (!dma_hidden()) return ceil_div(d.dh, TSG<T>::BN) * TSG<T>::WAVES_N;
     if (P.keep_pre) return ceil_div(d.dh, TS_SQ::BN) * TS_SQ::WAVES_N;
     return ceil_div(d.dh, TS_BWD::BN) * TS_BWD::WAVES_N;
   }
@@ -736,11 +751,17 @@ struct Runner {
       if (which == 4) LACT_LAUNCH_SMEM("k_update_bwd_hidden_kept_dma", "update_bwd_hidden", 6.0 * f, (k_update_bwd_hidden_kept_dma<TS_SQ>), g3, dim3(DMA_THREADS), SM3, s, q);
       }
     } else {
-      dim3 ga(ceil_div(T_, TSA::BM), ceil_div(d.dh, TSA::BN), d.b), gb(ceil_div(T_, TSB::BM), ceil_div(d.dh, TSB::BN), d.b);
-      if (which == 0) LACT_LAUNCH("k_apply_hidden", "apply_hidden", 4.0 * f, (k_apply_hidden<T, TSA>), ga, dim3(TSA::THREADS), s, hp);
-      if (which == 1) LACT_LAUNCH("k_update_hidden", "update_hidden", 6.0 * f, (k_update_hidden<T, TSA>), ga, dim3(TSA::THREADS), s, hp);
-      if (which == 2) LACT_LAUNCH("k_apply_bwd_hidden", "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden<T, TSA>), ga, dim3(TSA::THREADS), s, hp);
-      if (which == 3) LACT_LAUNCH("k_update_bwd_hidden", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden<T, TSB>), gb, dim3(TSB::THREADS), s, hp);
+      using TS = TSG<T>;
+      constexpr int SM = AsyncPipe<T, 1>::BYTES;
+      const dim3 g(ceil_div(T_, TS::BM), ceil_div(d.dh, TS::BN), d.b);
+      LACT_BIG_LDS(k_apply_hidden<T>, SM);
+      LACT_BIG_LDS(k_update_hidden<T>, SM);
+      LACT_BIG_LDS(k_apply_bwd_hidden<T>, SM);
+      LACT_BIG_LDS(k_update_bwd_hidden<T>, SM);
+      if (which == 0) LACT_LAUNCH_SMEM("k_apply_hidden", "apply_hidden", 4.0 * f, (k_apply_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
+      if (which == 1) LACT_LAUNCH_SMEM("k_update_hidden", "update_hidden", 6.0 * f, (k_update_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
+      if (which == 2) LACT_LAUNCH_SMEM("k_apply_bwd_hidden", "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
+      if (which == 3) LACT_LAUNCH_SMEM("k_update_bwd_hidden", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
     }
   }
   template <typename U> U* scr(size_t off) const { return reinterpret_cast<U*>(sc + off); }
@@ -761,8 +782,8 @@ struct Runner {
 
   // The three token-reduction GEMMs of a step.  Returns the number of partial-sum slots written to the scratch
   // buffer (the caller reduces them), or 0 when the result went straight to `add_out` = coeff*add_in + sum.
-  // bf16, 64 tokens or more: the asynchronous-copy kernel (straight to add_out when one split covers them; a token
-  // count that is not a multiple of 64 ends inside the last K-step, whose surplus rows the loader clears).
+  // (Either kernel writes straight to add_out when one split covers the tokens.)  bf16, 64 tokens or more: the dedicated-loader
+  // kernel (a token count that is not a multiple of 64 ends inside the last K-step, whose surplus rows the loader clears).
   // `prep` (forward update only): d_out / g16 / ss_part / m_prev / mbar of the momentum step; when the whole
   // reduction is one split of the asynchronous-copy kernel, its epilogue does that step and -1 is returned.
   struct PrepFold {
@@ -786,23 +807,21 @@ struct Runner {
     for (int i = 0; i < 3; ++i) p.job[i] = jobs[i];
     p.nb = d.b; p.mat_elems = P.g.elems;
     float* partial = scr<float>(partial_sel);
-    const dim3 flat((unsigned)((P.mat3 / 4 + 255) / 256));
-    int main_tokens = 0, slots = 0;
+    int slots = 0;
     bool direct = false;
     if constexpr (kBf16) {
-      if (tokens >= 64 && d.d % 8 == 0 && d.dh % 8 == 0) main_tokens = tokens;   // a ragged end is handled inside the last K-step
-      if (main_tokens > 0) {
+      if (tokens >= 64) {     // a ragged end is handled inside the last K-step
         const bool big = d.d % TS_NS::BM == 0 && d.dh % TS_NS::BM == 0;
         const int tiles = token_reduce_dma_tiles(d.d, d.dh);
-        const Split sp = choose_split(main_tokens, tiles * 3 * d.b, P.nsplit_max - 1);
+        const Split sp = choose_split(tokens, tiles * 3 * d.b, P.nsplit_max);
         TokenReduceDmaParams pd;
         static_cast<TokenReduceParams&>(pd) = p;
-        pd.tokens = main_tokens; pd.split_len = sp.len; pd.partial = partial;
+        pd.tokens = tokens; pd.split_len = sp.len; pd.partial = partial;
         pd.map = make_tile_map(sp.n, tiles, 3 * d.b);
         dim3 g(pd.map.grid());
-        const double fl = 6.0 * main_tokens * d.d * d.dh * d.b * jobs[0].nterms;
+        const double fl = 6.0 * tokens * d.d * d.dh * d.b * jobs[0].nterms;
         direct = add_out && sp.n == 1;
-        const bool folded = prep && sp.n == 1 && main_tokens == tokens;
+        const bool folded = prep && sp.n == 1;
         if (folded) {
           pd.prep_d_out = prep->d_out; pd.prep_m_prev = prep->m_prev; pd.prep_mbar = prep->mbar; pd.prep_skip_d = prep->skip_d ? 1 : 0;
           pd.prep_g16 = prep->g16; pd.prep_ss_part = prep->ss_part; pd.prep_clear = prep->clear;
@@ -846,28 +865,20 @@ struct Runner {
           LACT_BIG_LDS(k_token_reduce_dma<TS_SQ>, SM);
           LACT_LAUNCH_SMEM("k_token_reduce_dma<128x128>", site, fl, (k_token_reduce_dma<TS_SQ>), g, dim3(DMA_THREADS), SM, s, pd);
         }
-        if (folded) return -1;
-        if (main_tokens == tokens) return slots;
+        return folded ? -1 : slots;
       }
     }
-    // generic kernel: fp32, or fewer than 64 tokens
-    const int rest = tokens - main_tokens;
-    for (int i = 0; i < 3; ++i)
-      for (int t = 0; t < p.job[i].nterms; ++t) {
-        TokenReduceTerm& tt = p.job[i].t[t];
-        tt.A = static_cast<const T*>(tt.A) + (size_t)main_tokens * tt.lda;
-        tt.B = static_cast<const T*>(tt.B) + (size_t)main_tokens * tt.ldb;
-      }
-    const Split sp = main_tokens > 0 ? Split{1, ceil_div(rest, 32) * 32} : choose_split(rest, P.tiles * 3 * d.b, P.nsplit_max - 1);
-    p.tokens = rest; p.split_len = sp.len;
-    p.partial = partial + (size_t)slots * P.mat3;
-    dim3 grid(P.tiles, sp.n, 3 * d.b);
-    LACT_LAUNCH("k_token_reduce", site, 6.0 * rest * d.d * d.dh * d.b * jobs[0].nterms, (k_token_reduce<T, TSA>), grid, dim3(TSA::THREADS), s, p);
-    if (direct) {   // add the tail to what the main part wrote
-      LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, add_out, add_out, 1.f, partial, sp.n, (long long)P.mat3);
-      return 0;
-    }
-    return slots + sp.n;
+    // fp32, or fewer than 64 tokens
+    using TS = TSG<T>;
+    constexpr int SM = AsyncPipe<T, 2>::BYTES;
+    const Split sp = choose_split_async(tokens, P.tiles * 3 * d.b, P.nsplit_max, add_out != nullptr);
+    direct = add_out && sp.n == 1;
+    if (direct) { p.add_out = add_out; p.add_in = coeff != 0.f ? add_in : nullptr; p.coeff = coeff; }
+    p.tokens = tokens; p.split_len = sp.len; p.partial = partial;
+    LACT_BIG_LDS(k_token_reduce<T>, SM);
+    LACT_LAUNCH_SMEM("k_token_reduce", site, 6.0 * tokens * d.d * d.dh * d.b * jobs[0].nterms, (k_token_reduce<T>), dim3(P.tiles, sp.n, 3 * d.b),
+                     dim3(TS::THREADS), SM, s, p);
+    return direct ? 0 : sp.n;
   }
 
   RenormParams renorm_params(int u, int ver_prev) const {
@@ -1553,7 +1564,7 @@ struct Runner {
       bool lone_reduction = false;
       if constexpr (kBf16)
         lone_reduction = token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b *
-                             choose_split(T_, token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b, P.nsplit_max - 1).n < 160;
+                             choose_split(T_, token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b, P.nsplit_max).n < 160;
       const bool use_tail = s_tail != s_main && u > 0 && !lone_reduction;
       if (use_tail) {
         wait_for(s_tail, s_main);

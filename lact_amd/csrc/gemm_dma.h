@@ -50,7 +50,7 @@ struct DmaOperand {
   int ld;
   int rows;              // valid rows from base on (may exceed the tile); multiple of 8 when ks
   int ks;
-  int ktail = 0;         // K-strided only: valid k rows of the last K-step when K is not a multiple of 64 (0: all 64)
+  int ktail = 0;         // TAILS pipelines, K-strided only: valid k rows of the last K-step when the phase's K, given rounded up, ends inside it (0: all 64)
 };
 
 // One phase: acc[j] += A * B_j^T over K, j < nb.
@@ -66,8 +66,8 @@ constexpr int DMA_BK = 64;
 
 // Loader-wave addressing of one operand tile: the loader copies the whole tile, 8 rows (1 KiB) per
 // instruction.  Rows past the operand are clamped to its last row: what they bring in only reaches output
-// rows/columns that are never stored.  K must be a multiple of 64 (the host routes other shapes to the
-// generic kernels).
+// rows/columns that are never stored.  K must be a multiple of 16 (the host routes other shapes to the
+// kernels of gemm_kernels.h): a K-step that K does not fill runs fewer of its four 16-wide sub-steps.
 // K-strided tiles are copied as they lie in memory, [64 k][ROWS] with the 16-byte granules of k-row k rotated
 // by 4*(k % 4) positions, and read back with ds_read_b64_tr_b16: inside each group of 16 lanes, lane i
 // receives element (i & 3) of the 8 bytes addressed by lanes 4j + (i >> 2), j = 0..3 -- i.e. a 4(k) x 16(r)
@@ -110,18 +110,27 @@ struct DmaLane {
 #pragma unroll
     for (int ii = 0; ii < N; ++ii) dma16<SC1>(b, voff[ii], lds_tile + ii * DMA_LOADERS * 1024);
   }
-  // The last K-step of a K-strided operand whose K ends inside it (op.ktail valid k rows): the k rows past the end
-  // are read from the last valid one instead -- never past the operand.  Offsets computed here, once per phase.
+  // A last K-step of which only `kvalid` k exist: the k past the end are read from the last valid ones instead -- never
+  // past the operand.  Offsets computed here, once per phase.
   template <bool SC1>
-  __device__ __forceinline__ void issue_tail(int kt, uint32_t lds_tile, const DmaOperand& op, int lw) const {
+  __device__ __forceinline__ void issue_short(int kt, uint32_t lds_tile, const DmaOperand& op, int lw, int kvalid) const {
     const int lane = threadIdx.x & 63;
     const uint16_t* b = base + kt * kstride;
 #pragma unroll
     for (int ii = 0; ii < N; ++ii) {
-      const int L = (lw + ii * DMA_LOADERS) * 64 + lane, k = min(L / G, op.ktail - 1), p = L % G;
-      int g = (p + G - (4 * ((L / G) & 3)) % G) % G;
-      g = min(g, op.rows / 8 - 1);
-      dma16<SC1>(b, (uint32_t)(((size_t)k * op.ld + g * 8) * 2), lds_tile + ii * DMA_LOADERS * 1024);
+      const int i = lw + ii * DMA_LOADERS;
+      uint32_t off;
+      if (op.ks) {
+        const int L = i * 64 + lane, k = min(L / G, kvalid - 1), p = L % G;
+        int g = (p + G - (4 * ((L / G) & 3)) % G) % G;
+        g = min(g, op.rows / 8 - 1);
+        off = (uint32_t)(((size_t)k * op.ld + g * 8) * 2);
+      } else {
+        const int row = i * 8 + (lane >> 3);
+        const int kv = min(((lane & 7) ^ ((row >> 1) & 7)) * 8, kvalid - 8);
+        off = (uint32_t)(((size_t)min(row, op.rows - 1) * op.ld + kv) * 2);
+      }
+      dma16<SC1>(b, off, lds_tile + ii * DMA_LOADERS * 1024);
     }
   }
   // The k rows past the end of K in the K-strided tile that has landed at `tile` (LDS; ktail valid k rows): cleared,
@@ -253,7 +262,7 @@ struct DmaPipe {
 
   __device__ __forceinline__ DmaPipe(char* s, const DmaPhase<NBMAX>* phases) : smem(s), ph(phases), total(0) {
 #pragma unroll
-    for (int i = 0; i < NPH; ++i) total += ph[i].K / DMA_BK;
+    for (int i = 0; i < NPH; ++i) total += (ph[i].K + DMA_BK - 1) / DMA_BK;
   }
   __device__ static __forceinline__ bool is_loader() { return __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4; }
 
@@ -269,7 +278,7 @@ struct DmaPipe {
     const int lw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - 4;
     DmaLane<TS::BM> la;
     DmaLane<TS::BN> lb[NBMAX];
-    int cp = -1, ckt = 0, cnk = 0, cnb = 0, issued = 0;
+    int cp = -1, ckt = 0, cnk = 0, cnb = 0, cshort = 0, issued = 0;
     auto next_phase = [&]() {
       ++cp;
       ckt = 0;
@@ -280,26 +289,22 @@ struct DmaPipe {
 #pragma unroll
           for (int j = 0; j < NBMAX; ++j) lb[j].init(ph[i].b[j], lw);
           cnb = ph[i].nb;
-          cnk = ph[i].K / DMA_BK;
+          cnk = (ph[i].K + DMA_BK - 1) / DMA_BK;
+          cshort = TAILS ? (ph[i].a.ks ? ph[i].a.ktail : 0) : SC1 ? 0 : ph[i].K % DMA_BK;
         }
     };
     auto issue_stage = [&]() {
       const uint32_t base = lds_addr(smem + (issued % STAGES) * SM::STAGE) + lw * 1024;
-      bool tail = false;
-      if constexpr (TAILS) {
-        if (ckt + 1 == cnk) {
+      if (cshort > 0 && ckt + 1 == cnk) {
 #pragma unroll
-          for (int i = 0; i < NPH; ++i)
-            if (i == cp && ph[i].a.ks && ph[i].a.ktail > 0) {
-              tail = true;
-              la.template issue_tail<SC1>(ckt, base, ph[i].a, lw);
+        for (int i = 0; i < NPH; ++i)
+          if (i == cp) {
+            la.template issue_short<SC1>(ckt, base, ph[i].a, lw, cshort);
 #pragma unroll
-              for (int j = 0; j < NBMAX; ++j)
-                if (j < cnb) lb[j].template issue_tail<SC1>(ckt, base + SM::A_BYTES + j * SM::B_BYTES, ph[i].b[j], lw);
-            }
-        }
-      }
-      if (!tail) {
+            for (int j = 0; j < NBMAX; ++j)
+              if (j < cnb) lb[j].template issue_short<SC1>(ckt, base + SM::A_BYTES + j * SM::B_BYTES, ph[i].b[j], lw, cshort);
+          }
+      } else {
         la.template issue<SC1>(ckt, base);
 #pragma unroll
         for (int j = 0; j < NBMAX; ++j)
@@ -320,7 +325,7 @@ struct DmaPipe {
     if constexpr (TAILS) {
 #pragma unroll
       for (int i = 0; i < NPH; ++i) {
-        acc_steps += ph[i].K / DMA_BK;
+        acc_steps += (ph[i].K + DMA_BK - 1) / DMA_BK;
         tail_rows[i] = (ph[i].a.ks && ph[i].K > 0) ? ph[i].a.ktail : 0;
         tail_step[i] = acc_steps - 1;
       }
@@ -338,9 +343,9 @@ struct DmaPipe {
     }
   }
 
-  // ---- MFMA waves: one phase, nk K-steps into acc[0..NB).  `step` counts K-steps over all phases.
+  // ---- MFMA waves: one phase over K into acc[0..NB).  `step` counts K-steps over all phases.
   template <int NB, bool A_KS = false, bool B_KS = false>
-  __device__ __forceinline__ void run_phase(int nk, int& step, f32x16 (&acc)[NB][TS::TM][TS::TN]) {
+  __device__ __forceinline__ void run_phase(int K, int& step, f32x16 (&acc)[NB][TS::TM][TS::TN]) {
     const int wave = threadIdx.x >> 6;
     FragSrc<TS::BM, A_KS> sa[TS::TM];
     FragSrc<TS::BN, B_KS> sb[TS::TN];
@@ -348,7 +353,9 @@ struct DmaPipe {
     for (int i = 0; i < TS::TM; ++i) sa[i].init((wave / TS::WAVES_N) * TS::WM + i * 32);
 #pragma unroll
     for (int n = 0; n < TS::TN; ++n) sb[n].init((wave % TS::WAVES_N) * TS::WN + n * 32);
-    if (nk <= 0) return;
+    // whole K-steps, and sub-steps of a last, partial one (the fused Newton-Schulz kernel's SC1 pipelines have none)
+    const int nk = K / DMA_BK, rest = SC1 || TAILS ? 0 : (K % DMA_BK) / 16;
+    if (K <= 0) return;
     // Rolling fragment pipeline: the fragments of sub-step s+1 are fetched before the MFMAs of sub-step s
     // issue, across K-steps too -- the barrier that opens stage kt+1 and the fetch of its first fragments
     // sit in front of the last MFMA group of stage kt, which hides the LDS latency.
@@ -390,13 +397,23 @@ struct DmaPipe {
       mfmas(0);
       interleave();
       ++step;
-      if (kt + 1 < nk) {
+      if (kt + 1 < nk || rest > 0) {
         __syncthreads();
         st = smem + (step % STAGES) * SM::STAGE;
         fetch(0, 0);
       }
       mfmas(1);
       interleave();
+    }
+    if (rest > 0) {
+      if (rest > 1) fetch(1, 1);
+      mfmas(0);
+      if (rest > 1) {
+        if (rest > 2) fetch(0, 2);
+        mfmas(1);
+        if (rest > 2) mfmas(0);
+      }
+      ++step;
     }
   }
 };

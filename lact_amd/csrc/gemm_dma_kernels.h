@@ -155,7 +155,7 @@ __device__ __forceinline__ void row_gemm_tile(const RowGemmDmaParams<NT>& pp, in
     zero_acc<TS>(acc[0]);
     int step = 0;
 #pragma unroll
-    for (int t = 0; t < NT; ++t) pipe.template run_phase<1, false, B_KS>(p.t[t].K / DMA_BK, step, acc);
+    for (int t = 0; t < NT; ++t) pipe.template run_phase<1, false, B_KS>(p.t[t].K, step, acc);
   }
   __syncthreads();
   LACT_TS(2);
@@ -282,7 +282,6 @@ __global__ __launch_bounds__(DMA_THREADS) void k_apply_hidden_dma(const HiddenDm
   ph[0].b[1] = weight_operand(p.W2, p.bsw, p.d, z, n0, p.dh);
   ph[0].nb = 2;
   ph[0].K = p.d;
-  const int nk = (p.d + DMA_BK - 1) / DMA_BK;
   f32x16 acc[2][TS::TM][TS::TN];
   LACT_TS(0);
   Pipe pipe(smem, ph);
@@ -294,7 +293,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_apply_hidden_dma(const HiddenDm
     zero_acc<TS>(acc[0]);
     zero_acc<TS>(acc[1]);
     int step = 0;
-    pipe.template run_phase<2>(nk, step, acc);
+    pipe.template run_phase<2>(p.d, step, acc);
   }
   __syncthreads();
   LACT_TS(2);
@@ -334,7 +333,6 @@ __device__ __forceinline__ void three_acc_mainloop(const HiddenDmaParams& pp, ch
   ph[1].b[1] = ph[1].b[0];
   ph[1].nb = 1;
   ph[1].K = p.d;
-  const int nk = (p.d + DMA_BK - 1) / DMA_BK;
   Pipe pipe(smem, ph);
   if (Pipe::is_loader()) {
     pipe.template load_all<Pipe::loads(1)>();
@@ -343,8 +341,8 @@ __device__ __forceinline__ void three_acc_mainloop(const HiddenDmaParams& pp, ch
     zero_acc<TS>(a02[1]);
     zero_acc<TS>(a1[0]);
     int step = 0;
-    pipe.template run_phase<2>(nk, step, a02);
-    pipe.template run_phase<1, false, true>(nk, step, a1);
+    pipe.template run_phase<2>(p.d, step, a02);
+    pipe.template run_phase<1, false, true>(p.d, step, a1);
   }
   __syncthreads();
 }
@@ -524,7 +522,6 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_dma(const Hid
   ph[2].b[1] = weight_operand_ks(p.G1, p.bsw, p.dh, z, n0, p.dh);
   ph[0].K = ph[1].K = ph[2].K = p.d;
   ph[0].nb = ph[1].nb = ph[2].nb = 2;
-  const int nk = (p.d + DMA_BK - 1) / DMA_BK;
   f32x16 aw[2][TS::TM][TS::TN], ag[2][TS::TM][TS::TN], ay[2][TS::TM][TS::TN];
   Pipe pipe(smem, ph);
   const bool loader = Pipe::is_loader();
@@ -533,9 +530,9 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_dma(const Hid
   } else {
     zero_acc<TS>(aw[0]); zero_acc<TS>(aw[1]); zero_acc<TS>(ag[0]); zero_acc<TS>(ag[1]); zero_acc<TS>(ay[0]); zero_acc<TS>(ay[1]);
     int step = 0;
-    pipe.template run_phase<2>(nk, step, aw);
-    pipe.template run_phase<2>(nk, step, ag);
-    pipe.template run_phase<2, false, true>(nk, step, ay);
+    pipe.template run_phase<2>(p.d, step, aw);
+    pipe.template run_phase<2>(p.d, step, ag);
+    pipe.template run_phase<2, false, true>(p.d, step, ay);
   }
   __syncthreads();
   // Epilogue: the six rounded products staged as bf16 tiles, then the pointwise part on all eight waves, row-wise (a
@@ -664,8 +661,8 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
     zero_acc<TS>(ag[1]);
     zero_acc<TS>(ay[0]);
     int step = 0;
-    pipe.template run_phase<1, false, true>(nk, step, ay);
-    pipe.template run_phase<2>(nk, step, ag);
+    pipe.template run_phase<1, false, true>(p.d, step, ay);
+    pipe.template run_phase<2>(p.d, step, ag);
     LACT_TS(1);
     for (int i = 0; i < halves; ++i) __syncthreads();   // the input stages land behind these barriers
   }
@@ -808,8 +805,8 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
   } else {
     zero_acc<TS>(acc[0]);
     int step = 0;
-    pipe.template run_phase<1, true, true>(ph[0].K / DMA_BK, step, acc);
-    pipe.template run_phase<1, true, true>(ph[1].K / DMA_BK, step, acc);
+    pipe.template run_phase<1, true, true>(ph[0].K, step, acc);
+    pipe.template run_phase<1, true, true>(ph[1].K, step, acc);
   }
   __syncthreads();
   using ST = StageTile<TS, 4>;

@@ -237,7 +237,7 @@ struct ApplyHiddenPolicy {
   }
   template <class Pipe>
   __device__ static __forceinline__ void mma(Pipe& pipe, const HiddenParams& p, int& step, f32x16 (&a02)[2][2][2], f32x16 (&)[1][2][2]) {
-    pipe.template run_phase<2>(p.d / DMA_BK, step, a02);
+    pipe.template run_phase<2>(p.d, step, a02);
   }
   __device__ static __forceinline__ void epilogue(const HiddenParams& p, const FragPlace& f, const f32x16 (&a02)[2][2][2], const f32x16 (&)[1][2][2]) {
     // all four fragments of the wave staged, then stored
@@ -281,8 +281,8 @@ struct ApplyBwdHiddenPolicy {
   }
   template <class Pipe>
   __device__ static __forceinline__ void mma(Pipe& pipe, const HiddenParams& p, int& step, f32x16 (&a02)[2][2][2], f32x16 (&a1)[1][2][2]) {
-    pipe.template run_phase<2>(p.d / DMA_BK, step, a02);
-    pipe.template run_phase<1, false, true>(p.d / DMA_BK, step, a1);
+    pipe.template run_phase<2>(p.d, step, a02);
+    pipe.template run_phase<1, false, true>(p.d, step, a1);
   }
   __device__ static __forceinline__ void epilogue(const HiddenParams& p, const FragPlace& f, const f32x16 (&a02)[2][2][2], const f32x16 (&a1)[1][2][2]) {
     void* const o[3] = {p.O0, p.O1, p.O2};

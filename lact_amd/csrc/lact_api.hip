@@ -450,12 +450,12 @@ void launch_row_gemm_dma(const char* site, const RowGemmDmaParams<NT>& q, int ba
   LACT_LAUNCH_SMEM(name.c_str(), site, 2.0 * q.g.M * q.g.N * ksum * batch, (k_row_gemm_dma<TS, NT, EPI, B_KS>), dim3(qq.map.grid()),
                    dim3(DMA_THREADS), SMEM, s, qq);
 }
-// bf16 with every K a multiple of 64: asynchronous-copy kernels; anything else: the generic tile loop
+// bf16 with every K a multiple of 16: dedicated-loader kernels; anything else: the small-tile pipeline
 template <typename T, bool B_KC, int NT, int EPI>
 void launch_row_gemm(const char* site, const RowGemmParams<NT>& p, int batch, hipStream_t s, bool token_rows = false) {
   if constexpr (std::is_same<T, uint16_t>::value) {
     bool ok = p.N % 8 == 0;
-    for (int t = 0; t < NT; ++t) ok = ok && p.t[t].K % 64 == 0;
+    for (int t = 0; t < NT; ++t) ok = ok && p.t[t].K % 16 == 0;
     if (ok) {
       RowGemmDmaParams<NT> q;
       q.g = p;
@@ -559,7 +559,7 @@ struct Runner {
   }
   // ---- fused Newton-Schulz: launches of at most 256 resident blocks
   static bool tiles_fit(int r, int c, int bm, int bn) {
-    return r % bm == 0 && r % bn == 0 && c % bn == 0 && (r / bm) * (c / bn) <= 32;
+    return r % bm == 0 && r % bn == 0 && c % bn == 0 && r % 64 == 0 && c % 64 == 0 && (r / bm) * (c / bn) <= 32;   // whole K-steps
   }
   // Tile of the fused kernel for a batch: 0 = 192 x 192, 1 = 128 x 128, 2 = 128 x 64, 3 = 128 x 96, -1 = none fits.
   // 192 x 192 when the matrices fill at least half the chip with it, else 128 x 128 (more, smaller blocks), and
@@ -706,8 +706,8 @@ struct Runner {
   static constexpr bool kBf16 = std::is_same<T, uint16_t>::value;
   static constexpr bool kNsBf16 = std::is_same<TN, uint16_t>::value;
 
-  // the hidden-stage kernels with asynchronous copies need bf16 and whole 64-element K-steps
-  bool dma_hidden() const { return kBf16 && d.d % 64 == 0; }
+  // the hidden-stage kernels of the dedicated-loader engine need bf16 and whole 16-element sub-steps
+  bool dma_hidden() const { return kBf16 && d.d % 16 == 0; }
   // row-partial slots the update-backward hidden kernel in use writes: (hidden tiles) x (wave columns)
   int lr_parts() const {
     if (!dma_hidden()) return ceil_div(d.dh, TSG<T>::BN) * TSG<T>::WAVES_N;
@@ -732,7 +732,7 @@ struct Runner {
       LACT_BIG_LDS(k_apply_bwd_hidden_dma<TS_SQ>, SM3);
       LACT_BIG_LDS(k_update_bwd_hidden_dma<TS_BWD>, SM6);
       LACT_BIG_LDS(k_update_bwd_hidden_kept_dma<TS_SQ>, SM3);
-      if (which <= 2 && ((g_persist >> which) & 1) && side && side->cus > 0) {
+      if (which <= 2 && d.d % 64 == 0 && ((g_persist >> which) & 1) && side && side->cus > 0) {
         HiddenPersistParams hq;
         hq.h = hp; hq.map = m3;
         const dim3 gp(persist_grid(m3.grid(), side->cus));
@@ -830,8 +830,8 @@ struct Runner {
         else slots = sp.n;
         bool with_rows = rows != nullptr && rows->r4.N % 8 == 0 && rows->r2.N % 8 == 0;
         if (with_rows) {
-          for (int t = 0; t < 4; ++t) with_rows = with_rows && rows->r4.t[t].K % 64 == 0;
-          for (int t = 0; t < 2; ++t) with_rows = with_rows && rows->r2.t[t].K % 64 == 0;
+          for (int t = 0; t < 4; ++t) with_rows = with_rows && rows->r4.t[t].K % 16 == 0;
+          for (int t = 0; t < 2; ++t) with_rows = with_rows && rows->r2.t[t].K % 16 == 0;
         }
         if (with_rows) {
           TokenReduceRowsParams q;

@@ -31,3 +31,9 @@ def test_small_tiles_against_oracle(dtype, b, L, d, dh, C):
         if float(r.double().norm()) > 0:
             # one dot product per head and chunk: held to a looser bound in bf16, as everywhere
             assert O.rel_l2(a, r) < (tol if n != "momentum" or dtype == torch.float32 else 3e-2), n
+
+
+@pytest.mark.parametrize("b,L,d,dh,C", [(2, 300, 96, 96, 130), (1, 200, 16, 48, 100), (2, 290, 80, 112, 129), (3, 260, 160, 224, 128)])
+def test_partial_k_steps_against_oracle(b, L, d, dh, C):
+    """bf16 head sizes that end inside a K-step of the dedicated-loader kernels (one, two or three of its four sub-steps)."""
+    test_small_tiles_against_oracle(torch.bfloat16, b, L, d, dh, C)

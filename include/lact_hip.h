@@ -73,6 +73,9 @@ typedef struct lact_desc {
   /* The first update starts from a momentum state carried in by the caller (lact_forward_from_state) instead of
    * zero: ar_lact_swa_repeat_sp.py:215-217,266-269,309-317.  Needs use_momentum and forward_only. */
   int32_t momentum_state_in;
+  /* The w0, w1, w2 handed to lact_forward lie transposed in memory: w0, w2 [b, d, dh], w1 [b, dh, d] (lact_ttt.py:89-94).
+   * w_out, and every gradient of lact_backward, keep the layout of the header's first lines. */
+  int32_t w_transposed;
 } lact_desc_t;
 
 const char* lact_last_error(void);

@@ -905,7 +905,7 @@ struct Runner {
     const dim3 rowgrid(ceil_div(P.g.maxrows(), 4), 3 * d.b);
     // what depends on the inputs only may start on the tail stream right here, beside the first kernels of the call
     hipEvent_t entry = nullptr;
-    if (s_tail != s_main && side) {
+    if (s_tail != s_main && side && P.nupd > 0) {
       entry = side->event();
       (void)hipEventRecord(entry, s_main);
     }
@@ -917,9 +917,15 @@ struct Runner {
           return fail("copy of the carried momentum state failed");
     {
       InitParams p;
-      p.g = P.g; p.w[0] = w0; p.w[1] = w1; p.w[2] = w2; p.n0 = n0(); p.wf = wf(0);
+      memset(&p, 0, sizeof(p));
+      p.g = P.g; p.w[0] = w0; p.w[1] = w1; p.w[2] = w2; p.n0 = n0();
+      // a call without updates hands the weights back as they are; with bf16 activations nothing else reads the fp32 copy then
+      p.wf = (P.bf16 && P.nupd == 0 && d.forward_only) ? nullptr : wf(0);
       p.wc = P.bf16 ? (void*)wc(0) : nullptr;
-      LACT_LAUNCH("k_init_state", "k_init_state", 0.0, (k_init_state<T>), rowgrid, dim3(256), s, p);
+      if (P.nupd == 0 && w_out)
+        for (int j = 0; j < 3; ++j) p.w_ext[j] = w_out[j];
+      if (d.w_transposed) LACT_LAUNCH("k_init_state", "k_init_state", 0.0, (k_init_state_transposed<T>), dim3(ceil_div(P.g.maxrows(), 32), 3 * d.b), dim3(256), s, p);
+      else LACT_LAUNCH("k_init_state", "k_init_state", 0.0, (k_init_state<T>), rowgrid, dim3(256), s, p);
     }
     // mean of the momentum over the chunk of every update that weighs an earlier state (the first update of a
     // program has none unless the caller carried one in): they depend on the input only -- one launch up front
@@ -1130,10 +1136,7 @@ struct Runner {
     }
     flush_applies(false);
     if (side_used) wait_for(s_main, s_side);
-    // final weights and momentum state: written by the last update's kernels; copied only when no update ran
-    const dim3 eg((unsigned)((P.g.elems / 4 + 255) / 256), 3 * d.b);
-    if (u == 0 && w_out && (w_out[0] || w_out[1] || w_out[2]))
-      LACT_LAUNCH("k_unpack3", "k_unpack3", 0.0, k_unpack3, eg, dim3(256), s, wf(ver), P.g.elems, d.b, w_out[0], w_out[1], w_out[2]);
+    // final weights and momentum state: written by the last update's kernels, or by the first kernel when no update runs
     if (m_out && (m_out[0] || m_out[1] || m_out[2])) {
       if (u > 0 && P.momentum) {
       } else

@@ -71,28 +71,75 @@ struct FlatRange {
 // ---- init: row norms of the initial weights, fp32 state copy, compute-type copy -----------------
 struct InitParams {
   MatGeom g;
-  const float* w[3];      // [b, rows, cols] each
+  const float* w[3];      // [b, rows, cols] each; transposed: [b, cols, rows]
   float* n0;              // [3b][maxrows]
-  float* wf;              // [3b][elems]
+  float* wf;              // [3b][elems], or null when no update reads it
   void* wc;               // [3b][elems] compute type, or null when the compute type is fp32
+  float* w_ext[3];        // caller's weight outputs [b, rows, cols] when no update follows, each nullable
 };
+template <typename T>
+__device__ __forceinline__ void init_store(const InitParams& p, float* ext, size_t o, size_t in_batch, const float4& v) {
+  if (p.wf) st4(p.wf + o, v);
+  if (ext) st4(ext + in_batch, v);
+  if (p.wc) Elem<T>::store4(reinterpret_cast<T*>(p.wc) + o, v.x, v.y, v.z, v.w);
+}
 template <typename T>
 __global__ void k_init_state(const InitParams p) {
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= p.g.rows(j)) return;
   const int cols = p.g.cols(j);
-  const float* src = p.w[j] + (size_t)ib * p.g.elems + (size_t)row * cols;
+  const size_t in_batch = (size_t)ib * p.g.elems + (size_t)row * cols;
+  const float* src = p.w[j] + in_batch;
   const size_t o = (size_t)z * p.g.elems + (size_t)row * cols;
   float ss = 0.f;
   for (int c = lane * 4; c < cols; c += 256) {
     const float4 v = ld4(src + c);
     ss += dot4(v, v);
-    st4(p.wf + o + c, v);
-    if (p.wc) Elem<T>::store4(reinterpret_cast<T*>(p.wc) + o + c, v.x, v.y, v.z, v.w);
+    init_store<T>(p, p.w_ext[j], o + c, in_batch + c, v);
   }
   ss = wave_sum(ss);
   if (lane == 0) p.n0[(size_t)z * p.g.maxrows() + row] = sqrtf(ss);
+}
+// The same from weights that lie transposed in memory (the view-synthesis model's layout, lact_ttt.py:89-94): 64 columns of 32
+// rows at a time through LDS, so that no transposed copy has to be made first (three copies of 5 us in front of a 4 us kernel
+// at 18 matrices of 128 x 256).  Grid (ceil(max rows / 32), 3b), 256 threads.
+template <typename T>
+__global__ __launch_bounds__(256) void k_init_state_transposed(const InitParams p) {
+  __shared__ float tile[64][33];
+  const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb, row0 = blockIdx.x * 32;
+  const int rows = p.g.rows(j), cols = p.g.cols(j);
+  if (row0 >= rows) return;
+  const float* src = p.w[j] + (size_t)ib * p.g.elems;
+  const int lc = threadIdx.x >> 3, lr = (threadIdx.x & 7) * 4;          // load: column lc (+ 32), four rows from lr
+  const int sr = threadIdx.x >> 4, scol = (threadIdx.x & 15) * 4;       // store: row sr (+ 16), four columns from scol
+  float ss[2] = {0.f, 0.f};
+  for (int c0 = 0; c0 < cols; c0 += 64) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int c = lc + 32 * i;
+      const float4 v = (c0 + c < cols && row0 + lr < rows) ? ld4(src + (size_t)(c0 + c) * rows + row0 + lr) : f4(0.f, 0.f, 0.f, 0.f);
+      tile[c][lr] = v.x; tile[c][lr + 1] = v.y; tile[c][lr + 2] = v.z; tile[c][lr + 3] = v.w;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int r = sr + 16 * i;
+      if (row0 + r < rows && c0 + scol < cols) {
+        const float4 v = f4(tile[scol][r], tile[scol + 1][r], tile[scol + 2][r], tile[scol + 3][r]);
+        ss[i] += dot4(v, v);
+        const size_t e = (size_t)(row0 + r) * cols + c0 + scol;
+        init_store<T>(p, p.w_ext[j], (size_t)z * p.g.elems + e, (size_t)ib * p.g.elems + e, v);
+      }
+    }
+    __syncthreads();
+  }
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+#pragma unroll
+    for (int d = 1; d < 16; d <<= 1) ss[i] += __shfl_xor(ss[i], d, 64);
+    if ((threadIdx.x & 15) == 0 && row0 + sr + 16 * i < rows) p.n0[(size_t)z * p.g.maxrows() + row0 + sr + 16 * i] = sqrtf(ss[i]);
+  }
 }
 
 // ---- mean of the per-token momentum over one chunk (ttt_operation.py:171-172) --------------------
@@ -617,14 +664,7 @@ __global__ void k_finish_weight_grads(const FinishParams p) {
   st4(p.out[j] + (size_t)ib * p.g.elems + e, v);
 }
 
-// [3b][elems] <-> the three caller tensors, 4 elements per thread
-__global__ void k_unpack3(const float* src, long long elems, int nb, float* o0, float* o1, float* o2) {
-  const long long e = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  const int z = blockIdx.y;
-  if (e >= elems) return;
-  float* dst = (z / nb) == 0 ? o0 : ((z / nb) == 1 ? o1 : o2);
-  if (dst) st4(dst + (size_t)(z % nb) * elems + e, ld4(src + (size_t)z * elems + e));
-}
+// the three caller tensors (null: zeros) -> [3b][elems], 4 elements per thread
 __global__ void k_pack3(float* dst, long long elems, int nb, const float* i0, const float* i1, const float* i2) {
   const long long e = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   const int z = blockIdx.y;

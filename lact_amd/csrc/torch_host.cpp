@@ -138,12 +138,19 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
     o.lr2 = per_token(*lr2, b, L, "lr");
     if (momentum) o.momentum = per_token(*momentum, b, L, "momentum");
   }
-  const Tensor w[3] = {plain_f32(w0), plain_f32(w1), plain_f32(w2)};
+  // weights that are transposed views of contiguous fp32 tensors (the view-synthesis model's layout) are read as they lie
+  auto lies_transposed = [](const Tensor& t) {
+    return t.scalar_type() == at::kFloat && t.stride(1) == 1 && t.stride(2) == t.size(1) && t.stride(0) == t.size(1) * t.size(2) && t.size(2) > 1 &&
+           reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+  };
+  const bool transposed = lies_transposed(w0) && lies_transposed(w1) && lies_transposed(w2);
+  const Tensor w[3] = {transposed ? w0 : plain_f32(w0), transposed ? w1 : plain_f32(w1), transposed ? w2 : plain_f32(w2)};
   const auto act_opt = o.q.options();
   Tensor out = sc.covers ? at::empty({b, sc.out_len, d}, act_opt) : at::zeros({b, sc.out_len, d}, act_opt);
   lact_desc_t D = describe(sc, b, d, dh, o.q, o.k, o.v, out);
   D.use_momentum = o.momentum.defined();
   D.forward_only = !needs_backward;
+  D.w_transposed = transposed;
   Tensor m_in[3];
   const bool carried = !m_state.empty() && o.momentum.defined();
   if (carried) {
@@ -163,9 +170,8 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
   float* w_out[3] = {nullptr, nullptr, nullptr};
   float* m_out[3] = {nullptr, nullptr, nullptr};
   if (sc.return_state) {
-    for (int i = 0; i < 3; ++i) res.push_back(at::empty_like(w[i]));
-    if (o.momentum.defined())
-      for (int i = 0; i < 3; ++i) res.push_back(at::empty_like(w[i]));
+    const int sets = o.momentum.defined() ? 2 : 1;
+    for (int i = 0; i < 3 * sets; ++i) res.push_back(at::empty(w[i % 3].sizes(), w[i % 3].options()));
     for (int i = 0; i < 3; ++i) w_out[i] = fptr(res[1 + i]);
     if (o.momentum.defined())
       for (int i = 0; i < 3; ++i) m_out[i] = fptr(res[4 + i]);

@@ -37,3 +37,25 @@ def test_small_tiles_against_oracle(dtype, b, L, d, dh, C):
 def test_partial_k_steps_against_oracle(b, L, d, dh, C):
     """bf16 head sizes that end inside a K-step of the dedicated-loader kernels (one, two or three of its four sub-steps)."""
     test_small_tiles_against_oracle(torch.bfloat16, b, L, d, dh, C)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("d,dh", [(128, 256), (72, 40), (8, 72)])
+def test_transposed_weights_are_read_as_they_lie(dtype, d, dh):
+    """Fast weights given as transposed views (read in place) against contiguous ones: the row norms are summed in another
+    order, everything else is the same arithmetic.  With and without an update; the returned weights of the latter are exact."""
+    print("[gpu-test] transposed weights", dtype, d, dh, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    b, L = 3, 90
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(b, L, d, dh, seed=32, act_dtype=dtype).items()}
+    plain = [inp[n] for n in ORDER[:9]]
+    views = [w.transpose(1, 2).contiguous().transpose(1, 2) for w in plain[:3]] + plain[3:]
+    for steps in (((LACT_APPLY, 0, L, 0),), ((LACT_UPDATE, 0, L, 0), (LACT_APPLY, 0, L, 0))):
+        prog = ops.Program(steps=steps, out_len=L)
+        (out_p, w_p, _), (out_v, w_v, _) = ops.run_program(prog, *plain), ops.run_program(prog, *views)
+        assert O.rel_l2(out_v, out_p) < (2e-6 if dtype == torch.float32 else 1e-3)
+        for a, r, w in zip(w_v, w_p, plain[:3]):
+            assert O.rel_l2(a, r) < 1e-6
+            if len(steps) == 1:
+                assert torch.equal(a, w) and torch.equal(r, w)

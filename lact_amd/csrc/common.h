@@ -22,6 +22,15 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
 }
 // round a float to the nearest bf16-representable float
 __device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
+// Two values at once: one v_cvt_pk_bf16_f32 (lo in the lower half) where separate conversions take three instructions to pack.
+// The GEMM epilogues are bound by vector-ALU issue.
+__device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
+}
+__device__ __forceinline__ float bf16_lo(uint32_t u) { return __uint_as_float(u << 16); }
+__device__ __forceinline__ float bf16_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 
 // Element-type policies: T = uint16_t (bf16 storage) or float.
 template <typename T> struct Elem;
@@ -32,8 +41,8 @@ template <> struct Elem<uint16_t> {
   __device__ static __forceinline__ float rnd(float v) { return round_bf16(v); }
   __device__ static __forceinline__ void store4(uint16_t* p, float a, float b, float c, float d) {
     uint2 u;
-    u.x = (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16);
-    u.y = (uint32_t)f32_to_bf16(c) | ((uint32_t)f32_to_bf16(d) << 16);
+    u.x = pack_bf16(a, b);
+    u.y = pack_bf16(c, d);
     *reinterpret_cast<uint2*>(p) = u;
   }
   __device__ static __forceinline__ void load4(const uint16_t* p, float* o) {

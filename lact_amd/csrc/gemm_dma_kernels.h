@@ -85,7 +85,7 @@ __device__ __forceinline__ void row_gemm_copy_out_b16(const RowGemmParams<NT>& p
           for (int j = 0; j < 4; ++j) {
             const float lo = round_bf16(al * __uint_as_float(uu[j] << 16)) + round_bf16(be * __uint_as_float(ww[j] << 16));
             const float hi = round_bf16(al * __uint_as_float(uu[j] & 0xffff0000u)) + round_bf16(be * __uint_as_float(ww[j] & 0xffff0000u));
-            uu[j] = (uint32_t)f32_to_bf16(lo) | ((uint32_t)f32_to_bf16(hi) << 16);
+            uu[j] = pack_bf16(lo, hi);
           }
           u = make_uint4(uu[0], uu[1], uu[2], uu[3]);
         }
@@ -94,8 +94,7 @@ __device__ __forceinline__ void row_gemm_copy_out_b16(const RowGemmParams<NT>& p
           uint32_t uu[4] = {u.x, u.y, u.z, u.w};
 #pragma unroll
           for (int j = 0; j < 4; ++j)
-            uu[j] = (uint32_t)f32_to_bf16(p.alpha2 * __uint_as_float(uu[j] << 16)) |
-                    ((uint32_t)f32_to_bf16(p.alpha2 * __uint_as_float(uu[j] & 0xffff0000u)) << 16);
+            uu[j] = pack_bf16(p.alpha2 * bf16_lo(uu[j]), p.alpha2 * bf16_hi(uu[j]));
           *reinterpret_cast<uint4*>(dst2) = make_uint4(uu[0], uu[1], uu[2], uu[3]);
         }
       }
@@ -359,7 +358,7 @@ __device__ __forceinline__ void unpack8(const uint4& u, float (&f)[8]) {
 __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   uint32_t w[4];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) w[i] = (uint32_t)f32_to_bf16(f[2 * i]) | ((uint32_t)f32_to_bf16(f[2 * i + 1]) << 16);
+  for (int i = 0; i < 4; ++i) w[i] = pack_bf16(f[2 * i], f[2 * i + 1]);
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 

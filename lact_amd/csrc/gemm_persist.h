@@ -90,7 +90,7 @@ __device__ __forceinline__ void frag_put(char* frag, int g, uint32_t lo, uint32_
   *reinterpret_cast<uint2*>(frag + m * 64 + ((g ^ ((m >> 2) & 3)) << 4) + h * 8) = make_uint2(lo, hi);
 }
 __device__ __forceinline__ void frag_put4(char* frag, int g, float a, float b, float c, float d) {
-  frag_put(frag, g, (uint32_t)f32_to_bf16(a) | ((uint32_t)f32_to_bf16(b) << 16), (uint32_t)f32_to_bf16(c) | ((uint32_t)f32_to_bf16(d) << 16));
+  frag_put(frag, g, pack_bf16(a, b), pack_bf16(c, d));
 }
 // the fragment back, row-wise: lane l holds columns [8 (l & 3), + 8) of rows (l >> 2) and (l >> 2) + 16
 __device__ __forceinline__ void frag_read(const char* frag, uint4 (&v)[2]) {

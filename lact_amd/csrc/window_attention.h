@@ -125,10 +125,10 @@ __device__ __forceinline__ void attn_own_rows(bf16x8 (&f)[D / 16], const uint16_
 }
 
 __device__ __forceinline__ bf16x8 attn_pack(const f32x16& s, int st) {
-  bf16x8 r;
+  uint32_t r[4];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) r[i] = (__bf16)s[8 * st + i];
-  return r;
+  for (int i = 0; i < 4; ++i) r[i] = pack_bf16(s[8 * st + 2 * i], s[8 * st + 2 * i + 1]);
+  return __builtin_bit_cast(bf16x8, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
 // A wave's [D][32] accumulator (rows = D, columns = its own rows), times `f`, to 32 rows of a contiguous [B, L, H, D]

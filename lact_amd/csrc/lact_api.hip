@@ -16,6 +16,7 @@
 
 #include "gemm_dma_kernels.h"
 #include "ns_fused.h"
+#include "ns_local.h"
 #include "gemm_persist.h"
 #include "gemm_kernels.h"
 #include "state_kernels.h"
@@ -615,7 +616,43 @@ struct Runner {
       default: break;
     }
   }
-  // every batch runs fused (and at least one iteration): the Frobenius normalisation is the fused kernel's first stage
+  // Forward only: matrices that fit a compute unit whole (X in LDS: at most 128 x 256) run on one block each.
+  bool ns_local_ok(const NsBatch& B) const {
+    return g_fused_ns && kNsBf16 && P.S >= 1 && P.S <= NS_FUSED_MAX_STEPS && B.r % 32 == 0 && B.c % 32 == 0 && B.r <= 128 && B.c <= 256;
+  }
+  template <int RT, int XG>
+  void launch_ns_local_t(const NsLocalParams& p, const NsBatch& B) {
+    constexpr int SM = ns_local_lds<RT, XG>();
+    const double flops = 2.0 * B.r * B.r * (2.0 * B.c + B.r) * P.S * B.n;
+    LACT_BIG_LDS((k_ns_local<RT, XG, false>), SM);
+    LACT_BIG_LDS((k_ns_local<RT, XG, true>), SM);
+    if (d.ns_mode == LACT_NS_PLAIN_BF16) LACT_LAUNCH_SMEM("k_ns_local", "ns_fwd", flops, (k_ns_local<RT, XG, true>), dim3(B.n), dim3(512), SM, s, p);
+    else LACT_LAUNCH_SMEM("k_ns_local", "ns_fwd", flops, (k_ns_local<RT, XG, false>), dim3(B.n), dim3(512), SM, s, p);
+  }
+  void launch_ns_local(NsLocalParams p, const NsBatch& B) {
+    p.c = B.c; p.S = P.S; p.nb = B.nb; p.mask = B.mask;
+    for (int i = 0; i < 3 * P.S; ++i) p.coeffs[i] = P.coeffs[i];
+    const bool wide = B.c > 128;
+    switch (B.r / 32) {
+      case 1: wide ? launch_ns_local_t<1, 32>(p, B) : launch_ns_local_t<1, 16>(p, B); break;
+      case 2: wide ? launch_ns_local_t<2, 32>(p, B) : launch_ns_local_t<2, 16>(p, B); break;
+      case 3: wide ? launch_ns_local_t<3, 32>(p, B) : launch_ns_local_t<3, 16>(p, B); break;
+      default: wide ? launch_ns_local_t<4, 32>(p, B) : launch_ns_local_t<4, 16>(p, B); break;
+    }
+  }
+  // forward: every batch runs in one launch that normalises its matrices itself
+  bool ns_fwd_one_launch() const {
+    if (!P.muon || P.nsb.empty()) return false;
+    for (auto& B : P.nsb)
+      if (!ns_local_ok(B) && !ns_fused_ok(B)) return false;
+    return true;
+  }
+  bool ns_fwd_fused_any() const {
+    for (auto& B : P.nsb)
+      if (!ns_local_ok(B) && ns_fused_ok(B)) return true;
+    return false;
+  }
+  // every batch runs fused (and at least one iteration): the Frobenius normalisation's backward is the fused kernel's last stage
   bool ns_all_fused() const {
     if (!P.muon || P.nsb.empty()) return false;
     for (auto& B : P.nsb)
@@ -629,10 +666,10 @@ struct Runner {
   }
   unsigned* ns_error_word() const { return scr<unsigned>(P.t_nssync) + (size_t)P.g.ns_count() * 32; }
   // barrier lines and error word start at zero: once per Newton-Schulz phase, by the kernel in front of its batches
-  ClearWords ns_clear() const {
+  ClearWords ns_clear(bool forward) const {
     ClearWords c;
     c.ptr = nullptr; c.n = 0;
-    if (P.muon && ns_fused_any()) { c.ptr = scr<unsigned>(P.t_nssync); c.n = P.g.ns_count() * 32 + 32; }
+    if (P.muon && (forward ? ns_fwd_fused_any() : ns_fused_any())) { c.ptr = scr<unsigned>(P.t_nssync); c.n = P.g.ns_count() * 32 + 32; }
     return c;
   }
   template <class TS, bool BWD>
@@ -1050,7 +1087,7 @@ struct Runner {
           pf.mbar = has_prev(u) ? mbar(u) : nullptr;
           pf.g16 = reinterpret_cast<uint16_t*>(g16(u)); pf.ss_part = scr<float>(P.t_ss);
           pf.clear.ptr = nullptr; pf.clear.n = 0;
-          if (ns_all_fused()) pf.clear = ns_clear();
+          if (ns_fwd_one_launch()) pf.clear = ns_clear(true);
         }
         dw_slots = token_reduce("update_dw", jobs, T_, nullptr, nullptr, 0.f, can_fold ? &pf : nullptr);
       }
@@ -1068,12 +1105,12 @@ struct Runner {
         p.round_partial_bf16 = P.bf16;
         if (u + 1 == P.nupd && P.momentum && m_out)
           for (int j = 0; j < 3; ++j) p.m_ext[j] = m_out[j];
-        if (ns_all_fused()) p.clear = ns_clear();
+        if (ns_fwd_one_launch()) p.clear = ns_clear(true);
         LACT_LAUNCH("k_momentum_prep", "k_momentum_prep", 0.0, (k_momentum_prep<TN>), dim3(P.nblk, 3 * d.b), dim3(256), s, p);
       }
       flush_applies(true);
       if (P.muon) {
-        const bool scale_in_kernel = ns_all_fused();
+        const bool scale_in_kernel = ns_fwd_one_launch();
         if (!scale_in_kernel) {
           NsScaleParams p;
           memset(&p, 0, sizeof(p));
@@ -1081,10 +1118,27 @@ struct Runner {
           p.xf = scr<float>(P.t_xf[0]); p.xb = xb(u, 0);
           p.u = P.S == 0 ? usave(u) : nullptr;
           p.plain_bf16 = d.ns_mode == LACT_NS_PLAIN_BF16;
-          p.clear = ns_clear();
+          p.clear = ns_clear(true);
           LACT_LAUNCH("k_ns_scale", "k_ns_scale", 0.0, (k_ns_scale<TN>), dim3(P.nblk, P.g.ns_count()), dim3(256), s, p);
         }
         for (const NsBatch& B : P.nsb) {
+          if (scale_in_kernel && ns_local_ok(B)) {
+            if constexpr (kNsBf16) {
+              NsLocalParams f;
+              memset(&f, 0, sizeof(f));
+              f.g16 = g16(u) + B.xoff;
+              f.ss_part = scr<float>(P.t_ss); f.nparts = ss_parts;
+              f.part0 = B.first; f.part1 = (P.g.stacked && B.first == 0) ? 2 * d.b : -1;
+              f.norms = norms(u) + B.first;
+              if (!d.forward_only) {
+                f.xb = xb(u, 0) + B.xoff; f.xb_it_stride = (long long)P.mat3;
+                f.ab = ab(u, 0) + B.sqoff; f.bb = bb(u, 0) + B.sqoff; f.sq_it_stride = (long long)sq3();
+              }
+              f.u_out = usave(u) + B.xoff;
+              launch_ns_local(f, B);
+            }
+            continue;
+          }
           if (ns_fused_ok(B)) {
             if constexpr (kNsBf16) {
               NsFusedParams f;
@@ -1128,7 +1182,7 @@ struct Runner {
         p.wc_out = P.bf16 ? (void*)wc(ver + 1) : nullptr;
         if (u + 1 == P.nupd && w_out)
           for (int j = 0; j < 3; ++j) p.w_ext[j] = w_out[j];
-        if (P.muon && ns_fused_any()) p.poison = ns_error_word();
+        if (P.muon && ns_fwd_fused_any()) p.poison = ns_error_word();
         LACT_LAUNCH("k_update_renorm", "k_update_renorm", 0.0, (k_update_renorm<T>), rowgrid, dim3(256), s, p);
       }
       ++ver;
@@ -1395,7 +1449,7 @@ struct Runner {
         p.gw_hat = gwhat;
         p.gn0 = gn0; p.gn0_init = !gn0_written;
         gn0_written = true;
-        p.clear = ns_clear();
+        p.clear = ns_clear(false);
         if (P.muon) { p.gxf = scr<float>(P.t_gxf[0]); p.gxb = scr<TN>(P.t_gxb[0]); }
         LACT_LAUNCH("k_renorm_bwd", "k_renorm_bwd", 0.0, (k_renorm_bwd<TN>), rowgrid, dim3(256), s, p);
         if (side_valid[sb]) {

@@ -59,3 +59,32 @@ def test_transposed_weights_are_read_as_they_lie(dtype, d, dh):
             assert O.rel_l2(a, r) < 1e-6
             if len(steps) == 1:
                 assert torch.equal(a, w) and torch.equal(r, w)
+
+
+@pytest.mark.parametrize("b,d,dh,L,stacked", [
+    (3, 128, 256, 200, False), (2, 64, 64, 100, False), (1, 96, 96, 100, False), (2, 32, 224, 80, False), (2, 256, 64, 130, False),
+    (2, 96, 160, 90, False), (5, 128, 128, 90, False), (2, 128, 64, 90, True)])
+def test_newton_schulz_in_one_block_is_bit_identical(b, d, dh, L, stacked):
+    """Matrices that fit one block (csrc/ns_local.h) against the launches per iteration: the same bits in output, weights and, with
+    the iterates that the kernel keeps for it, every gradient."""
+    print("[gpu-test] local newton-schulz", b, d, dh, L, stacked, flush=True)
+    from lact_amd import _lib, ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(b, L, d, dh, seed=33, act_dtype=torch.bfloat16).items()}
+    go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(4)).bfloat16().to("cuda")
+    for coeffs, mode in ((ops.NS5_COEFFS, ops.NS_AUTOCAST), ((ops.NS_CLASSIC,) * 3, ops.NS_PLAIN_BF16)):
+        prog = ops.Program(steps=((LACT_UPDATE, 0, L, 0), (LACT_APPLY, 0, L, 0)), out_len=L, ns_coeffs=coeffs, ns_mode=mode, muon_stacked=stacked)
+        res = []
+        for fused in (1, 0):
+            _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, fused)
+            try:
+                leaves = [inp[n].clone().requires_grad_(True) for n in ORDER[:9]]
+                out, ws, _ = ops.run_program(prog, *leaves)
+                grads = torch.autograd.grad(out, leaves, go)
+                with torch.no_grad():
+                    out_inf, ws_inf, _ = ops.run_program(prog, *[inp[n] for n in ORDER[:9]])
+                res.append([out.detach(), *[w.detach() for w in ws], out_inf, *ws_inf, *grads])
+            finally:
+                _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 1)
+        for a, r in zip(*res):
+            assert torch.equal(a, r)

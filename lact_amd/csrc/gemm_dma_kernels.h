@@ -10,6 +10,7 @@ namespace lact {
 using TS_ROW = TileShape<256, 128, 2, 2>;   // token-row GEMMs, one accumulator: 128x64 per wave
 using TS_SQ = TileShape<128, 128, 2, 2>;    // small square GEMMs (Newton-Schulz) and 2-3 accumulator kernels
 using TS_BWD = TileShape<128, 64, 2, 2>;    // six accumulators (update backward): 64x32 per wave
+using TS_64 = TileShape<64, 64, 2, 2>;      // the same where two blocks share a compute unit
 using TS_NS = TileShape<192, 192, 2, 2>;    // 384-multiple square GEMMs (Newton-Schulz at d = dh = 384): 96x96 per wave
 using TS_N96 = TileShape<128, 96, 4, 1>;    // Newton-Schulz of few 384-multiple matrices: 12 instead of 9 blocks per 384 x 384 matrix
 
@@ -265,11 +266,11 @@ __device__ __forceinline__ DmaOperand weight_operand_ks(const void* base, long l
   return o;
 }
 
+// The hidden-stage kernels below: STAGES of the ring, WPE waves per SIMD (2: one block per compute unit, 4: two).
 // apply forward: O0 = silu(X W0^T) * (X W2^T)
-template <class TS>
-__global__ __launch_bounds__(DMA_THREADS) void k_apply_hidden_dma(const HiddenDmaParams pp) {
+template <class TS, int STAGES = 3, int WPE = 2>
+__global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int STAGES = 3;
   using Pipe = DmaPipe<TS, 2, 1, STAGES>;
   const HiddenParams& p = pp.h;
   int bx, by, z;
@@ -315,10 +316,9 @@ __global__ __launch_bounds__(DMA_THREADS) void k_apply_hidden_dma(const HiddenDm
 }
 
 // Shared main loop of the three-accumulator kernels: acc0 = X W0^T, acc1 = X W2^T, acc2 = Y W1 (via W1T).
-template <class TS>
+template <class TS, int STAGES>
 __device__ __forceinline__ void three_acc_mainloop(const HiddenDmaParams& pp, char* smem, int m0, int n0, int z,
                                                    f32x16 (&a02)[2][TS::TM][TS::TN], f32x16 (&a1)[1][TS::TM][TS::TN]) {
-  constexpr int STAGES = 3;
   using Pipe = DmaPipe<TS, 2, 2, STAGES>;
   const HiddenParams& p = pp.h;
   DmaPhase<2> ph[2];
@@ -371,10 +371,10 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
 // staged tiles instead of eight.  Element by element the same operations on the same rounded values as before.
 // The three accumulators of a hidden-stage tile, rounded to bf16, into three staged tiles at the start of the ring
 // (matrix waves only; the caller synchronises the block before anyone reads them).
-template <class TS>
+template <class TS, int STAGES>
 __device__ __forceinline__ void stage_three_products(char* smem, const f32x16 (&a02)[2][TS::TM][TS::TN], const f32x16 (&a1)[1][TS::TM][TS::TN]) {
   using SB = StageTile<TS, 2>;
-  static_assert(3 * SB::BYTES <= DmaSmem<TS, 2, 3>::BYTES, "the three staged tiles lie in the ring");
+  static_assert(3 * SB::BYTES <= DmaSmem<TS, 2, STAGES>::BYTES, "the three staged tiles lie in the ring");
   char* s0 = smem + SB::lane_base(); char* s1 = s0 + SB::BYTES; char* s2 = s0 + 2 * SB::BYTES;
   if (threadIdx.x < TS::THREADS) LACT_FOR_QUADS(TS) {
     SB::put4(s0, tm, tn, g, a02[0][tm][tn][4 * g], a02[0][tm][tn][4 * g + 1], a02[0][tm][tn][4 * g + 2], a02[0][tm][tn][4 * g + 3]);
@@ -383,8 +383,8 @@ __device__ __forceinline__ void stage_three_products(char* smem, const f32x16 (&
   }
 }
 
-template <class TS>
-__global__ __launch_bounds__(DMA_THREADS) void k_update_hidden_dma(const HiddenDmaParams pp) {
+template <class TS, int STAGES = 3, int WPE = 2>
+__global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const HiddenParams& p = pp.h;
   int bx, by, z;
@@ -393,8 +393,8 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_hidden_dma(const HiddenD
   using SB = StageTile<TS, 2>;
   {
     f32x16 a02[2][TS::TM][TS::TN], a1[1][TS::TM][TS::TN];
-    three_acc_mainloop<TS>(pp, smem, m0, n0, z, a02, a1);
-    stage_three_products<TS>(smem, a02, a1);
+    three_acc_mainloop<TS, STAGES>(pp, smem, m0, n0, z, a02, a1);
+    stage_three_products<TS, STAGES>(smem, a02, a1);
   }
   __syncthreads();
   if (!SB::active()) return;
@@ -450,8 +450,8 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_hidden_dma(const HiddenD
 // apply backward, hidden stage: Y0 = X W0^T, Y2 = X W2^T, GH = dOut W1 -> O0 = silu(Y0) * Y2 (the hidden activation,
 // recomputed), O1 = d Y0, O2 = d Y2 (lact_swiglu_ffn.py:46-76).  Epilogue as in k_update_hidden_dma: three staged
 // products, the pointwise part on all eight waves, stores straight from registers.
-template <class TS>
-__global__ __launch_bounds__(DMA_THREADS) void k_apply_bwd_hidden_dma(const HiddenDmaParams pp) {
+template <class TS, int STAGES = 3, int WPE = 2>
+__global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_bwd_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const HiddenParams& p = pp.h;
   int bx, by, z;
@@ -460,8 +460,8 @@ __global__ __launch_bounds__(DMA_THREADS) void k_apply_bwd_hidden_dma(const Hidd
   using SB = StageTile<TS, 2>;
   {
     f32x16 a02[2][TS::TM][TS::TN], a1[1][TS::TM][TS::TN];
-    three_acc_mainloop<TS>(pp, smem, m0, n0, z, a02, a1);
-    stage_three_products<TS>(smem, a02, a1);
+    three_acc_mainloop<TS, STAGES>(pp, smem, m0, n0, z, a02, a1);
+    stage_three_products<TS, STAGES>(smem, a02, a1);
   }
   __syncthreads();
   if (!SB::active()) return;
@@ -500,10 +500,9 @@ __global__ __launch_bounds__(DMA_THREADS) void k_apply_bwd_hidden_dma(const Hidd
 }
 
 // update backward, hidden stage: phases (X; W0,W2), (X; G0,G2), (Y; W1T,G1T)
-template <class TS>
-__global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_dma(const HiddenDmaParams pp) {
+template <class TS, int STAGES = 3, int WPE = 2>
+__global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_bwd_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int STAGES = 3;
   using Pipe = DmaPipe<TS, 2, 3, STAGES>;
   const HiddenParams& p = pp.h;
   int bx, by, z;

@@ -230,11 +230,14 @@ int token_reduce_tiles(int d, int dh) {
   return std::max(ceil_div(dh, TSG<T>::BM) * ceil_div(d, TSG<T>::BN), ceil_div(d, TSG<T>::BM) * ceil_div(dh, TSG<T>::BN));
 }
 
-// output tiles per matrix of the asynchronous-copy token reduction
-int token_reduce_dma_tiles(int d, int dh) {
-  const bool big = d % TS_NS::BM == 0 && dh % TS_NS::BM == 0;
-  return big ? (d / TS_NS::BM) * (dh / TS_NS::BN)
-             : std::max(ceil_div(dh, TS_SQ::BM) * ceil_div(d, TS_SQ::BN), ceil_div(d, TS_SQ::BM) * ceil_div(dh, TS_SQ::BN));
+// Tile of the dedicated-loader token reduction: 192 x 192 where it divides the matrices, else 128 x 128.  (128 x 64 where few
+// matrices leave the chip idle was measured: a block's K-step takes as long as with the large tile -- it waits for operands
+// that another kernel has just written -- and the launch copies more: 12 matrices of 384 x 384, 2048 tokens, 28.7 us in 48
+// blocks of 192 x 192, 28.2 us in 216 of 128 x 64, the launch that also holds the dk and dv GEMMs 34 against 42 us.)
+bool tr_big(int d, int dh) { return d % TS_NS::BM == 0 && dh % TS_NS::BM == 0; }
+int tr_tiles(int d, int dh) {   // output tiles per matrix
+  return tr_big(d, dh) ? (d / TS_NS::BM) * (dh / TS_NS::BN)
+                       : std::max(ceil_div(dh, TS_SQ::BM) * ceil_div(d, TS_SQ::BN), ceil_div(d, TS_SQ::BM) * ceil_div(dh, TS_SQ::BN));
 }
 
 // One Newton-Schulz launch group: n matrices of one geometry, laid out one after the other.
@@ -364,7 +367,7 @@ struct Plan {
     tiles = bf16 ? token_reduce_tiles<uint16_t>(d.d, d.dh) : token_reduce_tiles<float>(d.d, d.dh);
     // partial-sum slots: the larger split count of the two token-reduction kernels at the longest chunk (the
     // count grows with the tokens)
-    nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, 16, false).n, choose_split(Tcap, token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b, 16).n);
+    nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, 16, false).n, choose_split(Tcap, tr_tiles(d.d, d.dh) * 3 * d.b, 16).n);
 
     Bump sv;
     s_n0 = sv.take((size_t)3 * d.b * g.maxrows() * 4);
@@ -465,10 +468,14 @@ void launch_row_gemm(const char* site, const RowGemmParams<NT>& p, int batch, hi
         // 256 x 128 tiles copy a third fewer operand bytes per FLOP than 128 x 128 ones, but a launch whose blocks fill
         // the last round of compute units only partly wastes more than that: pick by the fuller last round
         static const int cus = [] { int dev = 0, n = 0; (void)hipGetDevice(&dev); return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256; }();
-        auto fill = [&](int bm) { const long long blocks = (long long)ceil_div(p.M, bm) * ceil_div(p.N, 128) * batch; return (double)blocks / ((double)((blocks + cus - 1) / cus) * cus); };
+        auto blocks = [&](int bm, int bn) { return (long long)ceil_div(p.M, bm) * ceil_div(p.N, bn) * batch; };
+        auto fill = [&](int bm) { const long long n = blocks(bm, 128); return (double)n / ((double)((n + cus - 1) / cus) * cus); };
+        // less than one round: the blocks that fit side by side, down to 128 x 64
+        if (blocks(128, 128) <= cus / 2) launch_row_gemm_dma<TS_BWD, NT, EPI, !B_KC>(site, q, batch, s);
+        else if (blocks(128, 128) <= cus) launch_row_gemm_dma<TS_SQ, NT, EPI, !B_KC>(site, q, batch, s);
         // (measured at 384 blocks on 256 units: one-term GEMM 27.0 -> 24.5 us with the small tile, two-term GEMM with
         // K-strided weights 34 -> 36 us: only the one-term case switches)
-        if (NT == 1 && fill(256) < 0.8 && fill(128) > fill(256) + 0.1) launch_row_gemm_dma<TS_SQ, NT, EPI, !B_KC>(site, q, batch, s);
+        else if (NT == 1 && fill(256) < 0.8 && fill(128) > fill(256) + 0.1) launch_row_gemm_dma<TS_SQ, NT, EPI, !B_KC>(site, q, batch, s);
         else launch_row_gemm_dma<TS_ROW, NT, EPI, !B_KC>(site, q, batch, s);
       }
       else if (p.M % TS_NS::BM == 0 && p.N % TS_NS::BN == 0) launch_row_gemm_dma<TS_NS, NT, EPI, !B_KC>(site, q, batch, s);
@@ -648,8 +655,9 @@ struct Runner {
     return true;
   }
   bool ns_fwd_fused_any() const {
+    const bool local = ns_fwd_one_launch();   // otherwise the normalisation is a launch of its own and nothing runs local
     for (auto& B : P.nsb)
-      if (!ns_local_ok(B) && ns_fused_ok(B)) return true;
+      if (ns_fused_ok(B) && !(local && ns_local_ok(B))) return true;
     return false;
   }
   // every batch runs fused (and at least one iteration): the Frobenius normalisation's backward is the fused kernel's last stage
@@ -751,6 +759,11 @@ struct Runner {
     if (P.keep_pre) return ceil_div(d.dh, TS_SQ::BN) * TS_SQ::WAVES_N;
     return ceil_div(d.dh, TS_BWD::BN) * TS_BWD::WAVES_N;
   }
+  bool hidden_small(int which) const { return which == 0 ? d.d <= 256 : which <= 3 && d.d <= 192; }   // the kernel from kept pre-activations has the large tile only
+  // LACT_OPT_PERSISTENT_TILES: its default, the apply alone, gives way to the small tiles; any other mask is taken as it is
+  bool hidden_persists(int which) const {
+    return d.d % 64 == 0 && ((g_persist >> which) & 1) && side && side->cus > 0 && !(g_persist == 1 && hidden_small(which));
+  }
   void launch_hidden(int which, const HiddenParams& hp, int ver, int T_) const {
     const double f = (double)T_ * d.d * d.dh * d.b;
     if (dma_hidden()) {
@@ -758,21 +771,29 @@ struct Runner {
       HiddenDmaParams q;
       q.h = hp;
       (void)ver;
+      // Tiles.  128 x 128 with three stages, one block per compute unit; where the products are at most three K-steps long
+      // (d <= 192) a block's time goes into its first copies and its epilogue, and two smaller blocks per unit overlap
+      // theirs.  Measured, us per launch, large / small: 12 heads, d = 128, dh = 256, 4680 tokens: update 52.8 / 46.6,
+      // apply backward 46.3 / 42.5, recomputing update backward 96 / 91; d = 96: 27.8 / 25.7, 23.7 / 21.5, 47.9 / 43;
+      // d = 256: even; d = 384: update 22.3 / 23.7, apply backward 18.5 / 19.7.  The apply's two accumulators: small tiles up
+      // to d = 256 (10.4 / 9.95 at d = 256; persistent blocks on large tiles beyond, where they are alone in running ahead).
       constexpr int SM3 = DmaSmem<TS_SQ, 2, 3>::BYTES;   // the epilogues stage at most three bf16 tiles, inside the ring
+      constexpr int SMS = DmaSmem<TS_BWD, 2, 2>::BYTES;
       constexpr int SM6 = cmax(DmaSmem<TS_BWD, 2, 3>::BYTES, 6 * StageTile<TS_BWD, 2>::BYTES);
-      const TileMap m3 = make_tile_map(ceil_div(T_, TS_SQ::BM), ceil_div(d.dh, TS_SQ::BN), d.b);
-      const TileMap m6 = make_tile_map(ceil_div(T_, TS_BWD::BM), ceil_div(d.dh, TS_BWD::BN), d.b);
-      q.map = which == 3 ? m6 : m3;
-      dim3 g3(m3.grid()), g6(m6.grid());
-      LACT_BIG_LDS(k_apply_hidden_dma<TS_SQ>, SM3);
-      LACT_BIG_LDS(k_update_hidden_dma<TS_SQ>, SM3);
-      LACT_BIG_LDS(k_apply_bwd_hidden_dma<TS_SQ>, SM3);
-      LACT_BIG_LDS(k_update_bwd_hidden_dma<TS_BWD>, SM6);
+      constexpr int SM6S = cmax(DmaSmem<TS_64, 2, 3>::BYTES, 6 * StageTile<TS_64, 2>::BYTES);
+      LACT_BIG_LDS((k_apply_hidden_dma<TS_SQ>), SM3);
+      LACT_BIG_LDS((k_update_hidden_dma<TS_SQ>), SM3);
+      LACT_BIG_LDS((k_apply_bwd_hidden_dma<TS_SQ>), SM3);
+      LACT_BIG_LDS((k_apply_hidden_dma<TS_BWD, 2, 4>), SMS);
+      LACT_BIG_LDS((k_update_hidden_dma<TS_BWD, 2, 4>), SMS);
+      LACT_BIG_LDS((k_apply_bwd_hidden_dma<TS_BWD, 2, 4>), SMS);
+      LACT_BIG_LDS((k_update_bwd_hidden_dma<TS_BWD>), SM6);
+      LACT_BIG_LDS((k_update_bwd_hidden_dma<TS_64, 3, 4>), SM6S);
       LACT_BIG_LDS(k_update_bwd_hidden_kept_dma<TS_SQ>, SM3);
-      if (which <= 2 && d.d % 64 == 0 && ((g_persist >> which) & 1) && side && side->cus > 0) {
+      if (which <= 2 && hidden_persists(which)) {
         HiddenPersistParams hq;
-        hq.h = hp; hq.map = m3;
-        const dim3 gp(persist_grid(m3.grid(), side->cus));
+        hq.h = hp; hq.map = make_tile_map(ceil_div(T_, TS_SQ::BM), ceil_div(d.dh, TS_SQ::BN), d.b);
+        const dim3 gp(persist_grid(hq.map.grid(), side->cus));
         LACT_BIG_LDS(k_hidden_persist<ApplyHiddenPolicy>, PersistLds<ApplyHiddenPolicy>::BYTES);
         LACT_BIG_LDS(k_hidden_persist<UpdateHiddenPolicy>, PersistLds<UpdateHiddenPolicy>::BYTES);
         LACT_BIG_LDS(k_hidden_persist<ApplyBwdHiddenPolicy>, PersistLds<ApplyBwdHiddenPolicy>::BYTES);
@@ -781,11 +802,27 @@ struct Runner {
         if (which == 2) LACT_LAUNCH_SMEM("k_hidden_persist<apply_bwd>", "apply_bwd_hidden", 6.0 * f, (k_hidden_persist<ApplyBwdHiddenPolicy>), gp, dim3(DMA_THREADS), PersistLds<ApplyBwdHiddenPolicy>::BYTES, s, hq);
         return;
       }
-      if (which == 0) LACT_LAUNCH_SMEM("k_apply_hidden_dma", "apply_hidden", 4.0 * f, (k_apply_hidden_dma<TS_SQ>), g3, dim3(DMA_THREADS), SM3, s, q);
-      if (which == 1) LACT_LAUNCH_SMEM("k_update_hidden_dma", "update_hidden", 6.0 * f, (k_update_hidden_dma<TS_SQ>), g3, dim3(DMA_THREADS), SM3, s, q);
-      if (which == 2) LACT_LAUNCH_SMEM("k_apply_bwd_hidden_dma", "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden_dma<TS_SQ>), g3, dim3(DMA_THREADS), SM3, s, q);
-      if (which == 3) LACT_LAUNCH_SMEM("k_update_bwd_hidden_dma", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden_dma<TS_BWD>), g6, dim3(DMA_THREADS), SM6, s, q);
-      if (which == 4) LACT_LAUNCH_SMEM("k_update_bwd_hidden_kept_dma", "update_bwd_hidden", 6.0 * f, (k_update_bwd_hidden_kept_dma<TS_SQ>), g3, dim3(DMA_THREADS), SM3, s, q);
+      const bool small = hidden_small(which);
+      // tile of the kernel that is launched below: the grid has to cover exactly its tiles
+      const int bm = which == 3 && small ? TS_64::BM : 128, bn = which == 3 || small ? 64 : 128;
+      static_assert(TS_SQ::BM == 128 && TS_SQ::BN == 128 && TS_BWD::BM == 128 && TS_BWD::BN == 64 && TS_64::BN == 64, "tiles of the hidden-stage kernels");
+      q.map = make_tile_map(ceil_div(T_, bm), ceil_div(d.dh, bn), d.b);
+      const dim3 g(q.map.grid()), t(DMA_THREADS);
+      if (which == 0) {
+        if (small) LACT_LAUNCH_SMEM("k_apply_hidden_dma", "apply_hidden", 4.0 * f, (k_apply_hidden_dma<TS_BWD, 2, 4>), g, t, SMS, s, q);
+        else LACT_LAUNCH_SMEM("k_apply_hidden_dma", "apply_hidden", 4.0 * f, (k_apply_hidden_dma<TS_SQ>), g, t, SM3, s, q);
+      } else if (which == 1) {
+        if (small) LACT_LAUNCH_SMEM("k_update_hidden_dma", "update_hidden", 6.0 * f, (k_update_hidden_dma<TS_BWD, 2, 4>), g, t, SMS, s, q);
+        else LACT_LAUNCH_SMEM("k_update_hidden_dma", "update_hidden", 6.0 * f, (k_update_hidden_dma<TS_SQ>), g, t, SM3, s, q);
+      } else if (which == 2) {
+        if (small) LACT_LAUNCH_SMEM("k_apply_bwd_hidden_dma", "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden_dma<TS_BWD, 2, 4>), g, t, SMS, s, q);
+        else LACT_LAUNCH_SMEM("k_apply_bwd_hidden_dma", "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden_dma<TS_SQ>), g, t, SM3, s, q);
+      } else if (which == 3) {
+        if (small) LACT_LAUNCH_SMEM("k_update_bwd_hidden_dma", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden_dma<TS_64, 3, 4>), g, t, SM6S, s, q);
+        else LACT_LAUNCH_SMEM("k_update_bwd_hidden_dma", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden_dma<TS_BWD>), g, t, SM6, s, q);
+      } else {
+        LACT_LAUNCH_SMEM("k_update_bwd_hidden_kept_dma", "update_bwd_hidden", 6.0 * f, (k_update_bwd_hidden_kept_dma<TS_SQ>), g, t, SM3, s, q);
+      }
       }
     } else {
       using TS = TSG<T>;
@@ -836,6 +873,21 @@ struct Runner {
     RowGemmParams<2> r2;
     bool done = false;
   };
+  template <class TS>
+  void launch_tr(const char* site, double flops, dim3 grid, const TokenReduceDmaParams& p) const {
+    constexpr int SM = cmax(DmaSmem<TS, 1, row_stages<TS>()>::BYTES, StageTile<TS, 4>::BYTES);
+    static const std::string name = "k_token_reduce_dma<" + std::to_string(TS::BM) + "x" + std::to_string(TS::BN) + ">";
+    LACT_BIG_LDS(k_token_reduce_dma<TS>, SM);
+    LACT_LAUNCH_SMEM(name.c_str(), site, flops, (k_token_reduce_dma<TS>), grid, dim3(DMA_THREADS), SM, s, p);
+  }
+  template <class TS>
+  void launch_tr_rows(const char* site, double flops, dim3 grid, const TokenReduceRowsParams& p) const {
+    constexpr int SM = cmax(cmax(DmaSmem<TS_ROW, 1, row_stages<TS_ROW>()>::BYTES, StageTile<TS_ROW, 4>::BYTES),
+                            cmax(DmaSmem<TS, 1, row_stages<TS>()>::BYTES, StageTile<TS, 4>::BYTES));
+    static const std::string name = "k_token_reduce_rows_dma<" + std::to_string(TS::BM) + "x" + std::to_string(TS::BN) + ">";
+    LACT_BIG_LDS(k_token_reduce_rows_dma<TS>, SM);
+    LACT_LAUNCH_SMEM(name.c_str(), site, flops, (k_token_reduce_rows_dma<TS>), grid, dim3(DMA_THREADS), SM, s, p);
+  }
   int token_reduce(const char* site, const TokenReduceJob (&jobs)[3], int tokens, float* add_out = nullptr,
                    const float* add_in = nullptr, float coeff = 0.f, const PrepFold* prep = nullptr,
                    RowCompanions* rows = nullptr) const {
@@ -848,8 +900,7 @@ struct Runner {
     bool direct = false;
     if constexpr (kBf16) {
       if (tokens >= 64) {     // a ragged end is handled inside the last K-step
-        const bool big = d.d % TS_NS::BM == 0 && d.dh % TS_NS::BM == 0;
-        const int tiles = token_reduce_dma_tiles(d.d, d.dh);
+        const int tiles = tr_tiles(d.d, d.dh);
         const Split sp = choose_split(tokens, tiles * 3 * d.b, P.nsplit_max);
         TokenReduceDmaParams pd;
         static_cast<TokenReduceParams&>(pd) = p;
@@ -882,26 +933,11 @@ struct Runner {
           double frows = 0;
           for (int t = 0; t < 4; ++t) frows += 2.0 * rows->r4.M * rows->r4.N * rows->r4.t[t].K * d.b;
           for (int t = 0; t < 2; ++t) frows += 2.0 * rows->r2.M * rows->r2.N * rows->r2.t[t].K * d.b;
-          constexpr int SMR = cmax(DmaSmem<TS_ROW, 1, row_stages<TS_ROW>()>::BYTES, StageTile<TS_ROW, 4>::BYTES);
-          if (big) {
-            constexpr int SM = cmax(SMR, cmax(DmaSmem<TS_NS, 1, row_stages<TS_NS>()>::BYTES, StageTile<TS_NS, 4>::BYTES));
-            LACT_BIG_LDS(k_token_reduce_rows_dma<TS_NS>, SM);
-            LACT_LAUNCH_SMEM("k_token_reduce_rows_dma<192x192>", site, fl + frows, (k_token_reduce_rows_dma<TS_NS>), gr, dim3(DMA_THREADS), SM, s, q);
-          } else {
-            constexpr int SM = cmax(SMR, cmax(DmaSmem<TS_SQ, 1, row_stages<TS_SQ>()>::BYTES, StageTile<TS_SQ, 4>::BYTES));
-            LACT_BIG_LDS(k_token_reduce_rows_dma<TS_SQ>, SM);
-            LACT_LAUNCH_SMEM("k_token_reduce_rows_dma<128x128>", site, fl + frows, (k_token_reduce_rows_dma<TS_SQ>), gr, dim3(DMA_THREADS), SM, s, q);
-          }
+          if (tr_big(d.d, d.dh)) launch_tr_rows<TS_NS>(site, fl + frows, gr, q);
+          else launch_tr_rows<TS_SQ>(site, fl + frows, gr, q);
           rows->done = true;
-        } else if (big) {
-          constexpr int SM = cmax(DmaSmem<TS_NS, 1, row_stages<TS_NS>()>::BYTES, StageTile<TS_NS, 4>::BYTES);
-          LACT_BIG_LDS(k_token_reduce_dma<TS_NS>, SM);
-          LACT_LAUNCH_SMEM("k_token_reduce_dma<192x192>", site, fl, (k_token_reduce_dma<TS_NS>), g, dim3(DMA_THREADS), SM, s, pd);
-        } else {
-          constexpr int SM = cmax(DmaSmem<TS_SQ, 1, row_stages<TS_SQ>()>::BYTES, StageTile<TS_SQ, 4>::BYTES);
-          LACT_BIG_LDS(k_token_reduce_dma<TS_SQ>, SM);
-          LACT_LAUNCH_SMEM("k_token_reduce_dma<128x128>", site, fl, (k_token_reduce_dma<TS_SQ>), g, dim3(DMA_THREADS), SM, s, pd);
-        }
+        } else if (tr_big(d.d, d.dh)) launch_tr<TS_NS>(site, fl, g, pd);
+        else launch_tr<TS_SQ>(site, fl, g, pd);
         return folded ? -1 : slots;
       }
     }
@@ -1092,7 +1128,7 @@ struct Runner {
         dw_slots = token_reduce("update_dw", jobs, T_, nullptr, nullptr, 0.f, can_fold ? &pf : nullptr);
       }
       const bool prep_folded = dw_slots < 0;
-      const int ss_parts = prep_folded ? token_reduce_dma_tiles(d.d, d.dh) : P.nblk;
+      const int ss_parts = prep_folded ? tr_tiles(d.d, d.dh) : P.nblk;
       if (!prep_folded) {
         MomentumPrepParams p;
         memset(&p, 0, sizeof(p));
@@ -1620,8 +1656,10 @@ struct Runner {
       // inside its launch (below) than beside the chain (config 2, 48 reduction blocks: -1.4 %; config 4, 216: +1 %)
       bool lone_reduction = false;
       if constexpr (kBf16)
-        lone_reduction = token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b *
-                             choose_split(T_, token_reduce_dma_tiles(d.d, d.dh) * 3 * d.b, P.nsplit_max).n < 160;
+        {
+          const int tiles = tr_tiles(d.d, d.dh) * 3 * d.b;
+          lone_reduction = tiles * choose_split(T_, tiles, P.nsplit_max).n < 160;
+        }
       const bool use_tail = s_tail != s_main && u > 0 && !lone_reduction;
       if (use_tail) {
         wait_for(s_tail, s_main);

@@ -204,24 +204,21 @@ int ceil_div(int a, int b) { return (a + b - 1) / b; }
 struct Split {
   int n, len;
 };
-// max_n: slots the partial-sum buffer holds for this launch
-Split choose_split(int tokens, int tiles_total, int max_n) {
+// max_n: slots the partial-sum buffer holds for this launch; min_len: tokens a split has at least
+Split choose_split(int tokens, int tiles_total, int max_n, int min_len) {
   // One split once the tiles alone occupy most of the 256 compute units: the partial sums then never exist.
-  // Otherwise enough splits for one round of blocks, each over at least 1536 tokens: partial sums cost a write, a
-  // read and (in the backward) a launch, which short splits do not earn back (measured at 36 to 72 tiles: 8.6 ->
-  // 7.4 ms at config 2, 3.63 -> 3.41 ms at config 4 against a target of two rounds and 128 tokens).
+  // Otherwise enough splits for one round of blocks, each over at least min_len tokens: partial sums cost a write and a
+  // read, which short splits do not earn back.
   int ns = tiles_total >= 160 ? 1 : std::max(1, 256 / std::max(1, tiles_total));
-  ns = std::min(std::min(ns, std::max(1, max_n)), std::max(1, tokens / 1536));
+  ns = std::min(std::min(ns, std::max(1, max_n)), std::max(1, tokens / min_len));
   int len = ceil_div(ceil_div(tokens, ns), 64) * 64;
   return Split{ceil_div(tokens, len), len};
 }
 
-// The same for the kernel of gemm_kernels.h, whose tiles are small: two rounds of blocks at most, each over at least 128
-// tokens where the consumer adds the partial sums up anyway (the momentum step of a forward update), over 1024 where a
-// launch of its own has to (`own_launch`; 5 us against 0.014 us per token of a split saved).
-Split choose_split_async(int tokens, int tiles_total, int max_n, bool own_launch) {
+// The same for the kernel of gemm_kernels.h, whose tiles are small: two rounds of blocks at most, each over at least 128 tokens.
+Split choose_split_async(int tokens, int tiles_total, int max_n) {
   int ns = std::max(1, 512 / std::max(1, tiles_total));
-  ns = std::min(std::min(ns, std::max(1, max_n)), std::max(1, tokens / (own_launch ? 1024 : 128)));
+  ns = std::min(std::min(ns, std::max(1, max_n)), std::max(1, tokens / 128));
   int len = ceil_div(ceil_div(tokens, ns), 64) * 64;
   return Split{ceil_div(tokens, len), len};
 }
@@ -256,7 +253,7 @@ struct Plan {
   std::vector<lact_step_t> live;    // the steps that are executed: `steps` without the apply rows a later step overwrites
   std::vector<float> coeffs;
   MatGeom g;
-  int nupd = 0, Tcap = 0, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1;
+  int nupd = 0, Tcap = 0, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 512;
   bool muon = false, bf16 = true, momentum = false, state_in = false;
   size_t mat3 = 0;  // 3*b*elems
   // saved
@@ -271,7 +268,7 @@ struct Plan {
   std::vector<int> pre_T;
   // scratch
   size_t t_h[6], t_partial, t_lrpart, t_xf[2], t_xbtmp, t_ss, t_dot, t_mdot, t_gwhat[2], t_gwcur, t_gmcarry, t_gc,
-      t_gxf[2], t_gxb[2], t_sg, t_gas, t_gn0, t_hs[3], t_partial_side, t_gwside[2], t_nssync, t_kl[2], t_ca, scratch_bytes;
+      t_gxf[2], t_gxb[2], t_sg, t_gas, t_gn0, t_hs[3], t_partial_side[2], t_gwside[2], t_nssync, t_kl[2], t_ca, scratch_bytes;
 
   int build(const lact_desc_t* desc) {
     if (!desc) return fail("null descriptor");
@@ -367,7 +364,12 @@ struct Plan {
     tiles = bf16 ? token_reduce_tiles<uint16_t>(d.d, d.dh) : token_reduce_tiles<float>(d.d, d.dh);
     // partial-sum slots: the larger split count of the two token-reduction kernels at the longest chunk (the
     // count grows with the tokens)
-    nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, 16, false).n, choose_split(Tcap, tr_tiles(d.d, d.dh) * 3 * d.b, 16).n);
+    // With Newton-Schulz the partial sums are read by a pass of its own, and one split lets the reduction's epilogue do the momentum
+    // step; without, the row kernels add them up on the way (12 matrices of 384 x 384, 2048 tokens, us of the reduction and of
+    // the renorm that reads it: one split 30.3 + 9.3, two 21.5 + 10.1, four 18.3 + 12.2).
+    split_min = muon ? 1536 : 1024;
+    nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, 16).n, choose_split(Tcap, tr_tiles(d.d, d.dh) * 3 * d.b, 16, split_min).n);
+    mdot_parts = std::max(std::max(nblk, 256), ceil_div(g.maxrows(), 4));
 
     Bump sv;
     s_n0 = sv.take((size_t)3 * d.b * g.maxrows() * 4);
@@ -406,7 +408,7 @@ struct Plan {
     t_xbtmp = sc.take(mat3 * nsz);
     t_ss = sc.take((size_t)3 * d.b * nblk * 4);
     t_dot = sc.take((size_t)3 * d.b * std::max(nblk, 32) * 4);   // partial dots: per chunk of a matrix, or per block of the fused kernel
-    t_mdot = sc.take((size_t)std::max(1, nupd) * 3 * d.b * std::max(nblk, 256) * 4);   // one slot per update: the momentum gradients are written at the end
+    t_mdot = sc.take((size_t)std::max(1, nupd) * 3 * d.b * mdot_parts * 4);   // one slot per update: the momentum gradients are written at the end
     for (int i = 0; i < 2; ++i) t_gwhat[i] = sc.take(mat3 * 4);
     t_gwcur = sc.take(mat3 * 4);
     t_gmcarry = sc.take(mat3 * 4);
@@ -418,7 +420,7 @@ struct Plan {
     t_gn0 = sc.take((size_t)3 * d.b * g.maxrows() * 4);
     // the apply steps' own buffers (they run beside the update chain)
     for (int i = 0; i < 3; ++i) t_hs[i] = sc.take((size_t)d.b * Tcap * d.dh * esz);
-    t_partial_side = sc.take((size_t)nsplit_max * mat3 * 4);
+    for (int i = 0; i < 2; ++i) t_partial_side[i] = sc.take((size_t)nsplit_max * mat3 * 4);
     for (int i = 0; i < 2; ++i) t_gwside[i] = sc.take(mat3 * 4);
     t_nssync = sc.take(((size_t)3 * d.b * 32 + 32) * 4);   // per-matrix barrier lines of the fused Newton-Schulz kernel + error word
     for (int i = 0; i < 2; ++i) t_kl[i] = sc.take((size_t)d.b * Tcap * d.d * esz);   // k * lr0, k * lr2 of the current update
@@ -722,7 +724,7 @@ struct Runner {
   // enqueue on the side chain (its stream and buffers) while this object lives
   struct OnSide {
     Runner& r;
-    explicit OnSide(Runner& rr) : r(rr) { r.s = r.s_side; r.hsel = r.P.t_hs; r.partial_sel = r.P.t_partial_side; }
+    explicit OnSide(Runner& rr, int sb = 0) : r(rr) { r.s = r.s_side; r.hsel = r.P.t_hs; r.partial_sel = r.P.t_partial_side[sb]; }
     ~OnSide() { r.s = r.s_main; r.hsel = r.P.t_h; r.partial_sel = r.P.t_partial; }
   };
 
@@ -901,7 +903,8 @@ struct Runner {
     if constexpr (kBf16) {
       if (tokens >= 64) {     // a ragged end is handled inside the last K-step
         const int tiles = tr_tiles(d.d, d.dh);
-        const Split sp = choose_split(tokens, tiles * 3 * d.b, P.nsplit_max);
+        // with the row GEMMs in the launch the chip is busy: short splits only cost (36.4 us in one split, 38.2 in two, 46.8 in four)
+        const Split sp = choose_split(tokens, tiles * 3 * d.b, P.nsplit_max, rows ? 1536 : P.split_min);
         TokenReduceDmaParams pd;
         static_cast<TokenReduceParams&>(pd) = p;
         pd.tokens = tokens; pd.split_len = sp.len; pd.partial = partial;
@@ -944,7 +947,7 @@ struct Runner {
     // fp32, or fewer than 64 tokens
     using TS = TSG<T>;
     constexpr int SM = AsyncPipe<T, 2>::BYTES;
-    const Split sp = choose_split_async(tokens, P.tiles * 3 * d.b, P.nsplit_max, add_out != nullptr);
+    const Split sp = choose_split_async(tokens, P.tiles * 3 * d.b, P.nsplit_max);
     direct = add_out && sp.n == 1;
     if (direct) { p.add_out = add_out; p.add_in = coeff != 0.f ? add_in : nullptr; p.coeff = coeff; }
     p.tokens = tokens; p.split_len = sp.len; p.partial = partial;
@@ -954,6 +957,7 @@ struct Runner {
     return direct ? 0 : sp.n;
   }
 
+  Partials partials(size_t buffer, int n) const { return Partials{scr<float>(buffer), n, (long long)P.mat3}; }
   RenormParams renorm_params(int u, int ver_prev) const {
     RenormParams p;
     memset(&p, 0, sizeof(p));
@@ -1006,7 +1010,7 @@ struct Runner {
       int u0 = P.state_in ? 0 : 1, ui = 0, n = 0;
       MomentumMeanRanges r;
       auto flush = [&]() {
-        if (n > 0) LACT_LAUNCH("k_momentum_mean", "k_momentum_mean", 0.0, k_momentum_mean, dim3(d.b, n), dim3(256), s, mom, (long long)d.kv_len, r, mbar(u0));
+        if (n > 0) LACT_LAUNCH("k_momentum_mean", "k_momentum_mean", 0.0, k_momentum_mean, dim3(d.b, n), dim3(1024), s, mom, (long long)d.kv_len, r, mbar(u0));
         u0 += n; n = 0;
       };
       for (const auto& st : P.live) {
@@ -1129,14 +1133,14 @@ struct Runner {
       }
       const bool prep_folded = dw_slots < 0;
       const int ss_parts = prep_folded ? tr_tiles(d.d, d.dh) : P.nblk;
-      if (!prep_folded) {
+      if (P.muon && !prep_folded) {
         MomentumPrepParams p;
         memset(&p, 0, sizeof(p));
-        p.g = P.g; p.partial = scr<float>(P.t_partial); p.nsplit = dw_slots;
+        p.g = P.g; p.dw = partials(P.t_partial, dw_slots);
         p.m_prev = mprev(u);
         p.mbar = has_prev(u) ? mbar(u) : nullptr;
         p.d_out = d_unread ? nullptr : dsave(u);
-        p.g16 = P.muon ? g16(u) : nullptr;
+        p.g16 = g16(u);
         p.ss_part = scr<float>(P.t_ss);
         p.round_partial_bf16 = P.bf16;
         if (u + 1 == P.nupd && P.momentum && m_out)
@@ -1211,6 +1215,15 @@ struct Runner {
       }
       {
         RenormParams p = renorm_params(u, ver);
+        if (!P.muon) {
+          p.dw = partials(P.t_partial, dw_slots);
+          p.round_dw_bf16 = P.bf16;
+          p.m_prev = mprev(u);
+          p.mbar = has_prev(u) ? mbar(u) : nullptr;
+          p.d_out = dsave(u);
+          if (u + 1 == P.nupd && P.momentum && m_out)
+            for (int j = 0; j < 3; ++j) p.m_ext[j] = m_out[j];
+        }
         p.main_out = d.prenorm ? main_(u + 1) : nullptr;
         // the fp32 copy of a weight version is the base of the next update (and of its backward): the last one has none
         // (with fp32 activations it is also what the apply steps read)
@@ -1303,14 +1316,28 @@ struct Runner {
     float* gwcur = scr<float>(P.t_gwcur);
     float* gn0 = scr<float>(P.t_gn0);
     float* gmcarry = scr<float>(P.t_gmcarry);
-    float* partial = scr<float>(P.t_partial);
     const long long gn0_n = (long long)3 * d.b * P.g.maxrows();
     // gn0 is written (not added to) by the first renorm backward; without any update the final kernel reads zeros
     bool gn0_written = false;
     if (P.nupd == 0) LACT_LAUNCH("k_fill_f32", "k_fill_f32", 0.0, k_fill_f32, dim3((unsigned)((gn0_n + 255) / 256)), dim3(256), s, gn0, 0.f, gn0_n);
-    // gwcur: gradient w.r.t. the current weight version; "not valid" stands for zero (nothing written yet)
-    bool gw_valid = dwf && (dwf[0] || dwf[1] || dwf[2]);
-    if (gw_valid) LACT_LAUNCH("k_pack3", "k_pack3", 0.0, k_pack3, eg, dim3(256), s, gwcur, P.g.elems, d.b, dwf[0], dwf[1], dwf[2]);
+    // gradient w.r.t. the current weight version: a full array plus partial sums that its reader (the renorm backward, the final
+    // kernel) adds up; nothing of either stands for zero
+    struct GradSum {
+      const float* base = nullptr; int n = 0;
+      bool any() const { return base || n; }
+    } gw;
+    // another contribution to `g`, on the current stream; `buf`: where a full array of it goes
+    auto contribute = [&](const char* site, const TokenReduceJob (&jobs)[3], int tokens, GradSum& g, float* buf, RowCompanions* rows) {
+      if (g.n)   // the partial-sum buffer is taken
+        LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, buf, g.base, 1.f, scr<float>(partial_sel), g.n, (long long)P.mat3);
+      if (g.n) g = GradSum{buf, 0};
+      const int n = token_reduce(site, jobs, tokens, buf, g.base, g.base ? 1.f : 0.f, nullptr, rows);
+      g = n ? GradSum{g.base, n} : GradSum{buf, 0};
+    };
+    if (dwf && (dwf[0] || dwf[1] || dwf[2])) {
+      gw.base = gwcur;
+      LACT_LAUNCH("k_pack3", "k_pack3", 0.0, k_pack3, eg, dim3(256), s, gwcur, P.g.elems, d.b, dwf[0], dwf[1], dwf[2]);
+    }
     // every gradient output is written in full by this call: rows that no step touches are zeroed here.
     // Rows of dq, dk, dv and of the per-token arrays that no step writes are disjoint from everything the steps
     // write: nothing waits for them, and they are cleared on the side stream -- unless ranges overlap partially,
@@ -1374,7 +1401,7 @@ struct Runner {
     // the final kernel); `free_ev` orders the reuse of a gw_side buffer after its consumer.
     wait_for(s_side, s_main);
     float* gw_side[2] = {scr<float>(P.t_gwside[0]), scr<float>(P.t_gwside[1])};
-    bool side_valid[2] = {false, false};
+    GradSum side_sum[2];
     hipEvent_t free_ev[2] = {nullptr, nullptr};
     hipEvent_t dw_done[2] = {nullptr, nullptr};   // newest weight-gradient kernel of the apply steps per buffer
     bool side_used = false;
@@ -1384,16 +1411,6 @@ struct Runner {
       if (main_dq_ev) (void)hipStreamWaitEvent(s_main, main_dq_ev, 0);
       main_dq_ev = nullptr;
     };
-    // dk, dv and the learning-rate gradients of an update: nothing in the call waits for them, so they run on the
-    // tail stream beside the rest of the chain.  They read the chain's token-major intermediates, the compute-type
-    // gradient copy and the row partials: the chain waits for `tail_ev` before it writes any of those again.
-    hipEvent_t tail_ev = nullptr;
-    bool tail_used = false;
-    auto wait_tail = [&]() {
-      if (tail_ev) (void)hipStreamWaitEvent(s_main, tail_ev, 0);
-      tail_ev = nullptr;
-    };
-    float* partial_side = scr<float>(P.t_partial_side);
     int ver = P.nupd, u = P.nupd;
     int carry_main = -1;       // index of the gwhat buffer holding the accumulator's gradient (pre-norm)
     bool gm_valid = false;     // gmcarry holds d loss / d (momentum state after update u-1)
@@ -1426,16 +1443,13 @@ struct Runner {
           // so they stay on the caller's stream (no event hand-over in the critical path); only dq, which nothing
           // waits for, goes to the side stream and reads this chain's intermediates.
           wait_main_dq();
-          wait_tail();
           HiddenParams hp = hidden_params(T_, qc, d.q_ld, d.q_bs, gc, d.do_ld, d.do_bs, ver);
           hp.O0 = h(0); hp.O1 = h(1); hp.O2 = h(2);
           launch_hidden(2, hp, ver, T_);
           wait_for(s_side, s_main);
           TokenReduceJob jobs[3];
           dw_jobs(jobs);
-          if (const int ns_ = token_reduce("apply_bwd_dw", jobs, T_, gwcur, gwcur, gw_valid ? 1.f : 0.f))
-            LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, gwcur, gw_valid ? gwcur : nullptr, 1.f, partial, ns_, (long long)P.mat3);
-          gw_valid = true;
+          contribute("apply_bwd_dw", jobs, T_, gw, gwcur, nullptr);
           s = s_side;
           dq_gemm();
           s = s_main;
@@ -1447,20 +1461,18 @@ struct Runner {
           continue;
         }
         const int sb = ver & 1;
-        if (!side_valid[sb] && free_ev[sb] && s_side != s_main) {
+        if (!side_sum[sb].any() && free_ev[sb] && s_side != s_main) {
           (void)hipStreamWaitEvent(s_side, free_ev[sb], 0);
           free_ev[sb] = nullptr;
         }
         side_used = true;
-        OnSide on_side(*this);
+        OnSide on_side(*this, sb);
         HiddenParams hp = hidden_params(T_, qc, d.q_ld, d.q_bs, gc, d.do_ld, d.do_bs, ver);
         hp.O0 = h(0); hp.O1 = h(1); hp.O2 = h(2);
         launch_hidden(2, hp, ver, T_);
         TokenReduceJob jobs[3];
         dw_jobs(jobs);
-        if (const int ns_ = token_reduce("apply_bwd_dw", jobs, T_, gw_side[sb], gw_side[sb], side_valid[sb] ? 1.f : 0.f))
-          LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, gw_side[sb], side_valid[sb] ? gw_side[sb] : nullptr, 1.f, partial_side, ns_, (long long)P.mat3);
-        side_valid[sb] = true;
+        contribute("apply_bwd_dw", jobs, T_, side_sum[sb], gw_side[sb], nullptr);
         dw_done[sb] = side ? side->event() : nullptr;
         if (dw_done[sb] && s_side != s_main) (void)hipEventRecord(dw_done[sb], s_side);
         dq_gemm();
@@ -1471,25 +1483,38 @@ struct Runner {
       const int vprev = ver - 1;
       const int gw_idx = carry_main == 0 ? 1 : 0;
       float* gwhat = scr<float>(P.t_gwhat[gw_idx]);
+      const bool carry_here = P.momentum && (u > 0 || gm_valid);
+      const size_t mslot = (size_t)3 * d.b * P.mdot_parts;   // partial momentum dots of one update
       int cur = 0;  // which gxf/gxb buffer holds the running Newton-Schulz gradient
       {
         RenormParams p = renorm_params(u, vprev);
-        p.gy = gw_valid ? gwcur : nullptr;
+        p.gy = gw.base;
+        p.gyp = partials(P.t_partial, gw.n);
         const int sb = ver & 1;
-        if (side_valid[sb]) {
+        if (side_sum[sb].any()) {
           // wait for the apply steps' weight gradients only (their dq GEMMs may still be running)
           if (dw_done[sb] && s_side != s_main) (void)hipStreamWaitEvent(s_main, dw_done[sb], 0);
-          p.gy2 = gw_side[sb];
+          p.gy2 = side_sum[sb].base;
+          p.gyp2 = partials(P.t_partial_side[sb], side_sum[sb].n);
         }
         p.carry_in = (d.prenorm && carry_main >= 0) ? scr<float>(P.t_gwhat[carry_main]) : nullptr;
         p.gw_hat = gwhat;
         p.gn0 = gn0; p.gn0_init = !gn0_written;
         gn0_written = true;
         p.clear = ns_clear(false);
-        if (P.muon) { p.gxf = scr<float>(P.t_gxf[0]); p.gxb = scr<TN>(P.t_gxb[0]); }
-        LACT_LAUNCH("k_renorm_bwd", "k_renorm_bwd", 0.0, (k_renorm_bwd<TN>), rowgrid, dim3(256), s, p);
-        if (side_valid[sb]) {
-          side_valid[sb] = false;
+        if (P.muon) {
+          p.gxf = scr<float>(P.t_gxf[0]); p.gxb = scr<TN>(P.t_gxb[0]);
+        } else {
+          p.gc = scr<T>(P.t_gc);
+          p.gm_carry = carry_here ? gmcarry : nullptr; p.carry_valid = gm_valid; p.carry_write = u > 0;
+          if (P.momentum && u > 0) {
+            p.m_prev = dsave(u - 1); p.mbar = mbar(u);
+            p.mdot_part = scr<float>(P.t_mdot) + (size_t)u * mslot;
+          }
+        }
+        LACT_LAUNCH("k_renorm_bwd", "k_renorm_bwd", 0.0, (k_renorm_bwd<T, TN>), rowgrid, dim3(256), s, p);
+        if (side_sum[sb].any()) {
+          side_sum[sb] = GradSum();
           if (side) {
             free_ev[sb] = side->event();
             (void)hipEventRecord(free_ev[sb], s_main);
@@ -1501,12 +1526,9 @@ struct Runner {
       // (one batch, every matrix fused); the gradient in the compute type too when nothing else enters it (no
       // momentum state to carry, no raw-gradient term) and every matrix is held as it lies (square shapes).
       const bool dot_in_kernel = ns_all_fused() && P.nsb.size() == 1;
-      const bool carry_here = P.momentum && (u > 0 || gm_valid);
       const bool prep_in_kernel = dot_in_kernel && kBf16 && !(P.muon && d.muon_replaces_weight) &&
                                   P.g.x_contiguous(0) && P.g.x_contiguous(1) && P.g.x_contiguous(2);
-      const size_t mslot = (size_t)3 * d.b * std::max(P.nblk, 256);   // partial momentum dots of one update
       if (P.muon) {
-        if (prep_in_kernel) wait_tail();   // the previous update's dk GEMM reads the gradient copy the fused kernel writes
         for (const NsBatch& B : P.nsb) {
           const int n = B.n, r = B.r, c = B.c;
           const long long xe = (long long)r * c, se = (long long)r * r;
@@ -1590,27 +1612,26 @@ struct Runner {
           LACT_LAUNCH("k_ns_bwd_dot", "k_ns_bwd_dot", 0.0, (k_ns_bwd_dot<TN>), dim3(P.nblk, P.g.ns_count()), dim3(256), s, dp);
         }
       }
-      if (!(P.muon && prep_in_kernel)) {
-        wait_tail();   // the previous update's dk GEMM reads the gradient copy written here
+      if (P.muon && !prep_in_kernel) {
         GradPrepParams p;
         memset(&p, 0, sizeof(p));
-        p.g = P.g; p.muon = P.muon;
-        p.gx0 = scr<float>(P.t_gxf[cur]); p.g16 = P.muon ? (const void*)g16(u) : nullptr; p.norms = norms(u);
-        p.dot_part = scr<float>(P.t_dot); p.nparts = (P.muon && (dot_in_kernel || ns_dot_by_tiles())) ? ns_fused_nbm(P.nsb[0]) : P.nblk;
-        p.gw_hat = gwhat; p.cr = (P.muon && d.muon_replaces_weight) ? 1.f : 0.f;
-        p.gm_carry = (P.momentum && (u > 0 || gm_valid)) ? gmcarry : nullptr; p.carry_valid = gm_valid;
+        p.g = P.g;
+        p.gx0 = scr<float>(P.t_gxf[cur]); p.g16 = g16(u); p.norms = norms(u);
+        p.dot_part = scr<float>(P.t_dot); p.nparts = (dot_in_kernel || ns_dot_by_tiles()) ? ns_fused_nbm(P.nsb[0]) : P.nblk;
+        p.gw_hat = gwhat; p.cr = d.muon_replaces_weight ? 1.f : 0.f;
+        p.gm_carry = carry_here ? gmcarry : nullptr; p.carry_valid = gm_valid;
         p.carry_write = u > 0;
         p.m_prev = (P.momentum && u > 0) ? dsave(u - 1) : nullptr;
         p.mbar = (P.momentum && u > 0) ? mbar(u) : nullptr;
         p.gc = scr<T>(P.t_gc);
         p.mdot_part = scr<float>(P.t_mdot) + (size_t)u * mslot;
-        if (P.muon && ns_fused_any()) p.poison = ns_error_word();
+        if (ns_fused_any()) p.poison = ns_error_word();
         LACT_LAUNCH("k_grad_prep", "k_grad_prep", 0.0, (k_grad_prep<T, TN>), dim3(P.nblk, 3 * d.b), dim3(256), s, p);
       }
       if (P.momentum) {
         gm_valid = true;
-        // partial momentum dots per matrix: one per block of k_grad_prep, or one per tile of the fused kernel
-        mg_parts = (P.muon && prep_in_kernel) ? ns_fused_nbm(P.nsb[0]) : P.nblk;
+        // partial momentum dots per matrix: one per block of the kernel that formed them, or one per tile of the fused kernel
+        mg_parts = !P.muon ? (int)rowgrid.x : prep_in_kernel ? ns_fused_nbm(P.nsb[0]) : P.nblk;
         // the gradient of the per-token momentum needs these dot products only: written by one launch at the end
         // (by one launch per update, in this order, when token ranges repeat and their shares add up)
         if (u > 0) {
@@ -1647,28 +1668,13 @@ struct Runner {
           z0 = pre(u, 0); z1 = pre(u, 1); z2 = pre(u, 2); zbs = pre_bs(u);
         }
         wait_main_dq();
-        wait_tail();
         launch_hidden(P.keep_pre ? 4 : 3, hp, vprev, T_);
       }
       const bool acc_kv = seen_kv.accumulate(st.start, st.end);
-      // worth a hand-over only when an earlier update's chain follows on the caller's stream
-      // ... unless the token reduction of this update leaves most of the chip idle: then the GEMMs are worth more
-      // inside its launch (below) than beside the chain (config 2, 48 reduction blocks: -1.4 %; config 4, 216: +1 %)
-      bool lone_reduction = false;
-      if constexpr (kBf16)
-        {
-          const int tiles = tr_tiles(d.d, d.dh) * 3 * d.b;
-          lone_reduction = tiles * choose_split(T_, tiles, P.nsplit_max).n < 160;
-        }
-      const bool use_tail = s_tail != s_main && u > 0 && !lone_reduction;
-      if (use_tail) {
-        wait_for(s_tail, s_main);
-        s = s_tail;
-      }
-      // without that hand-over the two GEMMs share the launch of the token reduction below (when it runs on the
-      // asynchronous-copy kernel; otherwise they are launched after it)
+      // dk and dv share the launch of the token reduction below (when it runs on the asynchronous-copy kernel; otherwise they are
+      // launched after it).  Measured against a stream of their own beside the rest of the chain: 2.32 against 2.45 ms with 216
+      // reduction blocks per update, 2.87 against 3.12 ms with 48; the hand-over costs more than what they fill.
       RowCompanions rows_job;
-      const bool rows_ride = !use_tail && kBf16;
       {  // dk = (dgate*lr0) G0 + (dh2*lr2) G2 + gG W0 + gH2 W2
         auto p = row_params<4>();
         set_term(p.t[0], z0, d.dh, zbs, g0, d.d, P.g.elems, d.dh);
@@ -1677,7 +1683,6 @@ struct Runner {
         set_term(p.t[3], h(2), d.dh, hbs(), wc(vprev, 2), d.d, P.g.elems, d.dh);
         p.M = T_; p.N = d.d; p.out = dk + (size_t)st.start * d.d; p.ldo = d.d; p.bso = (long long)d.kv_len * d.d;
         p.accumulate = acc_kv;
-        if (use_tail || !kBf16) launch_row_gemm<T, false, 4, EPI_STORE>("update_bwd_dk", p, d.b, s, true);
         rows_job.r4 = p;
       }
       {  // dv = (hidden*lr1) G1^T + gDH W1^T
@@ -1686,7 +1691,6 @@ struct Runner {
         set_term(p.t[1], h(1), d.dh, hbs(), wc(vprev, 1), d.dh, P.g.elems, d.dh);
         p.M = T_; p.N = d.d; p.out = dv + (size_t)st.start * d.d; p.ldo = d.d; p.bso = (long long)d.kv_len * d.d;
         p.accumulate = acc_kv;
-        if (use_tail || !kBf16) launch_row_gemm<T, true, 2, EPI_STORE>("update_bwd_dv", p, d.b, s, true);
         rows_job.r2 = p;
       }
       // learning-rate gradients: row partials of every update kept, one reduction launch at the end (one launch per
@@ -1700,12 +1704,6 @@ struct Runner {
       } else {
         lr_ranges.emplace_back(st.start, T_);
       }
-      if (use_tail) {
-        s = s_main;
-        tail_ev = side->event();
-        (void)hipEventRecord(tail_ev, s_tail);
-        tail_used = true;
-      }
       {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));
@@ -1716,12 +1714,10 @@ struct Runner {
         set_tr_term(jobs[1].t[0], vc, d.v_ld, d.v_bs, h(1), d.dh, hbs());
         jobs[2].M = d.dh; jobs[2].N = d.d;
         set_tr_term(jobs[2].t[0], h(2), d.dh, hbs(), kc, d.k_ld, d.k_bs);
-        const float pass = d.prenorm ? 0.f : ((P.muon && d.muon_replaces_weight) ? 0.f : 1.f);
-        if (const int ns_ = token_reduce(rows_ride ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gwcur, gwhat, pass, nullptr,
-                                         rows_ride ? &rows_job : nullptr))
-          LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, gwcur, pass != 0.f ? gwhat : nullptr, pass, partial, ns_, (long long)P.mat3);
-        gw_valid = true;
-        if (rows_ride && !rows_job.done) {
+        // the update before: its weights enter these as they are, unless Newton-Schulz output replaces them or an accumulator carries on
+        gw = GradSum{(d.prenorm || (P.muon && d.muon_replaces_weight)) ? nullptr : gwhat, 0};
+        contribute(kBf16 ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, gwcur, &rows_job);
+        if (!rows_job.done) {
           launch_row_gemm<T, false, 4, EPI_STORE>("update_bwd_dk", rows_job.r4, d.b, s, true);
           launch_row_gemm<T, true, 2, EPI_STORE>("update_bwd_dv", rows_job.r2, d.b, s, true);
         }
@@ -1745,7 +1741,7 @@ struct Runner {
     }
     if (!mg_updates.empty()) {
       // deferred updates are all updates but the first, met in descending order: slot u - 1 of the launch is update u
-      const size_t slot = (size_t)3 * d.b * std::max(P.nblk, 256);
+      const size_t slot = (size_t)3 * d.b * P.mdot_parts;
       const int total = (int)mg_updates.size();
       for (int i0 = 0; i0 < total; i0 += 256) {
         const int n = std::min(256, total - i0);
@@ -1761,10 +1757,10 @@ struct Runner {
     }
     {
       FinishParams p;
+      memset(&p, 0, sizeof(p));
       if (side_used) wait_for(s_main, s_side);
-      if (tail_used) wait_tail();
-      p.g = P.g; p.gw = gw_valid ? gwcur : nullptr;
-      p.gw2 = side_valid[0] ? gw_side[0] : nullptr;
+      p.g = P.g; p.gw = gw.base; p.gwp = partials(P.t_partial, gw.n);
+      p.gw2 = side_sum[0].base; p.gwp2 = partials(P.t_partial_side[0], side_sum[0].n);
       p.carry = (d.prenorm && carry_main >= 0) ? scr<float>(P.t_gwhat[carry_main]) : nullptr;
       p.gn0 = gn0; p.n0 = n0(); p.w_init = wf(0);
       p.through_norms = d.detach_norms ? 0 : 1;
@@ -1816,7 +1812,7 @@ int newton_schulz_t(int32_t n, int32_t rows, int32_t cols, const float* gin, flo
   // MatGeom treats index 0 as [dh, d] = [rows, cols]; launch with grid.y = n so z / nb == 0 throughout.
   MomentumPrepParams mp;
   memset(&mp, 0, sizeof(mp));
-  mp.g = P.g; mp.partial = gin; mp.nsplit = 1; mp.d_out = reinterpret_cast<float*>(ws + P.o_xf[1]);
+  mp.g = P.g; mp.dw = Partials{gin, 1, 0}; mp.d_out = reinterpret_cast<float*>(ws + P.o_xf[1]);
   mp.g16 = ws + P.o_g16; mp.ss_part = reinterpret_cast<float*>(ws + P.o_ss);
   // partial is indexed [s][3*nb][elems] with z < nb: the layout of gin ([n][elems]) matches for s = 0
   LACT_LAUNCH("k_momentum_prep", "k_momentum_prep", 0.0, (k_momentum_prep<TN>), dim3(P.nblk, n), dim3(256), s, mp);
@@ -1877,7 +1873,7 @@ int newton_schulz_bwd_t(int32_t n, int32_t rows, int32_t cols, const float* gin,
   // ---- forward again, keeping X_k, A_k, B_k
   MomentumPrepParams mp;
   memset(&mp, 0, sizeof(mp));
-  mp.g = F.g; mp.partial = gin; mp.nsplit = 1; mp.d_out = nullptr;
+  mp.g = F.g; mp.dw = Partials{gin, 1, 0}; mp.d_out = nullptr;
   mp.g16 = ws + F.o_g16; mp.ss_part = reinterpret_cast<float*>(ws + F.o_ss);
   LACT_LAUNCH("k_momentum_prep", "k_momentum_prep", 0.0, (k_momentum_prep<TN>), dim3(F.nblk, n), dim3(256), s, mp);
   NsScaleParams sp;
@@ -1950,7 +1946,7 @@ int newton_schulz_bwd_t(int32_t n, int32_t rows, int32_t cols, const float* gin,
   LACT_LAUNCH("k_ns_bwd_dot", "k_ns_bwd_dot", 0.0, (k_ns_bwd_dot<TN>), dim3(F.nblk, n), dim3(256), s, dp);
   GradPrepParams gp;
   memset(&gp, 0, sizeof(gp));
-  gp.g = F.g; gp.muon = 1; gp.gx0 = gxf[bc]; gp.g16 = ws + F.o_g16; gp.norms = reinterpret_cast<float*>(ws + F.o_norm);
+  gp.g = F.g; gp.gx0 = gxf[bc]; gp.g16 = ws + F.o_g16; gp.norms = reinterpret_cast<float*>(ws + F.o_norm);
   gp.dot_part = dp.dot_part; gp.nparts = F.nblk; gp.gc = dg;
   LACT_LAUNCH("k_grad_prep", "k_grad_prep", 0.0, (k_grad_prep<float, TN>), dim3(F.nblk, n), dim3(256), s, gp);
   LACT_CHECK_LAUNCH();

@@ -158,9 +158,37 @@ __global__ void k_momentum_mean(const float* mom, long long bs, const MomentumMe
 }
 
 // ---- reduce split partials, add momentum, emit the bf16 Newton-Schulz input ---------------------
+// Partial sums of a token reduction that was split over the tokens: n slots of `stride` elements, added in this order.
+struct Partials {
+  const float* p; int n; long long stride;
+};
+__device__ __forceinline__ void add_partials(float4& v, const Partials& q, size_t off) {
+  for (int i = 0; i < q.n; ++i) {
+    const float4 t = ld4(q.p + i * q.stride + off);
+    v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
+  }
+}
+
+// The gradient of an update: the sum of its partial sums (at least one), rounded as the reference's bf16 GEMM result if asked, plus
+// the earlier momentum state weighted by mb (or m_prev null).
+__device__ __forceinline__ float4 momentum4(const Partials& q, size_t off, int round, const float* m_prev, float mb) {
+  float4 v = ld4(q.p + off);
+  for (int i = 1; i < q.n; ++i) {
+    const float4 t = ld4(q.p + i * q.stride + off);
+    v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
+  }
+  if (round) v = f4(round_bf16(v.x), round_bf16(v.y), round_bf16(v.z), round_bf16(v.w));
+  if (m_prev) {
+    const float4 m = ld4(m_prev + off);
+    // product and sum rounded separately, as the reference's two tensor operations are (ttt_operation.py:174-176)
+    v.x = __fadd_rn(v.x, __fmul_rn(m.x, mb)); v.y = __fadd_rn(v.y, __fmul_rn(m.y, mb));
+    v.z = __fadd_rn(v.z, __fmul_rn(m.z, mb)); v.w = __fadd_rn(v.w, __fmul_rn(m.w, mb));
+  }
+  return v;
+}
 struct MomentumPrepParams {
   MatGeom g;
-  const float* partial; int nsplit;   // [nsplit][3b][elems]
+  Partials dw;                        // each [3b][elems]
   const float* m_prev;                // [3b][elems] or null (no momentum / first update uses zeros)
   const float* mbar;                  // [b] or null
   float* d_out;                       // [3b][elems]  dw (+ momentum): new momentum state, pre-Muon gradient (null: nothing reads it)
@@ -177,24 +205,13 @@ __global__ void k_momentum_prep(const MomentumPrepParams p) {
   clear_words(p.clear, blockIdx.x == 0 && blockIdx.y == 0);
   const FlatRange R(p.g.elems);
   const float mb = (p.m_prev && p.mbar) ? p.mbar[ib] : 0.f;
-  const size_t zo = (size_t)z * p.g.elems, stride = (size_t)3 * p.g.nb * p.g.elems;
+  const size_t zo = (size_t)z * p.g.elems;
   float* ext = p.m_ext[j] ? p.m_ext[j] + (size_t)ib * p.g.elems : nullptr;
   const bool contiguous = p.g.x_contiguous(j);
   const size_t xo = p.g.ns_base(p.g.ns_of(z));
   float ss = 0.f;
   for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
-    float4 v = ld4(p.partial + zo + e);
-    for (int s = 1; s < p.nsplit; ++s) {
-      const float4 t = ld4(p.partial + s * stride + zo + e);
-      v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
-    }
-    if (p.round_partial_bf16) v = f4(round_bf16(v.x), round_bf16(v.y), round_bf16(v.z), round_bf16(v.w));
-    if (p.m_prev) {
-      const float4 m = ld4(p.m_prev + zo + e);
-      // product and sum rounded separately, as the reference's two tensor operations are (ttt_operation.py:174-176)
-      v.x = __fadd_rn(v.x, __fmul_rn(m.x, mb)); v.y = __fadd_rn(v.y, __fmul_rn(m.y, mb));
-      v.z = __fadd_rn(v.z, __fmul_rn(m.z, mb)); v.w = __fadd_rn(v.w, __fmul_rn(m.w, mb));
-    }
+    const float4 v = momentum4(p.dw, zo + e, p.round_partial_bf16, p.m_prev, mb);
     if (p.d_out) st4(p.d_out + zo + e, v);
     if (ext) st4(ext + e, v);
     if (p.g16) {
@@ -280,19 +297,30 @@ struct RenormParams {
   float* wf_out; void* wc_out;     // new weights: fp32 state and compute-type copy (each may be null)
   float* w_ext[3];                 // caller's weight outputs [b][elems] (same values as wf_out), each nullable
   const unsigned* poison;          // nonzero word: an earlier kernel of this step failed (barrier timeout) -> results become NaN
+  // Without Newton-Schulz `u` is the (momentum) gradient itself: k_update_renorm then takes it from the token reduction's partial
+  // sums and does the momentum step on the way (what k_momentum_prep does where a Newton-Schulz iteration follows)
+  Partials dw;                     // partial sums of the gradient, or none: `u` is read
+  int round_dw_bf16;               // the reduction GEMM's result is a bf16 tensor in the reference
+  const float* m_prev; const float* mbar;   // momentum state before this update and [b] mean momentum, or null
+  float* d_out;                    // the gradient with its momentum (= new momentum state), written
+  float* m_ext[3];                 // caller's momentum outputs, each nullable
   // backward only
   const float* gy;                 // gradient w.r.t. the new weights, or null (= zero)
   const float* gy2;                // second addend of the same gradient (the apply steps' share), or null
+  Partials gyp, gyp2;              // more of it, as partial sums of token reductions
   const float* carry_in;           // gradient arriving at the accumulator from later steps (pre-norm) or null
   float* gw_hat;                   // gradient w.r.t. w_hat, original orientation
   float* gn0;                      // [3b][maxrows], accumulated (written when gn0_init: first use in a backward pass)
   int gn0_init;
   ClearWords clear;
   float* gxf; void* gxb;           // the same gradient in Newton-Schulz orientation (fp32 + Newton-Schulz type) or null
+  // Without Newton-Schulz the gradient w.r.t. w_hat is the one w.r.t. the update: its momentum step right here
+  void* gc;                        // compute-type copy of d loss / d dw (GEMM operand), or null
+  float* gm_carry; int carry_valid, carry_write;   // as in GradPrepParams
+  float* mdot_part;                // [3b][gridDim.x] partial <g, m_prev>
 };
-// off: offset in the packed arrays; uo: offset of the same element in `u`
-__device__ __forceinline__ float4 renorm_w_hat4(const RenormParams& p, size_t off, size_t uo) {
-  float4 v = ld4(p.u + uo);
+// off: offset in the packed arrays; v: the element of `u`
+__device__ __forceinline__ float4 renorm_w_hat4(const RenormParams& p, size_t off, float4 v) {
   if (p.cw != 0.f) {
     const float4 b = ld4(p.base + off);
     v.x += p.cw * b.x; v.y += p.cw * b.y; v.z += p.cw * b.z; v.w += p.cw * b.w;
@@ -303,8 +331,12 @@ __device__ __forceinline__ float4 renorm_w_hat4(const RenormParams& p, size_t of
   }
   return v;
 }
+// uo: offset of the same element in `u`
+__device__ __forceinline__ float4 renorm_w_hat4(const RenormParams& p, size_t off, size_t uo) { return renorm_w_hat4(p, off, ld4(p.u + uo)); }
 __device__ __forceinline__ float4 renorm_gy4(const RenormParams& p, size_t off) {
   float4 g = p.gy ? ld4(p.gy + off) : f4(0.f, 0.f, 0.f, 0.f);
+  add_partials(g, p.gyp, off);
+  add_partials(g, p.gyp2, off);
   if (p.gy2) {
     const float4 t = ld4(p.gy2 + off);
     g.x += t.x; g.y += t.y; g.z += t.z; g.w += t.w;
@@ -312,6 +344,8 @@ __device__ __forceinline__ float4 renorm_gy4(const RenormParams& p, size_t off) 
   return g;
 }
 constexpr int ROW_VEC_MAX = 4;   // a lane keeps up to 4 x 4 elements of its row in registers (rows up to 1024 columns)
+// One wave per row.  Bound by memory: with the momentum step inside, 12 matrices of 384 x 384 take 9.3 us from one partial sum
+// (39 MB, 4.2 TB/s) and 10.1 us from two; as two kernels they took 8.2 + 5.8 us.
 template <typename T>
 __global__ void k_update_renorm(const RenormParams p) {
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
@@ -322,18 +356,27 @@ __global__ void k_update_renorm(const RenormParams p) {
   const size_t uo = (p.u_stacked ? (size_t)p.g.u_off(z) : (size_t)z * p.g.elems) + (size_t)row * cols;
   float* ext = p.w_ext[j] ? p.w_ext[j] + (size_t)ib * p.g.elems + (size_t)row * cols : nullptr;
   const bool keep = cols <= 256 * ROW_VEC_MAX;
+  const float mb = (p.m_prev && p.mbar) ? p.mbar[ib] : 0.f;
+  float* mext = p.m_ext[j] ? p.m_ext[j] + (size_t)ib * p.g.elems + (size_t)row * cols : nullptr;
+  auto w_hat = [&](int c) {   // first visit of an element (a later one finds `u` = d_out in memory)
+    if (p.dw.n == 0) return renorm_w_hat4(p, o + c, uo + c);
+    const float4 m = momentum4(p.dw, o + c, p.round_dw_bf16, p.m_prev, mb);
+    st4(p.d_out + o + c, m);
+    if (mext) st4(mext + c, m);
+    return renorm_w_hat4(p, o + c, m);
+  };
   float4 vv[ROW_VEC_MAX];
   float ss = 0.f;
 #pragma unroll
   for (int i = 0; i < ROW_VEC_MAX; ++i) {
     const int c = lane * 4 + i * 256;
     if (c < cols) {
-      vv[i] = renorm_w_hat4(p, o + c, uo + c);
+      vv[i] = w_hat(c);
       ss += dot4(vv[i], vv[i]);
     }
   }
   for (int c = lane * 4 + ROW_VEC_MAX * 256; c < cols; c += 256) {
-    const float4 v = renorm_w_hat4(p, o + c, uo + c);
+    const float4 v = w_hat(c);
     ss += dot4(v, v);
   }
   ss = wave_sum(ss);
@@ -360,23 +403,30 @@ __global__ void k_update_renorm(const RenormParams p) {
 
 // backward of the line above.  y = w_hat*n0/(r+eps), r = ||w_hat||:
 //   g_w_hat = gy*n0/(r+eps) - w_hat * <gy,w_hat> * n0 / (r (r+eps)^2),   g_n0 = <gy,w_hat>/(r+eps)
-template <typename TN>
+// One wave per row, bound by memory: 14.9 us for 12 matrices of 384 x 384 with the momentum step's backward inside, 10.7 + 11.8 us
+// as two kernels.  T: compute type of gc.
+template <typename T, typename TN>
 __global__ void k_renorm_bwd(const RenormParams p) {
+  __shared__ float red[16];
   const int z = blockIdx.y, j = z / p.g.nb;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   clear_words(p.clear, blockIdx.x == 0 && blockIdx.y == 0);
-  if (row >= p.g.rows(j)) return;
-  const int cols = p.g.cols(j);
+  // rows past the matrix take no part but in the block's sum of <g, m_prev>
+  const bool valid = row < p.g.rows(j);
+  if (!valid && !p.mdot_part) return;
+  const int cols = valid ? p.g.cols(j) : 0, ib = z % p.g.nb;
+  const float mb = p.mbar ? p.mbar[ib] : 0.f;
+  float md = 0.f;
   const size_t o = (size_t)z * p.g.elems + (size_t)row * cols;
   const size_t uo = (p.u_stacked ? (size_t)p.g.u_off(z) : (size_t)z * p.g.elems) + (size_t)row * cols;
   const size_t xo = p.g.ns_base(p.g.ns_of(z));
   const bool contiguous = p.g.x_contiguous(j);
   float c0 = 1.f, c1 = 0.f;
   float* gn0 = p.gn0 + (size_t)z * p.g.maxrows() + row;
-  if (!p.weight_norm && p.gn0_init && lane == 0) *gn0 = 0.f;
+  if (!p.weight_norm && p.gn0_init && lane == 0 && valid) *gn0 = 0.f;
   // the first 1024 columns of a row stay in registers between the two passes (as in k_update_renorm)
   float4 wv[ROW_VEC_MAX], gk[ROW_VEC_MAX];
-  if (p.weight_norm) {
+  if (p.weight_norm && valid) {
     float ss = 0.f, dot = 0.f;
 #pragma unroll
     for (int i = 0; i < ROW_VEC_MAX; ++i) {
@@ -385,13 +435,13 @@ __global__ void k_renorm_bwd(const RenormParams p) {
         wv[i] = renorm_w_hat4(p, o + c, uo + c);
         gk[i] = renorm_gy4(p, o + c);
         ss += dot4(wv[i], wv[i]);
-        if (p.gy || p.gy2) dot += dot4(wv[i], gk[i]);
+        dot += dot4(wv[i], gk[i]);
       }
     }
     for (int c = lane * 4 + ROW_VEC_MAX * 256; c < cols; c += 256) {
       const float4 v = renorm_w_hat4(p, o + c, uo + c);
       ss += dot4(v, v);
-      if (p.gy || p.gy2) dot += dot4(v, renorm_gy4(p, o + c));
+      dot += dot4(v, renorm_gy4(p, o + c));
     }
     ss = wave_sum(ss);
     dot = wave_sum(dot);
@@ -418,6 +468,18 @@ __global__ void k_renorm_bwd(const RenormParams p) {
       gv.x += ci.x; gv.y += ci.y; gv.z += ci.z; gv.w += ci.w;
     }
     st4(p.gw_hat + o + c, gv);
+    if (p.gc) {   // no Newton-Schulz in between: momentum and the GEMM operand, as in k_grad_prep
+      float4 g = gv;
+      if (p.gm_carry) {
+        if (p.carry_valid) {
+          const float4 cv = ld4(p.gm_carry + o + c);
+          g.x += cv.x; g.y += cv.y; g.z += cv.z; g.w += cv.w;
+        }
+        if (p.carry_write) st4(p.gm_carry + o + c, f4(g.x * mb, g.y * mb, g.z * mb, g.w * mb));   // d/d M_prev of  dw + M_prev * mbar
+        if (p.m_prev) md += dot4(g, ld4(p.m_prev + o + c));
+      }
+      Elem<T>::store4(reinterpret_cast<T*>(p.gc) + o + c, g.x, g.y, g.z, g.w);
+    }
     if (p.gxf) {   // the same gradient where Newton-Schulz holds this matrix
       const long long e = (long long)row * cols + c;
       if (contiguous) {
@@ -446,6 +508,10 @@ __global__ void k_renorm_bwd(const RenormParams p) {
   }
   for (int c = lane * 4 + ROW_VEC_MAX * 256; c < cols; c += 256)
     emit(c, renorm_gy4(p, o + c), p.weight_norm ? renorm_w_hat4(p, o + c, uo + c) : zero4);
+  if (p.mdot_part) {
+    md = block_sum(md, red);
+    if (threadIdx.x == 0) p.mdot_part[(size_t)z * gridDim.x + blockIdx.x] = md;
+  }
 }
 
 // A gradient given in the original orientation of its matrices, copied to where Newton-Schulz holds them (fp32 and
@@ -505,7 +571,6 @@ __device__ __forceinline__ float ns_input_grad(float gx, float g16, float c0, fl
 
 struct GradPrepParams {
   MatGeom g;
-  int muon;
   const float* gx0; const void* g16; const float* norms; const float* dot_part; int nparts;
   const float* gw_hat; float cr;     // added when the raw gradient also enters w_hat
   float* gm_carry; int carry_valid;  // gradient w.r.t. the momentum state after this update (in/out)
@@ -519,16 +584,13 @@ template <typename T, typename TN>
 __global__ void k_grad_prep(const GradPrepParams p) {
   __shared__ float red[16];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
-  float c0 = 1.f, c1 = 0.f;
-  if (p.muon) {
-    const int m = p.g.ns_of(z);
-    float dot = 0.f;
-    for (int i = 0; i < p.nparts; ++i) dot += p.dot_part[(size_t)m * p.nparts + i];
-    const float n = p.norms[m];
-    c0 = 1.f / (n + 1e-7f);
-    c1 = n > 0.f ? dot / (n * (n + 1e-7f) * (n + 1e-7f)) : 0.f;
-    if (p.poison && *p.poison) c0 = __uint_as_float(0x7fc00000u);
-  }
+  const int m = p.g.ns_of(z);
+  float dot = 0.f;
+  for (int i = 0; i < p.nparts; ++i) dot += p.dot_part[(size_t)m * p.nparts + i];
+  const float n = p.norms[m];
+  float c0 = 1.f / (n + 1e-7f);
+  const float c1 = n > 0.f ? dot / (n * (n + 1e-7f) * (n + 1e-7f)) : 0.f;
+  if (p.poison && *p.poison) c0 = __uint_as_float(0x7fc00000u);
   const float mb = p.mbar ? p.mbar[ib] : 0.f;
   const FlatRange R(p.g.elems);
   const size_t zo = (size_t)z * p.g.elems;
@@ -537,34 +599,29 @@ __global__ void k_grad_prep(const GradPrepParams p) {
   float md = 0.f;
   for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
     const size_t o = zo + e;
-    float4 gv;
-    if (p.muon) {
-      float4 gx;
-      float g[4];
-      if (contiguous) {
-        const size_t x = xo + p.g.xidx(j, e);
-        gx = ld4(p.gx0 + x);
-        Elem<TN>::load4(reinterpret_cast<const TN*>(p.g16) + x, g);
-      } else {
-        float t[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const size_t x = xo + p.g.xidx(j, e + i);
-          t[i] = p.gx0[x];
-          g[i] = Elem<TN>::load(reinterpret_cast<const TN*>(p.g16) + x);
-        }
-        gx = f4(t[0], t[1], t[2], t[3]);
-      }
-      // the gradient that leaves Newton-Schulz through its input cast (G.bfloat16(), ttt_operation.py:45) has that type
-      // (two gradients arrive there, through the quotient and through the norm, :49; each is a tensor of that type, and so is their sum)
-      gv = f4(ns_input_grad<TN>(gx.x, g[0], c0, c1), ns_input_grad<TN>(gx.y, g[1], c0, c1), ns_input_grad<TN>(gx.z, g[2], c0, c1),
-              ns_input_grad<TN>(gx.w, g[3], c0, c1));
-      if (p.cr != 0.f) {
-        const float4 w = ld4(p.gw_hat + o);
-        gv.x += p.cr * w.x; gv.y += p.cr * w.y; gv.z += p.cr * w.z; gv.w += p.cr * w.w;
-      }
+    float4 gx;
+    float g[4];
+    if (contiguous) {
+      const size_t x = xo + p.g.xidx(j, e);
+      gx = ld4(p.gx0 + x);
+      Elem<TN>::load4(reinterpret_cast<const TN*>(p.g16) + x, g);
     } else {
-      gv = ld4(p.gw_hat + o);
+      float t[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const size_t x = xo + p.g.xidx(j, e + i);
+        t[i] = p.gx0[x];
+        g[i] = Elem<TN>::load(reinterpret_cast<const TN*>(p.g16) + x);
+      }
+      gx = f4(t[0], t[1], t[2], t[3]);
+    }
+    // the gradient that leaves Newton-Schulz through its input cast (G.bfloat16(), ttt_operation.py:45) has that type
+    // (two gradients arrive there, through the quotient and through the norm, :49; each is a tensor of that type, and so is their sum)
+    float4 gv = f4(ns_input_grad<TN>(gx.x, g[0], c0, c1), ns_input_grad<TN>(gx.y, g[1], c0, c1), ns_input_grad<TN>(gx.z, g[2], c0, c1),
+            ns_input_grad<TN>(gx.w, g[3], c0, c1));
+    if (p.cr != 0.f) {
+      const float4 w = ld4(p.gw_hat + o);
+      gv.x += p.cr * w.x; gv.y += p.cr * w.y; gv.z += p.cr * w.z; gv.w += p.cr * w.w;
     }
     if (p.gm_carry) {
       if (p.carry_valid) {
@@ -587,13 +644,13 @@ __global__ void k_grad_prep(const GradPrepParams p) {
 // ranges of one launch do not overlap (each row is written by one block).
 __global__ void k_momentum_grad(const float* mdot_part, long long slot_stride, int nparts, int nb, float* dmom, long long bs,
                                 const MomentumMeanRanges r, int accumulate) {
+  __shared__ float red[16];
   const int ib = blockIdx.x;
   const float* part = mdot_part + blockIdx.y * slot_stride;
   const int start = r.start[blockIdx.y], len = r.len[blockIdx.y];
   float s = 0.f;
-  for (int j = 0; j < 3; ++j)
-    for (int i = 0; i < nparts; ++i) s += part[(size_t)(j * nb + ib) * nparts + i];
-  s /= (float)len;
+  for (int i = threadIdx.x; i < 3 * nparts; i += blockDim.x) s += part[(size_t)(i / nparts * nb + ib) * nparts + i % nparts];
+  s = block_sum(s, red) / (float)len;
   for (int t = threadIdx.x; t < len; t += blockDim.x) {
     float* dst = dmom + ib * bs + start + t;
     *dst = accumulate ? *dst + s : s;
@@ -635,7 +692,7 @@ __global__ void k_lr_reduce(const float* lrpart, long long upd_stride, long long
 // final weight gradients: state gradient (+ accumulator carry) + the path through the initial row norms
 struct FinishParams {
   MatGeom g;
-  const float* gw; const float* gw2; const float* carry; const float* gn0; const float* n0; const float* w_init;   // gw, gw2: addends, nullable
+  const float* gw; const float* gw2; Partials gwp, gwp2; const float* carry; const float* gn0; const float* n0; const float* w_init;   // gw, gw2, gwp, gwp2: addends, nullable
   int through_norms;
   float* out[3];
 };
@@ -651,6 +708,8 @@ __global__ void k_finish_weight_grads(const FinishParams p) {
     const float4 t = ld4(p.gw2 + o);
     v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
   }
+  add_partials(v, p.gwp, o);
+  add_partials(v, p.gwp2, o);
   if (p.carry) {
     const float4 t = ld4(p.carry + o);
     v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;

@@ -39,6 +39,34 @@ def test_partial_k_steps_against_oracle(b, L, d, dh, C):
     test_small_tiles_against_oracle(torch.bfloat16, b, L, d, dh, C)
 
 
+@pytest.mark.parametrize("dtype,b,L,d,dh,C", [(torch.bfloat16, 1, 3 * 2112, 64, 1088, 2112), (torch.bfloat16, 2, 3 * 2100, 48, 32, 2100),
+                                              (torch.float32, 1, 600, 16, 1040, 200)])
+def test_partial_sums_are_read_by_the_row_kernels(dtype, b, L, d, dh, C):
+    """Three chunks whose token reductions run in several splits (the row kernels add them up, with the momentum step on the way),
+    and rows longer than what a wave keeps in registers (1024 columns)."""
+    test_small_tiles_against_oracle(dtype, b, L, d, dh, C)
+
+
+@pytest.mark.parametrize("dtype,C", [(torch.float32, 300), (torch.bfloat16, 2200)])
+def test_several_apply_steps_on_one_weight_version(dtype, C):
+    """Two apply steps where one would do, on the newest and on an earlier version: the gradients are those of the one step."""
+    print("[gpu-test] several applies", dtype, C, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(1, 2 * C, 64, 32, seed=35, act_dtype=dtype).items()}
+    go = torch.randn(1, 4 * C, 64, generator=torch.Generator().manual_seed(5)).to(dtype).to("cuda")
+    U = [(LACT_UPDATE, 0, C, 0), (LACT_UPDATE, C, 2 * C, 0)]
+    one = (U[0], (LACT_APPLY, 0, 2 * C, 0), U[1], (LACT_APPLY, 0, 2 * C, 2 * C))
+    two = (U[0], (LACT_APPLY, 0, C, 0), (LACT_APPLY, C, 2 * C, C), U[1], (LACT_APPLY, 0, C, 2 * C), (LACT_APPLY, C, 2 * C, 3 * C))
+    res = []
+    for steps in (one, two):
+        x = [inp[n].clone().requires_grad_(True) for n in ORDER]
+        out, _, _ = ops.run_program(ops.Program(steps=steps, out_len=4 * C), *x)
+        res.append([out] + list(torch.autograd.grad(out, x, go)))
+    for n, a, r in zip(("out",) + ORDER, res[1], res[0]):
+        assert O.rel_l2(a, r) < (1e-5 if dtype == torch.float32 else 1e-2), n
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("d,dh", [(128, 256), (72, 40), (8, 72)])
 def test_transposed_weights_are_read_as_they_lie(dtype, d, dh):

@@ -226,6 +226,7 @@ __device__ __forceinline__ void row_gemm_tile(const RowGemmDmaParams<NT>& pp, in
 template <class TS, int NT, int EPI, bool B_KS>
 __global__ __launch_bounds__(DMA_THREADS) void k_row_gemm_dma(const RowGemmDmaParams<NT> pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  prefetch_args<sizeof(pp)>();
   int bx, by, z;
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
   row_gemm_tile<TS, NT, EPI, B_KS, false>(pp, bx, by, z, smem);
@@ -272,6 +273,7 @@ template <class TS, int STAGES = 3, int WPE = 2>
 __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using Pipe = DmaPipe<TS, 2, 1, STAGES>;
+  prefetch_args<sizeof(pp)>();
   const HiddenParams& p = pp.h;
   int bx, by, z;
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
@@ -386,6 +388,7 @@ __device__ __forceinline__ void stage_three_products(char* smem, const f32x16 (&
 template <class TS, int STAGES = 3, int WPE = 2>
 __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  prefetch_args<sizeof(pp)>();
   const HiddenParams& p = pp.h;
   int bx, by, z;
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
@@ -453,6 +456,7 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_hidden_dma(const Hi
 template <class TS, int STAGES = 3, int WPE = 2>
 __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_bwd_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  prefetch_args<sizeof(pp)>();
   const HiddenParams& p = pp.h;
   int bx, by, z;
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
@@ -504,6 +508,7 @@ template <class TS, int STAGES = 3, int WPE = 2>
 __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_bwd_hidden_dma(const HiddenDmaParams pp) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using Pipe = DmaPipe<TS, 2, 3, STAGES>;
+  prefetch_args<sizeof(pp)>();
   const HiddenParams& p = pp.h;
   int bx, by, z;
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
@@ -624,6 +629,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
   constexpr int STAGES = 3;
   using Pipe = DmaPipe<TS, 2, 3, STAGES>;
   using SM = typename Pipe::SM;
+  prefetch_args<sizeof(pp)>();
   const HiddenParams& p = pp.h;
   int bx, by, z;
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
@@ -766,35 +772,32 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
 // ------------------------------------------------------------------------------------------------
 struct TokenReduceDmaParams : TokenReduceParams {
   TileMap map;   // token splits, output tiles, 3 * batch
+  UDiv by_nb, by_tn[3];   // nb; tiles along N of each job
 };
 // One block of the reduction; `lin` is the block's linear index in the reduction's tile map.
 template <class TS>
 __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParams& p, int lin, char* smem) {
   constexpr int STAGES = row_stages<TS>();
-  using Pipe = DmaPipe<TS, 1, 2, STAGES, false, true>;
+  using Pipe = DmaPipe<TS, 1, 1, STAGES, false, true>;
   int split, tile, bz;   // map: (splits, tiles, 3*nb)
   clear_words(p.prep_clear, lin == 0);
   if (!p.map.locate(lin, split, tile, bz)) return;
-  const int j = bz / p.nb, ib = bz % p.nb;
+  const int j = p.by_nb.div(bz), ib = bz - j * p.nb;
   const TokenReduceJob& job = p.job[j];
-  const int tiles_n = (job.N + TS::BN - 1) / TS::BN;
-  const int m0 = (tile / tiles_n) * TS::BM, n0 = (tile % tiles_n) * TS::BN;
+  const int tm = p.by_tn[j].div(tile);
+  const int m0 = tm * TS::BM, n0 = (tile - tm * (int)p.by_tn[j].d) * TS::BN;
   if (m0 >= job.M) return;
   const int k_begin = split * p.split_len;
   const int klen = min(p.split_len, p.tokens - k_begin);
-  DmaPhase<1> ph[2];
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const TokenReduceTerm& tt = job.t[t < job.nterms ? t : 0];
-    ph[t].a.base = reinterpret_cast<const uint16_t*>(tt.A) + ib * tt.bsA + (size_t)k_begin * tt.lda + m0;
-    ph[t].a.ld = tt.lda; ph[t].a.rows = job.M - m0; ph[t].a.ks = 1;
-    ph[t].b[0].base = reinterpret_cast<const uint16_t*>(tt.B) + ib * tt.bsB + (size_t)k_begin * tt.ldb + n0;
-    ph[t].b[0].ld = tt.ldb; ph[t].b[0].rows = job.N - n0; ph[t].b[0].ks = 1;
-    ph[t].nb = 1;
-    // a token count that is not a multiple of 64 ends inside the last K-step of the last split
-    ph[t].K = t < job.nterms ? (klen + DMA_BK - 1) / DMA_BK * DMA_BK : 0;
-    ph[t].a.ktail = ph[t].b[0].ktail = klen % DMA_BK;
-  }
+  DmaPhase<1> ph[1];
+  ph[0].a.base = reinterpret_cast<const uint16_t*>(job.t.A) + ib * job.t.bsA + (size_t)k_begin * job.t.lda + m0;
+  ph[0].a.ld = job.t.lda; ph[0].a.rows = job.M - m0; ph[0].a.ks = 1;
+  ph[0].b[0].base = reinterpret_cast<const uint16_t*>(job.t.B) + ib * job.t.bsB + (size_t)k_begin * job.t.ldb + n0;
+  ph[0].b[0].ld = job.t.ldb; ph[0].b[0].rows = job.N - n0; ph[0].b[0].ks = 1;
+  ph[0].nb = 1;
+  // a token count that is not a multiple of 64 ends inside the last K-step of the last split
+  ph[0].K = (klen + DMA_BK - 1) / DMA_BK * DMA_BK;
+  ph[0].a.ktail = ph[0].b[0].ktail = klen % DMA_BK;
   f32x16 acc[1][TS::TM][TS::TN];
   Pipe pipe(smem, ph);
   const bool loader = Pipe::is_loader();
@@ -804,7 +807,6 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
     zero_acc<TS>(acc[0]);
     int step = 0;
     pipe.template run_phase<1, true, true>(ph[0].K, step, acc);
-    pipe.template run_phase<1, true, true>(ph[1].K, step, acc);
   }
   __syncthreads();
   using ST = StageTile<TS, 4>;
@@ -897,6 +899,7 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
 
 template <class TS>
 __global__ __launch_bounds__(DMA_THREADS) void k_token_reduce_dma(const TokenReduceDmaParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   token_reduce_dma_block<TS>(p, blockIdx.x, smem);
 }
@@ -915,6 +918,7 @@ struct TokenReduceRowsParams {
 static_assert(sizeof(TokenReduceRowsParams) <= 4096, "kernel arguments must fit the 4 KiB argument segment");
 template <class TS>
 __global__ __launch_bounds__(DMA_THREADS) void k_token_reduce_rows_dma(const TokenReduceRowsParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   int lin = blockIdx.x;
   if (lin < p.ntr) {

@@ -399,7 +399,7 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_bwd_hidden
 
 // ------------------------------------------------------------------------------------------------
 // k_token_reduce: the three token-reduction GEMMs of one step, split over tokens.
-//   job j, batch ib:  P[j][ib][M_j, N_j] = sum over terms  A_t[tokens, M_j]^T * B_t[tokens, N_j]
+//   job j, batch ib:  P[j][ib][M_j, N_j] = A[tokens, M_j]^T * B[tokens, N_j]
 // Both operands K-strided.  Grid (max tiles, splits, 3*b); fp32 partials [split][3*b][M*N].
 // ------------------------------------------------------------------------------------------------
 struct TokenReduceTerm {
@@ -407,8 +407,8 @@ struct TokenReduceTerm {
   const void* B; int ldb; long long bsB;
 };
 struct TokenReduceJob {
-  TokenReduceTerm t[2];
-  int nterms, M, N;
+  TokenReduceTerm t;
+  int M, N;
 };
 struct TokenReduceParams {
   TokenReduceJob job[3];
@@ -438,17 +438,12 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_token_reduce(cons
   const int klen = min(p.split_len, p.tokens - k_begin);
   f32x16 acc[TS::TM][TS::TN];
   zero_acc<TS>(acc);
-  AsyncPipe<T, 2> pipe(smem);
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const TokenReduceTerm& tt = job.t[t < job.nterms ? t : 0];
-    const T* A = reinterpret_cast<const T*>(tt.A) + ib * tt.bsA + (size_t)k_begin * tt.lda + m0;
-    const T* B = reinterpret_cast<const T*>(tt.B) + ib * tt.bsB + (size_t)k_begin * tt.ldb + n0;
-    pipe.phase(t, A, tt.lda, job.M - m0, true, B, tt.ldb, job.N - n0, true, t < job.nterms ? klen : 0);
-  }
+  AsyncPipe<T, 1> pipe(smem);
+  const T* A = reinterpret_cast<const T*>(job.t.A) + ib * job.t.bsA + (size_t)k_begin * job.t.lda + m0;
+  const T* B = reinterpret_cast<const T*>(job.t.B) + ib * job.t.bsB + (size_t)k_begin * job.t.ldb + n0;
+  pipe.phase(0, A, job.t.lda, job.M - m0, true, B, job.t.ldb, job.N - n0, true, klen);
   pipe.start();
   pipe.template accumulate<true, true>(0, acc);
-  pipe.template accumulate<true, true>(1, acc);
   const size_t slot = (size_t)blockIdx.z * p.mat_elems;
   float* out = p.add_out ? p.add_out + slot : p.partial + (size_t)blockIdx.y * gridDim.z * p.mat_elems + slot;
   LACT_FOR_QUADS(TS) {

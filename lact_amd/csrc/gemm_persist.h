@@ -401,6 +401,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_hidden_persist(const HiddenPers
   using TS = typename POL::TS;
   using L = PersistLds<POL>;
   static_assert(TS::BM == 128 && TS::BN == 128 && TS::WM == 64 && TS::WN == 64, "64 x 64 per wave");
+  prefetch_args<sizeof(pp)>();
   const HiddenParams& p = pp.h;
   const bool service = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4;
   // K-steps of a tile (the same for every tile of the launch)

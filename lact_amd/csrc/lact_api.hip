@@ -909,8 +909,10 @@ struct Runner {
         static_cast<TokenReduceParams&>(pd) = p;
         pd.tokens = tokens; pd.split_len = sp.len; pd.partial = partial;
         pd.map = make_tile_map(sp.n, tiles, 3 * d.b);
+        pd.by_nb = make_udiv(d.b);
+        for (int j = 0; j < 3; ++j) pd.by_tn[j] = make_udiv(ceil_div(jobs[j].N, tr_big(d.d, d.dh) ? TS_NS::BN : TS_SQ::BN));
         dim3 g(pd.map.grid());
-        const double fl = 6.0 * tokens * d.d * d.dh * d.b * jobs[0].nterms;
+        const double fl = 6.0 * tokens * d.d * d.dh * d.b;
         direct = add_out && sp.n == 1;
         const bool folded = prep && sp.n == 1;
         if (folded) {
@@ -952,7 +954,7 @@ struct Runner {
     if (direct) { p.add_out = add_out; p.add_in = coeff != 0.f ? add_in : nullptr; p.coeff = coeff; }
     p.tokens = tokens; p.split_len = sp.len; p.partial = partial;
     LACT_BIG_LDS(k_token_reduce<T>, SM);
-    LACT_LAUNCH_SMEM("k_token_reduce", site, 6.0 * tokens * d.d * d.dh * d.b * jobs[0].nterms, (k_token_reduce<T>), dim3(P.tiles, sp.n, 3 * d.b),
+    LACT_LAUNCH_SMEM("k_token_reduce", site, 6.0 * tokens * d.d * d.dh * d.b, (k_token_reduce<T>), dim3(P.tiles, sp.n, 3 * d.b),
                      dim3(TS::THREADS), SM, s, p);
     return direct ? 0 : sp.n;
   }
@@ -1109,13 +1111,12 @@ struct Runner {
       {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));
-        jobs[0].nterms = jobs[1].nterms = jobs[2].nterms = 1;
         jobs[0].M = d.dh; jobs[0].N = d.d;
-        set_tr_term(jobs[0].t[0], upd_z[0], d.dh, upd_zbs, kl0, d.d, klbs);
+        set_tr_term(jobs[0].t, upd_z[0], d.dh, upd_zbs, kl0, d.d, klbs);
         jobs[1].M = d.d; jobs[1].N = d.dh;
-        set_tr_term(jobs[1].t[0], vc, d.v_ld, d.v_bs, upd_z[1], d.dh, upd_zbs);
+        set_tr_term(jobs[1].t, vc, d.v_ld, d.v_bs, upd_z[1], d.dh, upd_zbs);
         jobs[2].M = d.dh; jobs[2].N = d.d;
-        set_tr_term(jobs[2].t[0], upd_z[2], d.dh, upd_zbs, kl2, d.d, klbs);
+        set_tr_term(jobs[2].t, upd_z[2], d.dh, upd_zbs, kl2, d.d, klbs);
         // square shapes with Muon: the momentum step can ride in the reduction's epilogue (every tile exists for
         // every matrix, and the Newton-Schulz orientation is the packed one)
         PrepFold pf;
@@ -1422,13 +1423,12 @@ struct Runner {
         const T* gc = dout + (size_t)st.out_start * d.do_ld;
         auto dw_jobs = [&](TokenReduceJob (&jobs)[3]) {
           memset(jobs, 0, sizeof(jobs));
-          jobs[0].nterms = jobs[1].nterms = jobs[2].nterms = 1;
           jobs[0].M = d.dh; jobs[0].N = d.d;
-          set_tr_term(jobs[0].t[0], h(1), d.dh, hbs(), qc, d.q_ld, d.q_bs);
+          set_tr_term(jobs[0].t, h(1), d.dh, hbs(), qc, d.q_ld, d.q_bs);
           jobs[1].M = d.d; jobs[1].N = d.dh;
-          set_tr_term(jobs[1].t[0], gc, d.do_ld, d.do_bs, h(0), d.dh, hbs());
+          set_tr_term(jobs[1].t, gc, d.do_ld, d.do_bs, h(0), d.dh, hbs());
           jobs[2].M = d.dh; jobs[2].N = d.d;
-          set_tr_term(jobs[2].t[0], h(2), d.dh, hbs(), qc, d.q_ld, d.q_bs);
+          set_tr_term(jobs[2].t, h(2), d.dh, hbs(), qc, d.q_ld, d.q_bs);
         };
         auto dq_gemm = [&]() {   // dq = gY0 W0 + gY2 W2
           auto p = row_params<2>();
@@ -1707,13 +1707,12 @@ struct Runner {
       {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));
-        jobs[0].nterms = jobs[1].nterms = jobs[2].nterms = 1;
         jobs[0].M = d.dh; jobs[0].N = d.d;
-        set_tr_term(jobs[0].t[0], h(0), d.dh, hbs(), kc, d.k_ld, d.k_bs);
+        set_tr_term(jobs[0].t, h(0), d.dh, hbs(), kc, d.k_ld, d.k_bs);
         jobs[1].M = d.d; jobs[1].N = d.dh;
-        set_tr_term(jobs[1].t[0], vc, d.v_ld, d.v_bs, h(1), d.dh, hbs());
+        set_tr_term(jobs[1].t, vc, d.v_ld, d.v_bs, h(1), d.dh, hbs());
         jobs[2].M = d.dh; jobs[2].N = d.d;
-        set_tr_term(jobs[2].t[0], h(2), d.dh, hbs(), kc, d.k_ld, d.k_bs);
+        set_tr_term(jobs[2].t, h(2), d.dh, hbs(), kc, d.k_ld, d.k_bs);
         // the update before: its weights enter these as they are, unless Newton-Schulz output replaces them or an accumulator carries on
         gw = GradSum{(d.prenorm || (P.muon && d.muon_replaces_weight)) ? nullptr : gwhat, 0};
         contribute(kBf16 ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, gwcur, &rows_job);

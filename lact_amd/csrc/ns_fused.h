@@ -179,6 +179,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_bwd_dot_tiles(const NsTileDo
 template <class TS, bool BWD>
 __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
+  prefetch_args<sizeof(p)>();
   const int tr = p.r / TS::BM, tc = p.c / TS::BN, ts = p.r / TS::BN;   // tile rows; tile columns of [r, c] and of [r, r]
   const int nbm = tr * tc;                           // blocks per matrix (c >= r: the r x c stages have the most tiles)
   const int L = blockIdx.x, j = L >> 3;

@@ -186,6 +186,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_fwd(co
   using T = AttnTile<D>;
   using Copy = AttnCopy<D, NW>;
   constexpr int STAGE = 2 * T::BYTES;
+  prefetch_args<sizeof(p)>();
   int bx, by, z;
   if (!p.map.locate(blockIdx.x, bx, by, z)) return;
   bx = p.map.gx - 1 - bx;      // the longest windows first
@@ -280,6 +281,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_dq(con
   using T = AttnTile<D>;
   using Copy = AttnCopy<D, NW>;
   constexpr int STAGE = 2 * T::BYTES;
+  prefetch_args<sizeof(p)>();
   int bx, by, z;
   if (!p.map.locate(blockIdx.x, bx, by, z)) return;
   bx = p.map.gx - 1 - bx;
@@ -365,6 +367,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_dkv(co
   using T = AttnTile<D>;
   using Copy = AttnCopy<D, NW>;
   constexpr int STAGE = 2 * T::BYTES;
+  prefetch_args<sizeof(p)>();
   int bx, by, z;
   if (!p.map.locate(blockIdx.x, bx, by, z)) return;
   const int b = z / p.H, h = z % p.H, L = p.L;

@@ -100,4 +100,28 @@ __device__ __forceinline__ void clear_words(const ClearWords& c, bool first_bloc
     for (int i = threadIdx.x; i < c.n; i += blockDim.x) c.ptr[i] = 0u;
 }
 
+// Division of 0 <= n < 2^31 by a number that the host knows, without a division's forty dependent instructions: with
+// 2^(s-1) < d <= 2^s and m = ceil(2^(31+s) / d), the error n * (m d - 2^(31+s)) of the product stays below 2^(31+s).
+struct UDiv {
+  unsigned d, m, s;
+  __host__ __device__ __forceinline__ int div(int n) const { return (int)((unsigned)(((uint64_t)(2u * (unsigned)n) * m) >> 32) >> s); }
+};
+inline UDiv make_udiv(int d) {
+  UDiv u;
+  u.d = d > 0 ? d : 1; u.s = 0;
+  while ((1u << u.s) < u.d) ++u.s;
+  u.m = (unsigned)((((uint64_t)1 << (31 + u.s)) + u.d - 1) / u.d);
+  return u;
+}
+
+// Batch entry z = g * d + ib of a launch over several steps of a program: offset of an operand whose batch entries lie bs apart and
+// whose steps gs apart.  All zero: one step, z = ib.
+struct StepBatch {
+  UDiv by_nb;
+  __host__ __device__ __forceinline__ long long at(int z, long long bs, long long gs) const {
+    const int g = by_nb.div(z);
+    return (z - g * (int)by_nb.d) * bs + g * gs;
+  }
+};
+
 }  // namespace lact

@@ -165,20 +165,6 @@ __device__ __forceinline__ bf16x8 dma_fetch(const char* tile, int row, int kvec)
 // that XCD's order, so that the shared tiles are fetched from HBM once and not once per die.  A group is
 // one batch entry with all its tiles (batch count a multiple of 8) or one row of tiles of a batch entry.
 // Only the speed depends on the dealing order, never the result.
-// Division of 0 <= n < 2^31 by a number that the host knows, without a division's forty dependent instructions: with
-// 2^(s-1) < d <= 2^s and m = ceil(2^(31+s) / d), the error n * (m d - 2^(31+s)) of the product stays below 2^(31+s).
-struct UDiv {
-  unsigned d, m, s;
-  __host__ __device__ __forceinline__ int div(int n) const { return (int)((unsigned)(((uint64_t)(2u * (unsigned)n) * m) >> 32) >> s); }
-};
-inline UDiv make_udiv(int d) {
-  UDiv u;
-  u.d = d > 0 ? d : 1; u.s = 0;
-  while ((1u << u.s) < u.d) ++u.s;
-  u.m = (unsigned)((((uint64_t)1 << (31 + u.s)) + u.d - 1) / u.d);
-  return u;
-}
-
 // The arguments of a launch lie in memory, and the scalar cache is cold when a kernel begins: read one by one where the code
 // first needs them, they cost one memory latency per 64-byte line, in a row.  One load from every line of the first BYTES up
 // front makes that a single one: the token reduction's copy waves start 0.7 us after the block instead of 2.1 us (with the

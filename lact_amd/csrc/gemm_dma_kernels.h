@@ -35,7 +35,7 @@ __device__ __forceinline__ void row_gemm_phases(const RowGemmParams<NT>& p, int 
   for (int t = 0; t < NT; ++t) {
     ph[t].a.base = reinterpret_cast<const uint16_t*>(p.t[t].A) + z * p.t[t].bsA + (size_t)m0 * p.t[t].lda;
     ph[t].a.ld = p.t[t].lda; ph[t].a.rows = p.M - m0; ph[t].a.ks = 0;
-    ph[t].b[0].base = reinterpret_cast<const uint16_t*>(p.t[t].B) + z * p.t[t].bsB + (B_KS ? (size_t)n0 : (size_t)n0 * p.t[t].ldb);
+    ph[t].b[0].base = reinterpret_cast<const uint16_t*>(p.t[t].B) + p.steps.at(z, p.t[t].bsB, p.t[t].gsB) + (B_KS ? (size_t)n0 : (size_t)n0 * p.t[t].ldb);
     ph[t].b[0].ld = p.t[t].ldb; ph[t].b[0].rows = p.N - n0; ph[t].b[0].ks = B_KS;
     ph[t].nb = 1;
     ph[t].K = p.t[t].K;
@@ -50,7 +50,7 @@ __device__ __forceinline__ void row_gemm_copy_out_b16(const RowGemmParams<NT>& p
   const int r0 = ST::row0(), c0 = ST::col0();
   if (ST::active() && n0 + c0 < p.N) {
     const char* src = smem + (r0 * ST::LD + c0) * 2;
-    uint16_t* dst = reinterpret_cast<uint16_t*>(p.out) + z * p.bso + (size_t)(m0 + r0) * p.ldo + n0 + c0;
+    uint16_t* dst = reinterpret_cast<uint16_t*>(p.out) + p.steps.at(z, p.bso, p.gso) + (size_t)(m0 + r0) * p.ldo + n0 + c0;
     const uint16_t* aux = reinterpret_cast<const uint16_t*>(p.aux) + z * p.bsaux + (size_t)(m0 + r0) * p.ldaux + n0 + c0;
     const size_t dstep = (size_t)ST::RPP * p.ldo, astep = (size_t)ST::RPP * p.ldaux;
     const bool blend = EPI == EPI_AXPBY || p.accumulate;
@@ -241,26 +241,26 @@ struct HiddenDmaParams {
 };
 
 template <class TS>
-__device__ __forceinline__ DmaOperand token_operand(const void* base, long long bs, int ld, int z, int m0, int T) {
+__device__ __forceinline__ DmaOperand token_operand(const void* base, long long off, int ld, int m0, int T) {
   DmaOperand o;
-  o.base = reinterpret_cast<const uint16_t*>(base) + z * bs + (size_t)m0 * ld;
+  o.base = reinterpret_cast<const uint16_t*>(base) + off + (size_t)m0 * ld;
   o.ld = ld;
   o.rows = T - m0;
   o.ks = 0;
   return o;
 }
-__device__ __forceinline__ DmaOperand weight_operand(const void* base, long long bs, int ld, int z, int n0, int rows) {
+__device__ __forceinline__ DmaOperand weight_operand(const void* base, long long off, int ld, int n0, int rows) {
   DmaOperand o;
-  o.base = reinterpret_cast<const uint16_t*>(base) + z * bs + (size_t)n0 * ld;
+  o.base = reinterpret_cast<const uint16_t*>(base) + off + (size_t)n0 * ld;
   o.ld = ld;
   o.rows = rows - n0;
   o.ks = 0;
   return o;
 }
 // [K, rows] matrix (rows contiguous): the tile starts at column n0
-__device__ __forceinline__ DmaOperand weight_operand_ks(const void* base, long long bs, int ld, int z, int n0, int rows) {
+__device__ __forceinline__ DmaOperand weight_operand_ks(const void* base, long long off, int ld, int n0, int rows) {
   DmaOperand o;
-  o.base = reinterpret_cast<const uint16_t*>(base) + z * bs + n0;
+  o.base = reinterpret_cast<const uint16_t*>(base) + off + n0;
   o.ld = ld;
   o.rows = rows - n0;
   o.ks = 1;
@@ -279,9 +279,9 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_hidden_dma(const Hid
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
   const int m0 = bx * TS::BM, n0 = by * TS::BN;
   DmaPhase<2> ph[1];
-  ph[0].a = token_operand<TS>(p.X, p.bsx, p.ldx, z, m0, p.T);
-  ph[0].b[0] = weight_operand(p.W0, p.bsw, p.d, z, n0, p.dh);
-  ph[0].b[1] = weight_operand(p.W2, p.bsw, p.d, z, n0, p.dh);
+  ph[0].a = token_operand<TS>(p.X, p.steps.at(z, p.bsx, p.gsx), p.ldx, m0, p.T);
+  ph[0].b[0] = weight_operand(p.W0, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
+  ph[0].b[1] = weight_operand(p.W2, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
   ph[0].nb = 2;
   ph[0].K = p.d;
   f32x16 acc[2][TS::TM][TS::TN];
@@ -324,13 +324,13 @@ __device__ __forceinline__ void three_acc_mainloop(const HiddenDmaParams& pp, ch
   using Pipe = DmaPipe<TS, 2, 2, STAGES>;
   const HiddenParams& p = pp.h;
   DmaPhase<2> ph[2];
-  ph[0].a = token_operand<TS>(p.X, p.bsx, p.ldx, z, m0, p.T);
-  ph[0].b[0] = weight_operand(p.W0, p.bsw, p.d, z, n0, p.dh);
-  ph[0].b[1] = weight_operand(p.W2, p.bsw, p.d, z, n0, p.dh);
+  ph[0].a = token_operand<TS>(p.X, p.steps.at(z, p.bsx, p.gsx), p.ldx, m0, p.T);
+  ph[0].b[0] = weight_operand(p.W0, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
+  ph[0].b[1] = weight_operand(p.W2, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
   ph[0].nb = 2;
   ph[0].K = p.d;
-  ph[1].a = token_operand<TS>(p.Y, p.bsy, p.ldy, z, m0, p.T);
-  ph[1].b[0] = weight_operand_ks(p.W1, p.bsw, p.dh, z, n0, p.dh);   // V * W1: w1 is [d, dh]
+  ph[1].a = token_operand<TS>(p.Y, p.steps.at(z, p.bsy, p.gsy), p.ldy, m0, p.T);
+  ph[1].b[0] = weight_operand_ks(p.W1, p.steps.at(z, p.bsw, p.gsw), p.dh, n0, p.dh);   // V * W1: w1 is [d, dh]
   ph[1].b[1] = ph[1].b[0];
   ph[1].nb = 1;
   ph[1].K = p.d;
@@ -514,15 +514,15 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_bwd_hidden_dma(cons
   if (!pp.map.locate(blockIdx.x, bx, by, z)) return;
   const int m0 = bx * TS::BM, n0 = by * TS::BN;
   DmaPhase<2> ph[3];
-  ph[0].a = token_operand<TS>(p.X, p.bsx, p.ldx, z, m0, p.T);
-  ph[0].b[0] = weight_operand(p.W0, p.bsw, p.d, z, n0, p.dh);
-  ph[0].b[1] = weight_operand(p.W2, p.bsw, p.d, z, n0, p.dh);
+  ph[0].a = token_operand<TS>(p.X, z * p.bsx, p.ldx, m0, p.T);
+  ph[0].b[0] = weight_operand(p.W0, z * p.bsw, p.d, n0, p.dh);
+  ph[0].b[1] = weight_operand(p.W2, z * p.bsw, p.d, n0, p.dh);
   ph[1].a = ph[0].a;
-  ph[1].b[0] = weight_operand(p.G0, p.bsw, p.d, z, n0, p.dh);
-  ph[1].b[1] = weight_operand(p.G2, p.bsw, p.d, z, n0, p.dh);
-  ph[2].a = token_operand<TS>(p.Y, p.bsy, p.ldy, z, m0, p.T);
-  ph[2].b[0] = weight_operand_ks(p.W1, p.bsw, p.dh, z, n0, p.dh);
-  ph[2].b[1] = weight_operand_ks(p.G1, p.bsw, p.dh, z, n0, p.dh);
+  ph[1].b[0] = weight_operand(p.G0, z * p.bsw, p.d, n0, p.dh);
+  ph[1].b[1] = weight_operand(p.G2, z * p.bsw, p.d, n0, p.dh);
+  ph[2].a = token_operand<TS>(p.Y, z * p.bsy, p.ldy, m0, p.T);
+  ph[2].b[0] = weight_operand_ks(p.W1, z * p.bsw, p.dh, n0, p.dh);
+  ph[2].b[1] = weight_operand_ks(p.G1, z * p.bsw, p.dh, n0, p.dh);
   ph[0].K = ph[1].K = ph[2].K = p.d;
   ph[0].nb = ph[1].nb = ph[2].nb = 2;
   f32x16 aw[2][TS::TM][TS::TN], ag[2][TS::TM][TS::TN], ay[2][TS::TM][TS::TN];
@@ -639,19 +639,19 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
   DmaPhase<2> ph[3];
   // the one-accumulator phase first: the two-accumulator K-steps in front of the input stages are the longer ones,
   // which gives the input copies more time to land
-  ph[0].a = token_operand<TS>(p.Y, p.bsy, p.ldy, z, m0, p.T);
-  ph[0].b[0] = weight_operand_ks(p.G1, p.bsw, p.dh, z, n0, p.dh);
+  ph[0].a = token_operand<TS>(p.Y, z * p.bsy, p.ldy, m0, p.T);
+  ph[0].b[0] = weight_operand_ks(p.G1, z * p.bsw, p.dh, n0, p.dh);
   ph[0].b[1] = ph[0].b[0];
   ph[0].nb = 1;
   ph[0].K = p.d;
-  ph[1].a = token_operand<TS>(p.X, p.bsx, p.ldx, z, m0, p.T);
-  ph[1].b[0] = weight_operand(p.G0, p.bsw, p.d, z, n0, p.dh);
-  ph[1].b[1] = weight_operand(p.G2, p.bsw, p.d, z, n0, p.dh);
+  ph[1].a = token_operand<TS>(p.X, z * p.bsx, p.ldx, m0, p.T);
+  ph[1].b[0] = weight_operand(p.G0, z * p.bsw, p.d, n0, p.dh);
+  ph[1].b[1] = weight_operand(p.G2, z * p.bsw, p.d, n0, p.dh);
   ph[1].nb = 2;
   ph[1].K = p.d;
-  ph[2].a = token_operand<TS>(reinterpret_cast<const uint16_t*>(p.I0) + n0, p.bsi, p.dh, z, m0, p.T);
-  ph[2].b[0] = token_operand<TS>(reinterpret_cast<const uint16_t*>(p.I1) + n0, p.bsi, p.dh, z, m0, p.T);
-  ph[2].b[1] = token_operand<TS>(reinterpret_cast<const uint16_t*>(p.I2) + n0, p.bsi, p.dh, z, m0, p.T);
+  ph[2].a = token_operand<TS>(reinterpret_cast<const uint16_t*>(p.I0) + n0, z * p.bsi, p.dh, m0, p.T);
+  ph[2].b[0] = token_operand<TS>(reinterpret_cast<const uint16_t*>(p.I1) + n0, z * p.bsi, p.dh, m0, p.T);
+  ph[2].b[1] = token_operand<TS>(reinterpret_cast<const uint16_t*>(p.I2) + n0, z * p.bsi, p.dh, m0, p.T);
   ph[2].nb = 2;
   ph[2].K = halves * 64;
   f32x16 ag[2][TS::TM][TS::TN], ay[1][TS::TM][TS::TN];
@@ -772,7 +772,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
 // ------------------------------------------------------------------------------------------------
 struct TokenReduceDmaParams : TokenReduceParams {
   TileMap map;   // token splits, output tiles, 3 * batch
-  UDiv by_nb, by_tn[3];   // nb; tiles along N of each job
+  UDiv by_tn[3];   // tiles along N of each job
 };
 // One block of the reduction; `lin` is the block's linear index in the reduction's tile map.
 template <class TS>
@@ -782,7 +782,7 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
   int split, tile, bz;   // map: (splits, tiles, 3*nb)
   clear_words(p.prep_clear, lin == 0);
   if (!p.map.locate(lin, split, tile, bz)) return;
-  const int j = p.by_nb.div(bz), ib = bz - j * p.nb;
+  const int t = p.by_nb.div(bz), ib = bz - t * (int)p.by_nb.d, g = t / 3, j = t - 3 * g;
   const TokenReduceJob& job = p.job[j];
   const int tm = p.by_tn[j].div(tile);
   const int m0 = tm * TS::BM, n0 = (tile - tm * (int)p.by_tn[j].d) * TS::BN;
@@ -790,9 +790,9 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
   const int k_begin = split * p.split_len;
   const int klen = min(p.split_len, p.tokens - k_begin);
   DmaPhase<1> ph[1];
-  ph[0].a.base = reinterpret_cast<const uint16_t*>(job.t.A) + ib * job.t.bsA + (size_t)k_begin * job.t.lda + m0;
+  ph[0].a.base = reinterpret_cast<const uint16_t*>(job.t.A) + ib * job.t.bsA + g * job.t.gsA + (size_t)k_begin * job.t.lda + m0;
   ph[0].a.ld = job.t.lda; ph[0].a.rows = job.M - m0; ph[0].a.ks = 1;
-  ph[0].b[0].base = reinterpret_cast<const uint16_t*>(job.t.B) + ib * job.t.bsB + (size_t)k_begin * job.t.ldb + n0;
+  ph[0].b[0].base = reinterpret_cast<const uint16_t*>(job.t.B) + ib * job.t.bsB + g * job.t.gsB + (size_t)k_begin * job.t.ldb + n0;
   ph[0].b[0].ld = job.t.ldb; ph[0].b[0].rows = job.N - n0; ph[0].b[0].ks = 1;
   ph[0].nb = 1;
   // a token count that is not a multiple of 64 ends inside the last K-step of the last split

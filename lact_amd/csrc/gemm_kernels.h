@@ -28,7 +28,7 @@ __device__ __forceinline__ SiluParts silu_parts(float x) {
 // ------------------------------------------------------------------------------------------------
 struct RowGemmTerm {
   const void* A; int lda; long long bsA;
-  const void* B; int ldb; long long bsB;
+  const void* B; int ldb; long long bsB, gsB;   // gsB: between the steps of a launch over several
   int K;
 };
 enum { EPI_STORE = 0, EPI_AXPBY = 1, EPI_AXPBY_F32_DUAL = 2 };
@@ -37,6 +37,7 @@ struct RowGemmParams {
   RowGemmTerm t[NT];
   int M, N;
   void* out; int ldo; long long bso;          // EPI_STORE, EPI_AXPBY: type T; DUAL: fp32
+  StepBatch steps; long long gso;              // EPI_STORE: several steps in one launch (their A operands lie on one stride)
   int accumulate;                              // EPI_STORE only: out += result
   // EPI_STORE only, optional: out2 = round(alpha2 * round(acc)), type T, laid out like out (the product c*A that
   // ttt_operation.py:60 forms as a tensor of its own before the matmul)
@@ -69,7 +70,7 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_row_gemm(const Ro
 #pragma unroll
   for (int t = 0; t < NT; ++t) {
     const T* A = reinterpret_cast<const T*>(p.t[t].A) + z * p.t[t].bsA + (size_t)m0 * p.t[t].lda;
-    const T* B = reinterpret_cast<const T*>(p.t[t].B) + z * p.t[t].bsB + (B_KC ? (size_t)n0 * p.t[t].ldb : (size_t)n0);
+    const T* B = reinterpret_cast<const T*>(p.t[t].B) + p.steps.at(z, p.t[t].bsB, p.t[t].gsB) + (B_KC ? (size_t)n0 * p.t[t].ldb : (size_t)n0);
     pipe.phase(t, A, p.t[t].lda, p.M - m0, false, B, p.t[t].ldb, p.N - n0, !B_KC, p.t[t].K);
   }
   pipe.start();
@@ -82,7 +83,7 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_row_gemm(const Ro
 #pragma unroll
     for (int j = 0; j < 4; ++j) v[j] = acc[tm][tn][4 * g + j];
     if (EPI == EPI_STORE) {
-      T* o = reinterpret_cast<T*>(p.out) + z * p.bso + (size_t)m * p.ldo + n;
+      T* o = reinterpret_cast<T*>(p.out) + p.steps.at(z, p.bso, p.gso) + (size_t)m * p.ldo + n;
       if (p.accumulate) {
         float old[4];
         Elem<T>::load4(o, old);
@@ -131,6 +132,7 @@ struct HiddenParams {
   const void* X; int ldx; long long bsx;   // q (apply) or k (update)            [T, d]
   const void* Y; int ldy; long long bsy;   // v (update) or upstream grad (apply backward) [T, d]
   const void* W0; const void* W1; const void* W2; long long bsw;  // compute copies, type T
+  StepBatch steps; long long gsx, gsy, gsw;  // apply kernels: several steps in one launch (outputs on one stride)
   const float* lr0; const float* lr1; const float* lr2; long long bslr;  // [b, *] already offset to this step
   // gradients of the fast-weight gradients (backward of the update): G0,G2 [dh,d], G1 [d,dh], type T
   const void* G0; const void* G1; const void* G2;
@@ -150,9 +152,9 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_hidden(cons
   using TS = typename AsyncTile<T>::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
-  const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
-  const T* W0 = reinterpret_cast<const T*>(p.W0) + z * p.bsw + (size_t)n0 * p.d;
-  const T* W2 = reinterpret_cast<const T*>(p.W2) + z * p.bsw + (size_t)n0 * p.d;
+  const T* X = reinterpret_cast<const T*>(p.X) + p.steps.at(z, p.bsx, p.gsx) + (size_t)m0 * p.ldx;
+  const T* W0 = reinterpret_cast<const T*>(p.W0) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
+  const T* W2 = reinterpret_cast<const T*>(p.W2) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
   f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN];
   zero_acc<TS>(a0);
   zero_acc<TS>(a2);
@@ -275,11 +277,11 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_bwd_hidden(
   using TS = typename AsyncTile<T>::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
-  const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
-  const T* Y = reinterpret_cast<const T*>(p.Y) + z * p.bsy + (size_t)m0 * p.ldy;
-  const T* W0 = reinterpret_cast<const T*>(p.W0) + z * p.bsw + (size_t)n0 * p.d;
-  const T* W2 = reinterpret_cast<const T*>(p.W2) + z * p.bsw + (size_t)n0 * p.d;
-  const T* W1 = reinterpret_cast<const T*>(p.W1) + z * p.bsw + n0;
+  const T* X = reinterpret_cast<const T*>(p.X) + p.steps.at(z, p.bsx, p.gsx) + (size_t)m0 * p.ldx;
+  const T* Y = reinterpret_cast<const T*>(p.Y) + p.steps.at(z, p.bsy, p.gsy) + (size_t)m0 * p.ldy;
+  const T* W0 = reinterpret_cast<const T*>(p.W0) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
+  const T* W2 = reinterpret_cast<const T*>(p.W2) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
+  const T* W1 = reinterpret_cast<const T*>(p.W1) + p.steps.at(z, p.bsw, p.gsw) + n0;
   f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN], a1[TS::TM][TS::TN];
   zero_acc<TS>(a0);
   zero_acc<TS>(a2);
@@ -403,8 +405,8 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_bwd_hidden
 // Both operands K-strided.  Grid (max tiles, splits, 3*b); fp32 partials [split][3*b][M*N].
 // ------------------------------------------------------------------------------------------------
 struct TokenReduceTerm {
-  const void* A; int lda; long long bsA;
-  const void* B; int ldb; long long bsB;
+  const void* A; int lda; long long bsA, gsA;   // gs: between the steps of a launch over several
+  const void* B; int ldb; long long bsB, gsB;
 };
 struct TokenReduceJob {
   TokenReduceTerm t;
@@ -412,7 +414,8 @@ struct TokenReduceJob {
 };
 struct TokenReduceParams {
   TokenReduceJob job[3];
-  int nb, tokens, split_len;   // split_len: tokens per split (multiple of 32)
+  UDiv by_nb;                  // batch entries; matrix z = (step * 3 + job) * nb + batch entry
+  int tokens, split_len;   // split_len: tokens per split (multiple of 32)
   float* partial; long long mat_elems;
   // single split only: out = coeff*add_in + result written here instead of a partial
   float* add_out; const float* add_in; float coeff;
@@ -429,7 +432,7 @@ template <typename T>
 __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_token_reduce(const TokenReduceParams p) {
   using TS = typename AsyncTile<T>::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int j = blockIdx.z / p.nb, ib = blockIdx.z % p.nb;
+  const int t = p.by_nb.div(blockIdx.z), ib = blockIdx.z - t * p.by_nb.d, g = t / 3, j = t - 3 * g;
   const TokenReduceJob& job = p.job[j];
   const int tiles_n = (job.N + TS::BN - 1) / TS::BN;
   const int m0 = (blockIdx.x / tiles_n) * TS::BM, n0 = (blockIdx.x % tiles_n) * TS::BN;
@@ -439,8 +442,8 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_token_reduce(cons
   f32x16 acc[TS::TM][TS::TN];
   zero_acc<TS>(acc);
   AsyncPipe<T, 1> pipe(smem);
-  const T* A = reinterpret_cast<const T*>(job.t.A) + ib * job.t.bsA + (size_t)k_begin * job.t.lda + m0;
-  const T* B = reinterpret_cast<const T*>(job.t.B) + ib * job.t.bsB + (size_t)k_begin * job.t.ldb + n0;
+  const T* A = reinterpret_cast<const T*>(job.t.A) + ib * job.t.bsA + g * job.t.gsA + (size_t)k_begin * job.t.lda + m0;
+  const T* B = reinterpret_cast<const T*>(job.t.B) + ib * job.t.bsB + g * job.t.gsB + (size_t)k_begin * job.t.ldb + n0;
   pipe.phase(0, A, job.t.lda, job.M - m0, true, B, job.t.ldb, job.N - n0, true, klen);
   pipe.start();
   pipe.template accumulate<true, true>(0, acc);

@@ -229,9 +229,9 @@ struct ApplyHiddenPolicy {
   static constexpr int NACC = 2, NB = 2, NPH = 1;
   using TS = TS_SQ;
   __device__ static __forceinline__ void phases(const HiddenParams& p, int m0, int n0, int z, DmaPhase<2> (&ph)[1]) {
-    ph[0].a = token_operand<TS>(p.X, p.bsx, p.ldx, z, m0, p.T);
-    ph[0].b[0] = weight_operand(p.W0, p.bsw, p.d, z, n0, p.dh);
-    ph[0].b[1] = weight_operand(p.W2, p.bsw, p.d, z, n0, p.dh);
+    ph[0].a = token_operand<TS>(p.X, p.steps.at(z, p.bsx, p.gsx), p.ldx, m0, p.T);
+    ph[0].b[0] = weight_operand(p.W0, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
+    ph[0].b[1] = weight_operand(p.W2, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
     ph[0].nb = 2;
     ph[0].K = p.d;
   }
@@ -268,13 +268,13 @@ struct ApplyBwdHiddenPolicy {
   static constexpr int NACC = 3, NB = 2, NPH = 2;
   using TS = TS_SQ;
   __device__ static __forceinline__ void phases(const HiddenParams& p, int m0, int n0, int z, DmaPhase<2> (&ph)[2]) {
-    ph[0].a = token_operand<TS>(p.X, p.bsx, p.ldx, z, m0, p.T);
-    ph[0].b[0] = weight_operand(p.W0, p.bsw, p.d, z, n0, p.dh);
-    ph[0].b[1] = weight_operand(p.W2, p.bsw, p.d, z, n0, p.dh);
+    ph[0].a = token_operand<TS>(p.X, p.steps.at(z, p.bsx, p.gsx), p.ldx, m0, p.T);
+    ph[0].b[0] = weight_operand(p.W0, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
+    ph[0].b[1] = weight_operand(p.W2, p.steps.at(z, p.bsw, p.gsw), p.d, n0, p.dh);
     ph[0].nb = 2;
     ph[0].K = p.d;
-    ph[1].a = token_operand<TS>(p.Y, p.bsy, p.ldy, z, m0, p.T);
-    ph[1].b[0] = weight_operand_ks(p.W1, p.bsw, p.dh, z, n0, p.dh);
+    ph[1].a = token_operand<TS>(p.Y, p.steps.at(z, p.bsy, p.gsy), p.ldy, m0, p.T);
+    ph[1].b[0] = weight_operand_ks(p.W1, p.steps.at(z, p.bsw, p.gsw), p.dh, n0, p.dh);
     ph[1].b[1] = ph[1].b[0];
     ph[1].nb = 1;
     ph[1].K = p.d;

@@ -245,15 +245,24 @@ struct NsBatch {
   size_t xoff, sqoff;   // element offsets: [r, c]-shaped buffers (and the update in original orientation); [r, r]-shaped buffers
 };
 
+// Apply steps of consecutive weight versions, equally long and equally spaced: one launch covers all of them.
+struct ApplyGroup {
+  lact_step_t st;                  // the first step
+  int ver, n;                      // its weight version; number of steps
+  int dstart, dout;                // from one step's rows of q, of the output, to the next one's
+};
+
 struct Plan {
   lact_desc_t d;
   std::vector<NsBatch> nsb;
   size_t sq_total = 0;    // elements of one [r, r]-shaped buffer over all batches
   std::vector<lact_step_t> steps;
   std::vector<lact_step_t> live;    // the steps that are executed: `steps` without the apply rows a later step overwrites
+  std::vector<ApplyGroup> groups;   // the apply steps among them whose version is not the newest
+  int group_max = 1;                // largest group
   std::vector<float> coeffs;
   MatGeom g;
-  int nupd = 0, Tcap = 0, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 512;
+  int nupd = 0, Tcap = 0, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 1024, kl_begin = 0, kl_end = 0, side_slots = 1;
   bool muon = false, bf16 = true, momentum = false, state_in = false;
   size_t mat3 = 0;  // 3*b*elems
   // saved
@@ -268,7 +277,7 @@ struct Plan {
   std::vector<int> pre_T;
   // scratch
   size_t t_h[6], t_partial, t_lrpart, t_xf[2], t_xbtmp, t_ss, t_dot, t_mdot, t_gwhat[2], t_gwcur, t_gmcarry, t_gc,
-      t_gxf[2], t_gxb[2], t_sg, t_gas, t_gn0, t_hs[3], t_partial_side[2], t_gwside[2], t_nssync, t_kl[2], t_ca, scratch_bytes;
+      t_gxf[2], t_gxb[2], t_sg, t_gas, t_gn0, t_hs[3], t_hn[3], t_partial_side, t_gwside, t_nssync, t_kl[2], t_ca, scratch_bytes;
 
   int build(const lact_desc_t* desc) {
     if (!desc) return fail("null descriptor");
@@ -370,6 +379,10 @@ struct Plan {
     split_min = muon ? 1536 : 1024;
     nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, 16).n, choose_split(Tcap, tr_tiles(d.d, d.dh) * 3 * d.b, 16, split_min).n);
     mdot_parts = std::max(std::max(nblk, 256), ceil_div(g.maxrows(), 4));
+    build_groups();
+    side_slots = 1;
+    for (int n = 1; n <= group_max; ++n)
+      side_slots = std::max(side_slots, n * std::max(choose_split_async(Tcap, tiles * 3 * d.b * n, 16).n, choose_split(Tcap, tr_tiles(d.d, d.dh) * 3 * d.b * n, 16, split_min).n));
 
     Bump sv;
     s_n0 = sv.take((size_t)3 * d.b * g.maxrows() * 4);
@@ -419,14 +432,46 @@ struct Plan {
     t_gas = sc.take(sq3 * nsz);
     t_gn0 = sc.take((size_t)3 * d.b * g.maxrows() * 4);
     // the apply steps' own buffers (they run beside the update chain)
-    for (int i = 0; i < 3; ++i) t_hs[i] = sc.take((size_t)d.b * Tcap * d.dh * esz);
-    for (int i = 0; i < 2; ++i) t_partial_side[i] = sc.take((size_t)nsplit_max * mat3 * 4);
-    for (int i = 0; i < 2; ++i) t_gwside[i] = sc.take(mat3 * 4);
+    for (int i = 0; i < 3; ++i) t_hs[i] = sc.take((size_t)group_max * d.b * Tcap * d.dh * esz);
+    for (int i = 0; i < 3; ++i) t_hn[i] = sc.take((size_t)d.b * Tcap * d.dh * esz);   // those of the newest version
+    t_partial_side = sc.take((size_t)side_slots * mat3 * 4);
+    t_gwside = sc.take((size_t)std::max(1, groups.empty() ? 0 : nupd) * mat3 * 4);   // by weight version
     t_nssync = sc.take(((size_t)3 * d.b * 32 + 32) * 4);   // per-matrix barrier lines of the fused Newton-Schulz kernel + error word
-    for (int i = 0; i < 2; ++i) t_kl[i] = sc.take((size_t)d.b * Tcap * d.d * esz);   // k * lr0, k * lr2 of the current update
+    // k * lr0, k * lr2 of the tokens [kl_begin, kl_end) that updates read
+    kl_begin = d.kv_len; kl_end = 0;
+    for (const auto& st : steps)
+      if (st.kind == LACT_UPDATE) { kl_begin = std::min(kl_begin, st.start); kl_end = std::max(kl_end, st.end); }
+    for (int i = 0; i < 2; ++i) t_kl[i] = sc.take((size_t)d.b * std::max(0, kl_end - kl_begin) * d.d * esz);
     t_ca = muon ? sc.take(sq3 * nsz) : 0;                   // c * A of the current Newton-Schulz iteration
     scratch_bytes = sc.off + 256;
     return 0;
+  }
+  // Groups of as many steps as it takes to give every compute unit a 128 x 128 tile of the hidden stage.  Fewer, fuller launches,
+  // and fewer event waits at 12 us of host time each: 8 chunks of 64 rows in fp32 526 -> 480 us, 15 of 192 tiles
+  // 2.83 -> 2.79 ms; twice the size gains nothing more and delays the chain, which waits for whole groups (many small chunks with
+  // Newton-Schulz: 839 us, 853 with twice the size).
+  void build_groups() {
+    groups.clear();
+    group_max = 1;
+    int ver = 0;
+    for (const auto& st : live) {
+      if (st.kind == LACT_UPDATE) { ++ver; continue; }
+      if (ver == nupd) continue;
+      const int T = st.end - st.start;
+      const long long tiles1 = (long long)ceil_div(T, 128) * ceil_div(d.dh, 128) * d.b;
+      const int limit = (int)std::max(1LL, std::min(std::min(65535LL / (3 * d.b), 64LL), (256 + tiles1 - 1) / tiles1));
+      if (!groups.empty()) {
+        ApplyGroup& g = groups.back();
+        const int ds = st.start - (g.st.start + (g.n - 1) * g.dstart), dout = st.out_start - (g.st.out_start + (g.n - 1) * g.dout);
+        // rows of q that two steps share would be two additions to one gradient row
+        if (g.n < limit && ver == g.ver + g.n && T == g.st.end - g.st.start && (ds >= T || ds <= -T) && (g.n == 1 || (ds == g.dstart && dout == g.dout))) {
+          g.dstart = ds; g.dout = dout;
+          group_max = std::max(group_max, ++g.n);
+          continue;
+        }
+      }
+      groups.push_back(ApplyGroup{st, ver, 1, 0, 0});
+    }
   }
 };
 
@@ -565,7 +610,7 @@ struct Runner {
   Runner(const Plan& p, void* saved, void* scratch, hipStream_t st)
       : P(p), s(st), sv(align256(saved)), sc(align256(scratch)), d(p.d), s_main(st), s_side(st), s_tail(st), hsel(p.t_h), partial_sel(p.t_partial) {
     side = side_ctx();
-    if (side && g_overlap) { s_side = side->stream; s_tail = side->tail; }
+    if (side && g_overlap && !P.groups.empty()) { s_side = side->stream; s_tail = side->tail; }
   }
   // ---- fused Newton-Schulz: launches of at most 256 resident blocks
   static bool tiles_fit(int r, int c, int bm, int bn) {
@@ -724,7 +769,7 @@ struct Runner {
   // enqueue on the side chain (its stream and buffers) while this object lives
   struct OnSide {
     Runner& r;
-    explicit OnSide(Runner& rr, int sb = 0) : r(rr) { r.s = r.s_side; r.hsel = r.P.t_hs; r.partial_sel = r.P.t_partial_side[sb]; }
+    explicit OnSide(Runner& rr) : r(rr) { r.s = r.s_side; r.hsel = r.P.t_hs; r.partial_sel = r.P.t_partial_side; }
     ~OnSide() { r.s = r.s_main; r.hsel = r.P.t_h; r.partial_sel = r.P.t_partial; }
   };
 
@@ -766,13 +811,14 @@ struct Runner {
   bool hidden_persists(int which) const {
     return d.d % 64 == 0 && ((g_persist >> which) & 1) && side && side->cus > 0 && !(g_persist == 1 && hidden_small(which));
   }
-  void launch_hidden(int which, const HiddenParams& hp, int ver, int T_) const {
-    const double f = (double)T_ * d.d * d.dh * d.b;
+  // steps: steps of the program that the launch covers (apply kernels)
+  void launch_hidden(int which, const HiddenParams& hp, int T_, int steps = 1) const {
+    const int nz = d.b * steps;
+    const double f = (double)T_ * d.d * d.dh * nz;
     if (dma_hidden()) {
       if constexpr (kBf16) {
       HiddenDmaParams q;
       q.h = hp;
-      (void)ver;
       // Tiles.  128 x 128 with three stages, one block per compute unit; where the products are at most three K-steps long
       // (d <= 192) a block's time goes into its first copies and its epilogue, and two smaller blocks per unit overlap
       // theirs.  Measured, us per launch, large / small: 12 heads, d = 128, dh = 256, 4680 tokens: update 52.8 / 46.6,
@@ -794,7 +840,7 @@ struct Runner {
       LACT_BIG_LDS(k_update_bwd_hidden_kept_dma<TS_SQ>, SM3);
       if (which <= 2 && hidden_persists(which)) {
         HiddenPersistParams hq;
-        hq.h = hp; hq.map = make_tile_map(ceil_div(T_, TS_SQ::BM), ceil_div(d.dh, TS_SQ::BN), d.b);
+        hq.h = hp; hq.map = make_tile_map(ceil_div(T_, TS_SQ::BM), ceil_div(d.dh, TS_SQ::BN), nz);
         const dim3 gp(persist_grid(hq.map.grid(), side->cus));
         LACT_BIG_LDS(k_hidden_persist<ApplyHiddenPolicy>, PersistLds<ApplyHiddenPolicy>::BYTES);
         LACT_BIG_LDS(k_hidden_persist<UpdateHiddenPolicy>, PersistLds<UpdateHiddenPolicy>::BYTES);
@@ -808,7 +854,7 @@ struct Runner {
       // tile of the kernel that is launched below: the grid has to cover exactly its tiles
       const int bm = which == 3 && small ? TS_64::BM : 128, bn = which == 3 || small ? 64 : 128;
       static_assert(TS_SQ::BM == 128 && TS_SQ::BN == 128 && TS_BWD::BM == 128 && TS_BWD::BN == 64 && TS_64::BN == 64, "tiles of the hidden-stage kernels");
-      q.map = make_tile_map(ceil_div(T_, bm), ceil_div(d.dh, bn), d.b);
+      q.map = make_tile_map(ceil_div(T_, bm), ceil_div(d.dh, bn), nz);
       const dim3 g(q.map.grid()), t(DMA_THREADS);
       if (which == 0) {
         if (small) LACT_LAUNCH_SMEM("k_apply_hidden_dma", "apply_hidden", 4.0 * f, (k_apply_hidden_dma<TS_BWD, 2, 4>), g, t, SMS, s, q);
@@ -829,7 +875,7 @@ struct Runner {
     } else {
       using TS = TSG<T>;
       constexpr int SM = AsyncPipe<T, 1>::BYTES;
-      const dim3 g(ceil_div(T_, TS::BM), ceil_div(d.dh, TS::BN), d.b);
+      const dim3 g(ceil_div(T_, TS::BM), ceil_div(d.dh, TS::BN), nz);
       LACT_BIG_LDS(k_apply_hidden<T>, SM);
       LACT_BIG_LDS(k_update_hidden<T>, SM);
       LACT_BIG_LDS(k_apply_bwd_hidden<T>, SM);
@@ -892,11 +938,12 @@ struct Runner {
   }
   int token_reduce(const char* site, const TokenReduceJob (&jobs)[3], int tokens, float* add_out = nullptr,
                    const float* add_in = nullptr, float coeff = 0.f, const PrepFold* prep = nullptr,
-                   RowCompanions* rows = nullptr) const {
+                   RowCompanions* rows = nullptr, int steps = 1) const {
+    const int mats = 3 * d.b * steps, max_n = steps > 1 ? 16 : P.nsplit_max;
     TokenReduceParams p;
     memset(&p, 0, sizeof(p));
     for (int i = 0; i < 3; ++i) p.job[i] = jobs[i];
-    p.nb = d.b; p.mat_elems = P.g.elems;
+    p.by_nb = make_udiv(d.b); p.mat_elems = P.g.elems;
     float* partial = scr<float>(partial_sel);
     int slots = 0;
     bool direct = false;
@@ -904,15 +951,14 @@ struct Runner {
       if (tokens >= 64) {     // a ragged end is handled inside the last K-step
         const int tiles = tr_tiles(d.d, d.dh);
         // with the row GEMMs in the launch the chip is busy: short splits only cost (36.4 us in one split, 38.2 in two, 46.8 in four)
-        const Split sp = choose_split(tokens, tiles * 3 * d.b, P.nsplit_max, rows ? 1536 : P.split_min);
+        const Split sp = choose_split(tokens, tiles * mats, max_n, rows ? 1536 : P.split_min);
         TokenReduceDmaParams pd;
         static_cast<TokenReduceParams&>(pd) = p;
         pd.tokens = tokens; pd.split_len = sp.len; pd.partial = partial;
-        pd.map = make_tile_map(sp.n, tiles, 3 * d.b);
-        pd.by_nb = make_udiv(d.b);
+        pd.map = make_tile_map(sp.n, tiles, mats);
         for (int j = 0; j < 3; ++j) pd.by_tn[j] = make_udiv(ceil_div(jobs[j].N, tr_big(d.d, d.dh) ? TS_NS::BN : TS_SQ::BN));
         dim3 g(pd.map.grid());
-        const double fl = 6.0 * tokens * d.d * d.dh * d.b;
+        const double fl = 2.0 * tokens * d.d * d.dh * mats;
         direct = add_out && sp.n == 1;
         const bool folded = prep && sp.n == 1;
         if (folded) {
@@ -949,12 +995,12 @@ struct Runner {
     // fp32, or fewer than 64 tokens
     using TS = TSG<T>;
     constexpr int SM = AsyncPipe<T, 2>::BYTES;
-    const Split sp = choose_split_async(tokens, P.tiles * 3 * d.b, P.nsplit_max);
+    const Split sp = choose_split_async(tokens, P.tiles * mats, max_n);
     direct = add_out && sp.n == 1;
     if (direct) { p.add_out = add_out; p.add_in = coeff != 0.f ? add_in : nullptr; p.coeff = coeff; }
     p.tokens = tokens; p.split_len = sp.len; p.partial = partial;
     LACT_BIG_LDS(k_token_reduce<T>, SM);
-    LACT_LAUNCH_SMEM("k_token_reduce", site, 6.0 * tokens * d.d * d.dh * d.b, (k_token_reduce<T>), dim3(P.tiles, sp.n, 3 * d.b),
+    LACT_LAUNCH_SMEM("k_token_reduce", site, 2.0 * tokens * d.d * d.dh * mats, (k_token_reduce<T>), dim3(P.tiles, sp.n, mats),
                      dim3(TS::THREADS), SM, s, p);
     return direct ? 0 : sp.n;
   }
@@ -1027,65 +1073,63 @@ struct Runner {
     T* upd_z[3] = {nullptr, nullptr, nullptr};   // lr-scaled operands of the current update's gradient GEMMs
     long long upd_zbs = 0;
     bool side_used = false;
-    // Apply steps only need their weight version, which is final once they are met in program order.  They are
-    // held back and enqueued on the side stream at the point of the following update where the chip is least
-    // busy -- in front of its Newton-Schulz kernels, which leave a quarter of the compute units idle -- or at
-    // the end of the program.
-    std::vector<std::pair<const lact_step_t*, int>> pending;   // (apply step, weight version)
-    auto flush_applies = [&](bool beside_update) {
-      if (pending.empty()) return;
-      // with no update left to run beside, the caller's stream is the shortest way (no event hand-over)
-      std::unique_ptr<OnSide> on_side;
-      if (beside_update) {
-        wait_for(s_side, s_main);
-        side_used = true;
-        on_side.reset(new OnSide(*this));
+    // k * lr0, k * lr2 depend on the inputs only and are first read by the first token reduction: one launch, on the tail stream
+    // beside the first kernels of the call where there is one
+    hipEvent_t kl_ready = nullptr;
+    const long long klbs = (long long)(P.kl_end - P.kl_begin) * d.d;
+    if (klbs > 0) {
+      if (entry) {
+        (void)hipStreamWaitEvent(s_tail, entry, 0);
+        s = s_tail;
       }
-      for (auto& pa : pending) {
-        const lact_step_t& st = *pa.first;
-        const int T_ = st.end - st.start, av = pa.second;
-        HiddenParams hp = hidden_params(T_, q + (size_t)st.start * d.q_ld, d.q_ld, d.q_bs, nullptr, 0, 0, av);
-        hp.O0 = h(0);
-        launch_hidden(0, hp, av, T_);
-        auto p = row_params<1>();
-        set_term(p.t[0], h(0), d.dh, hbs(), wc(av, 1), d.dh, P.g.elems, d.dh);
-        p.M = T_; p.N = d.d; p.out = out + (size_t)st.out_start * d.o_ld; p.ldo = d.o_ld; p.bso = d.o_bs;
-        launch_row_gemm<T, true, 1, EPI_STORE>("apply_out", p, d.b, s, true);
+      LACT_LAUNCH("k_lr_scale_rows", "update_lr_k", 0.0, (k_lr_scale_rows<T>), dim3((unsigned)((klbs / 4 + 255) / 256), d.b), dim3(256), s,
+                  k + (size_t)P.kl_begin * d.k_ld, d.k_ld, d.k_bs, lr0 + P.kl_begin, lr2 + P.kl_begin, (long long)d.kv_len, P.kl_end - P.kl_begin, d.d,
+                  scr<T>(P.t_kl[0]), scr<T>(P.t_kl[1]), klbs);
+      if (entry) {
+        kl_ready = side->event();
+        (void)hipEventRecord(kl_ready, s_tail);
+        s = s_main;
       }
-      pending.clear();
+    }
+    // Apply steps only need their weight version.  A group of them is enqueued when its last version is final, on the side stream
+    // and at the point of the following update where the chip is least busy -- in front of its Newton-Schulz kernels, which leave
+    // a quarter of the compute units idle; the newest version's at the end, on the caller's stream.
+    auto apply = [&](const ApplyGroup& g) {
+      const int T_ = g.st.end - g.st.start;
+      HiddenParams hp = hidden_params(T_, q + (size_t)g.st.start * d.q_ld, d.q_ld, d.q_bs, nullptr, 0, 0, g.ver);
+      hp.O0 = h(0);
+      auto p = row_params<1>();
+      set_term(p.t[0], h(0), d.dh, hbs(), wc(g.ver, 1), d.dh, P.g.elems, d.dh);
+      p.M = T_; p.N = d.d; p.out = out + (size_t)g.st.out_start * d.o_ld; p.ldo = d.o_ld; p.bso = d.o_bs;
+      if (g.n > 1) {
+        hp.steps.by_nb = p.steps.by_nb = make_udiv(d.b);
+        hp.gsx = (long long)g.dstart * d.q_ld; hp.gsw = (long long)P.mat3;
+        p.t[0].gsB = (long long)P.mat3; p.gso = (long long)g.dout * d.o_ld;
+      }
+      launch_hidden(0, hp, T_, g.n);
+      launch_row_gemm<T, true, 1, EPI_STORE>("apply_out", p, d.b * g.n, s, true);
+    };
+    size_t next_group = 0;
+    auto flush_groups = [&]() {   // those whose versions exist
+      size_t end = next_group;
+      while (end < P.groups.size() && P.groups[end].ver + P.groups[end].n - 1 <= ver) ++end;
+      if (end == next_group) return;
+      wait_for(s_side, s_main);
+      side_used = true;
+      OnSide on_side(*this);
+      for (; next_group < end; ++next_group) apply(P.groups[next_group]);
     };
     for (const auto& st : P.live) {
       const int T_ = st.end - st.start;
       if (st.kind == LACT_APPLY) {
-        pending.emplace_back(&st, ver);
-        if (s_side == s_main) flush_applies(false);   // one stream: plain program order
+        if (ver == P.nupd) apply(ApplyGroup{st, ver, 1, 0, 0});
         continue;
       }
       // ---- update
       const T* kc = k + (size_t)st.start * d.k_ld;
       const T* vc = v + (size_t)st.start * d.v_ld;
-      T* kl0 = scr<T>(P.t_kl[0]);
-      T* kl2 = scr<T>(P.t_kl[1]);
-      const long long klbs = (long long)P.Tcap * d.d;
-      // k * lr0, k * lr2 depend on the inputs only and are first read by the token reduction: they are written on the
-      // tail stream beside the hidden stage -- after everything enqueued so far (which includes the previous update's
-      // reduction that read the same two buffers), the first update's already beside the state set-up of the call
-      hipEvent_t kl_ready = nullptr;
-      {
-        const bool aside = s_tail != s_main && side;
-        if (aside) {
-          if (u == 0 && entry) (void)hipStreamWaitEvent(s_tail, entry, 0);
-          else wait_for(s_tail, s_main);
-          s = s_tail;
-        }
-        LACT_LAUNCH("k_lr_scale_rows", "update_lr_k", 0.0, (k_lr_scale_rows<T>), dim3((unsigned)(((long long)T_ * d.d / 4 + 255) / 256), d.b), dim3(256), s,
-                    kc, d.k_ld, d.k_bs, lr0 + st.start, lr2 + st.start, (long long)d.kv_len, T_, d.d, kl0, kl2, klbs);
-        if (aside) {
-          kl_ready = side->event();
-          (void)hipEventRecord(kl_ready, s_tail);
-          s = s_main;
-        }
-      }
+      const T* kl0 = scr<T>(P.t_kl[0]) + (size_t)(st.start - P.kl_begin) * d.d;
+      const T* kl2 = scr<T>(P.t_kl[1]) + (size_t)(st.start - P.kl_begin) * d.d;
       {
         HiddenParams hp = hidden_params(T_, kc, d.k_ld, d.k_bs, vc, d.v_ld, d.v_bs, ver);
         hp.lr0 = lr0 + st.start; hp.lr1 = lr1 + st.start; hp.lr2 = lr2 + st.start; hp.bslr = d.kv_len;
@@ -1100,7 +1144,7 @@ struct Runner {
           hp.bso = zbs;
         }
         hp.O0 = z0; hp.O1 = z1; hp.O2 = z2;
-        launch_hidden(1, hp, ver, T_);
+        launch_hidden(1, hp, T_);
         upd_z[0] = z0; upd_z[1] = z1; upd_z[2] = z2; upd_zbs = zbs;
       }
       // the pre-Muon gradient (= the momentum state) of the last update: read by nothing when Newton-Schulz output is
@@ -1108,6 +1152,7 @@ struct Runner {
       const bool d_unread = P.muon && !d.muon_replaces_weight && u + 1 == P.nupd;
       int dw_slots = 0;
       if (kl_ready) (void)hipStreamWaitEvent(s_main, kl_ready, 0);
+      kl_ready = nullptr;
       {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));
@@ -1149,7 +1194,7 @@ struct Runner {
         if (ns_fwd_one_launch()) p.clear = ns_clear(true);
         LACT_LAUNCH("k_momentum_prep", "k_momentum_prep", 0.0, (k_momentum_prep<TN>), dim3(P.nblk, 3 * d.b), dim3(256), s, p);
       }
-      flush_applies(true);
+      flush_groups();
       if (P.muon) {
         const bool scale_in_kernel = ns_fwd_one_launch();
         if (!scale_in_kernel) {
@@ -1238,7 +1283,6 @@ struct Runner {
       ++ver;
       ++u;
     }
-    flush_applies(false);
     if (side_used) wait_for(s_main, s_side);
     // final weights and momentum state: written by the last update's kernels, or by the first kernel when no update runs
     if (m_out && (m_out[0] || m_out[1] || m_out[2])) {
@@ -1327,13 +1371,14 @@ struct Runner {
       const float* base = nullptr; int n = 0;
       bool any() const { return base || n; }
     } gw;
-    // another contribution to `g`, on the current stream; `buf`: where a full array of it goes
-    auto contribute = [&](const char* site, const TokenReduceJob (&jobs)[3], int tokens, GradSum& g, float* buf, RowCompanions* rows) {
-      if (g.n)   // the partial-sum buffer is taken
-        LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, buf, g.base, 1.f, scr<float>(partial_sel), g.n, (long long)P.mat3);
-      if (g.n) g = GradSum{buf, 0};
-      const int n = token_reduce(site, jobs, tokens, buf, g.base, g.base ? 1.f : 0.f, nullptr, rows);
-      g = n ? GradSum{g.base, n} : GradSum{buf, 0};
+    // another contribution to `g` on the main chain; `rows`: GEMMs that may ride in its launch
+    auto contribute = [&](const char* site, const TokenReduceJob (&jobs)[3], int tokens, GradSum& g, RowCompanions* rows) {
+      if (g.n) {   // the partial-sum buffer is taken
+        LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, flat, dim3(256), s, gwcur, g.base, 1.f, scr<float>(P.t_partial), g.n, (long long)P.mat3);
+        g = GradSum{gwcur, 0};
+      }
+      const int n = token_reduce(site, jobs, tokens, gwcur, g.base, g.base ? 1.f : 0.f, nullptr, rows);
+      g = n ? GradSum{g.base, n} : GradSum{gwcur, 0};
     };
     if (dwf && (dwf[0] || dwf[1] || dwf[2])) {
       gw.base = gwcur;
@@ -1397,21 +1442,92 @@ struct Runner {
       return zl.launched;
     };
     if (!rows_on_side) zero_rows(s_main);
-    // The apply steps run on the side stream.  Their weight gradients go to gw_side[version & 1] and are added
-    // by the consumer of that version's gradient (the renorm backward of the update that made the version, or
-    // the final kernel); `free_ev` orders the reuse of a gw_side buffer after its consumer.
-    wait_for(s_side, s_main);
-    float* gw_side[2] = {scr<float>(P.t_gwside[0]), scr<float>(P.t_gwside[1])};
-    GradSum side_sum[2];
-    hipEvent_t free_ev[2] = {nullptr, nullptr};
-    hipEvent_t dw_done[2] = {nullptr, nullptr};   // newest weight-gradient kernel of the apply steps per buffer
     bool side_used = false;
-    if (rows_on_side && zero_rows(s_side)) side_used = true;
-    hipEvent_t main_dq_ev = nullptr;   // a dq GEMM on the side stream still reads the main chain's intermediates
-    auto wait_main_dq = [&]() {
-      if (main_dq_ev) (void)hipStreamWaitEvent(s_main, main_dq_ev, 0);
-      main_dq_ev = nullptr;
+    // Backward of apply steps: weight gradients to full arrays by version (`g.ver` and on; `add`: to what they hold), dq
+    auto apply_jobs = [&](const ApplyGroup& g, TokenReduceJob (&jobs)[3]) {
+      const T* qc = q + (size_t)g.st.start * d.q_ld;
+      const T* gc = dout + (size_t)g.st.out_start * d.do_ld;
+      memset(jobs, 0, sizeof(jobs));
+      jobs[0].M = jobs[2].M = d.dh; jobs[0].N = jobs[2].N = d.d;
+      set_tr_term(jobs[0].t, h(1), d.dh, hbs(), qc, d.q_ld, d.q_bs);
+      jobs[1].M = d.d; jobs[1].N = d.dh;
+      set_tr_term(jobs[1].t, gc, d.do_ld, d.do_bs, h(0), d.dh, hbs());
+      set_tr_term(jobs[2].t, h(2), d.dh, hbs(), qc, d.q_ld, d.q_bs);
+      const long long gsh = (long long)d.b * hbs();
+      jobs[0].t.gsA = jobs[2].t.gsA = jobs[1].t.gsB = gsh;
+      jobs[0].t.gsB = jobs[2].t.gsB = (long long)g.dstart * d.q_ld;
+      jobs[1].t.gsA = (long long)g.dout * d.do_ld;
     };
+    auto apply_hidden_bwd = [&](const ApplyGroup& g) {
+      const int T_ = g.st.end - g.st.start;
+      HiddenParams hp = hidden_params(T_, q + (size_t)g.st.start * d.q_ld, d.q_ld, d.q_bs, dout + (size_t)g.st.out_start * d.do_ld, d.do_ld, d.do_bs, g.ver);
+      hp.O0 = h(0); hp.O1 = h(1); hp.O2 = h(2);
+      if (g.n > 1) {
+        hp.steps.by_nb = make_udiv(d.b);
+        hp.gsx = (long long)g.dstart * d.q_ld; hp.gsy = (long long)g.dout * d.do_ld; hp.gsw = (long long)P.mat3;
+      }
+      launch_hidden(2, hp, T_, g.n);
+    };
+    auto dq_gemm = [&](const ApplyGroup& g) {   // dq = gY0 W0 + gY2 W2
+      const int T_ = g.st.end - g.st.start;
+      auto p = row_params<2>();
+      set_term(p.t[0], h(1), d.dh, hbs(), wc(g.ver, 0), d.d, P.g.elems, d.dh);
+      set_term(p.t[1], h(2), d.dh, hbs(), wc(g.ver, 2), d.d, P.g.elems, d.dh);
+      p.M = T_; p.N = d.d; p.ldo = d.d; p.bso = (long long)d.q_len * d.d;
+      int acc = 0;
+      std::vector<char> accs(g.n);
+      for (int i = 0; i < g.n; ++i) acc += accs[i] = seen_q.accumulate(g.st.start + i * g.dstart, g.st.end + i * g.dstart);
+      const bool together = acc == 0 || acc == g.n;
+      for (int i = 0; i < (together ? 1 : g.n); ++i) {
+        auto pi = p;
+        pi.out = dq + (size_t)(g.st.start + i * g.dstart) * d.d;
+        pi.accumulate = accs[i];
+        if (together && g.n > 1) {
+          pi.steps.by_nb = make_udiv(d.b);
+          pi.t[0].gsB = pi.t[1].gsB = (long long)P.mat3; pi.gso = (long long)g.dstart * d.d;
+        }
+        for (int t = 0; t < 2 && i > 0; ++t) {
+          pi.t[t].A = (const T*)pi.t[t].A + (size_t)i * d.b * hbs();
+          pi.t[t].B = (const T*)pi.t[t].B + (size_t)i * P.mat3;
+        }
+        launch_row_gemm<T, false, 2, EPI_STORE>("apply_bwd_dq", pi, d.b * (together ? g.n : 1), s, true);
+      }
+    };
+    // The steps on earlier versions need nothing of the chain below: group by group in the order in which the chain asks for them,
+    // all enqueued in front of it on the side stream.  `ready[version]`: the newest kernel that its gradient waits for.
+    std::vector<float*> gw_side(P.nupd + 1, nullptr);   // null: no apply step on that version
+    std::vector<hipEvent_t> ready(P.nupd + 1, nullptr);
+    auto apply_groups = [&]() {
+      OnSide on_side(*this);
+      if (rows_on_side) zero_rows(s);
+      for (size_t gi = P.groups.size(); gi-- > 0;) {
+        const ApplyGroup& g = P.groups[gi];
+        const int T_ = g.st.end - g.st.start;
+        side_used = true;
+        apply_hidden_bwd(g);
+        float* dst = scr<float>(P.t_gwside) + (size_t)g.ver * P.mat3;
+        bool add = false;
+        for (int i = 0; i < g.n; ++i) add = add || gw_side[g.ver + i];
+        if (add)   // another step on one of these versions came before
+          for (int i = 0; i < g.n; ++i)
+            if (!gw_side[g.ver + i]) LACT_LAUNCH("k_fill_f32", "k_fill_f32", 0.0, k_fill_f32, dim3((unsigned)((P.mat3 + 255) / 256)), dim3(256), s, dst + i * P.mat3, 0.f, (long long)P.mat3);
+        TokenReduceJob jobs[3];
+        apply_jobs(g, jobs);
+        if (const int n = token_reduce("apply_bwd_dw", jobs, T_, dst, dst, add ? 1.f : 0.f, nullptr, nullptr, g.n)) {
+          const long long all = (long long)g.n * P.mat3;
+          LACT_LAUNCH("k_reduce_partials", "k_reduce_partials", 0.0, k_reduce_partials, dim3((unsigned)((all / 4 + 255) / 256)), dim3(256), s, dst, add ? dst : nullptr, 1.f, scr<float>(P.t_partial_side), n, all);
+        }
+        hipEvent_t e = nullptr;
+        if (s_side != s_main) {
+          e = side->event();
+          (void)hipEventRecord(e, s_side);
+        }
+        for (int i = 0; i < g.n; ++i) { gw_side[g.ver + i] = dst + i * P.mat3; ready[g.ver + i] = e; }
+        dq_gemm(g);
+      }
+    };
+    bool groups_started = false;
+    hipEvent_t waited = nullptr;
     int ver = P.nupd, u = P.nupd;
     int carry_main = -1;       // index of the gwhat buffer holding the accumulator's gradient (pre-norm)
     bool gm_valid = false;     // gmcarry holds d loss / d (momentum state after update u-1)
@@ -1419,64 +1535,32 @@ struct Runner {
       const lact_step_t& st = P.live[si];
       const int T_ = st.end - st.start;
       if (st.kind == LACT_APPLY) {
-        const T* qc = q + (size_t)st.start * d.q_ld;
-        const T* gc = dout + (size_t)st.out_start * d.do_ld;
-        auto dw_jobs = [&](TokenReduceJob (&jobs)[3]) {
-          memset(jobs, 0, sizeof(jobs));
-          jobs[0].M = d.dh; jobs[0].N = d.d;
-          set_tr_term(jobs[0].t, h(1), d.dh, hbs(), qc, d.q_ld, d.q_bs);
-          jobs[1].M = d.d; jobs[1].N = d.dh;
-          set_tr_term(jobs[1].t, gc, d.do_ld, d.do_bs, h(0), d.dh, hbs());
-          jobs[2].M = d.dh; jobs[2].N = d.d;
-          set_tr_term(jobs[2].t, h(2), d.dh, hbs(), qc, d.q_ld, d.q_bs);
-        };
-        auto dq_gemm = [&]() {   // dq = gY0 W0 + gY2 W2
-          auto p = row_params<2>();
-          set_term(p.t[0], h(1), d.dh, hbs(), wc(ver, 0), d.d, P.g.elems, d.dh);
-          set_term(p.t[1], h(2), d.dh, hbs(), wc(ver, 2), d.d, P.g.elems, d.dh);
-          p.M = T_; p.N = d.d; p.out = dq + (size_t)st.start * d.d; p.ldo = d.d; p.bso = (long long)d.q_len * d.d;
-          p.accumulate = seen_q.accumulate(st.start, st.end);
-          launch_row_gemm<T, false, 2, EPI_STORE>("apply_bwd_dq", p, d.b, s, true);
-        };
-        if (ver == P.nupd) {
-          // Applies of the newest weight version: the update chain cannot start before their weight gradients,
-          // so they stay on the caller's stream (no event hand-over in the critical path); only dq, which nothing
-          // waits for, goes to the side stream and reads this chain's intermediates.
-          wait_main_dq();
-          HiddenParams hp = hidden_params(T_, qc, d.q_ld, d.q_bs, gc, d.do_ld, d.do_bs, ver);
-          hp.O0 = h(0); hp.O1 = h(1); hp.O2 = h(2);
-          launch_hidden(2, hp, ver, T_);
-          wait_for(s_side, s_main);
-          TokenReduceJob jobs[3];
-          dw_jobs(jobs);
-          contribute("apply_bwd_dw", jobs, T_, gw, gwcur, nullptr);
-          s = s_side;
-          dq_gemm();
-          s = s_main;
-          if (side && s_side != s_main) {
-            main_dq_ev = side->event();
-            (void)hipEventRecord(main_dq_ev, s_side);
-            side_used = true;
-          }
-          continue;
-        }
-        const int sb = ver & 1;
-        if (!side_sum[sb].any() && free_ev[sb] && s_side != s_main) {
-          (void)hipStreamWaitEvent(s_side, free_ev[sb], 0);
-          free_ev[sb] = nullptr;
-        }
-        side_used = true;
-        OnSide on_side(*this, sb);
-        HiddenParams hp = hidden_params(T_, qc, d.q_ld, d.q_bs, gc, d.do_ld, d.do_bs, ver);
-        hp.O0 = h(0); hp.O1 = h(1); hp.O2 = h(2);
-        launch_hidden(2, hp, ver, T_);
+        if (ver < P.nupd) continue;   // in a group
+        // Applies of the newest weight version: the update chain cannot start before their weight gradients, so they stay on the
+        // caller's stream; only the last one's dq, which nothing waits for, goes to the side stream (its operands have buffers of
+        // their own).
+        const ApplyGroup g{st, ver, 1, 0, 0};
+        hsel = P.t_hn;
+        apply_hidden_bwd(g);
         TokenReduceJob jobs[3];
-        dw_jobs(jobs);
-        contribute("apply_bwd_dw", jobs, T_, side_sum[sb], gw_side[sb], nullptr);
-        dw_done[sb] = side ? side->event() : nullptr;
-        if (dw_done[sb] && s_side != s_main) (void)hipEventRecord(dw_done[sb], s_side);
-        dq_gemm();
+        apply_jobs(g, jobs);
+        contribute("apply_bwd_dw", jobs, T_, gw, nullptr);
+        const bool last = si == 0 || P.live[si - 1].kind == LACT_UPDATE;
+        if (last && s_side != s_main) {
+          wait_for(s_side, s_main);
+          groups_started = side_used = true;
+          s = s_side;
+        }
+        dq_gemm(g);
+        s = s_main;
+        hsel = P.t_h;
+        if (groups_started) apply_groups();
         continue;
+      }
+      if (!groups_started) {
+        groups_started = true;
+        wait_for(s_side, s_main);
+        apply_groups();
       }
       // ---- update u-1: weights ver-1 -> ver
       --u;
@@ -1490,13 +1574,11 @@ struct Runner {
         RenormParams p = renorm_params(u, vprev);
         p.gy = gw.base;
         p.gyp = partials(P.t_partial, gw.n);
-        const int sb = ver & 1;
-        if (side_sum[sb].any()) {
-          // wait for the apply steps' weight gradients only (their dq GEMMs may still be running)
-          if (dw_done[sb] && s_side != s_main) (void)hipStreamWaitEvent(s_main, dw_done[sb], 0);
-          p.gy2 = side_sum[sb].base;
-          p.gyp2 = partials(P.t_partial_side[sb], side_sum[sb].n);
+        if (ready[ver] && ready[ver] != waited) {   // for the weight gradients only: dq GEMMs may still be running
+          waited = ready[ver];
+          (void)hipStreamWaitEvent(s_main, waited, 0);
         }
+        p.gy2 = gw_side[ver];
         p.carry_in = (d.prenorm && carry_main >= 0) ? scr<float>(P.t_gwhat[carry_main]) : nullptr;
         p.gw_hat = gwhat;
         p.gn0 = gn0; p.gn0_init = !gn0_written;
@@ -1513,13 +1595,6 @@ struct Runner {
           }
         }
         LACT_LAUNCH("k_renorm_bwd", "k_renorm_bwd", 0.0, (k_renorm_bwd<T, TN>), rowgrid, dim3(256), s, p);
-        if (side_sum[sb].any()) {
-          side_sum[sb] = GradSum();
-          if (side) {
-            free_ev[sb] = side->event();
-            (void)hipEventRecord(free_ev[sb], s_main);
-          }
-        }
       }
       if (d.prenorm) carry_main = gw_idx;
       // The backward of the Frobenius normalisation as the fused kernel's last stages: the partial dots always
@@ -1667,8 +1742,7 @@ struct Runner {
           hp.O3 = hp.O4 = hp.O5 = nullptr;
           z0 = pre(u, 0); z1 = pre(u, 1); z2 = pre(u, 2); zbs = pre_bs(u);
         }
-        wait_main_dq();
-        launch_hidden(P.keep_pre ? 4 : 3, hp, vprev, T_);
+        launch_hidden(P.keep_pre ? 4 : 3, hp, T_);
       }
       const bool acc_kv = seen_kv.accumulate(st.start, st.end);
       // dk and dv share the launch of the token reduction below (when it runs on the asynchronous-copy kernel; otherwise they are
@@ -1715,7 +1789,7 @@ struct Runner {
         set_tr_term(jobs[2].t, h(2), d.dh, hbs(), kc, d.k_ld, d.k_bs);
         // the update before: its weights enter these as they are, unless Newton-Schulz output replaces them or an accumulator carries on
         gw = GradSum{(d.prenorm || (P.muon && d.muon_replaces_weight)) ? nullptr : gwhat, 0};
-        contribute(kBf16 ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, gwcur, &rows_job);
+        contribute(kBf16 ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, &rows_job);
         if (!rows_job.done) {
           launch_row_gemm<T, false, 4, EPI_STORE>("update_bwd_dk", rows_job.r4, d.b, s, true);
           launch_row_gemm<T, true, 2, EPI_STORE>("update_bwd_dv", rows_job.r2, d.b, s, true);
@@ -1759,7 +1833,7 @@ struct Runner {
       memset(&p, 0, sizeof(p));
       if (side_used) wait_for(s_main, s_side);
       p.g = P.g; p.gw = gw.base; p.gwp = partials(P.t_partial, gw.n);
-      p.gw2 = side_sum[0].base; p.gwp2 = partials(P.t_partial_side[0], side_sum[0].n);
+      p.gw2 = gw_side[0];
       p.carry = (d.prenorm && carry_main >= 0) ? scr<float>(P.t_gwhat[carry_main]) : nullptr;
       p.gn0 = gn0; p.n0 = n0(); p.w_init = wf(0);
       p.through_norms = d.detach_norms ? 0 : 1;

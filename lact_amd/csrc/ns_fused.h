@@ -118,11 +118,12 @@ __device__ __forceinline__ RowGemmDmaParams<NT> ns_row_params() {
   q.g.accumulate = 0; q.g.aux = nullptr; q.g.ldaux = 0; q.g.bsaux = 0; q.g.alpha = 1.f; q.g.beta = 0.f;
   q.g.out_c = nullptr; q.g.out_t = nullptr; q.g.transpose_mask = 0; q.g.nb = 1; q.g.round_out_bf16 = 0;
   q.g.out2 = nullptr; q.g.alpha2 = 0.f;
+  q.g.steps = StepBatch{{0, 0, 0}}; q.g.gso = 0;
   q.out_ct = nullptr;
   return q;
 }
 __device__ __forceinline__ void ns_term(RowGemmTerm& t, const void* A, int lda, long long bsA, const void* B, int ldb, long long bsB, int K) {
-  t.A = A; t.lda = lda; t.bsA = bsA; t.B = B; t.ldb = ldb; t.bsB = bsB; t.K = K;
+  t.A = A; t.lda = lda; t.bsA = bsA; t.B = B; t.ldb = ldb; t.bsB = bsB; t.gsB = 0; t.K = K;
 }
 
 // <gx, g16> over one TS::BM x TS::BN tile whose first element is at offset zo of both arrays (row stride c): every thread

@@ -307,7 +307,7 @@ struct RenormParams {
   // backward only
   const float* gy;                 // gradient w.r.t. the new weights, or null (= zero)
   const float* gy2;                // second addend of the same gradient (the apply steps' share), or null
-  Partials gyp, gyp2;              // more of it, as partial sums of token reductions
+  Partials gyp;                    // more of it, as partial sums of a token reduction
   const float* carry_in;           // gradient arriving at the accumulator from later steps (pre-norm) or null
   float* gw_hat;                   // gradient w.r.t. w_hat, original orientation
   float* gn0;                      // [3b][maxrows], accumulated (written when gn0_init: first use in a backward pass)
@@ -336,7 +336,6 @@ __device__ __forceinline__ float4 renorm_w_hat4(const RenormParams& p, size_t of
 __device__ __forceinline__ float4 renorm_gy4(const RenormParams& p, size_t off) {
   float4 g = p.gy ? ld4(p.gy + off) : f4(0.f, 0.f, 0.f, 0.f);
   add_partials(g, p.gyp, off);
-  add_partials(g, p.gyp2, off);
   if (p.gy2) {
     const float4 t = ld4(p.gy2 + off);
     g.x += t.x; g.y += t.y; g.z += t.z; g.w += t.w;
@@ -692,7 +691,7 @@ __global__ void k_lr_reduce(const float* lrpart, long long upd_stride, long long
 // final weight gradients: state gradient (+ accumulator carry) + the path through the initial row norms
 struct FinishParams {
   MatGeom g;
-  const float* gw; const float* gw2; Partials gwp, gwp2; const float* carry; const float* gn0; const float* n0; const float* w_init;   // gw, gw2, gwp, gwp2: addends, nullable
+  const float* gw; const float* gw2; Partials gwp; const float* carry; const float* gn0; const float* n0; const float* w_init;   // gw, gw2, gwp: addends, nullable
   int through_norms;
   float* out[3];
 };
@@ -709,7 +708,6 @@ __global__ void k_finish_weight_grads(const FinishParams p) {
     v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
   }
   add_partials(v, p.gwp, o);
-  add_partials(v, p.gwp2, o);
   if (p.carry) {
     const float4 t = ld4(p.carry + o);
     v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;

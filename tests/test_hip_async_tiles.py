@@ -67,6 +67,30 @@ def test_several_apply_steps_on_one_weight_version(dtype, C):
         assert O.rel_l2(a, r) < (1e-5 if dtype == torch.float32 else 1e-2), n
 
 
+@pytest.mark.parametrize("dtype,b,C,order", [(torch.float32, 2, 72, (0, 1, 2, 3, 4)), (torch.bfloat16, 3, 136, (4, 3, 2, 1, 0)),
+                                             (torch.bfloat16, 1, 64, (0, 2, 4, 1, 3)), (torch.float32, 1, 40, (2, 2, 2, 1, 0))])
+def test_apply_steps_of_several_versions_in_one_launch(dtype, b, C, order):
+    """Apply steps on consecutive weight versions, equally spaced (ascending, descending, in two runs) or on the same rows, against
+    the same steps cut in halves, which no launch covers together: outputs and gradients agree."""
+    print("[gpu-test] grouped applies", dtype, b, C, order, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    n = len(order)
+    inp = {k: t.to("cuda") for k, t in O.make_inputs(b, n * C, 48, 80, seed=36, act_dtype=dtype).items()}
+    go = torch.randn(b, n * C, 48, generator=torch.Generator().manual_seed(6)).to(dtype).to("cuda")
+    res = []
+    for parts in (1, 2):
+        steps, h = [], C // parts
+        for i, a in enumerate(order):
+            steps += [(LACT_APPLY, a * C + p * h, a * C + (p + 1) * h, i * C + p * h) for p in range(parts)]
+            steps.append((LACT_UPDATE, i * C, (i + 1) * C, 0))
+        x = [inp[k].clone().requires_grad_(True) for k in ORDER]
+        out, _, _ = ops.run_program(ops.Program(steps=tuple(steps), out_len=n * C), *x)
+        res.append([out] + list(torch.autograd.grad(out, x, go)))
+    for k, a, r in zip(("out",) + ORDER, *res):
+        assert O.rel_l2(a, r) < (1e-5 if dtype == torch.float32 else 1e-2), k
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("d,dh", [(128, 256), (72, 40), (8, 72)])
 def test_transposed_weights_are_read_as_they_lie(dtype, d, dh):

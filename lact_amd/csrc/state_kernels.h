@@ -198,32 +198,69 @@ struct MomentumPrepParams {
   int round_partial_bf16;             // the reduction GEMM's result is a bf16 tensor in the reference
   ClearWords clear;
 };
+// A matrix that Newton-Schulz holds transposed goes through LDS in tiles of 64 rows x 32 columns: whole 128-byte segments on both
+// sides.  Element by element the launch took 96 us for 6 matrices of 768 x 1536 (two of three transposed), bound by its 2-byte
+// stores; tile by tile 24 us.
 template <typename TN>
-__global__ void k_momentum_prep(const MomentumPrepParams p) {
+struct TallTile {
+  static constexpr int R = 64, C = 32, LD = R + 16 / sizeof(TN);   // a column of the tile is a row of the transposed matrix
+  __device__ static __forceinline__ int count(int rows, int cols) { return ((rows + R - 1) / R) * ((cols + C - 1) / C); }
+  // this thread's quads of four columns: row row(i), columns from col(), i < 2 (256 threads)
+  __device__ static __forceinline__ int row(int i) { return (threadIdx.x >> 3) + 32 * i; }
+  __device__ static __forceinline__ int col() { return (threadIdx.x & 7) * 4; }
+  __device__ static __forceinline__ void put(TN* tile, int i, const float4& f) {
+    TN* t = tile + col() * LD + row(i);
+    Elem<TN>::store(t, f.x); Elem<TN>::store(t + LD, f.y); Elem<TN>::store(t + 2 * LD, f.z); Elem<TN>::store(t + 3 * LD, f.w);
+  }
+  // the tile at (r0, c0) to the transposed matrix whose rows are nr long
+  __device__ static __forceinline__ void copy_out(const TN* tile, TN* out, int r0, int c0, int rows, int cols, int nr) {
+    constexpr int G = 16 / sizeof(TN), PER = R / G;   // granules of 16 bytes per column
+    for (int q = threadIdx.x; q < C * PER; q += 256) {
+      const int c = q / PER, r = (q % PER) * G;
+      // rows come in multiples of 8: a granule is there as a whole or not at all
+      if (c0 + c < cols && r0 + r < rows) *reinterpret_cast<uint4*>(out + (size_t)(c0 + c) * nr + r0 + r) = *reinterpret_cast<const uint4*>(tile + c * LD + r);
+    }
+  }
+};
+
+template <typename TN>
+__global__ __launch_bounds__(256) void k_momentum_prep(const MomentumPrepParams p) {
   __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) TN tile[TallTile<TN>::C * TallTile<TN>::LD];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   clear_words(p.clear, blockIdx.x == 0 && blockIdx.y == 0);
-  const FlatRange R(p.g.elems);
   const float mb = (p.m_prev && p.mbar) ? p.mbar[ib] : 0.f;
   const size_t zo = (size_t)z * p.g.elems;
   float* ext = p.m_ext[j] ? p.m_ext[j] + (size_t)ib * p.g.elems : nullptr;
-  const bool contiguous = p.g.x_contiguous(j);
-  const size_t xo = p.g.ns_base(p.g.ns_of(z));
+  TN* g16 = reinterpret_cast<TN*>(p.g16) + p.g.ns_base(p.g.ns_of(z));
   float ss = 0.f;
-  for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
+  // one quad of the gradient: stored where it goes in its own orientation; returned as Newton-Schulz takes it
+  auto quad = [&](long long e) {
     const float4 v = momentum4(p.dw, zo + e, p.round_partial_bf16, p.m_prev, mb);
     if (p.d_out) st4(p.d_out + zo + e, v);
     if (ext) st4(ext + e, v);
-    if (p.g16) {
-      const float4 f = f4(Elem<TN>::rnd(v.x), Elem<TN>::rnd(v.y), Elem<TN>::rnd(v.z), Elem<TN>::rnd(v.w));
-      TN* g = reinterpret_cast<TN*>(p.g16) + xo;
-      if (contiguous) {
-        Elem<TN>::store4(g + p.g.xidx(j, e), f.x, f.y, f.z, f.w);
-      } else {
-        Elem<TN>::store(g + p.g.xidx(j, e), f.x); Elem<TN>::store(g + p.g.xidx(j, e + 1), f.y);
-        Elem<TN>::store(g + p.g.xidx(j, e + 2), f.z); Elem<TN>::store(g + p.g.xidx(j, e + 3), f.w);
-      }
-      ss += dot4(f, f);
+    const float4 f = f4(Elem<TN>::rnd(v.x), Elem<TN>::rnd(v.y), Elem<TN>::rnd(v.z), Elem<TN>::rnd(v.w));
+    ss += dot4(f, f);
+    return f;
+  };
+  if (!p.g16 || p.g.x_contiguous(j)) {
+    const FlatRange R(p.g.elems);
+    for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
+      const float4 f = quad(e);
+      if (p.g16) Elem<TN>::store4(g16 + p.g.xidx(j, e), f.x, f.y, f.z, f.w);
+    }
+  } else {
+    using TT = TallTile<TN>;
+    const int rows = p.g.rows(j), cols = p.g.cols(j), tc = (cols + TT::C - 1) / TT::C, nr = p.g.ns_rows(j);
+    g16 += p.g.xidx(j, 0);   // row 0 of this matrix inside a stacked pair
+    for (int t = blockIdx.x; t < TT::count(rows, cols); t += gridDim.x) {
+      const int r0 = t / tc * TT::R, c0 = t % tc * TT::C;
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (r0 + TT::row(i) < rows && c0 + TT::col() < cols) TT::put(tile, i, quad((long long)(r0 + TT::row(i)) * cols + c0 + TT::col()));
+      __syncthreads();
+      TT::copy_out(tile, g16, r0, c0, rows, cols, nr);
+      __syncthreads();
     }
   }
   if (p.g16) {
@@ -516,26 +553,36 @@ __global__ void k_renorm_bwd(const RenormParams p) {
 // A gradient given in the original orientation of its matrices, copied to where Newton-Schulz holds them (fp32 and
 // Newton-Schulz type).  Grid (chunks, matrices).
 template <typename TN>
-__global__ void k_to_ns_orientation(const MatGeom g, const float* in, float* xf, void* xb) {
+__global__ __launch_bounds__(256) void k_to_ns_orientation(const MatGeom g, const float* in, float* xf, void* xb) {
+  __shared__ __attribute__((aligned(16))) float tf[TallTile<float>::C * TallTile<float>::LD];
+  __shared__ __attribute__((aligned(16))) TN tb[TallTile<TN>::C * TallTile<TN>::LD];
   const int z = blockIdx.y, j = z / g.nb;
-  const FlatRange R(g.elems);
-  const size_t zo = (size_t)z * g.elems, xo = g.ns_base(g.ns_of(z));
-  const bool contiguous = g.x_contiguous(j);
-  for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
-    const float4 v = ld4(in + zo + e);
-    if (contiguous) {
-      const size_t x = xo + g.xidx(j, e);
-      st4(xf + x, v);
-      Elem<TN>::store4(reinterpret_cast<TN*>(xb) + x, v.x, v.y, v.z, v.w);
-    } else {
-      const float a[4] = {v.x, v.y, v.z, v.w};
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const size_t x = xo + g.xidx(j, e + i);
-        xf[x] = a[i];
-        Elem<TN>::store(reinterpret_cast<TN*>(xb) + x, a[i]);
-      }
+  const size_t zo = (size_t)z * g.elems, xo = g.ns_base(g.ns_of(z)) + g.xidx(j, 0);
+  if (g.x_contiguous(j)) {
+    const FlatRange R(g.elems);
+    for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
+      const float4 v = ld4(in + zo + e);
+      st4(xf + xo + e, v);
+      Elem<TN>::store4(reinterpret_cast<TN*>(xb) + xo + e, v.x, v.y, v.z, v.w);
     }
+    return;
+  }
+  using TF = TallTile<float>;
+  using TB = TallTile<TN>;
+  const int rows = g.rows(j), cols = g.cols(j), tc = (cols + TF::C - 1) / TF::C, nr = g.ns_rows(j);
+  for (int t = blockIdx.x; t < TF::count(rows, cols); t += gridDim.x) {
+    const int r0 = t / tc * TF::R, c0 = t % tc * TF::C;
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (r0 + TF::row(i) < rows && c0 + TF::col() < cols) {
+        const float4 v = ld4(in + zo + (size_t)(r0 + TF::row(i)) * cols + c0 + TF::col());
+        TF::put(tf, i, v);
+        TB::put(tb, i, v);
+      }
+    __syncthreads();
+    TF::copy_out(tf, xf + xo, r0, c0, rows, cols, nr);
+    TB::copy_out(tb, reinterpret_cast<TN*>(xb) + xo, r0, c0, rows, cols, nr);
+    __syncthreads();
   }
 }
 

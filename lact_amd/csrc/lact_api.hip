@@ -1584,8 +1584,9 @@ struct Runner {
         p.gn0 = gn0; p.gn0_init = !gn0_written;
         gn0_written = true;
         p.clear = ns_clear(false);
+        const bool as_they_lie = P.g.x_contiguous(0) && P.g.x_contiguous(1) && P.g.x_contiguous(2);
         if (P.muon) {
-          p.gxf = scr<float>(P.t_gxf[0]); p.gxb = scr<TN>(P.t_gxb[0]);
+          if (as_they_lie) { p.gxf = scr<float>(P.t_gxf[0]); p.gxb = scr<TN>(P.t_gxb[0]); }
         } else {
           p.gc = scr<T>(P.t_gc);
           p.gm_carry = carry_here ? gmcarry : nullptr; p.carry_valid = gm_valid; p.carry_write = u > 0;
@@ -1595,6 +1596,8 @@ struct Runner {
           }
         }
         LACT_LAUNCH("k_renorm_bwd", "k_renorm_bwd", 0.0, (k_renorm_bwd<T, TN>), rowgrid, dim3(256), s, p);
+        if (P.muon && !as_they_lie)   // whole segments through LDS instead of two and four bytes at a time
+          LACT_LAUNCH("k_to_ns_orientation", "k_to_ns_orientation", 0.0, (k_to_ns_orientation<TN>), dim3(P.nblk, 3 * d.b), dim3(256), s, P.g, gwhat, scr<float>(P.t_gxf[0]), (void*)scr<TN>(P.t_gxb[0]));
       }
       if (d.prenorm) carry_main = gw_idx;
       // The backward of the Frobenius normalisation as the fused kernel's last stages: the partial dots always

@@ -212,6 +212,17 @@ struct TallTile {
     TN* t = tile + col() * LD + row(i);
     Elem<TN>::store(t, f.x); Elem<TN>::store(t + LD, f.y); Elem<TN>::store(t + 2 * LD, f.z); Elem<TN>::store(t + 3 * LD, f.w);
   }
+  __device__ static __forceinline__ float4 get(const TN* tile, int i) {
+    const TN* t = tile + col() * LD + row(i);
+    return f4(Elem<TN>::load(t), Elem<TN>::load(t + LD), Elem<TN>::load(t + 2 * LD), Elem<TN>::load(t + 3 * LD));
+  }
+  __device__ static __forceinline__ void copy_in(TN* tile, const TN* in, int r0, int c0, int rows, int cols, int nr) {
+    constexpr int G = 16 / sizeof(TN), PER = R / G;
+    for (int q = threadIdx.x; q < C * PER; q += 256) {
+      const int c = q / PER, r = (q % PER) * G;
+      if (c0 + c < cols && r0 + r < rows) *reinterpret_cast<uint4*>(tile + c * LD + r) = *reinterpret_cast<const uint4*>(in + (size_t)(c0 + c) * nr + r0 + r);
+    }
+  }
   // the tile at (r0, c0) to the transposed matrix whose rows are nr long
   __device__ static __forceinline__ void copy_out(const TN* tile, TN* out, int r0, int c0, int rows, int cols, int nr) {
     constexpr int G = 16 / sizeof(TN), PER = R / G;   // granules of 16 bytes per column
@@ -456,7 +467,6 @@ __global__ void k_renorm_bwd(const RenormParams p) {
   const size_t o = (size_t)z * p.g.elems + (size_t)row * cols;
   const size_t uo = (p.u_stacked ? (size_t)p.g.u_off(z) : (size_t)z * p.g.elems) + (size_t)row * cols;
   const size_t xo = p.g.ns_base(p.g.ns_of(z));
-  const bool contiguous = p.g.x_contiguous(j);
   float c0 = 1.f, c1 = 0.f;
   float* gn0 = p.gn0 + (size_t)z * p.g.maxrows() + row;
   if (!p.weight_norm && p.gn0_init && lane == 0 && valid) *gn0 = 0.f;
@@ -516,21 +526,10 @@ __global__ void k_renorm_bwd(const RenormParams p) {
       }
       Elem<T>::store4(reinterpret_cast<T*>(p.gc) + o + c, g.x, g.y, g.z, g.w);
     }
-    if (p.gxf) {   // the same gradient where Newton-Schulz holds this matrix
-      const long long e = (long long)row * cols + c;
-      if (contiguous) {
-        const size_t x = xo + p.g.xidx(j, e);
-        st4(p.gxf + x, gv);
-        Elem<TN>::store4(reinterpret_cast<TN*>(p.gxb) + x, gv.x, gv.y, gv.z, gv.w);
-      } else {
-        const float g[4] = {gv.x, gv.y, gv.z, gv.w};
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const size_t x = xo + p.g.xidx(j, e + i);
-          p.gxf[x] = g[i];
-          Elem<TN>::store(reinterpret_cast<TN*>(p.gxb) + x, g[i]);
-        }
-      }
+    if (p.gxf) {   // the same gradient where Newton-Schulz holds this matrix (all of them as they lie, or k_to_ns_orientation follows)
+      const size_t x = xo + p.g.xidx(j, (long long)row * cols + c);
+      st4(p.gxf + x, gv);
+      Elem<TN>::store4(reinterpret_cast<TN*>(p.gxb) + x, gv.x, gv.y, gv.z, gv.w);
     }
   };
   const float4 zero4 = f4(0.f, 0.f, 0.f, 0.f);
@@ -627,8 +626,10 @@ struct GradPrepParams {
   const unsigned* poison;            // nonzero word: an earlier kernel of this step failed (barrier timeout) -> results become NaN
 };
 template <typename T, typename TN>
-__global__ void k_grad_prep(const GradPrepParams p) {
+__global__ __launch_bounds__(256) void k_grad_prep(const GradPrepParams p) {
   __shared__ float red[16];
+  __shared__ __attribute__((aligned(16))) float tx[TallTile<float>::C * TallTile<float>::LD];
+  __shared__ __attribute__((aligned(16))) TN tg[TallTile<TN>::C * TallTile<TN>::LD];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   const int m = p.g.ns_of(z);
   float dot = 0.f;
@@ -638,33 +639,16 @@ __global__ void k_grad_prep(const GradPrepParams p) {
   const float c1 = n > 0.f ? dot / (n * (n + 1e-7f) * (n + 1e-7f)) : 0.f;
   if (p.poison && *p.poison) c0 = __uint_as_float(0x7fc00000u);
   const float mb = p.mbar ? p.mbar[ib] : 0.f;
-  const FlatRange R(p.g.elems);
   const size_t zo = (size_t)z * p.g.elems;
-  const size_t xo = p.g.ns_base(p.g.ns_of(z));
-  const bool contiguous = p.g.x_contiguous(j);
+  const size_t xo = p.g.ns_base(p.g.ns_of(z)) + p.g.xidx(j, 0);
+  const TN* g16 = reinterpret_cast<const TN*>(p.g16) + xo;
   float md = 0.f;
-  for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
+  auto quad = [&](long long e, const float4& gx, const float4& g) {
     const size_t o = zo + e;
-    float4 gx;
-    float g[4];
-    if (contiguous) {
-      const size_t x = xo + p.g.xidx(j, e);
-      gx = ld4(p.gx0 + x);
-      Elem<TN>::load4(reinterpret_cast<const TN*>(p.g16) + x, g);
-    } else {
-      float t[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const size_t x = xo + p.g.xidx(j, e + i);
-        t[i] = p.gx0[x];
-        g[i] = Elem<TN>::load(reinterpret_cast<const TN*>(p.g16) + x);
-      }
-      gx = f4(t[0], t[1], t[2], t[3]);
-    }
     // the gradient that leaves Newton-Schulz through its input cast (G.bfloat16(), ttt_operation.py:45) has that type
     // (two gradients arrive there, through the quotient and through the norm, :49; each is a tensor of that type, and so is their sum)
-    float4 gv = f4(ns_input_grad<TN>(gx.x, g[0], c0, c1), ns_input_grad<TN>(gx.y, g[1], c0, c1), ns_input_grad<TN>(gx.z, g[2], c0, c1),
-            ns_input_grad<TN>(gx.w, g[3], c0, c1));
+    float4 gv = f4(ns_input_grad<TN>(gx.x, g.x, c0, c1), ns_input_grad<TN>(gx.y, g.y, c0, c1), ns_input_grad<TN>(gx.z, g.z, c0, c1),
+            ns_input_grad<TN>(gx.w, g.w, c0, c1));
     if (p.cr != 0.f) {
       const float4 w = ld4(p.gw_hat + o);
       gv.x += p.cr * w.x; gv.y += p.cr * w.y; gv.z += p.cr * w.z; gv.w += p.cr * w.w;
@@ -678,6 +662,29 @@ __global__ void k_grad_prep(const GradPrepParams p) {
       if (p.m_prev) md += dot4(gv, ld4(p.m_prev + o));
     }
     Elem<T>::store4(reinterpret_cast<T*>(p.gc) + o, gv.x, gv.y, gv.z, gv.w);
+  };
+  if (p.g.x_contiguous(j)) {
+    const FlatRange R(p.g.elems);
+    for (long long e = R.e0 + threadIdx.x * 4; e < R.e1; e += blockDim.x * 4) {
+      float g[4];
+      Elem<TN>::load4(g16 + e, g);
+      quad(e, ld4(p.gx0 + xo + e), f4(g[0], g[1], g[2], g[3]));
+    }
+  } else {
+    using TX = TallTile<float>;
+    using TG = TallTile<TN>;
+    const int rows = p.g.rows(j), cols = p.g.cols(j), tc = (cols + TX::C - 1) / TX::C, nr = p.g.ns_rows(j);
+    for (int t = blockIdx.x; t < TX::count(rows, cols); t += gridDim.x) {
+      const int rb = t / tc * TX::R, cb = t % tc * TX::C;
+      TX::copy_in(tx, p.gx0 + xo, rb, cb, rows, cols, nr);
+      TG::copy_in(tg, g16, rb, cb, rows, cols, nr);
+      __syncthreads();
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+        if (rb + TX::row(i) < rows && cb + TX::col() < cols)
+          quad((long long)(rb + TX::row(i)) * cols + cb + TX::col(), TX::get(tx, i), TG::get(tg, i));
+      __syncthreads();
+    }
   }
   if (p.gm_carry && p.m_prev) {
     md = block_sum(md, red);

@@ -25,11 +25,6 @@
 #include "gemm_dma_kernels.h"
 #include "state_kernels.h"
 
-// Optional in-kernel timestamps (defined only by timing experiments; expands to nothing in the library).
-#ifndef LACT_NS_TS
-#define LACT_NS_TS(i)
-#endif
-
 namespace lact {
 
 constexpr int NS_FUSED_MAX_STEPS = 8;
@@ -98,7 +93,7 @@ struct GroupBarrier {
       long long spins = 0;
       while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
         __builtin_amdgcn_s_sleep(1);
-        if (++spins > limit) {
+        if (++spins >= limit) {
           __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           if (sticky) __hip_atomic_fetch_add(sticky, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
           break;
@@ -174,8 +169,204 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_bwd_dot_tiles(const NsTileDo
   if (threadIdx.x == 0) p.dot_part[(size_t)z * gridDim.x + member] = dot;
 }
 
+// The roles of a block's waves are split for the whole of the iterations, not stage by stage: the fp32 iterate (its gradient) of
+// this block's tile then lives in the copy waves' registers, 18 granules of 8 elements per thread at 192 x 192, and only its bf16
+// copy goes through memory.  In one code path for all waves it would have to live beside the matrix waves' accumulators.
+// Measured, 48 matrices of 384 x 384, forward: an iteration took 39 us, 7.4 of them in the epilogue that read and wrote the fp32
+// tile, whose 28 MB per direction also pushed the operands out of the L2s; now 36.
+template <class TS>
+struct NsTileRegs {
+  static constexpr int GR = TS::BN / 8, N = TS::BM * GR / 256;   // granules per row; per copy-wave thread
+  static_assert(TS::BM * GR % 256 == 0, "granules split evenly over the copy waves");
+  float v[N][8];
+};
+// Granule t of a copy-wave thread: its row and first column inside the tile
+template <class TS>
+__device__ __forceinline__ void ns_granule(int t, int& row, int& col) {
+  const int id = (threadIdx.x & 255) + t * 256;
+  row = id / NsTileRegs<TS>::GR;
+  col = (id - row * NsTileRegs<TS>::GR) * 8;
+}
+
+// One stage's product on this block's tile (bx, by): the copy waves' part ...
+template <class TS, int NT, bool B_KS>
+__device__ __forceinline__ void ns_stage_load(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem) {
+  DmaPhase<1> ph[NT];
+  row_gemm_phases<TS, NT, B_KS>(p, bx * TS::BM, by * TS::BN, z, ph);
+  using Pipe = DmaPipe<TS, 1, NT, row_stages<TS>(), true>;
+  Pipe pipe(smem, ph);
+  pipe.template load_all<Pipe::loads(1)>();
+  __syncthreads();   // the matrix waves are through with the ring
+  __syncthreads();   // and have staged the tile
+}
+// ... and the matrix waves'.  E: bytes per staged element (2: the product as bf16, 4: fp32)
+template <class TS, int NT, bool B_KS, int E>
+__device__ __forceinline__ void ns_stage_mma(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem) {
+  DmaPhase<1> ph[NT];
+  row_gemm_phases<TS, NT, B_KS>(p, bx * TS::BM, by * TS::BN, z, ph);
+  DmaPipe<TS, 1, NT, row_stages<TS>(), true> pipe(smem, ph);
+  f32x16 acc[1][TS::TM][TS::TN];
+  zero_acc<TS>(acc[0]);
+  int step = 0;
+#pragma unroll
+  for (int t = 0; t < NT; ++t) pipe.template run_phase<1, false, B_KS>(p.t[t].K, step, acc);
+  __syncthreads();
+  using ST = StageTile<TS, E>;
+  char* lb = smem + ST::lane_base();
+  LACT_FOR_QUADS(TS) ST::put4(lb, tm, tn, g, acc[0][tm][tn][4 * g], acc[0][tm][tn][4 * g + 1], acc[0][tm][tn][4 * g + 2], acc[0][tm][tn][4 * g + 3]);
+  __syncthreads();
+}
+template <class TS, int NT, int EPI, bool COPY>
+__device__ __forceinline__ void ns_stage_b16(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem) {
+  if (COPY) ns_stage_load<TS, NT, false>(p, bx, by, z, smem);
+  else ns_stage_mma<TS, NT, false, 2>(p, bx, by, z, smem);
+  row_gemm_copy_out_b16<TS, NT, EPI, COPY ? 3 : 64>(p, bx * TS::BM, by * TS::BN, z, smem);
+}
+// X' = beta X + product (the stage with B K-strided): the staged product blended with the fp32 tile in registers.
+// out_c: bf16 copy, out: fp32 (both [r, c]; nullable); out_t: fp32 in the original orientation, transposed if `tr`
+template <class TS, int NT, bool COPY>
+__device__ __forceinline__ void ns_stage_iterate(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, NsTileRegs<TS>* x, bool tr) {
+  using ST = StageTile<TS, 4>;
+  const int m0 = bx * TS::BM, n0 = by * TS::BN;
+  if constexpr (COPY) {
+    ns_stage_load<TS, NT, true>(p, bx, by, z, smem);
+    const size_t zo = z * p.bso + (size_t)m0 * p.ldo + n0;
+#pragma unroll
+    for (int t = 0; t < NsTileRegs<TS>::N; ++t) {
+      int row, col;
+      ns_granule<TS>(t, row, col);
+      float4* src = reinterpret_cast<float4*>(smem + (row * ST::LD + col) * 4);
+      const float4 a = src[0], b = src[1];
+      const float in[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      float (&v)[8] = x->v[t];
+      // the matrix product is a bf16 tensor in the reference (ttt_operation.py:62)
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = dual_blend(__fmul_rn(p.alpha, round_bf16(in[i])), __fmul_rn(p.beta, v[i]), p.round_out_bf16);
+      const size_t o = zo + (size_t)row * p.ldo + col;
+      if (p.out_c) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.out_c) + o) = pack8(v);
+      if (p.out) {
+        float* f = reinterpret_cast<float*>(p.out) + o;
+        *reinterpret_cast<float4*>(f) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4*>(f + 4) = make_float4(v[4], v[5], v[6], v[7]);
+      }
+      if (p.out_t && !tr) {
+        *reinterpret_cast<float4*>(p.out_t + o) = make_float4(v[0], v[1], v[2], v[3]);
+        *reinterpret_cast<float4*>(p.out_t + o + 4) = make_float4(v[4], v[5], v[6], v[7]);
+      }
+      if (p.out_t && tr) {
+        src[0] = make_float4(v[0], v[1], v[2], v[3]);
+        src[1] = make_float4(v[4], v[5], v[6], v[7]);
+      }
+    }
+  } else {
+    ns_stage_mma<TS, NT, true, 4>(p, bx, by, z, smem);
+  }
+  if (p.out_t && tr) {
+    __syncthreads();
+    row_gemm_copy_out_transposed<TS, NT>(p, nullptr, true, m0, n0, z, smem);
+  }
+}
+
+// This block's place in its matrix
+struct NsPlace {
+  int z;
+  bool sq_tile;              // owns a tile of the r x r stages: (sx, sy)
+  int sx, sy, rx, ry;        // (rx, ry): its tile of the r x c stages
+};
 // BWD = false: S iterations  A = X X^T;  B = b A + c A A;  X' = a X + B X
 // BWD = true:  the same iterations backwards:  Sg = G X^T + X G^T;  H = b Sg + c (Sg A + A Sg);  G' = a G + B G + H X
+// COPY: on the copy waves, else on the matrix waves.
+template <class TS, bool BWD, bool COPY>
+__device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarrier& bar, const NsPlace& b, char* smem) {
+  const int z = b.z;
+  NsTileRegs<TS> x;
+  if constexpr (COPY) {
+    const float* src = (BWD ? p.gxf[0] : p.xf[0]) + (size_t)z * p.r * p.c + (size_t)b.rx * TS::BM * p.c + b.ry * TS::BN;
+#pragma unroll
+    for (int t = 0; t < NsTileRegs<TS>::N; ++t) {
+      int row, col;
+      ns_granule<TS>(t, row, col);
+      const float4 lo = *reinterpret_cast<const float4*>(src + (size_t)row * p.c + col), hi = *reinterpret_cast<const float4*>(src + (size_t)row * p.c + col + 4);
+      x.v[t][0] = lo.x; x.v[t][1] = lo.y; x.v[t][2] = lo.z; x.v[t][3] = lo.w;
+      x.v[t][4] = hi.x; x.v[t][5] = hi.y; x.v[t][6] = hi.z; x.v[t][7] = hi.w;
+    }
+  }
+  const bool tr = (p.mask >> (z / p.nb)) & 1;
+  for (int step = 0; step < p.S; ++step) {
+    const int it = BWD ? p.S - 1 - step : step;
+    const bool last = step + 1 == p.S;
+    // r and c are made opaque once per iteration: otherwise the compiler hoists every stage's loop-invariant
+    // per-lane address registers out of this loop, keeps them all live and spills
+    int r = p.r, c = p.c;
+    asm volatile("" : "+s"(r), "+s"(c));
+    const long long xe = (long long)r * c, se = (long long)r * r;
+    const float ca = p.coeffs[3 * it], cb = p.coeffs[3 * it + 1], cc = p.coeffs[3 * it + 2];
+    const uint16_t* X = p.xb + it * p.xb_it_stride;
+    uint16_t* A = p.ab + it * p.sq_it_stride;
+    uint16_t* B = p.bb + it * p.sq_it_stride;
+    if (!BWD) {
+      if (b.sq_tile) {
+        auto q = ns_row_params<1>();
+        ns_term(q.g.t[0], X, c, xe, X, c, xe, c);
+        q.g.M = r; q.g.N = r; q.g.out = A; q.g.ldo = r; q.g.bso = se;
+        q.g.out2 = p.cab; q.g.alpha2 = cc;
+        ns_stage_b16<TS, 1, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem);
+      }
+      bar.sync(p.error);
+      if (b.sq_tile) {
+        auto q = ns_row_params<1>();
+        ns_term(q.g.t[0], p.cab, r, se, A, r, se, r);
+        q.g.M = r; q.g.N = r; q.g.out = B; q.g.ldo = r; q.g.bso = se;
+        q.g.aux = A; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = 1.f; q.g.beta = cb;
+        ns_stage_b16<TS, 1, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem);
+      }
+      bar.sync(p.error);
+      {
+        auto q = ns_row_params<1>();
+        ns_term(q.g.t[0], B, r, se, X, c, xe, r);
+        q.g.M = r; q.g.N = c; q.g.ldo = c; q.g.bso = xe;
+        q.g.alpha = 1.f; q.g.beta = ca; q.g.round_out_bf16 = p.plain;
+        q.g.out = nullptr;
+        q.g.out_c = last ? nullptr : p.xb + (it + 1) * p.xb_it_stride;   // nothing multiplies by the last iterate
+        q.g.out_t = last ? p.u_out : nullptr;
+        ns_stage_iterate<TS, 1, COPY>(q.g, b.rx, b.ry, z, smem, &x, tr);
+      }
+      bar.sync(p.error);
+    } else {
+      const int cur = step & 1;
+      const uint16_t* gb = p.gxb[cur];
+      if (b.sq_tile) {   // Sg = G X^T + X G^T
+        auto q = ns_row_params<2>();
+        ns_term(q.g.t[0], gb, c, xe, X, c, xe, c);
+        ns_term(q.g.t[1], X, c, xe, gb, c, xe, c);
+        q.g.M = r; q.g.N = r; q.g.out = p.sg; q.g.ldo = r; q.g.bso = se;
+        ns_stage_b16<TS, 2, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem);
+      }
+      bar.sync(p.error);
+      if (b.sq_tile) {   // H = b Sg + c (Sg A + A Sg)
+        auto q = ns_row_params<2>();
+        ns_term(q.g.t[0], p.sg, r, se, A, r, se, r);
+        ns_term(q.g.t[1], A, r, se, p.sg, r, se, r);
+        q.g.M = r; q.g.N = r; q.g.out = p.gas; q.g.ldo = r; q.g.bso = se;
+        q.g.aux = p.sg; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = cc; q.g.beta = cb;
+        ns_stage_b16<TS, 2, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem);
+      }
+      bar.sync(p.error);
+      {                  // G' = a G + B G + H X
+        auto q = ns_row_params<2>();
+        ns_term(q.g.t[0], B, r, se, gb, c, xe, r);
+        ns_term(q.g.t[1], p.gas, r, se, X, c, xe, r);
+        q.g.M = r; q.g.N = c; q.g.ldo = c; q.g.bso = xe;
+        q.g.alpha = 1.f; q.g.beta = ca;
+        q.g.out = last ? p.gxf[p.S & 1] : nullptr;
+        q.g.out_c = last ? nullptr : p.gxb[cur ^ 1];   // nothing multiplies by the final gradient
+        ns_stage_iterate<TS, 2, COPY>(q.g, b.rx, b.ry, z, smem, &x, false);
+      }
+      bar.sync(p.error);
+    }
+  }
+}
+
 // TS: 192 x 192 tiles, or 128 x 128 / 128 x 64 when there are too few matrices to fill the chip with the large tile.
 template <class TS, bool BWD>
 __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p) {
@@ -228,94 +419,9 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p)
     }
     bar.sync(p.error);
   }
-  LACT_NS_TS(0);
-  for (int step = 0; step < p.S; ++step) {
-    const int it = BWD ? p.S - 1 - step : step;
-    // r and c are made opaque once per iteration: otherwise the compiler hoists every stage's loop-invariant
-    // per-lane address registers out of this loop, keeps them all live and spills
-    int r = p.r, c = p.c;
-    asm volatile("" : "+s"(r), "+s"(c));
-    const long long xe = (long long)r * c, se = (long long)r * r;
-    const float ca = p.coeffs[3 * it], cb = p.coeffs[3 * it + 1], cc = p.coeffs[3 * it + 2];
-    const uint16_t* X = p.xb + it * p.xb_it_stride;
-    uint16_t* A = p.ab + it * p.sq_it_stride;
-    uint16_t* B = p.bb + it * p.sq_it_stride;
-    if (!BWD) {
-      const bool last = it + 1 == p.S;
-      if (sq_tile) {
-        auto q = ns_row_params<1>();
-        ns_term(q.g.t[0], X, c, xe, X, c, xe, c);
-        q.g.M = r; q.g.N = r; q.g.out = A; q.g.ldo = r; q.g.bso = se;
-        q.g.out2 = p.cab; q.g.alpha2 = cc;
-        row_gemm_tile<TS, 1, EPI_STORE, false, true>(q, sx, sy, z, smem);
-      }
-      LACT_NS_TS(1 + step * 6 + 0);
-      bar.sync(p.error);
-      LACT_NS_TS(1 + step * 6 + 1);
-      if (sq_tile) {
-        auto q = ns_row_params<1>();
-        ns_term(q.g.t[0], p.cab, r, se, A, r, se, r);
-        q.g.M = r; q.g.N = r; q.g.out = B; q.g.ldo = r; q.g.bso = se;
-        q.g.aux = A; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = 1.f; q.g.beta = cb;
-        row_gemm_tile<TS, 1, EPI_AXPBY, false, true>(q, sx, sy, z, smem);
-      }
-      LACT_NS_TS(1 + step * 6 + 2);
-      bar.sync(p.error);
-      LACT_NS_TS(1 + step * 6 + 3);
-      {
-        auto q = ns_row_params<1>();
-        ns_term(q.g.t[0], B, r, se, X, c, xe, r);
-        q.g.M = r; q.g.N = c; q.g.ldo = c; q.g.bso = xe;
-        q.g.aux = p.xf[it & 1]; q.g.ldaux = c; q.g.bsaux = xe; q.g.alpha = 1.f; q.g.beta = ca;
-        q.g.round_out_bf16 = p.plain;
-        q.g.out = last ? nullptr : p.xf[(it + 1) & 1];
-        q.g.out_c = last ? nullptr : p.xb + (it + 1) * p.xb_it_stride;   // nothing multiplies by the last iterate
-        q.g.out_t = last ? p.u_out : nullptr;
-        q.g.transpose_mask = p.mask; q.g.nb = p.nb;
-        row_gemm_tile<TS, 1, EPI_AXPBY_F32_DUAL, true, true>(q, rx, ry, z, smem);
-      }
-      LACT_NS_TS(1 + step * 6 + 4);
-      bar.sync(p.error);
-      LACT_NS_TS(1 + step * 6 + 5);
-    } else {
-      const int cur = step & 1;
-      const uint16_t* gb = p.gxb[cur];
-      if (sq_tile) {   // Sg = G X^T + X G^T
-        auto q = ns_row_params<2>();
-        ns_term(q.g.t[0], gb, c, xe, X, c, xe, c);
-        ns_term(q.g.t[1], X, c, xe, gb, c, xe, c);
-        q.g.M = r; q.g.N = r; q.g.out = p.sg; q.g.ldo = r; q.g.bso = se;
-        row_gemm_tile<TS, 2, EPI_STORE, false, true>(q, sx, sy, z, smem);
-      }
-      LACT_NS_TS(1 + step * 6 + 0);
-      bar.sync(p.error);
-      LACT_NS_TS(1 + step * 6 + 1);
-      if (sq_tile) {   // H = b Sg + c (Sg A + A Sg)
-        auto q = ns_row_params<2>();
-        ns_term(q.g.t[0], p.sg, r, se, A, r, se, r);
-        ns_term(q.g.t[1], A, r, se, p.sg, r, se, r);
-        q.g.M = r; q.g.N = r; q.g.out = p.gas; q.g.ldo = r; q.g.bso = se;
-        q.g.aux = p.sg; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = cc; q.g.beta = cb;
-        row_gemm_tile<TS, 2, EPI_AXPBY, false, true>(q, sx, sy, z, smem);
-      }
-      LACT_NS_TS(1 + step * 6 + 2);
-      bar.sync(p.error);
-      LACT_NS_TS(1 + step * 6 + 3);
-      {                // G' = a G + B G + H X
-        auto q = ns_row_params<2>();
-        ns_term(q.g.t[0], B, r, se, gb, c, xe, r);
-        ns_term(q.g.t[1], p.gas, r, se, X, c, xe, r);
-        q.g.M = r; q.g.N = c; q.g.ldo = c; q.g.bso = xe;
-        q.g.aux = p.gxf[cur]; q.g.ldaux = c; q.g.bsaux = xe; q.g.alpha = 1.f; q.g.beta = ca;
-        q.g.out = p.gxf[cur ^ 1];
-        q.g.out_c = step + 1 == p.S ? nullptr : p.gxb[cur ^ 1];   // nothing multiplies by the final gradient
-        row_gemm_tile<TS, 2, EPI_AXPBY_F32_DUAL, true, true>(q, rx, ry, z, smem);
-      }
-      LACT_NS_TS(1 + step * 6 + 4);
-      bar.sync(p.error);
-      LACT_NS_TS(1 + step * 6 + 5);
-    }
-  }
+  const NsPlace place{z, sq_tile, sx, sy, rx, ry};
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4) ns_iterations<TS, BWD, true>(p, bar, place, smem);
+  else ns_iterations<TS, BWD, false>(p, bar, place, smem);
   if (BWD && p.dot_part) {
     // the tile this block wrote in the last stage, and the same tile of the bf16 input: 12 granules of 8 elements
     // per thread at 192 x 192, kept in registers for the second pass

@@ -1,0 +1,60 @@
+// Host-side check of the buffer plan (no GPU needed): a token reduction never writes more partial-sum slots than the buffer of its
+// chain holds, whatever the lengths of the program's steps, and none of them is held below what its own length asks for on the side
+// chain, whose buffer is sized for exactly its launches.
+#include <cstdio>
+#include <cstring>
+#include <vector>
+#include "../../lact_amd/csrc/plan.h"
+
+using namespace lact;
+
+static int check(bool bf16, int b, int d, int dh, int rounds, int T_update, int T_apply, bool muon) {
+  std::vector<lact_step_t> steps;
+  int kv = 0, q = 0;
+  for (int i = 0; i < rounds; ++i) {
+    steps.push_back(lact_step_t{LACT_UPDATE, kv, kv + T_update, 0});
+    steps.push_back(lact_step_t{LACT_APPLY, q, q + T_apply, q});
+    kv += T_update; q += T_apply;
+  }
+  lact_desc_t D;
+  memset(&D, 0, sizeof(D));
+  std::vector<float> coeffs(15, 1.f);
+  D.b = b; D.d = d; D.dh = dh; D.q_len = q; D.kv_len = kv; D.out_len = q; D.act_dtype = bf16 ? LACT_BF16 : LACT_F32;
+  D.n_steps = (int)steps.size(); D.steps = steps.data(); D.ns_steps = muon ? 5 : -1; D.ns_coeffs = muon ? coeffs.data() : nullptr;
+  D.weight_norm = 1; D.q_ld = D.k_ld = D.v_ld = D.o_ld = D.do_ld = d;
+  Plan P;
+  if (P.build(&D)) { printf("plan refused: %s\n", g_err.c_str()); return 1; }
+  int bad = 0;
+  auto expect = [&](bool ok, const char* what, int a, int c) {
+    if (!ok) { printf("%s: %d against %d (%s b=%d d=%d dh=%d, %d rounds of %d and %d tokens)\n", what, a, c, bf16 ? "bf16" : "fp32", b, d, dh, rounds, T_update, T_apply); ++bad; }
+  };
+  for (const auto& g : P.groups) {
+    const int T = g.st.end - g.st.start, mats = 3 * b * g.n;
+    const int wanted = bf16 && T >= 64 ? choose_split(T, tr_tiles(d, dh) * mats, 16, P.split_min).n : choose_split_async(T, P.tiles * mats, 16).n;
+    const int used = P.reduce_split(T, g.n, P.max_splits(true, g.n), P.split_min).n;
+    expect(used * g.n <= P.side_slots, "slots of a grouped launch", used * g.n, P.side_slots);
+    expect(wanted * g.n <= P.side_slots && used == wanted, "splits of a grouped launch", used, wanted);
+  }
+  for (int T : {T_update, T_apply})
+    for (int min_len : {P.split_min, 1536}) {
+      const int used = P.reduce_split(T, 1, P.max_splits(false, 1), min_len).n;
+      expect(used <= P.nsplit_max, "slots of a launch of the main chain", used, P.nsplit_max);
+    }
+  expect(P.t_partial_side + (size_t)P.side_slots * P.mat3 * 4 <= P.t_gwside, "end of the side buffer", P.side_slots, 0);
+  return bad;
+}
+
+int main() {
+  int bad = 0, n = 0;
+  for (bool bf16 : {false, true})
+    for (int b : {1, 2, 5})
+      for (int d : {8, 64, 128, 192})
+        for (int T_update : {40, 256, 1024, 1100, 2049, 4680})
+          for (int T_apply : {24, 64, 1000, 1024, 2048, 3000})
+            for (int rounds : {1, 2, 4, 9, 70}) {
+              bad += check(bf16, b, d, d == 64 ? 96 : d, rounds, T_update, T_apply, rounds == 4) > 0;
+              ++n;
+            }
+  printf("%d plans checked, %d bad\n", n, bad);
+  return bad ? 1 : 0;
+}

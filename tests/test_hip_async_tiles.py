@@ -91,6 +91,30 @@ def test_apply_steps_of_several_versions_in_one_launch(dtype, b, C, order):
         assert O.rel_l2(a, r) < (1e-5 if dtype == torch.float32 else 1e-2), k
 
 
+@pytest.mark.parametrize("dtype,b,d,update,apply", [(torch.float32, 2, 64, 1100, 1024), (torch.float32, 1, 40, 2049, 2048),
+                                                     (torch.bfloat16, 2, 48, 1100, 1024), (torch.bfloat16, 2, 64, 1664, 1600)])
+def test_grouped_apply_steps_shorter_than_the_updates(dtype, b, d, update, apply):
+    """Apply steps that one launch covers, of fewer tokens than the updates and cut into at least as many splits (the buffers are
+    sized for the launch, not for the longest step): outputs and gradients against the oracle."""
+    print("[gpu-test] grouped applies, shorter than the updates", dtype, b, d, update, apply, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    L, rounds = 4 * update, range(0, 4 * update, update)
+    inp = O.make_inputs(b, L, d, 64, seed=38, act_dtype=dtype)
+    go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(8)).to(dtype)
+    prog = ops.Program(steps=tuple(st for r in rounds for st in ((LACT_UPDATE, r, r + update, 0), (LACT_APPLY, r, r + apply, r))), out_len=L)
+    steps = [st for r in rounds for st in (O.Step(O.UPDATE, r, r + update), O.Step(O.APPLY, r, r + apply))]
+    dev = [inp[n].to("cuda").requires_grad_(True) for n in ORDER]
+    out, _, _ = ops.run_program(prog, *dev)
+    res = [out] + list(torch.autograd.grad(out, dev, go.to("cuda")))
+    cpu = [inp[n].clone().requires_grad_(True) for n in ORDER]
+    ref, _, _ = O.run_program(*cpu[:9], steps, num=O.Numerics(autocast=dtype == torch.bfloat16), momentum=cpu[9])
+    refs = [ref] + list(torch.autograd.grad(ref, cpu, go))
+    for n, a, r in zip(("out",) + ORDER, res, refs):
+        # the bounds of test_small_tiles_against_oracle
+        assert O.rel_l2(a, r) < (1e-4 if dtype == torch.float32 else 3e-2 if n == "momentum" else 1e-2), n
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("d,dh", [(128, 256), (72, 40), (8, 72)])
 def test_transposed_weights_are_read_as_they_lie(dtype, d, dh):

@@ -250,7 +250,7 @@ struct Plan {
     t_lrpart = sc.take((size_t)std::max(1, nupd) * 3 * lr_slots * d.b * Tcap * 4);   // one slot per update: reduced by one launch at the end
     for (int i = 0; i < 2; ++i) t_xf[i] = sc.take(mat3 * 4);
     t_xbtmp = sc.take(mat3 * nsz);
-    t_ss = sc.take((size_t)3 * d.b * nblk * 4);
+    t_ss = sc.take((size_t)3 * d.b * std::max(nblk, tr_tiles(d.d, d.dh)) * 4);   // per block of a pass over the matrix, or per tile of the reduction that folds the pass in
     t_dot = sc.take((size_t)3 * d.b * std::max(nblk, 32) * 4);   // partial dots: per chunk of a matrix, or per block of the fused kernel
     t_mdot = sc.take((size_t)std::max(1, nupd) * 3 * d.b * mdot_parts * 4);   // one slot per update: the momentum gradients are written at the end
     for (int i = 0; i < 2; ++i) t_gwhat[i] = sc.take(mat3 * 4);

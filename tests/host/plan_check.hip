@@ -1,6 +1,7 @@
 // Host-side check of the buffer plan (no GPU needed): a token reduction never writes more partial-sum slots than the buffer of its
 // chain holds, whatever the lengths of the program's steps, and none of them is held below what its own length asks for on the side
-// chain, whose buffer is sized for exactly its launches.
+// chain, whose buffer is sized for exactly its launches; and the partial sums of squares of a reduction that folds the momentum step
+// in have a place per tile.
 #include <cstdio>
 #include <cstring>
 #include <vector>
@@ -41,6 +42,7 @@ static int check(bool bf16, int b, int d, int dh, int rounds, int T_update, int 
       expect(used <= P.nsplit_max, "slots of a launch of the main chain", used, P.nsplit_max);
     }
   expect(P.t_partial_side + (size_t)P.side_slots * P.mat3 * 4 <= P.t_gwside, "end of the side buffer", P.side_slots, 0);
+  if (muon) expect(P.t_ss + (size_t)3 * b * std::max(P.nblk, tr_tiles(d, dh)) * 4 <= P.t_dot, "sums of squares per matrix", std::max(P.nblk, tr_tiles(d, dh)), P.nblk);
   return bad;
 }
 
@@ -55,6 +57,7 @@ int main() {
               bad += check(bf16, b, d, d == 64 ? 96 : d, rounds, T_update, T_apply, rounds == 4) > 0;
               ++n;
             }
+  for (int d : {2176, 4096}) { bad += check(true, 1, d, d, 2, 256, 256, true) > 0; ++n; }   // more tiles than blocks of a pass over the matrix
   printf("%d plans checked, %d bad\n", n, bad);
   return bad ? 1 : 0;
 }

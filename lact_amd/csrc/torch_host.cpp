@@ -189,6 +189,27 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
 
 Tensor cast(const Tensor& t, at::ScalarType dtype) { return !t.defined() || t.scalar_type() == dtype ? t : t.to(dtype); }
 
+// Gradients that have no gradient of their own although they depend on the inputs of the function whose backward is running:
+// differentiating them is an error on every path to those inputs, not a silent zero.
+void refuse_second_derivative(variable_list& grads) {
+  const auto node = torch::autograd::get_current_node();
+  const auto err = std::make_shared<torch::autograd::Error>("trying to differentiate twice a function that was marked with @once_differentiable",
+                                                            node ? torch::autograd::edge_list(node->next_edges()) : torch::autograd::edge_list());
+  for (auto& g : grads)
+    if (g.defined()) {
+      g = g.detach();
+      torch::autograd::create_gradient_edge(g, err);
+    }
+}
+std::vector<OptTensor> refuse_second_derivative_py(std::vector<OptTensor> grads) {
+  variable_list list;
+  for (auto& g : grads) list.push_back(g ? *g : Tensor());
+  refuse_second_derivative(list);
+  for (size_t i = 0; i < grads.size(); ++i)
+    if (grads[i]) grads[i] = list[i];
+  return grads;
+}
+
 // What the backward of one call needs beside the saved tensors.
 struct CallRecord : torch::CustomClassHolder {
   c10::intrusive_ptr<Schedule> sc;
@@ -218,8 +239,7 @@ struct ProgramFn : torch::autograd::Function<ProgramFn> {
     return res;
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const bool twice = at::GradMode::is_enabled() &&
-                       std::any_of(grads.begin(), grads.end(), [](const Tensor& g) { return g.defined() && g.requires_grad(); });
+    const bool twice = at::GradMode::is_enabled();
     const at::AutoGradMode off(false);
     auto t = ctx->get_saved_variables();
     const Tensor &q = t[0], &k = t[1], &v = t[2], &momentum = t[6], &saved = t[7];
@@ -259,14 +279,7 @@ struct ProgramFn : torch::autograd::Function<ProgramFn> {
     variable_list res{Tensor(), cast(dw[0], type(0)), cast(dw[1], type(1)), cast(dw[2], type(2)), cast(dq, type(3)), cast(dk, type(4)), cast(dv, type(5))};
     for (auto& x : dlr) res.push_back(x.defined() ? cast(x.reshape(rec.lr_shape), type(6)) : x);
     res.push_back(dm.defined() ? cast(dm.reshape(rec.m_shape), type(7)) : dm);
-    if (twice) {   // the gradients have no backward of their own: an attempt at one is an error, not a silent zero
-      auto err = std::make_shared<torch::autograd::DelayedError>(
-          "trying to differentiate twice a function that was marked with @once_differentiable", (int64_t)res.size());
-      for (auto& x : res)
-        if (x.defined()) x = x.detach().set_requires_grad(true);
-      const at::AutoGradMode on(true);
-      res = (*err)(std::move(res));
-    }
+    if (twice) refuse_second_derivative(res);
     return res;
   }
 };
@@ -306,4 +319,5 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
       .def(py::init<const std::vector<std::vector<int>>&, int64_t, const std::optional<std::vector<float>>&, bool, bool, bool, bool, int, bool,
                     bool, bool>());
   m.def("run_program", &run_program);
+  m.def("refuse_second_derivative", &refuse_second_derivative_py);
 }

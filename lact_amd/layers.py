@@ -23,6 +23,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from . import _lib
+from ._autograd import once_differentiable
 from ._lib import LACT_BF16, LACT_F32
 from .minimal import bidirectional_lact_swiglu, block_causal_lact_swiglu, inv_softplus
 from .nvs import fast_weight_swish_glu_weight_norm_mini_batch_apply
@@ -62,6 +63,7 @@ class _PreFn(torch.autograd.Function):
         return q, k, v
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dq, dk, dv):
         (qkv,) = ctx.saved_tensors
         B, L, H, hd, l2norm = ctx.dims
@@ -94,6 +96,7 @@ class _PreAttnFn(torch.autograd.Function):
         return (*outs, *att)
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, *grads):
         qkv, scale = ctx.saved_tensors
         B, L, H, hd, l2norm = ctx.dims
@@ -131,6 +134,7 @@ class _LrFn(torch.autograd.Function):
         return outs[0], outs[1], outs[2], mom
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, d0, d1, d2, dm=None):
         lr_raw, mom_c = ctx.saved_tensors
         B, L, H, base, rates_major = ctx.dims
@@ -167,6 +171,7 @@ class _PostFn(torch.autograd.Function):
         return y
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, dy):
         o, w, g = ctx.saved_tensors
         B, L, H, hd, use_norm, eps = ctx.dims
@@ -254,6 +259,7 @@ class _WindowAttentionFn(torch.autograd.Function):
         return out
 
     @staticmethod
+    @once_differentiable
     def backward(ctx, g):
         q, k, v, out, lse = ctx.saved_tensors
         B, L, H, D = q.shape

@@ -14,6 +14,7 @@ from typing import Optional, Sequence, Tuple
 import torch
 
 from . import _lib
+from ._autograd import once_differentiable
 from ._lib import LACT_APPLY, LACT_UPDATE
 
 # lact_llm/lact_model/ttt_operation.py:51-57
@@ -138,7 +139,7 @@ class _NewtonSchulzFn(torch.autograd.Function):
         return out.to(torch.bfloat16) if ns_mode == NS_PLAIN_BF16 else out
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
+    @once_differentiable
     def backward(ctx, dout):
         (g,) = ctx.saved_tensors
         L = _lib.lib()

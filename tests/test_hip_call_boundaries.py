@@ -1,0 +1,51 @@
+"""What the layer functions around the operation do at the edges of an ordinary call: gradients that are differentiated again,
+transforms, tensors of other devices and shapes, views that start anywhere in memory."""
+import pytest
+import torch
+
+from lact_amd import layers as HL
+from lact_amd import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def randn(*shape, dtype=torch.float32, seed=1, grad=True):
+    return torch.randn(*shape, generator=torch.Generator().manual_seed(seed)).to(dtype).to(DEV).requires_grad_(grad)
+
+
+PROGRAM = ops.Program(steps=((ops.LACT_UPDATE, 0, 24, 0), (ops.LACT_APPLY, 0, 24, 0)), out_len=24)
+
+
+def operands(b, L, d, dh):
+    shapes = [(b, dh, d), (b, d, dh), (b, dh, d)] + [(b, L, d)] * 3 + [(b, L, 1)] * 3
+    return [randn(*s, seed=i) for i, s in enumerate(shapes)]
+
+
+CALLS = {
+    "pre": lambda: (lambda x: HL._PreFn.apply(x, 2, 16, True), [randn(1, 5, 96)]),
+    "pre_attn": lambda: (lambda x, s, o: HL._PreAttnFn.apply(x, s, o, 2, 16, True), [randn(1, 5, 96), randn(32, 2), randn(32, 2)]),
+    "lr": lambda: (lambda x, m: HL._LrFn.apply(x, m, 2, 0.1), [randn(1, 5, 6), randn(1, 5, 2)]),
+    "post": lambda: (lambda o, w, g, a: HL._PostFn.apply(o, w, g, 1, 2, True, 1e-5, a), [randn(2, 5, 16), randn(16), randn(1, 5, 2), randn(1, 5, 32)]),
+    "newton_schulz": lambda: (lambda x: ops.newton_schulz(x, ops.NS5_COEFFS), [randn(1, 16, 24)]),
+    "operation": lambda: (lambda *x: ops.run_program(PROGRAM, *x)[0], operands(1, 24, 16, 24)),
+    "window": lambda: (lambda q, k, v: HL.sliding_window_attention(q, k, v, 3), [randn(1, 5, 2, 64, dtype=torch.bfloat16, seed=i) for i in range(3)]),
+}
+
+
+@pytest.mark.parametrize("name", CALLS)
+def test_second_derivatives_are_refused(name):
+    """The kernels' gradients have no gradient of their own: differentiating them is an error, not a silent constant."""
+    print("[gpu-test] second derivative", name, flush=True)
+    fn, args = CALLS[name]()
+    outs = fn(*args)
+    outs = outs if isinstance(outs, tuple) else (outs,)
+    grads = torch.autograd.grad(outs, args, [torch.ones_like(o) for o in outs], create_graph=True)   # constants: only the saved tensors depend on the inputs
+    first = torch.autograd.grad(fn(*args), args, [torch.ones_like(o) for o in outs])
+    assert all(torch.equal(a, b) for a, b in zip(grads, first))
+    assert all(g.requires_grad for g in grads)
+    penalty = sum(g.float().square().sum() for g in grads)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        torch.autograd.grad(penalty + sum(x.float().sum() for x in args), args, retain_graph=True)
+    with pytest.raises(RuntimeError, match="once_differentiable"):
+        penalty.backward()

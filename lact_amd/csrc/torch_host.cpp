@@ -285,11 +285,20 @@ struct ProgramFn : torch::autograd::Function<ProgramFn> {
 };
 
 bool wants_grad(const OptTensor& t) { return t && t->requires_grad(); }
+bool has_tangent(const Tensor& t) { return t._fw_grad(/*level=*/0).defined(); }
+bool has_tangent(const OptTensor& t) { return t && has_tangent(*t); }
+template <typename... Ts>
+bool any_tangent(const Ts&... ts) { return (has_tangent(ts) || ...); }
 
 // (out, w0, w1, w2, m0, m1, m2), None where there is nothing to return
 py::tuple run_program(const c10::intrusive_ptr<Schedule>& sc, const Tensor& w0, const Tensor& w1, const Tensor& w2, const Tensor& q,
                       const OptTensor& k, const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1, const OptTensor& lr2,
                       const OptTensor& momentum, const OptTensor& m0, const OptTensor& m1, const OptTensor& m2) {
+  // forward-mode differentiation knows nothing of a call that passes the autograd function by: the tangents would be dropped
+  if (any_tangent(w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m0, m1, m2)) {
+    PyErr_SetString(PyExc_NotImplementedError, "the operation has no forward-mode derivative (jvp)");
+    throw py::error_already_set();
+  }
   const bool needs_backward = at::GradMode::is_enabled() &&
                               (w0.requires_grad() || w1.requires_grad() || w2.requires_grad() || q.requires_grad() || wants_grad(k) ||
                                wants_grad(v) || wants_grad(lr0) || wants_grad(lr1) || wants_grad(lr2) || wants_grad(momentum));

@@ -137,3 +137,25 @@ def test_cpu_tensors_are_refused():
     with pytest.raises(RuntimeError, match="no CPU path"):
         from lact_amd import block_causal_lact_swiglu
         block_causal_lact_swiglu(w, w, w, x, x, x, lr, lr, lr, 2)
+
+
+def cpu_call(**changed):
+    """run_program on CPU tensors: whatever it refuses for another reason comes before the device's."""
+    import torch
+    b, L, d = 1, 8, 8
+    t = {n: torch.randn(b, d, d) for n in ("w0", "w1", "w2")} | {n: torch.randn(b, L, d) for n in "qkv"} | {n: torch.rand(b, L, 1) for n in ("lr0", "lr1", "lr2")}
+    prog = ops.Program(steps=((LACT_UPDATE, 0, L, 0), (LACT_APPLY, 0, L, 0)), out_len=L)
+    return ops.run_program(prog, **(t | changed))
+
+
+@pytest.mark.parametrize("name", ["w1", "q", "v", "lr2"])
+def test_forward_mode_tangents_are_refused(name):
+    """Also where nothing requires a gradient and the autograd function is passed by."""
+    import torch
+    import torch.autograd.forward_ad as fwad
+    shape = {"w1": (1, 8, 8), "lr2": (1, 8, 1)}.get(name, (1, 8, 8))
+    with fwad.dual_level():
+        with pytest.raises(NotImplementedError, match="jvp"):
+            cpu_call(**{name: fwad.make_dual(torch.randn(shape), torch.randn(shape))})
+    with pytest.raises(RuntimeError, match="HIP device"):
+        cpu_call()

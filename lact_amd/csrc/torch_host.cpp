@@ -303,8 +303,10 @@ py::tuple run_program(const c10::intrusive_ptr<Schedule>& sc, const Tensor& w0, 
                               (w0.requires_grad() || w1.requires_grad() || w2.requires_grad() || q.requires_grad() || wants_grad(k) ||
                                wants_grad(v) || wants_grad(lr0) || wants_grad(lr1) || wants_grad(lr2) || wants_grad(momentum));
   std::vector<Tensor> m_state;
+  const bool carries = momentum && sc->has_update;      // otherwise no update would continue from it
   if (m0 && m1 && m2) m_state = {*m0, *m1, *m2};
-  if (needs_backward && !m_state.empty() && momentum && sc->has_update)
+  else if (carries && (m0 || m1 || m2)) throw std::invalid_argument("a carried momentum state is three tensors, one for each of w0, w1, w2");
+  if (needs_backward && !m_state.empty() && carries)
     throw std::runtime_error("a carried momentum state is an inference feature: call under torch.no_grad()");
   variable_list res;
   {

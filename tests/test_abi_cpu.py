@@ -159,3 +159,15 @@ def test_forward_mode_tangents_are_refused(name):
             cpu_call(**{name: fwad.make_dual(torch.randn(shape), torch.randn(shape))})
     with pytest.raises(RuntimeError, match="HIP device"):
         cpu_call()
+
+
+@pytest.mark.parametrize("missing", [0, 1, 2])
+def test_incomplete_momentum_states_are_refused(missing):
+    """Continuing from two of the three states would restart the momentum without a word."""
+    import torch
+    state = [torch.zeros(1, 8, 8) for _ in range(3)]
+    state[missing] = None
+    with pytest.raises(ValueError, match="three tensors"):
+        cpu_call(momentum=torch.rand(1, 8, 1), momentum_state=tuple(state))
+    with pytest.raises(RuntimeError, match="HIP device"):      # nothing reads it without a momentum
+        cpu_call(momentum_state=tuple(state))

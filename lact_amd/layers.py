@@ -47,6 +47,16 @@ def _act(t: torch.Tensor):
     raise TypeError(f"unsupported activation dtype {t.dtype}: bf16 or fp32")
 
 
+def _expect(t: Optional[torch.Tensor], device: torch.device, shape, name: str):
+    """The kernels take raw pointers: a tensor elsewhere, or of another shape, has to be refused here."""
+    if t is None:
+        return
+    if t.device != device:
+        raise RuntimeError(f"expected all tensors to be on the same device: {name} is on {t.device}, not on {device}")
+    if tuple(t.shape) != tuple(shape):
+        raise ValueError(f"{name}: expected shape {tuple(shape)}, got {tuple(t.shape)}")
+
+
 class _PreFn(torch.autograd.Function):
     """qkv [B, L, 3*H*hd] -> q, k, v [(B H), L, hd]."""
 
@@ -54,6 +64,7 @@ class _PreFn(torch.autograd.Function):
     def forward(ctx, qkv, H, hd, l2norm):
         qkv = qkv.contiguous()
         B, L, _ = qkv.shape
+        _expect(qkv, qkv.device, (B, L, 3 * H * hd), "qkv")
         q, k, v = (torch.empty((B * H, L, hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3))
         with torch.cuda.device(qkv.device):
             _lib.check(_lib.lib().lact_layer_pre_forward(_act(qkv), B, L, H, hd, int(l2norm), _ptr(qkv), _ptr(q), _ptr(k),
@@ -84,6 +95,9 @@ class _PreAttnFn(torch.autograd.Function):
     def forward(ctx, qkv, qk_scale, qk_offset, H, hd, l2norm):
         qkv = qkv.contiguous()
         B, L, _ = qkv.shape
+        _expect(qkv, qkv.device, (B, L, 3 * H * hd), "qkv")
+        _expect(qk_scale, qkv.device, (H * hd, 2), "qk_scale")
+        _expect(qk_offset, qkv.device, (H * hd, 2), "qk_offset")
         scale, offset = qk_scale.detach().float().contiguous(), qk_offset.detach().float().contiguous()
         outs = [torch.empty((B * H, L, hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3)]
         att = [torch.empty((B, L, H * hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3)]
@@ -120,6 +134,8 @@ class _LrFn(torch.autograd.Function):
         lr_raw = lr_raw.float().contiguous()
         mom_c = None if mom_raw is None else mom_raw.float().contiguous()
         B, L, _ = lr_raw.shape
+        _expect(lr_raw, lr_raw.device, (B, L, 3 * H), "lr_raw")
+        _expect(mom_c, lr_raw.device, (B, L, H), "momentum_raw")
         outs = [torch.empty((B * H, L, 1), dtype=torch.float32, device=lr_raw.device) for _ in range(3)]
         mom = torch.empty((B * H, L, 1), dtype=torch.float32, device=lr_raw.device) if mom_c is not None else None
         with torch.cuda.device(lr_raw.device):
@@ -157,6 +173,10 @@ class _PostFn(torch.autograd.Function):
     def forward(ctx, o, weight, gate_raw, B, H, use_norm, eps, add=None):
         o = o.contiguous()
         _, L, hd = o.shape
+        _expect(o, o.device, (B * H, L, hd), "o")
+        _expect(weight, o.device, (hd,), "weight")
+        _expect(gate_raw, o.device, (B, L, H), "gate_raw")
+        _expect(add, o.device, (B, L, H * hd), "add")
         w = None if weight is None else weight.float().contiguous()
         g = None if gate_raw is None else gate_raw.to(o.dtype).contiguous()
         add_c = None if add is None else add.to(o.dtype).contiguous()
@@ -279,7 +299,7 @@ def sliding_window_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
     bf16 with heads of 64 or 128 runs in this library's kernels; other types and head sizes through torch's attention, where
     query blocks of `window` rows attend to their own and the previous block under a band mask."""
     b, l, h, d = q.shape
-    if q.is_cuda and d in (64, 128) and b * l > 0 and q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype == torch.bfloat16:
+    if q.is_cuda and d in (64, 128) and b * l > 0 and q.device == k.device == v.device and q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype == torch.bfloat16:
         return _WindowAttentionFn.apply(q, k, v, l if window is None else min(window, l))
     q, k, v = (t.transpose(1, 2) for t in (q, k, v))              # [b, h, l, d]
     if window is None or window >= l:

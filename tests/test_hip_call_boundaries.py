@@ -49,3 +49,21 @@ def test_second_derivatives_are_refused(name):
         torch.autograd.grad(penalty + sum(x.float().sum() for x in args), args, retain_graph=True)
     with pytest.raises(RuntimeError, match="once_differentiable"):
         penalty.backward()
+
+
+def test_tensors_on_another_device_or_of_another_shape_are_refused():
+    """Before anything is launched: the kernels would read them through their addresses."""
+    print("[gpu-test] devices and shapes", flush=True)
+    for name, changes in (("pre_attn", {1: (64, 2), 2: (32, 1)}), ("lr", {0: (1, 5, 5), 1: (1, 4, 2)}),
+                          ("post", {0: (4, 5, 16), 1: (32,), 2: (1, 5, 4), 3: (1, 1, 32)}), ("pre", {0: (1, 5, 48)})):
+        for i, shape in changes.items():
+            fn, args = CALLS[name]()
+            with pytest.raises(ValueError, match="expected shape"):
+                fn(*[randn(*shape) if j == i else a for j, a in enumerate(args)])
+            if i > 0:
+                with pytest.raises(RuntimeError, match="same device"):
+                    fn(*[a.detach().cpu() if j == i else a for j, a in enumerate(args)])
+    fn, args = CALLS["window"]()
+    for i in (1, 2):
+        with pytest.raises(RuntimeError, match="device"):
+            fn(*[a.detach().cpu() if j == i else a for j, a in enumerate(args)])

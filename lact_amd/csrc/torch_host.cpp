@@ -123,6 +123,15 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
   const int64_t b = w0.size(0), dh = w0.size(1), d = w0.size(2);
   if (w1.sizes() != at::IntArrayRef({b, d, dh}) || w2.sizes() != at::IntArrayRef({b, dh, d}))
     throw std::invalid_argument("expected w0, w2: [b, dh, d] and w1: [b, d, dh] with equal key and value dims");
+  // the kernels take raw pointers: a tensor elsewhere, or too small for the steps, has to be refused here
+  auto same_device = [&](const Tensor& t) { return t.device() == q.device(); };
+  auto here = [&](const OptTensor& t) { return !t || same_device(*t); };
+  if (!same_device(w0) || !same_device(w1) || !same_device(w2) || !here(k) || !here(v) || !here(lr0) || !here(lr1) || !here(lr2) || !here(momentum) ||
+      !std::all_of(m_state.begin(), m_state.end(), same_device))
+    throw std::runtime_error("expected all tensors to be on the same device as q");
+  auto is_rows = [&](const Tensor& t) { return t.dim() == 3 && t.size(0) == b && t.size(2) == d; };
+  if (!is_rows(q) || (sc.has_update && k && v && (!is_rows(*k) || !is_rows(*v) || v->size(1) < k->size(1))))
+    throw std::invalid_argument("expected q, k, v: [b, l, d] with the batch and feature size of the weights, and a row of v for every row of k");
   auto act = (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) ? at::kBFloat16 : at::kFloat;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) act = at::kBFloat16;
   Operands o;

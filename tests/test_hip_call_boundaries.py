@@ -67,3 +67,22 @@ def test_tensors_on_another_device_or_of_another_shape_are_refused():
     for i in (1, 2):
         with pytest.raises(RuntimeError, match="device"):
             fn(*[a.detach().cpu() if j == i else a for j, a in enumerate(args)])
+
+
+@pytest.mark.parametrize("grad", [False, True])
+def test_operands_on_another_device_or_of_another_shape_are_refused(grad):
+    print("[gpu-test] operands", grad, flush=True)
+    args = [t.detach().requires_grad_(grad) for t in operands(2, 24, 16, 24)]
+    swap = lambda i, t: [t if j == i else a for j, a in enumerate(args)]
+    for i in [0, 1, 2, 4, 5, 6, 7, 8]:
+        with pytest.raises(RuntimeError, match="same device"):
+            ops.run_program(PROGRAM, *swap(i, args[i].detach().cpu()))
+    for i in (3, 4, 5):
+        for shape in ((1, 24, 16), (2, 24, 8), (2, 24, 24), (2, 24)) + (((2, 23, 16),) if i == 5 else ()):
+            with pytest.raises(ValueError, match="expected q, k, v"):
+                ops.run_program(PROGRAM, *swap(i, randn(*shape)))
+    with pytest.raises(RuntimeError, match="same device"):
+        ops.run_program(PROGRAM, *args, torch.rand(2, 24, 1))
+    state = [torch.zeros_like(w) for w in args[:3]]
+    with torch.no_grad(), pytest.raises(RuntimeError, match="same device"):
+        ops.run_program(PROGRAM, *args, randn(2, 24, 1), (state[0], state[1].cpu(), state[2]))

@@ -21,6 +21,8 @@ from typing import Optional
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+from torch.autograd import forward_ad as fwad
+from torch.utils._python_dispatch import _get_current_dispatch_mode
 
 from . import _lib
 from ._autograd import once_differentiable
@@ -254,53 +256,19 @@ class BidirectionalLaCTSwiGLU(nn.Module):
         return self.o_proj(_PostFn.apply(o, weight, None, B, self.num_heads, use_norm, eps))
 
 
+MAX_TOKEN_STRIDE = 1 << 24     # elements; the kernels' offsets inside a tile are 32-bit
+
+
 def _head_rows(t: torch.Tensor) -> torch.Tensor:
     """[b, l, h, d] whose heads lie next to each other inside a token, 16-byte aligned."""
     ok = (t.stride(3) == 1 and t.stride(2) == t.shape[3] and t.stride(1) % 8 == 0 and t.stride(0) % 8 == 0
-          and t.stride(1) >= t.shape[2] * t.shape[3] and t.data_ptr() % 16 == 0)
-    return t if ok else t.contiguous()
+          and t.shape[2] * t.shape[3] <= t.stride(1) <= MAX_TOKEN_STRIDE and t.data_ptr() % 16 == 0)
+    # clone: contiguous() hands back what merely starts off a 16-byte boundary or has odd strides in dimensions of size 1
+    return t if ok else t.clone(memory_format=torch.contiguous_format)
 
 
-class _WindowAttentionFn(torch.autograd.Function):
-    """bf16 sliding-window attention on [b, l, h, d], d = 64 or 128 (csrc/window_attention.h)."""
-
-    @staticmethod
-    def forward(ctx, q, k, v, window):
-        q, k, v = _head_rows(q), _head_rows(k), _head_rows(v)
-        B, L, H, D = q.shape
-        out = torch.empty((B, L, H, D), dtype=q.dtype, device=q.device)
-        lse = torch.empty((B, H, L), dtype=torch.float32, device=q.device)
-        with torch.cuda.device(q.device):
-            _lib.check(_lib.lib().lact_window_attention_forward(
-                B, L, H, D, window, _ptr(q), q.stride(1), q.stride(0), _ptr(k), k.stride(1), k.stride(0), _ptr(v), v.stride(1), v.stride(0),
-                _ptr(out), _ptr(lse), _stream(q)))
-        ctx.save_for_backward(q, k, v, out, lse)
-        ctx.window = window
-        return out
-
-    @staticmethod
-    @once_differentiable
-    def backward(ctx, g):
-        q, k, v, out, lse = ctx.saved_tensors
-        B, L, H, D = q.shape
-        g = _head_rows(g.to(q.dtype))
-        dq, dk, dv = (torch.empty((B, L, H, D), dtype=q.dtype, device=q.device) for _ in range(3))
-        delta = torch.empty_like(lse)
-        with torch.cuda.device(q.device):
-            _lib.check(_lib.lib().lact_window_attention_backward(
-                B, L, H, D, ctx.window, _ptr(q), q.stride(1), q.stride(0), _ptr(k), k.stride(1), k.stride(0), _ptr(v), v.stride(1), v.stride(0),
-                _ptr(out), _ptr(lse), _ptr(g), g.stride(1), g.stride(0), _ptr(delta), _ptr(dq), _ptr(dk), _ptr(dv), _stream(q)))
-        return dq, dk, dv, None
-
-
-def sliding_window_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window: Optional[int]) -> torch.Tensor:
-    """q, k, v: [b, l, h, d].  Causal attention where query i sees keys i-(window-1) .. i -- what the reference asks
-    of flash_attn_func(causal=True, window_size=(window-1, 0)) (causal_lact_with_sliding_window_attn.py:371-375).
-    bf16 with heads of 64 or 128 runs in this library's kernels; other types and head sizes through torch's attention, where
-    query blocks of `window` rows attend to their own and the previous block under a band mask."""
-    b, l, h, d = q.shape
-    if q.is_cuda and d in (64, 128) and b * l > 0 and q.device == k.device == v.device and q.shape == k.shape == v.shape and q.dtype == k.dtype == v.dtype == torch.bfloat16:
-        return _WindowAttentionFn.apply(q, k, v, l if window is None else min(window, l))
+def _torch_window_attention(q, k, v, window):
+    l = q.shape[1]
     q, k, v = (t.transpose(1, 2) for t in (q, k, v))              # [b, h, l, d]
     if window is None or window >= l:
         return F.scaled_dot_product_attention(q, k, v, is_causal=True).transpose(1, 2)
@@ -313,6 +281,116 @@ def sliding_window_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, 
         mask = (kj <= qi) & (kj >= qi - (window - 1))
         outs.append(F.scaled_dot_product_attention(q[:, :, s:e], k[:, :, ks:e], v[:, :, ks:e], attn_mask=mask))
     return torch.cat(outs, dim=2).transpose(1, 2)
+
+
+def _on_window_kernels(q, k, v) -> bool:
+    """Whether csrc/window_attention.h takes the call: its type, head sizes and limits, on plain tensors.  What sees the call as
+    tensor operations (vmap and the other function transforms, forward-mode differentiation, dispatch modes, tensor subclasses,
+    autocast to another type) gets them."""
+    b, l, h, d = q.shape
+    if not (q.is_cuda and d in (64, 128) and b * l * h > 0 and q.device == k.device == v.device and q.shape == k.shape == v.shape
+            and q.dtype == k.dtype == v.dtype == torch.bfloat16):
+        return False
+    if b * h > 1 << 20 or l * h * d > 1 << 31 or h * d > MAX_TOKEN_STRIDE:
+        return False
+    if torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") != torch.bfloat16:
+        return False
+    return torch.compiler.is_compiling() or not (
+        torch._C._are_functorch_transforms_active() or torch.jit.is_tracing() or _get_current_dispatch_mode() is not None
+        or any(type(t) not in (torch.Tensor, nn.Parameter) or torch._C._functorch.is_legacy_batchedtensor(t) for t in (q, k, v))
+        or (fwad._current_level >= 0 and any(fwad.unpack_dual(t).tangent is not None for t in (q, k, v))))
+
+
+def _window_forward(q, k, v, window):
+    B, L, H, D = q.shape
+    out = torch.empty((B, L, H, D), dtype=q.dtype, device=q.device)
+    lse = torch.empty((B, H, L), dtype=torch.float32, device=q.device)
+    with torch.cuda.device(q.device):
+        _lib.check(_lib.lib().lact_window_attention_forward(
+            B, L, H, D, window, _ptr(q), q.stride(1), q.stride(0), _ptr(k), k.stride(1), k.stride(0), _ptr(v), v.stride(1), v.stride(0),
+            _ptr(out), _ptr(lse), _stream(q)))
+    return out, lse
+
+
+def _window_backward(g, q, k, v, out, lse, window):
+    B, L, H, D = q.shape
+    g = _head_rows(g.to(q.dtype))
+    dq, dk, dv = (torch.empty((B, L, H, D), dtype=q.dtype, device=q.device) for _ in range(3))
+    delta = torch.empty_like(lse)
+    with torch.cuda.device(q.device):
+        _lib.check(_lib.lib().lact_window_attention_backward(
+            B, L, H, D, window, _ptr(q), q.stride(1), q.stride(0), _ptr(k), k.stride(1), k.stride(0), _ptr(v), v.stride(1), v.stride(0),
+            _ptr(out), _ptr(lse), _ptr(g), g.stride(1), g.stride(0), _ptr(delta), _ptr(dq), _ptr(dk), _ptr(dv), _stream(q)))
+    return dq, dk, dv
+
+
+class _WindowAttentionFn(torch.autograd.Function):
+    """bf16 sliding-window attention on [b, l, h, d], d = 64 or 128 (csrc/window_attention.h)."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, window):
+        q, k, v = _head_rows(q), _head_rows(k), _head_rows(v)
+        out, lse = _window_forward(q, k, v, window)
+        ctx.save_for_backward(q, k, v, out, lse)
+        ctx.window = window
+        return out
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, g):
+        q, k, v, out, lse = ctx.saved_tensors
+        if torch._C._functorch.is_legacy_batchedtensor(g):      # is_grads_batched: the batch is torch's business
+            with torch.enable_grad():
+                x = [t.detach().requires_grad_() for t in (q, k, v)]
+                return (*torch.autograd.grad(_torch_window_attention(*x, ctx.window), x, g), None)
+        return (*_window_backward(g, q, k, v, out, lse, ctx.window), None)
+
+
+# The same as operators, which torch.compile traces through (their dispatch costs an eager call more than the function above).
+@torch.library.custom_op("lact_amd::window_attention", mutates_args=(), schema="(Tensor q, Tensor k, Tensor v, int window) -> (Tensor, Tensor)")
+def _window_attention_op(q, k, v, window):
+    return _window_forward(_head_rows(q), _head_rows(k), _head_rows(v), window)
+
+
+@_window_attention_op.register_fake
+def _(q, k, v, window):
+    b, l, h, _ = q.shape
+    return q.new_empty(q.shape), q.new_empty((b, h, l), dtype=torch.float32)
+
+
+@torch.library.custom_op("lact_amd::window_attention_backward", mutates_args=(),
+                         schema="(Tensor g, Tensor q, Tensor k, Tensor v, Tensor out, Tensor lse, int window) -> (Tensor, Tensor, Tensor)")
+def _window_attention_backward_op(g, q, k, v, out, lse, window):
+    return _window_backward(g, _head_rows(q), _head_rows(k), _head_rows(v), out.contiguous(), lse.contiguous(), window)
+
+
+@_window_attention_backward_op.register_fake
+def _(g, q, k, v, out, lse, window):
+    return q.new_empty(q.shape), q.new_empty(q.shape), q.new_empty(q.shape)
+
+
+def _window_attention_setup(ctx, inputs, output):
+    ctx.save_for_backward(*inputs[:3], *output)
+    ctx.window = inputs[3]
+    ctx.mark_non_differentiable(output[1])
+
+
+def _window_attention_vjp(ctx, g, _):
+    return (*_window_attention_backward_op(g, *ctx.saved_tensors, ctx.window), None)
+
+
+_window_attention_op.register_autograd(_window_attention_vjp, setup_context=_window_attention_setup)
+
+
+def sliding_window_attention(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor, window: Optional[int]) -> torch.Tensor:
+    """q, k, v: [b, l, h, d].  Causal attention where query i sees keys i-(window-1) .. i -- what the reference asks
+    of flash_attn_func(causal=True, window_size=(window-1, 0)) (causal_lact_with_sliding_window_attn.py:371-375).
+    bf16 with heads of 64 or 128 runs in this library's kernels; other types and head sizes through torch's attention, where
+    query blocks of `window` rows attend to their own and the previous block under a band mask."""
+    if _on_window_kernels(q, k, v):
+        width = q.shape[1] if window is None else min(window, q.shape[1])
+        return _window_attention_op(q, k, v, width)[0] if torch.compiler.is_compiling() else _WindowAttentionFn.apply(q, k, v, width)
+    return _torch_window_attention(q, k, v, window)
 
 
 class CausalLaCTSwiGLUWithSlidingWindowAttn(nn.Module):

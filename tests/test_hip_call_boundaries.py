@@ -5,6 +5,7 @@ import torch
 
 from lact_amd import layers as HL
 from lact_amd import ops
+from oracle.lact_oracle import rel_l2
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda"
@@ -86,3 +87,65 @@ def test_operands_on_another_device_or_of_another_shape_are_refused(grad):
     state = [torch.zeros_like(w) for w in args[:3]]
     with torch.no_grad(), pytest.raises(RuntimeError, match="same device"):
         ops.run_program(PROGRAM, *args, randn(2, 24, 1), (state[0], state[1].cpu(), state[2]))
+
+
+def window_args(shape=(2, 70, 2, 64), seed=0):
+    return [randn(*shape, dtype=torch.bfloat16, seed=seed + i) for i in range(3)]
+
+
+def close(a, b):
+    """Two bf16 attentions of the same inputs, each within a few bf16 roundings of the exact one."""
+    assert a.shape == b.shape and rel_l2(a, b) < 1e-2
+
+
+def test_function_transforms_reach_the_window_attention():
+    """vmap, reverse and forward mode of torch.func, batched gradients: what sees tensor operations gets them."""
+    print("[gpu-test] window attention under transforms", flush=True)
+    attend = lambda *x: HL.sliding_window_attention(*x, 17)
+    x = [torch.stack([a, b]).detach() for a, b in zip(window_args(), window_args(seed=3))]
+    ref = torch.stack([attend(*[t[i] for t in x]) for i in (0, 1)])
+    close(torch.vmap(attend)(*x), ref)
+    one = [t[0].clone().requires_grad_() for t in x]
+    go = torch.stack([randn(2, 70, 2, 64, dtype=torch.bfloat16, seed=s, grad=False) for s in (7, 8)])
+    loops = [torch.autograd.grad(attend(*one), one, g) for g in go]
+    for i, a in enumerate(torch.autograd.grad(attend(*one), one, go, is_grads_batched=True)):
+        close(a, torch.stack([l[i] for l in loops]))
+    pulled = torch.func.vjp(attend, *[t.detach() for t in one])[1](go[0])
+    for a, b in zip(pulled, loops[0]):
+        close(a, b)
+    with torch.autocast("cuda", dtype=torch.float16):
+        assert attend(*one).dtype == torch.float16
+
+
+def test_window_attention_takes_views_that_start_anywhere():
+    """Off a 16-byte boundary, with odd strides in dimensions of size one, or with rows further apart than the kernels' limit."""
+    print("[gpu-test] window attention views", flush=True)
+    for shape in ((2, 70, 2, 64), (1, 1, 2, 64)):
+        n = torch.Size(shape).numel()
+        ref = [randn(*shape, dtype=torch.bfloat16, seed=i, grad=False) for i in range(3)]
+        flat = torch.zeros(n + 1, dtype=torch.bfloat16, device=DEV)
+        flat[1:] = ref[0].flatten()
+        off = flat[1:].view(shape)
+        wide = torch.zeros(shape[0], shape[1], 3 * 128 + 1, dtype=torch.bfloat16, device=DEV)
+        wide[..., :128] = ref[1].flatten(2)
+        odd = wide[..., :128].unflatten(2, (2, 64))
+        assert torch.equal(HL.sliding_window_attention(off, odd, ref[2], 9), HL.sliding_window_attention(*ref, 9))
+    far = torch.zeros(2, (1 << 24) + 8, dtype=torch.bfloat16, device=DEV)
+    rows = randn(1, 2, 1, 64, dtype=torch.bfloat16, grad=False)
+    far[:, :64] = rows[0, :, 0]
+    view = far[:, :64].view(1, 2, 1, 64)
+    assert torch.equal(HL.sliding_window_attention(view, view, view, None), HL.sliding_window_attention(rows, rows, rows, None))
+
+
+def test_window_attention_beyond_the_kernel_limits_and_compiled():
+    print("[gpu-test] window attention limits", flush=True)
+    many = torch.randn(59000, 1, 18, 64, dtype=torch.bfloat16, device=DEV)      # batch entries times heads beyond 2^20
+    assert not HL._on_window_kernels(many, many, many) and torch.equal(HL.sliding_window_attention(many, many, many, None), many)
+    x = window_args()
+    fn = torch.compile(lambda *t: HL.sliding_window_attention(*t, 17), fullgraph=True, backend="aot_eager")
+    go = torch.ones(2, 70, 2, 64, dtype=torch.bfloat16, device=DEV)
+    for call in (fn, lambda *t: HL.sliding_window_attention(*t, 17)):
+        out = call(*x)
+        res = [out] + list(torch.autograd.grad(out, x, go))
+        first = res if call is fn else first
+    assert all(torch.equal(a, b) for a, b in zip(first, res))

@@ -65,17 +65,20 @@ void check(int rc) {
   if (rc != 0) throw std::runtime_error(std::string("liblact_hip: ") + lact_last_error());
 }
 
-// [b, L, d] whose rows the kernels can read with 16-byte vectors
+bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0; }
+
+// [b, L, d] whose rows the kernels can read with 16-byte vectors.  A clone where they cannot: contiguous() hands back what merely
+// starts off a 16-byte boundary or has odd strides in dimensions of size 1.
 Tensor rows_view(Tensor t, at::ScalarType dtype) {
   if (t.scalar_type() != dtype) t = t.to(dtype);
   const int64_t align = 16 / t.element_size();
-  const bool ok = t.dim() == 3 && t.stride(2) == 1 && t.stride(1) % align == 0 && t.stride(0) % align == 0 && t.stride(1) >= t.size(2) &&
-                  reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
-  return ok ? t : t.contiguous();
+  const bool ok = t.dim() == 3 && t.stride(2) == 1 && t.stride(1) % align == 0 && t.stride(0) % align == 0 && t.stride(1) >= t.size(2) && aligned16(t);
+  return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 
 Tensor plain_f32(const Tensor& t) {
-  return t.scalar_type() == at::kFloat ? t.contiguous() : t.to(at::kFloat).contiguous();
+  const Tensor c = t.scalar_type() == at::kFloat ? t.contiguous() : t.to(at::kFloat).contiguous();
+  return aligned16(c) ? c : c.clone();
 }
 
 Tensor per_token(const Tensor& t, int64_t b, int64_t L, const char* name) {
@@ -149,8 +152,7 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
   }
   // weights that are transposed views of contiguous fp32 tensors (the view-synthesis model's layout) are read as they lie
   auto lies_transposed = [](const Tensor& t) {
-    return t.scalar_type() == at::kFloat && t.stride(1) == 1 && t.stride(2) == t.size(1) && t.stride(0) == t.size(1) * t.size(2) && t.size(2) > 1 &&
-           reinterpret_cast<uintptr_t>(t.const_data_ptr()) % 16 == 0;
+    return t.scalar_type() == at::kFloat && t.stride(1) == 1 && t.stride(2) == t.size(1) && t.stride(0) == t.size(1) * t.size(2) && t.size(2) > 1 && aligned16(t);
   };
   const bool transposed = lies_transposed(w0) && lies_transposed(w1) && lies_transposed(w2);
   const Tensor w[3] = {transposed ? w0 : plain_f32(w0), transposed ? w1 : plain_f32(w1), transposed ? w2 : plain_f32(w2)};

@@ -149,3 +149,29 @@ def test_window_attention_beyond_the_kernel_limits_and_compiled():
         res = [out] + list(torch.autograd.grad(out, x, go))
         first = res if call is fn else first
     assert all(torch.equal(a, b) for a, b in zip(first, res))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_operands_may_start_anywhere(dtype):
+    """Contiguous views off a 16-byte boundary, and odd strides in the batch dimension of one entry: the same bits."""
+    print("[gpu-test] operands that start anywhere", dtype, flush=True)
+
+    def shifted(t):
+        flat = torch.zeros(t.numel() + 1, dtype=t.dtype, device=DEV)
+        flat[1:] = t.flatten()
+        view = flat[1:].view(t.shape)
+        assert view.is_contiguous() and view.data_ptr() % 16
+        return view
+    args = [t.detach() for t in operands(1, 24, 16, 24)]
+    args[3:6] = [t.to(dtype) for t in args[3:6]]
+    for i in (3, 4, 5):      # a batch stride that no vector divides
+        args[i] = args[i].as_strided(args[i].shape, (24 * 16 + 1, 16, 1))
+    ref_args = [t.clone(memory_format=torch.contiguous_format) for t in args]
+    go = shifted(randn(1, 24, 16, dtype=dtype, seed=9, grad=False))
+    res = []
+    for xs in (ref_args, [shifted(t) for t in args], args):
+        x = [t.detach().requires_grad_() for t in xs]
+        out, ws, _ = ops.run_program(PROGRAM, *x)
+        res.append([out, *ws] + list(torch.autograd.grad([out, *ws], x, [go, *[torch.ones_like(w) for w in ws]])))
+    for other in res[1:]:
+        assert all(torch.equal(a, b) for a, b in zip(other, res[0]))

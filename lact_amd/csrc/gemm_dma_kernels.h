@@ -609,7 +609,7 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_bwd_hidden_dma(cons
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O5) + off) = pack8(o5);
       }
       if ((threadIdx.x & 3) == 0) {
-        const size_t lo = (size_t)(by * TS::WAVES_N + ((threadIdx.x & 7) >> 2)) * p.lrpart_stride + (size_t)z * p.Tcap + m;
+        const size_t lo = (size_t)(by * TS::WAVES_N + ((threadIdx.x & 7) >> 2)) * p.lrpart_stride + (size_t)z * p.Tupd + m;
         p.lrpart[0 * p.lrpart_mat_stride + lo] = s0;
         p.lrpart[1 * p.lrpart_mat_stride + lo] = s1;
         p.lrpart[2 * p.lrpart_mat_stride + lo] = s2;
@@ -752,7 +752,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + o) = pack8(o1);
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + o) = pack8(o2);
         if (j8 == 0) {
-          const size_t lo = (size_t)(by * TS::WAVES_N + h) * p.lrpart_stride + (size_t)z * p.Tcap + m;
+          const size_t lo = (size_t)(by * TS::WAVES_N + h) * p.lrpart_stride + (size_t)z * p.Tupd + m;
           p.lrpart[0 * p.lrpart_mat_stride + lo] = s0;
           p.lrpart[1 * p.lrpart_mat_stride + lo] = s1;
           p.lrpart[2 * p.lrpart_mat_stride + lo] = s2;
@@ -764,7 +764,7 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
   // a half past the end of dh contributes nothing, but its slot of partial sums is read all the same
   for (int h = halves; h < TS::WAVES_N; ++h)
     if ((int)threadIdx.x < TS::BM && m0 + (int)threadIdx.x < p.T) {
-      const size_t lo = (size_t)(by * TS::WAVES_N + h) * p.lrpart_stride + (size_t)z * p.Tcap + m0 + threadIdx.x;
+      const size_t lo = (size_t)(by * TS::WAVES_N + h) * p.lrpart_stride + (size_t)z * p.Tupd + m0 + threadIdx.x;
       p.lrpart[0 * p.lrpart_mat_stride + lo] = 0.f;
       p.lrpart[1 * p.lrpart_mat_stride + lo] = 0.f;
       p.lrpart[2 * p.lrpart_mat_stride + lo] = 0.f;

@@ -141,9 +141,9 @@ struct HiddenParams {
   long long bso;
   // update backward from kept pre-activations: I0 = k W0^T, I1 = k W2^T, I2 = v W1 as the forward rounded them
   const void* I0; const void* I1; const void* I2; long long bsi;
-  float* lrpart; long long lrpart_stride;  // partial row sums: [3][nparts][b*Tcap]; stride between parts
+  float* lrpart; long long lrpart_stride;  // partial row sums: [3][nparts][b*Tupd]; stride between parts
   long long lrpart_mat_stride;
-  int Tcap;
+  int Tupd;                        // longest update of the program
 };
 
 // apply forward:  O0 = silu(X W0^T) * (X W2^T)                       (ttt_operation.py:141-143)
@@ -266,7 +266,7 @@ __device__ __forceinline__ void store_row_partials(const HiddenParams& p, int wh
   v += __shfl_xor(v, 32, 64);
   if ((threadIdx.x & 63) < 32 && m < p.T) {
     const int slot = ytile * TS::WAVES_N + ((threadIdx.x >> 6) % TS::WAVES_N);
-    p.lrpart[which * p.lrpart_mat_stride + slot * p.lrpart_stride + (size_t)z * p.Tcap + m] = v;
+    p.lrpart[which * p.lrpart_mat_stride + slot * p.lrpart_stride + (size_t)z * p.Tupd + m] = v;
   }
 }
 

@@ -596,7 +596,7 @@ struct Runner {
   }
   template <typename U> U* scr(size_t off) const { return reinterpret_cast<U*>(sc + off); }
 
-  long long hbs() const { return (long long)P.Tcap * d.dh; }
+  long long hbs(int T_) const { return (long long)T_ * d.dh; }   // between the batch entries of a step's token-major arrays
 
   HiddenParams hidden_params(int T_, const void* X, int ldx, long long bsx, const void* Y, int ldy, long long bsy, int ver) const {
     HiddenParams p;
@@ -605,8 +605,8 @@ struct Runner {
     p.X = X; p.ldx = ldx; p.bsx = bsx;
     p.Y = Y; p.ldy = ldy; p.bsy = bsy;
     p.W0 = wc(ver, 0); p.W1 = wc(ver, 1); p.W2 = wc(ver, 2); p.bsw = P.g.elems;
-    p.bso = hbs();
-    p.Tcap = P.Tcap;
+    p.bso = hbs(T_);
+    p.Tupd = P.Tupd;
     return p;
   }
 
@@ -807,7 +807,7 @@ struct Runner {
       HiddenParams hp = hidden_params(T_, q + (size_t)g.st.start * d.q_ld, d.q_ld, d.q_bs, nullptr, 0, 0, g.ver);
       hp.O0 = h(0);
       auto p = row_params<1>();
-      set_term(p.t[0], h(0), d.dh, hbs(), wc(g.ver, 1), d.dh, P.g.elems, d.dh);
+      set_term(p.t[0], h(0), d.dh, hbs(T_), wc(g.ver, 1), d.dh, P.g.elems, d.dh);
       p.M = T_; p.N = d.d; p.out = out + (size_t)g.st.out_start * d.o_ld; p.ldo = d.o_ld; p.bso = d.o_bs;
       if (g.n > 1) {
         hp.steps.by_nb = p.steps.by_nb = make_udiv(d.b);
@@ -843,9 +843,9 @@ struct Runner {
         hp.lr0 = lr0 + st.start; hp.lr1 = lr1 + st.start; hp.lr2 = lr2 + st.start; hp.bslr = d.kv_len;
         // operands of the three gradient GEMMs: dgate_before_act, hidden * lr1, dhidden_before_mul
         T* z0 = h(0); T* z1 = h(1); T* z2 = h(2);
-        long long zbs = hbs();
+        long long zbs = hbs(T_);
         if (P.keep_pre) {
-          // the unscaled operands stay in scratch (each region holds b * Tcap * dh elements: room for this stride)
+          // the unscaled operands stay in scratch
           z0 = h(0); z1 = pre(u, 1); z2 = h(2); zbs = pre_bs(u);
           hp.O3 = pre(u, 3); hp.O4 = pre(u, 4); hp.O5 = pre(u, 5);
           hp.O6 = pre(u, 0); hp.O7 = pre(u, 2);
@@ -1130,7 +1130,7 @@ struct Runner {
           if (ups[i].start < ups[j].end && ups[j].start < ups[i].end) lr_each = true;
     }
     std::vector<std::pair<int, int>> lr_ranges;   // met in descending order of the update index, all updates
-    const size_t lrslot = (size_t)3 * P.lr_slots * d.b * P.Tcap;
+    const size_t lrslot = (size_t)3 * P.lr_slots * d.b * P.Tupd;
     std::vector<int> mg_updates;
     int mg_parts = P.nblk;   // partial dots per matrix in a momentum-gradient slot (the same for every update)
     std::vector<std::pair<int, int>> mg_ranges;
@@ -1153,15 +1153,16 @@ struct Runner {
     bool side_used = false;
     // Backward of apply steps: weight gradients to full arrays by version (`g.ver` and on; `add`: to what they hold), dq
     auto apply_jobs = [&](const ApplyGroup& g, TokenReduceJob (&jobs)[3]) {
+      const int T_ = g.st.end - g.st.start;
       const T* qc = q + (size_t)g.st.start * d.q_ld;
       const T* gc = dout + (size_t)g.st.out_start * d.do_ld;
       memset(jobs, 0, sizeof(jobs));
       jobs[0].M = jobs[2].M = d.dh; jobs[0].N = jobs[2].N = d.d;
-      set_tr_term(jobs[0].t, h(1), d.dh, hbs(), qc, d.q_ld, d.q_bs);
+      set_tr_term(jobs[0].t, h(1), d.dh, hbs(T_), qc, d.q_ld, d.q_bs);
       jobs[1].M = d.d; jobs[1].N = d.dh;
-      set_tr_term(jobs[1].t, gc, d.do_ld, d.do_bs, h(0), d.dh, hbs());
-      set_tr_term(jobs[2].t, h(2), d.dh, hbs(), qc, d.q_ld, d.q_bs);
-      const long long gsh = (long long)d.b * hbs();
+      set_tr_term(jobs[1].t, gc, d.do_ld, d.do_bs, h(0), d.dh, hbs(T_));
+      set_tr_term(jobs[2].t, h(2), d.dh, hbs(T_), qc, d.q_ld, d.q_bs);
+      const long long gsh = (long long)d.b * hbs(T_);
       jobs[0].t.gsA = jobs[2].t.gsA = jobs[1].t.gsB = gsh;
       jobs[0].t.gsB = jobs[2].t.gsB = (long long)g.dstart * d.q_ld;
       jobs[1].t.gsA = (long long)g.dout * d.do_ld;
@@ -1179,8 +1180,8 @@ struct Runner {
     auto dq_gemm = [&](const ApplyGroup& g) {   // dq = gY0 W0 + gY2 W2
       const int T_ = g.st.end - g.st.start;
       auto p = row_params<2>();
-      set_term(p.t[0], h(1), d.dh, hbs(), wc(g.ver, 0), d.d, P.g.elems, d.dh);
-      set_term(p.t[1], h(2), d.dh, hbs(), wc(g.ver, 2), d.d, P.g.elems, d.dh);
+      set_term(p.t[0], h(1), d.dh, hbs(T_), wc(g.ver, 0), d.d, P.g.elems, d.dh);
+      set_term(p.t[1], h(2), d.dh, hbs(T_), wc(g.ver, 2), d.d, P.g.elems, d.dh);
       p.M = T_; p.N = d.d; p.ldo = d.d; p.bso = (long long)d.q_len * d.d;
       int acc = 0;
       std::vector<char> accs(g.n);
@@ -1195,7 +1196,7 @@ struct Runner {
           pi.t[0].gsB = pi.t[1].gsB = (long long)P.mat3; pi.gso = (long long)g.dstart * d.d;
         }
         for (int t = 0; t < 2 && i > 0; ++t) {
-          pi.t[t].A = (const T*)pi.t[t].A + (size_t)i * d.b * hbs();
+          pi.t[t].A = (const T*)pi.t[t].A + (size_t)i * d.b * hbs(T_);
           pi.t[t].B = (const T*)pi.t[t].B + (size_t)i * P.mat3;
         }
         launch_row_gemm<T, false, 2, EPI_STORE>("apply_bwd_dq", pi, d.b * (together ? g.n : 1), s, true);
@@ -1213,7 +1214,7 @@ struct Runner {
         const int T_ = g.st.end - g.st.start;
         side_used = true;
         apply_hidden_bwd(g);
-        float* dst = scr<float>(P.t_gwside) + (size_t)g.ver * P.mat3;
+        float* dst = scr<float>(P.t_gwside) + (size_t)P.gw_slot[g.ver] * P.mat3;   // a group's versions have consecutive places
         bool add = false;
         for (int i = 0; i < g.n; ++i) add = add || gw_side[g.ver + i];
         if (add)   // another step on one of these versions came before
@@ -1439,15 +1440,15 @@ struct Runner {
       T* g0 = gcm; T* g1 = gcm + (size_t)d.b * P.g.elems; T* g2 = gcm + (size_t)2 * d.b * P.g.elems;
       // lr-scaled operands of the forward's gradient GEMMs: kept by the forward, or written again by the hidden kernel
       T* z0 = h(3); T* z1 = h(4); T* z2 = h(5);
-      long long zbs = hbs();
+      long long zbs = hbs(T_);
       {
         HiddenParams hp = hidden_params(T_, kc, d.k_ld, d.k_bs, vc, d.v_ld, d.v_bs, vprev);
         hp.lr0 = lr0 + st.start; hp.lr1 = lr1 + st.start; hp.lr2 = lr2 + st.start; hp.bslr = d.kv_len;
         hp.G0 = g0; hp.G1 = g1; hp.G2 = g2;
         hp.O0 = h(0); hp.O1 = h(1); hp.O2 = h(2); hp.O3 = h(3); hp.O4 = h(4); hp.O5 = h(5);
         hp.lrpart = scr<float>(P.t_lrpart) + (size_t)u * lrslot;
-        hp.lrpart_stride = (long long)d.b * P.Tcap;
-        hp.lrpart_mat_stride = (long long)P.lr_slots * d.b * P.Tcap;
+        hp.lrpart_stride = (long long)d.b * P.Tupd;
+        hp.lrpart_mat_stride = (long long)P.lr_slots * d.b * P.Tupd;
         if (P.keep_pre) {
           hp.I0 = pre(u, 3); hp.I1 = pre(u, 4); hp.I2 = pre(u, 5); hp.bsi = pre_bs(u);
           hp.O3 = hp.O4 = hp.O5 = nullptr;
@@ -1464,8 +1465,8 @@ struct Runner {
         auto p = row_params<4>();
         set_term(p.t[0], z0, d.dh, zbs, g0, d.d, P.g.elems, d.dh);
         set_term(p.t[1], z2, d.dh, zbs, g2, d.d, P.g.elems, d.dh);
-        set_term(p.t[2], h(0), d.dh, hbs(), wc(vprev, 0), d.d, P.g.elems, d.dh);
-        set_term(p.t[3], h(2), d.dh, hbs(), wc(vprev, 2), d.d, P.g.elems, d.dh);
+        set_term(p.t[2], h(0), d.dh, hbs(T_), wc(vprev, 0), d.d, P.g.elems, d.dh);
+        set_term(p.t[3], h(2), d.dh, hbs(T_), wc(vprev, 2), d.d, P.g.elems, d.dh);
         p.M = T_; p.N = d.d; p.out = dk + (size_t)st.start * d.d; p.ldo = d.d; p.bso = (long long)d.kv_len * d.d;
         p.accumulate = acc_kv;
         rows_job.r4 = p;
@@ -1473,7 +1474,7 @@ struct Runner {
       {  // dv = (hidden*lr1) G1^T + gDH W1^T
         auto p = row_params<2>();
         set_term(p.t[0], z1, d.dh, zbs, g1, d.dh, P.g.elems, d.dh);
-        set_term(p.t[1], h(1), d.dh, hbs(), wc(vprev, 1), d.dh, P.g.elems, d.dh);
+        set_term(p.t[1], h(1), d.dh, hbs(T_), wc(vprev, 1), d.dh, P.g.elems, d.dh);
         p.M = T_; p.N = d.d; p.out = dv + (size_t)st.start * d.d; p.ldo = d.d; p.bso = (long long)d.kv_len * d.d;
         p.accumulate = acc_kv;
         rows_job.r2 = p;
@@ -1484,8 +1485,8 @@ struct Runner {
         MomentumMeanRanges r1;
         r1.start[0] = st.start; r1.len[0] = T_;
         LACT_LAUNCH("k_lr_reduce", "k_lr_reduce", 0.0, k_lr_reduce, dim3(ceil_div(T_, 256), d.b, 3), dim3(256), s,
-                    scr<float>(P.t_lrpart) + (size_t)u * lrslot, 0LL, (long long)P.lr_slots * d.b * P.Tcap, (long long)d.b * P.Tcap, lr_parts(),
-                    P.Tcap, dlr0, dlr1, dlr2, (long long)d.kv_len, r1, acc_kv ? 1 : 0);
+                    scr<float>(P.t_lrpart) + (size_t)u * lrslot, 0LL, (long long)P.lr_slots * d.b * P.Tupd, (long long)d.b * P.Tupd, lr_parts(),
+                    P.Tupd, dlr0, dlr1, dlr2, (long long)d.kv_len, r1, acc_kv ? 1 : 0);
       } else {
         lr_ranges.emplace_back(st.start, T_);
       }
@@ -1493,11 +1494,11 @@ struct Runner {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));
         jobs[0].M = d.dh; jobs[0].N = d.d;
-        set_tr_term(jobs[0].t, h(0), d.dh, hbs(), kc, d.k_ld, d.k_bs);
+        set_tr_term(jobs[0].t, h(0), d.dh, hbs(T_), kc, d.k_ld, d.k_bs);
         jobs[1].M = d.d; jobs[1].N = d.dh;
-        set_tr_term(jobs[1].t, vc, d.v_ld, d.v_bs, h(1), d.dh, hbs());
+        set_tr_term(jobs[1].t, vc, d.v_ld, d.v_bs, h(1), d.dh, hbs(T_));
         jobs[2].M = d.dh; jobs[2].N = d.d;
-        set_tr_term(jobs[2].t, h(2), d.dh, hbs(), kc, d.k_ld, d.k_bs);
+        set_tr_term(jobs[2].t, h(2), d.dh, hbs(T_), kc, d.k_ld, d.k_bs);
         // the update before: its weights enter these as they are, unless Newton-Schulz output replaces them or an accumulator carries on
         gw = GradSum{(d.prenorm || (P.muon && d.muon_replaces_weight)) ? nullptr : gwhat, 0};
         contribute(kBf16 ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, &rows_job);
@@ -1519,8 +1520,8 @@ struct Runner {
           longest = std::max(longest, r.len[i]);
         }
         LACT_LAUNCH("k_lr_reduce", "k_lr_reduce", 0.0, k_lr_reduce, dim3(ceil_div(longest, 256), d.b, 3 * n), dim3(256), s,
-                    scr<float>(P.t_lrpart) + (size_t)u0 * lrslot, (long long)lrslot, (long long)P.lr_slots * d.b * P.Tcap, (long long)d.b * P.Tcap,
-                    lr_parts(), P.Tcap, dlr0, dlr1, dlr2, (long long)d.kv_len, r, 0);
+                    scr<float>(P.t_lrpart) + (size_t)u0 * lrslot, (long long)lrslot, (long long)P.lr_slots * d.b * P.Tupd, (long long)d.b * P.Tupd,
+                    lr_parts(), P.Tupd, dlr0, dlr1, dlr2, (long long)d.kv_len, r, 0);
       }
     }
     if (!mg_updates.empty()) {

@@ -91,10 +91,12 @@ struct Plan {
   std::vector<lact_step_t> steps;
   std::vector<lact_step_t> live;    // the steps that are executed: `steps` without the apply rows a later step overwrites
   std::vector<ApplyGroup> groups;   // the apply steps among them whose version is not the newest
-  int group_max = 1;                // largest group
+  std::vector<int> gw_slot;         // by version: place of the gradient that its grouped steps leave for the update chain; -1: it has none
+  int gw_slots = 0;
+  int Tnew = 0;                     // longest apply step on the newest version
   std::vector<float> coeffs;
   MatGeom g;
-  int nupd = 0, Tcap = 0, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 1024, kl_begin = 0, kl_end = 0, side_slots = 1;
+  int nupd = 0, Tcap = 0, Tupd = 1, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 1024, kl_begin = 0, kl_end = 0, side_slots = 1;
   bool muon = false, bf16 = true, momentum = false, state_in = false;
   size_t mat3 = 0;  // 3*b*elems
   // saved
@@ -140,12 +142,14 @@ struct Plan {
     nsz = d.ns_mode == LACT_NS_FP32 ? 4 : 2;
     nupd = 0;
     Tcap = 0;
+    Tupd = 1;
     for (const auto& s : steps) {
       if (s.kind != LACT_UPDATE && s.kind != LACT_APPLY) return fail("step kind must be LACT_UPDATE or LACT_APPLY");
       if (s.start < 0 || s.end <= s.start) return fail("empty or negative step range");
       if (s.kind == LACT_UPDATE) {
         if (s.end > d.kv_len) return fail("update range exceeds kv_len");
         ++nupd;
+        Tupd = std::max(Tupd, s.end - s.start);
       } else {
         if (s.end > d.q_len) return fail("apply range exceeds q_len");
         if (s.out_start < 0 || s.out_start + (s.end - s.start) > d.out_len) return fail("apply output range exceeds out_len");
@@ -213,7 +217,12 @@ struct Plan {
     mdot_parts = std::max(std::max(nblk, 256), ceil_div(g.maxrows(), 4));
     build_groups();
     side_slots = 1;
-    for (const ApplyGroup& g : groups) side_slots = std::max(side_slots, g.n * reduce_split(g.st.end - g.st.start, g.n, MAX_SPLITS, split_min).n);
+    size_t side_rows = 0;     // rows of the largest group
+    for (const ApplyGroup& g : groups) {
+      const int T = g.st.end - g.st.start;
+      side_slots = std::max(side_slots, g.n * reduce_split(T, g.n, MAX_SPLITS, split_min).n);
+      side_rows = std::max(side_rows, (size_t)g.n * T);
+    }
 
     Bump sv;
     s_n0 = sv.take((size_t)3 * d.b * g.maxrows() * 4);
@@ -244,29 +253,34 @@ struct Plan {
         }
     saved_bytes = sv.off + 256;
 
+    // What only a backward pass uses is left out of a forward-only call.
     Bump sc;
-    for (int i = 0; i < 6; ++i) t_h[i] = sc.take((size_t)d.b * Tcap * d.dh * esz);
+    const bool bwd = !d.forward_only;
+    auto take_bwd = [&](size_t bytes) { return sc.take(bwd ? bytes : 0); };
+    // Token-major arrays of the hidden size, the batch entries of a step one after the other: each as long as the steps that use it.
+    const size_t row = (size_t)d.b * d.dh * esz;
+    for (int i = 0; i < 3; ++i) t_h[i] = sc.take((i == 0 ? std::max(Tupd, Tnew) : Tupd) * row);
+    for (int i = 3; i < 6; ++i) t_h[i] = take_bwd(Tupd * row);
+    for (int i = 0; i < 3; ++i) t_hs[i] = i == 0 ? sc.take(side_rows * row) : take_bwd(side_rows * row);   // the grouped apply steps', which run beside the update chain
+    for (int i = 0; i < 3; ++i) t_hn[i] = take_bwd(Tnew * row);       // those of the newest version
     t_partial = sc.take((size_t)nsplit_max * mat3 * 4);
-    t_lrpart = sc.take((size_t)std::max(1, nupd) * 3 * lr_slots * d.b * Tcap * 4);   // one slot per update: reduced by one launch at the end
+    t_lrpart = take_bwd((size_t)std::max(1, nupd) * 3 * lr_slots * d.b * Tupd * 4);   // one slot per update: reduced by one launch at the end
     for (int i = 0; i < 2; ++i) t_xf[i] = sc.take(mat3 * 4);
     t_xbtmp = sc.take(mat3 * nsz);
     t_ss = sc.take((size_t)3 * d.b * std::max(nblk, tr_tiles(d.d, d.dh)) * 4);   // per block of a pass over the matrix, or per tile of the reduction that folds the pass in
-    t_dot = sc.take((size_t)3 * d.b * std::max(nblk, 32) * 4);   // partial dots: per chunk of a matrix, or per block of the fused kernel
-    t_mdot = sc.take((size_t)std::max(1, nupd) * 3 * d.b * mdot_parts * 4);   // one slot per update: the momentum gradients are written at the end
-    for (int i = 0; i < 2; ++i) t_gwhat[i] = sc.take(mat3 * 4);
-    t_gwcur = sc.take(mat3 * 4);
-    t_gmcarry = sc.take(mat3 * 4);
-    t_gc = sc.take(mat3 * esz);
-    for (int i = 0; i < 2; ++i) t_gxf[i] = sc.take(mat3 * 4);
-    for (int i = 0; i < 2; ++i) t_gxb[i] = sc.take(mat3 * nsz);
-    t_sg = sc.take(sq3 * nsz);
-    t_gas = sc.take(sq3 * nsz);
-    t_gn0 = sc.take((size_t)3 * d.b * g.maxrows() * 4);
-    // the apply steps' own buffers (they run beside the update chain)
-    for (int i = 0; i < 3; ++i) t_hs[i] = sc.take((size_t)group_max * d.b * Tcap * d.dh * esz);
-    for (int i = 0; i < 3; ++i) t_hn[i] = sc.take((size_t)d.b * Tcap * d.dh * esz);   // those of the newest version
-    t_partial_side = sc.take((size_t)side_slots * mat3 * 4);
-    t_gwside = sc.take((size_t)std::max(1, groups.empty() ? 0 : nupd) * mat3 * 4);   // by weight version
+    t_dot = take_bwd((size_t)3 * d.b * std::max(nblk, 32) * 4);   // partial dots: per chunk of a matrix, or per block of the fused kernel
+    t_mdot = take_bwd((size_t)std::max(1, nupd) * 3 * d.b * mdot_parts * 4);   // one slot per update: the momentum gradients are written at the end
+    for (int i = 0; i < 2; ++i) t_gwhat[i] = take_bwd(mat3 * 4);
+    t_gwcur = take_bwd(mat3 * 4);
+    t_gmcarry = take_bwd(mat3 * 4);
+    t_gc = take_bwd(mat3 * esz);
+    for (int i = 0; i < 2; ++i) t_gxf[i] = take_bwd(mat3 * 4);
+    for (int i = 0; i < 2; ++i) t_gxb[i] = take_bwd(mat3 * nsz);
+    t_sg = take_bwd(sq3 * nsz);
+    t_gas = take_bwd(sq3 * nsz);
+    t_gn0 = take_bwd((size_t)3 * d.b * g.maxrows() * 4);
+    t_partial_side = take_bwd((size_t)side_slots * mat3 * 4);
+    t_gwside = take_bwd((size_t)std::max(1, gw_slots) * mat3 * 4);   // by gw_slot
     t_nssync = sc.take(((size_t)3 * d.b * 32 + 32) * 4);   // per-matrix barrier lines of the fused Newton-Schulz kernel + error word
     // k * lr0, k * lr2 of the tokens [kl_begin, kl_end) that updates read
     kl_begin = d.kv_len; kl_end = 0;
@@ -293,12 +307,15 @@ struct Plan {
   // Newton-Schulz: 839 us, 853 with twice the size).
   void build_groups() {
     groups.clear();
-    group_max = 1;
+    gw_slot.assign(nupd + 1, -1);
+    gw_slots = 0;
+    Tnew = 0;
     int ver = 0;
     for (const auto& st : live) {
       if (st.kind == LACT_UPDATE) { ++ver; continue; }
-      if (ver == nupd) continue;
       const int T = st.end - st.start;
+      if (ver == nupd) { Tnew = std::max(Tnew, T); continue; }
+      if (gw_slot[ver] < 0) gw_slot[ver] = gw_slots++;
       const long long tiles1 = (long long)ceil_div(T, 128) * ceil_div(d.dh, 128) * d.b;
       const int limit = (int)std::max(1LL, std::min(std::min(65535LL / (3 * d.b), 64LL), (256 + tiles1 - 1) / tiles1));
       if (!groups.empty()) {
@@ -307,7 +324,7 @@ struct Plan {
         // rows of q that two steps share would be two additions to one gradient row
         if (g.n < limit && ver == g.ver + g.n && T == g.st.end - g.st.start && (ds >= T || ds <= -T) && (g.n == 1 || (ds == g.dstart && dout == g.dout))) {
           g.dstart = ds; g.dout = dout;
-          group_max = std::max(group_max, ++g.n);
+          ++g.n;
           continue;
         }
       }

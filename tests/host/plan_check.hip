@@ -42,6 +42,15 @@ static int check(bool bf16, int b, int d, int dh, int rounds, int T_update, int 
       expect(used <= P.nsplit_max, "slots of a launch of the main chain", used, P.nsplit_max);
     }
   expect(P.t_partial_side + (size_t)P.side_slots * P.mat3 * 4 <= P.t_gwside, "end of the side buffer", P.side_slots, 0);
+  for (const auto& g : P.groups) {
+    const size_t rows = (size_t)g.n * b * (g.st.end - g.st.start) * dh * P.esz;
+    expect(P.t_hs[0] + rows <= P.t_hs[1] && P.t_hs[1] + rows <= P.t_hs[2] && P.t_hs[2] + rows <= P.t_hn[0], "rows of a grouped launch", g.n, T_apply);
+    for (int i = 0; i < g.n; ++i) expect(P.gw_slot[g.ver + i] == P.gw_slot[g.ver] + i && P.gw_slot[g.ver + i] < P.gw_slots, "gradients of a group", g.ver + i, P.gw_slots);
+  }
+  const size_t newest = (size_t)b * T_apply * dh * P.esz, update = (size_t)b * T_update * dh * P.esz;
+  expect(P.t_h[0] + std::max(newest, update) <= P.t_h[1], "rows of the main chain", T_update, T_apply);
+  for (int i = 1; i < 6; ++i) expect(P.t_h[i] + update <= (i < 5 ? P.t_h[i + 1] : P.t_hs[0]), "rows of an update", i, T_update);
+  for (int i = 0; i < 3; ++i) expect(P.t_hn[i] + newest <= (i < 2 ? P.t_hn[i + 1] : P.t_partial), "rows of the newest version", i, T_apply);
   if (muon) expect(P.t_ss + (size_t)3 * b * std::max(P.nblk, tr_tiles(d, dh)) * 4 <= P.t_dot, "sums of squares per matrix", std::max(P.nblk, tr_tiles(d, dh)), P.nblk);
   return bad;
 }

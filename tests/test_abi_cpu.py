@@ -171,3 +171,14 @@ def test_incomplete_momentum_states_are_refused(missing):
         cpu_call(momentum=torch.rand(1, 8, 1), momentum_state=tuple(state))
     with pytest.raises(RuntimeError, match="HIP device"):      # nothing reads it without a momentum
         cpu_call(momentum_state=tuple(state))
+
+
+def test_scratch_grows_with_what_the_steps_hold():
+    """Many short steps beside one long one: the buffers of the steps that share a launch are as long as those, not as the longest."""
+    def steps(rounds):
+        short = [st for i in range(rounds) for st in ((LACT_UPDATE, 64 * i, 64 * (i + 1), 0), (LACT_APPLY, 64 * i, 64 * (i + 1), 64 * i))]
+        return short + [(LACT_APPLY, 0, 100000, 64 * rounds)]
+    need = lambda rounds, **kw: sizes(make_desc(steps(rounds), b=6, d=128, dh=256, L=110000, **kw))[2]
+    per_update = 6 * 3 * 128 * 256 * 4
+    assert need(64) < need(2) + 62 * 2 * per_update      # a gradient per version, and row sums and dot products per update
+    assert need(64, forward_only=1) < need(64) // 3

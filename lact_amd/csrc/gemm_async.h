@@ -165,9 +165,12 @@ struct AsyncPipe {
       for (int m = 0; m < TS::TM; ++m) fa[m].template fetch<TS::BM, A_KS>(st, wm0 + m * 32, g);
 #pragma unroll
       for (int n = 0; n < TS::TN; ++n) fb[n].template fetch<TS::BN, B_KS>(st + A_BYTES, wn0 + n * 32, g);
-      if (left < GROUP)
+      if (left < GROUP) {   // both operands: an infinity that one of them repeats there would make the other's zeros NaN
 #pragma unroll
         for (int m = 0; m < TS::TM; ++m) fa[m].mask(left);
+#pragma unroll
+        for (int n = 0; n < TS::TN; ++n) fb[n].mask(left);
+      }
 #pragma unroll
       for (int m = 0; m < TS::TM; ++m)
 #pragma unroll

@@ -140,9 +140,9 @@ struct DmaLane {
       dma16<SC1>(b, off, lds_tile + ii * DMA_LOADERS * 1024);
     }
   }
-  // The k rows past the end of K in the K-strided tile that has landed at `tile` (LDS; ktail valid k rows): cleared,
-  // so that whatever the other operand holds there adds nothing.  Every wave clears inside the chunks it copied
-  // itself (it has waited for exactly those).
+  // The k rows past the end of K in the K-strided tile that has landed at `tile` (LDS; ktail valid k rows): cleared, in both
+  // operands' tiles (an infinity that one of them repeats there would make the other's zeros NaN).  Every wave clears inside
+  // the chunks it copied itself (it has waited for exactly those).
   __device__ static __forceinline__ void clear_tail(char* tile, int lw, int ktail) {
     const int lane = threadIdx.x & 63;
     const int first = ktail * ROWS * 2;   // first byte of the tile that lies past the end of K
@@ -359,7 +359,7 @@ struct DmaPipe {
     };
     do next_phase(); while (cnk == 0 && cp + 1 < NPH);
     for (int i = 0; i < STAGES - 1 && issued < total; ++i) issue_stage();
-    // TAILS: the stage that holds a phase's ragged last K-step gets the k rows past the end of its A tile cleared
+    // TAILS: the stage that holds a phase's ragged last K-step gets the k rows past the end of its tiles cleared
     // once it has landed, before the MFMA waves are let in
     int tail_step[NPH], tail_rows[NPH], acc_steps = 0;
     if constexpr (TAILS) {
@@ -376,7 +376,13 @@ struct DmaPipe {
       if constexpr (TAILS) {
 #pragma unroll
         for (int i = 0; i < NPH; ++i)
-          if (tail_rows[i] > 0 && kt == tail_step[i]) DmaLane<TS::BM>::clear_tail(smem + (kt % STAGES) * SM::STAGE, lw, tail_rows[i]);
+          if (tail_rows[i] > 0 && kt == tail_step[i]) {
+            char* const st = smem + (kt % STAGES) * SM::STAGE;
+            DmaLane<TS::BM>::clear_tail(st, lw, tail_rows[i]);
+#pragma unroll
+            for (int j = 0; j < NBMAX; ++j)
+              if (j < ph[i].nb) DmaLane<TS::BN>::clear_tail(st + SM::A_BYTES + j * SM::B_BYTES, lw, tail_rows[i]);
+          }
       }
       __syncthreads();
       if (issued < total) issue_stage();

@@ -164,3 +164,35 @@ def test_newton_schulz_in_one_block_is_bit_identical(b, d, dh, L, stacked):
                 _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 1)
         for a, r in zip(*res):
             assert torch.equal(a, r)
+
+
+def same_specials(a, r):
+    a, r = a.detach().float().cpu(), r.detach().float()
+    assert torch.isinf(r).any()
+    assert torch.equal(torch.isnan(a), torch.isnan(r)) and torch.equal(torch.isinf(a), torch.isinf(r))
+    assert torch.equal(a[torch.isinf(a)], r[torch.isinf(r)])
+
+
+@pytest.mark.parametrize("dtype,d,T", [(torch.bfloat16, 24, 13), (torch.float32, 40, 13), (torch.bfloat16, 64, 70), (torch.bfloat16, 48, 135)])
+def test_infinities_pass_the_ragged_end_of_a_contraction(dtype, d, T):
+    """An infinite operand at the last place of a contraction that ends inside a K-step, in the features and in the tokens: what the
+    copies bring in past the end must add nothing, not the NaN of zero times infinity."""
+    print("[gpu-test] infinities", dtype, d, T, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    num = O.Numerics(autocast=dtype == torch.bfloat16)
+    inp = O.make_inputs(1, T, d, 40, seed=41, act_dtype=dtype)
+    inp["q"][..., -1] = 1
+    args = [inp[n] for n in ORDER[:9]]
+    hot = [t.clone() for t in args]
+    hot[0][0, 3, -1] = float("inf")      # the last feature of one row of w0
+    out, _, _ = ops.run_program(ops.Program(steps=((LACT_APPLY, 0, T, 0),), out_len=T), *[t.to("cuda") for t in hot])
+    same_specials(out, O.run_program(*hot, [O.Step(O.APPLY, 0, T)], num=num)[0])
+    hot = [t.clone() for t in args]
+    for lr in hot[6:]:
+        lr[:, -1] = float("inf")         # the last token of all three gradients, which the momentum states hold
+    prog = ops.Program(steps=((LACT_UPDATE, 0, T, 0), (LACT_APPLY, 0, T, 0)), out_len=T)
+    _, _, ms = ops.run_program(prog, *[t.to("cuda") for t in hot], inp["momentum"].to("cuda"))
+    _, _, refs = O.run_program(*hot, [O.Step(O.UPDATE, 0, T), O.Step(O.APPLY, 0, T)], num=num, momentum=inp["momentum"])
+    for a, r in zip(ms, refs):
+        same_specials(a, r)

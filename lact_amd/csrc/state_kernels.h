@@ -428,13 +428,14 @@ __global__ void k_update_renorm(const RenormParams p) {
   }
   ss = wave_sum(ss);
   float den = p.eps_in_sqrt ? sqrtf(ss + 1e-5f) : sqrtf(ss) + 1e-5f;
-  if (p.poison && *p.poison) den = __uint_as_float(0x7fc00000u);
+  const float bad = p.poison && *p.poison ? __uint_as_float(0x7fc00000u) : 0.f;
+  den += bad;
   const float n0 = p.weight_norm ? p.n0[(size_t)z * p.g.maxrows() + row] : 1.f;
   auto emit = [&](int c, const float4& v) {
     if (p.main_out) st4(p.main_out + o + c, v);
     // same operation order as the reference: (w / (norm + eps)) * w_norm
     const float4 y = p.weight_norm ? f4((v.x / den) * n0, (v.y / den) * n0, (v.z / den) * n0, (v.w / den) * n0)
-                                   : f4(v.x + 0.f * den, v.y + 0.f * den, v.z + 0.f * den, v.w + 0.f * den);
+                                   : f4(v.x + bad, v.y + bad, v.z + bad, v.w + bad);
     if (p.wf_out) st4(p.wf_out + o + c, y);
     if (ext) st4(ext + c, y);
     if (p.wc_out) Elem<T>::store4(reinterpret_cast<T*>(p.wc_out) + o + c, y.x, y.y, y.z, y.w);

@@ -196,3 +196,9 @@ def test_infinities_pass_the_ragged_end_of_a_contraction(dtype, d, T):
     _, _, refs = O.run_program(*hot, [O.Step(O.UPDATE, 0, T), O.Step(O.APPLY, 0, T)], num=num, momentum=inp["momentum"])
     for a, r in zip(ms, refs):
         same_specials(a, r)
+    # without the row norm the weights hold them too
+    prog = ops.Program(steps=((LACT_UPDATE, 0, T, 0), (LACT_APPLY, 0, T, 0)), out_len=T, weight_norm=False)
+    _, ws, _ = ops.run_program(prog, *[t.to("cuda") for t in hot])
+    _, refs, _ = O.run_program(*hot, [O.Step(O.UPDATE, 0, T), O.Step(O.APPLY, 0, T)], num=num, weight_norm=False)
+    for a, r in zip(ws, refs):
+        same_specials(a, r)

@@ -131,6 +131,15 @@ __device__ __forceinline__ bf16x8 attn_pack(const f32x16& s, int st) {
   return __builtin_bit_cast(bf16x8, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
+// What the lanes of a wave wrote to LDS is read by others of them behind this, and what they read is overwritten behind it.  The
+// wave's LDS accesses run in order, so this is no instruction; it keeps the compiler from moving one across (a wave barrier alone
+// orders no memory for it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // A wave's [D][32] accumulator (rows = D, columns = its own rows), times `f`, to 32 rows of a contiguous [B, L, H, D]
 // tensor, through 32 x (D + 8) halves of LDS of its own.
 template <int D>
@@ -144,7 +153,7 @@ __device__ __forceinline__ void attn_store_rows(char* lds, const f32x16 (&acc)[D
     for (int g = 0; g < 4; ++g)
       Elem<uint16_t>::store4(t + (l & 31) * LD + dt * 32 + 8 * g + 4 * (l >> 5), acc[dt][4 * g] * f, acc[dt][4 * g + 1] * f, acc[dt][4 * g + 2] * f,
                              acc[dt][4 * g + 3] * f);
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
   constexpr int LPR = D / 8, RPP = 64 / LPR;
 #pragma unroll
   for (int i = 0; i < 32 / RPP; ++i) {
@@ -152,7 +161,7 @@ __device__ __forceinline__ void attn_store_rows(char* lds, const f32x16 (&acc)[D
     const uint4 u = *reinterpret_cast<const uint4*>(t + r * LD + c);
     if (row0 + r < L) *reinterpret_cast<uint4*>(out + (size_t)(row0 + r) * ld + c) = u;
   }
-  __builtin_amdgcn_wave_barrier();
+  wave_lds_fence();
 }
 
 constexpr float ATTN_LOG2E = 1.4426950408889634f;

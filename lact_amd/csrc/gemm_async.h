@@ -168,8 +168,11 @@ struct AsyncPipe {
       if (left < GROUP) {   // both operands: an infinity that one of them repeats there would make the other's zeros NaN
 #pragma unroll
         for (int m = 0; m < TS::TM; ++m) fa[m].mask(left);
+        // feature sizes come in eights: groups of eight end ragged in contractions over tokens only (masking everywhere costs the
+        // fp32 training step of eight heads of 128, 2048 tokens, 2.5 of 478 us)
+        if constexpr ((A_KS && B_KS) || GROUP > 8)
 #pragma unroll
-        for (int n = 0; n < TS::TN; ++n) fb[n].mask(left);
+          for (int n = 0; n < TS::TN; ++n) fb[n].mask(left);
       }
 #pragma unroll
       for (int m = 0; m < TS::TM; ++m)

@@ -82,7 +82,11 @@ const char* lact_last_error(void);
 int lact_version(void);
 
 /* Bytes of the two caller-owned buffers: `saved` lives from forward to backward (fast-weight
- * versions, momentum states, Newton-Schulz iterates); `scratch` only during one call. */
+ * versions, momentum states, Newton-Schulz iterates); `scratch` only during one call.  scratch grows with the program:
+ * k times two rates for the tokens that updates read (twice k's bytes over that range); per update, row sums and, where a
+ * later apply step uses the version, an fp32 gradient of it (at most half of what `saved` holds per version); buffers as
+ * long as the longest update, the longest apply step on the newest version and the largest group of apply steps that one
+ * launch covers (a group ends once it fills the chip).  forward_only leaves out what only a backward uses. */
 int lact_query_sizes(const lact_desc_t* desc, size_t* saved_bytes, size_t* scratch_bytes);
 
 /* Whole forward of one program.  Replaces block_causal_lact_swiglu / prenorm_block_causal_lact_swiglu
@@ -210,10 +214,10 @@ int lact_window_attention_backward(int32_t B, int32_t L, int32_t H, int32_t D, i
 /* Execution options (process-wide; no counterpart in the reference, where PyTorch enqueues the whole layer on one
  * stream as separate kernels).  The switches are on by default and change no result bit.
  *   LACT_OPT_STREAM_OVERLAP: the apply steps of a program do not depend on the update chain that runs beside
- *     them, and nothing in a call waits for dk, dv or the learning-rate gradients of an update; lact_forward /
- *     lact_backward enqueue them on two library-owned streams (default priority, per device, created on first
- *     use) that are forked from and joined back into the caller's stream with events, so the call as a whole
- *     stays asynchronous and ordered on the caller's stream.
+ *     them, and k times the learning rates depends on the inputs only; where a program has apply steps on a
+ *     version that is not its newest, lact_forward / lact_backward enqueue them on two library-owned streams
+ *     (default priority, per device, created on first use) that are forked from and joined back into the caller's
+ *     stream with events, so the call as a whole stays asynchronous and ordered on the caller's stream.
  *   LACT_OPT_FUSED_NEWTON_SCHULZ: all Newton-Schulz iterations of an update (and of its backward) run as one
  *     kernel whose blocks meet at per-matrix barriers (bf16; rows and columns multiples of 192, of 128, or rows of
  *     128 and columns of 64; at most 8 iterations); otherwise three GEMM launches per iteration.

@@ -10,9 +10,9 @@
 // instructions per eight k; instruction i takes k = i from the lanes of the lower half and k = 4 + i from those of the upper
 // half, on both operands, so that a K-contiguous operand costs one ds_read_b128 per four instructions.
 //
-// What bounds it at the sizes that come here (fp32 heads of 64 to 256 and chunks of some hundred tokens; bf16 heads of 96 or
-// 40): the number of blocks and the latency of a block's first copies, less the matrix rate.  Hence small tiles and
-// everything of the first K-steps in flight at once.
+// What bounds it at the sizes that come here (fp32 heads of 64 to 256 and chunks of some hundred tokens; bf16 heads that are
+// no multiple of 16, as 40 or 72): the number of blocks and the latency of a block's first copies, less the matrix rate.  Hence
+// small tiles and everything of the first K-steps in flight at once.
 #pragma once
 #include "gemm_dma.h"
 
@@ -20,7 +20,7 @@ namespace lact {
 
 // 64 x 64 tiles: measured at eight fp32 heads of 128, 512 tokens, against the register-staged loop on 128 x 128 tiles: apply
 // hidden stage 35 -> 11 us, update 48 -> 17, update backward 53 -> 32, four-term row GEMM 72 -> 19, token reduction 55 + 5 (its
-// partial sums) -> 17.  bf16, 24 heads of 96, 2500 tokens: 231 -> 217 us over the eight kernels of a step (128 x 64 tiles: 254).
+// partial sums) -> 17.
 template <typename T> struct AsyncTile {
   using TS = TileShape<64, 64, 2, 2>;
   static constexpr int STAGES = sizeof(T) == 4 ? 4 : 3;

@@ -118,7 +118,7 @@ template <> const char* tname<float>() { return "f32"; }
 // pool per device, created on first use and kept until the process ends.
 struct SideCtx {
   hipStream_t stream = nullptr;
-  hipStream_t tail = nullptr;        // second side stream: results of the update chain that nothing in the call waits for
+  hipStream_t tail = nullptr;        // second side stream: what depends on the inputs of a forward only (k * lr0, k * lr2)
   std::vector<hipEvent_t> ev;
   size_t next = 0;
   // Fused Newton-Schulz kernels of this process must not overlap each other (each needs its groups resident as a whole).
@@ -311,7 +311,7 @@ struct Runner {
   char* sc;   // scratch
   const lact_desc_t& d;
   hipStream_t s_main, s_side;   // caller's stream; stream of the apply steps (= s_main when overlap is off)
-  hipStream_t s_tail;           // stream of dk, dv and the learning-rate gradients (= s_main when overlap is off)
+  hipStream_t s_tail;           // stream of k * lr0 and k * lr2 at the start of a forward (= s_main when overlap is off)
   SideCtx* side = nullptr;
   const size_t* hsel;           // token-major intermediates of the chain being enqueued
   size_t partial_sel;

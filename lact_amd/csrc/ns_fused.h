@@ -430,9 +430,9 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p)
     const size_t zo = (size_t)z * p.r * p.c + (size_t)rx * TS::BM * p.c + ry * TS::BN;
     float4 ga[NG], gb[NG];
     uint4 gi[NG];
-    // No fence: this tile of gx was written by this very block in the last stage (and in every second stage before),
-    // and the waves of a compute unit share its vector L1, which their own stores keep current.  The same holds for
-    // every auxiliary tile the blending epilogues read (always the block's own tile of a buffer it wrote itself).
+    // No fence: this tile of gx was written by this very block, in the last stage only (before, the iterate stays in the copy
+    // waves' registers), and the waves of a compute unit share its vector L1, which their own stores keep current.  The same
+    // holds for the auxiliary bf16 tile that a blending epilogue reads (the block's own tile of a buffer it wrote itself).
     float dot = ns_tile_dot<TS>(gx, p.g16, zo, p.c, ga, gb, gi);
     dot = block_sum(dot, reinterpret_cast<float*>(smem));
     if (threadIdx.x == 0) p.dot_part[(size_t)z * nbm + member] = dot;

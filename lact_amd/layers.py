@@ -9,8 +9,9 @@ The projections are torch.nn.Linear (hipBLASLt).  Everything between them runs i
 the to_qkv output into the operation's q, k, v (silu, per-head L2 norm, head layout), one makes the learning rates
 and the momentum, the operation itself, and one kernel turns its output into the o_proj input (per-head RMSNorm,
 per-head gate, head layout) -- each with a hand-written backward.  The sliding-window attention of the causal
-layer (flash_attn_func in the reference) is torch's scaled_dot_product_attention over blocks of the window size,
-which bounds the mask to [window, 2*window] per block.
+layer (flash_attn_func in the reference) is a pair of kernels for bf16 heads of 64 and 128, whose inputs the first
+kernel writes and whose output the last one adds; other types and head sizes go through torch's
+scaled_dot_product_attention over blocks of the window size, which bounds the mask to [window, 2*window] per block.
 """
 from __future__ import annotations
 

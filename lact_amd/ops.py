@@ -58,6 +58,9 @@ class Program:
             object.__setattr__(self, "_native", h)
         return h
 
+    def __getstate__(self):      # copies and pickles make their own
+        return {k: v for k, v in self.__dict__.items() if k != "_native"}
+
     @property
     def n_updates(self) -> int:
         return sum(1 for s in self.steps if s[0] == LACT_UPDATE)

@@ -182,3 +182,12 @@ def test_scratch_grows_with_what_the_steps_hold():
     per_update = 6 * 3 * 128 * 256 * 4
     assert need(64) < need(2) + 62 * 2 * per_update      # a gradient per version, and row sums and dot products per update
     assert need(64, forward_only=1) < need(64) // 3
+
+
+def test_programs_are_copied_and_pickled_after_use():
+    import copy
+    import pickle
+    prog = ops.Program(steps=((LACT_UPDATE, 0, 8, 0), (LACT_APPLY, 0, 8, 0)), out_len=8, ns_coeffs=ops.NS5_COEFFS)
+    prog.native()
+    for other in (copy.deepcopy(prog), copy.copy(prog), pickle.loads(pickle.dumps(prog))):
+        assert other == prog and hash(other) == hash(prog) and other.native() is not None

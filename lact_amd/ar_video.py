@@ -33,13 +33,13 @@ def _ar_steps(seq_len, q_len, mini_batch_size, update_length, update_every, num_
     return tuple(steps)
 
 
-@lru_cache(maxsize=256)
+@lru_cache(maxsize=256, typed=True)
 def _interleaved_program(kv_len, q_len, mini_batch_size, update_length, update_every, num_repeat, iters, weight_norm, ns_mode):
     return Program(steps=_ar_steps(kv_len, q_len, mini_batch_size, update_length, update_every, num_repeat), out_len=q_len,
                    ns_coeffs=None if iters is None else (NS_CLASSIC,) * iters, weight_norm=weight_norm, ns_mode=ns_mode)
 
 
-@lru_cache(maxsize=256)
+@lru_cache(maxsize=256, typed=True)
 def _inference_program(mini_batch, updates, q_len, iters, weight_norm, ns_mode):
     return Program(steps=((LACT_UPDATE, 0, mini_batch, 0),) * updates + ((LACT_APPLY, 0, q_len, 0),), out_len=q_len,
                    ns_coeffs=None if iters is None else (NS_CLASSIC,) * iters, weight_norm=weight_norm, ns_mode=ns_mode)

@@ -3,6 +3,7 @@ from __future__ import annotations
 
 import collections
 from functools import lru_cache
+from operator import index
 
 import torch
 
@@ -35,7 +36,7 @@ def fast_weight_swish_glu_weight_norm_mini_batch_apply(w0, w1, w2, q, k, v, lr0,
     """lact_ttt.py:71-147.  w0, w2: [b, d, dh]; w1: [b, dh, d]; returns (output, w0, w1, w2).
     Outputs of the apply operators are concatenated in program order (:142-145); the initial row norms
     are detached (:96-98); Newton-Schulz always runs, with `muon_update_steps` iterations (:120-128)."""
-    prog = _program(tuple((int(s), int(e), bool(u), bool(a)) for s, e, u, a in ttt_ua_order), int(muon_update_steps), ops._ns_mode(q))
+    prog = _program(tuple((index(s), index(e), bool(u), bool(a)) for s, e, u, a in ttt_ua_order), index(muon_update_steps), ops._ns_mode(q))
     out, (a0, a1, a2), _ = run_program(prog, w0.transpose(1, 2), w1.transpose(1, 2), w2.transpose(1, 2),
                                        q, k, v, lr0, lr1, lr2, None)
     return out, a0.transpose(1, 2), a1.transpose(1, 2), a2.transpose(1, 2)

@@ -191,3 +191,22 @@ def test_programs_are_copied_and_pickled_after_use():
     prog.native()
     for other in (copy.deepcopy(prog), copy.copy(prog), pickle.loads(pickle.dumps(prog))):
         assert other == prog and hash(other) == hash(prog) and other.native() is not None
+
+
+def test_fractional_sizes_are_refused():
+    """Also after a call with the whole number, whose schedule is kept."""
+    import torch
+    from lact_amd import ar_video, nvs, ttt_operation
+    t = {n: torch.randn(1, 8, 8) for n in ("w0", "w1", "w2", "q", "k", "v")} | {n: torch.rand(1, 8, 1) for n in ("lr0", "lr1", "lr2")}
+    args = list(t.values())
+    calls = (lambda x: ttt_operation.block_causal_lact_swiglu(*args, chunk_size=x),
+             lambda x: nvs.fast_weight_swish_glu_weight_norm_mini_batch_apply(*args, [(0, x, True, False), (0, 4, False, True)]),
+             lambda x: nvs.fast_weight_swish_glu_weight_norm_mini_batch_apply(*args, [(0, 4, True, True)], muon_update_steps=x),
+             lambda x: ar_video.ar_fast_weight_swish_glu_weight_norm_mini_batch(*args, 1.0, mini_batch_size=x),
+             lambda x: ar_video.ar_fast_weight_swish_glu_weight_norm_mini_batch_inference(*args, 1.0, num_repeat=x, do_update=True))
+    for call in calls:
+        with pytest.raises(RuntimeError, match="HIP device"):
+            call(4)
+        for x in (4.0, 4.5):
+            with pytest.raises(TypeError):
+                call(x)

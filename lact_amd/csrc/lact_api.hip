@@ -2198,6 +2198,7 @@ int lact_backward(const lact_desc_t* desc, const void* q, const void* k, const v
   if (P.nupd > 0 && P.momentum && (!momentum || !dmomentum)) return fail("use_momentum set but momentum or dmomentum is null");
   const int al = P.bf16 ? 8 : 4;
   if (P.d.do_ld % al || P.d.do_bs % al || P.d.do_ld < P.d.d) return fail("dout strides must keep 16-byte alignment");
+  if (P.d.do_ld > MAX_ROW_STRIDE) return fail("row stride too large");
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   std::lock_guard<std::mutex> lock(g_enqueue_mutex);
 #define LACT_BWD(T_, TN_)                                                                                            \

@@ -84,6 +84,9 @@ struct ApplyGroup {
   int dstart, dout;                // from one step's rows of q, of the output, to the next one's
 };
 
+// Largest distance of two rows, in elements: the kernels form a tile's byte offsets from 24-bit products.
+constexpr int MAX_ROW_STRIDE = (1 << 23) - 1;
+
 struct Plan {
   lact_desc_t d;
   std::vector<NsBatch> nsb;
@@ -126,6 +129,8 @@ struct Plan {
         d.o_bs % al)
       return fail("row and batch strides must keep 16-byte alignment");
     if (d.q_ld < d.d || d.k_ld < d.d || d.v_ld < d.d || d.o_ld < d.d) return fail("row stride smaller than d");
+    if (std::max(std::max(d.q_ld, d.k_ld), std::max(d.v_ld, d.o_ld)) > MAX_ROW_STRIDE || d.d > MAX_ROW_STRIDE || d.dh > MAX_ROW_STRIDE)
+      return fail("row stride too large");
     if (3LL * d.b > 65535) return fail("b too large (3*b must fit a grid dimension)");
     if (d.n_steps <= 0 || !d.steps) return fail("empty program");
     steps.assign(d.steps, d.steps + d.n_steps);

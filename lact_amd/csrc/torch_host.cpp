@@ -72,7 +72,8 @@ bool aligned16(const Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_dat
 Tensor rows_view(Tensor t, at::ScalarType dtype) {
   if (t.scalar_type() != dtype) t = t.to(dtype);
   const int64_t align = 16 / t.element_size();
-  const bool ok = t.dim() == 3 && t.stride(2) == 1 && t.stride(1) % align == 0 && t.stride(0) % align == 0 && t.stride(1) >= t.size(2) && aligned16(t);
+  const bool ok = t.dim() == 3 && t.stride(2) == 1 && t.stride(1) % align == 0 && t.stride(0) % align == 0 && t.stride(1) >= t.size(2) &&
+                  t.stride(1) < (1 << 23) && aligned16(t);   // (rows further apart are refused by the library)
   return ok ? t : t.clone(at::MemoryFormat::Contiguous);
 }
 

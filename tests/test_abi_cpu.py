@@ -76,6 +76,9 @@ def test_query_sizes_and_validation_messages():
     assert "ns_coeffs" in err(make_desc(ops.block_causal_steps(256, 64), ns_steps=5))
     assert "alignment" in err(make_desc(ops.block_causal_steps(256, 64), q_ld=68))
     assert "act_dtype" in err(make_desc(ops.block_causal_steps(256, 64), act_dtype=3))
+    for name in ("q_ld", "k_ld", "v_ld", "o_ld"):      # offsets inside a tile are 24-bit products
+        assert "too large" in err(make_desc(ops.block_causal_steps(256, 64), **{name: 1 << 23}))
+        assert sizes(make_desc(ops.block_causal_steps(256, 64), **{name: (1 << 23) - 8}))[0] == 0
     # a forward-only descriptor keeps less for the backward, and the backward entry point refuses it (before it
     # looks at any pointer: no GPU is needed for this check)
     # (at d = 256: the update's pre-activations are kept for the backward only above d = 128)

@@ -175,3 +175,15 @@ def test_operands_may_start_anywhere(dtype):
         res.append([out, *ws] + list(torch.autograd.grad([out, *ws], x, [go, *[torch.ones_like(w) for w in ws]])))
     for other in res[1:]:
         assert all(torch.equal(a, b) for a, b in zip(other, res[0]))
+
+
+def test_rows_further_apart_than_the_kernels_reach_are_copied():
+    print("[gpu-test] distant rows", flush=True)
+    args = [t.detach() for t in operands(1, 24, 16, 24)]
+    args[3:6] = [t.bfloat16() for t in args[3:6]]
+    far = torch.zeros(24, 1 << 23, dtype=torch.bfloat16, device=DEV)
+    far[:, :16] = args[3][0]
+    apart = list(args)
+    apart[3] = far[:, :16].unsqueeze(0)
+    with torch.no_grad():
+        assert torch.equal(ops.run_program(PROGRAM, *apart)[0], ops.run_program(PROGRAM, *args)[0])

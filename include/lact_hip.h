@@ -185,7 +185,7 @@ int lact_layer_lr_backward(int32_t B, int32_t L, int32_t H, int32_t rates_major,
  *      norm_weight [hd] fp32 (nullable = ones) when use_norm, times silu(gate_raw [B, L, H]) when gate_raw is
  *      given, head layout, and in the _add form plus add
  *      [B, L, H*hd] (nullable; its gradient is dy) (bidirectional_lact_layer.py:268-270; causal_lact_with_sliding_window_attn.py:351-357).
- *      The backward writes lact_layer_post_dw_rows(B, L, H) partial rows of the weight gradient into
+ *      The backward writes lact_layer_post_dw_rows(B, L, H) partial rows (one per block) of the weight gradient into
  *      dw_part [rows][hd] fp32 (the caller sums them), d_o and dgate_raw. */
 int lact_layer_post_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm,
                             float eps, const void* o, const float* norm_weight, const void* gate_raw, void* y,
@@ -197,6 +197,32 @@ int32_t lact_layer_post_dw_rows(int32_t B, int32_t L, int32_t H);
 int lact_layer_post_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm,
                              float eps, const void* o, const float* norm_weight, const void* gate_raw,
                              const void* dy, void* d_o, void* dgate_raw, float* dw_part, void* stream);
+
+/* out[dim] = sum of the rows of part [rows][dim], fp32, in a fixed order (the partial rows of lact_layer_post_backward). */
+int lact_layer_sum_rows(int32_t rows, int32_t dim, const float* part, float* out, void* stream);
+
+/* Weight gradient of a linear map: dw[M, N] (fp32, contiguous) = dy[T, M]^T x[T, N], bf16 operands with row strides *_ld
+ *      (elements, multiples of 8), M and N multiples of 8, T >= 64; fp32 sums throughout.  workspace:
+ *      lact_weight_grad_workspace_bytes bytes (may be 0), 16-byte aligned.  (The layers' to_qkv and output projections; in the
+ *      reference autograd's matmul.) */
+size_t lact_weight_grad_workspace_bytes(int32_t T, int32_t M, int32_t N);
+int lact_weight_grad(int32_t T, int32_t M, int32_t N, const void* dy, int32_t dy_ld, const void* x, int32_t x_ld, float* dw,
+                     void* workspace, void* stream);
+
+/* Small projections of a layer's input x [rows, dim] (fp32, contiguous, dim a multiple of 4) under bf16 autocast.  Forward, one
+ *      pass: xb = bf16 copy of x (input of to_qkv); mom_raw [rows, mom_n] (bf16 values in fp32) and gate_raw [rows, gate_n]
+ *      (bf16) = x w^T + b of x and parameters rounded to bf16, sum in fp32, result rounded once; one of the two may be 0 wide.
+ *      Backward of these and of an fp32 map of lr_n outputs: dx [rows, dim] fp32 = dxq (bf16, the gradient through to_qkv) + all
+ *      three maps' shares; parameter gradients fp32; gradients of the outputs nullable (zero), outputs nullable (not wanted).
+ *      lr_n at most 24, mom_n + gate_n at most 16; weights fp32 [n, dim], biases nullable.
+ *      (bidirectional_lact_layer.py:247-249; causal_lact_with_sliding_window_attn.py:326-348.) */
+int lact_layer_in_forward(int64_t rows, int32_t dim, const float* x, const float* mom_w, const float* mom_b, int32_t mom_n,
+                          const float* gate_w, const float* gate_b, int32_t gate_n, void* xb, float* mom_raw, void* gate_raw, void* stream);
+size_t lact_layer_in_backward_workspace_bytes(int64_t rows, int32_t dim, int32_t lr_n, int32_t mom_n, int32_t gate_n);
+int lact_layer_in_backward(int64_t rows, int32_t dim, const float* x, const float* lr_w, int32_t lr_n, const float* mom_w, int32_t mom_n,
+                           const float* gate_w, int32_t gate_n, const float* dlr_raw, const float* dmom_raw, const void* dgate_raw,
+                           const void* dxq, float* dx, float* dlr_w, float* dlr_b, float* dmom_w, float* dmom_b, float* dgate_w,
+                           float* dgate_b, void* workspace, void* stream);
 
 /* Causal attention inside a sliding window (query i sees keys i - window + 1 .. i; window >= L: plain causal), bf16, head
  * size D = 64 or 128, softmax scale 1/sqrt(D): flash_attn_func(causal=True, window_size=(window-1, 0)) of

@@ -780,30 +780,16 @@ struct TokenReduceDmaParams : TokenReduceParams {
   TileMap map;   // token splits, output tiles, 3 * batch
   UDiv by_tn[3];   // tiles along N of each job
 };
-// One block of the reduction; `lin` is the block's linear index in the reduction's tile map.
+// One output tile of a contraction over tokens, both operands K-strided: staged in LDS in fp32 (StageTile<TS, 4>).
 template <class TS>
-__device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParams& p, int lin, char* smem) {
-  constexpr int STAGES = row_stages<TS>();
-  using Pipe = DmaPipe<TS, 1, 1, STAGES, false, true>;
-  int split, tile, bz;   // map: (splits, tiles, 3*nb)
-  clear_words(p.prep_clear, lin == 0);
-  if (!p.map.locate(lin, split, tile, bz)) return;
-  const int t = p.by_nb.div(bz), ib = bz - t * (int)p.by_nb.d, g = t / 3, j = t - 3 * g;
-  const TokenReduceJob& job = p.job[j];
-  const int tm = p.by_tn[j].div(tile);
-  const int m0 = tm * TS::BM, n0 = (tile - tm * (int)p.by_tn[j].d) * TS::BN;
-  if (m0 >= job.M) return;
-  const int k_begin = split * p.split_len;
-  const int klen = min(p.split_len, p.tokens - k_begin);
+__device__ __forceinline__ void token_reduce_tile(DmaOperand a, DmaOperand b, int klen, char* smem) {
+  using Pipe = DmaPipe<TS, 1, 1, row_stages<TS>(), false, true>;
   DmaPhase<1> ph[1];
-  ph[0].a.base = reinterpret_cast<const uint16_t*>(job.t.A) + ib * job.t.bsA + g * job.t.gsA + (size_t)k_begin * job.t.lda + m0;
-  ph[0].a.ld = job.t.lda; ph[0].a.rows = job.M - m0; ph[0].a.ks = 1;
-  ph[0].b[0].base = reinterpret_cast<const uint16_t*>(job.t.B) + ib * job.t.bsB + g * job.t.gsB + (size_t)k_begin * job.t.ldb + n0;
-  ph[0].b[0].ld = job.t.ldb; ph[0].b[0].rows = job.N - n0; ph[0].b[0].ks = 1;
-  ph[0].nb = 1;
+  a.ks = b.ks = 1;
   // a token count that is not a multiple of 64 ends inside the last K-step of the last split
+  a.ktail = b.ktail = klen % DMA_BK;
+  ph[0].a = a; ph[0].b[0] = b; ph[0].nb = 1;
   ph[0].K = (klen + DMA_BK - 1) / DMA_BK * DMA_BK;
-  ph[0].a.ktail = ph[0].b[0].ktail = klen % DMA_BK;
   f32x16 acc[1][TS::TM][TS::TN];
   Pipe pipe(smem, ph);
   const bool loader = Pipe::is_loader();
@@ -821,6 +807,28 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
     LACT_FOR_QUADS(TS) ST::put4(lb, tm, tn, g, acc[0][tm][tn][4 * g], acc[0][tm][tn][4 * g + 1], acc[0][tm][tn][4 * g + 2], acc[0][tm][tn][4 * g + 3]);
   }
   __syncthreads();
+}
+
+// One block of the reduction; `lin` is the block's linear index in the reduction's tile map.
+template <class TS>
+__device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParams& p, int lin, char* smem) {
+  int split, tile, bz;   // map: (splits, tiles, 3*nb)
+  clear_words(p.prep_clear, lin == 0);
+  if (!p.map.locate(lin, split, tile, bz)) return;
+  const int t = p.by_nb.div(bz), ib = bz - t * (int)p.by_nb.d, g = t / 3, j = t - 3 * g;
+  const TokenReduceJob& job = p.job[j];
+  const int tm = p.by_tn[j].div(tile);
+  const int m0 = tm * TS::BM, n0 = (tile - tm * (int)p.by_tn[j].d) * TS::BN;
+  if (m0 >= job.M) return;
+  const int k_begin = split * p.split_len;
+  const int klen = min(p.split_len, p.tokens - k_begin);
+  DmaOperand a, b;
+  a.base = reinterpret_cast<const uint16_t*>(job.t.A) + ib * job.t.bsA + g * job.t.gsA + (size_t)k_begin * job.t.lda + m0;
+  a.ld = job.t.lda; a.rows = job.M - m0;
+  b.base = reinterpret_cast<const uint16_t*>(job.t.B) + ib * job.t.bsB + g * job.t.gsB + (size_t)k_begin * job.t.ldb + n0;
+  b.ld = job.t.ldb; b.rows = job.N - n0;
+  token_reduce_tile<TS>(a, b, klen, smem);
+  using ST = StageTile<TS, 4>;
   const size_t slot = (size_t)bz * p.mat_elems;
   if (p.prep_d_out) {   // forward update, one split: momentum, bf16 copy and its sum of squares right here
     const int r0 = ST::row0(), c0 = ST::col0();
@@ -908,6 +916,40 @@ __global__ __launch_bounds__(DMA_THREADS) void k_token_reduce_dma(const TokenRed
   prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   token_reduce_dma_block<TS>(p, blockIdx.x, smem);
+}
+
+// Weight gradient of a linear map, dw = dy^T x over T tokens: one matrix, so that the blocks of the map's groups (a split's
+// tiles, or a row of them) spread over the XCDs.  out: [splits][M][N].
+// Bound by the main loop at the rate a compute unit gets its operands (3 of 4 units busy with 192 tiles).  16384 tokens, 4608 x 1536:
+// 201 us, 1155 TFLOP/s (the library's product 383 us, and 10 for the cast of its bf16 result); 1536 x 1536 in four splits 69 + 8 us
+// (148 + 6); 7500 tokens, 2304 x 768 32 + 7, 768 x 768 24 + 4 (75 + 5, 53 + 4).
+struct WeightGradParams {
+  const uint16_t* dy; const uint16_t* x;
+  int ldy, ldx, T, M, N, split_len;
+  float* out;
+  TileMap map;   // tiles of M, tiles of N, splits
+};
+template <class TS>
+__global__ __launch_bounds__(DMA_THREADS) void k_weight_grad_dma(const WeightGradParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  int bx, by, split;
+  if (!p.map.locate(blockIdx.x, bx, by, split)) return;
+  const int m0 = bx * TS::BM, n0 = by * TS::BN, k_begin = split * p.split_len;
+  DmaOperand a, b;
+  a.base = p.dy + (size_t)k_begin * p.ldy + m0; a.ld = p.ldy; a.rows = p.M - m0;
+  b.base = p.x + (size_t)k_begin * p.ldx + n0; b.ld = p.ldx; b.rows = p.N - n0;
+  token_reduce_tile<TS>(a, b, min(p.split_len, p.T - k_begin), smem);
+  using ST = StageTile<TS, 4>;
+  const int r0 = ST::row0(), c0 = ST::col0();
+  if (!ST::active() || n0 + c0 >= p.N) return;
+  const char* src = smem + (r0 * ST::LD + c0) * 4;
+  float* dst = p.out + (size_t)split * p.M * p.N + (size_t)(m0 + r0) * p.N + n0 + c0;
+  const size_t rstep = (size_t)ST::RPP * p.N;
+#pragma unroll 8
+  for (int ps = 0; ps < ST::PASSES; ++ps) {
+    const int r = r0 + ps * ST::RPP;
+    if (r < TS::BM && m0 + r < p.M) *reinterpret_cast<float4*>(dst + ps * rstep) = *reinterpret_cast<const float4*>(src + ps * ST::RPP * ST::LD * 4);
+  }
 }
 
 // The token reduction of an update's backward together with the two token-row GEMMs that read the same

@@ -2037,7 +2037,7 @@ int lact_layer_post_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, 
 int32_t lact_layer_post_dw_rows(int32_t B, int32_t L, int32_t H) {
   LayerGeom g;
   if (layer_geom(B, L, H, 4, &g)) return -1;
-  return (int32_t)layer_post_bwd_blocks(g) * 4;
+  return (int32_t)layer_post_bwd_blocks(g);
 }
 
 int lact_layer_post_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t use_norm, float eps,
@@ -2054,6 +2054,188 @@ int lact_layer_post_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H,
   if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_post_bwd", "layer_post_bwd", 0.0, (k_layer_post<uint16_t, true>), dim3(layer_post_bwd_blocks(p.g)), dim3(256), s, p);
   else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_post_bwd", "layer_post_bwd", 0.0, (k_layer_post<float, true>), dim3(layer_post_bwd_blocks(p.g)), dim3(256), s, p);
   else return fail("act_dtype must be LACT_BF16 or LACT_F32");
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+}  // extern "C"
+namespace {
+// ---- weight gradient of a linear map: dw[M, N] = dy[T, M]^T x[T, N] on the token reduction's kernel ---------------------
+struct WeightGradPlan {
+  bool big;
+  int tiles;
+  Split sp;
+  size_t bytes;
+};
+// 192 x 192 tiles where they divide the matrix and are enough of them, else 128 x 128 (768 x 768 from 7500 tokens: 16 tiles of
+// 192 leave the split to fill the chip, at a read and a write of a partial sum per 576 tokens).
+int weight_grad_plan(int T, int M, int N, WeightGradPlan* w) {
+  if (T < 64 || M <= 0 || N <= 0 || M % 8 || N % 8) return fail("weight gradient: 64 tokens or more, features multiples of 8");
+  if (M > MAX_ROW_STRIDE || N > MAX_ROW_STRIDE) return fail("row stride too large");
+  w->big = M % TS_NS::BM == 0 && N % TS_NS::BN == 0 && (M / TS_NS::BM) * (N / TS_NS::BN) >= 48;
+  const int bm = w->big ? TS_NS::BM : TS_SQ::BM, bn = w->big ? TS_NS::BN : TS_SQ::BN;
+  w->tiles = ceil_div(M, bm) * ceil_div(N, bn);
+  w->sp = choose_split(T, w->tiles, Plan::MAX_SPLITS, 1024);
+  w->bytes = w->sp.n > 1 ? (size_t)w->sp.n * M * N * 4 : 0;
+  return 0;
+}
+template <class TS>
+void launch_weight_grad(const WeightGradParams& p, double flops, hipStream_t s) {
+  constexpr int SM = cmax(DmaSmem<TS, 1, row_stages<TS>()>::BYTES, StageTile<TS, 4>::BYTES);
+  LACT_BIG_LDS(k_weight_grad_dma<TS>, SM);
+  LACT_LAUNCH_SMEM("k_weight_grad_dma", "weight_grad", flops, (k_weight_grad_dma<TS>), dim3(p.map.grid()), dim3(DMA_THREADS), SM, s, p);
+}
+
+// ---- small projections of the layer input -------------------------------------------------------------
+constexpr int LAYER_IN_MAX_LR = 24, LAYER_IN_MAX_B16 = 16;   // outputs of the fp32 map and of the bf16 maps together
+int layer_in_check(LayerInParams& p, long long rows, int dim) {
+  if (rows <= 0 || dim <= 0 || dim % 4) return fail("layer input: rows must be positive, channels a multiple of 4");
+  if (p.lr.n < 0 || p.lr.n > LAYER_IN_MAX_LR || p.mom.n < 0 || p.gate.n < 0 || p.mom.n + p.gate.n > LAYER_IN_MAX_B16)
+    return fail("layer input: too many outputs");
+  if ((p.lr.n && !p.lr.w) || (p.mom.n && !p.mom.w) || (p.gate.n && !p.gate.w)) return fail("null pointer: layer input weights");
+  p.rows = rows; p.dim = dim;
+  return 0;
+}
+// The kernels are made for numbers of outputs in fours; a launch takes the next larger one.
+int layer_in_nl(const LayerInParams& p) { const int n = (p.lr.n + 3) / 4; return n <= 2 ? 2 : n <= 4 ? n : 6; }
+int layer_in_nb(const LayerInParams& p) { const int n = (p.mom.n + p.gate.n + 3) / 4; return n == 0 ? 0 : n <= 2 ? 2 : 4; }
+template <int NL, class F>
+void layer_in_with_nb(const LayerInParams& p, F f) {
+  const int nb = layer_in_nb(p);
+  if (nb == 0) f(std::integral_constant<int, NL>(), std::integral_constant<int, 0>());
+  else if (nb == 2) f(std::integral_constant<int, NL>(), std::integral_constant<int, 2>());
+  else f(std::integral_constant<int, NL>(), std::integral_constant<int, 4>());
+}
+template <class F>
+void layer_in_dispatch(const LayerInParams& p, F f) {
+  const int nl = layer_in_nl(p);
+  if (nl == 2) layer_in_with_nb<2>(p, f);
+  else if (nl == 3) layer_in_with_nb<3>(p, f);
+  else if (nl == 4) layer_in_with_nb<4>(p, f);
+  else layer_in_with_nb<6>(p, f);
+}
+// Tokens of a wave in the weight gradients: half as many where the chip would otherwise have fewer than two blocks per unit
+// (7500 tokens of 768 channels, 24 outputs: 35 us with 32, 18.6 with 16; more partial sums cost more than they bring at 16384
+// tokens of 1536).
+int layer_in_dw_tok(long long rows, int dim) { return (rows + 4 * LAYER_IN_DWTOK - 1) / (4 * LAYER_IN_DWTOK) * ceil_div(dim, 256) >= 512 ? LAYER_IN_DWTOK : LAYER_IN_DWTOK / 2; }
+int layer_in_parts(long long rows, int dim) { const int n = 4 * layer_in_dw_tok(rows, dim); return (int)((rows + n - 1) / n); }
+size_t layer_in_floats(const LayerInParams& p, long long rows, int dim) {
+  const int no = 4 * (layer_in_nl(p) + layer_in_nb(p));
+  return (size_t)layer_in_parts(rows, dim) * no * (dim + 4);
+}
+LayerInParams layer_in_maps(const float* wl, int nl, const float* wm, int nm, const float* wg, int ng) {
+  LayerInParams p;
+  memset(&p, 0, sizeof(p));
+  p.lr = LayerInMap{wl, nullptr, nl}; p.mom = LayerInMap{wm, nullptr, nm}; p.gate = LayerInMap{wg, nullptr, ng};
+  return p;
+}
+}  // namespace
+extern "C" {
+
+int lact_layer_sum_rows(int32_t rows, int32_t dim, const float* part, float* out, void* stream) {
+  if (rows <= 0 || dim <= 0) return fail("sum of rows: rows and columns must be positive");
+  if (check_ptrs({part, out}, "sum of rows")) return -1;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  LACT_LAUNCH("k_layer_sum_rows", "layer_sum_rows", 0.0, k_layer_sum_rows, dim3(ceil_div(dim, 64)), dim3(1024), s, part, rows, dim, out);
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+size_t lact_weight_grad_workspace_bytes(int32_t T, int32_t M, int32_t N) {
+  WeightGradPlan w;
+  return weight_grad_plan(T, M, N, &w) ? 0 : w.bytes;
+}
+
+int lact_weight_grad(int32_t T, int32_t M, int32_t N, const void* dy, int32_t dy_ld, const void* x, int32_t x_ld, float* dw,
+                     void* workspace, void* stream) {
+  WeightGradPlan w;
+  if (weight_grad_plan(T, M, N, &w)) return -1;
+  if (check_ptrs({dy, x, dw}, "weight gradient tensors")) return -1;
+  if (dy_ld < M || x_ld < N || dy_ld % 8 || x_ld % 8 || dy_ld > MAX_ROW_STRIDE || x_ld > MAX_ROW_STRIDE) return fail("weight gradient: row strides");
+  if (w.bytes && !workspace) return fail("null pointer: weight gradient workspace");
+  WeightGradParams p;
+  memset(&p, 0, sizeof(p));
+  p.dy = static_cast<const uint16_t*>(dy); p.ldy = dy_ld;
+  p.x = static_cast<const uint16_t*>(x); p.ldx = x_ld;
+  p.T = T; p.M = M; p.N = N; p.split_len = w.sp.len;
+  p.out = w.sp.n == 1 ? dw : static_cast<float*>(workspace);
+  p.map = make_tile_map(ceil_div(M, w.big ? TS_NS::BM : TS_SQ::BM), ceil_div(N, w.big ? TS_NS::BN : TS_SQ::BN), w.sp.n);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const double flops = 2.0 * T * M * N;
+  if (w.big) launch_weight_grad<TS_NS>(p, flops, s);
+  else launch_weight_grad<TS_SQ>(p, flops, s);
+  if (w.sp.n > 1) {
+    const long long n = (long long)M * N;
+    LACT_LAUNCH("k_reduce_partials", "weight_grad", 0.0, k_reduce_partials, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), s, dw, nullptr, 1.f, p.out, w.sp.n, n);
+  }
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+int lact_layer_in_forward(int64_t rows, int32_t dim, const float* x, const float* mom_w, const float* mom_b, int32_t mom_n,
+                          const float* gate_w, const float* gate_b, int32_t gate_n, void* xb, float* mom_raw, void* gate_raw, void* stream) {
+  LayerInParams p = layer_in_maps(nullptr, 0, mom_w, mom_n, gate_w, gate_n);
+  if (layer_in_check(p, rows, dim)) return -1;
+  if (mom_n + gate_n == 0) return fail("layer input: no outputs");
+  if (check_ptrs({x, xb}, "layer input tensors")) return -1;
+  if ((mom_n && !mom_raw) || (gate_n && !gate_raw)) return fail("null pointer: layer input outputs");
+  p.mom.bias = mom_b; p.gate.bias = gate_b;
+  p.x = x; p.xb = static_cast<uint16_t*>(xb); p.mom_raw = mom_raw; p.gate_raw = static_cast<uint16_t*>(gate_raw);
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const dim3 grid((unsigned)((rows + 4 * LAYER_IN_TOK - 1) / (4 * LAYER_IN_TOK)));
+  if (layer_in_nb(p) == 2) LACT_LAUNCH("k_layer_in", "layer_in", 0.0, (k_layer_in<2>), grid, dim3(256), s, p);
+  else LACT_LAUNCH("k_layer_in", "layer_in", 0.0, (k_layer_in<4>), grid, dim3(256), s, p);
+  LACT_CHECK_LAUNCH();
+  return 0;
+}
+
+size_t lact_layer_in_backward_workspace_bytes(int64_t rows, int32_t dim, int32_t lr_n, int32_t mom_n, int32_t gate_n) {
+  const LayerInParams p = layer_in_maps(nullptr, lr_n, nullptr, mom_n, nullptr, gate_n);
+  return layer_in_floats(p, rows, dim) * 4;
+}
+
+int lact_layer_in_backward(int64_t rows, int32_t dim, const float* x, const float* lr_w, int32_t lr_n, const float* mom_w, int32_t mom_n,
+                           const float* gate_w, int32_t gate_n, const float* dlr_raw, const float* dmom_raw, const void* dgate_raw,
+                           const void* dxq, float* dx, float* dlr_w, float* dlr_b, float* dmom_w, float* dmom_b, float* dgate_w,
+                           float* dgate_b, void* workspace, void* stream) {
+  LayerInParams p = layer_in_maps(lr_w, lr_n, mom_w, mom_n, gate_w, gate_n);
+  if (layer_in_check(p, rows, dim)) return -1;
+  if (check_ptrs({x}, "layer input tensors")) return -1;
+  if (dx && !dxq) return fail("null pointer: layer input gradient");
+  p.x = x; p.dlr = dlr_raw; p.dmom = dmom_raw; p.dgate = static_cast<const uint16_t*>(dgate_raw);
+  p.dxq = static_cast<const uint16_t*>(dxq); p.dx = dx;
+  p.dw[0] = dlr_w; p.dw[1] = dmom_w; p.dw[2] = dgate_w; p.db[0] = dlr_b; p.db[1] = dmom_b; p.db[2] = dgate_b;
+  hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+  const int chunks = ceil_div(dim, 256);
+  if (dx) {
+    int w = 4;                       // waves of a block: as few idle ones as possible
+    for (int i = 3; i >= 2; --i)
+      if (ceil_div(chunks, i) * i < ceil_div(chunks, w) * w) w = i;
+    if (chunks == 1) w = 1;
+    const dim3 grid((unsigned)((rows + LAYER_IN_DXTOK - 1) / LAYER_IN_DXTOK), ceil_div(chunks, w));
+    layer_in_dispatch(p, [&](auto nl, auto nb) {
+    constexpr int NL = decltype(nl)::value, NB = decltype(nb)::value;
+    LACT_LAUNCH("k_layer_in_dx", "layer_in_bwd", 0.0, (k_layer_in_dx<NL, NB>), grid, dim3(64 * w), s, p);
+  });
+  }
+  bool any = false;
+  for (int i = 0; i < 3; ++i) any = any || p.dw[i] || p.db[i];
+  if (any) {
+    if (!workspace) return fail("null pointer: layer input workspace");
+    const int no = 4 * (layer_in_nl(p) + layer_in_nb(p));
+    p.parts = layer_in_parts(rows, dim);
+    p.dw_tok = layer_in_dw_tok(rows, dim);
+    p.part = static_cast<float*>(workspace);
+    p.bpart = p.part + (size_t)p.parts * no * dim;
+    layer_in_dispatch(p, [&](auto nl, auto nb) {
+    constexpr int NL = decltype(nl)::value, NB = decltype(nb)::value;
+    LACT_LAUNCH("k_layer_in_dw", "layer_in_bwd", 0.0, (k_layer_in_dw<NL, NB>), dim3(p.parts, chunks), dim3(256), s, p);
+  });
+    layer_in_dispatch(p, [&](auto nl, auto nb) {
+    constexpr int NL = decltype(nl)::value, NB = decltype(nb)::value;
+    LACT_LAUNCH("k_layer_in_reduce", "layer_in_bwd", 0.0, (k_layer_in_reduce<NL, NB>), dim3(ceil_div(dim, 64), no), dim3(256), s, p);
+  });
+  }
   LACT_CHECK_LAUNCH();
   return 0;
 }

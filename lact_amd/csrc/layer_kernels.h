@@ -252,7 +252,7 @@ struct LayerPostParams {
   void* y;                    // [B, L, H*hd]
   // backward
   const void* dy; void* d_o; void* dgate_raw;
-  float* dw_part;             // [gridDim.x * 4][hd] partial sums of the weight gradient, or null
+  float* dw_part;             // [gridDim.x][hd] partial sums of the weight gradient, or null
 };
 // Backward: each wave walks rows row0, row0 + stride, ... so that its partial weight gradient stays in registers.
 template <typename T, bool BWD>
@@ -362,13 +362,286 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
       }
     }
   }
-  if (BWD && p.dw_part) {
-    float* dst = p.dw_part + ((size_t)blockIdx.x * 4 + wave) * hd;
+  if (BWD && p.dw_part) {      // the four waves' shares, in a fixed order
+    __shared__ float red[LAYER_VEC_MAX * 256];
+    for (int w = 0; w < 4; ++w) {
+      if (wave == w) {
 #pragma unroll
-    for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-      const int c = lane * 4 + i * 256;
-      if (c < hd) *reinterpret_cast<float4*>(dst + c) = make_float4(dwacc[i][0], dwacc[i][1], dwacc[i][2], dwacc[i][3]);
+        for (int i = 0; i < LAYER_VEC_MAX; ++i) {
+          const int c = lane * 4 + i * 256;
+          if (c < hd)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) red[c + j] = w == 0 ? dwacc[i][j] : red[c + j] + dwacc[i][j];
+        }
+      }
+      __syncthreads();
     }
+    for (int c = threadIdx.x; c < hd; c += 256) p.dw_part[(size_t)blockIdx.x * hd + c] = red[c];
+  }
+}
+
+// out[c] = sum over the rows of part [rows][dim], in a fixed order: 64 columns and 16 groups of rows a block.  Grid ceil(dim / 64),
+// 1024 threads.
+__global__ __launch_bounds__(1024) void k_layer_sum_rows(const float* part, int rows, int dim, float* out) {
+  __shared__ float red[16][64];
+  const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
+  float s = 0.f;
+  if (c < dim)
+#pragma unroll 16
+    for (int r = grp; r < rows; r += 16) s += part[(size_t)r * dim + c];
+  red[grp][lane] = s;
+  __syncthreads();
+  if (grp == 0 && c < dim) {
+    for (int i = 1; i < 16; ++i) s += red[i][lane];
+    out[c] = s;
+  }
+}
+
+// ---- small projections of the layer input -------------------------------------------------------------
+// lr_proj (fp32, outside autocast) and, in the causal layer, momentum_proj[0] and ttt_scale_proj (bf16 under autocast) read the
+// layer's input like to_qkv does, but have a handful of outputs.  One pass over the fp32 input makes the bf16 copy that the
+// to_qkv GEMM reads and the latter two, one all their parameter gradients, one the gradient of the input.
+//
+// Output n of the launch: n < NL * 4: rate row n (valid below n1), from the fp32 input and weights; behind them the rows of the
+// two bf16 maps, from input and weights rounded to bf16, the sum in fp32, the result rounded: what the GEMMs of autocast do.
+// Bound by HBM and vector-ALU issue alike.  16384 tokens of 1536 channels, 12 + 8 outputs, us: forward 28 (the two products and four
+// casts 85), gradient of the input 50, of the parameters 45 + 8 (six products with a dozen rows or columns each, two bias sums and
+// seven additions and casts: 520).  7500 tokens of 768 channels, 24 outputs: 20 and 19 + 5 (85).
+struct LayerInMap {
+  const float* w;      // [n][dim] fp32
+  const float* bias;   // [n] or null (forward)
+  int n;
+};
+struct LayerInParams {
+  long long rows;      // tokens
+  int dim;
+  const float* x;      // [rows, dim]
+  uint16_t* xb;        // forward: bf16 copy of x
+  LayerInMap lr, mom, gate;
+  float* mom_raw;      // [rows, mom.n], bf16 values
+  uint16_t* gate_raw;  // [rows, gate.n]
+  // backward
+  const float* dlr; const float* dmom; const uint16_t* dgate;   // each nullable: no gradient
+  const uint16_t* dxq; // gradient of the input through to_qkv, [rows, dim]
+  float* dx;           // [rows, dim]
+  float* part;         // [parts][(NL + NB) * 4][dim] partial sums of the weight gradients
+  float* bpart;        // [parts * 4][(NL + NB) * 4] and of the bias gradients
+  int parts, dw_tok;   // dw_tok: tokens of a wave in the weight gradients, at most LAYER_IN_DWTOK
+  float* dw[3]; float* db[3];   // by map; each nullable
+};
+constexpr int LAYER_IN_TOK = 4;     // tokens of a wave in the forward
+constexpr int LAYER_IN_DXTOK = 32;  // tokens of a block in the input gradient
+constexpr int LAYER_IN_DWTOK = 32;  // most tokens of a wave in the weight gradients
+
+// row `n` of the launch as (map, row inside it); map -1: padding
+template <int NL, int NB>
+__device__ __forceinline__ int layer_in_row(const LayerInParams& p, int n, int& r) {
+  if (n < 4 * NL) { r = n; return n < p.lr.n ? 0 : -1; }
+  r = n - 4 * NL;
+  if (r < p.mom.n) return 1;
+  r -= p.mom.n;
+  return r < p.gate.n ? 2 : -1;
+}
+template <int NL, int NB>
+__device__ __forceinline__ float4 layer_in_weight(const LayerInParams& p, int n, int c) {
+  int r;
+  const int m = layer_in_row<NL, NB>(p, n, r);
+  if (m < 0 || c >= p.dim) return make_float4(0.f, 0.f, 0.f, 0.f);
+  const float* w = m == 0 ? p.lr.w : m == 1 ? p.mom.w : p.gate.w;
+  float4 v = *reinterpret_cast<const float4*>(w + (size_t)r * p.dim + c);
+  if (m > 0) v = make_float4(round_bf16(v.x), round_bf16(v.y), round_bf16(v.z), round_bf16(v.w));
+  return v;
+}
+// gradient that arrives at output n of token t
+template <int NL, int NB>
+__device__ __forceinline__ float layer_in_grad(const LayerInParams& p, int n, long long t) {
+  int r;
+  const int m = layer_in_row<NL, NB>(p, n, r);
+  if (m < 0 || t >= p.rows) return 0.f;
+  if (m == 0) return p.dlr ? p.dlr[t * p.lr.n + r] : 0.f;
+  if (m == 1) return p.dmom ? round_bf16(p.dmom[t * p.mom.n + r]) : 0.f;
+  return p.dgate ? bf16_to_f32(p.dgate[t * p.gate.n + r]) : 0.f;
+}
+
+// Forward: the bf16 copy and the bf16 maps.  (The rates stay a library product: they decide the roundings of everything that
+// Newton-Schulz amplifies.)  A wave owns four tokens, its lanes the columns in chunks of 256; the chunk's weights are staged in
+// LDS for the block's 16 tokens.  The sums over the lanes of all outputs together: every step of the exchange halves the values a
+// lane holds (one shuffle a value instead of six).
+template <int NB>
+__global__ __launch_bounds__(256) void k_layer_in(const LayerInParams p) {
+  constexpr int NO = 4 * NB, TOK = LAYER_IN_TOK;
+  __shared__ float4 ws[NO][64];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long long t0 = ((long long)blockIdx.x * 4 + wave) * TOK;
+  float v[NO * TOK];
+#pragma unroll
+  for (int i = 0; i < NO * TOK; ++i) v[i] = 0.f;
+  const int chunks = (p.dim + 255) / 256;
+  float4 xn[TOK], wn[NB];
+  auto fetch = [&](int ch) {   // the next chunk's input and weights, while this one's are used
+    const int c = ch * 256 + lane * 4;
+#pragma unroll
+    for (int k = 0; k < TOK; ++k)
+      xn[k] = (c < p.dim && t0 + k < p.rows) ? *reinterpret_cast<const float4*>(p.x + (t0 + k) * p.dim + c) : make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int i = 0; i < NB; ++i) wn[i] = layer_in_weight<0, NB>(p, i * 4 + wave, c);
+  };
+  fetch(0);
+  for (int ch = 0; ch < chunks; ++ch) {
+    const int c = ch * 256 + lane * 4;
+    float4 x[TOK];
+#pragma unroll
+    for (int k = 0; k < TOK; ++k) x[k] = xn[k];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NB; ++i) ws[i * 4 + wave][lane] = wn[i];
+    __syncthreads();
+    if (ch + 1 < chunks) fetch(ch + 1);
+#pragma unroll
+    for (int k = 0; k < TOK; ++k) {
+      const uint32_t lo = pack_bf16(x[k].x, x[k].y), hi = pack_bf16(x[k].z, x[k].w);
+      if (c < p.dim && t0 + k < p.rows) *reinterpret_cast<uint2*>(p.xb + (t0 + k) * p.dim + c) = make_uint2(lo, hi);
+      x[k] = make_float4(bf16_lo(lo), bf16_hi(lo), bf16_lo(hi), bf16_hi(hi));
+    }
+#pragma unroll
+    for (int n = 0; n < NO; ++n) {
+      const float4 w = ws[n][lane];
+#pragma unroll
+      for (int k = 0; k < TOK; ++k) v[n * TOK + k] = fmaf(x[k].x, w.x, fmaf(x[k].y, w.y, fmaf(x[k].z, w.z, fmaf(x[k].w, w.w, v[n * TOK + k]))));
+    }
+  }
+  // value 16 i + 8 b(2) + 4 b(3) + 2 b(4) + b(5) ends up in v[i] of the lanes with these bits b
+#pragma unroll
+  for (int s = 0; s < 4; ++s) {
+    const int d = 32 >> s;
+    const bool up = (lane & d) != 0;
+#pragma unroll
+    for (int i = 0; i < (NO * TOK) >> (s + 1); ++i) {
+      const float keep = up ? v[2 * i + 1] : v[2 * i], send = up ? v[2 * i] : v[2 * i + 1];
+      v[i] = keep + __shfl_xor(send, d, 64);
+    }
+  }
+  const int tok = 2 * ((lane >> 4) & 1) + (lane >> 5), sub = 2 * ((lane >> 2) & 1) + ((lane >> 3) & 1);
+  const long long t = t0 + tok;
+#pragma unroll
+  for (int i = 0; i < NB; ++i) {
+    float s = v[i];
+    s += __shfl_xor(s, 2, 64);
+    s += __shfl_xor(s, 1, 64);
+    if ((lane & 3) == 0 && t < p.rows) {
+      int r;
+      const int m = layer_in_row<0, NB>(p, i * 4 + sub, r);
+      if (m == 1) p.mom_raw[t * p.mom.n + r] = round_bf16(p.mom.bias ? s + round_bf16(p.mom.bias[r]) : s);
+      else if (m == 2) p.gate_raw[t * p.gate.n + r] = f32_to_bf16(p.gate.bias ? s + round_bf16(p.gate.bias[r]) : s);
+    }
+  }
+}
+
+// Gradient of the input: dx = dxq + sum over the outputs of gradient times weight row.  A lane owns four columns and keeps their
+// weights, the block's tokens have their output gradients in LDS.  Grid (token blocks, column blocks of blockDim.x * 4).
+template <int NL, int NB>
+__global__ __launch_bounds__(256) void k_layer_in_dx(const LayerInParams p) {
+  constexpr int NO = 4 * (NL + NB), TOK = LAYER_IN_DXTOK;
+  __shared__ float gs[TOK][NO];
+  const long long t0 = (long long)blockIdx.x * TOK;
+  for (int i = threadIdx.x; i < TOK * NO; i += blockDim.x) gs[i / NO][i % NO] = layer_in_grad<NL, NB>(p, i % NO, t0 + i / NO);
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  float4 w[NO];
+#pragma unroll
+  for (int n = 0; n < NO; ++n) w[n] = layer_in_weight<NL, NB>(p, n, c);
+  __syncthreads();
+  if (c >= p.dim) return;
+  const int toks = (int)min((long long)TOK, p.rows - t0);
+#pragma unroll 8
+  for (int k = 0; k < toks; ++k) {
+    float o[4];
+    Elem<uint16_t>::load4(p.dxq + (t0 + k) * p.dim + c, o);
+#pragma unroll
+    for (int n = 0; n < NO; ++n) {
+      const float g = gs[k][n];
+      o[0] = fmaf(g, w[n].x, o[0]); o[1] = fmaf(g, w[n].y, o[1]); o[2] = fmaf(g, w[n].z, o[2]); o[3] = fmaf(g, w[n].w, o[3]);
+    }
+    *reinterpret_cast<float4*>(p.dx + (t0 + k) * p.dim + c) = make_float4(o[0], o[1], o[2], o[3]);
+  }
+}
+
+// Gradients of the small maps' parameters: a lane owns four columns of every row and sums its wave's tokens, the block its four
+// waves', in a fixed order; k_layer_in_reduce sums the blocks.  Grid (token blocks, chunks of 256 columns).
+template <int NL, int NB>
+__global__ __launch_bounds__(256) void k_layer_in_dw(const LayerInParams p) {
+  constexpr int NO = 4 * (NL + NB), TOK = LAYER_IN_DWTOK;
+  __shared__ float lds[(4 * TOK > 256 ? 4 * TOK : 256) * NO];   // output gradients of the block's tokens, then the sums of its waves
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tok = p.dw_tok;
+  const long long t0 = ((long long)blockIdx.x * 4 + wave) * tok;
+  float* gs = lds + wave * TOK * NO;
+  for (int i = lane; i < tok * NO; i += 64) gs[i] = layer_in_grad<NL, NB>(p, i % NO, t0 + i / NO);
+  __syncthreads();
+  const int c = blockIdx.y * 256 + lane * 4;
+  if (blockIdx.y == 0 && lane < NO) {
+    float s = 0.f;
+    for (int k = 0; k < tok; ++k) s += gs[k * NO + lane];
+    p.bpart[((size_t)blockIdx.x * 4 + wave) * NO + lane] = s;
+  }
+  float4 acc[NO];
+#pragma unroll
+  for (int n = 0; n < NO; ++n) acc[n] = make_float4(0.f, 0.f, 0.f, 0.f);
+  const int toks = (int)max(0LL, min((long long)tok, p.rows - t0));
+  if (c < p.dim) {
+#pragma unroll 8
+    for (int k = 0; k < toks; ++k) {
+      float4 x = *reinterpret_cast<const float4*>(p.x + (t0 + k) * p.dim + c);
+#pragma unroll
+      for (int n = 0; n < NO; ++n) {
+        if (n == 4 * NL) x = make_float4(round_bf16(x.x), round_bf16(x.y), round_bf16(x.z), round_bf16(x.w));
+        const float g = gs[k * NO + n];
+        acc[n].x = fmaf(g, x.x, acc[n].x); acc[n].y = fmaf(g, x.y, acc[n].y); acc[n].z = fmaf(g, x.z, acc[n].z); acc[n].w = fmaf(g, x.w, acc[n].w);
+      }
+    }
+  }
+  __syncthreads();
+  float4* sums = reinterpret_cast<float4*>(lds);
+  for (int w = 0; w < 4; ++w) {
+    if (wave == w) {
+#pragma unroll
+      for (int n = 0; n < NO; ++n) {
+        float4 v = acc[n];
+        if (w > 0) {
+          const float4 o = sums[n * 64 + lane];
+          v = make_float4(o.x + v.x, o.y + v.y, o.z + v.z, o.w + v.w);
+        }
+        sums[n * 64 + lane] = v;
+      }
+    }
+    __syncthreads();
+  }
+  for (int i = threadIdx.x; i < NO * 64; i += 256) {
+    const int n = i / 64, cc = blockIdx.y * 256 + (i % 64) * 4;
+    if (cc < p.dim) *reinterpret_cast<float4*>(p.part + ((size_t)blockIdx.x * NO + n) * p.dim + cc) = sums[i];
+  }
+}
+// Grid (ceil(dim / 64), NO): 64 columns of one row, four groups of partial sums.
+template <int NL, int NB>
+__global__ __launch_bounds__(256) void k_layer_in_reduce(const LayerInParams p) {
+  constexpr int NO = 4 * (NL + NB);
+  __shared__ float red[4][64];
+  const int n = blockIdx.y, lane = threadIdx.x & 63, grp = threadIdx.x >> 6, c = blockIdx.x * 64 + lane;
+  int r;
+  const int m = layer_in_row<NL, NB>(p, n, r);
+  if (m < 0) return;
+  float s = 0.f;
+  if (c < p.dim)
+#pragma unroll 8
+    for (int i = grp; i < p.parts; i += 4) s += p.part[((size_t)i * NO + n) * p.dim + c];
+  red[grp][lane] = s;
+  __syncthreads();
+  float* dw = m == 0 ? p.dw[0] : m == 1 ? p.dw[1] : p.dw[2];
+  float* db = m == 0 ? p.db[0] : m == 1 ? p.db[1] : p.db[2];
+  if (grp == 0 && c < p.dim && dw) dw[(size_t)r * p.dim + c] = red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane];
+  if (grp == 1 && blockIdx.x == 0 && db) {
+    float b = 0.f;
+    for (int i = lane; i < p.parts * 4; i += 64) b += p.bpart[(size_t)i * NO + n];
+    b = wave_sum(b);
+    if (lane == 0) db[r] = b;
   }
 }
 

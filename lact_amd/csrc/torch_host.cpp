@@ -335,6 +335,288 @@ py::tuple run_program(const c10::intrusive_ptr<Schedule>& sc, const Tensor& w0, 
   return out;
 }
 
+// ---- the layers' functions around the operation -----------------------------------------------------------------------
+// lact_amd/layers.py calls these on plain tensors (its Python functions of the same content take what wants to see Python: hooks,
+// transforms, modes).  Native because a layer at a few thousand tokens is bound by its host side: 45 launches and a dozen
+// autograd functions per training step took 800 us in Python for 650 us of kernels.
+void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
+Tensor dense(const Tensor& t) {
+  const Tensor c = t.contiguous();
+  return aligned16(c) ? c : c.clone();
+}
+Tensor dense(const Tensor& t, at::ScalarType dtype) { return dense(cast(t, dtype)); }
+int act_code(const Tensor& t) {
+  if (!t.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)");
+  TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat, "unsupported activation dtype ", t.scalar_type(), ": bf16 or fp32");
+  return t.scalar_type() == at::kBFloat16 ? LACT_BF16 : LACT_F32;
+}
+// The kernels take raw pointers: a tensor elsewhere, or of another shape, has to be refused here.
+void expect(const Tensor& t, const Tensor& like, at::IntArrayRef shape, const char* name) {
+  if (!t.defined()) return;
+  if (t.device() != like.device()) throw std::runtime_error(std::string("expected all tensors to be on the same device: ") + name);
+  if (t.sizes() != shape) throw std::invalid_argument(std::string(name) + ": expected shape " + c10::str(shape) + ", got " + c10::str(t.sizes()));
+}
+Tensor value(const OptTensor& t) { return t ? *t : Tensor(); }
+int64_t as_int(AutogradContext* ctx, const char* key) { return ctx->saved_data[key].toInt(); }
+// end of every backward: what must not be differentiated again says so
+variable_list finish(variable_list grads, bool twice) {
+  if (twice) refuse_second_derivative(grads);
+  return grads;
+}
+
+// qkv [B, L, 3*H*hd] -> q, k, v [(B H), L, hd], and with the rescaling parameters [H*hd, 2] the attention's q, k, v [B, L, H*hd]
+struct LayerPreFn : torch::autograd::Function<LayerPreFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& qkv_, const OptTensor& scale_, const OptTensor& offset_, int64_t H, int64_t hd, bool l2norm) {
+    const c10::hip::HIPGuard guard(qkv_.device().index());
+    const Tensor qkv = dense(qkv_);
+    const int act = act_code(qkv);
+    const int64_t B = qkv.size(0), L = qkv.size(1);
+    expect(qkv, qkv, {B, L, 3 * H * hd}, "qkv");
+    variable_list out;
+    for (int i = 0; i < 3; ++i) out.push_back(at::empty({B * H, L, hd}, qkv.options()));
+    Tensor scale;
+    if (scale_) {
+      expect(*scale_, qkv, {H * hd, 2}, "qk_scale");
+      expect(*offset_, qkv, {H * hd, 2}, "qk_offset");
+      scale = plain_f32(*scale_);
+      const Tensor offset = plain_f32(*offset_);
+      for (int i = 0; i < 3; ++i) out.push_back(at::empty({B, L, H * hd}, qkv.options()));
+      check(lact_layer_pre_attn_forward(act, (int)B, (int)L, (int)H, (int)hd, l2norm, scale_->scalar_type() == qkv.scalar_type(), ptr(qkv), fptr(scale),
+                                        fptr(offset), ptr(out[0]), ptr(out[1]), ptr(out[2]), ptr(out[3]), ptr(out[4]), ptr(out[5]), stream()));
+      ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)scale_->scalar_type(), (int64_t)offset_->scalar_type()};
+    } else {
+      check(lact_layer_pre_forward(act, (int)B, (int)L, (int)H, (int)hd, l2norm, ptr(qkv), ptr(out[0]), ptr(out[1]), ptr(out[2]), stream()));
+    }
+    ctx->save_for_backward({qkv, scale});
+    ctx->saved_data["H"] = H; ctx->saved_data["hd"] = hd; ctx->saved_data["l2"] = (int64_t)l2norm;
+    ctx->set_materialize_grads(false);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool twice = at::GradMode::is_enabled();
+    const at::AutoGradMode off(false);
+    const auto t = ctx->get_saved_variables();
+    const Tensor &qkv = t[0], &scale = t[1];
+    const c10::hip::HIPGuard guard(qkv.device().index());
+    const int64_t B = qkv.size(0), L = qkv.size(1), H = as_int(ctx, "H"), hd = as_int(ctx, "hd"), l2 = as_int(ctx, "l2");
+    for (size_t i = 0; i < grads.size(); ++i)
+      grads[i] = grads[i].defined() ? dense(grads[i], qkv.scalar_type())
+                                    : i < 3 ? at::zeros({B * H, L, hd}, qkv.options()) : at::zeros({B, L, H * hd}, qkv.options());
+    const Tensor dqkv = at::empty_like(qkv);
+    variable_list res{dqkv, Tensor(), Tensor(), Tensor(), Tensor(), Tensor()};
+    if (!scale.defined()) {
+      check(lact_layer_pre_backward(act_code(qkv), (int)B, (int)L, (int)H, (int)hd, (int)l2, ptr(qkv), ptr(grads[0]), ptr(grads[1]), ptr(grads[2]), ptr(dqkv), stream()));
+    } else {
+      const Tensor ds = at::empty_like(scale), doff = at::empty_like(scale);
+      const Tensor part = at::empty({lact_layer_pre_attn_part_rows((int)B, (int)L, (int)H) * 4 * H * hd}, scale.options());
+      check(lact_layer_pre_attn_backward(act_code(qkv), (int)B, (int)L, (int)H, (int)hd, (int)l2, ptr(qkv), fptr(scale), ptr(grads[0]), ptr(grads[1]), ptr(grads[2]),
+                                         ptr(grads[3]), ptr(grads[4]), ptr(grads[5]), ptr(dqkv), fptr(part), fptr(ds), fptr(doff), stream()));
+      const auto types = ctx->saved_data["types"].toIntVector();
+      res[1] = cast(ds, (at::ScalarType)types[0]);
+      res[2] = cast(doff, (at::ScalarType)types[1]);
+    }
+    return finish(res, twice);
+  }
+};
+
+// lr_raw [B, L, 3*H], momentum_raw [B, L, H] or none -> lr0, lr1, lr2 (, momentum) [(B H), L, 1] fp32
+struct LayerLrFn : torch::autograd::Function<LayerLrFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& lr_, const OptTensor& mom_, int64_t H, double base, bool rates_major) {
+    if (!lr_.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)");
+    const c10::hip::HIPGuard guard(lr_.device().index());
+    const Tensor lr = plain_f32(lr_), mom = mom_ ? plain_f32(*mom_) : Tensor();
+    const int64_t B = lr.size(0), L = lr.size(1);
+    expect(lr, lr, {B, L, 3 * H}, "lr_raw");
+    expect(mom, lr, {B, L, H}, "momentum_raw");
+    variable_list out;
+    for (int i = 0; i < (mom_ ? 4 : 3); ++i) out.push_back(at::empty({B * H, L, 1}, lr.options()));
+    check(lact_layer_lr_forward((int)B, (int)L, (int)H, rates_major, (float)base, fptr(lr), fptr(out[0]), fptr(out[1]), fptr(out[2]), fptr(mom),
+                                mom_ ? fptr(out[3]) : nullptr, stream()));
+    ctx->save_for_backward({lr, mom});
+    ctx->saved_data["H"] = H; ctx->saved_data["base"] = base; ctx->saved_data["major"] = (int64_t)rates_major;
+    ctx->saved_data["types"] = std::vector<int64_t>{(int64_t)lr_.scalar_type(), (int64_t)(mom_ ? mom_->scalar_type() : at::kFloat)};
+    ctx->set_materialize_grads(false);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool twice = at::GradMode::is_enabled();
+    const at::AutoGradMode off(false);
+    const auto t = ctx->get_saved_variables();
+    const Tensor &lr = t[0], &mom = t[1];
+    const c10::hip::HIPGuard guard(lr.device().index());
+    for (auto& g : grads)
+      if (g.defined()) g = plain_f32(g);
+    if (grads.size() < 4) grads.resize(4);
+    const Tensor dlr = at::empty_like(lr), dmom = mom.defined() ? at::empty_like(mom) : Tensor();
+    check(lact_layer_lr_backward((int)lr.size(0), (int)lr.size(1), (int)as_int(ctx, "H"), (int)as_int(ctx, "major"), (float)ctx->saved_data["base"].toDouble(),
+                                 fptr(lr), fptr(grads[0]), fptr(grads[1]), fptr(grads[2]), fptr(dlr), fptr(mom), fptr(grads[3]), fptr(dmom), stream()));
+    const auto types = ctx->saved_data["types"].toIntVector();
+    return finish({cast(dlr, (at::ScalarType)types[0]), cast(dmom, (at::ScalarType)types[1]), Tensor(), Tensor(), Tensor()}, twice);
+  }
+};
+
+// o [(B H), L, hd] -> y [B, L, H*hd]: RMSNorm per head, times silu(gate_raw [B, L, H]), plus add [B, L, H*hd]
+struct LayerPostFn : torch::autograd::Function<LayerPostFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& o_, const OptTensor& weight, const OptTensor& gate, int64_t B, int64_t H, bool use_norm, double eps,
+                        const OptTensor& add) {
+    const c10::hip::HIPGuard guard(o_.device().index());
+    const Tensor o = dense(o_);
+    const int act = act_code(o);
+    const int64_t L = o.size(1), hd = o.size(2);
+    expect(o, o, {B * H, L, hd}, "o");
+    expect(value(weight), o, {hd}, "weight");
+    expect(value(gate), o, {B, L, H}, "gate_raw");
+    expect(value(add), o, {B, L, H * hd}, "add");
+    const Tensor w = weight ? plain_f32(*weight) : Tensor(), g = gate ? dense(*gate, o.scalar_type()) : Tensor();
+    const Tensor a = add ? dense(*add, o.scalar_type()) : Tensor(), y = at::empty({B, L, H * hd}, o.options());
+    check(lact_layer_post_add_forward(act, (int)B, (int)L, (int)H, (int)hd, use_norm, (float)eps, ptr(o), fptr(w), ptr(g), ptr(a), ptr(y), stream()));
+    ctx->save_for_backward({o, w, g});
+    ctx->saved_data["B"] = B; ctx->saved_data["H"] = H; ctx->saved_data["norm"] = (int64_t)use_norm; ctx->saved_data["eps"] = eps;
+    auto type = [](const OptTensor& t) { return (int64_t)(t ? t->scalar_type() : at::ScalarType::Undefined); };
+    ctx->saved_data["types"] = std::vector<int64_t>{type(weight), type(gate), type(add)};
+    return y;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool twice = at::GradMode::is_enabled();
+    const at::AutoGradMode off(false);
+    const auto t = ctx->get_saved_variables();
+    const Tensor &o = t[0], &w = t[1], &g = t[2];
+    const c10::hip::HIPGuard guard(o.device().index());
+    const int64_t B = as_int(ctx, "B"), H = as_int(ctx, "H"), L = o.size(1), hd = o.size(2), norm = as_int(ctx, "norm");
+    const Tensor dy = dense(grads[0], o.scalar_type()), d_o = at::empty_like(o), dg = g.defined() ? at::empty_like(g) : Tensor();
+    const int64_t rows = lact_layer_post_dw_rows((int)B, (int)L, (int)H);
+    const Tensor part = norm && w.defined() ? at::empty({rows, hd}, w.options()) : Tensor();
+    check(lact_layer_post_backward(act_code(o), (int)B, (int)L, (int)H, (int)hd, (int)norm, (float)ctx->saved_data["eps"].toDouble(), ptr(o), fptr(w), ptr(g),
+                                   ptr(dy), ptr(d_o), ptr(dg), fptr(part), stream()));
+    Tensor dw;
+    if (part.defined()) {
+      dw = at::empty_like(w);
+      check(lact_layer_sum_rows((int)rows, (int)hd, fptr(part), fptr(dw), stream()));
+    }
+    const auto types = ctx->saved_data["types"].toIntVector();
+    auto as = [&](const Tensor& x, int i) { return x.defined() && (at::ScalarType)types[i] != at::ScalarType::Undefined ? cast(x, (at::ScalarType)types[i]) : Tensor(); };
+    return finish({d_o, as(dw, 0), as(dg, 1), Tensor(), Tensor(), Tensor(), Tensor(), as(grads[0], 2)}, twice);
+  }
+};
+
+// dy^T x in fp32 for bf16 rows dy [t, m], x [t, n]
+Tensor weight_grad(const Tensor& dy, const Tensor& x) {
+  const int64_t t = x.size(0), m = dy.size(1), n = x.size(1);
+  if (t < 64 || t >= (1LL << 31) || m % 8 || n % 8 || std::max(m, n) >= (1 << 23))   // outside the kernel's range
+    return at::mm(dy.to(at::kFloat).t(), x.to(at::kFloat));
+  const Tensor dw = at::empty({m, n}, x.options().dtype(at::kFloat));
+  const int64_t bytes = (int64_t)lact_weight_grad_workspace_bytes((int)t, (int)m, (int)n);
+  const Tensor ws = bytes ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();
+  check(lact_weight_grad((int)t, (int)m, (int)n, ptr(dy), (int)m, ptr(x), (int)n, fptr(dw), ptr(ws), stream()));
+  return dw;
+}
+Tensor rows_of(const Tensor& t, at::ScalarType dtype) { return dense(cast(t, dtype).reshape({-1, t.size(-1)})); }
+std::vector<int64_t> with_last(at::IntArrayRef sizes, int64_t last) {
+  auto s = sizes.vec();
+  s.back() = last;
+  return s;
+}
+
+// x w^T under bf16 autocast for fp32 w, whose gradient is summed, and returned, in fp32
+struct LinearFn : torch::autograd::Function<LinearFn> {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight) {
+    const c10::hip::HIPGuard guard(x.device().index());
+    const Tensor wb = weight.to(at::kBFloat16), xb = rows_of(x, at::kBFloat16);
+    ctx->save_for_backward({xb, wb});
+    ctx->saved_data["x"] = (int64_t)x.scalar_type();
+    ctx->saved_data["need"] = std::vector<int64_t>{x.requires_grad(), weight.requires_grad()};
+    ctx->saved_data["shape"] = x.sizes().vec();
+    return at::linear(xb, wb).view(with_last(x.sizes(), wb.size(0)));
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool twice = at::GradMode::is_enabled();
+    const at::AutoGradMode off(false);
+    const auto t = ctx->get_saved_variables();
+    const Tensor &xb = t[0], &wb = t[1];
+    const c10::hip::HIPGuard guard(xb.device().index());
+    const auto need = ctx->saved_data["need"].toIntVector();
+    const Tensor g = rows_of(grads[0], at::kBFloat16);
+    Tensor dx, dw;
+    if (need[0]) dx = cast(at::mm(g, wb).view(ctx->saved_data["shape"].toIntVector()), (at::ScalarType)as_int(ctx, "x"));
+    if (need[1]) dw = weight_grad(g, xb);
+    return finish({dx, dw}, twice);
+  }
+};
+
+// The maps of a layer's input x [B, L, dim] fp32 under bf16 autocast: to_qkv in bf16, the rates x lr_w^T + lr_b in fp32, the bf16
+// maps of the momentum (as fp32 values) and of the gate.  to_qkv and the rates are library products; the other maps, and what
+// their and the rates' backward is, csrc/layer_kernels.h.
+struct LayerInFn : torch::autograd::Function<LayerInFn> {
+  static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& qkv_w, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w,
+                               const OptTensor& mom_b, const OptTensor& gate_w, const OptTensor& gate_b) {
+    const c10::hip::HIPGuard guard(x_.device().index());
+    const int64_t B = x_.size(0), L = x_.size(1), dim = x_.size(2), n = B * L;
+    const Tensor x = rows_of(x_, at::kFloat), wb = qkv_w.to(at::kBFloat16);
+    const Tensor lw = plain_f32(lr_w), mw = mom_w ? plain_f32(*mom_w) : Tensor(), gw = gate_w ? plain_f32(*gate_w) : Tensor();
+    const Tensor mb = mom_b ? plain_f32(*mom_b) : Tensor(), gb = gate_b ? plain_f32(*gate_b) : Tensor();
+    const int64_t nm = mw.defined() ? mw.size(0) : 0, ng = gw.defined() ? gw.size(0) : 0;
+    Tensor lr, mom, gate, xb;
+    {
+      const c10::impl::ExcludeDispatchKeyGuard plain(c10::DispatchKey::AutocastCUDA);   // the reference keeps the rates out of autocast
+      lr = at::linear(x, lw, lr_b ? OptTensor(plain_f32(*lr_b)) : OptTensor());
+    }
+    if (nm) mom = at::empty({B, L, nm}, x.options());
+    if (ng) gate = at::empty({B, L, ng}, wb.options());
+    if (nm + ng == 0) {
+      xb = x.to(at::kBFloat16);
+    } else {
+      xb = at::empty({n, dim}, wb.options());
+      check(lact_layer_in_forward(n, (int)dim, fptr(x), fptr(mw), fptr(mb), (int)nm, fptr(gw), fptr(gb), (int)ng, ptr(xb), fptr(mom), ptr(gate), stream()));
+    }
+    ctx->save_for_backward({x, xb, wb, lw, mw, gw});
+    auto need = [](const OptTensor& t) { return (int64_t)(t && t->requires_grad()); };
+    ctx->saved_data["need"] = std::vector<int64_t>{x_.requires_grad(), qkv_w.requires_grad(), need(lr_w), need(lr_b), need(mom_w), need(mom_b), need(gate_w), need(gate_b)};
+    ctx->saved_data["B"] = B; ctx->saved_data["L"] = L;
+    ctx->set_materialize_grads(false);
+    variable_list out{at::linear(xb, wb).view({B, L, wb.size(0)}), lr.view({B, L, lw.size(0)})};
+    if (nm) out.push_back(mom);
+    if (ng) out.push_back(gate);
+    return out;
+  }
+  static variable_list backward(AutogradContext* ctx, variable_list grads) {
+    const bool twice = at::GradMode::is_enabled();
+    const at::AutoGradMode off(false);
+    const auto t = ctx->get_saved_variables();
+    const Tensor &x = t[0], &xb = t[1], &wb = t[2], &lw = t[3], &mw = t[4], &gw = t[5];
+    const c10::hip::HIPGuard guard(x.device().index());
+    const auto need = ctx->saved_data["need"].toIntVector();
+    const int64_t n = x.size(0), dim = x.size(1), counts[3] = {lw.size(0), mw.defined() ? mw.size(0) : 0, gw.defined() ? gw.size(0) : 0};
+    Tensor g, dlr, dmom, dgate;
+    if (grads[0].defined()) g = rows_of(grads[0], at::kBFloat16);
+    if (grads[1].defined()) dlr = plain_f32(grads[1]);
+    if (counts[1] && grads[2].defined()) dmom = plain_f32(grads[2]);
+    if (counts[2] && grads.back().defined()) dgate = dense(grads.back(), at::kBFloat16);
+    Tensor dxq, dx, d[6];
+    if (need[0]) {
+      dxq = g.defined() ? at::mm(g, wb) : at::zeros_like(xb);
+      dx = at::empty({as_int(ctx, "B"), as_int(ctx, "L"), dim}, x.options());
+    }
+    bool any = false;
+    for (int i = 0; i < 6; ++i)
+      if (need[2 + i]) {
+        d[i] = i % 2 == 0 ? at::empty({counts[i / 2], dim}, x.options()) : at::empty({counts[i / 2]}, x.options());
+        any = true;
+      }
+    const Tensor ws = any ? at::empty({(int64_t)lact_layer_in_backward_workspace_bytes(n, (int)dim, (int)counts[0], (int)counts[1], (int)counts[2])}, x.options().dtype(at::kByte)) : Tensor();
+    check(lact_layer_in_backward(n, (int)dim, fptr(x), fptr(lw), (int)counts[0], fptr(mw), (int)counts[1], fptr(gw), (int)counts[2], fptr(dlr), fptr(dmom), ptr(dgate),
+                                 ptr(dxq), fptr(dx), fptr(d[0]), fptr(d[1]), fptr(d[2]), fptr(d[3]), fptr(d[4]), fptr(d[5]), ptr(ws), stream()));
+    Tensor dw;
+    if (need[1]) dw = g.defined() ? weight_grad(g, xb) : at::zeros(wb.sizes(), x.options());
+    return finish({dx, dw, d[0], d[1], d[2], d[3], d[4], d[5]}, twice);
+  }
+};
+
+template <class F, class... Args>
+auto apply_released(Args&&... args) {
+  const py::gil_scoped_release nogil;
+  return F::apply(std::forward<Args>(args)...);
+}
+
 }  // namespace
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
@@ -343,4 +625,15 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
                     bool, bool>());
   m.def("run_program", &run_program);
   m.def("refuse_second_derivative", &refuse_second_derivative_py);
+  m.def("layer_pre", [](const Tensor& qkv, int64_t H, int64_t hd, bool l2norm) { return apply_released<LayerPreFn>(qkv, OptTensor(), OptTensor(), H, hd, l2norm); });
+  m.def("layer_pre_attn", [](const Tensor& qkv, const OptTensor& scale, const OptTensor& offset, int64_t H, int64_t hd, bool l2norm) {
+    return apply_released<LayerPreFn>(qkv, scale, offset, H, hd, l2norm);
+  });
+  m.def("layer_lr", [](const Tensor& lr, const OptTensor& mom, int64_t H, double base, bool rates_major) { return apply_released<LayerLrFn>(lr, mom, H, base, rates_major); });
+  m.def("layer_post", [](const Tensor& o, const OptTensor& weight, const OptTensor& gate, int64_t B, int64_t H, bool use_norm, double eps, const OptTensor& add) {
+    return apply_released<LayerPostFn>(o, weight, gate, B, H, use_norm, eps, add);
+  });
+  m.def("linear", [](const Tensor& x, const Tensor& weight) { return apply_released<LinearFn>(x, weight); });
+  m.def("layer_in", [](const Tensor& x, const Tensor& qkv_w, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w, const OptTensor& mom_b,
+                       const OptTensor& gate_w, const OptTensor& gate_b) { return apply_released<LayerInFn>(x, qkv_w, lr_w, lr_b, mom_w, mom_b, gate_w, gate_b); });
 }

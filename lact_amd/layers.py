@@ -212,6 +212,71 @@ class _PostFn(torch.autograd.Function):
         return d_o, dw, (None if dg is None else dg.to(gd)), None, None, None, None, (None if ctx.add_dtype is None else dy.to(ctx.add_dtype))
 
 
+def _plain(*ts) -> bool:
+    """Whether the host module's functions may take a call: plain tensors, and nobody around who wants to see Python functions or
+    tensor operations (compilation and tracing, function transforms, forward mode, modes, subclasses).  Others get the functions
+    above and the modules themselves."""
+    return (all(t is None or type(t) in (torch.Tensor, nn.Parameter) for t in ts)
+            and not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
+                     or torch._C._len_torch_function_stack() > 0 or _get_current_dispatch_mode() is not None or fwad._current_level >= 0
+                     or any(torch._C._functorch.is_legacy_batchedtensor(t) for t in ts if t is not None)))
+
+
+def _pre(qkv, H, hd, l2norm):
+    return _lib.host().layer_pre(qkv, H, hd, l2norm) if _plain(qkv) else _PreFn.apply(qkv, H, hd, l2norm)
+
+
+def _pre_attn(qkv, scale, offset, H, hd, l2norm):
+    fn = _lib.host().layer_pre_attn if _plain(qkv, scale, offset) else _PreAttnFn.apply
+    return fn(qkv, scale, offset, H, hd, l2norm)
+
+
+def _rates(lr_raw, mom_raw, H, base_lr_inv, rates_major=False):
+    fn = _lib.host().layer_lr if _plain(lr_raw, mom_raw) else _LrFn.apply
+    return fn(lr_raw, mom_raw, H, base_lr_inv, rates_major)
+
+
+def _post(o, weight, gate_raw, B, H, use_norm, eps, add=None):
+    fn = _lib.host().layer_post if _plain(o, weight, gate_raw, add) else _PostFn.apply
+    return fn(o, weight, gate_raw, B, H, use_norm, eps, add)
+
+
+def _plain_linear(m: nn.Module) -> bool:
+    """An nn.Linear in fp32 whose call is F.linear and nothing else: no subclass, hook, parametrisation or replaced forward."""
+    return (type(m) is nn.Linear and "forward" not in m.__dict__
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks)
+            and all(t is None or (t.is_cuda and t.dtype == torch.float32) for t in (m.weight, m.bias)))
+
+
+def _fused_linears(x: torch.Tensor, *mods: nn.Module) -> bool:
+    """Whether the host module may evaluate linear maps of x instead of their modules: plain fp32 ones under bf16 autocast."""
+    return (x.is_cuda and x.dim() == 3 and x.numel() > 0 and torch.is_autocast_enabled("cuda") and torch.get_autocast_dtype("cuda") == torch.bfloat16
+            and all(_plain_linear(m) and m.weight.device == x.device and m.in_features == x.shape[-1] for m in mods)
+            and not nn.modules.module._has_any_global_hook() and _plain(x, *[t for m in mods for t in (m.weight, m.bias)]))
+
+
+def _linear(m: nn.Module, x: torch.Tensor) -> torch.Tensor:
+    """m(x); the gradient of a fused map's weight comes from csrc/gemm_dma_kernels.h, summed and returned in fp32."""
+    return _lib.host().linear(x, m.weight) if m.bias is None and _fused_linears(x, m) else m(x)
+
+
+MAX_LR_OUTPUTS, MAX_BF16_OUTPUTS = 24, 16      # registers of the kernels in csrc/layer_kernels.h
+
+
+def _input_projections(x, to_qkv, lr_proj, momentum=None, gate=None):
+    """to_qkv(x), lr_proj(x) outside autocast, momentum(x), gate(x) (either may be absent: None)."""
+    mods = [m for m in (to_qkv, lr_proj, momentum, gate) if m is not None]
+    if (x.dtype == torch.float32 and to_qkv.bias is None and _fused_linears(x, *mods) and x.shape[-1] % 8 == 0 and x.shape[:-1].numel() < 1 << 31
+            and 0 < lr_proj.out_features <= MAX_LR_OUTPUTS and sum(m.out_features for m in mods[2:]) <= MAX_BF16_OUTPUTS):
+        maps = [t for m in (lr_proj, momentum, gate) for t in ((None, None) if m is None else (m.weight, m.bias))]
+        qkv, lr_raw, *rest = _lib.host().layer_in(x, to_qkv.weight, *maps)
+        return qkv, lr_raw, None if momentum is None else rest[0], None if gate is None else rest[-1]
+    qkv = _linear(to_qkv, x)
+    with torch.autocast(device_type="cuda", enabled=False):      # the reference keeps the rates out of autocast (:247-249)
+        lr_raw = lr_proj(x)
+    return qkv, lr_raw, None if momentum is None else momentum(x), None if gate is None else gate(x)
+
+
 def _fast_weights(layer, B):
     """[nh, ...] parameters -> [(B nh), ...] (bidirectional_lact_layer.py:259-261)."""
     return tuple(w.repeat(B, 1, 1) for w in (layer.w0, layer.w1, layer.w2))
@@ -247,14 +312,13 @@ class BidirectionalLaCTSwiGLU(nn.Module):
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         """x: [b, l, d] -> [b, l, d]"""
         B = x.shape[0]
-        q, k, v = _PreFn.apply(self.to_qkv(x), self.num_heads, self.head_dim, self.qk_l2_norm)
-        with torch.autocast(device_type="cuda", enabled=False):      # the reference keeps the rates out of autocast (:247-249)
-            lr_raw = self.lr_proj(x)
-        lr0, lr1, lr2 = _LrFn.apply(lr_raw, None, self.num_heads, self.base_lr_inv)
+        qkv, lr_raw, _, _ = _input_projections(x, self.to_qkv, self.lr_proj)
+        q, k, v = _pre(qkv, self.num_heads, self.head_dim, self.qk_l2_norm)
+        lr0, lr1, lr2 = _rates(lr_raw, None, self.num_heads, self.base_lr_inv)
         w0, w1, w2 = _fast_weights(self, B)
         o = bidirectional_lact_swiglu(w0, w1, w2, q, k, v, lr0, lr1, lr2, self.use_muon)
         weight, use_norm, eps = _norm_args(self.o_norm)
-        return self.o_proj(_PostFn.apply(o, weight, None, B, self.num_heads, use_norm, eps))
+        return _linear(self.o_proj, _post(o, weight, None, B, self.num_heads, use_norm, eps))
 
 
 MAX_TOKEN_STRIDE = 1 << 24     # elements; the kernels' offsets inside a tile are 32-bit
@@ -427,11 +491,11 @@ class CausalLaCTSwiGLUWithSlidingWindowAttn(nn.Module):
         """x: [b, l, d] -> [b, l, d]"""
         B, L, _ = x.shape
         H = self.num_ttt_heads
-        q, k, v, aq, ak, av = _PreAttnFn.apply(self.to_qkv(x), self.qk_scale, self.qk_offset, H, self.head_dim, True)
-        with torch.autocast(device_type="cuda", enabled=False):
-            lr_raw = self.lr_proj(x)
-        mom_raw = self.momentum_proj[0](x) if self.use_momentum else None      # the Sigmoid of the Sequential is in the kernel
-        res = _LrFn.apply(lr_raw, mom_raw, H, self.base_lr_inv)
+        # the Sigmoid of momentum_proj is in the kernel behind this
+        qkv, lr_raw, mom_raw, gate_raw = _input_projections(x, self.to_qkv, self.lr_proj, self.momentum_proj[0] if self.use_momentum else None,
+                                                            self.ttt_scale_proj)
+        q, k, v, aq, ak, av = _pre_attn(qkv, self.qk_scale, self.qk_offset, H, self.head_dim, True)
+        res = _rates(lr_raw, mom_raw, H, self.base_lr_inv)
         lr0, lr1, lr2 = res[:3]
         momentum = res[3] if self.use_momentum else None
         w0, w1, w2 = _fast_weights(self, B)
@@ -440,7 +504,7 @@ class CausalLaCTSwiGLUWithSlidingWindowAttn(nn.Module):
         sh = lambda t: t.reshape(B, L, self.num_attn_heads, self.attn_head_dim)
         attn = sliding_window_attention(sh(aq), sh(ak), sh(av), self.window_size).reshape(B, L, -1)
         weight, use_norm, eps = _norm_args(self.o_norm)
-        return self.o_proj(_PostFn.apply(o, weight, self.ttt_scale_proj(x), B, H, use_norm, eps, attn))
+        return _linear(self.o_proj, _post(o, weight, gate_raw, B, H, use_norm, eps, attn))
 
 
 class FastWeightGluMLPMultihead(nn.Module):
@@ -471,10 +535,14 @@ class FastWeightGluMLPMultihead(nn.Module):
     def forward(self, x: torch.Tensor, info={}, *args):
         """x: [b, l, d] -> ([b, l', d], {"w0", "w1", "w2"}) with l' the rows of the apply steps in program order."""
         B = x.shape[0]
-        q, k, v = _PreFn.apply(self.to_qkv(x), self.num_heads, self.head_dim, True)          # :203-210
-        with torch.autocast(device_type="cuda", enabled=False):                              # :212-213
-            lr_raw = self.lr_fc(x.float())
-        lr0, lr1, lr2 = _LrFn.apply(lr_raw, None, self.num_heads, self.base_lr_inv, True)    # '(lrs h d)', :215-219
+        if x.dtype == torch.float32:                                                         # :203-213
+            qkv, lr_raw, _, _ = _input_projections(x, self.to_qkv, self.lr_fc)
+        else:
+            qkv = _linear(self.to_qkv, x)
+            with torch.autocast(device_type="cuda", enabled=False):
+                lr_raw = self.lr_fc(x.float())
+        q, k, v = _pre(qkv, self.num_heads, self.head_dim, True)
+        lr0, lr1, lr2 = _rates(lr_raw, None, self.num_heads, self.base_lr_inv, True)    # '(lrs h d)', :215-219
         if "w0" in info:                                                                      # :221-229
             assert "w1" in info and "w2" in info
             w0, w1, w2 = info["w0"], info["w1"], info["w2"]
@@ -483,5 +551,5 @@ class FastWeightGluMLPMultihead(nn.Module):
         o, w0, w1, w2 = fast_weight_swish_glu_weight_norm_mini_batch_apply(
             w0, w1, w2, q, k, v, lr0, lr1, lr2, info["ttt_op_order"], muon_update_steps=self.muon_update_steps)
         weight, use_norm, eps = _norm_args(self.o_norm)
-        y = _PostFn.apply(o, weight, None, B, self.num_heads, use_norm, eps)
-        return self.c_proj(y), {"w0": w0, "w1": w1, "w2": w2}
+        y = _post(o, weight, None, B, self.num_heads, use_norm, eps)
+        return _linear(self.c_proj, y), {"w0": w0, "w1": w1, "w2": w2}

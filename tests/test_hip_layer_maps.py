@@ -1,0 +1,155 @@
+"""The linear maps of a layer's input and output under bf16 autocast: the fused functions of the host module against float64,
+against the modules they stand in for, and their way back to the modules."""
+import pytest
+import torch
+import torch.nn as nn
+import torch.nn.functional as F
+
+from lact_amd import _lib
+from lact_amd import layers as HL
+from oracle.lact_oracle import rel_l2
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def maps(dim, n_lr, n_mom, n_gate, bias, seed=3):
+    torch.manual_seed(seed)
+    mods = [nn.Linear(dim, 3 * dim, bias=False), nn.Linear(dim, n_lr, bias=bias)] + [nn.Linear(dim, n) if n else None for n in (n_mom, n_gate)]
+    return [m.to(DEV) if m is not None else None for m in mods]
+
+
+# numbers of outputs at the edges of the kernels' groups of four (8, 12, 16, 24; 8, 16), token counts at the edges of a wave's four,
+# a block's 16 and 32 and of the weight gradient's 64 and 128 (16 tokens a wave below 512 blocks, 32 from there), channels at
+# the edges of a wave's 256
+@pytest.mark.parametrize("B,L,dim,n_lr,n_mom,n_gate,bias", [
+    (1, 1, 8, 1, 1, 0, False), (1, 63, 256, 8, 0, 1, True), (2, 32, 264, 9, 4, 4, False), (1, 65, 520, 12, 8, 1, True),
+    (3, 43, 768, 13, 0, 0, True), (1, 129, 1032, 16, 8, 8, False), (2, 2100, 384, 24, 16, 0, False), (1, 16400, 1024, 17, 5, 5, True),
+])
+def test_input_maps_against_float64(B, L, dim, n_lr, n_mom, n_gate, bias):
+    """Sums of rounded operands in fp32: 2^-9 relative per rounding of x, of a weight, of a gradient and of a result, so a few 1e-3
+    in norm (5e-3 asserted; 1e-2 for the few values of a bias gradient); what stays in fp32 (the rates and their gradients) 1e-5."""
+    print("[gpu-test] input maps", B, L, dim, n_lr, n_mom, n_gate, bias, flush=True)
+    mods = maps(dim, n_lr, n_mom, n_gate, bias)
+    x = torch.randn(B, L, dim, device=DEV, requires_grad=True)
+    params = [p for m in mods if m is not None for p in m.parameters()]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert HL._fused_linears(x, *[m for m in mods if m is not None])
+        outs = [o for o in HL._input_projections(x, *mods) if o is not None]
+    go = [torch.randn(o.shape, device=DEV).to(o.dtype) for o in outs]
+    grads = torch.autograd.grad(outs, [x] + params, go)
+    xd, pd = x.detach().double().requires_grad_(True), [p.detach().double().requires_grad_(True) for p in params]
+    it, ref = iter(pd), []
+    for m in mods:
+        if m is not None:
+            ref.append(F.linear(xd, next(it), next(it) if m.bias is not None else None))
+    ref_grads = torch.autograd.grad(ref, [xd] + pd, [g.double() for g in go])
+    names = ["qkv", "lr"] + ["mom"] * (n_mom > 0) + ["gate"] * (n_gate > 0)
+    for n, a, r in zip(names, outs, ref):
+        assert rel_l2(a, r) < (1e-5 if n == "lr" else 5e-3), n
+    exact = {id(p) for p in mods[1].parameters()}
+    for p, g, r in zip([x] + params, grads, ref_grads):
+        assert g.dtype == torch.float32 and g.shape == p.shape
+        assert rel_l2(g, r) < (1e-5 if id(p) in exact else 1e-2 if p.dim() == 1 else 5e-3), p.shape
+
+
+# token counts around one K-step of 64 and around the split's 1024 tokens, tiles of 192 (48 or more of them) and of 128 with ragged
+# edges
+@pytest.mark.parametrize("T,m,n", [(64, 8, 8), (63, 72, 136), (65, 128, 128), (1000, 136, 264), (2049, 768, 384), (3333, 1344, 1344), (2048, 4608, 192), (5000, 1000, 512)])
+def test_weight_gradient_against_float64(T, m, n):
+    """Products of bf16 values are exact in fp32; a sum of T of them in fp32 blocks of 16 is good for sqrt(T) 2^-24: 1e-5."""
+    print("[gpu-test] weight gradient", T, m, n, flush=True)
+    lin = nn.Linear(n, m, bias=False).to(DEV)
+    x = torch.randn(1, T, n, device=DEV).bfloat16().requires_grad_(True)
+    go = torch.randn(1, T, m, device=DEV).bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = HL._linear(lin, x)
+    dx, dw = torch.autograd.grad(y, [x, lin.weight], go)
+    wb = lin.weight.detach().bfloat16().double()
+    assert dw.dtype == torch.float32 and rel_l2(dw, go[0].double().t() @ x.detach()[0].double()) < 1e-5
+    assert dx.dtype == torch.bfloat16 and rel_l2(dx, go.double() @ wb) < 4e-3 and rel_l2(y, x.detach().double() @ wb.t()) < 4e-3
+
+
+def test_partial_gradients_and_unused_outputs():
+    """Frozen parameters get no gradient, outputs that nobody uses count as zero, and nothing needs an input that is a leaf of data."""
+    print("[gpu-test] partial gradients", flush=True)
+    mods = maps(128, 6, 2, 2, True)
+    mods[0].weight.requires_grad_(False)
+    mods[2].bias.requires_grad_(False)
+    x = torch.randn(2, 50, 128, device=DEV)
+    wanted = [p for m in mods for p in m.parameters() if p.requires_grad]
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        outs = HL._input_projections(x, *mods)
+        full = torch.autograd.grad(sum(o.float().sum() for o in outs[1:]), wanted, retain_graph=True)
+        some = torch.autograd.grad(outs[1].sum(), wanted, allow_unused=True)
+    assert all(g is not None for g in full)
+    assert torch.equal(some[0], full[0]) and torch.equal(some[1], full[1])
+    assert all(g is None or not g.any() for g in some[2:])
+    with torch.no_grad(), torch.autocast("cuda", dtype=torch.bfloat16):
+        again = HL._input_projections(x, *mods)
+    assert all(torch.equal(a, b) for a, b in zip(outs, again)) and not again[0].requires_grad
+
+
+def test_second_derivatives_of_the_maps_are_refused():
+    print("[gpu-test] second derivative of the maps", flush=True)
+    mods = maps(64, 3, 1, 1, False)
+    x = torch.randn(1, 70, 64, device=DEV, requires_grad=True)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        for outs in (HL._input_projections(x, *mods), [HL._linear(mods[0], x)]):
+            g = torch.autograd.grad(sum(o.float().sum() for o in outs), x, create_graph=True)[0]
+            with pytest.raises(RuntimeError, match="once_differentiable"):
+                torch.autograd.grad(g.square().sum() + x.sum(), x)
+
+
+def test_modules_are_called_where_someone_may_look():
+    """Hooks, subclasses, replaced forwards, other types, no autocast: the modules run, as they did."""
+    print("[gpu-test] modules that are looked at", flush=True)
+    x = torch.randn(1, 70, 64, device=DEV)
+
+    def fused(mods, x=x, dtype=torch.bfloat16, enabled=True):
+        with torch.autocast("cuda", dtype=dtype, enabled=enabled):
+            return HL._fused_linears(x, *mods)
+    plain = [nn.Linear(64, 8).to(DEV)]
+    assert fused(plain) and not fused(plain, dtype=torch.float16) and not fused(plain, enabled=False) and not fused(plain, x=x[0])
+    seen = []
+    hooked = nn.Linear(64, 8).to(DEV)
+    hooked.register_forward_hook(lambda m, a, o: seen.append(o))
+    sub = type("Sub", (nn.Linear,), {})(64, 8).to(DEV)
+    replaced = nn.Linear(64, 8).to(DEV)
+    replaced.forward = lambda t: t
+    half = nn.Linear(64, 8).to(DEV).bfloat16()
+    assert not any(fused([m]) for m in (hooked, sub, replaced, half))
+    layer = HL.BidirectionalLaCTSwiGLU(64, 32, use_muon=False).to(DEV)
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = layer(x)
+        layer.lr_proj.register_forward_hook(lambda m, a, o: seen.append(o))
+        close = layer(x)
+        assert len(seen) == 1 and rel_l2(close, y) < 1e-2
+        assert not torch.func.functional_call(layer, {n: p.detach() for n, p in layer.named_parameters()}, (x,)).requires_grad
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_native_and_python_functions_agree(dtype):
+    """The layer functions of the host module and their Python counterparts launch the same kernels: same bits, same gradients (the
+    RMSNorm weight's sums over partial rows in another order: 1e-5)."""
+    print("[gpu-test] native functions", dtype, flush=True)
+    B, L, H, hd = 2, 37, 3, 32
+    r = lambda *s, d=dtype: torch.randn(*s, device=DEV).to(d).requires_grad_(True)
+    qkv, scale, offset = r(B, L, 3 * H * hd), r(H * hd, 2, d=torch.float32), r(H * hd, 2, d=torch.float32)
+    lr, mom = r(B, L, 3 * H, d=torch.float32), r(B, L, H)
+    o, w, gate, add = r(B * H, L, hd), r(hd, d=torch.float32), r(B, L, H), r(B, L, H * hd)
+    host = _lib.host()
+    for native, python, args, consts in (
+            (host.layer_pre, HL._PreFn.apply, (qkv,), (H, hd, True)),
+            (host.layer_pre_attn, HL._PreAttnFn.apply, (qkv, scale, offset), (H, hd, True)),
+            (host.layer_lr, HL._LrFn.apply, (lr, mom), (H, 0.3, True)),
+            (lambda a, b, c, d, *k: host.layer_post(a, b, c, *k, d), lambda a, b, c, d, *k: HL._PostFn.apply(a, b, c, *k, d), (o, w, gate, add), (B, H, True, 1e-5))):
+        res = []
+        for fn in (native, python):
+            out = fn(*args, *consts)
+            out = [out] if isinstance(out, torch.Tensor) else list(out)
+            torch.manual_seed(5)
+            res.append(out + list(torch.autograd.grad(out, args, [torch.randn_like(t) for t in out])))
+        for a, b in zip(*res):
+            assert a.dtype == b.dtype and a.shape == b.shape
+            assert torch.equal(a, b) or (a.shape == w.shape and rel_l2(a, b) < 1e-5)

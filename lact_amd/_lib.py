@@ -39,7 +39,8 @@ EXPORTS = ("lact_last_error", "lact_version", "lact_query_sizes", "lact_forward"
            "lact_newton_schulz_workspace_bytes", "lact_newton_schulz", "lact_newton_schulz_static_capacity",
            "lact_newton_schulz_static", "lact_newton_schulz_backward_workspace_bytes", "lact_newton_schulz_backward",
            "lact_check_async_error", "lact_mfma_calibration", "lact_set_option", "lact_profile_enable",
-           "lact_profile_report", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward",
+           "lact_profile_report", "lact_layer_in_forward", "lact_layer_in_backward", "lact_layer_in_backward_workspace_bytes",
+           "lact_weight_grad", "lact_weight_grad_workspace_bytes", "lact_layer_sum_rows", "lact_layer_pre_forward", "lact_layer_pre_backward", "lact_layer_lr_forward",
            "lact_layer_lr_backward", "lact_layer_post_forward", "lact_layer_post_dw_rows", "lact_layer_post_backward",
            "lact_window_attention_forward", "lact_window_attention_backward", "lact_layer_pre_attn_forward",
            "lact_layer_pre_attn_part_rows", "lact_layer_pre_attn_backward", "lact_layer_post_add_forward")

@@ -1802,27 +1802,50 @@ int lact_set_option(int32_t option, int32_t value) {
 namespace {
 int layer_geom(int32_t B, int32_t L, int32_t H, int32_t hd, LayerGeom* g) {
   if (B <= 0 || L <= 0 || H <= 0 || hd <= 0) return fail("layer: B, L, H, hd must be positive");
-  if (hd % 4 || hd > 256 * LAYER_VEC_MAX) return fail("layer: head dim must be a multiple of 4 and at most 1024");
+  if (hd % 4 || hd > LAYER_HD_MAX) return fail("layer: head dim must be a multiple of 4 and at most 1024");
   g->B = B; g->L = L; g->H = H; g->hd = hd;
   return 0;
 }
-unsigned layer_row_blocks(const LayerGeom& g) { return (unsigned)(((long long)g.B * g.L * g.H + 3) / 4); }
-unsigned layer_post_bwd_blocks(const LayerGeom& g) { return std::min(layer_row_blocks(g), 2048u); }
 }  // namespace
 
 }  // extern "C"
 namespace {
+// Calls f(G, NV) for the lanes and chunks (RowLanes) that hd fills best; in fp32 with fewer kernels to choose from.
+template <typename T, class F>
+void layer_lanes(int hd, F f) {
+#define LACT_LANES(limit, G, NV) if (hd <= limit) return f(std::integral_constant<int, G>(), std::integral_constant<int, NV>());
+  if constexpr (std::is_same<T, uint16_t>::value) {
+    LACT_LANES(64, 16, 1) LACT_LANES(96, 8, 3) LACT_LANES(128, 16, 2) LACT_LANES(192, 16, 3) LACT_LANES(384, 32, 3) LACT_LANES(768, 64, 3)
+  } else {
+    LACT_LANES(128, 16, 2)
+  }
+  LACT_LANES(512, 32, 4) LACT_LANES(LAYER_HD_MAX, 64, 4)
+#undef LACT_LANES
+}
+int layer_rows_per_wave(int act_dtype, int hd) {
+  int n = 1;
+  auto rows = [&](auto g, auto) { n = 64 / decltype(g)::value; };
+  if (act_dtype == LACT_BF16) layer_lanes<uint16_t>(hd, rows);
+  else layer_lanes<float>(hd, rows);
+  return n;
+}
+unsigned layer_row_blocks(int act_dtype, const LayerGeom& g) {
+  const long long n = 4LL * layer_rows_per_wave(act_dtype, g.hd);
+  return (unsigned)(((long long)g.B * g.L * g.H + n - 1) / n);
+}
+// (the number of partial rows that the caller asks for knows neither the type nor hd)
+unsigned layer_post_bwd_blocks(const LayerGeom& g) { return (unsigned)std::min(((long long)g.B * g.L * g.H + 3) / 4, 1024LL); }
 template <typename T, bool BWD, bool ATT>
-void launch_layer_pre_t(const char* name, const char* site, const LayerPreParams& p, int blocks_per_head, hipStream_t s) {
-  const dim3 grid((unsigned)(blocks_per_head * p.g.H)), block(256);
-  if (p.g.hd <= 256) LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, 1>), grid, block, s, p);
-  else if (p.g.hd <= 512) LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, 2>), grid, block, s, p);
-  else LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, LAYER_VEC_MAX>), grid, block, s, p);
+void launch_layer_pre_t(const char* name, const char* site, LayerPreParams p, int blocks_per_head, hipStream_t s) {
+  layer_lanes<T>(p.g.hd, [&](auto g, auto nv) {
+    constexpr int G = decltype(g)::value, NV = decltype(nv)::value;
+    p.tokens_per_pass = 4 * (64 / G) * blocks_per_head;
+    LACT_LAUNCH(name, site, 0.0, (k_layer_pre<T, BWD, ATT, G, NV>), dim3((unsigned)(blocks_per_head * p.g.H)), dim3(256), s, p);
+  });
 }
 template <bool BWD>
-int launch_layer_pre(int act_dtype, LayerPreParams& p, int blocks_per_head, hipStream_t s) {
+int launch_layer_pre(int act_dtype, const LayerPreParams& p, int blocks_per_head, hipStream_t s) {
   const bool att = p.att[0] || p.datt[0];
-  p.tokens_per_pass = 4 * blocks_per_head;
   const char* name = BWD ? "k_layer_pre_bwd" : "k_layer_pre";
   const char* site = BWD ? "layer_pre_bwd" : "layer_pre";
   if (act_dtype == LACT_BF16) {
@@ -1836,10 +1859,20 @@ int launch_layer_pre(int act_dtype, LayerPreParams& p, int blocks_per_head, hipS
   }
   return 0;
 }
-int layer_token_blocks(const LayerGeom& g) { return (int)(((long long)g.B * g.L + 3) / 4); }   // one token per wave
+template <typename T, bool BWD>
+void launch_layer_post(const LayerPostParams& p, unsigned blocks, hipStream_t s) {
+  layer_lanes<T>(p.g.hd, [&](auto g, auto nv) {
+    constexpr int G = decltype(g)::value, NV = decltype(nv)::value;
+    LACT_LAUNCH(BWD ? "k_layer_post_bwd" : "k_layer_post", BWD ? "layer_post_bwd" : "layer_post", 0.0, (k_layer_post<T, BWD, G, NV>), dim3(blocks), dim3(256), s, p);
+  });
+}
+int layer_token_blocks(int act_dtype, const LayerGeom& g) {   // one pass of every wave
+  const long long n = 4LL * layer_rows_per_wave(act_dtype, g.hd);
+  return (int)(((long long)g.B * g.L + n - 1) / n);
+}
 // blocks per head of the backward with parameter gradients: enough waves to hide the memory latency (16 per compute
 // unit), few enough that the partial sums stay small beside the activations
-int layer_pre_attn_blocks(const LayerGeom& g) { return std::max(1, std::min(layer_token_blocks(g), 1024 / g.H)); }
+int layer_pre_attn_blocks(const LayerGeom& g) { return (int)std::max(1LL, std::min(((long long)g.B * g.L + 3) / 4, 1024LL / g.H)); }
 }  // namespace
 extern "C" {
 
@@ -1850,7 +1883,7 @@ int lact_layer_pre_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, i
   if (layer_geom(B, L, H, hd, &p.g)) return -1;
   if (check_ptrs({qkv, q, k, v}, "layer pre tensors")) return -1;
   p.l2norm = l2norm; p.qkv = qkv; p.out[0] = q; p.out[1] = k; p.out[2] = v;
-  if (launch_layer_pre<false>(act_dtype, p, layer_token_blocks(p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
+  if (launch_layer_pre<false>(act_dtype, p, layer_token_blocks(act_dtype, p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
   LACT_CHECK_LAUNCH();
   return 0;
 }
@@ -1862,7 +1895,7 @@ int lact_layer_pre_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, 
   if (layer_geom(B, L, H, hd, &p.g)) return -1;
   if (check_ptrs({qkv, dq, dk, dv, dqkv}, "layer pre backward tensors")) return -1;
   p.l2norm = l2norm; p.qkv = qkv; p.dout[0] = dq; p.dout[1] = dk; p.dout[2] = dv; p.dqkv = dqkv;
-  if (launch_layer_pre<true>(act_dtype, p, layer_token_blocks(p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
+  if (launch_layer_pre<true>(act_dtype, p, layer_token_blocks(act_dtype, p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
   LACT_CHECK_LAUNCH();
   return 0;
 }
@@ -1876,7 +1909,7 @@ int lact_layer_pre_attn_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t
   if (check_ptrs({qkv, qk_scale, qk_offset, q, k, v, aq, ak, av}, "layer pre tensors")) return -1;
   p.l2norm = l2norm; p.qkv = qkv; p.out[0] = q; p.out[1] = k; p.out[2] = v;
   p.att[0] = aq; p.att[1] = ak; p.att[2] = av; p.qk_scale = qk_scale; p.qk_offset = qk_offset; p.round_product = round_product;
-  if (launch_layer_pre<false>(act_dtype, p, layer_token_blocks(p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
+  if (launch_layer_pre<false>(act_dtype, p, layer_token_blocks(act_dtype, p.g), reinterpret_cast<hipStream_t>(stream))) return -1;
   LACT_CHECK_LAUNCH();
   return 0;
 }
@@ -2022,8 +2055,8 @@ int lact_layer_post_add_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t
   if (check_ptrs({o, y}, "layer post tensors")) return -1;
   p.eps = eps; p.use_norm = use_norm; p.o = o; p.w = norm_weight; p.gate_raw = gate_raw; p.add = add; p.y = y;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_post", "layer_post", 0.0, (k_layer_post<uint16_t, false>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
-  else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_post", "layer_post", 0.0, (k_layer_post<float, false>), dim3(layer_row_blocks(p.g)), dim3(256), s, p);
+  if (act_dtype == LACT_BF16) launch_layer_post<uint16_t, false>(p, layer_row_blocks(act_dtype, p.g), s);
+  else if (act_dtype == LACT_F32) launch_layer_post<float, false>(p, layer_row_blocks(act_dtype, p.g), s);
   else return fail("act_dtype must be LACT_BF16 or LACT_F32");
   LACT_CHECK_LAUNCH();
   return 0;
@@ -2051,8 +2084,8 @@ int lact_layer_post_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H,
   p.eps = eps; p.use_norm = use_norm; p.o = o; p.w = norm_weight; p.gate_raw = gate_raw;
   p.dy = dy; p.d_o = d_o; p.dgate_raw = dgate_raw; p.dw_part = use_norm ? dw_part : nullptr;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (act_dtype == LACT_BF16) LACT_LAUNCH("k_layer_post_bwd", "layer_post_bwd", 0.0, (k_layer_post<uint16_t, true>), dim3(layer_post_bwd_blocks(p.g)), dim3(256), s, p);
-  else if (act_dtype == LACT_F32) LACT_LAUNCH("k_layer_post_bwd", "layer_post_bwd", 0.0, (k_layer_post<float, true>), dim3(layer_post_bwd_blocks(p.g)), dim3(256), s, p);
+  if (act_dtype == LACT_BF16) launch_layer_post<uint16_t, true>(p, layer_post_bwd_blocks(p.g), s);
+  else if (act_dtype == LACT_F32) launch_layer_post<float, true>(p, layer_post_bwd_blocks(p.g), s);
   else return fail("act_dtype must be LACT_BF16 or LACT_F32");
   LACT_CHECK_LAUNCH();
   return 0;

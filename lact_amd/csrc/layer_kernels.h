@@ -9,7 +9,7 @@
 //   post:  o [(B H), L, hd] -> y [B, L, H*hd]                    per-head RMSNorm (affine), optional silu gate per
 //          token and head, head layout, optionally plus the attention branch  (bidirectional_lact_layer.py:268-270, causal_...:351-357)
 //
-// and their backward passes.  One wave per (token, head) row of hd elements; 16 bytes per lane.
+// and their backward passes.  A group of lanes of a wave per (token, head) row of hd elements.
 // Element type T = uint16_t (bf16) or float; all statistics in fp32.
 #pragma once
 #include "common.h"
@@ -27,7 +27,37 @@ __device__ __forceinline__ float silu_grad_f(float x) {
   return s * (1.f + x * (1.f - s));
 }
 
-constexpr int LAYER_VEC_MAX = 4;   // a lane keeps up to 4 x 4 elements of its row (hd <= 1024)
+constexpr int LAYER_HD_MAX = 1024;   // 64 lanes, 4 chunks of 4 elements each
+
+// How a wave's lanes share rows of hd elements: G lanes per row (64 / G rows a wave), NV chunks of 4 * G elements each, so that
+// hd fills them: 96 = 8 lanes x 3 chunks, 384 = 32 x 3.  With all 64 lanes on one row 24 of them worked at hd = 96, three
+// quarters of the chunks at 384.
+template <int G, int NV>
+struct RowLanes {
+  static constexpr int ROWS = 64 / G;
+  __device__ static __forceinline__ int group() { return (threadIdx.x & 63) / G; }
+  __device__ static __forceinline__ int col(int i) { return (threadIdx.x & (G - 1)) * 4 + i * 4 * G; }
+  // Sum over the row of f(i, j), in the order of one lane per four elements of every 256: per such lane over its chunks, then
+  // over the lanes by halves.  The same bits for every split, which Newton-Schulz behind the L2 norms would amplify.
+  template <class F>
+  __device__ static __forceinline__ float sum(F f) {
+    float part[ROWS];
+#pragma unroll
+    for (int m = 0; m < ROWS; ++m) part[m] = 0.f;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) part[i % ROWS] = f(i, j, part[i % ROWS]);
+#pragma unroll
+    for (int d = ROWS / 2; d > 0; d /= 2)
+#pragma unroll
+      for (int m = 0; m < d; ++m) part[m] += part[m + d];
+    float v = part[0];
+#pragma unroll
+    for (int o = G / 2; o > 0; o /= 2) v += __shfl_xor(v, o, 64);
+    return v;
+  }
+};
 
 // ---- pre ------------------------------------------------------------------------------------------
 struct LayerPreParams {
@@ -49,23 +79,25 @@ struct LayerPreParams {
   int tokens_per_pass;        // tokens between two of a wave
 };
 
-// Grid: H * m blocks of 256 threads; a wave handles q, k and v of one head and the tokens wave, wave + tokens_per_pass, ...
-// NV: chunks of 256 elements that cover hd.
-// HBM bound: one read of qkv and of the gradients, one write of every output; all loads of a token are issued before the
-// first of them is used (the norms otherwise put three round trips in line).  The attention's inputs ride along because
-// the projection's output is in registers here: as tensor operations of their own (slices, rescaling, and in the backward
-// three zero-padded slice gradients to add up) they took 0.9 ms of a training step at 16384 tokens of 1536 channels.
-template <typename T, bool BWD, bool ATT, int NV>
+// Grid: H * m blocks of 256 threads; a wave handles q, k and v of one head and 64 / G tokens at a time.
+// HBM and vector-ALU issue bound it alike: one read of qkv and of the gradients, one write of every output; all loads of a token
+// are issued before the first of them is used (the norms otherwise put three round trips in line).  The attention's inputs ride
+// along because the projection's output is in registers here: as tensor operations of their own (slices, rescaling, and in the
+// backward three zero-padded slice gradients to add up) they took 0.9 ms of a training step at 16384 tokens of 1536 channels.
+// bf16, us forward / backward, with all 64 lanes on a row before: 16384 tokens, 4 heads of 384 (ATT) 134 / 172 (145 / 234: 450 and
+// 600 MB); 7500 tokens, 8 heads of 96 19 / 34 (37 / 65: 69 and 104 MB).
+template <typename T, bool BWD, bool ATT, int G, int NV>
 __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  using RL = RowLanes<G, NV>;
+  const int wave = threadIdx.x >> 6, grp = RL::group();
   const int hd = p.g.hd, h = blockIdx.x % p.g.H;
   const size_t dim = (size_t)p.g.H * hd;
   float sc[2][NV][4], off[2][NV][4];           // ATT: this lane's channels of the rescaling
-  float acc[4][NV][4];                         // ATT && BWD: this wave's share of the parameter gradients
+  float acc[4][NV][4];                         // ATT && BWD: this lane's share of the parameter gradients
   if (ATT) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-      const int c = min(lane * 4 + i * 256, hd - 4);
+      const int c = min(RL::col(i), hd - 4);
       const float* ps = p.qk_scale + ((size_t)h * hd + c) * 2;
       const float4 s0 = *reinterpret_cast<const float4*>(ps), s1 = *reinterpret_cast<const float4*>(ps + 4);
       sc[0][i][0] = s0.x; sc[1][i][0] = s0.y; sc[0][i][1] = s0.z; sc[1][i][1] = s0.w;
@@ -83,7 +115,7 @@ __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
       }
     }
   }
-  for (long long bl = (long long)(blockIdx.x / p.g.H) * 4 + wave; bl < (long long)p.g.B * p.g.L; bl += p.tokens_per_pass) {
+  for (long long bl = ((long long)(blockIdx.x / p.g.H) * 4 + wave) * RL::ROWS + grp; bl < (long long)p.g.B * p.g.L; bl += p.tokens_per_pass) {
     const int l = (int)(bl % p.g.L);
     const long long b = bl / p.g.L;
     const size_t oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd, ai = (size_t)bl * dim + (size_t)h * hd;
@@ -92,7 +124,7 @@ __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
     for (int which = 0; which < 3; ++which)
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const int c = lane * 4 + i * 256;
+        const int c = RL::col(i);
         if (c < hd) {
           Elem<T>::load4(reinterpret_cast<const T*>(p.qkv) + ((size_t)(bl * 3 + which) * p.g.H + h) * hd + c, xs[which][i]);
           if (BWD) Elem<T>::load4(reinterpret_cast<const T*>(p.dout[which]) + oi + c, gs[which][i]);
@@ -108,27 +140,22 @@ __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
       float (&x)[NV][4] = xs[which];
       float (&g)[NV][4] = gs[which];
       float y[NV][4];
-      float ss = 0.f, dot = 0.f;
 #pragma unroll
       for (int i = 0; i < NV; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          y[i][j] = Elem<T>::rnd(silu_f(x[i][j]));       // silu output is a tensor of type T in the reference
-          ss += y[i][j] * y[i][j];
-          if (BWD) dot += g[i][j] * y[i][j];
-        }
+        for (int j = 0; j < 4; ++j) y[i][j] = Elem<T>::rnd(silu_f(x[i][j]));       // silu output is a tensor of type T in the reference
       float n = 0.f;
-      if (norm) n = sqrtf(wave_sum(ss));
+      if (norm) n = sqrtf(RL::sum([&](int i, int j, float s) { return s + y[i][j] * y[i][j]; }));
       const float inv = norm ? 1.f / (n + 1e-5f) : 1.f;
       float c1 = 0.f;
       if (BWD && norm) {
         // z = y / (n + eps):  dy = dz / (n + eps) - y <dz, y> / (n (n + eps)^2);  dx = dy silu'(x)
-        dot = wave_sum(dot);
+        const float dot = RL::sum([&](int i, int j, float s) { return s + g[i][j] * y[i][j]; });
         c1 = n > 0.f ? dot / (n * (n + 1e-5f) * (n + 1e-5f)) : 0.f;
       }
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
-        const int c = lane * 4 + i * 256;
+        const int c = RL::col(i);
         if (c >= hd) continue;
         if (!BWD) {
           Elem<T>::store4(reinterpret_cast<T*>(p.out[which]) + oi + c, y[i][0] * inv, y[i][1] * inv, y[i][2] * inv, y[i][3] * inv);
@@ -166,17 +193,25 @@ __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
       }
     }
   }
-  if (ATT && BWD) {      // the four waves' shares, in a fixed order
-    __shared__ float red[4][NV * 256];
+  if (ATT && BWD) {      // the shares of the wave's rows, then the four waves', in a fixed order
+    __shared__ float red[4][NV * 4 * G];
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+      for (int i = 0; i < NV; ++i)
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+          for (int o = G; o < 64; o *= 2) acc[a][i][j] += __shfl_xor(acc[a][i][j], o, 64);
     for (int w = 0; w < 4; ++w) {
-      if (wave == w) {
+      if (wave == w && grp == 0) {
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
           for (int i = 0; i < NV; ++i)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-              float* r = &red[a][lane * 4 + i * 256 + j];
+              float* r = &red[a][RL::col(i) + j];
               *r = w == 0 ? acc[a][i][j] : *r + acc[a][i][j];
             }
       }
@@ -255,22 +290,25 @@ struct LayerPostParams {
   float* dw_part;             // [gridDim.x][hd] partial sums of the weight gradient, or null
 };
 // Backward: each wave walks rows row0, row0 + stride, ... so that its partial weight gradient stays in registers.
-template <typename T, bool BWD>
+// HBM bound.  bf16, us forward / backward, with all 64 lanes and four chunks on a row before: 16384 tokens, 4 heads of 384 42 / 46
+// (53 / 71: 150 MB each); 7500 tokens, 8 heads of 96 9.3 / 12.6 (22 / 36).
+template <typename T, bool BWD, int G, int NV>
 __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const long long nwaves = (long long)gridDim.x * 4;
+  using RL = RowLanes<G, NV>;
+  const int wave = threadIdx.x >> 6, grp = RL::group();
+  const long long step = (long long)gridDim.x * 4 * RL::ROWS;
   const int hd = p.g.hd;
-  float wv[LAYER_VEC_MAX][4], dwacc[LAYER_VEC_MAX][4];
+  float wv[NV][4], dwacc[NV][4];
 #pragma unroll
-  for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-    const int c = lane * 4 + i * 256;
+  for (int i = 0; i < NV; ++i) {
+    const int c = RL::col(i);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       wv[i][j] = (p.w && c < hd) ? p.w[c + j] : 1.f;
       dwacc[i][j] = 0.f;
     }
   }
-  for (long long row = (long long)blockIdx.x * 4 + wave; row < p.g.rows(); row += nwaves) {
+  for (long long row = ((long long)blockIdx.x * 4 + wave) * RL::ROWS + grp; row < p.g.rows(); row += step) {
     const int h = (int)(row % p.g.H);
     const long long bl = row / p.g.H;
     const int l = (int)(bl % p.g.L);
@@ -278,19 +316,20 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
     const size_t oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd;
     const size_t yi = ((size_t)bl * p.g.H + h) * hd;
     const T* src = reinterpret_cast<const T*>(p.o) + oi;
-    float x[LAYER_VEC_MAX][4];
-    float ss = 0.f;
+    const T* other = BWD ? reinterpret_cast<const T*>(p.dy) + yi : p.add ? reinterpret_cast<const T*>(p.add) + yi : nullptr;
+    float x[NV][4], z[NV][4];     // z: what is added, or the gradient
 #pragma unroll
-    for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-      const int c = lane * 4 + i * 256;
+    for (int i = 0; i < NV; ++i) {
+      const int c = RL::col(i);
+#pragma unroll
+      for (int j = 0; j < 4; ++j) x[i][j] = z[i][j] = 0.f;
       if (c < hd) {
         Elem<T>::load4(src + c, x[i]);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) ss += x[i][j] * x[i][j];
+        if (other) Elem<T>::load4(other + c, z[i]);
       }
     }
     float rstd = 1.f;
-    if (p.use_norm) rstd = rsqrtf(wave_sum(ss) / (float)hd + p.eps);
+    if (p.use_norm) rstd = rsqrtf(RL::sum([&](int i, int j, float s) { return s + x[i][j] * x[i][j]; }) / (float)hd + p.eps);
     float graw = 0.f, gate = 1.f;
     if (p.gate_raw) {
       graw = Elem<T>::load(reinterpret_cast<const T*>(p.gate_raw) + bl * p.g.H + h);
@@ -299,8 +338,8 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
     if (!BWD) {
       T* dst = reinterpret_cast<T*>(p.y) + yi;
 #pragma unroll
-      for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-        const int c = lane * 4 + i * 256;
+      for (int i = 0; i < NV; ++i) {
+        const int c = RL::col(i);
         if (c < hd) {
           float o[4];
 #pragma unroll
@@ -308,51 +347,35 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
             float t = x[i][j] * rstd;
             if (p.use_norm) t = Elem<T>::rnd(t * wv[i][j]);     // the normalised tensor has type T in the reference
             o[j] = t * gate;
-          }
-          if (p.add) {
-            float a[4];
-            Elem<T>::load4(reinterpret_cast<const T*>(p.add) + yi + c, a);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) o[j] = a[j] + Elem<T>::rnd(o[j]);
+            if (p.add) o[j] = z[i][j] + Elem<T>::rnd(o[j]);
           }
           Elem<T>::store4(dst + c, o[0], o[1], o[2], o[3]);
         }
       }
     } else {
       // n = x rstd; t = n w; y = t g.   dt = dy g; dg = <dy, t>; dn = dt w; dw += dt n; dx = rstd (dn - n mean(dn n))
-      const T* dyp = reinterpret_cast<const T*>(p.dy) + yi;
-      float dn[LAYER_VEC_MAX][4];
-      float dg = 0.f, dnn = 0.f;
+      float dn[NV][4];
 #pragma unroll
-      for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-        const int c = lane * 4 + i * 256;
-        if (c < hd) {
-          float dyv[4];
-          Elem<T>::load4(dyp + c, dyv);
+      for (int i = 0; i < NV; ++i)
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float n = x[i][j] * rstd;
-            const float t = p.use_norm ? n * wv[i][j] : n;
-            dg += dyv[j] * t;
-            const float dt = dyv[j] * gate;
-            if (p.use_norm) {
-              dwacc[i][j] += dt * n;
-              dn[i][j] = dt * wv[i][j];
-              dnn += dn[i][j] * n;
-            } else {
-              dn[i][j] = dt;
-            }
-          }
+        for (int j = 0; j < 4; ++j) {
+          const float dt = z[i][j] * gate;
+          if (p.use_norm) dwacc[i][j] += dt * (x[i][j] * rstd);
+          dn[i][j] = p.use_norm ? dt * wv[i][j] : dt;
         }
+      float dnn = 0.f;
+      if (p.use_norm) dnn = RL::sum([&](int i, int j, float s) { return s + dn[i][j] * (x[i][j] * rstd); }) / (float)hd;
+      if (p.gate_raw) {
+        const float dg = RL::sum([&](int i, int j, float s) {
+          const float n = x[i][j] * rstd;
+          return s + z[i][j] * (p.use_norm ? n * wv[i][j] : n);
+        });
+        if ((threadIdx.x & (G - 1)) == 0) Elem<T>::store(reinterpret_cast<T*>(p.dgate_raw) + bl * p.g.H + h, dg * silu_grad_f(graw));
       }
-      dg = wave_sum(dg);
-      if (p.use_norm) dnn = wave_sum(dnn) / (float)hd;
-      if (p.gate_raw && lane == 0)
-        Elem<T>::store(reinterpret_cast<T*>(p.dgate_raw) + bl * p.g.H + h, dg * silu_grad_f(graw));
       T* dx = reinterpret_cast<T*>(p.d_o) + oi;
 #pragma unroll
-      for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-        const int c = lane * 4 + i * 256;
+      for (int i = 0; i < NV; ++i) {
+        const int c = RL::col(i);
         if (c < hd) {
           float o[4];
 #pragma unroll
@@ -362,17 +385,23 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
       }
     }
   }
-  if (BWD && p.dw_part) {      // the four waves' shares, in a fixed order
-    __shared__ float red[LAYER_VEC_MAX * 256];
+  if (BWD && p.dw_part) {      // the shares of the wave's rows, then the four waves', in a fixed order
+    __shared__ float red[NV * 4 * G];
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+#pragma unroll
+        for (int o = G; o < 64; o *= 2) dwacc[i][j] += __shfl_xor(dwacc[i][j], o, 64);
     for (int w = 0; w < 4; ++w) {
-      if (wave == w) {
+      if (wave == w && grp == 0) {
 #pragma unroll
-        for (int i = 0; i < LAYER_VEC_MAX; ++i) {
-          const int c = lane * 4 + i * 256;
-          if (c < hd)
+        for (int i = 0; i < NV; ++i)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) red[c + j] = w == 0 ? dwacc[i][j] : red[c + j] + dwacc[i][j];
-        }
+          for (int j = 0; j < 4; ++j) {
+            float* r = &red[RL::col(i) + j];
+            *r = w == 0 ? dwacc[i][j] : *r + dwacc[i][j];
+          }
       }
       __syncthreads();
     }

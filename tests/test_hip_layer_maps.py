@@ -153,3 +153,42 @@ def test_native_and_python_functions_agree(dtype):
         for a, b in zip(*res):
             assert a.dtype == b.dtype and a.shape == b.shape
             assert torch.equal(a, b) or (a.shape == w.shape and rel_l2(a, b) < 1e-5)
+
+
+# head sizes at both sides of every change of lanes and chunks; a token count that no wave's rows divide
+@pytest.mark.parametrize("hd", [4, 64, 68, 96, 100, 128, 132, 192, 196, 384, 388, 512, 516, 768, 772, 1024])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_rows_of_every_head_size_against_float64(hd, dtype):
+    """silu, L2 norm, rescaling, RMSNorm and gate over rows of hd elements: a few roundings of the type per value."""
+    print("[gpu-test] rows", hd, dtype, flush=True)
+    B, L, H, tol = 2, 19, 3, 1e-2 if dtype == torch.bfloat16 else 1e-5
+    g = torch.Generator().manual_seed(hd)
+    r = lambda *s, t=dtype: torch.randn(*s, generator=g).to(t)
+    args = {"qkv": r(B, L, 3 * H * hd), "scale": r(H * hd, 2, t=torch.float32), "offset": r(H * hd, 2, t=torch.float32)}
+    post = {"o": r(B * H, L, hd), "w": r(hd, t=torch.float32), "gate": r(B, L, H), "add": r(B, L, H * hd)}
+
+    def ref_pre(qkv, scale, offset):
+        x = qkv.view(B, L, 3, H, hd).permute(2, 0, 3, 1, 4)
+        y = F.silu(x)
+        heads = lambda t: t.reshape(B * H, L, hd)
+        normed = [heads(y[i] / (y[i].norm(dim=-1, keepdim=True) + 1e-5)) for i in (0, 1)]
+        flat = qkv.view(B, L, 3, H * hd)
+        return (*normed, heads(y[2]), flat[:, :, 0] * scale[:, 0] + offset[:, 0], flat[:, :, 1] * scale[:, 1] + offset[:, 1], flat[:, :, 2])
+
+    def ref_post(o, w, gate, add):
+        n = o * torch.rsqrt(o.square().mean(dim=-1, keepdim=True) + 1e-5) * w
+        return (n.view(B, H, L, hd).transpose(1, 2) * F.silu(gate).unsqueeze(-1)).reshape(B, L, H * hd) + add,
+
+    host = _lib.host()
+    for fn, ref, inp in ((lambda qkv, scale, offset: host.layer_pre_attn(qkv, scale, offset, H, hd, True), ref_pre, args),
+                         (lambda qkv, **k: host.layer_pre(qkv, H, hd, True), lambda qkv, **k: ref_pre(qkv, **k)[:3], args),
+                         (lambda o, w, gate, add: [host.layer_post(o, w, gate, B, H, True, 1e-5, add)], ref_post, post)):
+        a = {n: t.to(DEV).requires_grad_(True) for n, t in inp.items()}
+        d = {n: t.double().requires_grad_(True) for n, t in inp.items()}
+        out, want = fn(**a), ref(**d)
+        assert all(rel_l2(x, y) < tol for x, y in zip(out, want))
+        go = [r(*t.shape) for t in want]
+        got = torch.autograd.grad(out, list(a.values()), [t.to(DEV) for t in go], allow_unused=True)
+        exact = torch.autograd.grad(want, list(d.values()), [t.double() for t in go], allow_unused=True)
+        for n, x, y in zip(inp, got, exact):
+            assert y is None or not y.any() or rel_l2(x, y) < tol, n

@@ -472,6 +472,15 @@ struct DmaPipe {
   }
 };
 
+// What the lanes of a wave wrote to LDS is read by others of them behind this, and what they read is overwritten behind it.  The
+// wave's LDS accesses run in order, so this is no instruction; it keeps the compiler from moving one across (a wave barrier alone
+// orders no memory for it).
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // ---- epilogue staging: accumulators -> LDS tile -> whole rows ------------------------------------
 // A lane owns 4 consecutive n of 32 different rows per fragment; storing that straight to memory touches
 // 32 cache lines per instruction.  Staging the tile in LDS lets every store instruction cover whole rows.

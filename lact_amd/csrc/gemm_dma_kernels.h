@@ -273,6 +273,15 @@ __device__ __forceinline__ DmaOperand weight_operand_ks(const void* base, long l
   return o;
 }
 
+// silu(y0) * y2 of two elements, every tensor of the reference's chain rounded to bf16 (pairs as in update_pointwise2)
+__device__ __forceinline__ void apply_pointwise2(float y0a, float y0b, float y2a, float y2b, float& va, float& vb) {
+  round_pair(y0a, y0b);
+  round_pair(y2a, y2b);
+  float sa = y0a * sigmoidf_(y0a), sb = y0b * sigmoidf_(y0b);
+  round_pair(sa, sb);
+  va = sa * y2a; vb = sb * y2b;
+}
+
 // The hidden-stage kernels below: STAGES of the ring, WPE waves per SIMD (2: one block per compute unit, 4: two).
 // apply forward: O0 = silu(X W0^T) * (X W2^T)
 template <class TS, int STAGES = 3, int WPE = 2>
@@ -310,10 +319,7 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_hidden_dma(const Hid
     LACT_FOR_QUADS(TS) {
       float v[4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float y0 = round_bf16(acc[0][tm][tn][4 * g + j]), y2 = round_bf16(acc[1][tm][tn][4 * g + j]);
-        v[j] = round_bf16(y0 * sigmoidf_(y0)) * y2;
-      }
+      for (int j = 0; j < 4; j += 2) apply_pointwise2(acc[0][tm][tn][4 * g + j], acc[0][tm][tn][4 * g + j + 1], acc[1][tm][tn][4 * g + j], acc[1][tm][tn][4 * g + j + 1], v[j], v[j + 1]);
       SB::put4(smem + SB::lane_base(), tm, tn, g, v[0], v[1], v[2], v[3]);
     }
   }
@@ -431,19 +437,24 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_hidden_dma(const Hi
   for (int ps = 0; ps < SB::PASSES; ++ps) {
     const int r = r0 + ps * SB::RPP;
     if (r < TS::BM && m0 + r < p.T) {
-      float gg[8], h2[8], dh[8], z0[8], z1[8], z2[8], y0[8], y2[8];
+      float gg[8], h2[8], dh[8], z1[8], y0[8], y2[8];
+      uint32_t z0[4], z2[4];
       unpack8(ug[ps], gg);
       unpack8(uh[ps], h2);
       unpack8(ud[ps], dh);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const UpdatePointwise u = update_pointwise<uint16_t>(gg[j], h2[j], dh[j], silu_parts(gg[j]));
-        z0[j] = u.dgpre; z1[j] = u.hid * l1[ps]; z2[j] = u.dh2;
-        y0[j] = u.dgpre * l0[ps]; y2[j] = u.dh2 * l2[ps];
+      for (int j = 0; j < 4; ++j) {
+        const UpdatePointwise2 u = update_pointwise2(gg + 2 * j, h2 + 2 * j, dh + 2 * j, silu_parts(gg[2 * j]), silu_parts(gg[2 * j + 1]));
+        z0[j] = u.dgpre_2; z2[j] = u.dh2_2;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          z1[2 * j + e] = u.hid[e] * l1[ps];
+          y0[2 * j + e] = u.dgpre[e] * l0[ps]; y2[2 * j + e] = u.dh2[e] * l2[ps];
+        }
       }
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = pack8(z0);
+      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = make_uint4(z0[0], z0[1], z0[2], z0[3]);
       *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(z1);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = pack8(z2);
+      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = make_uint4(z2[0], z2[1], z2[2], z2[3]);
       if (keep) {   // the backward is going to start from the rounded pre-activations instead of recomputing them
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O3) + off) = ug[ps];
         *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O4) + off) = uh[ps];
@@ -496,10 +507,13 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_bwd_hidden_dma(const
       unpack8(u2[ps], y2);
       unpack8(ug[ps], gh);
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const SiluParts sp = silu_parts(y0[j]);
-        const float sg = round_bf16(sp.silu);
-        hq[j] = sg * y2[j]; gy0[j] = round_bf16(gh[j] * y2[j]) * sp.d1; gy2[j] = gh[j] * sg;
+      for (int j = 0; j < 8; j += 2) {
+        const SiluParts s0 = silu_parts(y0[j]), s1 = silu_parts(y0[j + 1]);
+        float sg0 = s0.silu, sg1 = s1.silu, t0 = gh[j] * y2[j], t1 = gh[j + 1] * y2[j + 1];
+        round_pair(sg0, sg1);
+        round_pair(t0, t1);
+        hq[j] = sg0 * y2[j]; gy0[j] = t0 * s0.d1; gy2[j] = gh[j] * sg0;
+        hq[j + 1] = sg1 * y2[j + 1]; gy0[j + 1] = t1 * s1.d1; gy2[j + 1] = gh[j + 1] * sg1;
       }
       *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = pack8(hq);
       *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(gy0);
@@ -586,15 +600,20 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_bwd_hidden_dma(cons
     unpack8(u[ps][3], gz0); unpack8(u[ps][4], gz1); unpack8(u[ps][5], gz2);
     float s0 = 0.f, s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const SiluParts sp = silu_parts(gg[j]);
-      const UpdatePointwise up = update_pointwise<uint16_t>(gg[j], h2[j], dh[j], sp);
-      if (mv && nv) { s0 += gz0[j] * up.dgpre; s1 += gz1[j] * up.hid; s2 += gz2[j] * up.dh2; }
-      const float ghid = gz1[j] * l1[ps], gdh2 = gz2[j] * l2[ps], gdg = gz0[j] * l0[ps];
-      o0[j] = ghid * h2[j] * sp.d1 + gdh2 * dh[j] * sp.d1 + gdg * dh[j] * h2[j] * sp.d2;
-      o1[j] = gdh2 * sp.silu + gdg * h2[j] * sp.d1;
-      o2[j] = ghid * sp.silu + gdg * dh[j] * sp.d1;
-      o3[j] = up.dgpre * l0[ps]; o4[j] = up.hid * l1[ps]; o5[j] = up.dh2 * l2[ps];
+    for (int jj = 0; jj < 8; jj += 2) {
+      const SiluParts sps[2] = {silu_parts(gg[jj]), silu_parts(gg[jj + 1])};
+      const UpdatePointwise2 up = update_pointwise2(gg + jj, h2 + jj, dh + jj, sps[0], sps[1]);
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const int j = jj + e;
+        const SiluParts& sp = sps[e];
+        if (mv && nv) { s0 += gz0[j] * up.dgpre[e]; s1 += gz1[j] * up.hid[e]; s2 += gz2[j] * up.dh2[e]; }
+        const float ghid = gz1[j] * l1[ps], gdh2 = gz2[j] * l2[ps], gdg = gz0[j] * l0[ps];
+        o0[j] = ghid * h2[j] * sp.d1 + gdh2 * dh[j] * sp.d1 + gdg * dh[j] * h2[j] * sp.d2;
+        o1[j] = gdh2 * sp.silu + gdg * h2[j] * sp.d1;
+        o2[j] = ghid * sp.silu + gdg * dh[j] * sp.d1;
+        o3[j] = up.dgpre[e] * l0[ps]; o4[j] = up.hid[e] * l1[ps]; o5[j] = up.dh2[e] * l2[ps];
+      }
     }
     // learning-rate gradients: one partial per (row, wave column of 32 columns) = four lanes, slots as before
     s0 += __shfl_xor(s0, 1, 64); s1 += __shfl_xor(s1, 1, 64); s2 += __shfl_xor(s2, 1, 64);
@@ -732,14 +751,19 @@ __global__ __launch_bounds__(DMA_THREADS) void k_update_bwd_hidden_kept_dma(cons
       unpack8(uz[ps][0], gz0); unpack8(uz[ps][1], gz1); unpack8(uz[ps][2], gz2);
       float s0 = 0.f, s1 = 0.f, s2 = 0.f;
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const SiluParts sp = silu_parts(gg[j]);
-        const UpdatePointwise u = update_pointwise<uint16_t>(gg[j], h2[j], dh[j], sp);
-        s0 += gz0[j] * u.dgpre; s1 += gz1[j] * u.hid; s2 += gz2[j] * u.dh2;
-        const float ghid = gz1[j] * l1[ps], gdh2 = gz2[j] * l2[ps], gdg = gz0[j] * l0[ps];
-        o0[j] = ghid * h2[j] * sp.d1 + gdh2 * dh[j] * sp.d1 + gdg * dh[j] * h2[j] * sp.d2;
-        o1[j] = gdh2 * sp.silu + gdg * h2[j] * sp.d1;
-        o2[j] = ghid * sp.silu + gdg * dh[j] * sp.d1;
+      for (int jj = 0; jj < 8; jj += 2) {
+        const SiluParts sps[2] = {silu_parts(gg[jj]), silu_parts(gg[jj + 1])};
+        const UpdatePointwise2 u = update_pointwise2(gg + jj, h2 + jj, dh + jj, sps[0], sps[1]);
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          const int j = jj + e;
+          const SiluParts& sp = sps[e];
+          s0 += gz0[j] * u.dgpre[e]; s1 += gz1[j] * u.hid[e]; s2 += gz2[j] * u.dh2[e];
+          const float ghid = gz1[j] * l1[ps], gdh2 = gz2[j] * l2[ps], gdg = gz0[j] * l0[ps];
+          o0[j] = ghid * h2[j] * sp.d1 + gdh2 * dh[j] * sp.d1 + gdg * dh[j] * h2[j] * sp.d2;
+          o1[j] = gdh2 * sp.silu + gdg * h2[j] * sp.d1;
+          o2[j] = ghid * sp.silu + gdg * dh[j] * sp.d1;
+        }
       }
       // learning-rate gradients: the row's sum over this half's 64 columns (8 lanes), one partial per (row, half)
 #pragma unroll

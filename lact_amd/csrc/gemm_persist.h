@@ -249,10 +249,8 @@ struct ApplyHiddenPolicy {
         for (int g = 0; g < 4; ++g) {
           float v[4];
 #pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            const float y0 = round_bf16(a02[0][tm][tn][4 * g + j]), y2 = round_bf16(a02[1][tm][tn][4 * g + j]);
-            v[j] = round_bf16(y0 * sigmoidf_(y0)) * y2;
-          }
+          for (int j = 0; j < 4; j += 2)
+            apply_pointwise2(a02[0][tm][tn][4 * g + j], a02[0][tm][tn][4 * g + j + 1], a02[1][tm][tn][4 * g + j], a02[1][tm][tn][4 * g + j + 1], v[j], v[j + 1]);
           frag_put4(f.buf(tm * 2 + tn), g, v[0], v[1], v[2], v[3]);
         }
     void* const o[1] = {p.O0};

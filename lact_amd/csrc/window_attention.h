@@ -131,15 +131,6 @@ __device__ __forceinline__ bf16x8 attn_pack(const f32x16& s, int st) {
   return __builtin_bit_cast(bf16x8, make_uint4(r[0], r[1], r[2], r[3]));
 }
 
-// What the lanes of a wave wrote to LDS is read by others of them behind this, and what they read is overwritten behind it.  The
-// wave's LDS accesses run in order, so this is no instruction; it keeps the compiler from moving one across (a wave barrier alone
-// orders no memory for it).
-__device__ __forceinline__ void wave_lds_fence() {
-  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-  __builtin_amdgcn_wave_barrier();
-  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // A wave's [D][32] accumulator (rows = D, columns = its own rows), times `f`, to 32 rows of a contiguous [B, L, H, D]
 // tensor, through 32 x (D + 8) halves of LDS of its own.
 template <int D>

@@ -22,6 +22,7 @@
 #include "state_kernels.h"
 #include "layer_kernels.h"
 #include "window_attention.h"
+#include "small_heads.h"
 #include "plan.h"
 
 using namespace lact;
@@ -594,6 +595,35 @@ struct Runner {
       if (which == 3) LACT_LAUNCH_SMEM("k_update_bwd_hidden", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
     }
   }
+  // An apply step as one kernel, for the head sizes it exists for.  (A value of LACT_OPT_PERSISTENT_TILES other than the default
+  // asks for the hidden-stage kernels.)
+  template <int D, bool SPLIT>
+  void launch_apply_fused(ApplyFusedParams p, int nz) const {
+    constexpr int SM = apply_fused_lds<D, SPLIT>();
+    LACT_BIG_LDS((k_apply_fused<D, SPLIT>), SM);
+    p.map = make_tile_map(ceil_div(p.T, SPLIT ? 128 : 256), 1, nz);
+    LACT_LAUNCH_SMEM("k_apply_fused", "apply", 6.0 * p.T * D * p.dh * nz, (k_apply_fused<D, SPLIT>), dim3(p.map.grid()), dim3(512), SM, s, p);
+  }
+  bool apply_fused(const HiddenParams& hp, const RowGemmParams<1>& out, int T_, int steps) const {
+    if constexpr (kBf16) {
+      if (g_persist != 1 || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
+      ApplyFusedParams p;
+      memset(&p, 0, sizeof(p));
+      p.T = T_; p.dh = d.dh;
+      p.X = static_cast<const uint16_t*>(hp.X); p.ldx = hp.ldx; p.bsx = hp.bsx; p.gsx = hp.gsx;
+      p.W0 = static_cast<const uint16_t*>(hp.W0); p.W1 = static_cast<const uint16_t*>(hp.W1); p.W2 = static_cast<const uint16_t*>(hp.W2);
+      p.bsw = hp.bsw; p.gsw = hp.gsw;
+      p.out = static_cast<uint16_t*>(out.out); p.ldo = out.ldo; p.bso = out.bso; p.gso = out.gso;
+      p.steps = hp.steps;
+      const int nz = d.b * steps;
+      const bool split = ceil_div(T_, 128) * nz <= 256;
+      if (d.d == 64) split ? launch_apply_fused<64, true>(p, nz) : launch_apply_fused<64, false>(p, nz);
+      else if (d.d == 96) split ? launch_apply_fused<96, true>(p, nz) : launch_apply_fused<96, false>(p, nz);
+      else split ? launch_apply_fused<128, true>(p, nz) : launch_apply_fused<128, false>(p, nz);
+      return true;
+    }
+    return false;
+  }
   template <typename U> U* scr(size_t off) const { return reinterpret_cast<U*>(sc + off); }
 
   long long hbs(int T_) const { return (long long)T_ * d.dh; }   // between the batch entries of a step's token-major arrays
@@ -814,6 +844,7 @@ struct Runner {
         hp.gsx = (long long)g.dstart * d.q_ld; hp.gsw = (long long)P.mat3;
         p.t[0].gsB = (long long)P.mat3; p.gso = (long long)g.dout * d.o_ld;
       }
+      if (apply_fused(hp, p, T_, g.n)) return;
       launch_hidden(0, hp, T_, g.n);
       launch_row_gemm<T, true, 1, EPI_STORE>("apply_out", p, d.b * g.n, s, true);
     };

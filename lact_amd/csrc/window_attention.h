@@ -145,10 +145,10 @@ __device__ __forceinline__ void attn_store_rows(char* lds, const f32x16 (&acc)[D
       Elem<uint16_t>::store4(t + (l & 31) * LD + dt * 32 + 8 * g + 4 * (l >> 5), acc[dt][4 * g] * f, acc[dt][4 * g + 1] * f, acc[dt][4 * g + 2] * f,
                              acc[dt][4 * g + 3] * f);
   wave_lds_fence();
-  constexpr int LPR = D / 8, RPP = 64 / LPR;
+  constexpr int LPR = D / 8;
 #pragma unroll
-  for (int i = 0; i < 32 / RPP; ++i) {
-    const int r = i * RPP + l / LPR, c = (l % LPR) * 8;
+  for (int i = 0; i < 32 * LPR / 64; ++i) {
+    const int id = i * 64 + l, r = id / LPR, c = (id % LPR) * 8;
     const uint4 u = *reinterpret_cast<const uint4*>(t + r * LD + c);
     if (row0 + r < L) *reinterpret_cast<uint4*>(out + (size_t)(row0 + r) * ld + c) = u;
   }

@@ -260,6 +260,8 @@ int lact_window_attention_backward(int32_t B, int32_t L, int32_t H, int32_t D, i
  *     compute unit until its last tile costs the step more than it saves.
  *     With the default, apply steps of bf16 heads of 64, 96 and 128 (hidden size a multiple of 32) run as one kernel that keeps
  *     the hidden values in registers and sums them in another order (a result differs where its sum lies next to a rounding).
+ *     Updates of these heads that keep nothing for the backward run as one kernel likewise, also only with the default of
+ *     LACT_OPT_KEEP_PREACTIVATIONS.
  *   LACT_OPT_KEEP_PREACTIVATIONS: 1: the update's forward keeps its rounded pre-activations and lr-scaled operands
  *     for the backward (bf16, d and dh multiples of 64), 0: the backward recomputes them, -1 (default): by shape
  *     (kept when d > 128).  Same bits either way, except the learning-rate gradients (fp32 sums over tiles of another

@@ -6,6 +6,7 @@
 #include <algorithm>
 #include <atomic>
 #include <cstdio>
+#include <climits>
 #include <cstring>
 #include <string>
 #include <vector>
@@ -624,6 +625,49 @@ struct Runner {
     }
     return false;
   }
+  // Whether the program's updates run as one kernel each (the options that select among the kernels in pieces have their defaults).
+  // us per update, in pieces / as one kernel, without Newton-Schulz: 12 heads of 64 with 64 hidden units 128 tokens 16.2 / 11.1, 4096
+  // 27.6 / 20.2; 48 heads 128 tokens 20.2 / 14.9, 4096 62.5 / 44.5; 12 heads of 128 with 256 hidden units 128 tokens 22.9 / 18.7, 4096
+  // 61.7 / 55.6; 48 heads 42.2 / 40.4 and 281 / 160.  Where Newton-Schulz follows and the matrices are square, the reduction of a short
+  // update ends in the momentum step, which the one kernel leaves to a pass of its own (12 heads of 96, 128 tokens 28.5 / 27.1, 512
+  // 31.2 / 30.0; 48 heads of 128, 128 tokens 41.0 / 42.3, 512 47.7 / 50.0, 1024 60.3 / 59.8, 4096 157 / 118).
+  bool updates_fused() const {
+    if (!kBf16 || g_persist != 1 || g_keep_pre >= 0 || P.keep_pre || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
+    int shortest = INT_MAX, longest = 0;
+    for (const auto& st : P.live)
+      if (st.kind == LACT_UPDATE) {
+        shortest = std::min(shortest, st.end - st.start);
+        longest = std::max(longest, st.end - st.start);
+      }
+    const bool step_in_reduction = P.muon && !P.g.stacked && d.d == d.dh;
+    return shortest >= 64 && (!step_in_reduction || longest >= 1024);
+  }
+  template <int D>
+  void launch_update_fused(UpdateFusedParams p, int splits) const {
+    constexpr int SM = UpdatePatch<D>::LDS;
+    LACT_BIG_LDS((k_update_fused<D>), SM);
+    p.map = make_tile_map(splits, p.dh / 32, d.b);
+    LACT_LAUNCH_SMEM("k_update_fused", "update", 12.0 * p.T * D * p.dh * d.b, (k_update_fused<D>), dim3(p.map.grid()), dim3(256), SM, s, p);
+  }
+  // Returns the number of partial-sum slots written.
+  int update_fused(const HiddenParams& hp) const {
+    if constexpr (kBf16) {
+      const Split sp = choose_update_split(hp.T, d.b, d.d, d.dh, P.max_splits(false, 1));
+      UpdateFusedParams p;
+      memset(&p, 0, sizeof(p));
+      p.T = hp.T; p.dh = d.dh; p.split_len = sp.len;
+      p.K = static_cast<const uint16_t*>(hp.X); p.ldk = hp.ldx; p.bsk = hp.bsx;
+      p.V = static_cast<const uint16_t*>(hp.Y); p.ldv = hp.ldy; p.bsv = hp.bsy;
+      p.W0 = static_cast<const uint16_t*>(hp.W0); p.W1 = static_cast<const uint16_t*>(hp.W1); p.W2 = static_cast<const uint16_t*>(hp.W2); p.bsw = hp.bsw;
+      p.lr0 = hp.lr0; p.lr1 = hp.lr1; p.lr2 = hp.lr2; p.bslr = hp.bslr;
+      p.partial = scr<float>(P.t_partial); p.split_stride = (long long)P.mat3; p.mat_stride = (long long)d.b * P.g.elems;
+      if (d.d == 64) launch_update_fused<64>(p, sp.n);
+      else if (d.d == 96) launch_update_fused<96>(p, sp.n);
+      else launch_update_fused<128>(p, sp.n);
+      return sp.n;
+    }
+    return 0;
+  }
   template <typename U> U* scr(size_t off) const { return reinterpret_cast<U*>(sc + off); }
 
   long long hbs(int T_) const { return (long long)T_ * d.dh; }   // between the batch entries of a step's token-major arrays
@@ -815,7 +859,8 @@ struct Runner {
     // beside the first kernels of the call where there is one
     hipEvent_t kl_ready = nullptr;
     const long long klbs = (long long)(P.kl_end - P.kl_begin) * d.d;
-    if (klbs > 0) {
+    const bool fused = updates_fused();
+    if (klbs > 0 && !fused) {
       if (entry) {
         (void)hipStreamWaitEvent(s_tail, entry, 0);
         s = s_tail;
@@ -869,6 +914,7 @@ struct Runner {
       const T* vc = v + (size_t)st.start * d.v_ld;
       const T* kl0 = scr<T>(P.t_kl[0]) + (size_t)(st.start - P.kl_begin) * d.d;
       const T* kl2 = scr<T>(P.t_kl[1]) + (size_t)(st.start - P.kl_begin) * d.d;
+      int dw_slots = 0;
       {
         HiddenParams hp = hidden_params(T_, kc, d.k_ld, d.k_bs, vc, d.v_ld, d.v_bs, ver);
         hp.lr0 = lr0 + st.start; hp.lr1 = lr1 + st.start; hp.lr2 = lr2 + st.start; hp.bslr = d.kv_len;
@@ -883,16 +929,16 @@ struct Runner {
           hp.bso = zbs;
         }
         hp.O0 = z0; hp.O1 = z1; hp.O2 = z2;
-        launch_hidden(1, hp, T_);
+        if (fused) dw_slots = update_fused(hp);
+        else launch_hidden(1, hp, T_);
         upd_z[0] = z0; upd_z[1] = z1; upd_z[2] = z2; upd_zbs = zbs;
       }
       // the pre-Muon gradient (= the momentum state) of the last update: read by nothing when Newton-Schulz output is
       // what enters the weights (the next update and its backward would read it; the caller gets its own copy)
       const bool d_unread = P.muon && !d.muon_replaces_weight && u + 1 == P.nupd;
-      int dw_slots = 0;
       if (kl_ready) (void)hipStreamWaitEvent(s_main, kl_ready, 0);
       kl_ready = nullptr;
-      {
+      if (!fused) {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));
         jobs[0].M = d.dh; jobs[0].N = d.d;

@@ -54,6 +54,21 @@ inline Split choose_split_async(int tokens, int tiles_total, int max_n) {
   int len = ceil_div(ceil_div(tokens, ns), 64) * 64;
   return Split{ceil_div(tokens, len), len};
 }
+// Splits of an update of small heads (k_update_fused): blocks of 32 hidden units and a split of the tokens, one to a compute unit,
+// those of a batch entry or of a split on one XCD (TileMap).  The least of rounds of blocks times what a block takes -- 2.2 us a 128
+// tokens and 8 to start and to add its waves' sums -- and the partial sums' way through memory.  us of the kernel, 6 x 8192 tokens of 128,
+// 256 hidden units: 3 splits 74, 5 44, 11 62; 24 x 2500 of 96: 1 split 50, 2 30, 3 24; 8 x 2048 of 64: 4 splits 11.9, 8 8.5, 16 7.4.
+inline Split choose_update_split(int tokens, int nb, int d, int dh, int max_n) {
+  Split best{1, ceil_div(tokens, 128) * 128};
+  double least = 0;
+  for (int n = 1; n <= std::max(1, std::min(max_n, ceil_div(tokens, 128))); ++n) {
+    const int len = ceil_div(ceil_div(tokens, n), 128) * 128, used = ceil_div(tokens, len), slices = ceil_div(dh, 32);
+    const int per_xcd = nb % 8 == 0 ? nb / 8 * used * slices : ceil_div(nb * used, 8) * slices;
+    const double t = ceil_div(per_xcd, 32) * (len / 128 * 2.2 + 8.0) + (double)used * nb * 3 * d * dh * 8 / 4e6;
+    if (n == 1 || t < least) { least = t; best = Split{used, len}; }
+  }
+  return best;
+}
 template <typename T>
 int token_reduce_tiles(int d, int dh) {
   return std::max(ceil_div(dh, TSG<T>::BM) * ceil_div(d, TSG<T>::BN), ceil_div(d, TSG<T>::BM) * ceil_div(dh, TSG<T>::BN));
@@ -219,6 +234,7 @@ struct Plan {
     // the renorm that reads it: one split 30.3 + 9.3, two 21.5 + 10.1, four 18.3 + 12.2).
     split_min = muon ? 1536 : 1024;
     nsplit_max = std::max(choose_split_async(Tcap, tiles * 3 * d.b, MAX_SPLITS).n, choose_split(Tcap, tr_tiles(d.d, d.dh) * 3 * d.b, MAX_SPLITS, split_min).n);
+    if (bf16 && d.d <= 128) nsplit_max = std::max(nsplit_max, choose_update_split(Tcap, d.b, d.d, d.dh, MAX_SPLITS).n);
     mdot_parts = std::max(std::max(nblk, 256), ceil_div(g.maxrows(), 4));
     build_groups();
     side_slots = 1;

@@ -223,4 +223,386 @@ constexpr int apply_fused_lds() {
   return cmax(ST::STAGES * ST::BYTES, cmax(SPLIT ? 4 * 32 * D * 4 : 0, 8 * 32 * (D + 8) * 2));
 }
 
+// ---- update: the three weight gradients of a step -----------------------------------------------------------------------------
+//   g, u, e = k W0^T, k W2^T, v W1  ->  dW0 = dgate^T (k lr0), dW1 = v^T (hidden lr1), dW2 = dhidden^T (k lr2)
+// A wave keeps 32 hidden units: their rows of W0, W2 and W1^T as fragments and their rows (columns for dW1) of the three gradients as
+// accumulators, all in registers, and walks every fourth patch of 32 tokens of its block's split.  The products come out with a
+// token per register and a hidden unit per lane, which is how the gradients' products read them: nothing is exchanged.  A wave's
+// tokens travel through a ring of its own, five half patches (k and v of two patches and one under way), so that the waves of a block
+// meet only at the end, where the sums of the four are added in LDS.
+//
+// What bounds it: issue of vector operations by the one wave on a SIMD -- 820 for a patch of d = 128, of which 30 % scale k and half of
+// the rest round, in 5600 clocks (the 48 matrix instructions take 1540 of them and hide behind the others; the copies always arrive
+// in time) -- and 8 us a block to start, finish its last patch and add the sums.  us, this kernel against the hidden stage and the
+// token reduction as kernels of their own (and a pass that scales k): 6 x 8192 tokens, d = 128, dh = 256 44 / 36 + 21 (+ 8); 12 x 4680
+// tokens 58 / 65 + 27 (+ 10); 24 x 2500 tokens, d = dh = 96 24 / 28 + 14 (+ 7).  One matrix instruction after each pair of tokens'
+// pointwise part: 52 (the pair's operations wait for each other); the rates by ds_bpermute, 48 a patch: 49.
+struct UpdateFusedParams {
+  int T, dh, split_len;
+  const uint16_t* K; int ldk; long long bsk;               // [T, d]
+  const uint16_t* V; int ldv; long long bsv;
+  const uint16_t* W0; const uint16_t* W1; const uint16_t* W2; long long bsw;
+  const float* lr0; const float* lr1; const float* lr2; long long bslr;
+  float* partial; long long split_stride, mat_stride;      // sums of split s, matrix j, batch entry z: partial + s, j * strides + z * d * dh
+  TileMap map;                                             // splits, 32 hidden units, batch
+};
+
+template <int D>
+struct UpdatePatch {
+  static constexpr int P = D == 64 ? 64 : 128;             // columns of a row in LDS (those past D repeat its last granule)
+  using T = AttnTile<P>;
+  static constexpr int THREADS = 256, BYTES = 32 * T::ROWB, COPIES = BYTES / 1024, UNITS = 5;
+  static constexpr int RING = 4 * UNITS * BYTES, SUMS = 4 * D * 128;
+  static constexpr int LDS = cmax(RING, 2 * SUMS);
+  static_assert(LDS <= 160 * 1024, "the rings do not fit the LDS");
+};
+// Copies of one operand's patch: four offsets a lane, the fifth to eighth copy 16 rows further down.
+template <int D>
+struct UpdateCopies {
+  using U = UpdatePatch<D>;
+  uint32_t voff[4];
+  __device__ __forceinline__ void init(int ld) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int n = i * 64 + (threadIdx.x & 63), row = n / U::T::G, slot = n % U::T::G;
+      voff[i] = (uint32_t)(row * ld + min(slot ^ U::T::key(row), D / 8 - 1) * 8) * 2;
+    }
+  }
+  __device__ __forceinline__ void issue_one(const uint16_t* base, int ld, uint32_t lds, int i) const {
+    dma16<false>(base + (size_t)(i / 4) * 16 * ld, voff[i % 4], lds + i * 1024);
+  }
+  __device__ __forceinline__ void issue(const uint16_t* base, int ld, uint32_t lds) const {
+#pragma unroll
+    for (int i = 0; i < U::COPIES; ++i) issue_one(base, ld, lds, i);
+  }
+};
+
+// The rate of the token in register I of an accumulator: lane i of every 16 holds that of the lane half's i-th token, and the
+// multiplication that takes it reads it from there.
+__device__ __forceinline__ int slot_token(int lane) { return 8 * ((lane & 15) / 4) + 4 * (lane >> 5) + lane % 4; }
+template <int I>
+__device__ __forceinline__ float of_slot(float v) {
+  constexpr int ROW_NEWBCAST = 0x150;
+  return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), ROW_NEWBCAST + I, 0xf, 0xf, true));
+}
+
+// Eight tokens of k from slot I on, times their rates, as the reference rounds the product.
+template <int I>
+__device__ __forceinline__ bf16x8 scaled(const float (&k)[8], float r) {
+  return __builtin_bit_cast(bf16x8, make_uint4(pack_bf16(k[0] * of_slot<I>(r), k[1] * of_slot<I + 1>(r)), pack_bf16(k[2] * of_slot<I + 2>(r), k[3] * of_slot<I + 3>(r)),
+                                               pack_bf16(k[4] * of_slot<I + 4>(r), k[5] * of_slot<I + 5>(r)), pack_bf16(k[6] * of_slot<I + 6>(r), k[7] * of_slot<I + 7>(r))));
+}
+
+// update_pointwise2 on two pairs of tokens, and hidden * lr1, in six steps of some twenty operations each: a matrix instruction is
+// issued after every step, and a wave that is alone on its SIMD needs independent operations to issue one every 4 clocks (one that
+// waits for the last takes 8).
+struct UpdateSteps {
+  float g[4], h2[4], dh[4], sg[4], sb[4], t[4], hid[4];
+  uint32_t z0[2], z1[2], z2[2];
+  __device__ __forceinline__ void round4(float (&x)[4]) const {
+    round_pair(x[0], x[1]);
+    round_pair(x[2], x[3]);
+  }
+  template <int STEP, int I>
+  __device__ __forceinline__ void step(const f32x16& ag, const f32x16& ah, const f32x16& ad, float lr1) {
+    auto each = [](auto f) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) f(j);
+    };
+    if (STEP == 0) {
+      each([&](int j) { g[j] = ag[4 * I + j]; h2[j] = ah[4 * I + j]; dh[j] = ad[4 * I + j]; });
+      round4(g);
+      round4(h2);
+      round4(dh);
+    } else if (STEP == 1) {
+      each([&](int j) { const SiluParts s = silu_parts(g[j]); sg[j] = s.silu; sb[j] = s.sig; });
+    } else if (STEP == 2) {
+      round4(sg);
+      round4(sb);
+      each([&](int j) { hid[j] = sg[j] * h2[j]; });
+    } else if (STEP == 3) {
+      round4(hid);
+      float x[4];
+      each([&](int j) { x[j] = dh[j] * sg[j]; t[j] = dh[j] * h2[j]; });
+      z2[0] = pack_bf16(x[0], x[1]); z2[1] = pack_bf16(x[2], x[3]);
+      x[0] = hid[0] * of_slot<4 * I>(lr1); x[1] = hid[1] * of_slot<4 * I + 1>(lr1);
+      x[2] = hid[2] * of_slot<4 * I + 2>(lr1); x[3] = hid[3] * of_slot<4 * I + 3>(lr1);
+      z1[0] = pack_bf16(x[0], x[1]); z1[1] = pack_bf16(x[2], x[3]);
+    } else if (STEP == 4) {
+      round4(t);
+      each([&](int j) { t[j] *= sb[j]; sb[j] = 1.f - sb[j]; });
+      round4(t);
+      round4(sb);
+    } else {
+      each([&](int j) { sb[j] *= g[j]; });
+      round4(sb);
+      each([&](int j) { sb[j] += 1.f; });
+      round4(sb);
+      each([&](int j) { t[j] *= sb[j]; });
+      z0[0] = pack_bf16(t[0], t[1]); z0[1] = pack_bf16(t[2], t[3]);
+    }
+  }
+};
+
+template <int D>
+__global__ __launch_bounds__(256, 1) void k_update_fused(const UpdateFusedParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  using U = UpdatePatch<D>;
+  int bx, by, z;
+  if (!p.map.locate(blockIdx.x, bx, by, z)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, h = lane >> 5;
+  const int hid0 = by * 32, tok0 = bx * p.split_len, len = min(p.split_len, p.T - tok0);
+  const uint16_t* K = p.K + z * p.bsk;
+  const uint16_t* V = p.V + z * p.bsv;
+  const float *lr0 = p.lr0 + z * p.bslr, *lr1 = p.lr1 + z * p.bslr, *lr2 = p.lr2 + z * p.bslr;
+  // Patches of this wave; one that would run past the last token starts earlier, its `over` first rows are cleared after the copy.
+  const int patches = (len + 31) / 32, mine = patches > wave ? (patches - wave + 3) / 4 : 0;
+  auto token = [&](int i) { return min(tok0 + (wave + 4 * min(i, mine - 1)) * 32, p.T - 32); };
+  const int over = mine > 0 ? tok0 + (wave + 4 * (mine - 1)) * 32 - token(mine - 1) : 0;
+
+  // The weights' slices come once for the block, into units of the first wave's ring that its tokens need later: rows of W0 and W2 like
+  // a patch of tokens, [d][32 hidden] of W1 in rows of 64 bytes, to be read transposed.  (Each wave's fragments straight from memory
+  // are 96 KiB a block instead of 24, at 40 to 70 GB/s that reach a compute unit: 1.5 us.)
+  constexpr int KS = D / 16;
+  bf16x8 w0[KS], w1[KS], w2[KS];
+  AttnFrag<U::P> frag;
+  frag.init();
+  char* const weights = smem + 2 * U::BYTES;
+  {
+    const uint32_t to = lds_addr(weights);
+    const long long w = z * p.bsw;
+    UpdateCopies<D> cw;
+    cw.init(D);
+#pragma unroll
+    for (int i = 0; i < U::COPIES; ++i)
+      if (i % 4 == wave) {
+        cw.issue_one(p.W0 + w + (size_t)hid0 * D, D, to, i);
+        cw.issue_one(p.W2 + w + (size_t)hid0 * D, D, to + U::BYTES, i);
+      }
+    for (int i = wave; i < D / 16; i += 4) {
+      const int n = i * 64 + lane;
+      dma16<false>(p.W1 + w + hid0, (uint32_t)((n >> 2) * p.dh + (n & 3) * 8) * 2, to + 2 * U::BYTES + i * 1024);
+    }
+  }
+  char* ring = smem + wave * U::UNITS * U::BYTES;
+  const uint32_t lds0 = lds_addr(ring);
+  UpdateCopies<D> ck, cv;
+  ck.init(p.ldk);
+  cv.init(p.ldv);
+  auto unit = [&](int n) { return ring + n * U::BYTES; };
+  auto issue_k = [&](int i, int n) { ck.issue(K + (size_t)token(i) * p.ldk, p.ldk, lds0 + n * U::BYTES); };
+  auto issue_v = [&](int i, int n) { cv.issue(V + (size_t)token(i) * p.ldv, p.ldv, lds0 + n * U::BYTES); };
+  struct Rates { float r[3]; };
+  auto rates = [&](int i) {
+    const int t = token(i) + slot_token(lane);
+    return Rates{{lr0[t], lr1[t], lr2[t]}};
+  };
+  Rates rc{};
+  if (mine > 0) {
+    rc = rates(0);
+    issue_k(0, 0);
+    issue_v(0, 1);
+  }
+  wait_vmcnt<0>();
+  __syncthreads();
+  {
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const char* t = weights + 2 * U::BYTES + (8 * h + ((lane & 15) >> 2)) * 64 + ((lane >> 4) & 1) * 32 + (lane & 3) * 8;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      w0[s] = frag.rows(weights, 0, s);
+      w2[s] = frag.rows(weights + U::BYTES, 0, s);
+      const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + s * 1024)), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(t + s * 1024 + 256));
+      const s16x8 v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+      w1[s] = __builtin_bit_cast(bf16x8, v);
+    }
+  }
+  f32x16 d0[D / 32], d1[D / 32], d2[D / 32];
+#pragma unroll
+  for (int i = 0; i < D / 32; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) d0[i][j] = d1[i][j] = d2[i][j] = 0.f;
+  __syncthreads();       // the first wave's units are its own again
+  if (mine > 0) {
+    auto settle = [&](Rates& r, int i) {
+      const int cut = i == mine - 1 ? over : 0;
+#pragma unroll
+      for (int j = 0; j < 3; ++j) r.r[j] = slot_token(lane) < cut ? 0.f : r.r[j];
+    };
+    settle(rc, 0);
+    issue_k(1, 2);
+    issue_v(1, 3);
+    Rates rn = rates(1);
+    auto clear = [&](int i, int nk, int nv) {
+      if (i != mine - 1 || over == 0) return;
+      wait_vmcnt<0>();
+      for (int e = lane; e < over * U::T::G; e += 64) {
+        *reinterpret_cast<uint4*>(unit(nk) + e * 16) = make_uint4(0, 0, 0, 0);
+        *reinterpret_cast<uint4*>(unit(nv) + e * 16) = make_uint4(0, 0, 0, 0);
+      }
+      wave_lds_fence();
+    };
+    constexpr std::true_type yes{};
+    constexpr std::false_type no{};
+    uint32_t q0[8], q1[8], q2[8];      // dgate, hidden * lr1, dhidden of the patch in hand, two tokens a word
+    // The products of the next patch (FIRST), between them the pointwise part of the patch in g, u, e (GATE).
+    auto products = [&](auto first, auto gate, const char* kt, const char* vt, f32x16& gn, f32x16& un, f32x16& en, const f32x16& g, const f32x16& u,
+                        const f32x16& e, float lr, auto between) {
+      constexpr bool FIRST = decltype(first)::value, GATE = decltype(gate)::value;
+      // fragments two ahead; the steps of the pointwise part spread over the matrix instructions
+      constexpr int N = 2 * KS, STEPS = 24;
+      bf16x8 f[3];
+      auto read = [&](int ks) {
+        if (ks == KS) between();
+        if (ks < N) f[ks % 3] = ks < KS ? frag.rows(kt, 0, ks) : frag.rows(vt, 0, ks - KS);
+      };
+      if (FIRST) {
+        read(0);
+        read(1);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) gn[j] = un[j] = en[j] = 0.f;
+      }
+      UpdateSteps st;
+      int done = 0;
+      auto round = [&](auto at, int n) {
+        constexpr int I = decltype(at)::value;
+        switch (n) {
+          case 0: st.template step<0, I>(g, u, e, lr); break;
+          case 1: st.template step<1, I>(g, u, e, lr); break;
+          case 2: st.template step<2, I>(g, u, e, lr); break;
+          case 3: st.template step<3, I>(g, u, e, lr); break;
+          case 4: st.template step<4, I>(g, u, e, lr); break;
+          default:
+            st.template step<5, I>(g, u, e, lr);
+#pragma unroll
+            for (int w = 0; w < 2; ++w) { q0[2 * I + w] = st.z0[w]; q1[2 * I + w] = st.z1[w]; q2[2 * I + w] = st.z2[w]; }
+        }
+      };
+      auto steps = [&](int upto) {
+        if (!GATE) return;
+#pragma unroll
+        for (int n = 0; n < STEPS; ++n) {
+          if (n < done || n >= upto) continue;
+          switch (n / 6) {
+            case 0: round(std::integral_constant<int, 0>{}, n % 6); break;
+            case 1: round(std::integral_constant<int, 1>{}, n % 6); break;
+            case 2: round(std::integral_constant<int, 2>{}, n % 6); break;
+            default: round(std::integral_constant<int, 3>{}, n % 6);
+          }
+        }
+        done = upto;
+      };
+#pragma unroll
+      for (int ks = 0; ks < N; ++ks) {
+        const int before = ks < KS ? 2 * ks : KS + ks;        // matrix instructions issued before this fragment's
+        if (FIRST) {
+          read(ks + 2);
+          if (ks < KS) gn = mma32(f[ks % 3], w0[ks % KS], gn);
+          else en = mma32(f[ks % 3], w1[ks % KS], en);
+        }
+        steps((before + 1) * STEPS / (3 * KS));
+        __builtin_amdgcn_sched_barrier(0);
+        if (ks < KS) {
+          if (FIRST) un = mma32(f[ks % 3], w2[ks % KS], un);
+          steps((before + 2) * STEPS / (3 * KS));
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    };
+    auto slots = [&](const uint32_t* q, int st) { return __builtin_bit_cast(bf16x8, make_uint4(q[4 * st], q[4 * st + 1], q[4 * st + 2], q[4 * st + 3])); };
+    // The gradients' products over the patch in hand.
+    auto gradients = [&](const char* kt, const char* vt, const Rates& r, auto after_v) {
+      constexpr int N = D / 32 * 2;
+      bf16x8 fk[3], fv[3];
+      auto read = [&](int n) {
+        if (n >= N) return;
+        fk[n % 3] = frag.cols(kt, n / 2, n % 2);
+        fv[n % 3] = frag.cols(vt, n / 2, n % 2);
+      };
+      read(0);
+      read(1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int n = 0; n < N; ++n) {
+        const int dt = n / 2, st = n % 2;
+        read(n + 2);
+        d1[dt] = mma32(fv[n % 3], slots(q1, st), d1[dt]);
+        const uint4 x = __builtin_bit_cast(uint4, fk[n % 3]);
+        const float k[8] = {bf16_lo(x.x), bf16_hi(x.x), bf16_lo(x.y), bf16_hi(x.y), bf16_lo(x.z), bf16_hi(x.z), bf16_lo(x.w), bf16_hi(x.w)};
+        const bf16x8 k0 = st == 0 ? scaled<0>(k, r.r[0]) : scaled<8>(k, r.r[0]);
+        __builtin_amdgcn_sched_barrier(0);
+        d0[dt] = mma32(slots(q0, st), k0, d0[dt]);
+        const bf16x8 k2 = st == 0 ? scaled<0>(k, r.r[2]) : scaled<8>(k, r.r[2]);
+        __builtin_amdgcn_sched_barrier(0);
+        d2[dt] = mma32(slots(q2, st), k2, d2[dt]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      after_v();
+    };
+    f32x16 g, u, e, gn, un, en;
+    clear(0, 0, 1);
+    products(yes, no, unit(0), unit(1), g, u, e, gn, un, en, 0.f, [] {});
+    int kc = 0, vc = 1, k1 = 2, v1 = 3, idle = 4;      // units of the current and the next patch
+    for (int i = 0; i + 1 < mine; ++i) {
+      wait_vmcnt<U::COPIES>();          // the next patch's k: nothing but its v (and its rates) was asked for later
+      clear(i + 1, k1, v1);
+      products(yes, yes, unit(k1), unit(v1), gn, un, en, g, u, e, rc.r[1], [&] {
+        wait_vmcnt<0>();
+        settle(rn, i + 1);              // (before the copies to come, which would have to arrive first)
+        __builtin_amdgcn_sched_barrier(0);
+        issue_k(i + 2, idle);
+      });
+      gradients(unit(kc), unit(vc), rc, [&] { issue_v(i + 2, vc); });
+      g = gn; u = un; e = en;
+      rc = rn;
+      rn = rates(i + 2);
+      const int k2 = idle, v2 = vc;
+      idle = kc; kc = k1; vc = v1; k1 = k2; v1 = v2;
+    }
+    products(no, yes, smem, smem, gn, un, en, g, u, e, rc.r[1], [] {});
+    gradients(unit(kc), unit(vc), rc, [] {});
+  }
+  wait_vmcnt<0>();
+  __syncthreads();
+
+  // the waves' sums, a matrix at a time: [wave][32 columns or rows of d][four registers][lane]
+  auto put = [&](const f32x16 (&d)[D / 32], int buf) {
+    float4* o = reinterpret_cast<float4*>(smem + buf * U::SUMS) + wave * D * 8 + lane;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t)
+#pragma unroll
+      for (int q = 0; q < 4; ++q) o[(t * 4 + q) * 64] = make_float4(d[t][4 * q], d[t][4 * q + 1], d[t][4 * q + 2], d[t][4 * q + 3]);
+  };
+  float* out = p.partial + bx * p.split_stride + (long long)z * D * p.dh;
+  auto add = [&](int mat, int buf) {
+    const float4* s = reinterpret_cast<const float4*>(smem + buf * U::SUMS) + wave * 64 + lane;
+    float* o = out + mat * p.mat_stride;
+#pragma unroll
+    for (int t = 0; t < D / 32; ++t) {
+      float4 v = s[t * 256];
+#pragma unroll
+      for (int w = 1; w < 4; ++w) {
+        const float4 a = s[t * 256 + w * D * 8];
+        v.x += a.x; v.y += a.y; v.z += a.z; v.w += a.w;
+      }
+      const float x[4] = {v.x, v.y, v.z, v.w};
+      const int row = 8 * wave + 4 * h, col = lane & 31;
+#pragma unroll
+      for (int j = 0; j < 4; ++j)
+        if (mat == 1) o[(size_t)(t * 32 + row + j) * p.dh + hid0 + col] = x[j];
+        else o[(size_t)(hid0 + row + j) * D + t * 32 + col] = x[j];
+    }
+  };
+  put(d0, 0);
+  __syncthreads();
+  put(d1, 1);
+  add(0, 0);
+  __syncthreads();
+  put(d2, 0);
+  add(1, 1);
+  __syncthreads();
+  add(2, 0);
+}
+
 }  // namespace lact

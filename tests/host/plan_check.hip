@@ -41,6 +41,11 @@ static int check(bool bf16, int b, int d, int dh, int rounds, int T_update, int 
       const int used = P.reduce_split(T, 1, P.max_splits(false, 1), min_len).n;
       expect(used <= P.nsplit_max, "slots of a launch of the main chain", used, P.nsplit_max);
     }
+  if (bf16 && d <= 128)      // an update of small heads as one kernel
+    for (int T : {T_update, T_apply}) {
+      const Split sp = choose_update_split(T, b, d, dh, P.max_splits(false, 1));
+      expect(sp.n <= P.nsplit_max && (sp.n - 1) * sp.len < T && sp.n * sp.len >= T && sp.len % 128 == 0, "splits of an update in one kernel", sp.n, sp.len);
+    }
   expect(P.t_partial_side + (size_t)P.side_slots * P.mat3 * 4 <= P.t_gwside, "end of the side buffer", P.side_slots, 0);
   for (const auto& g : P.groups) {
     const size_t rows = (size_t)g.n * b * (g.st.end - g.st.start) * dh * P.esz;

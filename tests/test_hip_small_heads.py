@@ -58,3 +58,53 @@ def test_infinite_queries_stay_in_their_rows():
         out, ref = run(), in_pieces(run)
     rows = torch.isfinite(out.float()).all(dim=-1)
     assert torch.equal(rows, torch.isfinite(ref.float()).all(dim=-1)) and int((~rows).sum()) == 1 and not rows[0, 40]
+
+
+# tokens at the edges of a wave's 32, of a block's round of 128 and of its splits (down to the 64 that the kernel takes); one and many
+# slices of 32 hidden units; more blocks than the chip holds at once; a step that starts inside the sequence, with tokens around
+# it that nothing may read
+@pytest.mark.parametrize("b,T,d,dh", [(1, 64, 64, 32), (2, 65, 96, 96), (1, 95, 128, 160), (3, 127, 64, 128), (8, 129, 128, 32), (2, 255, 96, 64),
+                                      (1, 1500, 128, 256), (5, 1025, 64, 96), (70, 130, 128, 128), (24, 777, 96, 96)])
+def test_update_in_one_kernel(b, T, d, dh):
+    """The gradients of a step (the momentum states, when there is no earlier one) and the weights it leaves: the same products of the same
+    rounded values, summed in another order and rounded to bf16.  A sum is 1e-6 to 1e-5 off, so that one in 1e2 to 1e3 lands on the
+    other side of a rounding and moves by 2^-8: 4e-4 in norm at most; 1e-3."""
+    print("[gpu-test] update in one kernel", b, T, d, dh, flush=True)
+    at, L = 7, T + 40
+    t = {n: x.to(DEV) for n, x in O.make_inputs(b, L, d, dh, seed=63, act_dtype=torch.bfloat16).items()}
+    for n in ("k", "v", "lr0", "lr1", "lr2"):
+        t[n] = t[n].clone()
+        t[n][:, :at] = t[n][:, at + T:] = float("nan")
+    momentum = torch.full((b, L, 1), 0.9, device=DEV)
+    wide = torch.full((b, L, 2 * d + 16), float("nan"), dtype=torch.bfloat16, device=DEV)
+    wide[..., 8:d + 8], wide[..., d + 8:2 * d + 8] = t["k"], t["v"]
+    prog = ops.Program(steps=((LACT_UPDATE, at, at + T, 0), (LACT_UPDATE, at, at + T, 0), (LACT_APPLY, 0, 32, 0)), out_len=32)
+    args = [t[n] for n in ORDER]
+
+    def run(k, v):
+        out, w, m = ops.run_program(prog, *args[:4], k, v, *args[6:], momentum=momentum)
+        return [out, *w, *m]
+
+    with torch.no_grad():
+        whole, view, ref = run(t["k"], t["v"]), run(wide[..., 8:d + 8], wide[..., d + 8:2 * d + 8]), in_pieces(lambda: run(t["k"], t["v"]))
+    for i, (a, c, r) in enumerate(zip(whole, view, ref)):
+        assert torch.equal(a, c) and torch.isfinite(a.float()).all()
+        assert O.rel_l2(a, r) < 1e-3, (i, O.rel_l2(a, r))
+
+
+@pytest.mark.parametrize("token", [0, 30, 31, 66, 69])
+def test_infinite_tokens_stay_in_their_head(token):
+    """70 tokens: the last patch starts at token 38 and clears the 26 that the patch before it holds as well."""
+    print("[gpu-test] infinite tokens of an update", token, flush=True)
+    t = {n: x.to(DEV) for n, x in O.make_inputs(3, 70, 128, 64, seed=64, act_dtype=torch.bfloat16).items()}
+    t["v"][1, token] = float("inf")
+    prog = ops.Program(steps=((LACT_UPDATE, 0, 70, 0), (LACT_APPLY, 0, 70, 0)), out_len=70)
+
+    def run():
+        out, w, _ = ops.run_program(prog, *[t[n] for n in ORDER])
+        return [out, *w]
+
+    with torch.no_grad():
+        for a, r in zip(run(), in_pieces(run)):
+            fine = torch.isfinite(a.float()).flatten(1).all(dim=1)
+            assert torch.equal(fine, torch.isfinite(r.float()).flatten(1).all(dim=1)) and fine.tolist() == [True, False, True]

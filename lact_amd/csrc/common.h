@@ -20,8 +20,6 @@ __device__ __forceinline__ uint16_t f32_to_bf16(float f) {
   __bf16 h = (__bf16)f;
   return __builtin_bit_cast(uint16_t, h);
 }
-// round a float to the nearest bf16-representable float
-__device__ __forceinline__ float round_bf16(float f) { return bf16_to_f32(f32_to_bf16(f)); }
 // Two values at once: one v_cvt_pk_bf16_f32 (lo in the lower half) where separate conversions take three instructions to pack.
 // The GEMM epilogues are bound by vector-ALU issue.
 __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
@@ -29,6 +27,10 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
   typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
   return __builtin_bit_cast(uint32_t, __builtin_convertvector((f32x2{lo, hi}), bf16x2));
 }
+// Round a float to the nearest bf16-representable float.  Converted into the upper half beside a zero, the value is a float again
+// where it stands: one instruction of 4 clocks.  (Clocks a wave-wide operation takes of a SIMD with several waves: 2 for fp32 multiply
+// and add, and / or / right shift; 4 for conversions, fma and left shift; 8 for exp and rcp.  One wave alone: 4 at least.)
+__device__ __forceinline__ float round_bf16(float f) { return __uint_as_float(pack_bf16(0.f, f)); }
 __device__ __forceinline__ float bf16_lo(uint32_t u) { return __uint_as_float(u << 16); }
 __device__ __forceinline__ float bf16_hi(uint32_t u) { return __uint_as_float(u & 0xffff0000u); }
 

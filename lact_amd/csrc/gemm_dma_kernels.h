@@ -275,10 +275,10 @@ __device__ __forceinline__ DmaOperand weight_operand_ks(const void* base, long l
 
 // silu(y0) * y2 of two elements, every tensor of the reference's chain rounded to bf16 (pairs as in update_pointwise2)
 __device__ __forceinline__ void apply_pointwise2(float y0a, float y0b, float y2a, float y2b, float& va, float& vb) {
-  round_pair(y0a, y0b);
-  round_pair(y2a, y2b);
+  round_both(y0a, y0b);
+  round_both(y2a, y2b);
   float sa = y0a * sigmoidf_(y0a), sb = y0b * sigmoidf_(y0b);
-  round_pair(sa, sb);
+  round_both(sa, sb);
   va = sa * y2a; vb = sb * y2b;
 }
 
@@ -510,8 +510,8 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_bwd_hidden_dma(const
       for (int j = 0; j < 8; j += 2) {
         const SiluParts s0 = silu_parts(y0[j]), s1 = silu_parts(y0[j + 1]);
         float sg0 = s0.silu, sg1 = s1.silu, t0 = gh[j] * y2[j], t1 = gh[j + 1] * y2[j + 1];
-        round_pair(sg0, sg1);
-        round_pair(t0, t1);
+        round_both(sg0, sg1);
+        round_both(t0, t1);
         hq[j] = sg0 * y2[j]; gy0[j] = t0 * s0.d1; gy2[j] = gh[j] * sg0;
         hq[j + 1] = sg1 * y2[j + 1]; gy0[j + 1] = t1 * s1.d1; gy2[j + 1] = gh[j + 1] * sg1;
       }

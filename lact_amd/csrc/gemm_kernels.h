@@ -196,13 +196,16 @@ __device__ __forceinline__ UpdatePointwise update_pointwise(float g, float h2, f
   return u;
 }
 
-// The same for two bf16 elements at a time: every rounding is one conversion of the pair and two instructions to take it apart,
-// three for what costs four one by one.  The epilogues that call this are bound by vector-ALU issue, and half of that is rounding
-// (46 -> 40 issue slots per element of the update's forward).  dgpre2, dh2_2: the pairs as they are stored.
+// The same for two bf16 elements at a time.  The epilogues that call this are bound by vector-ALU issue, and half of that is
+// rounding: values that go on as floats are rounded one by one in place, those that are also stored as a pair, which takes two more
+// instructions to take it apart.  dgpre_2, dh2_2: the pairs as they are stored.
 __device__ __forceinline__ uint32_t round_pair(float& a, float& b) {
   const uint32_t u = pack_bf16(a, b);
   a = bf16_lo(u); b = bf16_hi(u);
   return u;
+}
+__device__ __forceinline__ void round_both(float& a, float& b) {
+  a = round_bf16(a); b = round_bf16(b);
 }
 struct UpdatePointwise2 {
   float hid[2], dh2[2], dgpre[2];
@@ -211,22 +214,22 @@ struct UpdatePointwise2 {
 __device__ __forceinline__ UpdatePointwise2 update_pointwise2(const float* g, const float* h2, const float* dh, const SiluParts& s0, const SiluParts& s1) {
   UpdatePointwise2 u;
   float sg0 = s0.silu, sg1 = s1.silu, sb0 = s0.sig, sb1 = s1.sig;
-  round_pair(sg0, sg1);
+  round_both(sg0, sg1);
   u.hid[0] = sg0 * h2[0]; u.hid[1] = sg1 * h2[1];
-  round_pair(u.hid[0], u.hid[1]);
+  round_both(u.hid[0], u.hid[1]);
   u.dh2[0] = dh[0] * sg0; u.dh2[1] = dh[1] * sg1;
   u.dh2_2 = round_pair(u.dh2[0], u.dh2[1]);
-  round_pair(sb0, sb1);
+  round_both(sb0, sb1);
   float t0 = dh[0] * h2[0], t1 = dh[1] * h2[1];
-  round_pair(t0, t1);
+  round_both(t0, t1);
   t0 *= sb0; t1 *= sb1;
-  round_pair(t0, t1);
+  round_both(t0, t1);
   float r0 = 1.f - sb0, r1 = 1.f - sb1;
-  round_pair(r0, r1);
+  round_both(r0, r1);
   r0 *= g[0]; r1 *= g[1];
-  round_pair(r0, r1);
+  round_both(r0, r1);
   r0 += 1.f; r1 += 1.f;
-  round_pair(r0, r1);
+  round_both(r0, r1);
   u.dgpre[0] = t0 * r0; u.dgpre[1] = t1 * r1;
   u.dgpre_2 = round_pair(u.dgpre[0], u.dgpre[1]);
   return u;

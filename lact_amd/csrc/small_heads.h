@@ -231,11 +231,11 @@ constexpr int apply_fused_lds() {
 // tokens travel through a ring of its own, five half patches (k and v of two patches and one under way), so that the waves of a block
 // meet only at the end, where the sums of the four are added in LDS.
 //
-// What bounds it: issue of vector operations by the one wave on a SIMD -- 820 for a patch of d = 128, of which 30 % scale k and half of
-// the rest round, in 5600 clocks (the 48 matrix instructions take 1540 of them and hide behind the others; the copies always arrive
+// What bounds it: issue of vector operations by the one wave on a SIMD -- 730 for a patch of d = 128, of which 30 % scale k and a third of
+// the rest rounds, in 5300 clocks (the 48 matrix instructions take 1540 of them and hide behind the others; the copies always arrive
 // in time) -- and 8 us a block to start, finish its last patch and add the sums.  us, this kernel against the hidden stage and the
-// token reduction as kernels of their own (and a pass that scales k): 6 x 8192 tokens, d = 128, dh = 256 44 / 36 + 21 (+ 8); 12 x 4680
-// tokens 58 / 65 + 27 (+ 10); 24 x 2500 tokens, d = dh = 96 24 / 28 + 14 (+ 7).  One matrix instruction after each pair of tokens'
+// token reduction as kernels of their own (and a pass that scales k): 6 x 8192 tokens, d = 128, dh = 256 43 / 36 + 21 (+ 8); 12 x 4680
+// tokens 55 / 65 + 27 (+ 10); 24 x 2500 tokens, d = dh = 96 23 / 28 + 14 (+ 7).  One matrix instruction after each pair of tokens'
 // pointwise part: 52 (the pair's operations wait for each other); the rates by ds_bpermute, 48 a patch: 49.
 struct UpdateFusedParams {
   int T, dh, split_len;
@@ -300,8 +300,8 @@ struct UpdateSteps {
   float g[4], h2[4], dh[4], sg[4], sb[4], t[4], hid[4];
   uint32_t z0[2], z1[2], z2[2];
   __device__ __forceinline__ void round4(float (&x)[4]) const {
-    round_pair(x[0], x[1]);
-    round_pair(x[2], x[3]);
+    round_both(x[0], x[1]);
+    round_both(x[2], x[3]);
   }
   template <int STEP, int I>
   __device__ __forceinline__ void step(const f32x16& ag, const f32x16& ah, const f32x16& ad, float lr1) {

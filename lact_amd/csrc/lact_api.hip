@@ -394,7 +394,7 @@ struct Runner {
     else LACT_LAUNCH_SMEM("k_ns_local", "ns_fwd", flops, (k_ns_local<RT, XG, false>), dim3(B.n), dim3(512), SM, s, p);
   }
   void launch_ns_local(NsLocalParams p, const NsBatch& B) {
-    p.c = B.c; p.S = P.S; p.nb = B.nb; p.mask = B.mask;
+    p.c = B.c; p.S = P.S; p.nb = B.nb; p.mask = B.mask; p.by_granules = make_udiv(B.c / 8);
     for (int i = 0; i < 3 * P.S; ++i) p.coeffs[i] = P.coeffs[i];
     const bool wide = B.c > 128;
     switch (B.r / 32) {

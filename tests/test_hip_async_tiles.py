@@ -166,6 +166,33 @@ def test_newton_schulz_in_one_block_is_bit_identical(b, d, dh, L, stacked):
             assert torch.equal(a, r)
 
 
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** -70, 2.0 ** -101, 2.0 ** -118, 2.0 ** 40])
+@pytest.mark.parametrize("zeros", [False, True])
+def test_normalisation_of_extreme_gradients(scale, zeros):
+    """The quotient in front of the iterations: by two fused multiply-adds where nothing leaves the normal range, by a division where an
+    entry is zero or below 2^-100 or the norm above 2^25.  The launch of its own always divides: the same bits."""
+    print("[gpu-test] normalisation", scale, zeros, flush=True)
+    from lact_amd import _lib, ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(2, 90, 64, 96, seed=35, act_dtype=torch.bfloat16).items()}
+    for n in ("lr0", "lr1", "lr2"):
+        inp[n] = inp[n] * scale
+    if zeros:
+        inp["k"][..., 5] = 0
+    prog = ops.Program(steps=((LACT_UPDATE, 0, 90, 0), (LACT_APPLY, 0, 90, 0)), out_len=90, ns_coeffs=ops.NS5_COEFFS[:1])
+    res = []
+    for fused in (1, 0):
+        _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, fused)
+        try:
+            with torch.no_grad():
+                out, ws, _ = ops.run_program(prog, *[inp[n] for n in ORDER[:9]])
+            res.append([out, *ws])
+        finally:
+            _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 1)
+    for a, r in zip(*res):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, r)
+
+
 def same_specials(a, r):
     a, r = a.detach().float().cpu(), r.detach().float()
     assert torch.isinf(r).any()

@@ -668,6 +668,47 @@ struct Runner {
     }
     return 0;
   }
+  // Whether the backward of the program's updates forms the tokens' gradients in one kernel.  A round of its blocks takes 14 us and 3.3 to
+  // 4 (d = 64 to 128) per 32 hidden units however few blocks there are, the kernels in pieces 17 us and then by the work: 126 us at
+  // 12 x 4680 tokens, d = 128, dh = 256 (hidden stage 92, token rows beside the reduction 34).  us of a training step of four updates and
+  // applies, in pieces / with the one kernel (without Newton-Schulz): 12 x 4096 tokens, 128 x 256 1260 / 1044, 12 x 1024 497 / 488,
+  // 12 x 256 368 / 394; 48 x 1024, 64 x 128 691 / 558.
+  bool update_bwd_fused() const {
+    if (!kBf16 || g_persist != 1 || g_keep_pre >= 0 || P.keep_pre || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
+    double pieces = 0, one = 0;
+    for (const auto& st : P.live)
+      if (st.kind == LACT_UPDATE) {
+        const int T_ = st.end - st.start;
+        pieces += 17 + 126.0 * d.b * T_ / (12 * 4680) * d.d * d.dh / (128 * 256);
+        one += ceil_div(ceil_div(T_, 128) * d.b, 256) * (14 + (2.6 + d.d / 90.0) * (d.dh / 32));
+      }
+    return one < pieces;
+  }
+  template <int D>
+  void launch_update_bwd_fused(UpdateBwdFusedParams p) const {
+    constexpr int SM = BwdStage<D>::LDS;
+    LACT_BIG_LDS((k_update_bwd_fused<D>), SM);
+    p.map = make_tile_map(ceil_div(p.T, 128), 1, d.b);
+    LACT_LAUNCH_SMEM("k_update_bwd_fused", "update_bwd", 24.0 * p.T * D * p.dh * d.b, (k_update_bwd_fused<D>), dim3(p.map.grid()), dim3(256), SM, s, p);
+  }
+  void update_bwd_fused(const HiddenParams& hp, T* dk, T* dv, long long bsd) const {
+    if constexpr (kBf16) {
+      auto u16 = [](const void* x) { return static_cast<const uint16_t*>(x); };
+      UpdateBwdFusedParams p;
+      memset(&p, 0, sizeof(p));
+      p.T = hp.T; p.dh = d.dh;
+      p.K = u16(hp.X); p.ldk = hp.ldx; p.bsk = hp.bsx;
+      p.V = u16(hp.Y); p.ldv = hp.ldy; p.bsv = hp.bsy;
+      p.W0 = u16(hp.W0); p.W1 = u16(hp.W1); p.W2 = u16(hp.W2); p.G0 = u16(hp.G0); p.G1 = u16(hp.G1); p.G2 = u16(hp.G2); p.bsw = hp.bsw;
+      p.lr0 = hp.lr0; p.lr1 = hp.lr1; p.lr2 = hp.lr2; p.bslr = hp.bslr;
+      p.O0 = static_cast<uint16_t*>(hp.O0); p.O1 = static_cast<uint16_t*>(hp.O1); p.O2 = static_cast<uint16_t*>(hp.O2); p.bso = hp.bso;
+      p.dk = reinterpret_cast<uint16_t*>(dk); p.dv = reinterpret_cast<uint16_t*>(dv); p.bsd = bsd;
+      p.lrpart = hp.lrpart; p.lr_stride = hp.lrpart_mat_stride; p.ldlr = hp.Tupd;
+      if (d.d == 64) launch_update_bwd_fused<64>(p);
+      else if (d.d == 96) launch_update_bwd_fused<96>(p);
+      else launch_update_bwd_fused<128>(p);
+    }
+  }
   template <typename U> U* scr(size_t off) const { return reinterpret_cast<U*>(sc + off); }
 
   long long hbs(int T_) const { return (long long)T_ * d.dh; }   // between the batch entries of a step's token-major arrays
@@ -1211,6 +1252,7 @@ struct Runner {
     std::vector<int> mg_updates;
     int mg_parts = P.nblk;   // partial dots per matrix in a momentum-gradient slot (the same for every update)
     std::vector<std::pair<int, int>> mg_ranges;
+    const bool bwd_fused = update_bwd_fused() && !lr_each;      // (ranges that repeat add their gradients up)
     const bool rows_on_side = !seen_q.force && !seen_kv.force && s_side != s_main;
     auto zero_rows = [&](hipStream_t zs) {
       ZeroList zl(d.b, zs);
@@ -1531,7 +1573,8 @@ struct Runner {
           hp.O3 = hp.O4 = hp.O5 = nullptr;
           z0 = pre(u, 0); z1 = pre(u, 1); z2 = pre(u, 2); zbs = pre_bs(u);
         }
-        launch_hidden(P.keep_pre ? 4 : 3, hp, T_);
+        if (bwd_fused) update_bwd_fused(hp, dk + (size_t)st.start * d.d, dv + (size_t)st.start * d.d, (long long)d.kv_len * d.d);
+        else launch_hidden(P.keep_pre ? 4 : 3, hp, T_);
       }
       const bool acc_kv = seen_kv.accumulate(st.start, st.end);
       // dk and dv share the launch of the token reduction below (when it runs on the asynchronous-copy kernel; otherwise they are
@@ -1562,7 +1605,7 @@ struct Runner {
         MomentumMeanRanges r1;
         r1.start[0] = st.start; r1.len[0] = T_;
         LACT_LAUNCH("k_lr_reduce", "k_lr_reduce", 0.0, k_lr_reduce, dim3(ceil_div(T_, 256), d.b, 3), dim3(256), s,
-                    scr<float>(P.t_lrpart) + (size_t)u * lrslot, 0LL, (long long)P.lr_slots * d.b * P.Tupd, (long long)d.b * P.Tupd, lr_parts(),
+                    scr<float>(P.t_lrpart) + (size_t)u * lrslot, 0LL, (long long)P.lr_slots * d.b * P.Tupd, (long long)d.b * P.Tupd, bwd_fused ? 1 : lr_parts(),
                     P.Tupd, dlr0, dlr1, dlr2, (long long)d.kv_len, r1, acc_kv ? 1 : 0);
       } else {
         lr_ranges.emplace_back(st.start, T_);
@@ -1578,8 +1621,8 @@ struct Runner {
         set_tr_term(jobs[2].t, h(2), d.dh, hbs(T_), kc, d.k_ld, d.k_bs);
         // the update before: its weights enter these as they are, unless Newton-Schulz output replaces them or an accumulator carries on
         gw = GradSum{(d.prenorm || (P.muon && d.muon_replaces_weight)) ? nullptr : gwhat, 0};
-        contribute(kBf16 ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, &rows_job);
-        if (!rows_job.done) {
+        contribute(kBf16 && !bwd_fused ? "update_bwd_dw_dk_dv" : "update_bwd_dw", jobs, T_, gw, bwd_fused ? nullptr : &rows_job);
+        if (!bwd_fused && !rows_job.done) {
           launch_row_gemm<T, false, 4, EPI_STORE>("update_bwd_dk", rows_job.r4, d.b, s, true);
           launch_row_gemm<T, true, 2, EPI_STORE>("update_bwd_dv", rows_job.r2, d.b, s, true);
         }
@@ -1598,7 +1641,7 @@ struct Runner {
         }
         LACT_LAUNCH("k_lr_reduce", "k_lr_reduce", 0.0, k_lr_reduce, dim3(ceil_div(longest, 256), d.b, 3 * n), dim3(256), s,
                     scr<float>(P.t_lrpart) + (size_t)u0 * lrslot, (long long)lrslot, (long long)P.lr_slots * d.b * P.Tupd, (long long)d.b * P.Tupd,
-                    lr_parts(), P.Tupd, dlr0, dlr1, dlr2, (long long)d.kv_len, r, 0);
+                    bwd_fused ? 1 : lr_parts(), P.Tupd, dlr0, dlr1, dlr2, (long long)d.kv_len, r, 0);
       }
     }
     if (!mg_updates.empty()) {

@@ -605,4 +605,291 @@ __global__ __launch_bounds__(256, 1) void k_update_fused(const UpdateFusedParams
   add(2, 0);
 }
 
+// ---- backward of an update: the tokens' gradients -------------------------------------------------------------------------------
+// From k, v, the weights and the gradients G of their gradients: the gradients of the pre-activations (stored, for the weights'
+// reduction over the tokens), dk, dv and the learning rates'.  A wave owns 32 tokens as matrix columns and walks the hidden units 32
+// at a time: six products, the pointwise part in registers, and the six terms of dk and dv, which take its results as they lie.  The
+// weights' and gradients' 32 rows (or columns) travel through a ring shared by the block.
+//
+// What bounds it: issue of the one wave on a SIMD, 1130 vector operations a stage (64 a hidden value, of which 19 round) in 6300 clocks; the
+// terms' matrix instructions hide behind them, the six products' do not (1800), and 512 registers hold no second set of their sums.
+// Copies: 800.  us, this kernel and the reduction / hidden stage and the reduction with dk and dv beside it: 12 x 4680 tokens, d = 128,
+// dh = 256 96 + 28 / 92 + 62; 24 x 2500 tokens, d = dh = 96 39 + 14 / 46 + 38.  Six arrays of [tokens, hidden] less written and nine
+// less read than there: three are written here, for the reduction.
+struct UpdateBwdFusedParams {
+  int T, dh;
+  const uint16_t* K; int ldk; long long bsk;               // [T, d]
+  const uint16_t* V; int ldv; long long bsv;
+  const uint16_t* W0; const uint16_t* W1; const uint16_t* W2;
+  const uint16_t* G0; const uint16_t* G1; const uint16_t* G2; long long bsw;
+  const float* lr0; const float* lr1; const float* lr2; long long bslr;
+  uint16_t* O0; uint16_t* O1; uint16_t* O2; long long bso; // [T, dh]: gradients of k W0^T, v W1, k W2^T
+  uint16_t* dk; uint16_t* dv; long long bsd;               // [T, d], rows one after the other
+  float* lrpart; long long lr_stride;                      // [3][b][..]: sums for the learning rates
+  int ldlr;
+  TileMap map;                                             // 128 tokens, 1, batch
+};
+
+template <int D>
+struct BwdStage {
+  using U = UpdatePatch<D>;
+  static constexpr int SIDE = U::BYTES, TALL = D * 64;     // 32 rows of W0, W2, G0, G2; [d][32] of W1, G1
+  static constexpr int BYTES = 4 * SIDE + 2 * TALL, RING = 3 * BYTES, LDS = cmax(RING, 4 * 32 * (D + 8) * 2);
+  static_assert(LDS <= 160 * 1024, "the ring does not fit the LDS");
+};
+
+// The pointwise part on four hidden units of a token, in eight steps.  Roundings as in update_pointwise2.  One operation on all four
+// after the other: in the compiler's order, each result right behind its operands, a wave alone on its SIMD waits for most of them.
+struct BwdSteps {
+  float g[4], h2[4], dh[4], z0[4], z1[4], z2[4];           // the rounded products
+  float sig[4], silu[4], om[4], d1[4], d2[4], sg[4], sb[4], hid[4], dh2[4], p[4], t[4], x[4];
+  uint32_t w[6][2];                                        // gradients of k W0^T, k W2^T; lr-scaled dgate, dhidden; gradient of v W1; lr-scaled hidden
+  template <class F>
+  __device__ __forceinline__ void each(F f) const {
+#pragma unroll
+    for (int j = 0; j < 4; ++j) f(j);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  __device__ __forceinline__ void pack(uint32_t (&o)[2]) const {
+    o[0] = pack_bf16(x[0], x[1]); o[1] = pack_bf16(x[2], x[3]);
+  }
+  template <int STEP, int I>
+  __device__ __forceinline__ void step(const f32x16 (&a)[6], float l0, float l1, float l2, float& s0, float& s1, float& s2) {
+    if (STEP == 0) {
+      each([&](int j) { g[j] = round_bf16(a[0][4 * I + j]); h2[j] = round_bf16(a[1][4 * I + j]); dh[j] = round_bf16(a[4][4 * I + j]); });
+      each([&](int j) { z0[j] = round_bf16(a[2][4 * I + j]); z2[j] = round_bf16(a[3][4 * I + j]); z1[j] = round_bf16(a[5][4 * I + j]); });
+    } else if (STEP == 1) {
+      each([&](int j) { sig[j] = sigmoidf_(g[j]); p[j] = dh[j] * h2[j]; });
+      each([&](int j) { silu[j] = g[j] * sig[j]; om[j] = 1.f - sig[j]; });
+      each([&](int j) { sg[j] = round_bf16(silu[j]); sb[j] = round_bf16(sig[j]); });
+    } else if (STEP == 2) {
+      each([&](int j) { hid[j] = sg[j] * h2[j]; dh2[j] = dh[j] * sg[j]; });
+      each([&](int j) { hid[j] = round_bf16(hid[j]); dh2[j] = round_bf16(dh2[j]); t[j] = round_bf16(p[j]); });
+      each([&](int j) { t[j] *= sb[j]; sb[j] = 1.f - sb[j]; d1[j] = __builtin_fmaf(g[j], om[j], 1.f); });
+      each([&](int j) { t[j] = round_bf16(t[j]); sb[j] = round_bf16(sb[j]); d1[j] *= sig[j]; });
+    } else if (STEP == 3) {
+      each([&](int j) { sb[j] *= g[j]; d2[j] = __builtin_fmaf(-2.f, sig[j], 1.f); om[j] *= sig[j]; });
+      each([&](int j) { sb[j] = round_bf16(sb[j]); d2[j] = __builtin_fmaf(g[j], d2[j], 2.f); });
+      each([&](int j) { sb[j] += 1.f; d2[j] *= om[j]; });
+      each([&](int j) { sb[j] = round_bf16(sb[j]); d2[j] *= p[j]; });
+    } else if (STEP == 4) {
+      each([&](int j) { t[j] *= sb[j]; s1 = __builtin_fmaf(z1[j], hid[j], s1); x[j] = hid[j] * l1; });
+      pack(w[5]);
+      each([&](int j) { t[j] = round_bf16(t[j]); s2 = __builtin_fmaf(z2[j], dh2[j], s2); x[j] = dh2[j] * l2; });      // t: dgate before the activation
+      pack(w[3]);
+    } else if (STEP == 5) {
+      each([&](int j) { s0 = __builtin_fmaf(z0[j], t[j], s0); x[j] = t[j] * l0; });
+      pack(w[2]);
+      each([&](int j) { z0[j] *= l0; z1[j] *= l1; z2[j] *= l2; });
+      each([&](int j) { h2[j] *= d1[j]; dh[j] *= d1[j]; });
+    } else if (STEP == 6) {
+      each([&](int j) { x[j] = z0[j] * h2[j]; t[j] = z0[j] * dh[j]; });
+      each([&](int j) { x[j] = __builtin_fmaf(z2[j], silu[j], x[j]); t[j] = __builtin_fmaf(z1[j], silu[j], t[j]); });
+      pack(w[4]);
+      each([&](int j) { x[j] = t[j]; });
+      pack(w[1]);
+    } else {
+      each([&](int j) { x[j] = z0[j] * d2[j]; });
+      each([&](int j) { x[j] = __builtin_fmaf(z2[j], dh[j], x[j]); });
+      each([&](int j) { x[j] = __builtin_fmaf(z1[j], h2[j], x[j]); });
+      pack(w[0]);
+    }
+  }
+};
+
+template <int D>
+__global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFusedParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  using ST = BwdStage<D>;
+  using U = UpdatePatch<D>;
+  int bx, by, z;
+  if (!p.map.locate(blockIdx.x, bx, by, z)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, h = lane >> 5;
+  const int row0 = (bx * 4 + wave) * 32, row = row0 + (lane & 31), dh = p.dh, n = dh / 32;
+  const uint32_t lds0 = lds_addr(smem);
+  const long long w = z * p.bsw;
+  // copies: a quarter of every operand's KiB each, the operands of a kind at the same offsets
+  UpdateCopies<D> cp;
+  cp.init(D);
+  const uint32_t tall_off = (uint32_t)((lane >> 2) * dh + ((lane & 3) ^ ((lane >> 4) & 3)) * 8) * 2;
+  uint32_t side_off = cp.voff[0];
+#pragma unroll
+  for (int i = 1; i < 4; ++i) side_off = wave == i ? cp.voff[i] : side_off;
+  auto issue = [&](int t, int slot) {
+    const uint32_t to = lds0 + slot;
+    const long long rows = w + (long long)t * 32 * D, cols = w + t * 32;
+    const uint16_t* const side[4] = {p.W0 + rows, p.W2 + rows, p.G0 + rows, p.G2 + rows};
+    const uint16_t* const tall[2] = {p.W1 + cols, p.G1 + cols};
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int j = 0; j < U::COPIES / 4; ++j) dma16<false>(side[m] + (size_t)j * 16 * D, side_off, to + m * ST::SIDE + (wave + 4 * j) * 1024);
+#pragma unroll
+    for (int m = 0; m < 2; ++m)
+#pragma unroll
+      for (int j = 0; j < (D / 16 + 3) / 4; ++j)
+        if (wave + 4 * j < D / 16)
+          dma16<false>(tall[m] + (size_t)(wave + 4 * j) * 16 * dh, tall_off, to + 4 * ST::SIDE + m * ST::TALL + (wave + 4 * j) * 1024);
+  };
+  issue(0, 0);
+  constexpr int KS = D / 16, DT = D / 32;
+  bf16x8 kf[KS], vf[KS];
+  attn_own_rows<D>(kf, p.K + z * p.bsk, p.ldk, row, p.T);
+  attn_own_rows<D>(vf, p.V + z * p.bsv, p.ldv, row, p.T);
+  const int token = min(row, p.T - 1);
+  const float l0 = p.lr0[z * p.bslr + token], l1 = p.lr1[z * p.bslr + token], l2 = p.lr2[z * p.bslr + token];
+  AttnFrag<U::P> frag;
+  frag.init();
+  // [d][32 hidden]: 16 rows of d transposed; 32 rows of d over 16 hidden units in the order of the products' results
+  uint32_t tr_off[2], row_off[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    tr_off[i] = (8 * h + ((lane & 15) >> 2) + 4 * i) * 64 + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ ((2 * h + i) & 3)) << 4) + (lane & 1) * 8;
+    row_off[i] = (lane & 31) * 64 + ((i ^ ((lane >> 2) & 3)) << 4) + h * 8;
+  }
+  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+  typedef short s16x8 __attribute__((ext_vector_type(8)));
+  auto tall_tr = [&](const char* m, int ks) {
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(m + tr_off[0] + ks * 1024)), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(m + tr_off[1] + ks * 1024));
+    const s16x8 v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return __builtin_bit_cast(bf16x8, v);
+  };
+  auto tall_rows = [&](const char* m, int dt, int st) {      // (16 hidden units further: the granules two on, a bit of the slot)
+    const uint2 a = *reinterpret_cast<const uint2*>(m + dt * 2048 + (row_off[0] ^ (st << 5))), b = *reinterpret_cast<const uint2*>(m + dt * 2048 + (row_off[1] ^ (st << 5)));
+    return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
+  };
+
+  f32x16 dk[DT], dv[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) dk[i][j] = dv[i][j] = 0.f;
+  uint32_t res[6][8];      // of the units in hand, two a word, in the order of the operands in LDS
+#pragma unroll
+  for (int m = 0; m < 6; ++m)
+#pragma unroll
+    for (int j = 0; j < 8; ++j) res[m][j] = 0;
+  float s0 = 0.f, s1 = 0.f, s2 = 0.f;
+
+  // terms [from, to) of dk and dv over 16 hidden units (half st of the stage), their weights read two ahead
+  constexpr int TERMS = 6 * DT;
+  bf16x8 tf[3];
+  auto term_read = [&](const char* stage, int st, int i) {
+    if (i >= TERMS) return;
+    const int m = i / DT, dt = i % DT;
+    tf[i % 3] = m < 4 ? frag.cols(stage + m * ST::SIDE, dt, st) : tall_rows(stage + 4 * ST::SIDE + (m - 4) * ST::TALL, dt, st);
+  };
+  auto term = [&](const char* stage, int st, int i) {
+    const int m = i / DT, dt = i % DT;
+    term_read(stage, st, i + 2);
+    const bf16x8 r = __builtin_bit_cast(bf16x8, make_uint4(res[m][4 * st], res[m][4 * st + 1], res[m][4 * st + 2], res[m][4 * st + 3]));
+    if (m < 4) dk[dt] = mma32(tf[i % 3], r, dk[dt]);
+    else dv[dt] = mma32(tf[i % 3], r, dv[dt]);
+  };
+  f32x16 a[6];
+  // Two rounds of four hidden units, between their steps the terms of the 16 units before.
+  auto rounds = [&](auto half, const char* stage, int st) {
+    constexpr int H = decltype(half)::value;
+    BwdSteps b;
+    int done = 0;
+    term_read(stage, st, 0);
+    term_read(stage, st, 1);
+    auto terms = [&](int upto) {
+#pragma unroll
+      for (int i = 0; i < TERMS; ++i)
+        if (i >= done && i < upto) term(stage, st, i);
+      done = upto;
+      __builtin_amdgcn_sched_barrier(0);
+    };
+    auto round = [&](auto rd) {
+      constexpr int I = decltype(rd)::value, AT = (I - 2 * H) * 8;
+      b.step<0, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 1) * TERMS / 16);
+      b.step<1, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 2) * TERMS / 16);
+      b.step<2, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 3) * TERMS / 16);
+      b.step<3, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 4) * TERMS / 16);
+      b.step<4, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 5) * TERMS / 16);
+      b.step<5, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 6) * TERMS / 16);
+      b.step<6, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 7) * TERMS / 16);
+      b.step<7, I>(a, l0, l1, l2, s0, s1, s2); terms((AT + 8) * TERMS / 16);
+#pragma unroll
+      for (int m = 0; m < 6; ++m)
+#pragma unroll
+        for (int i = 0; i < 2; ++i) res[m][2 * I + i] = b.w[m][i];
+    };
+    round(std::integral_constant<int, 2 * H>{});
+    round(std::integral_constant<int, 2 * H + 1>{});
+  };
+  // 16 bytes a lane: the lower half of the wave gets the eight units of the first round, the upper half those of the second
+  // (lanes past the last token hold its values and write them once more: no branch between the steps, across which the compiler would
+  // move work that the matrix instructions are to hide behind)
+  const long long mine = z * p.bso + (long long)token * dh + 8 * h;
+  uint16_t* const out[3] = {p.O0 + mine, p.O2 + mine, p.O1 + mine};
+  auto store = [&](int t, int H) {
+#pragma unroll
+    for (int o = 0; o < 3; ++o) {
+      const uint32_t* r = res[o == 2 ? 4 : o];
+      const auto x = __builtin_amdgcn_permlane32_swap(r[4 * H], r[4 * H + 2], false, false), y = __builtin_amdgcn_permlane32_swap(r[4 * H + 1], r[4 * H + 3], false, false);
+      *reinterpret_cast<uint4*>(out[o] + t * 32 + 16 * H) = make_uint4(x[0], y[0], x[1], y[1]);
+    }
+  };
+  wait_vmcnt<0>();
+  int prev = 0, cur = 0, next = ST::BYTES;      // the ring's stages (the first one stands for the one before it)
+  for (int t = 0; t < n; ++t) {
+    wait_vmcnt<6>();      // behind this stage's copies come the six stores of the stage before only
+    __builtin_amdgcn_s_barrier();      // (__syncthreads would wait for the stores as well; what LDS was asked for has been used)
+    issue(min(t + 1, n - 1), next);
+    const char* stage = smem + cur;
+    {
+      bf16x8 f[2][4];
+      auto read = [&](int ks) {
+#pragma unroll
+        for (int m = 0; m < 4; ++m)
+          if (ks < KS) f[ks & 1][m] = frag.rows(stage + m * ST::SIDE, 0, ks);
+        if (ks >= KS && ks < 2 * KS)
+#pragma unroll
+          for (int m = 0; m < 2; ++m) f[ks & 1][m] = tall_tr(stage + 4 * ST::SIDE + m * ST::TALL, ks - KS);
+      };
+      read(0);
+#pragma unroll
+      for (int m = 0; m < 6; ++m)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) a[m][j] = 0.f;
+#pragma unroll
+      for (int ks = 0; ks < 2 * KS; ++ks) {
+        read(ks + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (ks < KS) {
+#pragma unroll
+          for (int m = 0; m < 4; ++m) a[m] = mma32(f[ks & 1][m], kf[ks % KS], a[m]);
+        } else {
+#pragma unroll
+          for (int m = 0; m < 2; ++m) a[4 + m] = mma32(f[ks & 1][m], vf[ks % KS], a[4 + m]);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+    rounds(std::integral_constant<int, 0>{}, smem + prev, 1);      // (the first time of zeros)
+    store(t, 0);
+    rounds(std::integral_constant<int, 1>{}, stage, 0);
+    store(t, 1);
+    prev = cur; cur = next; next = next == 2 * ST::BYTES ? 0 : next + ST::BYTES;
+  }
+  term_read(smem + prev, 1, 0);
+  term_read(smem + prev, 1, 1);
+#pragma unroll
+  for (int i = 0; i < TERMS; ++i) term(smem + prev, 1, i);
+  s0 += __shfl_xor(s0, 32, 64); s1 += __shfl_xor(s1, 32, 64); s2 += __shfl_xor(s2, 32, 64);
+  if (lane < 32 && row < p.T) {
+    float* o = p.lrpart + (size_t)z * p.ldlr + row;
+    o[0] = s0; o[p.lr_stride] = s1; o[2 * p.lr_stride] = s2;
+  }
+  wait_vmcnt<0>();
+  __syncthreads();
+  char* t = smem + wave * 32 * (D + 8) * 2;
+  if (row0 < p.T) {
+    attn_store_rows<D>(t, dk, 1.f, p.dk + z * p.bsd, D, row0, p.T);
+    attn_store_rows<D>(t, dv, 1.f, p.dv + z * p.bsd, D, row0, p.T);
+  }
+}
+
 }  // namespace lact

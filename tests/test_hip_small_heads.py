@@ -108,3 +108,47 @@ def test_infinite_tokens_stay_in_their_head(token):
         for a, r in zip(run(), in_pieces(run)):
             fine = torch.isfinite(a.float()).flatten(1).all(dim=1)
             assert torch.equal(fine, torch.isfinite(r.float()).flatten(1).all(dim=1)) and fine.tolist() == [True, False, True]
+
+
+# tokens at the edges of a wave's 32 and a block's 128; one and several stages of 32 hidden units (the ring has three places); all with
+# batch enough that the one kernel is taken
+@pytest.mark.parametrize("b,T,d,dh", [(200, 33, 64, 32), (128, 129, 64, 64), (5, 4700, 64, 96), (90, 200, 96, 96), (100, 127, 128, 64), (120, 129, 128, 96),
+                                      (250, 100, 128, 160), (250, 63, 128, 256)])
+def test_tokens_gradients_in_one_kernel(b, T, d, dh):
+    """Gradients of a program of two updates: the same products of the same rounded values in another order, on top of weights that the
+    forward's kernels sum in another order too (an entry in 1e2 to 1e3 moved by 2^-8, 4e-4 in norm, through a chain of a few
+    products; 3e-3).  Rows around the steps stay zero."""
+    print("[gpu-test] tokens' gradients in one kernel", b, T, d, dh, flush=True)
+    at, L = 5, 2 * T + 9
+    inp = {n: x.to(DEV) for n, x in O.make_inputs(b, L, d, dh, seed=65, act_dtype=torch.bfloat16).items()}
+    inp["momentum"] = torch.full((b, L, 1), 0.7, device=DEV)
+    wide = torch.zeros(b, L, 2 * d + 8, dtype=torch.bfloat16, device=DEV)
+    wide[..., 8:d + 8], wide[..., d + 8:] = inp["k"], inp["v"]
+    prog = ops.Program(steps=((LACT_UPDATE, at, at + T, 0), (LACT_APPLY, 0, T, 0), (LACT_UPDATE, at + T, at + 2 * T, 0), (LACT_APPLY, T, L, T)), out_len=L)
+    go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(3)).bfloat16().to(DEV)
+    names = list(ORDER) + ["momentum"]
+
+    def run(views):
+        t = {n: x.clone().requires_grad_(True) for n, x in inp.items() if n in names}
+        if views:
+            packed = wide.clone().requires_grad_(True)
+            k, v = packed[..., 8:d + 8], packed[..., d + 8:]
+        else:
+            k, v = t["k"], t["v"]
+        out, ws, _ = ops.run_program(prog, *[t[n] for n in ORDER[:4]], k, v, *[t[n] for n in ORDER[6:]], momentum=t["momentum"])
+        loss = [out] + list(ws)
+        seeds = [go] + [torch.ones_like(w) * 0.01 for w in ws]
+        wanted = [t[n] for n in names if n not in ("k", "v")] + ([packed] if views else [t["k"], t["v"]])
+        g = list(torch.autograd.grad(loss, wanted, seeds))
+        if views:
+            p = g.pop()
+            assert float(p[..., :8].float().abs().max()) == 0
+            g += [p[..., 8:d + 8], p[..., d + 8:]]
+        return g
+
+    whole, view, ref = run(False), run(True), in_pieces(lambda: run(False))
+    for n, a, c, r in zip([n for n in names if n not in ("k", "v")] + ["k", "v"], whole, view, ref):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, c), n
+        assert O.rel_l2(a, r) < 3e-3, (n, O.rel_l2(a, r))
+        if n in ("k", "v", "lr0", "lr1", "lr2"):
+            assert float(a[:, :at].float().abs().max()) == 0 and float(a[:, at + 2 * T:].float().abs().max()) == 0

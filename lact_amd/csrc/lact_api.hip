@@ -668,19 +668,52 @@ struct Runner {
     }
     return 0;
   }
-  // Whether the backward of the program's updates forms the tokens' gradients in one kernel.  A round of its blocks takes 14 us and 3.3 to
-  // 4 (d = 64 to 128) per 32 hidden units however few blocks there are, the kernels in pieces 17 us and then by the work: 126 us at
-  // 12 x 4680 tokens, d = 128, dh = 256 (hidden stage 92, token rows beside the reduction 34).  us of a training step of four updates and
-  // applies, in pieces / with the one kernel (without Newton-Schulz): 12 x 4096 tokens, 128 x 256 1260 / 1044, 12 x 1024 497 / 488,
-  // 12 x 256 368 / 394; 48 x 1024, 64 x 128 691 / 558.
+  // The hidden stage of an apply's backward and dq as one kernel, for the head sizes it exists for; `dq`: rows of the (first) step.
+  template <int D>
+  void launch_apply_bwd_fused(ApplyBwdFusedParams p, int nz) const {
+    constexpr int SM = ApplyBwdStage<D>::LDS;
+    LACT_BIG_LDS((k_apply_bwd_fused<D>), SM);
+    p.map = make_tile_map(ceil_div(p.T, 256), 1, nz);
+    LACT_LAUNCH_SMEM("k_apply_bwd_fused", "apply_bwd", 10.0 * p.T * D * p.dh * nz, (k_apply_bwd_fused<D>), dim3(p.map.grid()), dim3(512), SM, s, p);
+  }
+  // us of a training step of four updates and applies with Newton-Schulz, in pieces / as one kernel: 12 x 4096 tokens, 96 x 96 705 / 668,
+  // 48 x 1024, 128 x 256 1643 / 1600, 2 x 1024 463 / 477.  A round takes 8 us and 2.4 per 32 hidden units, the hidden stage and dq as kernels of
+  // their own 18 us and then by the hidden values (43 + 17 us at 12 x 4680 tokens, d = 128, dh = 256; 35 as one).
+  bool apply_bwd_fused(int tokens, int nz) const {
+    if (!kBf16 || g_persist != 1 || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
+    const double pieces = 18 + 45.0 * tokens * nz / (12 * 4680) * d.dh / 256 * (0.5 + d.d / 256.0);
+    return 8 + ceil_div(ceil_div(tokens, 256) * nz, 256) * 2.4 * (d.dh / 32) < pieces;
+  }
+  void apply_bwd_fused(const HiddenParams& hp, T* dq, long long gsd, int nz) const {
+    if constexpr (kBf16) {
+      auto u16 = [](const void* x) { return static_cast<const uint16_t*>(x); };
+      ApplyBwdFusedParams p;
+      memset(&p, 0, sizeof(p));
+      p.T = hp.T; p.dh = d.dh;
+      p.X = u16(hp.X); p.ldx = hp.ldx; p.bsx = hp.bsx; p.gsx = hp.gsx;
+      p.Y = u16(hp.Y); p.ldy = hp.ldy; p.bsy = hp.bsy; p.gsy = hp.gsy;
+      p.W0 = u16(hp.W0); p.W1 = u16(hp.W1); p.W2 = u16(hp.W2); p.bsw = hp.bsw; p.gsw = hp.gsw;
+      p.O0 = static_cast<uint16_t*>(hp.O0); p.O1 = static_cast<uint16_t*>(hp.O1); p.O2 = static_cast<uint16_t*>(hp.O2); p.bso = hp.bso;
+      p.dq = reinterpret_cast<uint16_t*>(dq); p.bsd = (long long)d.q_len * d.d; p.gsd = gsd;
+      p.steps = hp.steps;
+      if (d.d == 64) launch_apply_bwd_fused<64>(p, nz);
+      else if (d.d == 96) launch_apply_bwd_fused<96>(p, nz);
+      else launch_apply_bwd_fused<128>(p, nz);
+    }
+  }
+  // Whether the backward of the program's updates forms the tokens' gradients in one kernel.  It takes 10 us and, a round of its blocks
+  // however few there are, 6 and 3.3 to 4 (d = 64 to 128) per 32 hidden units; the kernels in pieces 17 us and then by the hidden values,
+  // more so the longer the products: 126 us at 12 x 4680 tokens, d = 128, dh = 256 (hidden stage 92, token rows beside the reduction 34).
+  // us of a training step of four updates and applies (without Newton-Schulz), with this part in pieces / as one kernel: 12 x 4096 tokens,
+  // 128 x 256 1195 / 1044, 12 x 256 tokens 337 / 394; 48 x 1024, 64 x 128 630 / 558, 96 x 96 648 / 568.
   bool update_bwd_fused() const {
     if (!kBf16 || g_persist != 1 || g_keep_pre >= 0 || P.keep_pre || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
     double pieces = 0, one = 0;
     for (const auto& st : P.live)
       if (st.kind == LACT_UPDATE) {
         const int T_ = st.end - st.start;
-        pieces += 17 + 126.0 * d.b * T_ / (12 * 4680) * d.d * d.dh / (128 * 256);
-        one += ceil_div(ceil_div(T_, 128) * d.b, 256) * (14 + (2.6 + d.d / 90.0) * (d.dh / 32));
+        pieces += 17 + 126.0 * d.b * T_ / (12 * 4680) * d.dh / 256 * (0.5 + d.d / 256.0);
+        one += 10 + ceil_div(ceil_div(T_, 128) * d.b, 256) * (6 + (2.6 + d.d / 90.0) * (d.dh / 32));
       }
     return one < pieces;
   }
@@ -1252,7 +1285,13 @@ struct Runner {
     std::vector<int> mg_updates;
     int mg_parts = P.nblk;   // partial dots per matrix in a momentum-gradient slot (the same for every update)
     std::vector<std::pair<int, int>> mg_ranges;
-    const bool bwd_fused = update_bwd_fused() && !lr_each;      // (ranges that repeat add their gradients up)
+    // (ranges that repeat add their gradients up)
+    const bool bwd_fused = update_bwd_fused() && !lr_each;
+    bool q_repeats = seen_q.force;
+    for (size_t i = 0; i < P.live.size(); ++i)
+      for (size_t j = i + 1; j < P.live.size() && P.live[i].kind == LACT_APPLY; ++j)
+        if (P.live[j].kind == LACT_APPLY && P.live[i].start < P.live[j].end && P.live[j].start < P.live[i].end) q_repeats = true;
+    auto dq_fused = [&](const ApplyGroup& g) { return !q_repeats && apply_bwd_fused(g.st.end - g.st.start, d.b * g.n); };
     const bool rows_on_side = !seen_q.force && !seen_kv.force && s_side != s_main;
     auto zero_rows = [&](hipStream_t zs) {
       ZeroList zl(d.b, zs);
@@ -1294,9 +1333,11 @@ struct Runner {
         hp.steps.by_nb = make_udiv(d.b);
         hp.gsx = (long long)g.dstart * d.q_ld; hp.gsy = (long long)g.dout * d.do_ld; hp.gsw = (long long)P.mat3;
       }
-      launch_hidden(2, hp, T_, g.n);
+      if (dq_fused(g)) apply_bwd_fused(hp, dq + (size_t)g.st.start * d.d, (long long)g.dstart * d.d, d.b * g.n);
+      else launch_hidden(2, hp, T_, g.n);
     };
     auto dq_gemm = [&](const ApplyGroup& g) {   // dq = gY0 W0 + gY2 W2
+      if (dq_fused(g)) return;
       const int T_ = g.st.end - g.st.start;
       auto p = row_params<2>();
       set_term(p.t[0], h(1), d.dh, hbs(T_), wc(g.ver, 0), d.d, P.g.elems, d.dh);

@@ -638,6 +638,43 @@ struct BwdStage {
   static_assert(LDS <= 160 * 1024, "the ring does not fit the LDS");
 };
 
+// A stage of W1 or G1 in LDS: [d][32 hidden], rows of 64 bytes, granule g of row r at slot g ^ (r >> 2) & 3.
+struct TallFrag {
+  uint32_t tr_off[2], row_off[2];
+  // of a copy of 16 rows, within the operand
+  __device__ static __forceinline__ uint32_t copy_offset(int dh) {
+    const int lane = threadIdx.x & 63;
+    return (uint32_t)((lane >> 2) * dh + ((lane & 3) ^ ((lane >> 4) & 3)) * 8) * 2;
+  }
+  __device__ __forceinline__ void init() {
+    const int lane = threadIdx.x & 63, h = lane >> 5;
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      tr_off[i] = (8 * h + ((lane & 15) >> 2) + 4 * i) * 64 + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ ((2 * h + i) & 3)) << 4) + (lane & 1) * 8;
+      row_off[i] = (lane & 31) * 64 + ((i ^ ((lane >> 2) & 3)) << 4) + h * 8;
+    }
+  }
+  // the 32 hidden units as matrix rows over 16 of d
+  __device__ __forceinline__ bf16x8 columns(const char* m, int ks) const {
+    typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+    typedef short s16x8 __attribute__((ext_vector_type(8)));
+    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(m + tr_off[0] + ks * 1024)), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(m + tr_off[1] + ks * 1024));
+    const s16x8 v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
+    return __builtin_bit_cast(bf16x8, v);
+  }
+  // 32 of d as matrix rows over 16 hidden units in the order of the products' results (the upper 16: granules two on, a bit of the slot)
+  __device__ __forceinline__ bf16x8 rows(const char* m, int dt, int st) const {
+    const uint2 a = *reinterpret_cast<const uint2*>(m + dt * 2048 + (row_off[0] ^ (st << 5))), b = *reinterpret_cast<const uint2*>(m + dt * 2048 + (row_off[1] ^ (st << 5)));
+    return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
+  }
+};
+// Sixteen hidden units (two rounds of four a lane half, two words each, r and r + 2) of a token, 16 bytes a lane: the lower half of
+// the wave writes the eight units of the first round, the upper half those of the second.
+__device__ __forceinline__ void store_units(uint16_t* out, const uint32_t* r) {
+  const auto x = __builtin_amdgcn_permlane32_swap(r[0], r[2], false, false), y = __builtin_amdgcn_permlane32_swap(r[1], r[3], false, false);
+  *reinterpret_cast<uint4*>(out) = make_uint4(x[0], y[0], x[1], y[1]);
+}
+
 // The pointwise part on four hidden units of a token, in eight steps.  Roundings as in update_pointwise2.  One operation on all four
 // after the other: in the compiler's order, each result right behind its operands, a wave alone on its SIMD waits for most of them.
 struct BwdSteps {
@@ -711,7 +748,7 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
   // copies: a quarter of every operand's KiB each, the operands of a kind at the same offsets
   UpdateCopies<D> cp;
   cp.init(D);
-  const uint32_t tall_off = (uint32_t)((lane >> 2) * dh + ((lane & 3) ^ ((lane >> 4) & 3)) * 8) * 2;
+  const uint32_t tall_off = TallFrag::copy_offset(dh);
   uint32_t side_off = cp.voff[0];
 #pragma unroll
   for (int i = 1; i < 4; ++i) side_off = wave == i ? cp.voff[i] : side_off;
@@ -740,25 +777,8 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
   const float l0 = p.lr0[z * p.bslr + token], l1 = p.lr1[z * p.bslr + token], l2 = p.lr2[z * p.bslr + token];
   AttnFrag<U::P> frag;
   frag.init();
-  // [d][32 hidden]: 16 rows of d transposed; 32 rows of d over 16 hidden units in the order of the products' results
-  uint32_t tr_off[2], row_off[2];
-#pragma unroll
-  for (int i = 0; i < 2; ++i) {
-    tr_off[i] = (8 * h + ((lane & 15) >> 2) + 4 * i) * 64 + (((2 * ((lane >> 4) & 1) + ((lane & 3) >> 1)) ^ ((2 * h + i) & 3)) << 4) + (lane & 1) * 8;
-    row_off[i] = (lane & 31) * 64 + ((i ^ ((lane >> 2) & 3)) << 4) + h * 8;
-  }
-  typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
-  typedef short s16x8 __attribute__((ext_vector_type(8)));
-  auto tall_tr = [&](const char* m, int ks) {
-    const s16x4 a = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(m + tr_off[0] + ks * 1024)), b = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(m + tr_off[1] + ks * 1024));
-    const s16x8 v = {a[0], a[1], a[2], a[3], b[0], b[1], b[2], b[3]};
-    return __builtin_bit_cast(bf16x8, v);
-  };
-  auto tall_rows = [&](const char* m, int dt, int st) {      // (16 hidden units further: the granules two on, a bit of the slot)
-    const uint2 a = *reinterpret_cast<const uint2*>(m + dt * 2048 + (row_off[0] ^ (st << 5))), b = *reinterpret_cast<const uint2*>(m + dt * 2048 + (row_off[1] ^ (st << 5)));
-    return __builtin_bit_cast(bf16x8, make_uint4(a.x, a.y, b.x, b.y));
-  };
-
+  TallFrag tall_frag;
+  tall_frag.init();
   f32x16 dk[DT], dv[DT];
 #pragma unroll
   for (int i = 0; i < DT; ++i)
@@ -777,7 +797,7 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
   auto term_read = [&](const char* stage, int st, int i) {
     if (i >= TERMS) return;
     const int m = i / DT, dt = i % DT;
-    tf[i % 3] = m < 4 ? frag.cols(stage + m * ST::SIDE, dt, st) : tall_rows(stage + 4 * ST::SIDE + (m - 4) * ST::TALL, dt, st);
+    tf[i % 3] = m < 4 ? frag.cols(stage + m * ST::SIDE, dt, st) : tall_frag.rows(stage + 4 * ST::SIDE + (m - 4) * ST::TALL, dt, st);
   };
   auto term = [&](const char* stage, int st, int i) {
     const int m = i / DT, dt = i % DT;
@@ -819,18 +839,13 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
     round(std::integral_constant<int, 2 * H>{});
     round(std::integral_constant<int, 2 * H + 1>{});
   };
-  // 16 bytes a lane: the lower half of the wave gets the eight units of the first round, the upper half those of the second
   // (lanes past the last token hold its values and write them once more: no branch between the steps, across which the compiler would
   // move work that the matrix instructions are to hide behind)
   const long long mine = z * p.bso + (long long)token * dh + 8 * h;
   uint16_t* const out[3] = {p.O0 + mine, p.O2 + mine, p.O1 + mine};
   auto store = [&](int t, int H) {
 #pragma unroll
-    for (int o = 0; o < 3; ++o) {
-      const uint32_t* r = res[o == 2 ? 4 : o];
-      const auto x = __builtin_amdgcn_permlane32_swap(r[4 * H], r[4 * H + 2], false, false), y = __builtin_amdgcn_permlane32_swap(r[4 * H + 1], r[4 * H + 3], false, false);
-      *reinterpret_cast<uint4*>(out[o] + t * 32 + 16 * H) = make_uint4(x[0], y[0], x[1], y[1]);
-    }
+    for (int o = 0; o < 3; ++o) store_units(out[o] + t * 32 + 16 * H, res[o == 2 ? 4 : o] + 4 * H);
   };
   wait_vmcnt<0>();
   int prev = 0, cur = 0, next = ST::BYTES;      // the ring's stages (the first one stands for the one before it)
@@ -847,7 +862,7 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
           if (ks < KS) f[ks & 1][m] = frag.rows(stage + m * ST::SIDE, 0, ks);
         if (ks >= KS && ks < 2 * KS)
 #pragma unroll
-          for (int m = 0; m < 2; ++m) f[ks & 1][m] = tall_tr(stage + 4 * ST::SIDE + m * ST::TALL, ks - KS);
+          for (int m = 0; m < 2; ++m) f[ks & 1][m] = tall_frag.columns(stage + 4 * ST::SIDE + m * ST::TALL, ks - KS);
       };
       read(0);
 #pragma unroll
@@ -890,6 +905,135 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
     attn_store_rows<D>(t, dk, 1.f, p.dk + z * p.bsd, D, row0, p.T);
     attn_store_rows<D>(t, dv, 1.f, p.dv + z * p.bsd, D, row0, p.T);
   }
+}
+
+// ---- backward of an apply: the hidden stage and dq ------------------------------------------------------------------------------
+//   g, u, e = q W0^T, q W2^T, dout W1  ->  hidden, dg, du [T, dh] (stored, for the weights' gradients);  dq = dg W0 + du W2
+// As above with three products and two terms: two waves fit a SIMD and cover each other's latencies, 256 tokens a block.
+//
+// What bounds it: memory, 130 MB read and written at 12 x 4680 tokens, d = 128, dh = 256 in 35 us (27 at a large copy's rate); as kernels
+// of their own the hidden stage takes 43 us and dq 17, and dq reads two of the arrays again.  24 x 2500 tokens, d = dh = 96: 20 / 23 + 9.
+struct ApplyBwdFusedParams {
+  int T, dh;
+  const uint16_t* X; int ldx; long long bsx;               // [T, d] queries
+  const uint16_t* Y; int ldy; long long bsy;               // [T, d] gradients of the output
+  const uint16_t* W0; const uint16_t* W1; const uint16_t* W2; long long bsw;
+  uint16_t* O0; uint16_t* O1; uint16_t* O2; long long bso; // [T, dh]: hidden, gradients of q W0^T and of q W2^T
+  uint16_t* dq; long long bsd;
+  StepBatch steps; long long gsx, gsy, gsw, gsd;           // several steps of the program in one launch
+  TileMap map;                                             // 256 tokens, 1, batch
+};
+template <int D>
+struct ApplyBwdStage {
+  using U = UpdatePatch<D>;
+  static constexpr int SIDE = U::BYTES, BYTES = 2 * SIDE + D * 64, LDS = cmax(2 * BYTES, 8 * 32 * (D + 8) * 2);
+};
+
+template <int D>
+__global__ __launch_bounds__(512, 2) void k_apply_bwd_fused(const ApplyBwdFusedParams p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  using ST = ApplyBwdStage<D>;
+  using U = UpdatePatch<D>;
+  int bx, by, z;
+  if (!p.map.locate(blockIdx.x, bx, by, z)) return;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63, h = lane >> 5;
+  const int row0 = (bx * 8 + wave) * 32, row = row0 + (lane & 31), dh = p.dh, n = dh / 32;
+  const long long w = p.steps.at(z, p.bsw, p.gsw);
+  const uint32_t lds0 = lds_addr(smem), tall_off = TallFrag::copy_offset(dh);
+  uint32_t side_off;
+  {
+    UpdateCopies<D> cp;
+    cp.init(D);
+    side_off = cp.voff[0];
+#pragma unroll
+    for (int i = 1; i < 4; ++i) side_off = wave % 4 == i ? cp.voff[i] : side_off;
+  }
+  auto issue = [&](int t) {
+    const uint32_t to = lds0 + (t & 1) * ST::BYTES + wave * 1024;
+    const long long rows = w + ((long long)t * 32 + wave / 4 * 16) * D;
+    if (wave < U::COPIES) {
+      dma16<false>(p.W0 + rows, side_off, to);
+      dma16<false>(p.W2 + rows, side_off, to + ST::SIDE);
+    }
+    if (wave < D / 16) dma16<false>(p.W1 + w + (size_t)wave * 16 * dh + t * 32, tall_off, to + 2 * ST::SIDE);
+  };
+  issue(0);
+  constexpr int KS = D / 16, DT = D / 32;
+  bf16x8 qf[KS], gf[KS];
+  attn_own_rows<D>(qf, p.X + p.steps.at(z, p.bsx, p.gsx), p.ldx, row, p.T);
+  attn_own_rows<D>(gf, p.Y + p.steps.at(z, p.bsy, p.gsy), p.ldy, row, p.T);
+  AttnFrag<U::P> frag;
+  frag.init();
+  TallFrag tall;
+  tall.init();
+  // (lanes past the last token hold its values and write them once more)
+  const long long mine = z * p.bso + (long long)min(row, p.T - 1) * dh + 8 * h;
+  uint16_t* const out[3] = {p.O0 + mine, p.O1 + mine, p.O2 + mine};
+  f32x16 dq[DT];
+#pragma unroll
+  for (int i = 0; i < DT; ++i)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) dq[i][j] = 0.f;
+  wait_vmcnt<0>();
+  for (int t = 0; t < n; ++t) {
+    wait_vmcnt<6>();      // behind this stage's copies come the six stores of the stage before only
+    __builtin_amdgcn_s_barrier();
+    issue(min(t + 1, n - 1));
+    const char* stage = smem + (t & 1) * ST::BYTES;
+    f32x16 g, u, e;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) g[j] = u[j] = e[j] = 0.f;
+    bf16x8 f[2][2];
+    auto read = [&](int ks) {
+      if (ks < KS) {
+        f[ks & 1][0] = frag.rows(stage, 0, ks);
+        f[ks & 1][1] = frag.rows(stage + ST::SIDE, 0, ks);
+      } else if (ks < 2 * KS) {
+        f[ks & 1][0] = tall.columns(stage + 2 * ST::SIDE, ks - KS);
+      }
+    };
+    read(0);
+#pragma unroll
+    for (int ks = 0; ks < 2 * KS; ++ks) {
+      read(ks + 1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (ks < KS) {
+        g = mma32(f[ks & 1][0], qf[ks % KS], g);
+        u = mma32(f[ks & 1][1], qf[ks % KS], u);
+      } else {
+        e = mma32(f[ks & 1][0], gf[ks % KS], e);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int st = 0; st < 2; ++st) {
+      uint32_t r[3][4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        float o[3][2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+          const float y0 = round_bf16(g[8 * st + 2 * i + j]), y2 = round_bf16(u[8 * st + 2 * i + j]), gh = round_bf16(e[8 * st + 2 * i + j]);
+          const SiluParts s = silu_parts(y0);
+          const float sg = round_bf16(s.silu), dy = round_bf16(gh * y2);
+          o[0][j] = sg * y2; o[1][j] = dy * s.d1; o[2][j] = gh * sg;
+        }
+#pragma unroll
+        for (int m = 0; m < 3; ++m) r[m][i] = pack_bf16(o[m][0], o[m][1]);
+      }
+#pragma unroll
+      for (int m = 0; m < 3; ++m) store_units(out[m] + t * 32 + 16 * st, r[m]);
+      const bf16x8 dg = __builtin_bit_cast(bf16x8, make_uint4(r[1][0], r[1][1], r[1][2], r[1][3])), du = __builtin_bit_cast(bf16x8, make_uint4(r[2][0], r[2][1], r[2][2], r[2][3]));
+#pragma unroll
+      for (int dt = 0; dt < DT; ++dt) {
+        dq[dt] = mma32(frag.cols(stage, dt, st), dg, dq[dt]);
+        dq[dt] = mma32(frag.cols(stage + ST::SIDE, dt, st), du, dq[dt]);
+      }
+    }
+  }
+  wait_vmcnt<0>();
+  __syncthreads();
+  if (row0 < p.T) attn_store_rows<D>(smem + wave * 32 * (D + 8) * 2, dq, 1.f, p.dq + p.steps.at(z, p.bsd, p.gsd), D, row0, p.T);
 }
 
 }  // namespace lact

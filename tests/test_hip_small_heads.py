@@ -110,9 +110,9 @@ def test_infinite_tokens_stay_in_their_head(token):
             assert torch.equal(fine, torch.isfinite(r.float()).flatten(1).all(dim=1)) and fine.tolist() == [True, False, True]
 
 
-# tokens at the edges of a wave's 32 and a block's 128; one and several stages of 32 hidden units (the ring has three places); all with
-# batch enough that the one kernel is taken
-@pytest.mark.parametrize("b,T,d,dh", [(200, 33, 64, 32), (128, 129, 64, 64), (5, 4700, 64, 96), (90, 200, 96, 96), (100, 127, 128, 64), (120, 129, 128, 96),
+# tokens at the edges of a wave's 32 and a block's 128 or 256; one and several stages of 32 hidden units (the rings have two and three
+# places); all with batch enough that the kernels are taken
+@pytest.mark.parametrize("b,T,d,dh", [(255, 127, 64, 32), (128, 129, 64, 64), (5, 4700, 64, 96), (90, 200, 96, 96), (100, 127, 128, 64), (120, 129, 128, 96),
                                       (250, 100, 128, 160), (250, 63, 128, 256)])
 def test_tokens_gradients_in_one_kernel(b, T, d, dh):
     """Gradients of a program of two updates: the same products of the same rounded values in another order, on top of weights that the
@@ -152,3 +152,20 @@ def test_tokens_gradients_in_one_kernel(b, T, d, dh):
         assert O.rel_l2(a, r) < 3e-3, (n, O.rel_l2(a, r))
         if n in ("k", "v", "lr0", "lr1", "lr2"):
             assert float(a[:, :at].float().abs().max()) == 0 and float(a[:, at + 2 * T:].float().abs().max()) == 0
+
+
+# three applies between updates: two of them share launches; small steps, which only the apply's kernel takes
+@pytest.mark.parametrize("b,T,d,dh", [(1, 1, 64, 32), (2, 33, 96, 64), (3, 127, 128, 96), (1, 257, 128, 160), (2, 300, 64, 96)])
+def test_queries_gradients_in_one_kernel(b, T, d, dh):
+    print("[gpu-test] queries' gradients in one kernel", b, T, d, dh, flush=True)
+    L = 3 * T
+    inp = {n: x.to(DEV) for n, x in O.make_inputs(b, L, d, dh, seed=66, act_dtype=torch.bfloat16).items()}
+    prog = ops.Program(steps=tuple(s for i in range(3) for s in ((LACT_APPLY, i * T, (i + 1) * T, i * T), (LACT_UPDATE, i * T, (i + 1) * T, 0))), out_len=L)
+    go = torch.randn(b, L, d + 8, generator=torch.Generator().manual_seed(3)).bfloat16().to(DEV)[..., :d]      # (rows with a stride)
+
+    def run():
+        t = [inp[n].clone().requires_grad_(True) for n in ORDER]
+        return torch.autograd.grad(ops.run_program(prog, *t)[0], t, go)
+
+    for n, a, r in zip(ORDER, run(), in_pieces(run)):
+        assert torch.isfinite(a.float()).all() and O.rel_l2(a, r) < 3e-3, (n, O.rel_l2(a, r))

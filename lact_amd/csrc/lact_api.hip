@@ -19,6 +19,7 @@
 #include "ns_fused.h"
 #include "ns_local.h"
 #include "gemm_persist.h"
+#include "gemm_wide.h"
 #include "gemm_kernels.h"
 #include "state_kernels.h"
 #include "layer_kernels.h"
@@ -517,6 +518,13 @@ struct Runner {
     return ceil_div(d.dh, TS_BWD::BN) * TS_BWD::WAVES_N;
   }
   bool hidden_small(int which) const { return which == 0 ? d.d <= 256 : which <= 3 && d.d <= 192; }   // the kernel from kept pre-activations has the large tile only
+  // 256 x 128 tiles where their rounds of blocks, one to a compute unit and 1.6 times as long as those of 128 x 128 tiles, take less
+  // time (gemm_wide.h).
+  bool hidden_wide(int T_, int nz) const {
+    if (d.d % 64 || d.d < 384 || d.dh % 8) return false;
+    const int cols = ceil_div(d.dh, TS_WIDE::BN) * nz;
+    return ceil_div(ceil_div(T_, TS_WIDE::BM) * cols, 256) * 1.62 < ceil_div(ceil_div(T_, 128) * cols, 256);
+  }
   // LACT_OPT_PERSISTENT_TILES: its default, the apply alone, gives way to the small tiles; any other mask is taken as it is
   bool hidden_persists(int which) const {
     return d.d % 64 == 0 && ((g_persist >> which) & 1) && side && side->cus > 0 && !(g_persist == 1 && hidden_small(which));
@@ -561,6 +569,15 @@ struct Runner {
         return;
       }
       const bool small = hidden_small(which);
+      if ((which == 1 || which == 2) && hidden_wide(T_, nz)) {
+        q.map = make_tile_map(ceil_div(T_, TS_WIDE::BM), ceil_div(d.dh, TS_WIDE::BN), nz);
+        LACT_BIG_LDS(k_update_hidden_wide, WIDE_LDS);
+        LACT_BIG_LDS(k_apply_bwd_hidden_wide, WIDE_LDS);
+        const dim3 gw(q.map.grid());
+        if (which == 1) LACT_LAUNCH_SMEM("k_update_hidden_wide", "update_hidden", 6.0 * f, k_update_hidden_wide, gw, dim3(DMA_THREADS), WIDE_LDS, s, q);
+        else LACT_LAUNCH_SMEM("k_apply_bwd_hidden_wide", "apply_bwd_hidden", 6.0 * f, k_apply_bwd_hidden_wide, gw, dim3(DMA_THREADS), WIDE_LDS, s, q);
+        return;
+      }
       // tile of the kernel that is launched below: the grid has to cover exactly its tiles
       const int bm = which == 3 && small ? TS_64::BM : 128, bn = which == 3 || small ? 64 : 128;
       static_assert(TS_SQ::BM == 128 && TS_SQ::BN == 128 && TS_BWD::BM == 128 && TS_BWD::BN == 64 && TS_64::BN == 64, "tiles of the hidden-stage kernels");

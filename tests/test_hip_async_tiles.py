@@ -193,6 +193,31 @@ def test_normalisation_of_extreme_gradients(scale, zeros):
         assert torch.isfinite(a.float()).all() and torch.equal(a, r)
 
 
+# tokens that end inside a tile of 256 and inside its first half, hidden units inside one of 128; K-steps 6, 7, 12; steps that share a launch
+@pytest.mark.parametrize("b,d,dh,T", [(6, 384, 640, 1100), (9, 448, 392, 1000), (4, 768, 832, 1300), (3, 512, 1536, 1152)])
+def test_wide_hidden_tiles_have_the_same_bits(b, d, dh, T):
+    """The 256 x 128 tiles of an update's and an apply backward's hidden stage (which these shapes take: two rounds of 128 x 128 tiles against
+    one) against persistent 128 x 128 tiles: every product over k in the same order."""
+    print("[gpu-test] wide tiles", b, d, dh, T, flush=True)
+    from lact_amd import _lib, ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    L = 2 * T
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(b, L, d, dh, seed=71, act_dtype=torch.bfloat16).items()}
+    go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(5)).bfloat16().to("cuda")
+    prog = ops.Program(steps=((LACT_APPLY, 0, T, 0), (LACT_UPDATE, 0, T, 0), (LACT_APPLY, T, L, T), (LACT_UPDATE, T, L, 0)), out_len=L)
+    res = []
+    for mask in (1, 7):
+        prev = _lib.lib().lact_set_option(_lib.OPT_PERSISTENT_TILES, mask)
+        try:
+            leaves = [inp[n].clone().requires_grad_(True) for n in ORDER[:9]]
+            out, ws, _ = ops.run_program(prog, *leaves)
+            res.append([out.detach(), *[w.detach() for w in ws], *torch.autograd.grad(out, leaves, go)])
+        finally:
+            _lib.lib().lact_set_option(_lib.OPT_PERSISTENT_TILES, prev)
+    for a, r in zip(*res):
+        assert torch.isfinite(a.float()).all() and torch.equal(a, r)
+
+
 def same_specials(a, r):
     a, r = a.detach().float().cpu(), r.detach().float()
     assert torch.isinf(r).any()

@@ -38,7 +38,7 @@ CONFIGS = {
     "layer": (4, 4, 4096, 384, 384, 2048, 1005,
               "layer: CausalLaCTSwiGLUWithSlidingWindowAttn fwd+bwd under bf16 autocast, 760M shape (dim 1536 = 4 heads of "
               "384, 12 attention heads of 128, window 2048), B=4, L=4096, chunk 2048, Muon + momentum; projections are "
-              "rocBLAS GEMMs through torch.nn.Linear, attention and the rest are this library"),
+              "library GEMMs, their weight gradients, attention and the rest are this library"),
 }
 
 

@@ -5,7 +5,8 @@ arguments and parameter names (a state_dict moves over unchanged):
   CausalLaCTSwiGLUWithSlidingWindowAttn  minimal_implementations/causal_lact_with_sliding_window_attn.py:222-391
   FastWeightGluMLPMultihead              lact_nvs/lact_ttt.py:150-258
 
-The projections are torch.nn.Linear (hipBLASLt).  Everything between them runs in liblact_hip.so: one kernel turns
+The projections are torch.nn.Linear: their large products run in hipBLASLt, the weight gradients of plain ones and the
+small maps of the layer's input (learning rates, momentum, gates) in liblact_hip.so, as does everything between: one kernel turns
 the to_qkv output into the operation's q, k, v (silu, per-head L2 norm, head layout), one makes the learning rates
 and the momentum, the operation itself, and one kernel turns its output into the o_proj input (per-head RMSNorm,
 per-head gate, head layout) -- each with a hand-written backward.  The sliding-window attention of the causal

@@ -101,35 +101,43 @@ __global__ void k_init_state(const InitParams p) {
   ss = wave_sum(ss);
   if (lane == 0) p.n0[(size_t)z * p.g.maxrows() + row] = sqrtf(ss);
 }
-// The same from weights that lie transposed in memory (the view-synthesis model's layout, lact_ttt.py:89-94): 64 columns of 32
+// The same from weights that lie transposed in memory (the view-synthesis model's layout, lact_ttt.py:89-94): 256 columns of 32
 // rows at a time through LDS, so that no transposed copy has to be made first (three copies of 5 us in front of a 4 us kernel
-// at 18 matrices of 128 x 256).  Grid (ceil(max rows / 32), 3b), 256 threads.
+// at 18 matrices of 128 x 256).  Bound by the latency of its loads: with 64 columns at a time, one after the other, 6.1 us there; all
+// eight loads of a thread at once 5.4.  Grid (ceil(max rows / 32), 3b), 256 threads.
 template <typename T>
 __global__ __launch_bounds__(256) void k_init_state_transposed(const InitParams p) {
-  __shared__ float tile[64][33];
+  __shared__ float tile[256][33];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb, row0 = blockIdx.x * 32;
   const int rows = p.g.rows(j), cols = p.g.cols(j);
   if (row0 >= rows) return;
   const float* src = p.w[j] + (size_t)ib * p.g.elems;
-  const int lc = threadIdx.x >> 3, lr = (threadIdx.x & 7) * 4;          // load: column lc (+ 32), four rows from lr
+  const int lc = threadIdx.x >> 3, lr = (threadIdx.x & 7) * 4;          // load: column lc (+ 32 i), four rows from lr
   const int sr = threadIdx.x >> 4, scol = (threadIdx.x & 15) * 4;       // store: row sr (+ 16), four columns from scol
   float ss[2] = {0.f, 0.f};
-  for (int c0 = 0; c0 < cols; c0 += 64) {
+  for (int b0 = 0; b0 < cols; b0 += 256) {
+    float4 in[8];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int c = lc + 32 * i;
-      const float4 v = (c0 + c < cols && row0 + lr < rows) ? ld4(src + (size_t)(c0 + c) * rows + row0 + lr) : f4(0.f, 0.f, 0.f, 0.f);
-      tile[c][lr] = v.x; tile[c][lr + 1] = v.y; tile[c][lr + 2] = v.z; tile[c][lr + 3] = v.w;
+    for (int i = 0; i < 8; ++i) {
+      const int c = b0 + lc + 32 * i;
+      in[i] = (c < cols && row0 + lr < rows) ? ld4(src + (size_t)c * rows + row0 + lr) : f4(0.f, 0.f, 0.f, 0.f);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      float* t = tile[lc + 32 * i] + lr;
+      t[0] = in[i].x; t[1] = in[i].y; t[2] = in[i].z; t[3] = in[i].w;
     }
     __syncthreads();
+    for (int c0 = b0; c0 < min(b0 + 256, cols); c0 += 64) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      const int r = sr + 16 * i;
-      if (row0 + r < rows && c0 + scol < cols) {
-        const float4 v = f4(tile[scol][r], tile[scol + 1][r], tile[scol + 2][r], tile[scol + 3][r]);
-        ss[i] += dot4(v, v);
-        const size_t e = (size_t)(row0 + r) * cols + c0 + scol;
-        init_store<T>(p, p.w_ext[j], (size_t)z * p.g.elems + e, (size_t)ib * p.g.elems + e, v);
+      for (int i = 0; i < 2; ++i) {
+        const int r = sr + 16 * i, c = c0 - b0 + scol;
+        if (row0 + r < rows && c0 + scol < cols) {
+          const float4 v = f4(tile[c][r], tile[c + 1][r], tile[c + 2][r], tile[c + 3][r]);
+          ss[i] += dot4(v, v);
+          const size_t e = (size_t)(row0 + r) * cols + c0 + scol;
+          init_store<T>(p, p.w_ext[j], (size_t)z * p.g.elems + e, (size_t)ib * p.g.elems + e, v);
+        }
       }
     }
     __syncthreads();

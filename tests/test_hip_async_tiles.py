@@ -137,6 +137,24 @@ def test_transposed_weights_are_read_as_they_lie(dtype, d, dh):
                 assert torch.equal(a, w) and torch.equal(r, w)
 
 
+# rows of one, one and a little, and two and a half passes of 256 columns
+@pytest.mark.parametrize("d,dh", [(256, 40), (264, 33 * 8), (640, 72)])
+def test_transposed_weights_of_many_columns(d, dh):
+    """The weights a call without updates hands back and what it applies, from transposed views and contiguous ones: the same bits."""
+    print("[gpu-test] transposed weights, many columns", d, dh, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(2, 40, d, dh, seed=36, act_dtype=torch.bfloat16).items()}
+    plain = [inp[n] for n in ORDER[:9]]
+    views = [w.transpose(1, 2).contiguous().transpose(1, 2) for w in plain[:3]] + plain[3:]
+    prog = ops.Program(steps=((LACT_APPLY, 0, 40, 0),), out_len=40)
+    with torch.no_grad():
+        (out_p, w_p, _), (out_v, w_v, _) = ops.run_program(prog, *plain), ops.run_program(prog, *views)
+    assert torch.equal(out_p, out_v)
+    for a, r, w in zip(w_v, w_p, plain[:3]):
+        assert torch.equal(a, w) and torch.equal(r, w)
+
+
 @pytest.mark.parametrize("b,d,dh,L,stacked", [
     (3, 128, 256, 200, False), (2, 64, 64, 100, False), (1, 96, 96, 100, False), (2, 32, 224, 80, False), (2, 256, 64, 130, False),
     (2, 96, 160, 90, False), (5, 128, 128, 90, False), (2, 128, 64, 90, True)])

@@ -638,6 +638,13 @@ struct BwdStage {
   static_assert(LDS <= 160 * 1024, "the ring does not fit the LDS");
 };
 
+// The barrier alone: __syncthreads would wait for the wave's stores to memory as well.  What the wave has asked LDS for has been used by
+// then (its matrix instructions), and its copies into LDS are waited for by name; no access of the program moves across.
+__device__ __forceinline__ void block_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 // A stage of W1 or G1 in LDS: [d][32 hidden], rows of 64 bytes, granule g of row r at slot g ^ (r >> 2) & 3.
 struct TallFrag {
   uint32_t tr_off[2], row_off[2];
@@ -851,7 +858,7 @@ __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFuse
   int prev = 0, cur = 0, next = ST::BYTES;      // the ring's stages (the first one stands for the one before it)
   for (int t = 0; t < n; ++t) {
     wait_vmcnt<6>();      // behind this stage's copies come the six stores of the stage before only
-    __builtin_amdgcn_s_barrier();      // (__syncthreads would wait for the stores as well; what LDS was asked for has been used)
+    block_barrier();
     issue(min(t + 1, n - 1), next);
     const char* stage = smem + cur;
     {
@@ -977,7 +984,7 @@ __global__ __launch_bounds__(512, 2) void k_apply_bwd_fused(const ApplyBwdFusedP
   wait_vmcnt<0>();
   for (int t = 0; t < n; ++t) {
     wait_vmcnt<6>();      // behind this stage's copies come the six stores of the stage before only
-    __builtin_amdgcn_s_barrier();
+    block_barrier();
     issue(min(t + 1, n - 1));
     const char* stage = smem + (t & 1) * ST::BYTES;
     f32x16 g, u, e;

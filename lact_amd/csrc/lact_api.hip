@@ -622,9 +622,19 @@ struct Runner {
     p.map = make_tile_map(ceil_div(p.T, SPLIT ? 128 : 256), 1, nz);
     LACT_LAUNCH_SMEM("k_apply_fused", "apply", 6.0 * p.T * D * p.dh * nz, (k_apply_fused<D, SPLIT>), dim3(p.map.grid()), dim3(512), SM, s, p);
   }
+  // Where two waves share 32 tokens (SPLIT, below), the chip is not full and the kernel takes as long as one wave needs for all hidden
+  // units, which the kernels in pieces spread over blocks: it loses where there are many of them and few tokens.  us on the GPU (a graph
+  // of calls, the initial state's kernel included), in pieces / as one: d = 128, 64 tokens, dh = 128 10.3 / 10.9, 256 10.7 / 14.2, 1024
+  // 14.7 / 35.9, 2048 20 / 65; 6 x 1024 tokens, dh = 256 14.6 / 17.0, 512 18.7 / 25.3, 2048 41 / 72; 12 x 1024, dh = 256 18.2 / 19.2; d = 64,
+  // 6 x 1024, dh = 512 16.4 / 18.3.  Against that stands one launch less, 3.5 us of host time, which is what a short call is bound by (nvs
+  // rendering of 6 x 1024 tokens, dh = 256: 19.5 / 17.7): the one kernel may be 3 us behind.  Whole blocks never are (dh = 64 to 2048).
+  bool apply_fused_pays(int T_, int nz) const {
+    const double longer = d.dh / 32 * (0.23 + d.d / 256.0) - 1.05e-6 * T_ * nz * d.dh - 2.2;     // (fitted: 1.3 us off on average)
+    return ceil_div(T_, 128) * nz > 256 || longer <= 3;
+  }
   bool apply_fused(const HiddenParams& hp, const RowGemmParams<1>& out, int T_, int steps) const {
     if constexpr (kBf16) {
-      if (g_persist != 1 || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
+      if (g_persist != 1 || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32 || !apply_fused_pays(T_, d.b * steps)) return false;
       ApplyFusedParams p;
       memset(&p, 0, sizeof(p));
       p.T = T_; p.dh = d.dh;
@@ -695,7 +705,9 @@ struct Runner {
   }
   // us of a training step of four updates and applies with Newton-Schulz, in pieces / as one kernel: 12 x 4096 tokens, 96 x 96 705 / 668,
   // 48 x 1024, 128 x 256 1643 / 1600, 2 x 1024 463 / 477.  A round takes 8 us and 2.4 per 32 hidden units, the hidden stage and dq as kernels of
-  // their own 18 us and then by the hidden values (43 + 17 us at 12 x 4680 tokens, d = 128, dh = 256; 35 as one).
+  // their own 18 us and then by the hidden values (43 + 17 us at 12 x 4680 tokens, d = 128, dh = 256; 35 as one).  With this rule and
+  // update_bwd_fused's, steps of four updates and applies of 1 to 48 heads, 64 to 128 features, 64 to 1024 hidden units and 128 to 2048 tokens
+  // (219 of them) take at most 1.02 of their time in pieces on the GPU.
   bool apply_bwd_fused(int tokens, int nz) const {
     if (!kBf16 || g_persist != 1 || (d.d != 64 && d.d != 96 && d.d != 128) || d.dh % 32) return false;
     const double pieces = 18 + 45.0 * tokens * nz / (12 * 4680) * d.dh / 256 * (0.5 + d.d / 256.0);

@@ -1,4 +1,7 @@
 """The kernels that run a whole step of small bf16 heads (csrc/small_heads.h) against the ones that run it in pieces."""
+import ctypes
+import json
+
 import pytest
 import torch
 
@@ -19,10 +22,39 @@ def in_pieces(fn):
         _lib.lib().lact_set_option(_lib.OPT_PERSISTENT_TILES, prev)
 
 
+def kernels(fn):
+    """What fn returns, and the names of the kernels that it launched."""
+    lib, buf = _lib.lib(), ctypes.create_string_buffer(1 << 16)
+    _lib.check(lib.lact_profile_enable(1))
+    try:
+        res = fn()
+        _lib.check(lib.lact_profile_report(buf, len(buf)))
+    finally:
+        _lib.check(lib.lact_profile_enable(0))
+    return res, {r["kernel"] for r in json.loads(buf.value)}
+
+
+# both sides of the line: hidden units at few tokens, tokens at many hidden units, whole blocks
+@pytest.mark.parametrize("b,T,d,dh,one", [
+    (1, 64, 128, 128, True), (1, 64, 128, 256, False), (6, 1024, 128, 256, True), (2, 1024, 128, 256, False), (1, 64, 64, 320, True),
+    (1, 64, 64, 512, False), (1, 64, 96, 256, True), (2, 129, 96, 512, False), (6, 1024, 128, 512, False), (20, 1024, 128, 512, True),
+    (1, 1, 64, 2048, False), (33, 1024, 96, 1024, True), (260, 64, 128, 1024, True)])
+def test_apply_takes_the_faster_kernels(b, T, d, dh, one):
+    """A wave of the one kernel walks all hidden units, however few tokens there are: few tokens with many of them go in pieces."""
+    print("[gpu-test] apply's rule", b, T, d, dh, one, flush=True)
+    t = {n: x.to(DEV) for n, x in O.make_inputs(b, T, d, dh, seed=60, act_dtype=torch.bfloat16).items()}
+    prog = ops.Program(steps=((LACT_APPLY, 0, T, 0),), out_len=T)
+    with torch.no_grad():
+        out, names = kernels(lambda: ops.run_program(prog, *[t[n] for n in ORDER])[0])
+        ref, pieces = kernels(lambda: in_pieces(lambda: ops.run_program(prog, *[t[n] for n in ORDER])[0]))
+    assert ("k_apply_fused" in names) == one and "k_apply_fused" not in pieces
+    assert O.rel_l2(out, ref) < 1e-3
+
+
 # tokens at the edges of a wave's 32, of a split block's 128 and of a block's 256; the hidden size in halves of a stage; more than
 # 256 split blocks, which is where whole blocks begin; several steps in one launch
 @pytest.mark.parametrize("b,T,d,dh,steps", [
-    (1, 1, 64, 32, 1), (2, 33, 64, 96, 1), (3, 127, 96, 64, 1), (2, 129, 96, 160, 1), (5, 300, 128, 32, 1), (2, 257, 128, 288, 1), (3, 128, 128, 128, 3),
+    (1, 1, 64, 32, 1), (2, 33, 64, 96, 1), (3, 127, 96, 64, 1), (2, 129, 96, 160, 1), (5, 300, 128, 32, 1), (30, 257, 128, 288, 1), (3, 128, 128, 128, 3),
     (90, 300, 64, 160, 1), (129, 200, 96, 96, 1), (65, 513, 128, 96, 1), (40, 300, 128, 64, 3)])
 def test_apply_in_one_kernel(b, T, d, dh, steps):
     """The same rounded hidden values, summed in another order: a result differs by a rounding where its sum lies next to one (2^-9 of
@@ -42,8 +74,8 @@ def test_apply_in_one_kernel(b, T, d, dh, steps):
     prog = ops.Program(steps=tuple(prog), out_len=L)
     run = lambda q: ops.run_program(prog, *args[:3], q, *args[4:])[0]
     with torch.no_grad():
-        out, view, ref = run(t["q"]), run(wide[..., 8:d + 8]), in_pieces(lambda: run(t["q"]))
-    assert torch.equal(out, view) and torch.isfinite(out.float()).all()
+        (out, names), view, ref = kernels(lambda: run(t["q"])), run(wide[..., 8:d + 8]), in_pieces(lambda: run(t["q"]))
+    assert "k_apply_fused" in names and torch.equal(out, view) and torch.isfinite(out.float()).all()
     assert O.rel_l2(out, ref) < (1e-3 if steps == 1 else 1e-2)
     assert torch.equal(out[:, :T], run(t["q"])[:, :T])
 

@@ -517,11 +517,14 @@ std::vector<int64_t> with_last(at::IntArrayRef sizes, int64_t last) {
   return s;
 }
 
-// x w^T under bf16 autocast for fp32 w, whose gradient is summed, and returned, in fp32
+// A weight as autocast casts it: once in an autocast region, however often the layer is called there.
+Tensor autocast_weight(const Tensor& w) { return at::autocast::cached_cast(at::kBFloat16, w); }
+
+// x w^T under bf16 autocast for fp32 w, whose gradient is summed, and returned, in fp32; wb: autocast_weight(w)
 struct LinearFn : torch::autograd::Function<LinearFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight) {
+  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const Tensor& wb) {
     const c10::hip::HIPGuard guard(x.device().index());
-    const Tensor wb = weight.to(at::kBFloat16), xb = rows_of(x, at::kBFloat16);
+    const Tensor xb = rows_of(x, at::kBFloat16);
     ctx->save_for_backward({xb, wb});
     ctx->saved_data["x"] = (int64_t)x.scalar_type();
     ctx->saved_data["need"] = std::vector<int64_t>{x.requires_grad(), weight.requires_grad()};
@@ -539,19 +542,19 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
     Tensor dx, dw;
     if (need[0]) dx = cast(at::mm(g, wb).view(ctx->saved_data["shape"].toIntVector()), (at::ScalarType)as_int(ctx, "x"));
     if (need[1]) dw = weight_grad(g, xb);
-    return finish({dx, dw}, twice);
+    return finish({dx, dw, Tensor()}, twice);
   }
 };
 
 // The maps of a layer's input x [B, L, dim] fp32 under bf16 autocast: to_qkv in bf16, the rates x lr_w^T + lr_b in fp32, the bf16
 // maps of the momentum (as fp32 values) and of the gate.  to_qkv and the rates are library products; the other maps, and what
-// their and the rates' backward is, csrc/layer_kernels.h.
+// their and the rates' backward is, csrc/layer_kernels.h.  wb: autocast_weight(qkv_w)
 struct LayerInFn : torch::autograd::Function<LayerInFn> {
-  static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& qkv_w, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w,
+  static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& qkv_w, const Tensor& wb, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w,
                                const OptTensor& mom_b, const OptTensor& gate_w, const OptTensor& gate_b) {
     const c10::hip::HIPGuard guard(x_.device().index());
     const int64_t B = x_.size(0), L = x_.size(1), dim = x_.size(2), n = B * L;
-    const Tensor x = rows_of(x_, at::kFloat), wb = qkv_w.to(at::kBFloat16);
+    const Tensor x = rows_of(x_, at::kFloat);
     const Tensor lw = plain_f32(lr_w), mw = mom_w ? plain_f32(*mom_w) : Tensor(), gw = gate_w ? plain_f32(*gate_w) : Tensor();
     const Tensor mb = mom_b ? plain_f32(*mom_b) : Tensor(), gb = gate_b ? plain_f32(*gate_b) : Tensor();
     const int64_t nm = mw.defined() ? mw.size(0) : 0, ng = gw.defined() ? gw.size(0) : 0;
@@ -607,7 +610,7 @@ struct LayerInFn : torch::autograd::Function<LayerInFn> {
                                  ptr(dxq), fptr(dx), fptr(d[0]), fptr(d[1]), fptr(d[2]), fptr(d[3]), fptr(d[4]), fptr(d[5]), ptr(ws), stream()));
     Tensor dw;
     if (need[1]) dw = g.defined() ? weight_grad(g, xb) : at::zeros(wb.sizes(), x.options());
-    return finish({dx, dw, d[0], d[1], d[2], d[3], d[4], d[5]}, twice);
+    return finish({dx, dw, Tensor(), d[0], d[1], d[2], d[3], d[4], d[5]}, twice);
   }
 };
 
@@ -633,7 +636,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("layer_post", [](const Tensor& o, const OptTensor& weight, const OptTensor& gate, int64_t B, int64_t H, bool use_norm, double eps, const OptTensor& add) {
     return apply_released<LayerPostFn>(o, weight, gate, B, H, use_norm, eps, add);
   });
-  m.def("linear", [](const Tensor& x, const Tensor& weight) { return apply_released<LinearFn>(x, weight); });
+  m.def("linear", [](const Tensor& x, const Tensor& weight) { return apply_released<LinearFn>(x, weight, autocast_weight(weight)); });
   m.def("layer_in", [](const Tensor& x, const Tensor& qkv_w, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w, const OptTensor& mom_b,
-                       const OptTensor& gate_w, const OptTensor& gate_b) { return apply_released<LayerInFn>(x, qkv_w, lr_w, lr_b, mom_w, mom_b, gate_w, gate_b); });
+                       const OptTensor& gate_w, const OptTensor& gate_b) { return apply_released<LayerInFn>(x, qkv_w, autocast_weight(qkv_w), lr_w, lr_b, mom_w, mom_b, gate_w, gate_b); });
 }

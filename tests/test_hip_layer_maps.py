@@ -90,6 +90,37 @@ def test_partial_gradients_and_unused_outputs():
     assert all(torch.equal(a, b) for a, b in zip(outs, again)) and not again[0].requires_grad
 
 
+def test_weights_are_cast_once_in_an_autocast_region():
+    """As autocast does for the modules: a layer that is called several times in one region keeps one bf16 copy of each weight."""
+    print("[gpu-test] casts of the weights", flush=True)
+    layer = HL.BidirectionalLaCTSwiGLU(64, 32, use_muon=False).to(DEV)
+    x = torch.randn(1, 70, 64, device=DEV)
+    copies = {layer.to_qkv.weight: [], layer.o_proj.weight: []}
+
+    def pack(t):
+        for w, seen in copies.items():
+            if t.dtype == torch.bfloat16 and t.shape == w.shape and torch.equal(t, w.detach().bfloat16()):
+                seen.append(t)
+        return t
+
+    def step(regions):
+        before = {w: len(seen) for w, seen in copies.items()}
+        with torch.autograd.graph.saved_tensors_hooks(pack, lambda t: t):
+            for _ in range(regions):
+                with torch.autocast("cuda", dtype=torch.bfloat16):
+                    y = layer(x) + layer(x)
+        assert all(len(seen) == before[w] + 2 * regions for w, seen in copies.items())
+        return y
+
+    first = torch.autograd.grad(step(1).float().square().sum(), [layer.to_qkv.weight, layer.o_proj.weight])
+    assert all(seen[0].data_ptr() == seen[1].data_ptr() for seen in copies.values())
+    with torch.no_grad():
+        for w in copies:
+            w.mul_(-1)
+    again = torch.autograd.grad(step(1).float().square().sum(), [layer.to_qkv.weight, layer.o_proj.weight])   # the next region casts anew
+    assert all(not torch.equal(a, b) for a, b in zip(first, again))
+
+
 def test_second_derivatives_of_the_maps_are_refused():
     print("[gpu-test] second derivative of the maps", flush=True)
     mods = maps(64, 3, 1, 1, False)

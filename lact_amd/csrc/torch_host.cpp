@@ -499,11 +499,16 @@ struct LayerPostFn : torch::autograd::Function<LayerPostFn> {
   }
 };
 
+// a b of bf16 matrices in fp32, inside autocast regions too
+Tensor mm_f32(const Tensor& a, const Tensor& b) {
+  const c10::impl::ExcludeDispatchKeyGuard plain(c10::DispatchKey::AutocastCUDA);
+  return at::mm(a.to(at::kFloat), b.to(at::kFloat));
+}
 // dy^T x in fp32 for bf16 rows dy [t, m], x [t, n]
 Tensor weight_grad(const Tensor& dy, const Tensor& x) {
   const int64_t t = x.size(0), m = dy.size(1), n = x.size(1);
   if (t < 64 || t >= (1LL << 31) || m % 8 || n % 8 || std::max(m, n) >= (1 << 23))   // outside the kernel's range
-    return at::mm(dy.to(at::kFloat).t(), x.to(at::kFloat));
+    return mm_f32(dy.t(), x);
   const Tensor dw = at::empty({m, n}, x.options().dtype(at::kFloat));
   const int64_t bytes = (int64_t)lact_weight_grad_workspace_bytes((int)t, (int)m, (int)n);
   const Tensor ws = bytes ? at::empty({bytes}, x.options().dtype(at::kByte)) : Tensor();

@@ -68,6 +68,9 @@ def test_weight_gradient_against_float64(T, m, n):
     wb = lin.weight.detach().bfloat16().double()
     assert dw.dtype == torch.float32 and rel_l2(dw, go[0].double().t() @ x.detach()[0].double()) < 1e-5
     assert dx.dtype == torch.bfloat16 and rel_l2(dx, go.double() @ wb) < 4e-3 and rel_l2(y, x.detach().double() @ wb.t()) < 4e-3
+    with torch.autocast("cuda", dtype=torch.bfloat16):      # a backward inside the region: the same bits
+        inside = torch.autograd.grad(HL._linear(lin, x), [x, lin.weight], go)
+    assert torch.equal(inside[0], dx) and torch.equal(inside[1], dw)
 
 
 def test_partial_gradients_and_unused_outputs():

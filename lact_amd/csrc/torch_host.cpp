@@ -499,6 +499,9 @@ struct LayerPostFn : torch::autograd::Function<LayerPostFn> {
   }
 };
 
+// As autocast casts: a weight once in a region, however often the layer is called there.
+Tensor autocast_bf16(const Tensor& t) { return at::autocast::cached_cast(at::kBFloat16, t); }
+
 // a b of bf16 matrices in fp32, inside autocast regions too
 Tensor mm_f32(const Tensor& a, const Tensor& b) {
   const c10::impl::ExcludeDispatchKeyGuard plain(c10::DispatchKey::AutocastCUDA);
@@ -522,38 +525,37 @@ std::vector<int64_t> with_last(at::IntArrayRef sizes, int64_t last) {
   return s;
 }
 
-// A weight as autocast casts it: once in an autocast region, however often the layer is called there.
-Tensor autocast_weight(const Tensor& w) { return at::autocast::cached_cast(at::kBFloat16, w); }
-
-// x w^T under bf16 autocast for fp32 w, whose gradient is summed, and returned, in fp32; wb: autocast_weight(w)
+// x w^T under bf16 autocast for fp32 w, whose gradient is summed, and returned, in fp32; xb, wb: both as autocast casts them.  It can be
+// differentiated again, and over batches of gradients, as the module could: the gradient is then made of torch's operations.
 struct LinearFn : torch::autograd::Function<LinearFn> {
-  static Tensor forward(AutogradContext* ctx, const Tensor& x, const Tensor& weight, const Tensor& wb) {
-    const c10::hip::HIPGuard guard(x.device().index());
-    const Tensor xb = rows_of(x, at::kBFloat16);
+  static Tensor forward(AutogradContext* ctx, const Tensor& xb, const Tensor& weight, const Tensor& wb) {
+    const c10::hip::HIPGuard guard(xb.device().index());
     ctx->save_for_backward({xb, wb});
-    ctx->saved_data["x"] = (int64_t)x.scalar_type();
-    ctx->saved_data["need"] = std::vector<int64_t>{x.requires_grad(), weight.requires_grad()};
-    ctx->saved_data["shape"] = x.sizes().vec();
-    return at::linear(xb, wb).view(with_last(x.sizes(), wb.size(0)));
+    ctx->saved_data["need"] = std::vector<int64_t>{xb.requires_grad(), weight.requires_grad()};
+    return at::linear(dense(xb.reshape({-1, xb.size(-1)})), wb).view(with_last(xb.sizes(), wb.size(0)));
   }
   static variable_list backward(AutogradContext* ctx, variable_list grads) {
-    const bool twice = at::GradMode::is_enabled();
-    const at::AutoGradMode off(false);
     const auto t = ctx->get_saved_variables();
     const Tensor &xb = t[0], &wb = t[1];
     const c10::hip::HIPGuard guard(xb.device().index());
     const auto need = ctx->saved_data["need"].toIntVector();
-    const Tensor g = rows_of(grads[0], at::kBFloat16);
     Tensor dx, dw;
-    if (need[0]) dx = cast(at::mm(g, wb).view(ctx->saved_data["shape"].toIntVector()), (at::ScalarType)as_int(ctx, "x"));
-    if (need[1]) dw = weight_grad(g, xb);
-    return finish({dx, dw, Tensor()}, twice);
+    if (at::GradMode::is_enabled() || grads[0].key_set().has_any(c10::DispatchKeySet({c10::DispatchKey::Batched, c10::DispatchKey::FuncTorchBatched}))) {
+      const Tensor g = grads[0].reshape({-1, wb.size(0)});
+      if (need[0]) dx = at::mm(g, wb).view(xb.sizes());
+      if (need[1]) dw = mm_f32(g.t(), xb.reshape({-1, xb.size(-1)}));
+      return {dx, dw, Tensor()};
+    }
+    const Tensor g = rows_of(grads[0], at::kBFloat16);
+    if (need[0]) dx = at::mm(g, wb).view(xb.sizes());
+    if (need[1]) dw = weight_grad(g, rows_of(xb, at::kBFloat16));
+    return {dx, dw, Tensor()};
   }
 };
 
 // The maps of a layer's input x [B, L, dim] fp32 under bf16 autocast: to_qkv in bf16, the rates x lr_w^T + lr_b in fp32, the bf16
 // maps of the momentum (as fp32 values) and of the gate.  to_qkv and the rates are library products; the other maps, and what
-// their and the rates' backward is, csrc/layer_kernels.h.  wb: autocast_weight(qkv_w)
+// their and the rates' backward is, csrc/layer_kernels.h.  wb: autocast_bf16(qkv_w)
 struct LayerInFn : torch::autograd::Function<LayerInFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& qkv_w, const Tensor& wb, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w,
                                const OptTensor& mom_b, const OptTensor& gate_w, const OptTensor& gate_b) {
@@ -641,7 +643,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
   m.def("layer_post", [](const Tensor& o, const OptTensor& weight, const OptTensor& gate, int64_t B, int64_t H, bool use_norm, double eps, const OptTensor& add) {
     return apply_released<LayerPostFn>(o, weight, gate, B, H, use_norm, eps, add);
   });
-  m.def("linear", [](const Tensor& x, const Tensor& weight) { return apply_released<LinearFn>(x, weight, autocast_weight(weight)); });
+  m.def("linear", [](const Tensor& x, const Tensor& weight) { return apply_released<LinearFn>(autocast_bf16(x), weight, autocast_bf16(weight)); });
   m.def("layer_in", [](const Tensor& x, const Tensor& qkv_w, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w, const OptTensor& mom_b,
-                       const OptTensor& gate_w, const OptTensor& gate_b) { return apply_released<LayerInFn>(x, qkv_w, autocast_weight(qkv_w), lr_w, lr_b, mom_w, mom_b, gate_w, gate_b); });
+                       const OptTensor& gate_w, const OptTensor& gate_b) { return apply_released<LayerInFn>(x, qkv_w, autocast_bf16(qkv_w), lr_w, lr_b, mom_w, mom_b, gate_w, gate_b); });
 }

@@ -124,15 +124,78 @@ def test_weights_are_cast_once_in_an_autocast_region():
     assert all(not torch.equal(a, b) for a, b in zip(first, again))
 
 
-def test_second_derivatives_of_the_maps_are_refused():
+def test_second_derivatives_of_the_input_maps_are_refused():
+    """(What follows them has none either.)"""
     print("[gpu-test] second derivative of the maps", flush=True)
     mods = maps(64, 3, 1, 1, False)
     x = torch.randn(1, 70, 64, device=DEV, requires_grad=True)
     with torch.autocast("cuda", dtype=torch.bfloat16):
-        for outs in (HL._input_projections(x, *mods), [HL._linear(mods[0], x)]):
-            g = torch.autograd.grad(sum(o.float().sum() for o in outs), x, create_graph=True)[0]
-            with pytest.raises(RuntimeError, match="once_differentiable"):
-                torch.autograd.grad(g.square().sum() + x.sum(), x)
+        outs = HL._input_projections(x, *mods)
+        g = torch.autograd.grad(sum(o.float().sum() for o in outs), x, create_graph=True)[0]
+        with pytest.raises(RuntimeError, match="once_differentiable"):
+            torch.autograd.grad(g.square().sum() + x.sum(), x)
+
+
+@pytest.mark.parametrize("T,dtype", [(70, torch.bfloat16), (63, torch.bfloat16), (200, torch.float32)])
+def test_output_projection_differentiates_twice(T, dtype):
+    """Like the module it stands in for: gradients with a graph are the gradients without one (the weight's summed in fp32 in another
+    order: 1e-5), and their derivatives those of float64 within a few bf16 roundings of factors (2^-9 each: 1e-2)."""
+    print("[gpu-test] output projection twice", T, dtype, flush=True)
+    torch.manual_seed(7)
+    lin = nn.Linear(96, 64, bias=False).to(DEV)
+    x = torch.randn(2, T, 96, device=DEV).to(dtype).requires_grad_(True)
+    go, c = torch.randn(2, T, 64, device=DEV).bfloat16(), torch.randn(64, 96, device=DEV)
+    e = torch.randn(2, T, 96, device=DEV)
+
+    def derivatives(f, x, w, go, c, e):
+        y = f(x)
+        once = torch.autograd.grad(y, [x, w], go, retain_graph=True)
+        twice = torch.autograd.grad(y.pow(2), [x, w], go, create_graph=True)
+        return y, once, twice, torch.autograd.grad((twice[0] * e).sum() + (twice[1] * c).sum(), [x, w])
+
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        assert HL._fused_linears(x, lin)
+        y, once, twice, second = derivatives(lambda t: HL._linear(lin, t), x, lin.weight, go, c, e)
+        graph = torch.autograd.grad(HL._linear(lin, x), [x, lin.weight], go, create_graph=True)
+    xd, wd = x.detach().double().requires_grad_(True), lin.weight.detach().double().requires_grad_(True)
+    _, once_d, twice_d, second_d = derivatives(lambda t: F.linear(t, wd), xd, wd, go.double(), c.double(), e.double())
+    assert once[1].dtype == graph[1].dtype == torch.float32 and torch.equal(once[0], graph[0]) and rel_l2(once[1], graph[1]) < 1e-5
+    for a, r in zip([*once, *twice, *second], [*once_d, *twice_d, *second_d]):
+        assert rel_l2(a, r) < 1e-2
+
+
+def test_output_projection_takes_batches_of_gradients():
+    print("[gpu-test] batches of gradients", flush=True)
+    lin = nn.Linear(96, 64, bias=False).to(DEV)
+    x = torch.randn(2, 70, 96, device=DEV).bfloat16().requires_grad_(True)
+    go = torch.randn(3, 2, 70, 64, device=DEV).bfloat16()
+    with torch.autocast("cuda", dtype=torch.bfloat16):
+        y = HL._linear(lin, x)
+    batch = torch.autograd.grad(y, [x, lin.weight], go, retain_graph=True, is_grads_batched=True)
+    mapped = torch.func.vmap(lambda g: torch.autograd.grad(y, [x, lin.weight], g, retain_graph=True))(go)
+    for i in range(3):
+        single = torch.autograd.grad(y, [x, lin.weight], go[i], retain_graph=True)
+        for got in (batch, mapped):      # sums in another order in front of dx's rounding: one in a hundred lands beside it
+            assert rel_l2(got[0][i], single[0]) < 1e-3 and rel_l2(got[1][i], single[1]) < 1e-5
+
+
+def test_gradient_penalty_on_the_output_projection():
+    """|d loss / d o_proj.weight|^2 as part of a loss: a second derivative through o_proj and first ones through everything else."""
+    print("[gpu-test] gradient penalty", flush=True)
+    torch.manual_seed(9)
+    layer = HL.BidirectionalLaCTSwiGLU(64, 32, use_muon=False).to(DEV)
+    x = torch.randn(1, 90, 64, device=DEV)
+
+    def penalty():
+        with torch.autocast("cuda", dtype=torch.bfloat16):
+            y = layer(x)
+        g = torch.autograd.grad(y.float().square().mean(), layer.o_proj.weight, create_graph=True)[0]
+        return torch.autograd.grad(g.square().sum(), [layer.o_proj.weight, layer.o_norm.weight, layer.to_qkv.weight, layer.w1])
+
+    fused = penalty()
+    layer.o_proj.register_forward_hook(lambda m, a, o: None)
+    for a, r in zip(fused, penalty()):      # the module rounds the weight's gradient, and its gradient's, to bf16
+        assert rel_l2(a, r) < 2e-2
 
 
 def test_modules_are_called_where_someone_may_look():

@@ -345,8 +345,11 @@ Tensor dense(const Tensor& t) {
   return aligned16(c) ? c : c.clone();
 }
 Tensor dense(const Tensor& t, at::ScalarType dtype) { return dense(cast(t, dtype)); }
+// (in front of a device guard, whose own error names neither the tensor's device nor the reason)
+void on_gpu(const Tensor& t) {
+  if (!t.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path), got one on " + t.device().str());
+}
 int act_code(const Tensor& t) {
-  if (!t.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)");
   TORCH_CHECK_TYPE(t.scalar_type() == at::kBFloat16 || t.scalar_type() == at::kFloat, "unsupported activation dtype ", t.scalar_type(), ": bf16 or fp32");
   return t.scalar_type() == at::kBFloat16 ? LACT_BF16 : LACT_F32;
 }
@@ -367,6 +370,7 @@ variable_list finish(variable_list grads, bool twice) {
 // qkv [B, L, 3*H*hd] -> q, k, v [(B H), L, hd], and with the rescaling parameters [H*hd, 2] the attention's q, k, v [B, L, H*hd]
 struct LayerPreFn : torch::autograd::Function<LayerPreFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& qkv_, const OptTensor& scale_, const OptTensor& offset_, int64_t H, int64_t hd, bool l2norm) {
+    on_gpu(qkv_);
     const c10::hip::HIPGuard guard(qkv_.device().index());
     const Tensor qkv = dense(qkv_);
     const int act = act_code(qkv);
@@ -422,7 +426,7 @@ struct LayerPreFn : torch::autograd::Function<LayerPreFn> {
 // lr_raw [B, L, 3*H], momentum_raw [B, L, H] or none -> lr0, lr1, lr2 (, momentum) [(B H), L, 1] fp32
 struct LayerLrFn : torch::autograd::Function<LayerLrFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& lr_, const OptTensor& mom_, int64_t H, double base, bool rates_major) {
-    if (!lr_.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)");
+    on_gpu(lr_);
     const c10::hip::HIPGuard guard(lr_.device().index());
     const Tensor lr = plain_f32(lr_), mom = mom_ ? plain_f32(*mom_) : Tensor();
     const int64_t B = lr.size(0), L = lr.size(1);
@@ -459,6 +463,7 @@ struct LayerLrFn : torch::autograd::Function<LayerLrFn> {
 struct LayerPostFn : torch::autograd::Function<LayerPostFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& o_, const OptTensor& weight, const OptTensor& gate, int64_t B, int64_t H, bool use_norm, double eps,
                         const OptTensor& add) {
+    on_gpu(o_);
     const c10::hip::HIPGuard guard(o_.device().index());
     const Tensor o = dense(o_);
     const int act = act_code(o);
@@ -529,6 +534,7 @@ std::vector<int64_t> with_last(at::IntArrayRef sizes, int64_t last) {
 // differentiated again, and over batches of gradients, as the module could: the gradient is then made of torch's operations.
 struct LinearFn : torch::autograd::Function<LinearFn> {
   static Tensor forward(AutogradContext* ctx, const Tensor& xb, const Tensor& weight, const Tensor& wb) {
+    on_gpu(xb);
     const c10::hip::HIPGuard guard(xb.device().index());
     ctx->save_for_backward({xb, wb});
     ctx->saved_data["need"] = std::vector<int64_t>{xb.requires_grad(), weight.requires_grad()};
@@ -559,6 +565,7 @@ struct LinearFn : torch::autograd::Function<LinearFn> {
 struct LayerInFn : torch::autograd::Function<LayerInFn> {
   static variable_list forward(AutogradContext* ctx, const Tensor& x_, const Tensor& qkv_w, const Tensor& wb, const Tensor& lr_w, const OptTensor& lr_b, const OptTensor& mom_w,
                                const OptTensor& mom_b, const OptTensor& gate_w, const OptTensor& gate_b) {
+    on_gpu(x_);
     const c10::hip::HIPGuard guard(x_.device().index());
     const int64_t B = x_.size(0), L = x_.size(1), dim = x_.size(2), n = B * L;
     const Tensor x = rows_of(x_, at::kFloat);

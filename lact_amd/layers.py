@@ -43,7 +43,7 @@ def _stream(t: torch.Tensor):
 
 def _act(t: torch.Tensor):
     if not t.is_cuda:
-        raise RuntimeError("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)")
+        raise RuntimeError(f"lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path), got one on {t.device}")
     if t.dtype == torch.bfloat16:
         return LACT_BF16
     if t.dtype == torch.float32:
@@ -66,12 +66,12 @@ class _PreFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qkv, H, hd, l2norm):
-        qkv = qkv.contiguous()
+        qkv, act = qkv.contiguous(), _act(qkv)
         B, L, _ = qkv.shape
         _expect(qkv, qkv.device, (B, L, 3 * H * hd), "qkv")
         q, k, v = (torch.empty((B * H, L, hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3))
         with torch.cuda.device(qkv.device):
-            _lib.check(_lib.lib().lact_layer_pre_forward(_act(qkv), B, L, H, hd, int(l2norm), _ptr(qkv), _ptr(q), _ptr(k),
+            _lib.check(_lib.lib().lact_layer_pre_forward(act, B, L, H, hd, int(l2norm), _ptr(qkv), _ptr(q), _ptr(k),
                                                          _ptr(v), _stream(qkv)))
         ctx.save_for_backward(qkv)
         ctx.dims = (B, L, H, hd, int(l2norm))
@@ -97,7 +97,7 @@ class _PreAttnFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, qkv, qk_scale, qk_offset, H, hd, l2norm):
-        qkv = qkv.contiguous()
+        qkv, act = qkv.contiguous(), _act(qkv)
         B, L, _ = qkv.shape
         _expect(qkv, qkv.device, (B, L, 3 * H * hd), "qkv")
         _expect(qk_scale, qkv.device, (H * hd, 2), "qk_scale")
@@ -107,7 +107,7 @@ class _PreAttnFn(torch.autograd.Function):
         att = [torch.empty((B, L, H * hd), dtype=qkv.dtype, device=qkv.device) for _ in range(3)]
         with torch.cuda.device(qkv.device):
             _lib.check(_lib.lib().lact_layer_pre_attn_forward(
-                _act(qkv), B, L, H, hd, int(l2norm), int(qk_scale.dtype == qkv.dtype), _ptr(qkv), _ptr(scale), _ptr(offset),
+                act, B, L, H, hd, int(l2norm), int(qk_scale.dtype == qkv.dtype), _ptr(qkv), _ptr(scale), _ptr(offset),
                 *[_ptr(t) for t in outs], *[_ptr(t) for t in att], _stream(qkv)))
         ctx.save_for_backward(qkv, scale)
         ctx.dims, ctx.dtypes = (B, L, H, hd, int(l2norm)), (qk_scale.dtype, qk_offset.dtype)
@@ -136,6 +136,7 @@ class _LrFn(torch.autograd.Function):
     @staticmethod
     def forward(ctx, lr_raw, mom_raw, H, base_lr_inv, rates_major=False):
         lr_raw = lr_raw.float().contiguous()
+        _act(lr_raw)
         mom_c = None if mom_raw is None else mom_raw.float().contiguous()
         B, L, _ = lr_raw.shape
         _expect(lr_raw, lr_raw.device, (B, L, 3 * H), "lr_raw")
@@ -175,7 +176,7 @@ class _PostFn(torch.autograd.Function):
 
     @staticmethod
     def forward(ctx, o, weight, gate_raw, B, H, use_norm, eps, add=None):
-        o = o.contiguous()
+        o, act = o.contiguous(), _act(o)
         _, L, hd = o.shape
         _expect(o, o.device, (B * H, L, hd), "o")
         _expect(weight, o.device, (hd,), "weight")
@@ -186,7 +187,7 @@ class _PostFn(torch.autograd.Function):
         add_c = None if add is None else add.to(o.dtype).contiguous()
         y = torch.empty((B, L, H * hd), dtype=o.dtype, device=o.device)
         with torch.cuda.device(o.device):
-            _lib.check(_lib.lib().lact_layer_post_add_forward(_act(o), B, L, H, hd, int(use_norm), float(eps), _ptr(o), _ptr(w),
+            _lib.check(_lib.lib().lact_layer_post_add_forward(act, B, L, H, hd, int(use_norm), float(eps), _ptr(o), _ptr(w),
                                                           _ptr(g), _ptr(add_c), _ptr(y), _stream(o)))
         ctx.save_for_backward(o, w, g)
         ctx.add_dtype = None if add is None else add.dtype

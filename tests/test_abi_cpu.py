@@ -213,3 +213,19 @@ def test_fractional_sizes_are_refused():
         for x in (4.0, 4.5):
             with pytest.raises(TypeError):
                 call(x)
+
+
+def test_layer_functions_refuse_cpu_tensors_by_name():
+    """The host module's and their Python counterparts: the reason and the device, not an error of a device guard."""
+    import torch
+    from lact_amd import layers as HL
+    host, r = _lib.host(), torch.randn
+    pre, scale = (r(1, 5, 96), r(32, 2), r(32, 2)), (1, 32, True)
+    post = (r(2, 5, 32), None, None, 1, 2, True, 1e-5, None)
+    calls = [(host.layer_pre, (pre[0], *scale)), (host.layer_pre_attn, (*pre, *scale)), (host.layer_lr, (r(1, 5, 3), None, 1, 0.1, False)),
+             (host.layer_post, post), (host.linear, (r(1, 5, 32), r(8, 32))), (host.layer_in, (r(1, 5, 32), r(96, 32), r(3, 32), None, None, None, None, None)),
+             (HL._PreFn.apply, (pre[0], *scale)), (HL._PreAttnFn.apply, (*pre, *scale)), (HL._LrFn.apply, (r(1, 5, 3), None, 1, 0.1, False)),
+             (HL._PostFn.apply, post), (HL.BidirectionalLaCTSwiGLU(32, 16), (r(1, 5, 32),))]
+    for fn, args in calls:
+        with pytest.raises(RuntimeError, match="runs on an MI355X only.*cpu"):
+            fn(*args)

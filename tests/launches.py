@@ -1,0 +1,17 @@
+"""Which kernels a call launched, from the library's launch report: a comparison of two paths has to know that it took both."""
+import ctypes
+import json
+
+from lact_amd import _lib
+
+
+def kernels(fn):
+    """What fn returns, and the names of the kernels that it launched."""
+    lib, buf = _lib.lib(), ctypes.create_string_buffer(1 << 16)
+    _lib.check(lib.lact_profile_enable(1))
+    try:
+        res = fn()
+        _lib.check(lib.lact_profile_report(buf, len(buf)))
+    finally:
+        _lib.check(lib.lact_profile_enable(0))
+    return res, {r["kernel"] for r in json.loads(buf.value)}

@@ -2,6 +2,7 @@
 backward passes of the operation against the oracle, fp32 and bf16 with head sizes that are no multiple of 16."""
 import pytest
 import torch
+from launches import kernels
 
 from oracle import lact_oracle as O
 
@@ -223,13 +224,20 @@ def test_wide_hidden_tiles_have_the_same_bits(b, d, dh, T):
     inp = {n: t.to("cuda") for n, t in O.make_inputs(b, L, d, dh, seed=71, act_dtype=torch.bfloat16).items()}
     go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(5)).bfloat16().to("cuda")
     prog = ops.Program(steps=((LACT_APPLY, 0, T, 0), (LACT_UPDATE, 0, T, 0), (LACT_APPLY, T, L, T), (LACT_UPDATE, T, L, 0)), out_len=L)
+
+    def step():
+        leaves = [inp[n].clone().requires_grad_(True) for n in ORDER[:9]]
+        out, ws, _ = ops.run_program(prog, *leaves)
+        return [out.detach(), *[w.detach() for w in ws], *torch.autograd.grad(out, leaves, go)]
+
     res = []
     for mask in (1, 7):
         prev = _lib.lib().lact_set_option(_lib.OPT_PERSISTENT_TILES, mask)
         try:
-            leaves = [inp[n].clone().requires_grad_(True) for n in ORDER[:9]]
-            out, ws, _ = ops.run_program(prog, *leaves)
-            res.append([out.detach(), *[w.detach() for w in ws], *torch.autograd.grad(out, leaves, go)])
+            values, names = kernels(step)
+            res.append(values)
+            assert ({"k_update_hidden_wide", "k_apply_bwd_hidden_wide"} <= names) == (mask == 1)
+            assert ({"k_hidden_persist<update>", "k_hidden_persist<apply_bwd>"} <= names) == (mask == 7)
         finally:
             _lib.lib().lact_set_option(_lib.OPT_PERSISTENT_TILES, prev)
     for a, r in zip(*res):

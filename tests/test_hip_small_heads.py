@@ -1,9 +1,7 @@
 """The kernels that run a whole step of small bf16 heads (csrc/small_heads.h) against the ones that run it in pieces."""
-import ctypes
-import json
-
 import pytest
 import torch
+from launches import kernels
 
 from lact_amd import _lib, ops
 from lact_amd._lib import LACT_APPLY, LACT_UPDATE
@@ -20,18 +18,6 @@ def in_pieces(fn):
         return fn()
     finally:
         _lib.lib().lact_set_option(_lib.OPT_PERSISTENT_TILES, prev)
-
-
-def kernels(fn):
-    """What fn returns, and the names of the kernels that it launched."""
-    lib, buf = _lib.lib(), ctypes.create_string_buffer(1 << 16)
-    _lib.check(lib.lact_profile_enable(1))
-    try:
-        res = fn()
-        _lib.check(lib.lact_profile_report(buf, len(buf)))
-    finally:
-        _lib.check(lib.lact_profile_enable(0))
-    return res, {r["kernel"] for r in json.loads(buf.value)}
 
 
 # both sides of the line: hidden units at few tokens, tokens at many hidden units, whole blocks
@@ -118,7 +104,8 @@ def test_update_in_one_kernel(b, T, d, dh):
         return [out, *w, *m]
 
     with torch.no_grad():
-        whole, view, ref = run(t["k"], t["v"]), run(wide[..., 8:d + 8], wide[..., d + 8:2 * d + 8]), in_pieces(lambda: run(t["k"], t["v"]))
+        (whole, names), view, ref = kernels(lambda: run(t["k"], t["v"])), run(wide[..., 8:d + 8], wide[..., d + 8:2 * d + 8]), in_pieces(lambda: run(t["k"], t["v"]))
+    assert "k_update_fused" in names
     for i, (a, c, r) in enumerate(zip(whole, view, ref)):
         assert torch.equal(a, c) and torch.isfinite(a.float()).all()
         assert O.rel_l2(a, r) < 1e-3, (i, O.rel_l2(a, r))
@@ -178,7 +165,8 @@ def test_tokens_gradients_in_one_kernel(b, T, d, dh):
             g += [p[..., 8:d + 8], p[..., d + 8:]]
         return g
 
-    whole, view, ref = run(False), run(True), in_pieces(lambda: run(False))
+    (whole, launched), view, ref = kernels(lambda: run(False)), run(True), in_pieces(lambda: run(False))
+    assert "k_update_bwd_fused" in launched
     for n, a, c, r in zip([n for n in names if n not in ("k", "v")] + ["k", "v"], whole, view, ref):
         assert torch.isfinite(a.float()).all() and torch.equal(a, c), n
         assert O.rel_l2(a, r) < 3e-3, (n, O.rel_l2(a, r))
@@ -187,7 +175,7 @@ def test_tokens_gradients_in_one_kernel(b, T, d, dh):
 
 
 # three applies between updates: two of them share launches; small steps, which only the apply's kernel takes
-@pytest.mark.parametrize("b,T,d,dh", [(1, 1, 64, 32), (2, 33, 96, 64), (3, 127, 128, 96), (1, 257, 128, 160), (2, 300, 64, 96)])
+@pytest.mark.parametrize("b,T,d,dh", [(1, 1, 64, 32), (2, 33, 96, 64), (3, 127, 128, 96), (24, 257, 128, 160), (2, 300, 64, 96)])
 def test_queries_gradients_in_one_kernel(b, T, d, dh):
     print("[gpu-test] queries' gradients in one kernel", b, T, d, dh, flush=True)
     L = 3 * T
@@ -199,5 +187,40 @@ def test_queries_gradients_in_one_kernel(b, T, d, dh):
         t = [inp[n].clone().requires_grad_(True) for n in ORDER]
         return torch.autograd.grad(ops.run_program(prog, *t)[0], t, go)
 
-    for n, a, r in zip(ORDER, run(), in_pieces(run)):
+    whole, names = kernels(run)
+    assert "k_apply_bwd_fused" in names
+    for n, a, r in zip(ORDER, whole, in_pieces(run)):
         assert torch.isfinite(a.float()).all() and O.rel_l2(a, r) < 3e-3, (n, O.rel_l2(a, r))
+
+
+# the first and the last token of a wave's 32, the last one of a ragged block (whose surplus lanes repeat it)
+@pytest.mark.parametrize("token", [0, 31, 32, 69])
+def test_infinities_in_the_backward(token):
+    """An infinite token of an update spoils its head's gradients, an infinite row of an apply's gradient that head's first weights and its
+    own query: nothing else, and the same places as in pieces."""
+    print("[gpu-test] infinities in the backward", token, flush=True)
+    b, T, d, dh = 200, 70, 64, 32
+    inp = {n: x.to(DEV) for n, x in O.make_inputs(b, 2 * T, d, dh, seed=67, act_dtype=torch.bfloat16).items()}
+    inp["v"][1, token] = float("inf")
+    prog = ops.Program(steps=((LACT_APPLY, 0, T, 0), (LACT_UPDATE, 0, T, 0), (LACT_APPLY, T, 2 * T, T)), out_len=2 * T)
+    go = torch.randn(b, 2 * T, d, generator=torch.Generator().manual_seed(3)).bfloat16().to(DEV)
+    go[3, token] = float("inf")
+
+    def run():
+        t = [inp[n].clone().requires_grad_(True) for n in ORDER]
+        return torch.autograd.grad(ops.run_program(prog, *t)[0], t, go)
+
+    whole, names = kernels(run)
+    assert {"k_update_bwd_fused", "k_apply_bwd_fused"} <= names
+    for n, a, r in zip(ORDER, whole, in_pieces(run)):
+        fine = torch.isfinite(a.float())
+        assert torch.equal(fine, torch.isfinite(r.float())), n
+        heads = set(range(b)) - {1} - ({3} if n in ("w0", "w1", "w2", "q") else set())
+        assert fine[sorted(heads)].all() and not fine[1].all(), n
+        if n == "q":
+            rows = fine[3].all(dim=-1)
+            assert int((~rows).sum()) == 1 and not rows[token]
+        elif n in ("w0", "w1", "w2"):
+            assert not fine[3].all()
+        a, r = a.float()[sorted(heads)], r.float()[sorted(heads)]
+        assert O.rel_l2(a, r) < 3e-3, n

@@ -376,6 +376,55 @@ __device__ __forceinline__ uint4 pack8(const float (&f)[8]) {
   return make_uint4(w[0], w[1], w[2], w[3]);
 }
 
+// Pointwise parts of the hidden stages, eight neighbours in a row at `off`, from the rounded products to the stores; shared by the kernels
+// of every tile.  An update's: gate, hidden and dhidden as in update_pointwise2, `keep` as below; an apply's backward: y0, y2 and
+// the gradient of the gated hidden values.
+__device__ __forceinline__ void update_pointwise8(const HiddenParams& p, size_t off, bool keep, const uint4& ug, const uint4& uh, const uint4& ud, float l0, float l1, float l2) {
+  float gg[8], h2[8], dh[8], z1[8], y0[8], y2[8];
+  uint32_t z0[4], z2[4];
+  unpack8(ug, gg);
+  unpack8(uh, h2);
+  unpack8(ud, dh);
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const UpdatePointwise2 u = update_pointwise2(gg + 2 * j, h2 + 2 * j, dh + 2 * j, silu_parts(gg[2 * j]), silu_parts(gg[2 * j + 1]));
+    z0[j] = u.dgpre_2; z2[j] = u.dh2_2;
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      z1[2 * j + e] = u.hid[e] * l1;
+      y0[2 * j + e] = u.dgpre[e] * l0; y2[2 * j + e] = u.dh2[e] * l2;
+    }
+  }
+  *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = make_uint4(z0[0], z0[1], z0[2], z0[3]);
+  *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(z1);
+  *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = make_uint4(z2[0], z2[1], z2[2], z2[3]);
+  if (keep) {   // the backward is going to start from the rounded pre-activations instead of recomputing them
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O3) + off) = ug;
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O4) + off) = uh;
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O5) + off) = ud;
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O6) + off) = pack8(y0);
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O7) + off) = pack8(y2);
+  }
+}
+__device__ __forceinline__ void apply_bwd_pointwise8(const HiddenParams& p, size_t off, const uint4& u0, const uint4& u2, const uint4& ug) {
+  float y0[8], y2[8], gh[8], hq[8], gy0[8], gy2[8];
+  unpack8(u0, y0);
+  unpack8(u2, y2);
+  unpack8(ug, gh);
+#pragma unroll
+  for (int j = 0; j < 8; j += 2) {
+    const SiluParts s0 = silu_parts(y0[j]), s1 = silu_parts(y0[j + 1]);
+    float sg0 = s0.silu, sg1 = s1.silu, t0 = gh[j] * y2[j], t1 = gh[j + 1] * y2[j + 1];
+    round_both(sg0, sg1);
+    round_both(t0, t1);
+    hq[j] = sg0 * y2[j]; gy0[j] = t0 * s0.d1; gy2[j] = gh[j] * sg0;
+    hq[j + 1] = sg1 * y2[j + 1]; gy0[j + 1] = t1 * s1.d1; gy2[j + 1] = gh[j + 1] * sg1;
+  }
+  *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = pack8(hq);
+  *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(gy0);
+  *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = pack8(gy2);
+}
+
 // update forward.  O0 = dgate_before_act, O1 = hidden * lr1, O2 = dhidden_before_mul (the operands of the three
 // fast-weight gradient GEMMs: lr0 and lr2 scale k there, ttt_operation.py:166-168).  For the backward, when O3 is set:
 // O3..O5 = the rounded pre-activations, O6 = O0 * lr0, O7 = O2 * lr2.
@@ -437,31 +486,7 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_update_hidden_dma(const Hi
   for (int ps = 0; ps < SB::PASSES; ++ps) {
     const int r = r0 + ps * SB::RPP;
     if (r < TS::BM && m0 + r < p.T) {
-      float gg[8], h2[8], dh[8], z1[8], y0[8], y2[8];
-      uint32_t z0[4], z2[4];
-      unpack8(ug[ps], gg);
-      unpack8(uh[ps], h2);
-      unpack8(ud[ps], dh);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const UpdatePointwise2 u = update_pointwise2(gg + 2 * j, h2 + 2 * j, dh + 2 * j, silu_parts(gg[2 * j]), silu_parts(gg[2 * j + 1]));
-        z0[j] = u.dgpre_2; z2[j] = u.dh2_2;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          z1[2 * j + e] = u.hid[e] * l1[ps];
-          y0[2 * j + e] = u.dgpre[e] * l0[ps]; y2[2 * j + e] = u.dh2[e] * l2[ps];
-        }
-      }
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = make_uint4(z0[0], z0[1], z0[2], z0[3]);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(z1);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = make_uint4(z2[0], z2[1], z2[2], z2[3]);
-      if (keep) {   // the backward is going to start from the rounded pre-activations instead of recomputing them
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O3) + off) = ug[ps];
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O4) + off) = uh[ps];
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O5) + off) = ud[ps];
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O6) + off) = pack8(y0);
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O7) + off) = pack8(y2);
-      }
+      update_pointwise8(p, off, keep, ug[ps], uh[ps], ud[ps], l0[ps], l1[ps], l2[ps]);
     }
     off += step;
   }
@@ -502,22 +527,7 @@ __global__ __launch_bounds__(DMA_THREADS, WPE) void k_apply_bwd_hidden_dma(const
   for (int ps = 0; ps < SB::PASSES; ++ps) {
     const int r = r0 + ps * SB::RPP;
     if (r < TS::BM && m0 + r < p.T) {
-      float y0[8], y2[8], gh[8], hq[8], gy0[8], gy2[8];
-      unpack8(u0[ps], y0);
-      unpack8(u2[ps], y2);
-      unpack8(ug[ps], gh);
-#pragma unroll
-      for (int j = 0; j < 8; j += 2) {
-        const SiluParts s0 = silu_parts(y0[j]), s1 = silu_parts(y0[j + 1]);
-        float sg0 = s0.silu, sg1 = s1.silu, t0 = gh[j] * y2[j], t1 = gh[j + 1] * y2[j + 1];
-        round_both(sg0, sg1);
-        round_both(t0, t1);
-        hq[j] = sg0 * y2[j]; gy0[j] = t0 * s0.d1; gy2[j] = gh[j] * sg0;
-        hq[j + 1] = sg1 * y2[j + 1]; gy0[j + 1] = t1 * s1.d1; gy2[j + 1] = gh[j + 1] * sg1;
-      }
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = pack8(hq);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(gy0);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = pack8(gy2);
+      apply_bwd_pointwise8(p, off, u0[ps], u2[ps], ug[ps]);
     }
     off += step;
   }

@@ -282,32 +282,7 @@ __global__ __launch_bounds__(512, 2) void k_update_hidden_wide(const HiddenDmaPa
       const int m = m0 + r;
       if (m >= p.T || n0 + c >= p.dh) return;
       const float l0 = p.lr0[z * p.bslr + m], l1 = p.lr1[z * p.bslr + m], l2 = p.lr2[z * p.bslr + m];
-      float gg[8], h2[8], dh[8], z1[8], y0[8], y2[8];
-      uint32_t z0[4], z2[4];
-      unpack8(u[0], gg);
-      unpack8(u[1], h2);
-      unpack8(u[2], dh);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const UpdatePointwise2 w = update_pointwise2(gg + 2 * j, h2 + 2 * j, dh + 2 * j, silu_parts(gg[2 * j]), silu_parts(gg[2 * j + 1]));
-        z0[j] = w.dgpre_2; z2[j] = w.dh2_2;
-#pragma unroll
-        for (int e = 0; e < 2; ++e) {
-          z1[2 * j + e] = w.hid[e] * l1;
-          y0[2 * j + e] = w.dgpre[e] * l0; y2[2 * j + e] = w.dh2[e] * l2;
-        }
-      }
-      const size_t off = z * p.bso + (size_t)m * p.dh + n0 + c;
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = make_uint4(z0[0], z0[1], z0[2], z0[3]);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(z1);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = make_uint4(z2[0], z2[1], z2[2], z2[3]);
-      if (keep) {
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O3) + off) = u[0];
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O4) + off) = u[1];
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O5) + off) = u[2];
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O6) + off) = pack8(y0);
-        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O7) + off) = pack8(y2);
-      }
+      update_pointwise8(p, z * p.bso + (size_t)m * p.dh + n0 + c, keep, u[0], u[1], u[2], l0, l1, l2);
     });
 }
 
@@ -325,20 +300,7 @@ __global__ __launch_bounds__(512, 2) void k_apply_bwd_hidden_wide(const HiddenDm
   wide_epilogue<3>(smem, [&](int i, int tm, int tn, int g) { return i == 2 ? y[tm][tn][g] : pack4(x[i][tm][tn], g); },
     [&](int r, int c, const uint4 (&u)[3]) {
       if (m0 + r >= p.T || n0 + c >= p.dh) return;
-      float y0[8], y2[8], gh[8], hq[8], gy0[8], gy2[8];
-      unpack8(u[0], y0);
-      unpack8(u[1], y2);
-      unpack8(u[2], gh);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const SiluParts sp = silu_parts(y0[j]);
-        const float sg = round_bf16(sp.silu);
-        hq[j] = sg * y2[j]; gy0[j] = round_bf16(gh[j] * y2[j]) * sp.d1; gy2[j] = gh[j] * sg;
-      }
-      const size_t off = z * p.bso + (size_t)(m0 + r) * p.dh + n0 + c;
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O0) + off) = pack8(hq);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O1) + off) = pack8(gy0);
-      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.O2) + off) = pack8(gy2);
+      apply_bwd_pointwise8(p, z * p.bso + (size_t)(m0 + r) * p.dh + n0 + c, u[0], u[1], u[2]);
     });
 }
 

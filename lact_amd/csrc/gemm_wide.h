@@ -9,7 +9,8 @@
 // 28, matrix instructions and fragments 20.  The apply's two products run as fast on persistent 128 x 128 tiles.
 //
 // Ring: three slots of the token tile (32 KiB) and two of the weight tiles (2 x 16 KiB), all 160 KiB of LDS.  The token rows come
-// from HBM and are asked for three K-steps ahead, the weights from the L2 two ahead.  One barrier per K-step.
+// from HBM and are asked for three K-steps ahead, the weights from the L2 two ahead.  One barrier per K-step.  All 256 registers of a wave
+// are in use; eight more (36 bytes a lane) are stored and read back once a block, outside the loops.
 #pragma once
 #include <type_traits>
 

@@ -567,7 +567,8 @@ __global__ __launch_bounds__(256) void k_layer_in(const LayerInParams p) {
 }
 
 // Gradient of the input: dx = dxq + sum over the outputs of gradient times weight row.  A lane owns four columns and keeps their
-// weights, the block's tokens have their output gradients in LDS.  Grid (token blocks, column blocks of blockDim.x * 4).
+// weights, the block's tokens have their output gradients in LDS.  Grid (token blocks, column blocks of blockDim.x * 4).  All 40 outputs take
+// 256 registers and seven accumulation registers, one wave a SIMD; more outputs would need a second pass.
 template <int NL, int NB>
 __global__ __launch_bounds__(256) void k_layer_in_dx(const LayerInParams p) {
   constexpr int NO = 4 * (NL + NB), TOK = LAYER_IN_DXTOK;

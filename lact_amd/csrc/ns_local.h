@@ -13,7 +13,8 @@
 // barriers, 1.7 us of vector issue of the two waves on a SIMD.  Measured at 18 matrices of 128 x 256: 33 us; all 16 tiles of A, c A
 // from LDS for B only, divisions for the normalisation and the products in the compiler's order 40; 66-68 us as k_ns_fused (four
 // compute units per matrix, every stage handed over through the L2).  24 of 96 x 96: 20 us against 25; 6 of 64 x 64 14 against 15, and
-// 74 as three launches per iteration.
+// 74 as three launches per iteration.  At 96 and 128 rows of more than 128 columns all 256 registers are in use and one or three
+// addresses (up to 12 bytes a lane) are stored once and read back once an iteration, outside the products' loops.
 #pragma once
 #include "ns_fused.h"
 

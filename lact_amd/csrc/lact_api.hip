@@ -518,7 +518,7 @@ struct Runner {
     return ceil_div(d.dh, TS_BWD::BN) * TS_BWD::WAVES_N;
   }
   bool hidden_small(int which) const { return which == 0 ? d.d <= 256 : which <= 3 && d.d <= 192; }   // the kernel from kept pre-activations has the large tile only
-  // 256 x 128 tiles where their rounds of blocks, one to a compute unit and 1.6 times as long as those of 128 x 128 tiles, take less
+  // 256 x 128 tiles where their rounds of blocks, one to a compute unit and 1.62 times as long as those of 128 x 128 tiles, take less
   // time (gemm_wide.h).
   bool hidden_wide(int T_, int nz) const {
     if (d.d % 64 || d.d < 384 || d.dh % 8) return false;

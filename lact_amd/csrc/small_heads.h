@@ -638,10 +638,11 @@ struct BwdStage {
   static_assert(LDS <= 160 * 1024, "the ring does not fit the LDS");
 };
 
-// The barrier alone: __syncthreads would wait for the wave's stores to memory as well.  What the wave has asked LDS for has been used by
-// then (its matrix instructions), and its copies into LDS are waited for by name; no access of the program moves across.
+// The barrier without the wait for the wave's stores to memory that __syncthreads adds.  The wave's reads of LDS are done, which a slot's
+// next copy has to be sure of (they are used by then, so the wait costs nothing; but where their last uses stand is the compiler's
+// choice), and its copies into LDS are waited for by name; no access of the program moves across.
 __device__ __forceinline__ void block_barrier() {
-  asm volatile("" ::: "memory");
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
 }

@@ -626,11 +626,12 @@ struct Runner {
   // units, which the kernels in pieces spread over blocks: it loses where there are many of them and few tokens.  us on the GPU (a graph
   // of calls, the initial state's kernel included), in pieces / as one: d = 128, 64 tokens, dh = 128 10.3 / 10.9, 256 10.7 / 14.2, 1024
   // 14.7 / 35.9, 2048 20 / 65; 6 x 1024 tokens, dh = 256 14.6 / 17.0, 512 18.7 / 25.3, 2048 41 / 72; 12 x 1024, dh = 256 18.2 / 19.2; d = 64,
-  // 6 x 1024, dh = 512 16.4 / 18.3.  Against that stands one launch less, 3.5 us of host time, which is what a short call is bound by (nvs
-  // rendering of 6 x 1024 tokens, dh = 256: 19.5 / 17.7): the one kernel may be 3 us behind.  Whole blocks never are (dh = 64 to 2048).
+  // 6 x 1024, dh = 512 16.4 / 18.3.  Against that stands one launch less, 3.5 us of host time (calls one after the other, 64 tokens, dh =
+  // 64: 14.7 us in pieces, 10.8 as one), which is what a short call is bound by (nvs rendering of 6 x 1024 tokens, dh = 256: 19.5 / 17.7):
+  // the one kernel may be that far behind, which it is at 256 hidden units of d = 128.  Whole blocks never lose (dh = 64 to 2048).
   bool apply_fused_pays(int T_, int nz) const {
     const double longer = d.dh / 32 * (0.23 + d.d / 256.0) - 1.05e-6 * T_ * nz * d.dh - 2.2;     // (fitted: 1.3 us off on average)
-    return ceil_div(T_, 128) * nz > 256 || longer <= 3;
+    return ceil_div(T_, 128) * nz > 256 || longer <= 4;
   }
   bool apply_fused(const HiddenParams& hp, const RowGemmParams<1>& out, int T_, int steps) const {
     if constexpr (kBf16) {

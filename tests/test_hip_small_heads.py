@@ -22,8 +22,8 @@ def in_pieces(fn):
 
 # both sides of the line: hidden units at few tokens, tokens at many hidden units, whole blocks
 @pytest.mark.parametrize("b,T,d,dh,one", [
-    (1, 64, 128, 128, True), (1, 64, 128, 256, False), (6, 1024, 128, 256, True), (2, 1024, 128, 256, False), (1, 64, 64, 320, True),
-    (1, 64, 64, 512, False), (1, 64, 96, 256, True), (2, 129, 96, 512, False), (6, 1024, 128, 512, False), (20, 1024, 128, 512, True),
+    (1, 64, 128, 256, True), (1, 64, 128, 288, False), (6, 1024, 128, 320, True), (2, 1024, 128, 320, False), (1, 64, 64, 384, True),
+    (1, 64, 64, 512, False), (1, 64, 96, 320, True), (2, 129, 96, 512, False), (6, 1024, 128, 512, False), (20, 1024, 128, 512, True),
     (1, 1, 64, 2048, False), (33, 1024, 96, 1024, True), (260, 64, 128, 1024, True)])
 def test_apply_takes_the_faster_kernels(b, T, d, dh, one):
     """A wave of the one kernel walks all hidden units, however few tokens there are: few tokens with many of them go in pieces."""

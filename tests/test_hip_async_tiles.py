@@ -174,7 +174,8 @@ def test_newton_schulz_in_one_block_is_bit_identical(b, d, dh, L, stacked):
             _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, fused)
             try:
                 leaves = [inp[n].clone().requires_grad_(True) for n in ORDER[:9]]
-                out, ws, _ = ops.run_program(prog, *leaves)
+                (out, ws, _), launched = kernels(lambda: ops.run_program(prog, *leaves))
+                assert ("k_ns_local" in launched) == (fused == 1)
                 grads = torch.autograd.grad(out, leaves, go)
                 with torch.no_grad():
                     out_inf, ws_inf, _ = ops.run_program(prog, *[inp[n] for n in ORDER[:9]])
@@ -204,7 +205,8 @@ def test_normalisation_of_extreme_gradients(scale, zeros):
         _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, fused)
         try:
             with torch.no_grad():
-                out, ws, _ = ops.run_program(prog, *[inp[n] for n in ORDER[:9]])
+                (out, ws, _), launched = kernels(lambda: ops.run_program(prog, *[inp[n] for n in ORDER[:9]]))
+            assert ("k_ns_local" in launched) == (fused == 1)
             res.append([out, *ws])
         finally:
             _lib.lib().lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 1)

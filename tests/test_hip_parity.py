@@ -22,6 +22,7 @@ import sys
 import numpy as np
 import pytest
 import torch
+from launches import kernels
 
 from lact_amd import ar_video, minimal, nvs, ops
 from lact_amd import ttt_operation as T
@@ -1150,10 +1151,13 @@ def test_persistent_tiles_are_bit_identical(b, L, d, dh, C, muon):
         return res
     L_ = _lib.lib()
     prev = L_.lact_set_option(_lib.OPT_PERSISTENT_TILES, 7)      # all three hidden-stage kernels persistent
+    persistent = {f"k_hidden_persist<{n}>" for n in ("apply", "update", "apply_bwd")}
     try:
         on = run()
+        assert persistent <= kernels(run)[1]
         L_.lact_set_option(_lib.OPT_PERSISTENT_TILES, 0)
         off = run()
+        assert not persistent & kernels(run)[1]
     finally:
         L_.lact_set_option(_lib.OPT_PERSISTENT_TILES, prev)
     for (o1, g1), (o0, g0) in zip(on, off):
@@ -1187,9 +1191,11 @@ def test_kept_and_recomputed_update_backward_agree(b, L, d, dh, C, muon):
     L_ = _lib.lib()
     prev = L_.lact_set_option(_lib.OPT_KEEP_PREACTIVATIONS, 1)
     try:
-        o1, g1 = run()
+        (o1, g1), launched = kernels(run)
+        assert "k_update_bwd_hidden_kept_dma" in launched
         L_.lact_set_option(_lib.OPT_KEEP_PREACTIVATIONS, 0)
-        o0, g0 = run()
+        (o0, g0), launched = kernels(run)
+        assert "k_update_bwd_hidden_dma" in launched and "k_update_bwd_hidden_kept_dma" not in launched
     finally:
         L_.lact_set_option(_lib.OPT_KEEP_PREACTIVATIONS, prev)
     assert torch.equal(o1, o0)
@@ -1230,10 +1236,13 @@ def test_fused_newton_schulz_is_bit_identical(b, d, dh, chunks):
         return res
     L_ = _lib.lib()
     prev = L_.lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 1)
+    fused = lambda: {n[-4:-1] for n in kernels(run)[1] if n.startswith("k_ns_fused")}
     try:
         on = run()
+        assert "bwd" in fused()      # (the forward of small matrices runs in one block each)
         L_.lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 0)
         off = run()
+        assert not fused()
     finally:
         L_.lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, prev)
     for (o1, g1), (o0, g0) in zip(on, off):

@@ -311,8 +311,13 @@ struct DmaPipe {
   // issue the copies, not only with the bytes in flight (measured with loads that hit the L2: 22 / 45 / 75 GB/s
   // per compute unit from 2 / 4 / 8 issuing waves at the same depth), so four loader waves beside the four MFMA
   // waves: eight waves are what the register budget of the MFMA waves (256 each) allows.
+  // gate(p) is called in front of the first copy of phase p.
   template <int MINLOADS>
   __device__ __forceinline__ void load_all() {
+    load_all<MINLOADS>([](int) {});
+  }
+  template <int MINLOADS, class GATE>
+  __device__ __forceinline__ void load_all(GATE gate) {
     constexpr int PER_WAVE = MINLOADS / DMA_LOADERS;
     constexpr int AHEAD = (STAGES - 2) * PER_WAVE > 63 ? 63 : (STAGES - 2) * PER_WAVE;
     const int lw = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) - 4;
@@ -335,6 +340,7 @@ struct DmaPipe {
     };
     auto issue_stage = [&]() {
       const uint32_t base = lds_addr(smem + (issued % STAGES) * SM::STAGE) + lw * 1024;
+      if (ckt == 0) gate(cp);
       if (cshort > 0 && ckt + 1 == cnk) {
 #pragma unroll
         for (int i = 0; i < NPH; ++i)

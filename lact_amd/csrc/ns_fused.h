@@ -10,8 +10,17 @@
 //   * a stage's stores are complete in that L2 once the block has waited for them (vmcnt) -- no L2
 //     write-back is needed inside an XCD -- and the operands written by the partner blocks are read with
 //     device-scope loads that miss the (non-coherent) vector L1;
-//   * the barrier is a counter in that L2: arrive = atomic add, wait = poll (measured ~1.3 us per barrier
-//     against ~4.5 us of launch gap plus the write-back of everything the kernel stored).
+//   * the barrier is a counter in that L2: arrive = atomic add, wait = poll (measured ~0.6 us per barrier
+//     against ~4.5 us of launch gap plus the write-back of everything the kernel stored).  Only the waves that copy
+//     the operands wait, and only in front of the first operand that a partner block has just written.
+//
+// What bounds it: a stage is a main loop of six K-steps (twelve backwards), the staging of its tile and the exchange.  48 matrices
+// of 384 x 384 on 192 compute units, forward / backward: a stage 11 / 16.5 us, of which the matrix instructions take 3.6 / 7.2; 6.5 /
+// 13 main loop (8 matrices, whose operands stay in the L2s, 5.1 / 8.5: the rest is misses), 2.7 epilogue, 1.5 stores, barrier and set-up.
+// Launch: 214 -> 166 and 260 -> 249 us against epilogues that chose their case element by element, read the auxiliary tile behind
+// the staging and had every wave wait at the barrier; six matrices of 768 x 1536, three iterations: 195 -> 173.
+// Tried: the next stage's saved operand asked for into the L2 in the epilogue (-3 % there, +2 % at 12 matrices of 384 x 768);
+// non-temporal loads where an operand is read for the last time (+5 %: the partner block reads it too).
 //
 // Should the hardware place a group's blocks on different XCDs (each block publishes its XCC id at the
 // start and the group checks), the group falls back to device-scope release/acquire fences around every
@@ -44,7 +53,7 @@ struct NsFusedParams {
   // backward: incoming gradient in gxf[0] / gxb[0]; the result ends in gxf[S & 1]
   float* gxf[2]; uint16_t* gxb[2]; uint16_t* sg; uint16_t* gas;
   // forward, optional first stage: X_0 = G / (|G|_F + 1e-7) from the bf16 gradient g16 (laid out like xb) and the
-  // partial sums of its squares; writes xf[0], xb (iteration 0) and the norms.  Null g16: X_0 is there already.
+  // partial sums of its squares; writes xb (iteration 0) and the norms.  Null g16: X_0 is there already.
   const uint16_t* g16; const float* ss_part; int nparts, part0, part1;   // partial rows part0 + z and (if >= 0) part1 + z
   float* norms;              // [n] of this batch
   // backward, optional last stages (the backward of that normalisation): every block writes <G_final, g16> over
@@ -78,32 +87,41 @@ struct GroupBarrier {
     unsigned m = __hip_atomic_load(line + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     split = (m & (m - 1)) != 0;
   }
-  // all threads of the block call it
-  __device__ __forceinline__ void sync(unsigned* error, bool heavy = false) {
+  // All threads of the block call it: the block's stores are there for its partners.
+  __device__ __forceinline__ void arrive(bool heavy = false) {
     // Every wave waits for its own stores of the stage: a store that has been waited for is in this XCD's L2 (the
     // vector L1 writes through), which is where the partner blocks' device-scope loads look.  Without the wait the
     // arrival below could overtake a store that is still on its way to another L2 channel.
     wait_vmcnt<0>();
     __syncthreads();
+    ++epoch;
     if (threadIdx.x == 0) {
-      const bool fence = heavy || split;
-      if (fence) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      if (heavy || split) __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
       __hip_atomic_fetch_add(ctr, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-      const unsigned target = members * (++epoch);
-      long long spins = 0;
-      while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
-        __builtin_amdgcn_s_sleep(1);
-        if (++spins >= limit) {
-          __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          if (sticky) __hip_atomic_fetch_add(sticky, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-          break;
-        }
-      }
-      if (fence) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
-    } else {
-      ++epoch;
     }
+  }
+  // One lane of every wave that is going to read what the partners stored polls until all of them have arrived.
+  __device__ __forceinline__ void wait(unsigned* error, bool heavy = false) const {
+    const unsigned target = members * epoch;
+    long long spins = 0;
+    while (__hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) < target) {
+      __builtin_amdgcn_s_sleep(1);
+      if (++spins >= limit) {
+        __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (sticky) __hip_atomic_fetch_add(sticky, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        break;
+      }
+    }
+    if (heavy || split) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+  }
+  // All threads of the block call it.  A block waits for every arrival of its own before the next one: the count tells no two apart.
+  __device__ __forceinline__ void pass(unsigned* error, bool heavy = false) const {
+    if (threadIdx.x == 0) wait(error, heavy);
     __syncthreads();
+  }
+  __device__ __forceinline__ void sync(unsigned* error, bool heavy = false) {
+    arrive(heavy);
+    pass(error, heavy);
   }
 };
 
@@ -169,102 +187,167 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_bwd_dot_tiles(const NsTileDo
   if (threadIdx.x == 0) p.dot_part[(size_t)z * gridDim.x + member] = dot;
 }
 
+// Granules of 8 elements of a TS tile, dealt to THREADS threads: LPR lanes cover CB neighbouring columns of a row and the threads RP
+// rows; granule t of a thread lies at a distance from its first one that is a compile-time multiple of the row stride and columns.
+template <class TS, int THREADS>
+struct NsGranules {
+  static constexpr int LPR = TS::BN % 64 == 0 ? 8 : 4, CB = LPR * 8, RP = THREADS / LPR, NR = TS::BM / RP, NC = TS::BN / CB, N = NR * NC;
+  static_assert(TS::BM % RP == 0 && TS::BN % CB == 0, "granules split evenly over the threads");
+  __device__ static __forceinline__ int row0() { return (threadIdx.x & (THREADS - 1)) / LPR; }
+  __device__ static __forceinline__ int col0() { return (threadIdx.x % LPR) * 8; }
+  __device__ static constexpr int row(int t) { return (t % NR) * RP; }
+  __device__ static constexpr int col(int t) { return (t / NR) * CB; }
+};
+
 // The roles of a block's waves are split for the whole of the iterations, not stage by stage: the fp32 iterate (its gradient) of
 // this block's tile then lives in the copy waves' registers, 18 granules of 8 elements per thread at 192 x 192, and only its bf16
 // copy goes through memory.  In one code path for all waves it would have to live beside the matrix waves' accumulators.
-// Measured, 48 matrices of 384 x 384, forward: an iteration took 39 us, 7.4 of them in the epilogue that read and wrote the fp32
-// tile, whose 28 MB per direction also pushed the operands out of the L2s; now 36.
 template <class TS>
 struct NsTileRegs {
-  static constexpr int GR = TS::BN / 8, N = TS::BM * GR / 256;   // granules per row; per copy-wave thread
-  static_assert(TS::BM * GR % 256 == 0, "granules split evenly over the copy waves");
-  float v[N][8];
+  using G = NsGranules<TS, 256>;
+  float v[G::N][8];
 };
-// Granule t of a copy-wave thread: its row and first column inside the tile
-template <class TS>
-__device__ __forceinline__ void ns_granule(int t, int& row, int& col) {
-  const int id = (threadIdx.x & 255) + t * 256;
-  row = id / NsTileRegs<TS>::GR;
-  col = (id - row * NsTileRegs<TS>::GR) * 8;
-}
 
-// One stage's product on this block's tile (bx, by): the copy waves' part ...
-template <class TS, int NT, bool B_KS>
-__device__ __forceinline__ void ns_stage_load(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem) {
+// One stage's product on this block's tile (bx, by): the copy waves' part ...  They wait at the group's barrier in front of the first
+// copy of phase GATE, the matrix waves not at all (what they read comes through the ring): the phases before it run while the
+// partner blocks finish the stage before this one.
+template <class TS, int NT, bool B_KS, int GATE>
+__device__ __forceinline__ void ns_stage_load(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, const GroupBarrier& bar, unsigned* error) {
   DmaPhase<1> ph[NT];
   row_gemm_phases<TS, NT, B_KS>(p, bx * TS::BM, by * TS::BN, z, ph);
   using Pipe = DmaPipe<TS, 1, NT, row_stages<TS>(), true>;
   Pipe pipe(smem, ph);
-  pipe.template load_all<Pipe::loads(1)>();
-  __syncthreads();   // the matrix waves are through with the ring
-  __syncthreads();   // and have staged the tile
+  pipe.template load_all<Pipe::loads(1)>([&](int phase) {
+    if (phase == GATE && (threadIdx.x & 63) == 0) bar.wait(error);
+  });
 }
-// ... and the matrix waves'.  E: bytes per staged element (2: the product as bf16, 4: fp32)
-template <class TS, int NT, bool B_KS, int E>
-__device__ __forceinline__ void ns_stage_mma(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem) {
+// ... and the matrix waves'
+template <class TS, int NT, bool B_KS>
+__device__ __forceinline__ void ns_stage_mma(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, f32x16 (&acc)[1][TS::TM][TS::TN]) {
   DmaPhase<1> ph[NT];
   row_gemm_phases<TS, NT, B_KS>(p, bx * TS::BM, by * TS::BN, z, ph);
   DmaPipe<TS, 1, NT, row_stages<TS>(), true> pipe(smem, ph);
-  f32x16 acc[1][TS::TM][TS::TN];
   zero_acc<TS>(acc[0]);
   int step = 0;
 #pragma unroll
   for (int t = 0; t < NT; ++t) pipe.template run_phase<1, false, B_KS>(p.t[t].K, step, acc);
-  __syncthreads();
-  using ST = StageTile<TS, E>;
+}
+template <class TS>
+__device__ __forceinline__ void ns_put_tile(char* smem, const f32x16 (&acc)[1][TS::TM][TS::TN]) {   // rounded to bf16
+  using ST = StageTile<TS, 2>;
   char* lb = smem + ST::lane_base();
   LACT_FOR_QUADS(TS) ST::put4(lb, tm, tn, g, acc[0][tm][tn][4 * g], acc[0][tm][tn][4 * g + 1], acc[0][tm][tn][4 * g + 2], acc[0][tm][tn][4 * g + 3]);
-  __syncthreads();
 }
+// EPI_STORE: out = round(product), and out2 = round(alpha2 * out) if there is one.  EPI_AXPBY: out = round(round(alpha product) + round(beta aux));
+// the auxiliary tile is asked for in front of the staging.
 template <class TS, int NT, int EPI, bool COPY>
-__device__ __forceinline__ void ns_stage_b16(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem) {
-  if (COPY) ns_stage_load<TS, NT, false>(p, bx, by, z, smem);
-  else ns_stage_mma<TS, NT, false, 2>(p, bx, by, z, smem);
-  row_gemm_copy_out_b16<TS, NT, EPI, COPY ? 3 : 64>(p, bx * TS::BM, by * TS::BN, z, smem);
-}
-// X' = beta X + product (the stage with B K-strided): the staged product blended with the fp32 tile in registers.
-// out_c: bf16 copy, out: fp32 (both [r, c]; nullable); out_t: fp32 in the original orientation, transposed if `tr`
-template <class TS, int NT, bool COPY>
-__device__ __forceinline__ void ns_stage_iterate(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, NsTileRegs<TS>* x, bool tr) {
-  using ST = StageTile<TS, 4>;
-  const int m0 = bx * TS::BM, n0 = by * TS::BN;
-  if constexpr (COPY) {
-    ns_stage_load<TS, NT, true>(p, bx, by, z, smem);
-    const size_t zo = z * p.bso + (size_t)m0 * p.ldo + n0;
+__device__ __forceinline__ void ns_stage_b16(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, const GroupBarrier& bar, unsigned* error) {
+  using G = NsGranules<TS, DMA_THREADS>;
+  using ST = StageTile<TS, 2>;
+  f32x16 acc[1][TS::TM][TS::TN];   // matrix waves only
+  if constexpr (COPY) ns_stage_load<TS, NT, false, 0>(p, bx, by, z, smem, bar, error);
+  else ns_stage_mma<TS, NT, false>(p, bx, by, z, smem, acc);
+  __syncthreads();   // the matrix waves are through with the ring
+  const int r0 = G::row0(), c0 = G::col0();
+  const size_t o0 = z * p.bso + (size_t)(bx * TS::BM + r0) * p.ldo + by * TS::BN + c0;
+  uint4 w[G::N];
+  if constexpr (EPI == EPI_AXPBY) {
 #pragma unroll
-    for (int t = 0; t < NsTileRegs<TS>::N; ++t) {
-      int row, col;
-      ns_granule<TS>(t, row, col);
-      float4* src = reinterpret_cast<float4*>(smem + (row * ST::LD + col) * 4);
-      const float4 a = src[0], b = src[1];
-      const float in[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
-      float (&v)[8] = x->v[t];
-      // the matrix product is a bf16 tensor in the reference (ttt_operation.py:62)
+    for (int t = 0; t < G::N; ++t) w[t] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.aux) + o0 + (size_t)G::row(t) * p.ldo + G::col(t));
+  }
+  if constexpr (!COPY) ns_put_tile<TS>(smem, acc);
+  __syncthreads();
+  const char* src = smem + (r0 * ST::LD + c0) * 2;
+  constexpr int LG = COPY ? 3 : G::N;   // LDS reads in flight together: the copy waves are short of registers
+  uint4 u[LG];
 #pragma unroll
-      for (int i = 0; i < 8; ++i) v[i] = dual_blend(__fmul_rn(p.alpha, round_bf16(in[i])), __fmul_rn(p.beta, v[i]), p.round_out_bf16);
-      const size_t o = zo + (size_t)row * p.ldo + col;
-      if (p.out_c) *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.out_c) + o) = pack8(v);
-      if (p.out) {
-        float* f = reinterpret_cast<float*>(p.out) + o;
-        *reinterpret_cast<float4*>(f) = make_float4(v[0], v[1], v[2], v[3]);
-        *reinterpret_cast<float4*>(f + 4) = make_float4(v[4], v[5], v[6], v[7]);
-      }
-      if (p.out_t && !tr) {
-        *reinterpret_cast<float4*>(p.out_t + o) = make_float4(v[0], v[1], v[2], v[3]);
-        *reinterpret_cast<float4*>(p.out_t + o + 4) = make_float4(v[4], v[5], v[6], v[7]);
-      }
-      if (p.out_t && tr) {
-        src[0] = make_float4(v[0], v[1], v[2], v[3]);
-        src[1] = make_float4(v[4], v[5], v[6], v[7]);
+  for (int t = 0; t < G::N; ++t) {
+    if (t % LG == 0) {
+      if (COPY) asm volatile("" ::: "memory");
+#pragma unroll
+      for (int g = 0; g < LG; ++g)
+        if (t + g < G::N) u[g] = *reinterpret_cast<const uint4*>(src + (G::row(t + g) * ST::LD + G::col(t + g)) * 2);
+    }
+    const size_t o = o0 + (size_t)G::row(t) * p.ldo + G::col(t);
+    uint32_t uu[4] = {u[t % LG].x, u[t % LG].y, u[t % LG].z, u[t % LG].w};
+    if constexpr (EPI == EPI_AXPBY) {
+      const uint32_t ww[4] = {w[t].x, w[t].y, w[t].z, w[t].w};
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        float alo = NT == 1 ? bf16_lo(uu[j]) : p.alpha * bf16_lo(uu[j]), ahi = NT == 1 ? bf16_hi(uu[j]) : p.alpha * bf16_hi(uu[j]);   // one term: alpha is 1
+        if (NT > 1) round_both(alo, ahi);
+        float blo = p.beta * bf16_lo(ww[j]), bhi = p.beta * bf16_hi(ww[j]);
+        round_both(blo, bhi);
+        uu[j] = pack_bf16(alo + blo, ahi + bhi);
       }
     }
-  } else {
-    ns_stage_mma<TS, NT, true, 4>(p, bx, by, z, smem);
+    *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.out) + o) = make_uint4(uu[0], uu[1], uu[2], uu[3]);
+    if (EPI == EPI_STORE && NT == 1) {
+#pragma unroll
+      for (int j = 0; j < 4; ++j) uu[j] = pack_bf16(p.alpha2 * bf16_lo(uu[j]), p.alpha2 * bf16_hi(uu[j]));
+      *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(p.out2) + o) = make_uint4(uu[0], uu[1], uu[2], uu[3]);
+    }
   }
-  if (p.out_t && tr) {
+}
+
+// The stage that makes the next iterate, X' = beta X + product (B K-strided): the staged product, a bf16 tensor in the reference
+// (ttt_operation.py:62), blended with the fp32 tile in the copy waves' registers.  out_c: bf16 copy; of the last one instead out_t: fp32
+// ([r, c]; transposed, [c, r], if `tr`).  PLAIN: X' is a bf16 tensor; decided inside the loop it costs as much as the blend (5.7 us a
+// tile of 192 x 192).
+template <class TS, int NT, bool COPY, int GATE, bool PLAIN>
+__device__ __forceinline__ void ns_stage_iterate(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, NsTileRegs<TS>* x, bool tr, const GroupBarrier& bar, unsigned* error) {
+  using G = NsGranules<TS, 256>;
+  const int m0 = bx * TS::BM, n0 = by * TS::BN;
+  if constexpr (COPY) {
+    using ST = StageTile<TS, 2>;
+    ns_stage_load<TS, NT, true, GATE>(p, bx, by, z, smem, bar, error);
+    __syncthreads();   // the matrix waves are through with the ring
+    __syncthreads();   // and have staged the tile
+    const char* src = smem + (G::row0() * ST::LD + G::col0()) * 2;
+    const size_t o = z * p.bso + (size_t)(m0 + G::row0()) * p.ldo + n0 + G::col0();
+    uint16_t* oc = reinterpret_cast<uint16_t*>(p.out_c) + o;
+#pragma unroll
+    for (int t = 0; t < G::N; ++t) {
+      if (t % 3 == 0) asm volatile("" ::: "memory");   // three granules' reads at a time: more of them do not fit beside the tile
+      float in[8];
+      unpack8(*reinterpret_cast<const uint4*>(src + (G::row(t) * ST::LD + G::col(t)) * 2), in);
+      float (&v)[8] = x->v[t];
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = dual_blend(in[i], __fmul_rn(p.beta, v[i]), PLAIN);
+      if (p.out_c) *reinterpret_cast<uint4*>(oc + (size_t)G::row(t) * p.ldo + G::col(t)) = pack8(v);
+    }
+  } else {
+    f32x16 acc[1][TS::TM][TS::TN];
+    ns_stage_mma<TS, NT, true>(p, bx, by, z, smem, acc);
+    __syncthreads();
+    ns_put_tile<TS>(smem, acc);
+    __syncthreads();
+  }
+  if (!p.out_t) return;
+  const bool turn = NT == 1 && tr;
+  if (turn) __syncthreads();   // the staged product has been read
+  if constexpr (COPY) {
+    using ST = StageTile<TS, 4>;
+    float* dst = turn ? reinterpret_cast<float*>(smem) + G::row0() * ST::LD + G::col0()
+                      : p.out_t + z * p.bso + (size_t)(m0 + G::row0()) * p.ldo + n0 + G::col0();
+    const int ld = turn ? ST::LD : p.ldo;
+#pragma unroll
+    for (int t = 0; t < G::N; ++t) {
+      const float (&v)[8] = x->v[t];
+      float4* f = reinterpret_cast<float4*>(dst + (size_t)G::row(t) * ld + G::col(t));
+      f[0] = make_float4(v[0], v[1], v[2], v[3]);
+      f[1] = make_float4(v[4], v[5], v[6], v[7]);
+    }
+  }
+  if (NT == 1 && turn) {
     __syncthreads();
     row_gemm_copy_out_transposed<TS, NT>(p, nullptr, true, m0, n0, z, smem);
   }
+}
+
+__device__ __forceinline__ void ns_load8(const float* src, float (&v)[8]) {
+  const float4 lo = reinterpret_cast<const float4*>(src)[0], hi = reinterpret_cast<const float4*>(src)[1];
+  v[0] = lo.x; v[1] = lo.y; v[2] = lo.z; v[3] = lo.w; v[4] = hi.x; v[5] = hi.y; v[6] = hi.z; v[7] = hi.w;
 }
 
 // This block's place in its matrix
@@ -275,22 +358,25 @@ struct NsPlace {
 };
 // BWD = false: S iterations  A = X X^T;  B = b A + c A A;  X' = a X + B X
 // BWD = true:  the same iterations backwards:  Sg = G X^T + X G^T;  H = b Sg + c (Sg A + A Sg);  G' = a G + B G + H X
-// COPY: on the copy waves, else on the matrix waves.
-template <class TS, bool BWD, bool COPY>
+// COPY: on the copy waves, else on the matrix waves.  PLAIN: the iterate is a bf16 tensor (reference without autocast).
+template <class TS, bool BWD, bool COPY, bool PLAIN = false>
 __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarrier& bar, const NsPlace& b, char* smem) {
   const int z = b.z;
   NsTileRegs<TS> x;
   if constexpr (COPY) {
-    const float* src = (BWD ? p.gxf[0] : p.xf[0]) + (size_t)z * p.r * p.c + (size_t)b.rx * TS::BM * p.c + b.ry * TS::BN;
+    using G = NsGranules<TS, 256>;
+    if (!BWD && p.g16) {          // staged in LDS by the normalisation
+      using ST = StageTile<TS, 4>;
+      const char* src = smem + (G::row0() * ST::LD + G::col0()) * 4;
 #pragma unroll
-    for (int t = 0; t < NsTileRegs<TS>::N; ++t) {
-      int row, col;
-      ns_granule<TS>(t, row, col);
-      const float4 lo = *reinterpret_cast<const float4*>(src + (size_t)row * p.c + col), hi = *reinterpret_cast<const float4*>(src + (size_t)row * p.c + col + 4);
-      x.v[t][0] = lo.x; x.v[t][1] = lo.y; x.v[t][2] = lo.z; x.v[t][3] = lo.w;
-      x.v[t][4] = hi.x; x.v[t][5] = hi.y; x.v[t][6] = hi.z; x.v[t][7] = hi.w;
+      for (int t = 0; t < G::N; ++t) ns_load8(reinterpret_cast<const float*>(src) + G::row(t) * ST::LD + G::col(t), x.v[t]);
+    } else {
+      const float* src = (BWD ? p.gxf[0] : p.xf[0]) + (size_t)z * p.r * p.c + (size_t)(b.rx * TS::BM + G::row0()) * p.c + b.ry * TS::BN + G::col0();
+#pragma unroll
+      for (int t = 0; t < G::N; ++t) ns_load8(src + (size_t)G::row(t) * p.c + G::col(t), x.v[t]);
     }
   }
+  if (!BWD) __syncthreads();      // the staging area becomes the ring
   const bool tr = (p.mask >> (z / p.nb)) & 1;
   for (int step = 0; step < p.S; ++step) {
     const int it = BWD ? p.S - 1 - step : step;
@@ -310,28 +396,27 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
         ns_term(q.g.t[0], X, c, xe, X, c, xe, c);
         q.g.M = r; q.g.N = r; q.g.out = A; q.g.ldo = r; q.g.bso = se;
         q.g.out2 = p.cab; q.g.alpha2 = cc;
-        ns_stage_b16<TS, 1, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem);
-      }
-      bar.sync(p.error);
+        ns_stage_b16<TS, 1, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+      } else bar.pass(p.error);
+      bar.arrive();
       if (b.sq_tile) {
         auto q = ns_row_params<1>();
         ns_term(q.g.t[0], p.cab, r, se, A, r, se, r);
         q.g.M = r; q.g.N = r; q.g.out = B; q.g.ldo = r; q.g.bso = se;
         q.g.aux = A; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = 1.f; q.g.beta = cb;
-        ns_stage_b16<TS, 1, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem);
-      }
-      bar.sync(p.error);
+        ns_stage_b16<TS, 1, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+      } else bar.pass(p.error);
+      bar.arrive();
       {
         auto q = ns_row_params<1>();
         ns_term(q.g.t[0], B, r, se, X, c, xe, r);
         q.g.M = r; q.g.N = c; q.g.ldo = c; q.g.bso = xe;
-        q.g.alpha = 1.f; q.g.beta = ca; q.g.round_out_bf16 = p.plain;
-        q.g.out = nullptr;
+        q.g.alpha = 1.f; q.g.beta = ca;
         q.g.out_c = last ? nullptr : p.xb + (it + 1) * p.xb_it_stride;   // nothing multiplies by the last iterate
         q.g.out_t = last ? p.u_out : nullptr;
-        ns_stage_iterate<TS, 1, COPY>(q.g, b.rx, b.ry, z, smem, &x, tr);
+        ns_stage_iterate<TS, 1, COPY, 0, PLAIN>(q.g, b.rx, b.ry, z, smem, &x, tr, bar, p.error);
       }
-      bar.sync(p.error);
+      if (!last) bar.arrive();
     } else {
       const int cur = step & 1;
       const uint16_t* gb = p.gxb[cur];
@@ -340,29 +425,29 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
         ns_term(q.g.t[0], gb, c, xe, X, c, xe, c);
         ns_term(q.g.t[1], X, c, xe, gb, c, xe, c);
         q.g.M = r; q.g.N = r; q.g.out = p.sg; q.g.ldo = r; q.g.bso = se;
-        ns_stage_b16<TS, 2, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem);
-      }
-      bar.sync(p.error);
+        ns_stage_b16<TS, 2, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+      } else bar.pass(p.error);
+      bar.arrive();
       if (b.sq_tile) {   // H = b Sg + c (Sg A + A Sg)
         auto q = ns_row_params<2>();
         ns_term(q.g.t[0], p.sg, r, se, A, r, se, r);
         ns_term(q.g.t[1], A, r, se, p.sg, r, se, r);
         q.g.M = r; q.g.N = r; q.g.out = p.gas; q.g.ldo = r; q.g.bso = se;
         q.g.aux = p.sg; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = cc; q.g.beta = cb;
-        ns_stage_b16<TS, 2, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem);
-      }
-      bar.sync(p.error);
+        ns_stage_b16<TS, 2, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+      } else bar.pass(p.error);
+      bar.arrive();
       {                  // G' = a G + B G + H X
         auto q = ns_row_params<2>();
         ns_term(q.g.t[0], B, r, se, gb, c, xe, r);
         ns_term(q.g.t[1], p.gas, r, se, X, c, xe, r);
         q.g.M = r; q.g.N = c; q.g.ldo = c; q.g.bso = xe;
         q.g.alpha = 1.f; q.g.beta = ca;
-        q.g.out = last ? p.gxf[p.S & 1] : nullptr;
+        q.g.out_t = last ? p.gxf[p.S & 1] : nullptr;
         q.g.out_c = last ? nullptr : p.gxb[cur ^ 1];   // nothing multiplies by the final gradient
-        ns_stage_iterate<TS, 2, COPY>(q.g, b.rx, b.ry, z, smem, &x, false);
+        ns_stage_iterate<TS, 2, COPY, 1, false>(q.g, b.rx, b.ry, z, smem, &x, false, bar, p.error);   // B G needs nothing that this stage's barrier waits for
       }
-      bar.sync(p.error);
+      if (!last) bar.arrive();
     }
   }
 }
@@ -386,8 +471,9 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p)
 
   if (!BWD && p.g16) {
     // Frobenius normalisation in front of the first iteration: every block of the group sums the same partials
-    // in the same order, then scales its own tile of [r, c]
+    // in the same order, then scales its own tile of [r, c], for its copy waves in LDS and in bf16 for its partners
     float ss = 0.f;
+#pragma unroll 4
     for (int i = 0; i < p.nparts; ++i) ss += p.ss_part[(size_t)(p.part0 + z) * p.nparts + i];
     if (p.part1 >= 0)
       for (int i = 0; i < p.nparts; ++i) ss += p.ss_part[(size_t)(p.part1 + z) * p.nparts + i];
@@ -396,32 +482,38 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p)
     if (member == 0 && threadIdx.x == 0) p.norms[z] = n;
     float den = n + 1e-7f;
     if (p.plain) den = round_bf16(den);
-    const size_t zo = (size_t)z * p.r * p.c + (size_t)rx * TS::BM * p.c + ry * TS::BN;
-    constexpr int GR = TS::BN / 8;   // 16-byte granules per tile row
-    for (int id = threadIdx.x; id < TS::BM * GR; id += DMA_THREADS) {
-      const size_t o = zo + (size_t)(id / GR) * p.c + (id % GR) * 8;
-      const uint4 u = *reinterpret_cast<const uint4*>(p.g16 + o);
-      const uint32_t w[4] = {u.x, u.y, u.z, u.w};
-      float v[8];
+    using G = NsGranules<TS, DMA_THREADS>;
+    using ST = StageTile<TS, 4>;
+    const size_t o = (size_t)z * p.r * p.c + (size_t)(rx * TS::BM + G::row0()) * p.c + ry * TS::BN + G::col0();
+    float* stage = reinterpret_cast<float*>(smem) + G::row0() * ST::LD + G::col0();
+    uint4 u[G::N];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        v[2 * i] = __fdiv_rn(__uint_as_float(w[i] << 16), den);            // the quotient itself (ttt_operation.py:49), not a product with 1 / den
-        v[2 * i + 1] = __fdiv_rn(__uint_as_float(w[i] & 0xffff0000u), den);
-      }
+    for (int t = 0; t < G::N; ++t) u[t] = *reinterpret_cast<const uint4*>(p.g16 + o + (size_t)G::row(t) * p.c + G::col(t));
+#pragma unroll
+    for (int t = 0; t < G::N; ++t) {
+      float v[8];
+      unpack8(u[t], v);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) v[i] = __fdiv_rn(v[i], den);   // the quotient itself (ttt_operation.py:49), not a product with 1 / den
       if (p.plain) {
 #pragma unroll
         for (int i = 0; i < 8; ++i) v[i] = round_bf16(v[i]);
       }
-      *reinterpret_cast<float4*>(p.xf[0] + o) = make_float4(v[0], v[1], v[2], v[3]);
-      *reinterpret_cast<float4*>(p.xf[0] + o + 4) = make_float4(v[4], v[5], v[6], v[7]);
-      Elem<uint16_t>::store4(p.xb + o, v[0], v[1], v[2], v[3]);
-      Elem<uint16_t>::store4(p.xb + o + 4, v[4], v[5], v[6], v[7]);
+      float4* f = reinterpret_cast<float4*>(stage + G::row(t) * ST::LD + G::col(t));   // for the copy waves, which keep the fp32 tile
+      f[0] = make_float4(v[0], v[1], v[2], v[3]);
+      f[1] = make_float4(v[4], v[5], v[6], v[7]);
+      *reinterpret_cast<uint4*>(p.xb + o + (size_t)G::row(t) * p.c + G::col(t)) = pack8(v);
     }
-    bar.sync(p.error);
+    bar.arrive();
   }
   const NsPlace place{z, sq_tile, sx, sy, rx, ry};
-  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4) ns_iterations<TS, BWD, true>(p, bar, place, smem);
+  if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4) {
+    if (!BWD && p.plain) ns_iterations<TS, BWD, true, !BWD>(p, bar, place, smem);
+    else ns_iterations<TS, BWD, true>(p, bar, place, smem);
+  }
   else ns_iterations<TS, BWD, false>(p, bar, place, smem);
+  wait_vmcnt<0>();   // the last stage's stores, for the other waves of this block
+  __syncthreads();
   if (BWD && p.dot_part) {
     // the tile this block wrote in the last stage, and the same tile of the bf16 input: 12 granules of 8 elements
     // per thread at 192 x 192, kept in registers for the second pass

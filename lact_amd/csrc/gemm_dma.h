@@ -170,7 +170,8 @@ __device__ __forceinline__ bf16x8 dma_fetch(const char* tile, int row, int kvec)
 // front makes that a single one: the token reduction's copy waves start 0.7 us after the block instead of 2.1 us (with the
 // divisions gone and the offsets of the copies computed without 64-bit products), the hidden stage's 0.6 instead of 1.1 us.
 #define LACT_TOUCH(o) "s_load_dword %0, %1, " #o "*64\n\t"
-#define LACT_TOUCH4 LACT_TOUCH(0) LACT_TOUCH(1) LACT_TOUCH(2) LACT_TOUCH(3)
+#define LACT_TOUCH3 LACT_TOUCH(0) LACT_TOUCH(1) LACT_TOUCH(2)
+#define LACT_TOUCH4 LACT_TOUCH3 LACT_TOUCH(3)
 #define LACT_TOUCH8 LACT_TOUCH4 LACT_TOUCH(4) LACT_TOUCH(5) LACT_TOUCH(6) LACT_TOUCH(7)
 #define LACT_TOUCH12 LACT_TOUCH8 LACT_TOUCH(8) LACT_TOUCH(9) LACT_TOUCH(10) LACT_TOUCH(11)
 #define LACT_TOUCH16 LACT_TOUCH12 LACT_TOUCH(12) LACT_TOUCH(13) LACT_TOUCH(14) LACT_TOUCH(15)
@@ -181,8 +182,9 @@ __device__ __forceinline__ void prefetch_args() {
   const uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
   constexpr int N = (BYTES + 63) / 64;
   int unused;
-  static_assert(N >= 4, "too few lines to be worth it");
-  if constexpr (N == 4) LACT_TOUCH_ARGS(LACT_TOUCH4);
+  static_assert(N >= 3, "too few lines to be worth it");
+  if constexpr (N == 3) LACT_TOUCH_ARGS(LACT_TOUCH3);
+  else if constexpr (N == 4) LACT_TOUCH_ARGS(LACT_TOUCH4);
   else if constexpr (N == 5) LACT_TOUCH_ARGS(LACT_TOUCH4 LACT_TOUCH(4));
   else if constexpr (N == 6) LACT_TOUCH_ARGS(LACT_TOUCH4 LACT_TOUCH(4) LACT_TOUCH(5));
   else if constexpr (N == 7) LACT_TOUCH_ARGS(LACT_TOUCH4 LACT_TOUCH(4) LACT_TOUCH(5) LACT_TOUCH(6));

@@ -2150,8 +2150,8 @@ int attn_rows(const void* ptr, int ld, long long bs, int H, int D, const uint16_
 // Waves per block: 8 (256 rows, two waves per SIMD) once that gives every compute unit a block, else 4.
 template <int D, int NW>
 void launch_window_attn(int which, WindowAttnParams p, hipStream_t s) {
-  p.map = make_tile_map(ceil_div(p.L, 32 * NW), 1, p.B * p.H);
-  const dim3 grid(p.map.grid()), block(64 * NW);
+  p.by_heads = make_udiv(p.B * p.H);
+  const dim3 grid(ceil_div(p.L, 32 * NW) * p.B * p.H), block(64 * NW);
   constexpr int SM = attn_lds_bytes<D, NW>(false), SMS = attn_lds_bytes<D, NW>(true);
   LACT_BIG_LDS((k_window_attn_fwd<D, NW>), SM);
   LACT_BIG_LDS((k_window_attn_dq<D, NW>), SM);

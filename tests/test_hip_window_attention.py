@@ -29,6 +29,34 @@ def test_window_attention_against_oracle(b, l, h, d, window):
         assert rel_l2(a, r) < 1e-2, i
 
 
+@pytest.mark.parametrize("b,l,h,d,window,growth", [
+    (1, 70, 2, 128, 1, 1.0),        # every query sees itself alone
+    (2, 300, 64, 64, 64, 1.0),      # 256-row blocks of heads of 64, the window one tile
+    (1, 515, 3, 128, 190, 40.0),    # scores that grow along the sequence: the rows' maxima follow them from tile to tile
+    (2, 600, 70, 128, 600, 300.0)])
+def test_window_attention_scores_and_window_edges(b, l, h, d, window, growth):
+    """The scores of a tile are formed one step ahead of their exponentials: window edges inside and on the tiles, and maxima that grow
+    from tile to tile by far more than exp2 reaches.  Grown scores leave a handful of probabilities per row, which bf16 rounds to 2^-9
+    each and the kernel's output once more; gradients pass through their differences: twice the bounds of the test above."""
+    print("[gpu-test] window attention edges", b, l, h, d, window, growth, flush=True)
+    from lact_amd import layers as HL
+    g = torch.Generator().manual_seed(8)
+    q, k, v, go = [torch.randn(b, l, h, d, generator=g) for _ in range(4)]
+    k = k * torch.linspace(1.0, growth, l).view(1, l, 1, 1)
+    q, k, v, go = [t.bfloat16() for t in (q, k, v, go)]
+    dev = [t.to("cuda").requires_grad_(True) for t in (q, k, v)]
+    out = HL.sliding_window_attention(*dev, window)
+    grads = torch.autograd.grad(out, dev, go.to("cuda"))
+    ref_in = [t.double().requires_grad_(True) for t in (q, k, v)]
+    ref = LO.sliding_window_attention(*ref_in, window)
+    ref_grads = torch.autograd.grad(ref, ref_in, go.double())
+    assert rel_l2(out, ref) < 1e-2
+    for i, (a, r) in enumerate(zip(grads, ref_grads)):
+        assert bool(torch.isfinite(a).all()), i
+        if float(r.norm()) > 1e-6 * float(go.double().norm()):      # one visible key: the probabilities are constant
+            assert rel_l2(a, r) < 2e-2, i
+
+
 @pytest.mark.parametrize("dtype,B,L,H,hd", [(torch.float32, 2, 37, 3, 16), (torch.float32, 1, 5, 2, 520), (torch.bfloat16, 1, 4099, 2, 384)])
 def test_pre_attention_kernel_against_torch(dtype, B, L, H, hd):
     """The layer's pre-processing with the attention's inputs: outputs, and the gradients of the projection and of the rescaling."""

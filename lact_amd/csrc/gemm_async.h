@@ -20,11 +20,24 @@ namespace lact {
 
 // 64 x 64 tiles: measured at eight fp32 heads of 128, 512 tokens, against the register-staged loop on 128 x 128 tiles: apply
 // hidden stage 35 -> 11 us, update 48 -> 17, update backward 53 -> 32, four-term row GEMM 72 -> 19, token reduction 55 + 5 (its
-// partial sums) -> 17.
-template <typename T> struct AsyncTile {
-  using TS = TileShape<64, 64, 2, 2>;
+// partial sums) -> 17.  With one A tile for the B operands that share it and one small piece of code for the copies of all contractions,
+// instead of a fully unrolled one for each, whose instructions a launch waited for: update backward 31 -> 24.5, apply hidden 14 -> 9.
+// HALF, for launches whose 64 x 64 tiles leave compute units without a block: 64 x 32 tiles, two waves to each 32 x 32 of
+// them, which take half of the k of every K-step each and add their halves of the sums at the end: twice the blocks, half the serial chain of matrix instructions in each (update backward 24.5 ->
+// 18.9 us, apply hidden 9.0 -> 7.4).
+template <typename T, bool HALF = false> struct AsyncTile {
+  static_assert(!HALF || sizeof(T) == 4, "half tiles: fp32");
+  using TS = TileShape<64, HALF ? 32 : 64, 2, HALF ? 1 : 2>;
+  static constexpr int KG = HALF ? 2 : 1, NQ = 4 / KG;     // waves to a 32 x 32 tile; quads of its columns that one of them ends up with
+  static constexpr int THREADS = TS::THREADS * KG;
   static constexpr int STAGES = sizeof(T) == 4 ? 4 : 3;
   static constexpr int GROUP = sizeof(T) == 4 ? 8 : 16;    // k of one group of matrix instructions
+  static_assert(TS::TM == 1 && TS::TN == 1 && THREADS == 256, "a wave owns one 32 x 32 tile, or half the k of one");
+  __device__ static __forceinline__ int place() { return (threadIdx.x >> 6) % (TS::WAVES_M * TS::WAVES_N); }   // of the wave's 32 x 32 tile
+  __device__ static __forceinline__ int kgroup() { return KG == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) / (TS::WAVES_M * TS::WAVES_N); }
+  // rows and columns of the accumulators inside the block's tile, as quad_m and quad_n; quad g < NQ is in entries 4g .. 4g + 3
+  __device__ static __forceinline__ int m() { return place() / TS::WAVES_N * 32 + (threadIdx.x & 31); }
+  __device__ static __forceinline__ int n(int g) { return place() % TS::WAVES_N * 32 + 8 * (g + NQ * kgroup()) + 4 * ((threadIdx.x & 63) >> 5); }
 };
 
 template <typename T>
@@ -87,65 +100,92 @@ template <> struct AsyncFrag<uint16_t> {
   __device__ static __forceinline__ int rotation(int k) { return G >= 16 ? 4 * (k & 3) : 4 * ((k >> 1) & 1); }
 };
 
-template <typename T, int NPH>
-struct AsyncPipe {
-  using TS = typename AsyncTile<T>::TS;
-  static constexpr int STAGES = AsyncTile<T>::STAGES, GROUP = AsyncTile<T>::GROUP;
-  static constexpr int EPG = 16 / sizeof(T), BK = 8 * EPG, WAVES = TS::THREADS / 64;
-  static constexpr int A_BYTES = TS::BM * 128, B_BYTES = TS::BN * 128, STAGE = A_BYTES + B_BYTES, BYTES = STAGE * STAGES;
-  static constexpr int NA = TS::BM / 8 / WAVES, NB = TS::BN / 8 / WAVES, COPIES = NA + NB;   // per wave and stage
+// NB: B operands that share the A tile of a stage, up to.  PHASES: contractions one after the other; set(i) (the constructor's argument) calls
+// phase() with the operands of contraction i when its copies begin, so that only these are held.
+template <typename T, int NB, bool HALF = false>
+struct AsyncRing {
+  using AT = AsyncTile<T, HALF>;
+  using TS = typename AT::TS;
+  static constexpr int EPG = 16 / sizeof(T), BK = 8 * EPG, WAVES = AT::THREADS / 64;
+  static constexpr int A_BYTES = TS::BM * 128, B_BYTES = TS::BN * 128, STAGE = A_BYTES + NB * B_BYTES;
+  // two blocks to a compute unit: with a third stage of four whole B tiles (120 KiB, one block) launches of 512 blocks and more were slower
+  static constexpr int STAGES = NB > 2 && !HALF ? 2 : NB > 1 ? 3 : AT::STAGES, BYTES = STAGE * STAGES;
+  static constexpr int NA = TS::BM / 8 / WAVES, NBC = TS::BN / 8 / WAVES, COPIES = NA + NBC;   // per wave and stage, with one B operand
   static_assert(TS::BM / 8 % WAVES == 0 && TS::BN / 8 % WAVES == 0, "copies must split evenly over the waves");
+  static_assert(BYTES <= 160 * 1024, "ring does not fit the 160 KiB LDS");
+};
+template <typename T, int NB, int PHASES, bool HALF, class SET>
+struct AsyncPipe : AsyncRing<T, NB, HALF> {
+  using R = AsyncRing<T, NB, HALF>;
+  using AT = typename R::AT;
+  using TS = typename R::TS;
+  using R::EPG; using R::BK; using R::WAVES; using R::A_BYTES; using R::B_BYTES; using R::STAGE; using R::STAGES; using R::NA; using R::NBC; using R::COPIES;
+  static constexpr int GROUP = AT::GROUP, KG = AT::KG;
 
   char* smem;
-  AsyncOperand<T> a[NPH], b[NPH];
-  int K[NPH];
-  int total = 0, issued = 0, used = 0, cp = 0, ckt = 0;
+  SET set;
+  int total, issued = 0, used = 0;
+  // the contraction that is being copied: operands at the next K-step, elements from one to the next, k left
+  int cp = 0, cnb = 0, cleft = 0;
+  AsyncOperand<T> a, b;
+  const T* bs[NB];
+  size_t astep = 0, bstep = 0;
+  uint32_t va[NA], vb[NBC];   // this lane's offsets inside a K-step (the B operands' are alike)
 
-  __device__ __forceinline__ AsyncPipe(char* s) : smem(s) {}
-  __device__ __forceinline__ void phase(int i, const T* A, int lda, int a_rows, bool a_ks, const T* B, int ldb, int b_rows, bool b_ks, int k) {
-    a[i] = AsyncOperand<T>{A, lda, a_rows, a_ks};
-    b[i] = AsyncOperand<T>{B, ldb, b_rows, b_ks};
-    K[i] = k;
-    total += (k + BK - 1) / BK;
+  // steps: K-steps of all contractions
+  __device__ __forceinline__ AsyncPipe(char* s, int steps, SET f) : smem(s), set(f), total(steps) {
+    set(*this, 0);
+    for (int i = 0; i < STAGES - 1 && issued < total; ++i) issue();
+  }
+  __host__ __device__ static constexpr int steps(int k) { return (k + BK - 1) / BK; }
+  __device__ __forceinline__ void phase(int k, const T* A, int lda, int a_rows, bool a_ks, int ldb, int b_rows, bool b_ks, int nb) {
+    a = AsyncOperand<T>{A, lda, a_rows, a_ks};
+    b = AsyncOperand<T>{nullptr, ldb, b_rows, b_ks};
+    astep = a_ks ? (size_t)BK * lda : (size_t)BK;
+    bstep = b_ks ? (size_t)BK * ldb : (size_t)BK;
+    cnb = nb; cleft = k;
+    offsets<TS::BM, NA>(a, va);
+    offsets<TS::BN, NBC>(b, vb);
   }
   // Rows and k past the operand repeat its last ones: they reach only output rows that are never stored, or are left
   // out of the sum by accumulate().
   template <int ROWS, int N>
-  __device__ __forceinline__ void copy(const AsyncOperand<T>& op, int k0, int k_end, uint32_t lds) const {
+  __device__ __forceinline__ void offsets(const AsyncOperand<T>& op, uint32_t (&off)[N]) const {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
 #pragma unroll
     for (int i = 0; i < N; ++i) {
       const int n = (wave + i * WAVES) * 64 + lane;      // granule of the tile
-      uint32_t off;
       if (op.ks) {
         constexpr int G = ROWS / EPG;
         const int k = n / G, rot = sizeof(T) == 2 ? AsyncFrag<uint16_t>::rotation<G>(k) : 0, g = (n % G + G - rot) % G;
-        off = (uint32_t)(min(k, k_end - 1 - k0) * op.ld + min(g * EPG, op.rows - EPG)) * (uint32_t)sizeof(T);
+        off[i] = (uint32_t)(min(k, cleft - 1) * op.ld + min(g * EPG, op.rows - EPG)) * (uint32_t)sizeof(T);
       } else {
         const int row = n / 8, j = (n % 8) ^ ((row >> 1) & 7);
-        off = (uint32_t)(min(row, op.rows - 1) * op.ld + min(j * EPG, k_end - EPG - k0)) * (uint32_t)sizeof(T);
+        off[i] = (uint32_t)(min(row, op.rows - 1) * op.ld + min(j * EPG, cleft - EPG)) * (uint32_t)sizeof(T);
       }
-      dma16<false>(op.base + (op.ks ? (size_t)k0 * op.ld : (size_t)k0), off, lds + (wave + i * WAVES) * 1024);
     }
   }
   __device__ __forceinline__ void issue() {
-    const uint32_t lds = lds_addr(smem + (issued % STAGES) * STAGE);
-    int k = 0;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lds = lds_addr(smem + (issued % STAGES) * STAGE) + wave * 1024;
 #pragma unroll
-    for (int i = 0; i < NPH; ++i)
-      if (i == cp) {
-        copy<TS::BM, NA>(a[i], ckt * BK, K[i], lds);
-        copy<TS::BN, NB>(b[i], ckt * BK, K[i], lds + A_BYTES);
-        k = K[i];
+    for (int i = 0; i < NA; ++i) dma16<false>(uniform(a.base), va[i], lds + i * WAVES * 1024);
+#pragma unroll
+    for (int j = 0; j < NB; ++j)
+      if (j < cnb) {
+#pragma unroll
+        for (int i = 0; i < NBC; ++i) dma16<false>(uniform(bs[j]), vb[i], lds + A_BYTES + j * B_BYTES + i * WAVES * 1024);
+        bs[j] += bstep;
       }
-    if (++ckt * BK >= k) {
-      ckt = 0;
-      ++cp;
-    }
+    a.base += astep;
     ++issued;
-  }
-  __device__ __forceinline__ void start() {
-    for (int i = 0; i < STAGES - 1 && issued < total; ++i) issue();
+    cleft -= BK;
+    if (cleft <= 0) {
+      if (++cp < PHASES) set(*this, PHASES == 2 ? 1 : cp);   // a constant where it can be: a choice between operands keeps them all in memory
+    } else if (cleft < BK) {      // a last K-step that K does not fill
+      offsets<TS::BM, NA>(a, va);
+      offsets<TS::BN, NBC>(b, vb);
+    }
   }
   __device__ static __forceinline__ void mma(f32x16& acc, const AsyncFrag<float>& fb, const AsyncFrag<float>& fa) {
 #pragma unroll
@@ -154,46 +194,82 @@ struct AsyncPipe {
   __device__ static __forceinline__ void mma(f32x16& acc, const AsyncFrag<uint16_t>& fb, const AsyncFrag<uint16_t>& fa) {
     acc = mma32(fb.v, fa.v, acc);
   }
-  // Phase i into acc; the phases run in their order, each once.
-  template <bool A_KS, bool B_KS>
-  __device__ __forceinline__ void accumulate(int i, f32x16 (&acc)[TS::TM][TS::TN]) {
-    const int wave = threadIdx.x >> 6;
-    const int wm0 = (wave / TS::WAVES_N) * TS::WM, wn0 = (wave % TS::WAVES_N) * TS::WN;
-    auto group = [&](const char* st, int g, int left) {
-      AsyncFrag<T> fa[TS::TM], fb[TS::TN];
+  // The next contraction, over k, its B operands into one accumulator each.
+  template <bool A_KS, bool B_KS, class... ACC>
+  __device__ __forceinline__ void accumulate(int k, ACC&... acc) {
+    static_assert(sizeof...(ACC) <= NB, "as many B operands as the stages hold");
+    constexpr int GROUPS = BK / GROUP / KG;       // of a K-step that are this wave's, from first on
+    const int place = AT::place(), wm0 = (place / TS::WAVES_N) * TS::WM, wn0 = (place % TS::WAVES_N) * TS::WN, first = AT::kgroup() * GROUPS;
+    auto group = [&](const char* st, int g, int left) LACT_INLINE_LAMBDA {
+      AsyncFrag<T> fa, fb[sizeof...(ACC)];
+      fa.template fetch<TS::BM, A_KS>(st, wm0, g);
 #pragma unroll
-      for (int m = 0; m < TS::TM; ++m) fa[m].template fetch<TS::BM, A_KS>(st, wm0 + m * 32, g);
-#pragma unroll
-      for (int n = 0; n < TS::TN; ++n) fb[n].template fetch<TS::BN, B_KS>(st + A_BYTES, wn0 + n * 32, g);
+      for (int j = 0; j < (int)sizeof...(ACC); ++j) fb[j].template fetch<TS::BN, B_KS>(st + A_BYTES + j * B_BYTES, wn0, g);
       if (left < GROUP) {   // both operands: an infinity that one of them repeats there would make the other's zeros NaN
-#pragma unroll
-        for (int m = 0; m < TS::TM; ++m) fa[m].mask(left);
+        fa.mask(left);
         // feature sizes come in eights: groups of eight end ragged in contractions over tokens only (masking everywhere costs the
         // fp32 training step of eight heads of 128, 2048 tokens, 2.5 of 478 us)
         if constexpr ((A_KS && B_KS) || GROUP > 8)
 #pragma unroll
-          for (int n = 0; n < TS::TN; ++n) fb[n].mask(left);
+          for (int j = 0; j < (int)sizeof...(ACC); ++j) fb[j].mask(left);
       }
-#pragma unroll
-      for (int m = 0; m < TS::TM; ++m)
-#pragma unroll
-        for (int n = 0; n < TS::TN; ++n) mma(acc[m][n], fb[n], fa[m]);
+      int j = 0;
+      (mma(acc, fb[j++], fa), ...);
     };
-    for (int k0 = 0; k0 < K[i]; k0 += BK) {
+    for (int left = k; left > 0; left -= BK) {
       if (used + STAGES - 2 < total) wait_vmcnt<(STAGES - 2) * COPIES>();
       else wait_vmcnt<0>();
       __syncthreads();
       if (issued < total) issue();
       const char* st = smem + (used % STAGES) * STAGE;
       ++used;
-      if (K[i] - k0 >= BK) {
+      if (left >= BK) {
 #pragma unroll
-        for (int g = 0; g < BK / GROUP; ++g) group(st, g, GROUP);
+        for (int g = 0; g < GROUPS; ++g) group(st, first + g, GROUP);
       } else {
-        for (int g = 0; g * GROUP < K[i] - k0; ++g) group(st, g, K[i] - k0 - g * GROUP);
+        for (int g = first; g < first + GROUPS && g * GROUP < left; ++g) group(st, g, left - g * GROUP);
       }
     }
   }
+  // Behind the last contraction: the sums of the waves that share a tile.  Each hands the other two quads of its columns and adds the two it
+  // gets to those it keeps, which end in entries 0 .. 7.
+  template <class... ACC>
+  __device__ __forceinline__ void combine(ACC&... acc) {
+    if constexpr (KG == 2) {
+      static_assert(sizeof...(ACC) * 2 * AT::THREADS * 16 <= R::BYTES, "the sums are exchanged inside the ring");
+      const int kg = AT::kgroup();
+      float4* const area = reinterpret_cast<float4*>(smem);
+      __syncthreads();                     // the ring is free
+      int slot = 0;
+      ([&]() LACT_INLINE_LAMBDA {
+#pragma unroll
+        for (int q = 0; q < 2; ++q, ++slot)
+          area[slot * AT::THREADS + threadIdx.x] = kg ? make_float4(acc[4 * q], acc[4 * q + 1], acc[4 * q + 2], acc[4 * q + 3])
+                                                      : make_float4(acc[4 * q + 8], acc[4 * q + 9], acc[4 * q + 10], acc[4 * q + 11]);
+      }(), ...);
+      __syncthreads();
+      slot = 0;
+      ([&]() LACT_INLINE_LAMBDA {
+#pragma unroll
+        for (int q = 0; q < 2; ++q, ++slot) {
+          const float4 o = area[slot * AT::THREADS + (threadIdx.x ^ TS::THREADS)];
+          const float in[4] = {o.x, o.y, o.z, o.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) acc[4 * q + j] = (kg ? acc[4 * q + j + 8] : acc[4 * q + j]) + in[j];
+        }
+      }(), ...);
+    }
+  }
 };
+template <typename T, int NB, int PHASES, bool HALF, class SET>
+__device__ __forceinline__ AsyncPipe<T, NB, PHASES, HALF, SET> async_pipe(char* smem, int steps, SET set) {
+  return AsyncPipe<T, NB, PHASES, HALF, SET>(smem, steps, set);
+}
+__device__ __forceinline__ f32x16 zero16() {
+  f32x16 v;
+#pragma unroll
+  for (int i = 0; i < 16; ++i) v[i] = 0.f;
+  return v;
+}
 
 }  // namespace lact

@@ -165,34 +165,6 @@ __device__ __forceinline__ bf16x8 dma_fetch(const char* tile, int row, int kvec)
 // that XCD's order, so that the shared tiles are fetched from HBM once and not once per die.  A group is
 // one batch entry with all its tiles (batch count a multiple of 8) or one row of tiles of a batch entry.
 // Only the speed depends on the dealing order, never the result.
-// The arguments of a launch lie in memory, and the scalar cache is cold when a kernel begins: read one by one where the code
-// first needs them, they cost one memory latency per 64-byte line, in a row.  One load from every line of the first BYTES up
-// front makes that a single one: the token reduction's copy waves start 0.7 us after the block instead of 2.1 us (with the
-// divisions gone and the offsets of the copies computed without 64-bit products), the hidden stage's 0.6 instead of 1.1 us.
-#define LACT_TOUCH(o) "s_load_dword %0, %1, " #o "*64\n\t"
-#define LACT_TOUCH3 LACT_TOUCH(0) LACT_TOUCH(1) LACT_TOUCH(2)
-#define LACT_TOUCH4 LACT_TOUCH3 LACT_TOUCH(3)
-#define LACT_TOUCH8 LACT_TOUCH4 LACT_TOUCH(4) LACT_TOUCH(5) LACT_TOUCH(6) LACT_TOUCH(7)
-#define LACT_TOUCH12 LACT_TOUCH8 LACT_TOUCH(8) LACT_TOUCH(9) LACT_TOUCH(10) LACT_TOUCH(11)
-#define LACT_TOUCH16 LACT_TOUCH12 LACT_TOUCH(12) LACT_TOUCH(13) LACT_TOUCH(14) LACT_TOUCH(15)
-// one block with its wait: nothing else may hold the register while a load is on its way to it
-#define LACT_TOUCH_ARGS(lines) asm volatile(lines "s_waitcnt lgkmcnt(0)" : "=&s"(unused) : "s"(args) : "memory")
-template <int BYTES>
-__device__ __forceinline__ void prefetch_args() {
-  const uint64_t args = (uint64_t)__builtin_amdgcn_kernarg_segment_ptr();
-  constexpr int N = (BYTES + 63) / 64;
-  int unused;
-  static_assert(N >= 3, "too few lines to be worth it");
-  if constexpr (N == 3) LACT_TOUCH_ARGS(LACT_TOUCH3);
-  else if constexpr (N == 4) LACT_TOUCH_ARGS(LACT_TOUCH4);
-  else if constexpr (N == 5) LACT_TOUCH_ARGS(LACT_TOUCH4 LACT_TOUCH(4));
-  else if constexpr (N == 6) LACT_TOUCH_ARGS(LACT_TOUCH4 LACT_TOUCH(4) LACT_TOUCH(5));
-  else if constexpr (N == 7) LACT_TOUCH_ARGS(LACT_TOUCH4 LACT_TOUCH(4) LACT_TOUCH(5) LACT_TOUCH(6));
-  else if constexpr (N < 12) LACT_TOUCH_ARGS(LACT_TOUCH8);
-  else if constexpr (N < 16) LACT_TOUCH_ARGS(LACT_TOUCH12);
-  else LACT_TOUCH_ARGS(LACT_TOUCH16);
-}
-
 struct TileMap {
   int gx, gy, gz;   // tiles along x and y, batch entries
   int by_batch;     // 1: group = batch entry (gx*gy members); 0: group = (batch entry, x tile) (gy members)

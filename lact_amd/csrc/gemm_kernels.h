@@ -59,29 +59,34 @@ __device__ __forceinline__ float dual_blend(float prod, float ax, int plain_bf16
   return plain_bf16 ? round_bf16(round_bf16(prod) + round_bf16(ax)) : __fadd_rn(ax, prod);
 }
 
-template <typename T, bool B_KC, int NT, int EPI>
-__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_row_gemm(const RowGemmParams<NT> p) {
-  using TS = typename AsyncTile<T>::TS;
+template <typename T, bool B_KC, int NT, int EPI, bool HALF = false>
+__global__ __launch_bounds__((AsyncTile<T, HALF>::THREADS)) void k_row_gemm(const RowGemmParams<NT> p) {
+  prefetch_args<sizeof(p)>();
+  using AT = AsyncTile<T, HALF>;
+  using TS = typename AT::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
-  f32x16 acc[TS::TM][TS::TN];
-  zero_acc<TS>(acc);
-  AsyncPipe<T, NT> pipe(smem);
+  f32x16 acc = zero16();
+  using R = AsyncRing<T, 1, HALF>;
+  int steps = 0;
 #pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const T* A = reinterpret_cast<const T*>(p.t[t].A) + z * p.t[t].bsA + (size_t)m0 * p.t[t].lda;
-    const T* B = reinterpret_cast<const T*>(p.t[t].B) + p.steps.at(z, p.t[t].bsB, p.t[t].gsB) + (B_KC ? (size_t)n0 * p.t[t].ldb : (size_t)n0);
-    pipe.phase(t, A, p.t[t].lda, p.M - m0, false, B, p.t[t].ldb, p.N - n0, !B_KC, p.t[t].K);
-  }
-  pipe.start();
+  for (int t = 0; t < NT; ++t) steps += (p.t[t].K + R::BK - 1) / R::BK;
+  // the terms one after the other through one piece of code: with a copy of it for each, a launch waited for its instructions
+  auto pipe = async_pipe<T, 1, NT, HALF>(smem, steps, [&](auto& q, int t) LACT_INLINE_LAMBDA {
+    const RowGemmTerm& term = p.t[t];
+    q.phase(term.K, reinterpret_cast<const T*>(term.A) + z * term.bsA + (size_t)m0 * term.lda, term.lda, p.M - m0, false, term.ldb, p.N - n0, !B_KC, 1);
+    q.bs[0] = reinterpret_cast<const T*>(term.B) + p.steps.at(z, term.bsB, term.gsB) + (B_KC ? (size_t)n0 * term.ldb : (size_t)n0);
+  });
+#pragma unroll 1
+  for (int t = 0; t < NT; ++t) pipe.template accumulate<false, !B_KC>(p.t[t].K, acc);
+  pipe.combine(acc);
 #pragma unroll
-  for (int t = 0; t < NT; ++t) pipe.template accumulate<false, !B_KC>(t, acc);
-  LACT_FOR_QUADS(TS) {
-    const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
+  for (int g = 0; g < AT::NQ; ++g) {
+    const int m = m0 + AT::m(), n = n0 + AT::n(g);
     if (m >= p.M || n >= p.N) continue;
     float v[4];
 #pragma unroll
-    for (int j = 0; j < 4; ++j) v[j] = acc[tm][tn][4 * g + j];
+    for (int j = 0; j < 4; ++j) v[j] = acc[4 * g + j];
     if (EPI == EPI_STORE) {
       T* o = reinterpret_cast<T*>(p.out) + p.steps.at(z, p.bso, p.gso) + (size_t)m * p.ldo + n;
       if (p.accumulate) {
@@ -147,30 +152,31 @@ struct HiddenParams {
 };
 
 // apply forward:  O0 = silu(X W0^T) * (X W2^T)                       (ttt_operation.py:141-143)
-template <typename T>
-__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_hidden(const HiddenParams p) {
-  using TS = typename AsyncTile<T>::TS;
+template <typename T, bool HALF = false>
+__global__ __launch_bounds__((AsyncTile<T, HALF>::THREADS)) void k_apply_hidden(const HiddenParams p) {
+  prefetch_args<sizeof(p)>();
+  using AT = AsyncTile<T, HALF>;
+  using TS = typename AT::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + p.steps.at(z, p.bsx, p.gsx) + (size_t)m0 * p.ldx;
   const T* W0 = reinterpret_cast<const T*>(p.W0) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
   const T* W2 = reinterpret_cast<const T*>(p.W2) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
-  f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN];
-  zero_acc<TS>(a0);
-  zero_acc<TS>(a2);
-  AsyncPipe<T, 2> pipe(smem);
-  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
-  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
-  pipe.start();
-  pipe.template accumulate<false, false>(0, a0);
-  pipe.template accumulate<false, false>(1, a2);
-  LACT_FOR_QUADS(TS) {
-    const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
+  f32x16 a0 = zero16(), a2 = zero16();
+  auto pipe = async_pipe<T, 2, 1, HALF>(smem, (p.d + AsyncRing<T, 2, HALF>::BK - 1) / AsyncRing<T, 2, HALF>::BK, [&](auto& q, int) LACT_INLINE_LAMBDA {
+    q.phase(p.d, X, p.ldx, p.T - m0, false, p.d, p.dh - n0, false, 2);
+    q.bs[0] = W0; q.bs[1] = W2;
+  });
+  pipe.template accumulate<false, false>(p.d, a0, a2);
+  pipe.combine(a0, a2);
+#pragma unroll
+  for (int g = 0; g < AT::NQ; ++g) {
+    const int m = m0 + AT::m(), n = n0 + AT::n(g);
     if (m >= p.T || n >= p.dh) continue;
     float v[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float y0 = Elem<T>::rnd(a0[tm][tn][4 * g + j]), y2 = Elem<T>::rnd(a2[tm][tn][4 * g + j]);
+      const float y0 = Elem<T>::rnd(a0[4 * g + j]), y2 = Elem<T>::rnd(a2[4 * g + j]);
       v[j] = Elem<T>::rnd(y0 * sigmoidf_(y0)) * y2;
     }
     Elem<T>::store4(reinterpret_cast<T*>(p.O0) + z * p.bso + (size_t)m * p.dh + n, v[0], v[1], v[2], v[3]);
@@ -237,9 +243,11 @@ __device__ __forceinline__ UpdatePointwise2 update_pointwise2(const float* g, co
 
 // update forward:  O0 = dgate_before_act, O1 = hidden * lr1, O2 = dhidden_before_mul
 // (ttt_operation.py:147-168: lr1 scales the hidden-side operand of dw1, lr0 and lr2 scale k -- see k_lr_scale_rows).
-template <typename T>
-__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_hidden(const HiddenParams p) {
-  using TS = typename AsyncTile<T>::TS;
+template <typename T, bool HALF = false>
+__global__ __launch_bounds__((AsyncTile<T, HALF>::THREADS)) void k_update_hidden(const HiddenParams p) {
+  prefetch_args<sizeof(p)>();
+  using AT = AsyncTile<T, HALF>;
+  using TS = typename AT::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
@@ -247,27 +255,29 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_hidden(con
   const T* W0 = reinterpret_cast<const T*>(p.W0) + z * p.bsw + (size_t)n0 * p.d;
   const T* W2 = reinterpret_cast<const T*>(p.W2) + z * p.bsw + (size_t)n0 * p.d;
   const T* W1 = reinterpret_cast<const T*>(p.W1) + z * p.bsw + n0;  // [d, dh]: K-strided for V*W1
-  f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN], a1[TS::TM][TS::TN];
-  zero_acc<TS>(a0);
-  zero_acc<TS>(a2);
-  zero_acc<TS>(a1);
-  AsyncPipe<T, 3> pipe(smem);
-  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
-  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
-  pipe.phase(2, Y, p.ldy, p.T - m0, false, W1, p.dh, p.dh - n0, true, p.d);
-  pipe.start();
-  pipe.template accumulate<false, false>(0, a0);
-  pipe.template accumulate<false, false>(1, a2);
-  pipe.template accumulate<false, true>(2, a1);
-  LACT_FOR_QUADS(TS) {
-    const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
+  f32x16 a0 = zero16(), a2 = zero16(), a1 = zero16();
+  auto pipe = async_pipe<T, 2, 2, HALF>(smem, 2 * ((p.d + AsyncRing<T, 2, HALF>::BK - 1) / AsyncRing<T, 2, HALF>::BK), [&](auto& q, int i) LACT_INLINE_LAMBDA {
+    if (i == 0) {
+      q.phase(p.d, X, p.ldx, p.T - m0, false, p.d, p.dh - n0, false, 2);
+      q.bs[0] = W0; q.bs[1] = W2;
+    } else {
+      q.phase(p.d, Y, p.ldy, p.T - m0, false, p.dh, p.dh - n0, true, 1);
+      q.bs[0] = W1;
+    }
+  });
+  pipe.template accumulate<false, false>(p.d, a0, a2);
+  pipe.template accumulate<false, true>(p.d, a1);
+  pipe.combine(a0, a2, a1);
+#pragma unroll
+  for (int g = 0; g < AT::NQ; ++g) {
+    const int m = m0 + AT::m(), n = n0 + AT::n(g);
     if (m >= p.T || n >= p.dh) continue;
     const float l1 = p.lr1[z * p.bslr + m];
     float z0[4], z1[4], z2[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float gg = Elem<T>::rnd(a0[tm][tn][4 * g + j]), h2 = Elem<T>::rnd(a2[tm][tn][4 * g + j]);
-      const float dh = Elem<T>::rnd(a1[tm][tn][4 * g + j]);
+      const float gg = Elem<T>::rnd(a0[4 * g + j]), h2 = Elem<T>::rnd(a2[4 * g + j]);
+      const float dh = Elem<T>::rnd(a1[4 * g + j]);
       const UpdatePointwise u = update_pointwise<T>(gg, h2, dh, silu_parts(gg));
       z0[j] = u.dgpre;
       z1[j] = u.hid * l1;
@@ -301,7 +311,7 @@ __global__ void k_lr_scale_rows(const T* k, int ld, long long bs, const float* l
 // Row sums over the hidden dimension of a per-thread partial: lanes l and l^32 hold the same token.
 // Each wave then owns one partial per token; the slot index is (hidden tile, wave column).
 template <class TS>
-__device__ __forceinline__ void store_row_partials(const HiddenParams& p, int which, int tm, int m, int z, float v, int ytile) {
+__device__ __forceinline__ void store_row_partials(const HiddenParams& p, int which, int m, int z, float v, int ytile) {
   v += __shfl_xor(v, 32, 64);
   if ((threadIdx.x & 63) < 32 && m < p.T) {
     const int slot = ytile * TS::WAVES_N + ((threadIdx.x >> 6) % TS::WAVES_N);
@@ -311,9 +321,11 @@ __device__ __forceinline__ void store_row_partials(const HiddenParams& p, int wh
 
 // apply backward, hidden stage:  O0 = hidden (recomputed), O1 = d/d(X W0^T), O2 = d/d(X W2^T)
 // with Y = upstream gradient of the apply output  (lact_triton_kernels/lact_swiglu_ffn.py:57-65).
-template <typename T>
-__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_bwd_hidden(const HiddenParams p) {
-  using TS = typename AsyncTile<T>::TS;
+template <typename T, bool HALF = false>
+__global__ __launch_bounds__((AsyncTile<T, HALF>::THREADS)) void k_apply_bwd_hidden(const HiddenParams p) {
+  prefetch_args<sizeof(p)>();
+  using AT = AsyncTile<T, HALF>;
+  using TS = typename AT::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + p.steps.at(z, p.bsx, p.gsx) + (size_t)m0 * p.ldx;
@@ -321,26 +333,28 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_bwd_hidden(
   const T* W0 = reinterpret_cast<const T*>(p.W0) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
   const T* W2 = reinterpret_cast<const T*>(p.W2) + p.steps.at(z, p.bsw, p.gsw) + (size_t)n0 * p.d;
   const T* W1 = reinterpret_cast<const T*>(p.W1) + p.steps.at(z, p.bsw, p.gsw) + n0;
-  f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN], a1[TS::TM][TS::TN];
-  zero_acc<TS>(a0);
-  zero_acc<TS>(a2);
-  zero_acc<TS>(a1);
-  AsyncPipe<T, 3> pipe(smem);
-  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
-  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
-  pipe.phase(2, Y, p.ldy, p.T - m0, false, W1, p.dh, p.dh - n0, true, p.d);
-  pipe.start();
-  pipe.template accumulate<false, false>(0, a0);
-  pipe.template accumulate<false, false>(1, a2);
-  pipe.template accumulate<false, true>(2, a1);
-  LACT_FOR_QUADS(TS) {
-    const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
+  f32x16 a0 = zero16(), a2 = zero16(), a1 = zero16();
+  auto pipe = async_pipe<T, 2, 2, HALF>(smem, 2 * ((p.d + AsyncRing<T, 2, HALF>::BK - 1) / AsyncRing<T, 2, HALF>::BK), [&](auto& q, int i) LACT_INLINE_LAMBDA {
+    if (i == 0) {
+      q.phase(p.d, X, p.ldx, p.T - m0, false, p.d, p.dh - n0, false, 2);
+      q.bs[0] = W0; q.bs[1] = W2;
+    } else {
+      q.phase(p.d, Y, p.ldy, p.T - m0, false, p.dh, p.dh - n0, true, 1);
+      q.bs[0] = W1;
+    }
+  });
+  pipe.template accumulate<false, false>(p.d, a0, a2);
+  pipe.template accumulate<false, true>(p.d, a1);
+  pipe.combine(a0, a2, a1);
+#pragma unroll
+  for (int g = 0; g < AT::NQ; ++g) {
+    const int m = m0 + AT::m(), n = n0 + AT::n(g);
     if (m >= p.T || n >= p.dh) continue;
     float hq[4], gy0[4], gy2[4];
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      const float y0 = Elem<T>::rnd(a0[tm][tn][4 * g + j]), y2 = Elem<T>::rnd(a2[tm][tn][4 * g + j]);
-      const float gh = Elem<T>::rnd(a1[tm][tn][4 * g + j]);
+      const float y0 = Elem<T>::rnd(a0[4 * g + j]), y2 = Elem<T>::rnd(a2[4 * g + j]);
+      const float gh = Elem<T>::rnd(a1[4 * g + j]);
       const SiluParts s = silu_parts(y0);
       const float sg = Elem<T>::rnd(s.silu);
       hq[j] = sg * y2;
@@ -360,9 +374,11 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_apply_bwd_hidden(
 //   O0 = d/d gate_before_act, O1 = d/d dhidden, O2 = d/d hidden_before_mul,
 //   O3 = dgate_before_act*lr0, O4 = hidden*lr1, O5 = dhidden_before_mul*lr2 (recomputed operands)
 // plus per-token partial sums of the lr gradients.
-template <typename T>
-__global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_bwd_hidden(const HiddenParams p) {
-  using TS = typename AsyncTile<T>::TS;
+template <typename T, bool HALF = false>
+__global__ __launch_bounds__((AsyncTile<T, HALF>::THREADS)) void k_update_bwd_hidden(const HiddenParams p) {
+  prefetch_args<sizeof(p)>();
+  using AT = AsyncTile<T, HALF>;
+  using TS = typename AT::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int m0 = blockIdx.x * TS::BM, n0 = blockIdx.y * TS::BN, z = blockIdx.z;
   const T* X = reinterpret_cast<const T*>(p.X) + z * p.bsx + (size_t)m0 * p.ldx;
@@ -373,68 +389,68 @@ __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_update_bwd_hidden
   const T* G0 = reinterpret_cast<const T*>(p.G0) + z * p.bsw + (size_t)n0 * p.d;
   const T* G2 = reinterpret_cast<const T*>(p.G2) + z * p.bsw + (size_t)n0 * p.d;
   const T* G1 = reinterpret_cast<const T*>(p.G1) + z * p.bsw + n0;
-  f32x16 a0[TS::TM][TS::TN], a2[TS::TM][TS::TN], a1[TS::TM][TS::TN];
-  f32x16 b0[TS::TM][TS::TN], b2[TS::TM][TS::TN], b1[TS::TM][TS::TN];
-  zero_acc<TS>(a0); zero_acc<TS>(a2); zero_acc<TS>(a1);
-  zero_acc<TS>(b0); zero_acc<TS>(b2); zero_acc<TS>(b1);
-  AsyncPipe<T, 6> pipe(smem);
-  pipe.phase(0, X, p.ldx, p.T - m0, false, W0, p.d, p.dh - n0, false, p.d);
-  pipe.phase(1, X, p.ldx, p.T - m0, false, W2, p.d, p.dh - n0, false, p.d);
-  pipe.phase(2, X, p.ldx, p.T - m0, false, G0, p.d, p.dh - n0, false, p.d);
-  pipe.phase(3, X, p.ldx, p.T - m0, false, G2, p.d, p.dh - n0, false, p.d);
-  pipe.phase(4, Y, p.ldy, p.T - m0, false, W1, p.dh, p.dh - n0, true, p.d);
-  pipe.phase(5, Y, p.ldy, p.T - m0, false, G1, p.dh, p.dh - n0, true, p.d);
-  pipe.start();
-  pipe.template accumulate<false, false>(0, a0);
-  pipe.template accumulate<false, false>(1, a2);
-  pipe.template accumulate<false, false>(2, b0);
-  pipe.template accumulate<false, false>(3, b2);
-  pipe.template accumulate<false, true>(4, a1);
-  pipe.template accumulate<false, true>(5, b1);
-#pragma unroll
-  for (int tm = 0; tm < TS::TM; ++tm) {
-    const int m = m0 + quad_m<TS>(tm);
+  f32x16 a0 = zero16(), a2 = zero16(), a1 = zero16(), b0 = zero16(), b2 = zero16(), b1 = zero16();
+  auto pipe = async_pipe<T, 4, 2, HALF>(smem, 2 * ((p.d + AsyncRing<T, 4, HALF>::BK - 1) / AsyncRing<T, 4, HALF>::BK), [&](auto& q, int i) LACT_INLINE_LAMBDA {
+    if (i == 0) {
+      q.phase(p.d, X, p.ldx, p.T - m0, false, p.d, p.dh - n0, false, 4);
+      q.bs[0] = W0; q.bs[1] = W2; q.bs[2] = G0; q.bs[3] = G2;
+    } else {
+      q.phase(p.d, Y, p.ldy, p.T - m0, false, p.dh, p.dh - n0, true, 2);
+      q.bs[0] = W1; q.bs[1] = G1;
+    }
+  });
+  pipe.template accumulate<false, false>(p.d, a0, a2, b0, b2);
+  pipe.template accumulate<false, true>(p.d, a1, b1);
+  pipe.combine(a0, a2, a1, b0, b2, b1);
+  {
+    const int m = m0 + AT::m();
     const bool mv = m < p.T;
     const float l0 = mv ? p.lr0[z * p.bslr + m] : 0.f, l1 = mv ? p.lr1[z * p.bslr + m] : 0.f;
     const float l2 = mv ? p.lr2[z * p.bslr + m] : 0.f;
     float s0 = 0.f, s1 = 0.f, s2 = 0.f;
 #pragma unroll
-    for (int tn = 0; tn < TS::TN; ++tn)
+    for (int g = 0; g < AT::NQ; ++g) {
+      const int n = n0 + AT::n(g);
+      if (!mv || n >= p.dh) continue;
+      float o0[4], o1[4], o2[4], o3[4], o4[4], o5[4];
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + quad_n<TS>(tn, g);
-        if (!mv || n >= p.dh) continue;
-        float o0[4], o1[4], o2[4], o3[4], o4[4], o5[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float gg = Elem<T>::rnd(a0[tm][tn][4 * g + j]), h2 = Elem<T>::rnd(a2[tm][tn][4 * g + j]);
-          const float dh = Elem<T>::rnd(a1[tm][tn][4 * g + j]);
-          const float gz0 = Elem<T>::rnd(b0[tm][tn][4 * g + j]), gz2 = Elem<T>::rnd(b2[tm][tn][4 * g + j]);
-          const float gz1 = Elem<T>::rnd(b1[tm][tn][4 * g + j]);
-          const SiluParts s = silu_parts(gg);
-          const UpdatePointwise u = update_pointwise<T>(gg, h2, dh, s);
-          s0 += gz0 * u.dgpre;
-          s1 += gz1 * u.hid;
-          s2 += gz2 * u.dh2;
-          const float ghid = gz1 * l1, gdh2 = gz2 * l2, gdg = gz0 * l0;
-          o0[j] = ghid * h2 * s.d1 + gdh2 * dh * s.d1 + gdg * dh * h2 * s.d2;   // d gate_before_act
-          o1[j] = gdh2 * s.silu + gdg * h2 * s.d1;                             // d dhidden
-          o2[j] = ghid * s.silu + gdg * dh * s.d1;                             // d hidden_before_mul
-          o3[j] = u.dgpre * l0;
-          o4[j] = u.hid * l1;
-          o5[j] = u.dh2 * l2;
-        }
-        const size_t off = z * p.bso + (size_t)m * p.dh + n;
-        Elem<T>::store4(reinterpret_cast<T*>(p.O0) + off, o0[0], o0[1], o0[2], o0[3]);
-        Elem<T>::store4(reinterpret_cast<T*>(p.O1) + off, o1[0], o1[1], o1[2], o1[3]);
-        Elem<T>::store4(reinterpret_cast<T*>(p.O2) + off, o2[0], o2[1], o2[2], o2[3]);
-        Elem<T>::store4(reinterpret_cast<T*>(p.O3) + off, o3[0], o3[1], o3[2], o3[3]);
-        Elem<T>::store4(reinterpret_cast<T*>(p.O4) + off, o4[0], o4[1], o4[2], o4[3]);
-        Elem<T>::store4(reinterpret_cast<T*>(p.O5) + off, o5[0], o5[1], o5[2], o5[3]);
+      for (int j = 0; j < 4; ++j) {
+        const float gg = Elem<T>::rnd(a0[4 * g + j]), h2 = Elem<T>::rnd(a2[4 * g + j]);
+        const float dh = Elem<T>::rnd(a1[4 * g + j]);
+        const float gz0 = Elem<T>::rnd(b0[4 * g + j]), gz2 = Elem<T>::rnd(b2[4 * g + j]);
+        const float gz1 = Elem<T>::rnd(b1[4 * g + j]);
+        const SiluParts s = silu_parts(gg);
+        const UpdatePointwise u = update_pointwise<T>(gg, h2, dh, s);
+        s0 += gz0 * u.dgpre;
+        s1 += gz1 * u.hid;
+        s2 += gz2 * u.dh2;
+        const float ghid = gz1 * l1, gdh2 = gz2 * l2, gdg = gz0 * l0;
+        o0[j] = ghid * h2 * s.d1 + gdh2 * dh * s.d1 + gdg * dh * h2 * s.d2;   // d gate_before_act
+        o1[j] = gdh2 * s.silu + gdg * h2 * s.d1;                             // d dhidden
+        o2[j] = ghid * s.silu + gdg * dh * s.d1;                             // d hidden_before_mul
+        o3[j] = u.dgpre * l0;
+        o4[j] = u.hid * l1;
+        o5[j] = u.dh2 * l2;
       }
-    store_row_partials<TS>(p, 0, tm, m, z, s0, blockIdx.y);
-    store_row_partials<TS>(p, 1, tm, m, z, s1, blockIdx.y);
-    store_row_partials<TS>(p, 2, tm, m, z, s2, blockIdx.y);
+      const size_t off = z * p.bso + (size_t)m * p.dh + n;
+      Elem<T>::store4(reinterpret_cast<T*>(p.O0) + off, o0[0], o0[1], o0[2], o0[3]);
+      Elem<T>::store4(reinterpret_cast<T*>(p.O1) + off, o1[0], o1[1], o1[2], o1[3]);
+      Elem<T>::store4(reinterpret_cast<T*>(p.O2) + off, o2[0], o2[1], o2[2], o2[3]);
+      Elem<T>::store4(reinterpret_cast<T*>(p.O3) + off, o3[0], o3[1], o3[2], o3[3]);
+      Elem<T>::store4(reinterpret_cast<T*>(p.O4) + off, o4[0], o4[1], o4[2], o4[3]);
+      Elem<T>::store4(reinterpret_cast<T*>(p.O5) + off, o5[0], o5[1], o5[2], o5[3]);
+    }
+    if constexpr (HALF) {   // the other half of the tile's columns
+      __syncthreads();
+      float* const part = reinterpret_cast<float*>(smem) + (threadIdx.x & (TS::THREADS - 1));
+      if (AT::kgroup()) { part[0] = s0; part[TS::THREADS] = s1; part[2 * TS::THREADS] = s2; }
+      __syncthreads();
+      if (AT::kgroup()) return;
+      s0 += part[0]; s1 += part[TS::THREADS]; s2 += part[2 * TS::THREADS];
+    }
+    store_row_partials<TS>(p, 0, m, z, s0, blockIdx.y);
+    store_row_partials<TS>(p, 1, m, z, s1, blockIdx.y);
+    store_row_partials<TS>(p, 2, m, z, s2, blockIdx.y);
   }
 }
 
@@ -469,36 +485,38 @@ struct TokenReduceParams {
 
 template <typename T>
 __global__ __launch_bounds__(AsyncTile<T>::TS::THREADS) void k_token_reduce(const TokenReduceParams p) {
+  prefetch_args<sizeof(p)>();
   using TS = typename AsyncTile<T>::TS;
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int t = p.by_nb.div(blockIdx.z), ib = blockIdx.z - t * p.by_nb.d, g = t / 3, j = t - 3 * g;
+  const int t = p.by_nb.div(blockIdx.z), ib = blockIdx.z - t * p.by_nb.d, step = t / 3, j = t - 3 * step;
   const TokenReduceJob& job = p.job[j];
   const int tiles_n = (job.N + TS::BN - 1) / TS::BN;
   const int m0 = (blockIdx.x / tiles_n) * TS::BM, n0 = (blockIdx.x % tiles_n) * TS::BN;
   if (m0 >= job.M) return;
   const int k_begin = blockIdx.y * p.split_len;
   const int klen = min(p.split_len, p.tokens - k_begin);
-  f32x16 acc[TS::TM][TS::TN];
-  zero_acc<TS>(acc);
-  AsyncPipe<T, 1> pipe(smem);
-  const T* A = reinterpret_cast<const T*>(job.t.A) + ib * job.t.bsA + g * job.t.gsA + (size_t)k_begin * job.t.lda + m0;
-  const T* B = reinterpret_cast<const T*>(job.t.B) + ib * job.t.bsB + g * job.t.gsB + (size_t)k_begin * job.t.ldb + n0;
-  pipe.phase(0, A, job.t.lda, job.M - m0, true, B, job.t.ldb, job.N - n0, true, klen);
-  pipe.start();
-  pipe.template accumulate<true, true>(0, acc);
+  f32x16 acc = zero16();
+  const T* A = reinterpret_cast<const T*>(job.t.A) + ib * job.t.bsA + step * job.t.gsA + (size_t)k_begin * job.t.lda + m0;
+  const T* B = reinterpret_cast<const T*>(job.t.B) + ib * job.t.bsB + step * job.t.gsB + (size_t)k_begin * job.t.ldb + n0;
+  auto pipe = async_pipe<T, 1, 1, false>(smem, (klen + AsyncRing<T, 1>::BK - 1) / AsyncRing<T, 1>::BK, [&](auto& q, int) LACT_INLINE_LAMBDA {
+    q.phase(klen, A, job.t.lda, job.M - m0, true, job.t.ldb, job.N - n0, true, 1);
+    q.bs[0] = B;
+  });
+  pipe.template accumulate<true, true>(klen, acc);
   const size_t slot = (size_t)blockIdx.z * p.mat_elems;
   float* out = p.add_out ? p.add_out + slot : p.partial + (size_t)blockIdx.y * gridDim.z * p.mat_elems + slot;
-  LACT_FOR_QUADS(TS) {
-    const int m = m0 + quad_m<TS>(tm), n = n0 + quad_n<TS>(tn, g);
+#pragma unroll
+  for (int g = 0; g < 4; ++g) {
+    const int m = m0 + quad_m<TS>(0), n = n0 + quad_n<TS>(0, g);
     if (m >= job.M || n >= job.N) continue;
     if (p.add_out && p.add_in) {
       float in[4];
       Elem<float>::load4(p.add_in + slot + (size_t)m * job.N + n, in);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) acc[tm][tn][4 * g + j] += p.coeff * in[j];
+      for (int j = 0; j < 4; ++j) acc[4 * g + j] += p.coeff * in[j];
     }
-    Elem<float>::store4(out + (size_t)m * job.N + n, acc[tm][tn][4 * g], acc[tm][tn][4 * g + 1], acc[tm][tn][4 * g + 2],
-                        acc[tm][tn][4 * g + 3]);
+    Elem<float>::store4(out + (size_t)m * job.N + n, acc[4 * g], acc[4 * g + 1], acc[4 * g + 2],
+                        acc[4 * g + 3]);
   }
 }
 

@@ -191,10 +191,10 @@ inline const char* align256(const void* p) {
   return reinterpret_cast<const char*>((reinterpret_cast<uintptr_t>(p) + 255) & ~uintptr_t(255));
 }
 
-template <typename T, bool B_KC, int NT, int EPI>
+template <typename T, bool B_KC, int NT, int EPI, bool HALF>
 const char* row_gemm_name() {
   static const std::string n = std::string("k_row_gemm<") + tname<T>() + (B_KC ? ",Bkc," : ",Bks,") + std::to_string(NT) +
-                               (EPI == EPI_STORE ? ",store>" : (EPI == EPI_AXPBY ? ",axpby>" : ",axpby_dual>"));
+                               (EPI == EPI_STORE ? ",store" : (EPI == EPI_AXPBY ? ",axpby" : ",axpby_dual")) + (HALF ? ",half>" : ">");
   return n.c_str();
 }
 template <class TS, int NT, int EPI, bool B_KS>
@@ -212,6 +212,26 @@ void launch_row_gemm_dma(const char* site, const RowGemmDmaParams<NT>& q, int ba
   LACT_LAUNCH_SMEM(name.c_str(), site, 2.0 * q.g.M * q.g.N * ksum * batch, (k_row_gemm_dma<TS, NT, EPI, B_KS>), dim3(qq.map.grid()),
                    dim3(DMA_THREADS), SMEM, s, qq);
 }
+int device_cus() {
+  static const int cus = [] { int dev = 0, n = 0; (void)hipGetDevice(&dev); return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256; }();
+  return cus;
+}
+// fp32 launches that would leave a compute unit without a 64 x 64 tile take half tiles instead (gemm_async.h).  us, whole tiles / half: at
+// 128 of the former (8 x 512 tokens, d = dh = 128) apply hidden stage 12.1 / 7.4, update 14.8 / 12.2, update backward 24.6 / 18.9, four-term
+// row GEMM 17.1 / 13.6; at 192 even; at 384 still 1.1 to 1.15 times faster, but at 256, 512 and 1024 up to 1.4 times slower (two-term row
+// GEMM 18.6 / 26.3 at 512), as the half tiles read every A row twice.
+bool half_tiles(long long blocks) { return blocks < device_cus(); }
+template <typename T, bool B_KC, int NT, int EPI, bool HALF>
+void launch_row_gemm_async(const char* site, const RowGemmParams<NT>& p, int batch, hipStream_t s) {
+  using AT = AsyncTile<T, HALF>;
+  constexpr int SM = AsyncRing<T, 1, HALF>::BYTES;
+  const dim3 grid(ceil_div(p.M, AT::TS::BM), ceil_div(p.N, AT::TS::BN), batch);
+  double ksum = 0;
+  for (int t = 0; t < NT; ++t) ksum += p.t[t].K;
+  LACT_BIG_LDS((k_row_gemm<T, B_KC, NT, EPI, HALF>), SM);
+  LACT_LAUNCH_SMEM((row_gemm_name<T, B_KC, NT, EPI, HALF>()), site, 2.0 * p.M * p.N * ksum * batch,
+                   (k_row_gemm<T, B_KC, NT, EPI, HALF>), grid, dim3(AT::THREADS), SM, s, p);
+}
 // bf16 with every K a multiple of 16: dedicated-loader kernels; anything else: the small-tile pipeline
 template <typename T, bool B_KC, int NT, int EPI>
 void launch_row_gemm(const char* site, const RowGemmParams<NT>& p, int batch, hipStream_t s, bool token_rows = false) {
@@ -225,7 +245,7 @@ void launch_row_gemm(const char* site, const RowGemmParams<NT>& p, int batch, hi
       if (token_rows) {
         // 256 x 128 tiles copy a third fewer operand bytes per FLOP than 128 x 128 ones, but a launch whose blocks fill
         // the last round of compute units only partly wastes more than that: pick by the fuller last round
-        static const int cus = [] { int dev = 0, n = 0; (void)hipGetDevice(&dev); return hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0 ? n : 256; }();
+        const int cus = device_cus();
         auto blocks = [&](int bm, int bn) { return (long long)ceil_div(p.M, bm) * ceil_div(p.N, bn) * batch; };
         auto fill = [&](int bm) { const long long n = blocks(bm, 128); return (double)n / ((double)((n + cus - 1) / cus) * cus); };
         // less than one round: the blocks that fit side by side, down to 128 x 64
@@ -241,14 +261,9 @@ void launch_row_gemm(const char* site, const RowGemmParams<NT>& p, int batch, hi
       return;
     }
   }
-  using TS = TSG<T>;
-  constexpr int SM = AsyncPipe<T, NT>::BYTES;
-  dim3 grid(ceil_div(p.M, TS::BM), ceil_div(p.N, TS::BN), batch);
-  double ksum = 0;
-  for (int t = 0; t < NT; ++t) ksum += p.t[t].K;
-  LACT_BIG_LDS((k_row_gemm<T, B_KC, NT, EPI>), SM);
-  LACT_LAUNCH_SMEM((row_gemm_name<T, B_KC, NT, EPI>()), site, 2.0 * p.M * p.N * ksum * batch,
-                   (k_row_gemm<T, B_KC, NT, EPI>), grid, dim3(TS::THREADS), SM, s, p);
+  if constexpr (!std::is_same<T, uint16_t>::value)
+    if (half_tiles((long long)ceil_div(p.M, TSG<T>::BM) * ceil_div(p.N, TSG<T>::BN) * batch)) return launch_row_gemm_async<T, B_KC, NT, EPI, true>(site, p, batch, s);
+  launch_row_gemm_async<T, B_KC, NT, EPI, false>(site, p, batch, s);
 }
 
 template <int NT>
@@ -513,7 +528,7 @@ struct Runner {
   bool dma_hidden() const { return kBf16 && d.d % 16 == 0; }
   // row-partial slots the update-backward hidden kernel in use writes: (hidden tiles) x (wave columns)
   int lr_parts() const {
-    if (!dma_hidden()) return ceil_div(d.dh, TSG<T>::BN) * TSG<T>::WAVES_N;
+    if (!dma_hidden()) return hidden_half(3, P.Tupd, d.b) ? ceil_div(d.dh, 32) : ceil_div(d.dh, TSG<T>::BN) * TSG<T>::WAVES_N;
     if (P.keep_pre) return ceil_div(d.dh, TS_SQ::BN) * TS_SQ::WAVES_N;
     return ceil_div(d.dh, TS_BWD::BN) * TS_BWD::WAVES_N;
   }
@@ -524,6 +539,12 @@ struct Runner {
     if (d.d % 64 || d.d < 384 || d.dh % 8) return false;
     const int cols = ceil_div(d.dh, TS_WIDE::BN) * nz;
     return ceil_div(ceil_div(T_, TS_WIDE::BM) * cols, 256) * 1.62 < ceil_div(ceil_div(T_, 128) * cols, 256);
+  }
+  // fp32: half tiles (gemm_async.h).  One answer for all updates of a program: it decides where the rates' partial sums lie.
+  bool hidden_half(int which, int T_, int nz) const {
+    if constexpr (kBf16) return false;
+    const int t = which == 3 ? P.Tupd : T_;
+    return half_tiles((long long)ceil_div(t, TSG<T>::BM) * ceil_div(d.dh, TSG<T>::BN) * nz);
   }
   // LACT_OPT_PERSISTENT_TILES: its default, the apply alone, gives way to the small tiles; any other mask is taken as it is
   bool hidden_persists(int which) const {
@@ -600,18 +621,24 @@ struct Runner {
       }
       }
     } else {
-      using TS = TSG<T>;
-      constexpr int SM = AsyncPipe<T, 1>::BYTES;
-      const dim3 g(ceil_div(T_, TS::BM), ceil_div(d.dh, TS::BN), nz);
-      LACT_BIG_LDS(k_apply_hidden<T>, SM);
-      LACT_BIG_LDS(k_update_hidden<T>, SM);
-      LACT_BIG_LDS(k_apply_bwd_hidden<T>, SM);
-      LACT_BIG_LDS(k_update_bwd_hidden<T>, SM);
-      if (which == 0) LACT_LAUNCH_SMEM("k_apply_hidden", "apply_hidden", 4.0 * f, (k_apply_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
-      if (which == 1) LACT_LAUNCH_SMEM("k_update_hidden", "update_hidden", 6.0 * f, (k_update_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
-      if (which == 2) LACT_LAUNCH_SMEM("k_apply_bwd_hidden", "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
-      if (which == 3) LACT_LAUNCH_SMEM("k_update_bwd_hidden", "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden<T>), g, dim3(TS::THREADS), SM, s, hp);
+      if constexpr (!kBf16)
+        if (hidden_half(which, T_, nz)) return launch_hidden_async<true>(which, hp, T_, nz, f);
+      launch_hidden_async<false>(which, hp, T_, nz, f);
     }
+  }
+  template <bool HALF>
+  void launch_hidden_async(int which, const HiddenParams& hp, int T_, int nz, double f) const {
+    using AT = AsyncTile<T, HALF>;
+    constexpr int SM = AsyncRing<T, 2, HALF>::BYTES, SM4 = AsyncRing<T, 4, HALF>::BYTES;
+    const dim3 g(ceil_div(T_, AT::TS::BM), ceil_div(d.dh, AT::TS::BN), nz), t(AT::THREADS);
+    LACT_BIG_LDS((k_apply_hidden<T, HALF>), SM);
+    LACT_BIG_LDS((k_update_hidden<T, HALF>), SM);
+    LACT_BIG_LDS((k_apply_bwd_hidden<T, HALF>), SM);
+    LACT_BIG_LDS((k_update_bwd_hidden<T, HALF>), SM4);
+    if (which == 0) LACT_LAUNCH_SMEM((HALF ? "k_apply_hidden<half>" : "k_apply_hidden"), "apply_hidden", 4.0 * f, (k_apply_hidden<T, HALF>), g, t, SM, s, hp);
+    if (which == 1) LACT_LAUNCH_SMEM((HALF ? "k_update_hidden<half>" : "k_update_hidden"), "update_hidden", 6.0 * f, (k_update_hidden<T, HALF>), g, t, SM, s, hp);
+    if (which == 2) LACT_LAUNCH_SMEM((HALF ? "k_apply_bwd_hidden<half>" : "k_apply_bwd_hidden"), "apply_bwd_hidden", 6.0 * f, (k_apply_bwd_hidden<T, HALF>), g, t, SM, s, hp);
+    if (which == 3) LACT_LAUNCH_SMEM((HALF ? "k_update_bwd_hidden<half>" : "k_update_bwd_hidden"), "update_bwd_hidden", 12.0 * f, (k_update_bwd_hidden<T, HALF>), g, t, SM4, s, hp);
   }
   // An apply step as one kernel, for the head sizes it exists for.  (A value of LACT_OPT_PERSISTENT_TILES other than the default
   // asks for the hidden-stage kernels.)
@@ -880,7 +907,7 @@ struct Runner {
     }
     // fp32, or fewer than 64 tokens
     using TS = TSG<T>;
-    constexpr int SM = AsyncPipe<T, 2>::BYTES;
+    constexpr int SM = AsyncRing<T, 1>::BYTES;
     const Split sp = P.reduce_split(tokens, steps, max_n, P.split_min);
     direct = add_out && sp.n == 1;
     if (direct) { p.add_out = add_out; p.add_in = coeff != 0.f ? add_in : nullptr; p.coeff = coeff; }

@@ -88,6 +88,7 @@ struct LayerPreParams {
 // 600 MB); 7500 tokens, 8 heads of 96 19 / 34 (37 / 65: 69 and 104 MB).
 template <typename T, bool BWD, bool ATT, int G, int NV>
 __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
+  prefetch_args<sizeof(p)>();
   using RL = RowLanes<G, NV>;
   const int wave = threadIdx.x >> 6, grp = RL::group();
   const int hd = p.g.hd, h = blockIdx.x % p.g.H;
@@ -254,6 +255,7 @@ struct LayerLrParams {
 };
 template <bool BWD>
 __global__ void k_layer_lr(const LayerLrParams p) {
+  prefetch_args<sizeof(p)>();
   const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;   // over (b, l, h)
   if (i >= p.g.rows()) return;
   const int h = (int)(i % p.g.H);
@@ -294,6 +296,7 @@ struct LayerPostParams {
 // (53 / 71: 150 MB each); 7500 tokens, 8 heads of 96 9.3 / 12.6 (22 / 36).
 template <typename T, bool BWD, int G, int NV>
 __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
+  prefetch_args<sizeof(p)>();
   using RL = RowLanes<G, NV>;
   const int wave = threadIdx.x >> 6, grp = RL::group();
   const long long step = (long long)gridDim.x * 4 * RL::ROWS;
@@ -498,6 +501,7 @@ __device__ __forceinline__ float layer_in_grad(const LayerInParams& p, int n, lo
 // lane holds (one shuffle a value instead of six).
 template <int NB>
 __global__ __launch_bounds__(256) void k_layer_in(const LayerInParams p) {
+  prefetch_args<sizeof(p)>();
   constexpr int NO = 4 * NB, TOK = LAYER_IN_TOK;
   __shared__ float4 ws[NO][64];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -571,6 +575,7 @@ __global__ __launch_bounds__(256) void k_layer_in(const LayerInParams p) {
 // 256 registers and seven accumulation registers, one wave a SIMD; more outputs would need a second pass.
 template <int NL, int NB>
 __global__ __launch_bounds__(256) void k_layer_in_dx(const LayerInParams p) {
+  prefetch_args<sizeof(p)>();
   constexpr int NO = 4 * (NL + NB), TOK = LAYER_IN_DXTOK;
   __shared__ float gs[TOK][NO];
   const long long t0 = (long long)blockIdx.x * TOK;
@@ -599,6 +604,7 @@ __global__ __launch_bounds__(256) void k_layer_in_dx(const LayerInParams p) {
 // waves', in a fixed order; k_layer_in_reduce sums the blocks.  Grid (token blocks, chunks of 256 columns).
 template <int NL, int NB>
 __global__ __launch_bounds__(256) void k_layer_in_dw(const LayerInParams p) {
+  prefetch_args<sizeof(p)>();
   constexpr int NO = 4 * (NL + NB), TOK = LAYER_IN_DWTOK;
   __shared__ float lds[(4 * TOK > 256 ? 4 * TOK : 256) * NO];   // output gradients of the block's tokens, then the sums of its waves
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tok = p.dw_tok;

@@ -99,6 +99,7 @@ constexpr int ns_local_lds() { return RT * 32 * (XG + 3 * 16) * 16; }
 // PLAIN: the reference without autocast, every value a bf16 tensor.
 template <int RT, int XG, bool PLAIN>
 __global__ __launch_bounds__(512, 2) void k_ns_local(const NsLocalParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int WPR = RT == 3 ? 2 : 8 / RT;                       // waves that share a row of tiles
   constexpr int CX = (XG / 4 + WPR - 1) / WPR, CS = (RT + WPR - 1) / WPR;   // tiles per wave of an [r, c] and of an [r, r] matrix

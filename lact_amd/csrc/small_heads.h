@@ -78,6 +78,7 @@ struct ApplyCopies {
 
 template <int D, bool SPLIT>
 __global__ __launch_bounds__(512, 2) void k_apply_fused(const ApplyFusedParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using ST = ApplyStage<D>;
   int bx, by, z;
@@ -167,6 +168,7 @@ __global__ __launch_bounds__(512, 2) void k_apply_fused(const ApplyFusedParams p
   constexpr std::false_type no{};
   auto at = [&](int t) { return smem + (t % 3) * ST::BYTES; };
   f32x16 ga, ua, gb, ub;
+  attn_arrived(qf);
   open(0);
   if (!SPLIT) {
     step(yes, no, at(0), ga, ua, at(0), 0, gb, ub);
@@ -346,6 +348,7 @@ struct UpdateSteps {
 
 template <int D>
 __global__ __launch_bounds__(256, 1) void k_update_fused(const UpdateFusedParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using U = UpdatePatch<D>;
   int bx, by, z;
@@ -744,6 +747,7 @@ struct BwdSteps {
 
 template <int D>
 __global__ __launch_bounds__(256, 1) void k_update_bwd_fused(const UpdateBwdFusedParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using ST = BwdStage<D>;
   using U = UpdatePatch<D>;
@@ -939,6 +943,7 @@ struct ApplyBwdStage {
 
 template <int D>
 __global__ __launch_bounds__(512, 2) void k_apply_bwd_fused(const ApplyBwdFusedParams p) {
+  prefetch_args<sizeof(p)>();
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using ST = ApplyBwdStage<D>;
   using U = UpdatePatch<D>;

@@ -85,6 +85,7 @@ __device__ __forceinline__ void init_store(const InitParams& p, float* ext, size
 }
 template <typename T>
 __global__ void k_init_state(const InitParams p) {
+  prefetch_args<sizeof(p)>();
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= p.g.rows(j)) return;
@@ -107,6 +108,7 @@ __global__ void k_init_state(const InitParams p) {
 // eight loads of a thread at once 5.4.  Grid (ceil(max rows / 32), 3b), 256 threads.
 template <typename T>
 __global__ __launch_bounds__(256) void k_init_state_transposed(const InitParams p) {
+  prefetch_args<sizeof(p)>();
   __shared__ float tile[256][33];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb, row0 = blockIdx.x * 32;
   const int rows = p.g.rows(j), cols = p.g.cols(j);
@@ -244,6 +246,7 @@ struct TallTile {
 
 template <typename TN>
 __global__ __launch_bounds__(256) void k_momentum_prep(const MomentumPrepParams p) {
+  prefetch_args<sizeof(p)>();
   __shared__ float red[16];
   __shared__ __attribute__((aligned(16))) TN tile[TallTile<TN>::C * TallTile<TN>::LD];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
@@ -301,6 +304,7 @@ struct NsScaleParams {
 // Grid (chunks, Newton-Schulz matrices).  ss_part is indexed by packed matrix.
 template <typename TN>
 __global__ void k_ns_scale(const NsScaleParams p) {
+  prefetch_args<sizeof(p)>();
   const int m = blockIdx.y;
   clear_words(p.clear, blockIdx.x == 0 && blockIdx.y == 0);
   float ss = 0.f;
@@ -403,6 +407,7 @@ constexpr int ROW_VEC_MAX = 4;   // a lane keeps up to 4 x 4 elements of its row
 // (39 MB, 4.2 TB/s) and 10.1 us from two; as two kernels they took 8.2 + 5.8 us.
 template <typename T>
 __global__ void k_update_renorm(const RenormParams p) {
+  prefetch_args<sizeof(p)>();
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
   if (row >= p.g.rows(j)) return;
@@ -463,6 +468,7 @@ __global__ void k_update_renorm(const RenormParams p) {
 // as two kernels.  T: compute type of gc.
 template <typename T, typename TN>
 __global__ void k_renorm_bwd(const RenormParams p) {
+  prefetch_args<sizeof(p)>();
   __shared__ float red[16];
   const int z = blockIdx.y, j = z / p.g.nb;
   const int row = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6), lane = threadIdx.x & 63;
@@ -636,6 +642,7 @@ struct GradPrepParams {
 };
 template <typename T, typename TN>
 __global__ __launch_bounds__(256) void k_grad_prep(const GradPrepParams p) {
+  prefetch_args<sizeof(p)>();
   __shared__ float red[16];
   __shared__ __attribute__((aligned(16))) float tx[TallTile<float>::C * TallTile<float>::LD];
   __shared__ __attribute__((aligned(16))) TN tg[TallTile<TN>::C * TallTile<TN>::LD];
@@ -759,6 +766,7 @@ struct FinishParams {
   float* out[3];
 };
 __global__ void k_finish_weight_grads(const FinishParams p) {
+  prefetch_args<sizeof(p)>();
   // flat over a matrix, 4 consecutive elements per thread (a row holds a multiple of 4): every lane works
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   const long long e = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
@@ -800,6 +808,7 @@ struct ZeroSegments {
   long long bs[16], off[16], len[16];
 };
 __global__ void k_zero_segments(const ZeroSegments z) {
+  prefetch_args<sizeof(z)>();
   const int i = blockIdx.z;
   const long long e = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 16;
   if (e >= z.len[i]) return;

@@ -29,9 +29,6 @@
 #pragma once
 #include "gemm_dma.h"
 
-// a lambda of many lines with several calls stays a function of its own otherwise, its captures in memory
-#define LACT_INLINE_LAMBDA __attribute__((always_inline))
-
 namespace lact {
 
 struct WindowAttnParams {
@@ -78,8 +75,7 @@ struct AttnCopy {
   const uint16_t* base;           // the head's first row that the tiles cover
   int step, last;
   __device__ __forceinline__ void init(int wave, const uint16_t* head, int ld, int first, int n, int L) {
-    const uint64_t a = reinterpret_cast<uint64_t>(head + (size_t)first * ld);   // in scalar registers, wherever it was computed
-    base = reinterpret_cast<const uint16_t*>((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)a) | (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(a >> 32)) << 32);
+    base = uniform(head + (size_t)first * ld);
     step = 64 * ld; last = n - 1;
     const int rows = L - 1 - (first + last * 64);
 #pragma unroll

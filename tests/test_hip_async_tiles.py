@@ -246,6 +246,39 @@ def test_wide_hidden_tiles_have_the_same_bits(b, d, dh, T):
         assert torch.isfinite(a.float()).all() and torch.equal(a, r)
 
 
+# 64 x 64 tiles of the hidden stages and of the row GEMMs: 224 and 224, 256 and 256, 255 and 85 (dh = 136: the last half tile holds eight
+# units), 270 and 90; an update of 70 tokens among long ones, which takes the tiles of the longest
+@pytest.mark.parametrize("b,d,dh,T,last,half", [(14, 128, 128, 512, 512, {"hidden", "rows"}), (16, 128, 128, 512, 70, set()),
+                                                (17, 40, 136, 265, 265, {"hidden", "rows"}), (18, 40, 136, 300, 70, {"rows"}),
+                                                (3, 72, 104, 333, 70, {"hidden", "rows"})])
+def test_half_tiles_against_oracle(b, d, dh, T, last, half):
+    """fp32 launches on either side of the number of tiles below which half tiles are taken: forward and backward, the learning rates'
+    gradients (sums over the columns of a tile) among them."""
+    print("[gpu-test] half tiles", b, d, dh, T, last, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    L = T + last
+    inp = O.make_inputs(b, L, d, dh, seed=39, act_dtype=torch.float32)
+    go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(9))
+    prog = ops.Program(steps=((LACT_UPDATE, 0, T, 0), (LACT_APPLY, 0, T, 0), (LACT_UPDATE, T, L, 0), (LACT_APPLY, T, L, T)), out_len=L)
+    steps = [O.Step(O.UPDATE, 0, T), O.Step(O.APPLY, 0, T), O.Step(O.UPDATE, T, L), O.Step(O.APPLY, T, L)]
+
+    def step():
+        dev = [inp[n].to("cuda").requires_grad_(True) for n in ORDER]
+        out, _, _ = ops.run_program(prog, *dev)
+        return [out] + list(torch.autograd.grad(out, dev, go.to("cuda")))
+
+    res, names = kernels(step)
+    assert ("k_update_bwd_hidden<half>" in names) == ("hidden" in half) and ("k_update_bwd_hidden" in names) == ("hidden" not in half)
+    # the update's products of the short second one are few whatever the first one's are
+    assert any(n.startswith("k_row_gemm<") and n.endswith(",half>") for n in names) == ("rows" in half or last < T)
+    cpu = [inp[n].clone().requires_grad_(True) for n in ORDER]
+    ref, _, _ = O.run_program(*cpu[:9], steps, num=O.Numerics(autocast=False), momentum=cpu[9])
+    refs = [ref] + list(torch.autograd.grad(ref, cpu, go))
+    for n, a, r in zip(("out",) + ORDER, res, refs):
+        assert O.rel_l2(a, r) < 1e-4, n       # the bound of test_small_tiles_against_oracle
+
+
 def same_specials(a, r):
     a, r = a.detach().float().cpu(), r.detach().float()
     assert torch.isinf(r).any()

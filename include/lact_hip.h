@@ -122,6 +122,18 @@ int lact_backward(const lact_desc_t* desc, const void* q, const void* k, const v
                   float* dw2, void* dq, void* dk, void* dv, float* dlr0, float* dlr1, float* dlr2,
                   float* dmomentum, void* stream);
 
+/* lact_forward and lact_backward where batch entries share initial weights: w0, w1, w2 hold n_weights matrices each, which divides
+ * desc->b, and batch entry i starts from matrix i % n_weights; dw0, dw1, dw2 hold as many, each the sum over its entries.  What a
+ * layer's parameters [heads, ...] are to its batch of sequences (bidirectional_lact_layer.py:259-261 repeats them).  Final weights,
+ * momentum states and everything else keep one matrix per entry. */
+int lact_forward_shared_weights(const lact_desc_t* desc, int32_t n_weights, const float* w0, const float* w1, const float* w2, const void* q,
+                                const void* k, const void* v, const float* lr0, const float* lr1, const float* lr2, const float* momentum,
+                                void* out, float* const w_out[3], float* const m_out[3], void* saved, void* scratch, void* stream);
+int lact_backward_shared_weights(const lact_desc_t* desc, int32_t n_weights, const void* q, const void* k, const void* v, const float* lr0,
+                                 const float* lr1, const float* lr2, const float* momentum, const void* dout, const float* const dw_final[3],
+                                 const void* saved, void* scratch, float* dw0, float* dw1, float* dw2, void* dq, void* dk, void* dv, float* dlr0,
+                                 float* dlr1, float* dlr2, float* dmomentum, void* stream);
+
 /* zeropower_via_newtonschulz5 (ttt_operation.py:30-66; with a repeated coefficient triple:
  * lact_ttt.py:33-67, functions.py:38-72).  g, out: [n, rows, cols] fp32. */
 size_t lact_newton_schulz_workspace_bytes(int32_t n, int32_t rows, int32_t cols, int32_t steps);

@@ -36,6 +36,7 @@ class Desc(Structure):
 
 OPT_STREAM_OVERLAP, OPT_FUSED_NEWTON_SCHULZ, OPT_NS_BARRIER_SPIN_LIMIT, OPT_PERSISTENT_TILES, OPT_KEEP_PREACTIVATIONS = 0, 1, 2, 3, 4
 EXPORTS = ("lact_last_error", "lact_version", "lact_query_sizes", "lact_forward", "lact_forward_from_state", "lact_backward",
+           "lact_forward_shared_weights", "lact_backward_shared_weights",
            "lact_newton_schulz_workspace_bytes", "lact_newton_schulz", "lact_newton_schulz_static_capacity",
            "lact_newton_schulz_static", "lact_newton_schulz_backward_workspace_bytes", "lact_newton_schulz_backward",
            "lact_check_async_error", "lact_mfma_calibration", "lact_set_option", "lact_profile_enable",
@@ -86,6 +87,10 @@ def lib():
     L.lact_forward_from_state.restype = c_int32
     L.lact_backward.argtypes = [POINTER(Desc)] + [vp] * 8 + [POINTER(vp), vp, vp] + [vp] * 10 + [vp]
     L.lact_backward.restype = c_int32
+    L.lact_forward_shared_weights.argtypes = [POINTER(Desc), c_int32] + [vp] * 10 + [vp, POINTER(vp), POINTER(vp), vp, vp, vp]
+    L.lact_forward_shared_weights.restype = c_int32
+    L.lact_backward_shared_weights.argtypes = [POINTER(Desc), c_int32] + [vp] * 8 + [POINTER(vp), vp, vp] + [vp] * 10 + [vp]
+    L.lact_backward_shared_weights.restype = c_int32
     L.lact_newton_schulz_workspace_bytes.argtypes = [c_int32] * 4
     L.lact_newton_schulz_workspace_bytes.restype = c_size_t
     L.lact_newton_schulz.argtypes = [c_int32, c_int32, c_int32, vp, vp, c_int32, POINTER(c_float), c_int32, vp, vp]

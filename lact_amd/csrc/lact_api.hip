@@ -956,7 +956,7 @@ struct Runner {
     {
       InitParams p;
       memset(&p, 0, sizeof(p));
-      p.g = P.g; p.w[0] = w0; p.w[1] = w1; p.w[2] = w2; p.n0 = n0();
+      p.g = P.g; p.w[0] = w0; p.w[1] = w1; p.w[2] = w2; p.nw = P.nw; p.n0 = n0();
       // a call without updates hands the weights back as they are; with bf16 activations nothing else reads the fp32 copy then
       p.wf = (P.bf16 && P.nupd == 0 && d.forward_only) ? nullptr : wf(0);
       p.wc = P.bf16 ? (void*)wc(0) : nullptr;
@@ -1767,8 +1767,8 @@ struct Runner {
       p.carry = (d.prenorm && carry_main >= 0) ? scr<float>(P.t_gwhat[carry_main]) : nullptr;
       p.gn0 = gn0; p.n0 = n0(); p.w_init = wf(0);
       p.through_norms = d.detach_norms ? 0 : 1;
-      p.out[0] = dw0; p.out[1] = dw1; p.out[2] = dw2;
-      LACT_LAUNCH("k_finish_weight_grads", "k_finish_weight_grads", 0.0, k_finish_weight_grads, eg, dim3(256), s, p);
+      p.out[0] = dw0; p.out[1] = dw1; p.out[2] = dw2; p.nw = P.nw;
+      LACT_LAUNCH("k_finish_weight_grads", "k_finish_weight_grads", 0.0, k_finish_weight_grads, dim3(eg.x, 3 * P.nw), dim3(256), s, p);
     }
     LACT_CHECK_LAUNCH();
     return 0;
@@ -2585,19 +2585,35 @@ int lact_query_sizes(const lact_desc_t* desc, size_t* saved_bytes, size_t* scrat
   return 0;
 }
 
+static int run_forward(const lact_desc_t* desc, int n_weights, const float* w0, const float* w1, const float* w2, const void* q, const void* k,
+                       const void* v, const float* lr0, const float* lr1, const float* lr2, const float* momentum, const float* const m_in[3],
+                       void* out, float* const w_out[3], float* const m_out[3], void* saved, void* scratch, void* stream);
+
 int lact_forward(const lact_desc_t* desc, const float* w0, const float* w1, const float* w2, const void* q, const void* k,
                  const void* v, const float* lr0, const float* lr1, const float* lr2, const float* momentum, void* out,
                  float* const w_out[3], float* const m_out[3], void* saved, void* scratch, void* stream) {
-  return lact_forward_from_state(desc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, nullptr, out, w_out, m_out, saved,
-                                 scratch, stream);
+  return run_forward(desc, 0, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, nullptr, out, w_out, m_out, saved, scratch, stream);
+}
+
+int lact_forward_shared_weights(const lact_desc_t* desc, int32_t n_weights, const float* w0, const float* w1, const float* w2, const void* q,
+                                const void* k, const void* v, const float* lr0, const float* lr1, const float* lr2, const float* momentum,
+                                void* out, float* const w_out[3], float* const m_out[3], void* saved, void* scratch, void* stream) {
+  if (n_weights < 1) return fail("the number of shared weights must be positive");
+  return run_forward(desc, n_weights, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, nullptr, out, w_out, m_out, saved, scratch, stream);
 }
 
 int lact_forward_from_state(const lact_desc_t* desc, const float* w0, const float* w1, const float* w2, const void* q,
                             const void* k, const void* v, const float* lr0, const float* lr1, const float* lr2,
                             const float* momentum, const float* const m_in[3], void* out, float* const w_out[3],
                             float* const m_out[3], void* saved, void* scratch, void* stream) {
+  return run_forward(desc, 0, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m_in, out, w_out, m_out, saved, scratch, stream);
+}
+
+static int run_forward(const lact_desc_t* desc, int n_weights, const float* w0, const float* w1, const float* w2, const void* q, const void* k,
+                       const void* v, const float* lr0, const float* lr1, const float* lr2, const float* momentum, const float* const m_in[3],
+                       void* out, float* const w_out[3], float* const m_out[3], void* saved, void* scratch, void* stream) {
   Plan P;
-  if (P.build(desc)) return -1;
+  if (P.build(desc, n_weights)) return -1;
   if (P.state_in && (!m_in || !m_in[0] || !m_in[1] || !m_in[2])) return fail("momentum_state_in set but a state pointer is null");
   if (!P.state_in && m_in) return fail("momentum state passed without momentum_state_in in the descriptor");
   if (check_ptrs({w0, w1, w2, q, out, saved, scratch}, "forward tensors")) return -1;
@@ -2619,12 +2635,12 @@ int lact_forward_from_state(const lact_desc_t* desc, const float* w0, const floa
 #undef LACT_FWD
 }
 
-int lact_backward(const lact_desc_t* desc, const void* q, const void* k, const void* v, const float* lr0, const float* lr1,
-                  const float* lr2, const float* momentum, const void* dout, const float* const dw_final[3], const void* saved,
-                  void* scratch, float* dw0, float* dw1, float* dw2, void* dq, void* dk, void* dv, float* dlr0, float* dlr1,
-                  float* dlr2, float* dmomentum, void* stream) {
+static int run_backward(const lact_desc_t* desc, int n_weights, const void* q, const void* k, const void* v, const float* lr0, const float* lr1,
+                        const float* lr2, const float* momentum, const void* dout, const float* const dw_final[3], const void* saved,
+                        void* scratch, float* dw0, float* dw1, float* dw2, void* dq, void* dk, void* dv, float* dlr0, float* dlr1,
+                        float* dlr2, float* dmomentum, void* stream) {
   Plan P;
-  if (P.build(desc)) return -1;
+  if (P.build(desc, n_weights)) return -1;
   if (P.d.forward_only) return fail("the forward ran with forward_only set: nothing was kept for a backward pass");
   if (check_ptrs({q, dout, saved, scratch, dw0, dw1, dw2, dq}, "backward tensors")) return -1;
   if (P.nupd > 0 && check_ptrs({k, v, lr0, lr1, lr2, dk, dv, dlr0, dlr1, dlr2}, "k, v, lr and their gradients")) return -1;
@@ -2646,6 +2662,23 @@ int lact_backward(const lact_desc_t* desc, const void* q, const void* k, const v
   if (!ns32) LACT_BWD(float, uint16_t)
   LACT_BWD(float, float)
 #undef LACT_BWD
+}
+
+int lact_backward(const lact_desc_t* desc, const void* q, const void* k, const void* v, const float* lr0, const float* lr1,
+                  const float* lr2, const float* momentum, const void* dout, const float* const dw_final[3], const void* saved,
+                  void* scratch, float* dw0, float* dw1, float* dw2, void* dq, void* dk, void* dv, float* dlr0, float* dlr1,
+                  float* dlr2, float* dmomentum, void* stream) {
+  return run_backward(desc, 0, q, k, v, lr0, lr1, lr2, momentum, dout, dw_final, saved, scratch, dw0, dw1, dw2, dq, dk, dv, dlr0, dlr1, dlr2,
+                      dmomentum, stream);
+}
+
+int lact_backward_shared_weights(const lact_desc_t* desc, int32_t n_weights, const void* q, const void* k, const void* v, const float* lr0,
+                                 const float* lr1, const float* lr2, const float* momentum, const void* dout, const float* const dw_final[3],
+                                 const void* saved, void* scratch, float* dw0, float* dw1, float* dw2, void* dq, void* dk, void* dv, float* dlr0,
+                                 float* dlr1, float* dlr2, float* dmomentum, void* stream) {
+  if (n_weights < 1) return fail("the number of shared weights must be positive");
+  return run_backward(desc, n_weights, q, k, v, lr0, lr1, lr2, momentum, dout, dw_final, saved, scratch, dw0, dw1, dw2, dq, dk, dv, dlr0, dlr1, dlr2,
+                      dmomentum, stream);
 }
 
 size_t lact_newton_schulz_workspace_bytes(int32_t n, int32_t rows, int32_t cols, int32_t steps) {

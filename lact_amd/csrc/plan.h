@@ -115,6 +115,7 @@ struct Plan {
   std::vector<float> coeffs;
   MatGeom g;
   int nupd = 0, Tcap = 0, Tupd = 1, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 1024, kl_begin = 0, kl_end = 0, side_slots = 1;
+  int nw = 0;       // initial weights and their gradients: matrices of each kind, batch entry i uses i % nw
   bool muon = false, bf16 = true, momentum = false, state_in = false;
   size_t mat3 = 0;  // 3*b*elems
   // saved
@@ -131,10 +132,13 @@ struct Plan {
   size_t t_h[6], t_partial, t_lrpart, t_xf[2], t_xbtmp, t_ss, t_dot, t_mdot, t_gwhat[2], t_gwcur, t_gmcarry, t_gc,
       t_gxf[2], t_gxb[2], t_sg, t_gas, t_gn0, t_hs[3], t_hn[3], t_partial_side, t_gwside, t_nssync, t_kl[2], t_ca, scratch_bytes;
 
-  int build(const lact_desc_t* desc) {
+  // n_weights: matrices of each kind that the batch entries share, 0: every entry has its own
+  int build(const lact_desc_t* desc, int n_weights = 0) {
     if (!desc) return fail("null descriptor");
     d = *desc;
     if (d.b <= 0 || d.d <= 0 || d.dh <= 0) return fail("b, d, dh must be positive");
+    if (n_weights < 0 || (n_weights > 0 && d.b % n_weights)) return fail("the number of shared weights must divide b");
+    nw = n_weights > 0 ? n_weights : d.b;
     if (d.d % 8 || d.dh % 8) return fail("d and dh must be multiples of 8");
     if (d.act_dtype != LACT_BF16 && d.act_dtype != LACT_F32) return fail("act_dtype must be LACT_BF16 or LACT_F32");
     bf16 = d.act_dtype == LACT_BF16;

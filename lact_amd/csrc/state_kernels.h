@@ -71,7 +71,8 @@ struct FlatRange {
 // ---- init: row norms of the initial weights, fp32 state copy, compute-type copy -----------------
 struct InitParams {
   MatGeom g;
-  const float* w[3];      // [b, rows, cols] each; transposed: [b, cols, rows]
+  const float* w[3];      // [nw, rows, cols] each; transposed: [nw, cols, rows]
+  int nw;                 // batch entry i starts from matrix i % nw
   float* n0;              // [3b][maxrows]
   float* wf;              // [3b][elems], or null when no update reads it
   void* wc;               // [3b][elems] compute type, or null when the compute type is fp32
@@ -91,7 +92,7 @@ __global__ void k_init_state(const InitParams p) {
   if (row >= p.g.rows(j)) return;
   const int cols = p.g.cols(j);
   const size_t in_batch = (size_t)ib * p.g.elems + (size_t)row * cols;
-  const float* src = p.w[j] + in_batch;
+  const float* src = p.w[j] + (size_t)(ib % p.nw) * p.g.elems + (size_t)row * cols;
   const size_t o = (size_t)z * p.g.elems + (size_t)row * cols;
   float ss = 0.f;
   for (int c = lane * 4; c < cols; c += 256) {
@@ -113,7 +114,7 @@ __global__ __launch_bounds__(256) void k_init_state_transposed(const InitParams 
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb, row0 = blockIdx.x * 32;
   const int rows = p.g.rows(j), cols = p.g.cols(j);
   if (row0 >= rows) return;
-  const float* src = p.w[j] + (size_t)ib * p.g.elems;
+  const float* src = p.w[j] + (size_t)(ib % p.nw) * p.g.elems;
   const int lc = threadIdx.x >> 3, lr = (threadIdx.x & 7) * 4;          // load: column lc (+ 32 i), four rows from lr
   const int sr = threadIdx.x >> 4, scol = (threadIdx.x & 15) * 4;       // store: row sr (+ 16), four columns from scol
   float ss[2] = {0.f, 0.f};
@@ -763,33 +764,40 @@ struct FinishParams {
   MatGeom g;
   const float* gw; const float* gw2; Partials gwp; const float* carry; const float* gn0; const float* n0; const float* w_init;   // gw, gw2, gwp: addends, nullable
   int through_norms;
-  float* out[3];
+  float* out[3];          // [nw, rows, cols] each
+  int nw;                 // matrices: where fewer than batch entries, a gradient is the sum over the entries i, i + nw, ...
 };
 __global__ void k_finish_weight_grads(const FinishParams p) {
   prefetch_args<sizeof(p)>();
   // flat over a matrix, 4 consecutive elements per thread (a row holds a multiple of 4): every lane works
-  const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
+  const int j = blockIdx.y / p.nw, iw = blockIdx.y % p.nw;
   const long long e = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (e >= p.g.elems) return;
   const int cols = p.g.cols(j), row = (int)(e / cols);
-  const size_t o = (size_t)z * p.g.elems + e;
-  float4 v = p.gw ? ld4(p.gw + o) : f4(0.f, 0.f, 0.f, 0.f);
-  if (p.gw2) {
-    const float4 t = ld4(p.gw2 + o);
-    v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
+  float4 sum = f4(0.f, 0.f, 0.f, 0.f);
+  for (int ib = iw; ib < p.g.nb; ib += p.nw) {
+    const int z = j * p.g.nb + ib;
+    const size_t o = (size_t)z * p.g.elems + e;
+    float4 v = p.gw ? ld4(p.gw + o) : f4(0.f, 0.f, 0.f, 0.f);
+    if (p.gw2) {
+      const float4 t = ld4(p.gw2 + o);
+      v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
+    }
+    add_partials(v, p.gwp, o);
+    if (p.carry) {
+      const float4 t = ld4(p.carry + o);
+      v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
+    }
+    if (p.through_norms) {
+      const float n = p.n0[(size_t)z * p.g.maxrows() + row];
+      const float c = n > 0.f ? p.gn0[(size_t)z * p.g.maxrows() + row] / n : 0.f;
+      const float4 w = ld4(p.w_init + o);
+      v.x += c * w.x; v.y += c * w.y; v.z += c * w.z; v.w += c * w.w;
+    }
+    if (ib == iw) sum = v;
+    else { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; }
   }
-  add_partials(v, p.gwp, o);
-  if (p.carry) {
-    const float4 t = ld4(p.carry + o);
-    v.x += t.x; v.y += t.y; v.z += t.z; v.w += t.w;
-  }
-  if (p.through_norms) {
-    const float n = p.n0[(size_t)z * p.g.maxrows() + row];
-    const float c = n > 0.f ? p.gn0[(size_t)z * p.g.maxrows() + row] / n : 0.f;
-    const float4 w = ld4(p.w_init + o);
-    v.x += c * w.x; v.y += c * w.y; v.z += c * w.z; v.w += c * w.w;
-  }
-  st4(p.out[j] + (size_t)ib * p.g.elems + e, v);
+  st4(p.out[j] + (size_t)iw * p.g.elems + e, sum);
 }
 
 // the three caller tensors (null: zeros) -> [3b][elems], 4 elements per thread

@@ -114,19 +114,21 @@ lact_desc_t describe(const Schedule& sc, int64_t b, int64_t d, int64_t dh, const
 
 struct Operands {      // what a forward call hands to its backward
   Tensor q, k, v, lr0, lr1, lr2, momentum, saved;
-  int64_t b = 0, d = 0, dh = 0;
+  int64_t b = 0, nw = 0, d = 0, dh = 0;
 };
 
 // Returns the output, the three final weights (when the schedule returns its state) and the three momentum states (when it
 // does and there is momentum).
 std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& w1, const Tensor& w2, const Tensor& q, const OptTensor& k,
                             const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1, const OptTensor& lr2, const OptTensor& momentum,
-                            const std::vector<Tensor>& m_state, bool needs_backward, Operands* keep) {
+                            const std::vector<Tensor>& m_state, bool needs_backward, bool shared, Operands* keep) {
   if (!q.is_cuda()) throw std::runtime_error("lact_amd runs on an MI355X only: tensors must be on a HIP device (no CPU path)");
   const c10::hip::HIPGuard guard(q.device().index());
-  const int64_t b = w0.size(0), dh = w0.size(1), d = w0.size(2);
-  if (w1.sizes() != at::IntArrayRef({b, d, dh}) || w2.sizes() != at::IntArrayRef({b, dh, d}))
+  const int64_t nw = w0.size(0), dh = w0.size(1), d = w0.size(2), b = shared && q.dim() > 0 ? q.size(0) : nw;
+  if (w1.sizes() != at::IntArrayRef({nw, d, dh}) || w2.sizes() != at::IntArrayRef({nw, dh, d}))
     throw std::invalid_argument("expected w0, w2: [b, dh, d] and w1: [b, d, dh] with equal key and value dims");
+  if (shared && (nw < 1 || b % nw || sc.return_state || !m_state.empty()))
+    throw std::invalid_argument("shared weights: their number must divide the batch, and no state is carried in or out");
   // the kernels take raw pointers: a tensor elsewhere, or too small for the steps, has to be refused here
   auto same_device = [&](const Tensor& t) { return t.device() == q.device(); };
   auto here = [&](const OptTensor& t) { return !t || same_device(*t); };
@@ -139,7 +141,7 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
   auto act = (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kHalf) ? at::kBFloat16 : at::kFloat;
   if (at::autocast::is_autocast_enabled(at::kCUDA)) act = at::kBFloat16;
   Operands o;
-  o.b = b; o.d = d; o.dh = dh;
+  o.b = b; o.nw = nw; o.d = d; o.dh = dh;
   o.q = rows_view(q, act);
   if (sc.has_update) {
     if (!k || !v || !lr0 || !lr1 || !lr2) throw std::invalid_argument("a schedule with an update needs k, v and the three learning rates");
@@ -189,7 +191,10 @@ std::vector<Tensor> forward(const Schedule& sc, const Tensor& w0, const Tensor& 
       for (int i = 0; i < 3; ++i) m_out[i] = fptr(res[4 + i]);
   }
   const float* m_ptr[3] = {fptr(m_in[0]), fptr(m_in[1]), fptr(m_in[2])};
-  check(lact_forward_from_state(&D, fptr(w[0]), fptr(w[1]), fptr(w[2]), ptr(o.q), ptr(o.k), ptr(o.v), fptr(o.lr0), fptr(o.lr1), fptr(o.lr2),
+  if (shared)
+    check(lact_forward_shared_weights(&D, (int)nw, fptr(w[0]), fptr(w[1]), fptr(w[2]), ptr(o.q), ptr(o.k), ptr(o.v), fptr(o.lr0), fptr(o.lr1), fptr(o.lr2),
+                                      fptr(o.momentum), ptr(out), w_out, m_out, ptr(o.saved), ptr(scratch), c10::hip::getCurrentHIPStream().stream()));
+  else check(lact_forward_from_state(&D, fptr(w[0]), fptr(w[1]), fptr(w[2]), ptr(o.q), ptr(o.k), ptr(o.v), fptr(o.lr0), fptr(o.lr1), fptr(o.lr2),
                                 fptr(o.momentum), carried ? m_ptr : nullptr, ptr(out), w_out, m_out, ptr(o.saved), ptr(scratch),
                                 c10::hip::getCurrentHIPStream().stream()));
   auto out_dtype = (q.scalar_type() == at::kBFloat16 || q.scalar_type() == at::kFloat) ? q.scalar_type() : act;
@@ -225,20 +230,20 @@ std::vector<OptTensor> refuse_second_derivative_py(std::vector<OptTensor> grads)
 // What the backward of one call needs beside the saved tensors.
 struct CallRecord : torch::CustomClassHolder {
   c10::intrusive_ptr<Schedule> sc;
-  int64_t b = 0, d = 0, dh = 0;
+  int64_t b = 0, nw = 0, d = 0, dh = 0;
   at::ScalarType dtype[8];                 // of w0, w1, w2, q, k, v, the rates, momentum
   std::vector<int64_t> lr_shape, m_shape;
 };
 
 struct ProgramFn : torch::autograd::Function<ProgramFn> {
-  static variable_list forward(AutogradContext* ctx, c10::intrusive_ptr<Schedule> sc, const Tensor& w0, const Tensor& w1, const Tensor& w2,
+  static variable_list forward(AutogradContext* ctx, c10::intrusive_ptr<Schedule> sc, bool shared, const Tensor& w0, const Tensor& w1, const Tensor& w2,
                                const Tensor& q, const OptTensor& k, const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1,
                                const OptTensor& lr2, const OptTensor& momentum) {
     Operands o;
-    auto res = ::forward(*sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, {}, true, &o);
+    auto res = ::forward(*sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, {}, true, shared, &o);
     auto rec = c10::make_intrusive<CallRecord>();
     rec->sc = sc;
-    rec->b = o.b; rec->d = o.d; rec->dh = o.dh;
+    rec->b = o.b; rec->nw = o.nw; rec->d = o.d; rec->dh = o.dh;
     auto type = [](const OptTensor& t) { return t ? t->scalar_type() : at::kFloat; };
     const at::ScalarType types[8] = {type(w0), type(w1), type(w2), type(q), type(k), type(v), type(lr0), type(momentum)};
     std::copy(types, types + 8, rec->dtype);
@@ -258,7 +263,7 @@ struct ProgramFn : torch::autograd::Function<ProgramFn> {
     const auto capsule = ctx->saved_data["call"].toCapsule();
     const auto& rec = static_cast<const CallRecord&>(*capsule);
     const Schedule& sc = *rec.sc;
-    const int64_t b = rec.b, d = rec.d, dh = rec.dh;
+    const int64_t b = rec.b, nw = rec.nw, d = rec.d, dh = rec.dh;
     const c10::hip::HIPGuard guard(q.device().index());
     const auto act_opt = q.options(), f32 = act_opt.dtype(at::kFloat);
     Tensor g_out = grads[0].defined() ? rows_view(grads[0], q.scalar_type()) : at::zeros({b, sc.out_len, d}, act_opt);
@@ -275,7 +280,7 @@ struct ProgramFn : torch::autograd::Function<ProgramFn> {
     check(lact_query_sizes(&D, &saved_bytes, &scratch_bytes));
     const Tensor scratch = at::empty({(int64_t)scratch_bytes}, act_opt.dtype(at::kByte));
     // lact_backward writes every element of its outputs (rows no step touches are zeroed by the library)
-    const Tensor dw[3] = {at::empty({b, dh, d}, f32), at::empty({b, d, dh}, f32), at::empty({b, dh, d}, f32)};
+    const Tensor dw[3] = {at::empty({nw, dh, d}, f32), at::empty({nw, d, dh}, f32), at::empty({nw, dh, d}, f32)};
     const Tensor dq = at::empty({b, q.size(1), d}, act_opt);
     Tensor dk, dv, dlr[3], dm;
     if (sc.has_update) {
@@ -284,11 +289,11 @@ struct ProgramFn : torch::autograd::Function<ProgramFn> {
       for (auto& x : dlr) x = at::empty({b, k.size(1)}, f32);
       if (momentum.defined()) dm = at::empty({b, k.size(1)}, f32);
     }
-    check(lact_backward(&D, ptr(q), ptr(k), ptr(v), fptr(t[3]), fptr(t[4]), fptr(t[5]), fptr(momentum), ptr(g_out), gwp, ptr(saved),
+    check(lact_backward_shared_weights(&D, (int)nw, ptr(q), ptr(k), ptr(v), fptr(t[3]), fptr(t[4]), fptr(t[5]), fptr(momentum), ptr(g_out), gwp, ptr(saved),
                         ptr(scratch), fptr(dw[0]), fptr(dw[1]), fptr(dw[2]), ptr(dq), ptr(dk), ptr(dv), fptr(dlr[0]), fptr(dlr[1]), fptr(dlr[2]),
                         fptr(dm), c10::hip::getCurrentHIPStream().stream()));
     auto type = [&](int i) { return rec.dtype[i]; };
-    variable_list res{Tensor(), cast(dw[0], type(0)), cast(dw[1], type(1)), cast(dw[2], type(2)), cast(dq, type(3)), cast(dk, type(4)), cast(dv, type(5))};
+    variable_list res{Tensor(), Tensor(), cast(dw[0], type(0)), cast(dw[1], type(1)), cast(dw[2], type(2)), cast(dq, type(3)), cast(dk, type(4)), cast(dv, type(5))};
     for (auto& x : dlr) res.push_back(x.defined() ? cast(x.reshape(rec.lr_shape), type(6)) : x);
     res.push_back(dm.defined() ? cast(dm.reshape(rec.m_shape), type(7)) : dm);
     if (twice) refuse_second_derivative(res);
@@ -305,7 +310,7 @@ bool any_tangent(const Ts&... ts) { return (has_tangent(ts) || ...); }
 // (out, w0, w1, w2, m0, m1, m2), None where there is nothing to return
 py::tuple run_program(const c10::intrusive_ptr<Schedule>& sc, const Tensor& w0, const Tensor& w1, const Tensor& w2, const Tensor& q,
                       const OptTensor& k, const OptTensor& v, const OptTensor& lr0, const OptTensor& lr1, const OptTensor& lr2,
-                      const OptTensor& momentum, const OptTensor& m0, const OptTensor& m1, const OptTensor& m2) {
+                      const OptTensor& momentum, const OptTensor& m0, const OptTensor& m1, const OptTensor& m2, bool shared) {
   // forward-mode differentiation knows nothing of a call that passes the autograd function by: the tangents would be dropped
   if (any_tangent(w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m0, m1, m2)) {
     PyErr_SetString(PyExc_NotImplementedError, "the operation has no forward-mode derivative (jvp)");
@@ -324,10 +329,10 @@ py::tuple run_program(const c10::intrusive_ptr<Schedule>& sc, const Tensor& w0, 
   {
     const py::gil_scoped_release nogil;
     if (needs_backward) {
-      res = ProgramFn::apply(sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum);
+      res = ProgramFn::apply(sc, shared, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum);
     } else {
       const at::AutoGradMode off(false);
-      res = forward(*sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m_state, false, nullptr);
+      res = forward(*sc, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m_state, false, shared, nullptr);
     }
   }
   py::tuple out(7);

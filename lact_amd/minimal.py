@@ -37,6 +37,10 @@ def bidirectional_lact_swiglu(w0, w1, w2, q, k, v, lr0, lr1, lr2, use_muon: bool
     """bidirectional_lact_layer.py:74-160: one update on every token, then apply to every query.
     muon_mode="reference" reproduces :139-146 (the orthogonalised gradient replaces the weight and the
     raw gradient is added); "intended" adds the orthogonalised gradient to the weight."""
+    return _bidirectional(w0, w1, w2, q, k, v, lr0, lr1, lr2, use_muon, muon_mode)
+
+
+def _bidirectional(w0, w1, w2, q, k, v, lr0, lr1, lr2, use_muon, muon_mode="reference", shared_weights=False):
     prog = _bidirectional_program(k.shape[1], q.shape[1], bool(use_muon), bool(use_muon and muon_mode == "reference"), ops._ns_mode(q))
-    out, _, _ = run_program(prog, w0, w1, w2, q, k, v, lr0, lr1, lr2, None)
+    out, _, _ = run_program(prog, w0, w1, w2, q, k, v, lr0, lr1, lr2, None, shared_weights=shared_weights)
     return out

@@ -83,12 +83,13 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 @torch.compiler.disable
-def run_program(prog: Program, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum=None, momentum_state=None):
+def run_program(prog: Program, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum=None, momentum_state=None, shared_weights=False):
     """Runs `prog`.  Returns (out, (w0, w1, w2) after the last update, (m0, m1, m2) momentum states; None each
     without momentum).
+    `shared_weights`: w0, w1, w2 hold fewer matrices than q has batch entries, and entry i starts from matrix i modulo their number.
     `momentum_state` = the (m0, m1, m2) of an earlier call: the first update continues from it (inference only)."""
     m0, m1, m2 = momentum_state if momentum_state is not None else (None, None, None)
-    res = _lib.host().run_program(prog.native(), w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m0, m1, m2)
+    res = _lib.host().run_program(prog.native(), w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, m0, m1, m2, shared_weights)
     return res[0], res[1:4], res[4:7]
 
 

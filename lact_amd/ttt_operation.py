@@ -36,9 +36,9 @@ def _block_causal_program(kv_len, q_len, chunk_size, use_muon, prenorm, ns_mode,
 
 
 def _block_causal(w0, w1, w2, q, k, v, lr0, lr1, lr2, chunk_size, use_muon, momentum, prenorm,
-                  muon_stacked=False, renorm_eps_in_sqrt=False):
+                  muon_stacked=False, renorm_eps_in_sqrt=False, shared_weights=False):
     prog = _block_causal_program(k.shape[1], q.shape[1], index(chunk_size), bool(use_muon), prenorm, ops._ns_mode(q), muon_stacked, renorm_eps_in_sqrt)
-    out, _, _ = run_program(prog, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum)
+    out, _, _ = run_program(prog, w0, w1, w2, q, k, v, lr0, lr1, lr2, momentum, shared_weights=shared_weights)
     return out
 
 

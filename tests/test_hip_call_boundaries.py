@@ -5,6 +5,7 @@ import torch
 
 from lact_amd import layers as HL
 from lact_amd import ops
+from oracle import lact_oracle as O
 from oracle.lact_oracle import rel_l2
 
 pytestmark = pytest.mark.gpu
@@ -187,3 +188,52 @@ def test_rows_further_apart_than_the_kernels_reach_are_copied():
     apart[3] = far[:, :16].unsqueeze(0)
     with torch.no_grad():
         assert torch.equal(ops.run_program(PROGRAM, *apart)[0], ops.run_program(PROGRAM, *args)[0])
+
+
+@pytest.mark.parametrize("dtype,nw,b,d,dh,L,C,muon,momentum", [
+    (torch.bfloat16, 3, 6, 64, 96, 300, 130, True, True), (torch.bfloat16, 1, 5, 128, 40, 250, 200, False, False),
+    (torch.float32, 2, 2, 40, 72, 150, 60, False, True), (torch.float32, 4, 12, 128, 32, 90, 40, True, False)])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_shared_weights_are_repeated_ones(dtype, nw, b, d, dh, L, C, muon, momentum, transposed):
+    """Batch entries that share initial weights: the bits of a call with the weights repeated, its weight gradients summed over the
+    entries (in fp32, one order against another: b / nw roundings of 2^-24 of the sum of magnitudes)."""
+    print("[gpu-test] shared weights", dtype, nw, b, d, dh, L, C, muon, momentum, transposed, flush=True)
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(b, L, d, dh, seed=51, act_dtype=dtype).items()}
+    ws = [inp[n][:nw].clone() for n in ("w0", "w1", "w2")]
+    if transposed:
+        ws = [w.transpose(1, 2).contiguous().transpose(1, 2) for w in ws]
+    rest = [inp[n] for n in ("q", "k", "v", "lr0", "lr1", "lr2")] + ([inp["momentum"]] if momentum else [])
+    go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(5)).to(dtype).to("cuda")
+    prog = ops.Program(steps=ops.block_causal_steps(L, C), out_len=L, return_state=False, ns_coeffs=ops.NS5_COEFFS if muon else None)
+    res = []
+    for shared in (True, False):
+        x = [w.detach().requires_grad_(True) for w in ws] + [t.clone().requires_grad_(True) for t in rest]
+        w = x[:3] if shared else [t.repeat(b // nw, 1, 1) for t in x[:3]]
+        if not shared and transposed:     # the layout of the other call's weights, and so the order of their row norms
+            w = [t.transpose(1, 2).contiguous().transpose(1, 2) for t in w]
+        out, _, _ = ops.run_program(prog, *w, *x[3:], shared_weights=shared)
+        with torch.no_grad():
+            again, _, _ = ops.run_program(prog, *w, *x[3:], shared_weights=shared)
+        if not shared:
+            for t in w:
+                t.retain_grad()
+        out.backward(go)
+        res.append(([out.detach(), again] + [t.grad for t in x[3:]], [t.grad for t in x[:3]], None if shared else [t.grad for t in w]))
+    for a, r in zip(res[0][0], res[1][0]):
+        assert torch.equal(a, r)
+    for a, each in zip(res[0][1], res[1][2]):
+        each = each.reshape(b // nw, nw, *each.shape[1:]).double()
+        assert a.dtype == torch.float32
+        assert bool(((a.double() - each.sum(0)).abs() <= b // nw * 2.0 ** -24 * each.abs().sum(0)).all())
+
+
+def test_shared_weights_are_refused_where_they_do_not_fit():
+    inp = {n: t.to("cuda") for n, t in O.make_inputs(4, 60, 32, 32, seed=52, act_dtype=torch.float32).items()}
+    rest = [inp[n] for n in ("q", "k", "v", "lr0", "lr1", "lr2")]
+    prog = ops.Program(steps=ops.block_causal_steps(60, 30), out_len=60, return_state=False)
+    with pytest.raises(ValueError):      # three matrices for four entries
+        ops.run_program(prog, *[inp[n][:3] for n in ("w0", "w1", "w2")], *rest, shared_weights=True)
+    with pytest.raises(ValueError):      # not asked for
+        ops.run_program(prog, *[inp[n][:2] for n in ("w0", "w1", "w2")], *rest)
+    with pytest.raises(ValueError):      # the state has one matrix per entry
+        ops.run_program(ops.Program(steps=prog.steps, out_len=60), *[inp[n][:2] for n in ("w0", "w1", "w2")], *rest, shared_weights=True)

@@ -866,18 +866,20 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
   const size_t slot = (size_t)bz * p.mat_elems;
   if (p.prep_d_out) {   // forward update, one split: momentum, bf16 copy and its sum of squares right here
     const int r0 = ST::row0(), c0 = ST::col0();
+    const bool tall = job.M > job.N;    // held transposed: written from the tile behind this pass
     float ss = 0.f;
     if (ST::active() && n0 + c0 < job.N) {
-      const char* src = smem + (r0 * ST::LD + c0) * 4;
+      char* src = smem + (r0 * ST::LD + c0) * 4;
       const size_t e0 = slot + (size_t)(m0 + r0) * job.N + n0 + c0, rstep = (size_t)ST::RPP * job.N;
-      const float mb = (p.prep_m_prev && p.prep_mbar) ? p.prep_mbar[ib] : 0.f;
+      const float* prev = p.prep_m_prev[j] ? p.prep_m_prev[j] + (size_t)ib * p.mat_elems + (e0 - slot) : nullptr;
+      const float mb = (prev && p.prep_mbar) ? p.prep_mbar[ib] : 0.f;
       float* ext = p.prep_m_ext[j] ? p.prep_m_ext[j] + (size_t)ib * p.mat_elems + (e0 - slot) : nullptr;
       float4 x4[ST::PASSES];
-      if (p.prep_m_prev) {
+      if (prev) {
 #pragma unroll
         for (int ps = 0; ps < ST::PASSES; ++ps) {
           const int r = r0 + ps * ST::RPP;
-          x4[ps] = (r < TS::BM && m0 + r < job.M) ? *reinterpret_cast<const float4*>(p.prep_m_prev + e0 + ps * rstep) : make_float4(0.f, 0.f, 0.f, 0.f);
+          x4[ps] = (r < TS::BM && m0 + r < job.M) ? *reinterpret_cast<const float4*>(prev + ps * rstep) : make_float4(0.f, 0.f, 0.f, 0.f);
         }
       }
       uint4 vg[8];
@@ -892,17 +894,34 @@ __device__ __forceinline__ void token_reduce_dma_block(const TokenReduceDmaParam
         if (r < TS::BM && m0 + r < job.M) {
           float4 v = __builtin_bit_cast(float4, vg[ps % 8]);
           v = make_float4(round_bf16(v.x), round_bf16(v.y), round_bf16(v.z), round_bf16(v.w));
-          if (p.prep_m_prev) {   // product and sum rounded separately, as the reference's two tensor operations are
+          if (prev) {   // product and sum rounded separately, as the reference's two tensor operations are
             v.x = __fadd_rn(v.x, __fmul_rn(x4[ps].x, mb)); v.y = __fadd_rn(v.y, __fmul_rn(x4[ps].y, mb));
             v.z = __fadd_rn(v.z, __fmul_rn(x4[ps].z, mb)); v.w = __fadd_rn(v.w, __fmul_rn(x4[ps].w, mb));
           }
           if (!p.prep_skip_d) *reinterpret_cast<float4*>(p.prep_d_out + e0 + ps * rstep) = v;
           if (ext) *reinterpret_cast<float4*>(ext + ps * rstep) = v;
           const float f0 = round_bf16(v.x), f1 = round_bf16(v.y), f2 = round_bf16(v.z), f3 = round_bf16(v.w);
-          Elem<uint16_t>::store4(p.prep_g16 + e0 + ps * rstep, f0, f1, f2, f3);
+          if (tall) *reinterpret_cast<float4*>(src + ps * ST::RPP * ST::LD * 4) = make_float4(f0, f1, f2, f3);
+          else Elem<uint16_t>::store4(p.prep_g16 + e0 + ps * rstep, f0, f1, f2, f3);
           ss += f0 * f0 + f1 * f1 + f2 * f2 + f3 * f3;
         }
       }
+    }
+    if (tall) {
+      // eight rows of a column a lane, eight such granules (128 bytes of the transposed matrix) and eight columns a wave
+      __syncthreads();
+      const int g0 = (threadIdx.x & 7), cw = threadIdx.x >> 3;
+      for (int c = cw; c < TS::BN && n0 + c < job.N; c += DMA_THREADS / 8) {
+        uint16_t* to = p.prep_g16 + slot + (size_t)(n0 + c) * job.M + m0;
+#pragma unroll
+        for (int g = g0; g < TS::BM / 8; g += 8) {
+          if (m0 + g * 8 >= job.M) continue;     // rows come in eights
+          const float* t = reinterpret_cast<const float*>(smem) + g * 8 * ST::LD + c;
+          *reinterpret_cast<uint4*>(to + g * 8) = make_uint4(pack_bf16(t[0], t[ST::LD]), pack_bf16(t[2 * ST::LD], t[3 * ST::LD]),
+                                                             pack_bf16(t[4 * ST::LD], t[5 * ST::LD]), pack_bf16(t[6 * ST::LD], t[7 * ST::LD]));
+        }
+      }
+      __syncthreads();
     }
     ss = block_sum(ss, reinterpret_cast<float*>(smem));
     if (threadIdx.x == 0) p.prep_ss_part[(size_t)bz * p.map.gy + tile] = ss;

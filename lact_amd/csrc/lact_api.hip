@@ -508,7 +508,11 @@ struct Runner {
   float* dsave(int u) const { return reinterpret_cast<float*>(sv + P.s_d) + (size_t)u * P.mat3; }
   // momentum state that update `u` starts from: the previous update's, or the one the caller carried in
   bool has_prev(int u) const { return P.momentum && (u > 0 || P.state_in); }
-  const float* mprev(int u) const { return !has_prev(u) ? nullptr : u > 0 ? dsave(u - 1) : reinterpret_cast<const float*>(sv + P.s_min); }
+  const float* carried[3] = {nullptr, nullptr, nullptr};    // of a forward call that starts from a state: [b][elems] each
+  void mprev(const float* (&m)[3], int u) const {
+    if (!has_prev(u)) return;
+    for (int j = 0; j < 3; ++j) m[j] = u > 0 ? dsave(u - 1) + (size_t)j * d.b * P.g.elems : carried[j];
+  }
   float* mbar(int u) const { return reinterpret_cast<float*>(sv + P.s_mbar) + (size_t)u * d.b; }
   float* usave(int u) const { return reinterpret_cast<float*>(sv + P.s_u) + (size_t)u * P.mat3; }
   TN* g16(int u) const { return reinterpret_cast<TN*>(sv + P.s_g16) + (size_t)u * P.mat3; }
@@ -822,7 +826,7 @@ struct Runner {
   // `prep` (forward update only): d_out / g16 / ss_part / m_prev / mbar of the momentum step; when the whole
   // reduction is one split of the asynchronous-copy kernel, its epilogue does that step and -1 is returned.
   struct PrepFold {
-    float* d_out; const float* m_prev; const float* mbar; uint16_t* g16; float* ss_part;
+    float* d_out; const float* m_prev[3]; const float* mbar; uint16_t* g16; float* ss_part;
     bool skip_d;
     float* m_ext[3];
     ClearWords clear;
@@ -875,9 +879,9 @@ struct Runner {
         direct = add_out && sp.n == 1;
         const bool folded = prep && sp.n == 1;
         if (folded) {
-          pd.prep_d_out = prep->d_out; pd.prep_m_prev = prep->m_prev; pd.prep_mbar = prep->mbar; pd.prep_skip_d = prep->skip_d ? 1 : 0;
+          pd.prep_d_out = prep->d_out; pd.prep_mbar = prep->mbar; pd.prep_skip_d = prep->skip_d ? 1 : 0;
           pd.prep_g16 = prep->g16; pd.prep_ss_part = prep->ss_part; pd.prep_clear = prep->clear;
-          for (int j = 0; j < 3; ++j) pd.prep_m_ext[j] = prep->m_ext[j];
+          for (int j = 0; j < 3; ++j) { pd.prep_m_prev[j] = prep->m_prev[j]; pd.prep_m_ext[j] = prep->m_ext[j]; }
         } else if (direct) { pd.add_out = add_out; pd.add_in = coeff != 0.f ? add_in : nullptr; pd.coeff = coeff; }
         else slots = sp.n;
         bool with_rows = rows != nullptr && rows->r4.N % 8 == 0 && rows->r2.N % 8 == 0;
@@ -947,12 +951,17 @@ struct Runner {
       entry = side->event();
       (void)hipEventRecord(entry, s_main);
     }
-    // carried momentum state: packed like every other state array (a device-to-device copy node when captured)
+    // carried momentum state: read where it lies (three copies took 18 us at 3 matrices of 768 x 1536 and two batch entries), but for one
+    // that 16-byte loads do not reach (a device-to-device copy node when captured)
     if (P.state_in && P.nupd > 0)
-      for (int j = 0; j < 3; ++j)
-        if (hipMemcpyAsync(sv + P.s_min + (size_t)j * d.b * P.g.elems * 4, m_in[j], (size_t)d.b * P.g.elems * 4,
-                           hipMemcpyDeviceToDevice, s) != hipSuccess)
+      for (int j = 0; j < 3; ++j) {
+        carried[j] = m_in[j];
+        if (reinterpret_cast<uintptr_t>(m_in[j]) % 16 == 0) continue;
+        char* to = sv + P.s_min + (size_t)j * d.b * P.g.elems * 4;
+        if (hipMemcpyAsync(to, m_in[j], (size_t)d.b * P.g.elems * 4, hipMemcpyDeviceToDevice, s) != hipSuccess)
           return fail("copy of the carried momentum state failed");
+        carried[j] = reinterpret_cast<const float*>(to);
+      }
     {
       InitParams p;
       memset(&p, 0, sizeof(p));
@@ -1078,14 +1087,14 @@ struct Runner {
         set_tr_term(jobs[1].t, vc, d.v_ld, d.v_bs, upd_z[1], d.dh, upd_zbs);
         jobs[2].M = d.dh; jobs[2].N = d.d;
         set_tr_term(jobs[2].t, upd_z[2], d.dh, upd_zbs, kl2, d.d, klbs);
-        // square shapes with Muon: the momentum step can ride in the reduction's epilogue (every tile exists for
-        // every matrix, and the Newton-Schulz orientation is the packed one)
+        // Muon: the momentum step rides in the reduction's epilogue where one split covers the tokens (every tile exists for every matrix).
+        // Three matrices of 768 x 1536 and two batch entries, two of three held transposed: 83 + 24 us as a pass of its own, 98 in it.
         PrepFold pf;
-        pf.skip_d = false;
-        const bool can_fold = kBf16 && kNsBf16 && P.muon && !P.g.stacked && d.d == d.dh;
+        memset(&pf, 0, sizeof(pf));
+        const bool can_fold = kBf16 && kNsBf16 && P.muon && !P.g.stacked;
         if (can_fold) {
           for (int j = 0; j < 3; ++j) pf.m_ext[j] = (u + 1 == P.nupd && P.momentum && m_out) ? m_out[j] : nullptr;
-          pf.d_out = dsave(u); pf.m_prev = mprev(u); pf.skip_d = d_unread;
+          pf.d_out = dsave(u); mprev(pf.m_prev, u); pf.skip_d = d_unread;
           pf.mbar = has_prev(u) ? mbar(u) : nullptr;
           pf.g16 = reinterpret_cast<uint16_t*>(g16(u)); pf.ss_part = scr<float>(P.t_ss);
           pf.clear.ptr = nullptr; pf.clear.n = 0;
@@ -1099,7 +1108,7 @@ struct Runner {
         MomentumPrepParams p;
         memset(&p, 0, sizeof(p));
         p.g = P.g; p.dw = partials(P.t_partial, dw_slots);
-        p.m_prev = mprev(u);
+        mprev(p.m_prev, u);
         p.mbar = has_prev(u) ? mbar(u) : nullptr;
         p.d_out = d_unread ? nullptr : dsave(u);
         p.g16 = g16(u);
@@ -1180,7 +1189,7 @@ struct Runner {
         if (!P.muon) {
           p.dw = partials(P.t_partial, dw_slots);
           p.round_dw_bf16 = P.bf16;
-          p.m_prev = mprev(u);
+          mprev(p.m_prev, u);
           p.mbar = has_prev(u) ? mbar(u) : nullptr;
           p.d_out = dsave(u);
           if (u + 1 == P.nupd && P.momentum && m_out)
@@ -1517,7 +1526,7 @@ struct Runner {
           p.gc = scr<T>(P.t_gc);
           p.gm_carry = carry_here ? gmcarry : nullptr; p.carry_valid = gm_valid; p.carry_write = u > 0;
           if (P.momentum && u > 0) {
-            p.m_prev = dsave(u - 1); p.mbar = mbar(u);
+            mprev(p.m_prev, u); p.mbar = mbar(u);
             p.mdot_part = scr<float>(P.t_mdot) + (size_t)u * mslot;
           }
         }

@@ -181,7 +181,7 @@ __device__ __forceinline__ void add_partials(float4& v, const Partials& q, size_
 }
 
 // The gradient of an update: the sum of its partial sums (at least one), rounded as the reference's bf16 GEMM result if asked, plus
-// the earlier momentum state weighted by mb (or m_prev null).
+// the earlier momentum state's quad at m_prev weighted by mb (or m_prev null).
 __device__ __forceinline__ float4 momentum4(const Partials& q, size_t off, int round, const float* m_prev, float mb) {
   float4 v = ld4(q.p + off);
   for (int i = 1; i < q.n; ++i) {
@@ -190,7 +190,7 @@ __device__ __forceinline__ float4 momentum4(const Partials& q, size_t off, int r
   }
   if (round) v = f4(round_bf16(v.x), round_bf16(v.y), round_bf16(v.z), round_bf16(v.w));
   if (m_prev) {
-    const float4 m = ld4(m_prev + off);
+    const float4 m = ld4(m_prev);
     // product and sum rounded separately, as the reference's two tensor operations are (ttt_operation.py:174-176)
     v.x = __fadd_rn(v.x, __fmul_rn(m.x, mb)); v.y = __fadd_rn(v.y, __fmul_rn(m.y, mb));
     v.z = __fadd_rn(v.z, __fmul_rn(m.z, mb)); v.w = __fadd_rn(v.w, __fmul_rn(m.w, mb));
@@ -200,7 +200,7 @@ __device__ __forceinline__ float4 momentum4(const Partials& q, size_t off, int r
 struct MomentumPrepParams {
   MatGeom g;
   Partials dw;                        // each [3b][elems]
-  const float* m_prev;                // [3b][elems] or null (no momentum / first update uses zeros)
+  const float* m_prev[3];             // [b][elems] each, or null (no momentum / first update uses zeros)
   const float* mbar;                  // [b] or null
   float* d_out;                       // [3b][elems]  dw (+ momentum): new momentum state, pre-Muon gradient (null: nothing reads it)
   float* m_ext[3];                    // caller's momentum outputs [b][elems] (same values as d_out), each nullable
@@ -252,14 +252,15 @@ __global__ __launch_bounds__(256) void k_momentum_prep(const MomentumPrepParams 
   __shared__ __attribute__((aligned(16))) TN tile[TallTile<TN>::C * TallTile<TN>::LD];
   const int z = blockIdx.y, j = z / p.g.nb, ib = z % p.g.nb;
   clear_words(p.clear, blockIdx.x == 0 && blockIdx.y == 0);
-  const float mb = (p.m_prev && p.mbar) ? p.mbar[ib] : 0.f;
+  const float* m_prev = p.m_prev[j] ? p.m_prev[j] + (size_t)ib * p.g.elems : nullptr;
+  const float mb = (m_prev && p.mbar) ? p.mbar[ib] : 0.f;
   const size_t zo = (size_t)z * p.g.elems;
   float* ext = p.m_ext[j] ? p.m_ext[j] + (size_t)ib * p.g.elems : nullptr;
   TN* g16 = reinterpret_cast<TN*>(p.g16) + p.g.ns_base(p.g.ns_of(z));
   float ss = 0.f;
   // one quad of the gradient: stored where it goes in its own orientation; returned as Newton-Schulz takes it
   auto quad = [&](long long e) {
-    const float4 v = momentum4(p.dw, zo + e, p.round_partial_bf16, p.m_prev, mb);
+    const float4 v = momentum4(p.dw, zo + e, p.round_partial_bf16, m_prev ? m_prev + e : nullptr, mb);
     if (p.d_out) st4(p.d_out + zo + e, v);
     if (ext) st4(ext + e, v);
     const float4 f = f4(Elem<TN>::rnd(v.x), Elem<TN>::rnd(v.y), Elem<TN>::rnd(v.z), Elem<TN>::rnd(v.w));
@@ -362,7 +363,7 @@ struct RenormParams {
   // sums and does the momentum step on the way (what k_momentum_prep does where a Newton-Schulz iteration follows)
   Partials dw;                     // partial sums of the gradient, or none: `u` is read
   int round_dw_bf16;               // the reduction GEMM's result is a bf16 tensor in the reference
-  const float* m_prev; const float* mbar;   // momentum state before this update and [b] mean momentum, or null
+  const float* m_prev[3]; const float* mbar;   // momentum state before this update ([b][elems] each) and [b] mean momentum, or null
   float* d_out;                    // the gradient with its momentum (= new momentum state), written
   float* m_ext[3];                 // caller's momentum outputs, each nullable
   // backward only
@@ -417,11 +418,12 @@ __global__ void k_update_renorm(const RenormParams p) {
   const size_t uo = (p.u_stacked ? (size_t)p.g.u_off(z) : (size_t)z * p.g.elems) + (size_t)row * cols;
   float* ext = p.w_ext[j] ? p.w_ext[j] + (size_t)ib * p.g.elems + (size_t)row * cols : nullptr;
   const bool keep = cols <= 256 * ROW_VEC_MAX;
-  const float mb = (p.m_prev && p.mbar) ? p.mbar[ib] : 0.f;
+  const float* m_prev = p.m_prev[j] ? p.m_prev[j] + (size_t)ib * p.g.elems + (size_t)row * cols : nullptr;
+  const float mb = (m_prev && p.mbar) ? p.mbar[ib] : 0.f;
   float* mext = p.m_ext[j] ? p.m_ext[j] + (size_t)ib * p.g.elems + (size_t)row * cols : nullptr;
   auto w_hat = [&](int c) {   // first visit of an element (a later one finds `u` = d_out in memory)
     if (p.dw.n == 0) return renorm_w_hat4(p, o + c, uo + c);
-    const float4 m = momentum4(p.dw, o + c, p.round_dw_bf16, p.m_prev, mb);
+    const float4 m = momentum4(p.dw, o + c, p.round_dw_bf16, m_prev ? m_prev + c : nullptr, mb);
     st4(p.d_out + o + c, m);
     if (mext) st4(mext + c, m);
     return renorm_w_hat4(p, o + c, m);
@@ -538,7 +540,7 @@ __global__ void k_renorm_bwd(const RenormParams p) {
           g.x += cv.x; g.y += cv.y; g.z += cv.z; g.w += cv.w;
         }
         if (p.carry_write) st4(p.gm_carry + o + c, f4(g.x * mb, g.y * mb, g.z * mb, g.w * mb));   // d/d M_prev of  dw + M_prev * mbar
-        if (p.m_prev) md += dot4(g, ld4(p.m_prev + o + c));
+        if (p.m_prev[j]) md += dot4(g, ld4(p.m_prev[j] + (size_t)ib * p.g.elems + (size_t)row * cols + c));
       }
       Elem<T>::store4(reinterpret_cast<T*>(p.gc) + o + c, g.x, g.y, g.z, g.w);
     }

@@ -315,3 +315,33 @@ def test_infinities_pass_the_ragged_end_of_a_contraction(dtype, d, T):
     _, refs, _ = O.run_program(*hot, [O.Step(O.UPDATE, 0, T), O.Step(O.APPLY, 0, T)], num=num, weight_norm=False)
     for a, r in zip(ws, refs):
         same_specials(a, r)
+
+
+# w0 and w2 held transposed (dh > d), w1 (d > dh); whole tiles of 192 and of 128, tiles that end inside one; one split of the tokens
+@pytest.mark.parametrize("b,d,dh,T", [(2, 256, 512, 1000), (1, 384, 192, 700), (3, 208, 328, 130), (1, 392, 144, 90), (1, 192, 576, 64)])
+@pytest.mark.parametrize("carried", [False, True])
+def test_momentum_step_of_matrices_held_transposed(b, d, dh, T, carried):
+    """The momentum step in the epilogue of the token reduction, without Newton-Schulz iterations behind it (they amplify a rounding):
+    returned weights and momentum states against the oracle, from a carried state (read where it lies) and without one."""
+    print("[gpu-test] folded momentum step", b, d, dh, T, carried, flush=True)
+    from lact_amd import ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    inp = O.make_inputs(b, T, d, dh, seed=61, act_dtype=torch.bfloat16)
+    g = torch.Generator().manual_seed(7)
+    state = [1e-3 * torch.randn(b, *s, generator=g) for s in ((dh, d), (d, dh), (dh, d))] if carried else None
+    num = O.Numerics(autocast=True)
+    prog = ops.Program(steps=((LACT_UPDATE, 0, T, 0), (LACT_APPLY, 0, T, 0)), out_len=T, ns_coeffs=())
+    dev = [inp[n].to("cuda") for n in ORDER]
+
+    def step():
+        with torch.no_grad():
+            return ops.run_program(prog, *dev, momentum_state=[m.to("cuda") for m in state] if carried else None)
+
+    (out, ws, ms), names = kernels(step)
+    assert "k_momentum_prep" not in names and any(n.startswith("k_token_reduce_dma") for n in names)
+    ref, wr, mr = O.run_program(*[inp[n] for n in ORDER[:9]], [O.Step(O.UPDATE, 0, T), O.Step(O.APPLY, 0, T)], num=num, momentum=inp["momentum"],
+                                ns_coeffs=(), **({"momentum_state": state} if carried else {}))
+    # bounds: a token sum rounded to bf16 after the roundings of its operands (test_small_tiles_against_oracle); the weights take the
+    # gradient's direction at the norm of one
+    for a, r in zip([out, *ws, *ms], [ref, *wr, *mr]):
+        assert O.rel_l2(a, r) < 1e-2

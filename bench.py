@@ -52,7 +52,7 @@ def _library_label(profile_name):
     n = profile_name.strip()
     n = re.sub(r"^void\s+", "", n).split("(")[0].replace("lact::", "")
     n = re.sub(r"TileShape<(\d+), (\d+), \d+, \d+>\s*", r"\1x\2", n).replace(" ", "")
-    m = re.match(r"k_ns_fused<(\d+x\d+),(true|false)>", n)
+    m = re.match(r"k_ns_fused<(\d+x\d+),(true|false)(?:,\d+x\d+)?>", n)
     if m:
         return f"k_ns_fused<{m.group(1)},{'bwd' if m.group(2) == 'true' else 'fwd'}>"
     m = re.match(r"k_row_gemm_dma<(\d+x\d+),(\d+),(\d+),(true|false)>", n)

@@ -369,6 +369,10 @@ struct DmaPipe {
     }
   }
 
+  // A wave of the first four that owns no part of the tile: it only passes the K-steps' barriers.
+  __device__ __forceinline__ void idle() const {
+    for (int i = 0; i < total; ++i) __syncthreads();
+  }
   // ---- MFMA waves: one phase over K into acc[0..NB).  `step` counts K-steps over all phases.
   template <int NB, bool A_KS = false, bool B_KS = false>
   __device__ __forceinline__ void run_phase(int K, int& step, f32x16 (&acc)[NB][TS::TM][TS::TN]) {

@@ -12,6 +12,7 @@ using TS_SQ = TileShape<128, 128, 2, 2>;    // small square GEMMs (Newton-Schulz
 using TS_BWD = TileShape<128, 64, 2, 2>;    // six accumulators (update backward): 64x32 per wave
 using TS_64 = TileShape<64, 64, 2, 2>;      // the same where two blocks share a compute unit
 using TS_NS = TileShape<192, 192, 2, 2>;    // 384-multiple square GEMMs (Newton-Schulz at d = dh = 384): 96x96 per wave
+using TS_H96 = TileShape<192, 96, 3, 1>;     // half a TS_NS tile, for three matrix waves: 96 columns are no two 32-column tiles
 using TS_N96 = TileShape<128, 96, 4, 1>;    // Newton-Schulz of few 384-multiple matrices: 12 instead of 9 blocks per 384 x 384 matrix
 
 template <class TS> constexpr int row_stages() { return TS::BM == 128 ? 4 : 3; }

@@ -454,9 +454,16 @@ struct Runner {
     return c;
   }
   template <class TS, bool BWD>
+  void launch_ns_fused_ts(const NsFusedParams& p, const NsBatch& B) {
+    using Half = typename NsHalfTile<TS>::type;
+    if constexpr (!std::is_void<Half>::value)
+      if (B.c >= 2 * B.r) return launch_ns_fused_ts<TS, BWD, Half>(p, B);
+    launch_ns_fused_ts<TS, BWD, TS>(p, B);
+  }
+  template <class TS, bool BWD, class TSQ>
   void launch_ns_fused_ts(NsFusedParams p, const NsBatch& B) {
-    constexpr int SM = cmax(DmaSmem<TS, 1, row_stages<TS>()>::BYTES, StageTile<TS, 4>::BYTES);
-    LACT_BIG_LDS((k_ns_fused<TS, BWD>), SM);
+    constexpr int SM = cmax(cmax(DmaSmem<TS, 1, ns_stages<TS>()>::BYTES, StageTile<TS, 4>::BYTES), DmaSmem<TSQ, 1, ns_stages<TSQ>()>::BYTES);
+    LACT_BIG_LDS((k_ns_fused<TS, BWD, TSQ>), SM);
     const int nbm = (B.r / TS::BM) * (B.c / TS::BN);
     const int per = (256 / nbm) / 8 * 8;
     unsigned* sync = scr<unsigned>(P.t_nssync) + (size_t)B.first * 32;
@@ -472,7 +479,7 @@ struct Runner {
       const int grid = 8 * ((p.n + 7) / 8) * nbm;
       side->order_fused_launch(s);
       LACT_LAUNCH_SMEM(name.c_str(), BWD ? "ns_bwd" : "ns_fwd", terms * 2.0 * B.r * B.r * B.c * P.S * p.n,
-                       (k_ns_fused<TS, BWD>), dim3(grid), dim3(DMA_THREADS), SM, s, p);
+                       (k_ns_fused<TS, BWD, TSQ>), dim3(grid), dim3(DMA_THREADS), SM, s, p);
     }
   }
   template <bool BWD>

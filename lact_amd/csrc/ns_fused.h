@@ -19,6 +19,9 @@
 // 13 main loop (8 matrices, whose operands stay in the L2s, 5.1 / 8.5: the rest is misses), 2.7 epilogue, 1.5 stores, barrier and set-up.
 // Launch: 214 -> 166 and 260 -> 249 us against epilogues that chose their case element by element, read the auxiliary tile behind
 // the staging and had every wave wait at the barrier; six matrices of 768 x 1536, three iterations: 195 -> 173.
+// Matrices with c >= 2 r take half tiles in the r x r stages (NsHalfTile), where whole ones leave half of the blocks waiting: forward /
+// backward us, six of 768 x 1536, three iterations 190 / 267 -> 175 / 248; 24 of 384 x 768, five 197 / 257 -> 178 / 224; 30 of 256 x 512
+// 96 / 115 -> 81 / 97; 18 of 384 x 1152, where a third of the blocks still waits, 200 / 273 -> 180 / 235.
 // Tried: the next stage's saved operand asked for into the L2 in the epilogue (-3 % there, +2 % at 12 matrices of 384 x 768);
 // non-temporal loads where an operand is read for the last time (+5 %: the partner block reads it too).
 //
@@ -191,8 +194,11 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_bwd_dot_tiles(const NsTileDo
 // rows; granule t of a thread lies at a distance from its first one that is a compile-time multiple of the row stride and columns.
 template <class TS, int THREADS>
 struct NsGranules {
-  static constexpr int LPR = TS::BN % 64 == 0 ? 8 : 4, CB = LPR * 8, RP = THREADS / LPR, NR = TS::BM / RP, NC = TS::BN / CB, N = NR * NC;
-  static_assert(TS::BM % RP == 0 && TS::BN % CB == 0, "granules split evenly over the threads");
+  static constexpr int LPR = TS::BN % 64 == 0 ? 8 : 4, CB = LPR * 8, RP = THREADS / LPR, NR = (TS::BM + RP - 1) / RP, NC = TS::BN / CB, N = NR * NC;
+  static_assert((TS::BM % RP == 0 || (THREADS == DMA_THREADS && TS::BM % RP == RP / 2)) && TS::BN % CB == 0, "granules split evenly over the threads");
+  // rows end with a pass of the lower half of the threads (the matrix waves) only: row(t) is past the tile for the others
+  static constexpr bool UPPER_SHORT = TS::BM % RP != 0;
+  __device__ static constexpr bool none(bool upper, int t) { return UPPER_SHORT && upper && t % NR == NR - 1; }
   __device__ static __forceinline__ int row0() { return (threadIdx.x & (THREADS - 1)) / LPR; }
   __device__ static __forceinline__ int col0() { return (threadIdx.x % LPR) * 8; }
   __device__ static constexpr int row(int t) { return (t % NR) * RP; }
@@ -202,6 +208,16 @@ struct NsGranules {
 // The roles of a block's waves are split for the whole of the iterations, not stage by stage: the fp32 iterate (its gradient) of
 // this block's tile then lives in the copy waves' registers, 18 granules of 8 elements per thread at 192 x 192, and only its bf16
 // copy goes through memory.  In one code path for all waves it would have to live beside the matrix waves' accumulators.
+// The tile of the r x r stages where c >= 2 r: their whole tiles would leave half of the matrix' blocks without work.
+template <class TS> struct NsHalfTile { using type = void; };
+template <> struct NsHalfTile<TS_NS> { using type = TS_H96; };
+template <> struct NsHalfTile<TS_SQ> { using type = TS_BWD; };
+template <class TS> constexpr int ns_stages() { return TS::BM == 192 && TS::BN == 96 ? 4 : row_stages<TS>(); }
+template <class TS> constexpr int ns_waves() { return TS::WAVES_M * TS::WAVES_N; }   // that own a part of the tile
+template <class TS> __device__ __forceinline__ bool ns_idle_wave() {
+  return ns_waves<TS>() < 4 && __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= ns_waves<TS>();
+}
+
 template <class TS>
 struct NsTileRegs {
   using G = NsGranules<TS, 256>;
@@ -215,7 +231,7 @@ template <class TS, int NT, bool B_KS, int GATE>
 __device__ __forceinline__ void ns_stage_load(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, const GroupBarrier& bar, unsigned* error) {
   DmaPhase<1> ph[NT];
   row_gemm_phases<TS, NT, B_KS>(p, bx * TS::BM, by * TS::BN, z, ph);
-  using Pipe = DmaPipe<TS, 1, NT, row_stages<TS>(), true>;
+  using Pipe = DmaPipe<TS, 1, NT, ns_stages<TS>(), true>;
   Pipe pipe(smem, ph);
   pipe.template load_all<Pipe::loads(1)>([&](int phase) {
     if (phase == GATE && (threadIdx.x & 63) == 0) bar.wait(error);
@@ -226,7 +242,8 @@ template <class TS, int NT, bool B_KS>
 __device__ __forceinline__ void ns_stage_mma(const RowGemmParams<NT>& p, int bx, int by, int z, char* smem, f32x16 (&acc)[1][TS::TM][TS::TN]) {
   DmaPhase<1> ph[NT];
   row_gemm_phases<TS, NT, B_KS>(p, bx * TS::BM, by * TS::BN, z, ph);
-  DmaPipe<TS, 1, NT, row_stages<TS>(), true> pipe(smem, ph);
+  DmaPipe<TS, 1, NT, ns_stages<TS>(), true> pipe(smem, ph);
+  if (ns_idle_wave<TS>()) return pipe.idle();
   zero_acc<TS>(acc[0]);
   int step = 0;
 #pragma unroll
@@ -235,6 +252,7 @@ __device__ __forceinline__ void ns_stage_mma(const RowGemmParams<NT>& p, int bx,
 template <class TS>
 __device__ __forceinline__ void ns_put_tile(char* smem, const f32x16 (&acc)[1][TS::TM][TS::TN]) {   // rounded to bf16
   using ST = StageTile<TS, 2>;
+  if (ns_idle_wave<TS>()) return;
   char* lb = smem + ST::lane_base();
   LACT_FOR_QUADS(TS) ST::put4(lb, tm, tn, g, acc[0][tm][tn][4 * g], acc[0][tm][tn][4 * g + 1], acc[0][tm][tn][4 * g + 2], acc[0][tm][tn][4 * g + 3]);
 }
@@ -253,7 +271,8 @@ __device__ __forceinline__ void ns_stage_b16(const RowGemmParams<NT>& p, int bx,
   uint4 w[G::N];
   if constexpr (EPI == EPI_AXPBY) {
 #pragma unroll
-    for (int t = 0; t < G::N; ++t) w[t] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.aux) + o0 + (size_t)G::row(t) * p.ldo + G::col(t));
+    for (int t = 0; t < G::N; ++t)
+      if (!G::none(COPY, t)) w[t] = *reinterpret_cast<const uint4*>(reinterpret_cast<const uint16_t*>(p.aux) + o0 + (size_t)G::row(t) * p.ldo + G::col(t));
   }
   if constexpr (!COPY) ns_put_tile<TS>(smem, acc);
   __syncthreads();
@@ -266,8 +285,9 @@ __device__ __forceinline__ void ns_stage_b16(const RowGemmParams<NT>& p, int bx,
       if (COPY) asm volatile("" ::: "memory");
 #pragma unroll
       for (int g = 0; g < LG; ++g)
-        if (t + g < G::N) u[g] = *reinterpret_cast<const uint4*>(src + (G::row(t + g) * ST::LD + G::col(t + g)) * 2);
+        if (t + g < G::N && !G::none(COPY, t + g)) u[g] = *reinterpret_cast<const uint4*>(src + (G::row(t + g) * ST::LD + G::col(t + g)) * 2);
     }
+    if (G::none(COPY, t)) continue;
     const size_t o = o0 + (size_t)G::row(t) * p.ldo + G::col(t);
     uint32_t uu[4] = {u[t % LG].x, u[t % LG].y, u[t % LG].z, u[t % LG].w};
     if constexpr (EPI == EPI_AXPBY) {
@@ -359,7 +379,8 @@ struct NsPlace {
 // BWD = false: S iterations  A = X X^T;  B = b A + c A A;  X' = a X + B X
 // BWD = true:  the same iterations backwards:  Sg = G X^T + X G^T;  H = b Sg + c (Sg A + A Sg);  G' = a G + B G + H X
 // COPY: on the copy waves, else on the matrix waves.  PLAIN: the iterate is a bf16 tensor (reference without autocast).
-template <class TS, bool BWD, bool COPY, bool PLAIN = false>
+// TSQ: tile of the r x r stages, TS or half of one.
+template <class TS, class TSQ, bool BWD, bool COPY, bool PLAIN = false>
 __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarrier& bar, const NsPlace& b, char* smem) {
   const int z = b.z;
   NsTileRegs<TS> x;
@@ -396,7 +417,7 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
         ns_term(q.g.t[0], X, c, xe, X, c, xe, c);
         q.g.M = r; q.g.N = r; q.g.out = A; q.g.ldo = r; q.g.bso = se;
         q.g.out2 = p.cab; q.g.alpha2 = cc;
-        ns_stage_b16<TS, 1, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+        ns_stage_b16<TSQ, 1, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
       } else bar.pass(p.error);
       bar.arrive();
       if (b.sq_tile) {
@@ -404,7 +425,7 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
         ns_term(q.g.t[0], p.cab, r, se, A, r, se, r);
         q.g.M = r; q.g.N = r; q.g.out = B; q.g.ldo = r; q.g.bso = se;
         q.g.aux = A; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = 1.f; q.g.beta = cb;
-        ns_stage_b16<TS, 1, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+        ns_stage_b16<TSQ, 1, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
       } else bar.pass(p.error);
       bar.arrive();
       {
@@ -425,7 +446,7 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
         ns_term(q.g.t[0], gb, c, xe, X, c, xe, c);
         ns_term(q.g.t[1], X, c, xe, gb, c, xe, c);
         q.g.M = r; q.g.N = r; q.g.out = p.sg; q.g.ldo = r; q.g.bso = se;
-        ns_stage_b16<TS, 2, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+        ns_stage_b16<TSQ, 2, EPI_STORE, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
       } else bar.pass(p.error);
       bar.arrive();
       if (b.sq_tile) {   // H = b Sg + c (Sg A + A Sg)
@@ -434,7 +455,7 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
         ns_term(q.g.t[1], A, r, se, p.sg, r, se, r);
         q.g.M = r; q.g.N = r; q.g.out = p.gas; q.g.ldo = r; q.g.bso = se;
         q.g.aux = p.sg; q.g.ldaux = r; q.g.bsaux = se; q.g.alpha = cc; q.g.beta = cb;
-        ns_stage_b16<TS, 2, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
+        ns_stage_b16<TSQ, 2, EPI_AXPBY, COPY>(q.g, b.sx, b.sy, z, smem, bar, p.error);
       } else bar.pass(p.error);
       bar.arrive();
       {                  // G' = a G + B G + H X
@@ -453,11 +474,12 @@ __device__ __forceinline__ void ns_iterations(const NsFusedParams& p, GroupBarri
 }
 
 // TS: 192 x 192 tiles, or 128 x 128 / 128 x 64 when there are too few matrices to fill the chip with the large tile.
-template <class TS, bool BWD>
+template <class TS, bool BWD, class TSQ = TS>
 __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   prefetch_args<sizeof(p)>();
-  const int tr = p.r / TS::BM, tc = p.c / TS::BN, ts = p.r / TS::BN;   // tile rows; tile columns of [r, c] and of [r, r]
+  const int tr = p.r / TS::BM, tc = p.c / TS::BN, ts = p.r / TSQ::BN;   // tile rows; tile columns of [r, c] and of [r, r]
+  static_assert(TSQ::BM == TS::BM, "the tiles of both kinds of stages have the same rows");
   const int nbm = tr * tc;                           // blocks per matrix (c >= r: the r x c stages have the most tiles)
   const int L = blockIdx.x, j = L >> 3;
   const int group = (L & 7) + 8 * (j / nbm), member = j % nbm;
@@ -508,10 +530,10 @@ __global__ __launch_bounds__(DMA_THREADS) void k_ns_fused(const NsFusedParams p)
   }
   const NsPlace place{z, sq_tile, sx, sy, rx, ry};
   if (__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) >= 4) {
-    if (!BWD && p.plain) ns_iterations<TS, BWD, true, !BWD>(p, bar, place, smem);
-    else ns_iterations<TS, BWD, true>(p, bar, place, smem);
+    if (!BWD && p.plain) ns_iterations<TS, TSQ, BWD, true, !BWD>(p, bar, place, smem);
+    else ns_iterations<TS, TSQ, BWD, true>(p, bar, place, smem);
   }
-  else ns_iterations<TS, BWD, false>(p, bar, place, smem);
+  else ns_iterations<TS, TSQ, BWD, false>(p, bar, place, smem);
   wait_vmcnt<0>();   // the last stage's stores, for the other waves of this block
   __syncthreads();
   if (BWD && p.dot_part) {

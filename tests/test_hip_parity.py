@@ -1260,6 +1260,13 @@ def test_fused_newton_schulz_is_bit_identical(b, d, dh, chunks):
     assert all(torch.equal(on[0][1][n], on[1][1][n]) for n in on[0][1])     # and each path repeats its own bits
 
 
+@pytest.mark.parametrize("b,d,dh", [(6, 256, 512), (6, 384, 1152), (1, 192, 384)])
+def test_fused_newton_schulz_on_half_tiles_is_bit_identical(b, d, dh):
+    """Matrices at least twice as wide as high: the stages of the square matrices on half tiles (128 x 64; 192 x 96, of which twice as
+    many as 384 x 384 holds in whole ones leave a third of the blocks idle; one matrix row of tiles)."""
+    test_fused_newton_schulz_is_bit_identical(b, d, dh, 2)
+
+
 # ---- fused-kernel variant (ttt_operation_fused_kernel.py): stacked Muon, eps inside the sqrt -------------
 def fused_variant_pair(C, use_muon, prenorm):
     hf = T.prenorm_block_causal_lact_swiglu_fused_kernel_triton if prenorm else T.postnorm_block_causal_lact_swiglu_fused_kernel_triton

@@ -50,8 +50,9 @@ template <> struct Elem<uint16_t> {
     u.y = pack_bf16(c, d);
     *reinterpret_cast<uint2*>(p) = u;
   }
-  __device__ static __forceinline__ void load4(const uint16_t* p, float* o) {
-    uint2 u = *reinterpret_cast<const uint2*>(p);
+  using Raw4 = uint2;       // four elements as they lie in memory
+  __device__ static __forceinline__ void load4(const uint16_t* p, float* o) { unpack4(*reinterpret_cast<const uint2*>(p), o); }
+  __device__ static __forceinline__ void unpack4(const uint2& u, float* o) {
     o[0] = __uint_as_float(u.x << 16);
     o[1] = __uint_as_float(u.x & 0xffff0000u);
     o[2] = __uint_as_float(u.y << 16);
@@ -66,8 +67,9 @@ template <> struct Elem<float> {
   __device__ static __forceinline__ void store4(float* p, float a, float b, float c, float d) {
     *reinterpret_cast<float4*>(p) = make_float4(a, b, c, d);
   }
-  __device__ static __forceinline__ void load4(const float* p, float* o) {
-    float4 u = *reinterpret_cast<const float4*>(p);
+  using Raw4 = float4;
+  __device__ static __forceinline__ void load4(const float* p, float* o) { unpack4(*reinterpret_cast<const float4*>(p), o); }
+  __device__ static __forceinline__ void unpack4(const float4& u, float* o) {
     o[0] = u.x; o[1] = u.y; o[2] = u.z; o[3] = u.w;
   }
 };

@@ -2104,9 +2104,9 @@ int layer_token_blocks(int act_dtype, const LayerGeom& g) {   // one pass of eve
   const long long n = 4LL * layer_rows_per_wave(act_dtype, g.hd);
   return (int)(((long long)g.B * g.L + n - 1) / n);
 }
-// blocks per head of the backward with parameter gradients: enough waves to hide the memory latency (16 per compute
-// unit), few enough that the partial sums stay small beside the activations
-int layer_pre_attn_blocks(const LayerGeom& g) { return (int)std::max(1LL, std::min(((long long)g.B * g.L + 3) / 4, 1024LL / g.H)); }
+// blocks per head of the backward with parameter gradients: as many as are resident at once (three waves a SIMD), few enough
+// that the partial sums stay small beside the activations
+int layer_pre_attn_blocks(const LayerGeom& g) { return (int)std::max(1LL, std::min(((long long)g.B * g.L + 3) / 4, 768LL / g.H)); }
 }  // namespace
 extern "C" {
 
@@ -2289,8 +2289,8 @@ int lact_layer_post_add_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t
   if (check_ptrs({o, y}, "layer post tensors")) return -1;
   p.eps = eps; p.use_norm = use_norm; p.o = o; p.w = norm_weight; p.gate_raw = gate_raw; p.add = add; p.y = y;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  if (act_dtype == LACT_BF16) launch_layer_post<uint16_t, false>(p, layer_row_blocks(act_dtype, p.g), s);
-  else if (act_dtype == LACT_F32) launch_layer_post<float, false>(p, layer_row_blocks(act_dtype, p.g), s);
+  if (act_dtype == LACT_BF16) launch_layer_post<uint16_t, false>(p, std::min(layer_row_blocks(act_dtype, p.g), 2048u), s);
+  else if (act_dtype == LACT_F32) launch_layer_post<float, false>(p, std::min(layer_row_blocks(act_dtype, p.g), 2048u), s);
   else return fail("act_dtype must be LACT_BF16 or LACT_F32");
   LACT_CHECK_LAUNCH();
   return 0;

@@ -84,63 +84,75 @@ struct LayerPreParams {
 // are issued before the first of them is used (the norms otherwise put three round trips in line).  The attention's inputs ride
 // along because the projection's output is in registers here: as tensor operations of their own (slices, rescaling, and in the
 // backward three zero-padded slice gradients to add up) they took 0.9 ms of a training step at 16384 tokens of 1536 channels.
-// bf16, us forward / backward, with all 64 lanes on a row before: 16384 tokens, 4 heads of 384 (ATT) 134 / 172 (145 / 234: 450 and
-// 600 MB); 7500 tokens, 8 heads of 96 19 / 34 (37 / 65: 69 and 104 MB).
+// Waves in flight decide (layer_pre_waves): operands stay packed until they are used, and the backward keeps the rescaling in LDS and asks
+// for v's when q is done.  bf16, us forward / backward, and unpacked, with three and two waves a SIMD instead of four and three: 16384
+// tokens, 4 heads of 384 (ATT) 77 / 121 (134 / 172: 450 and 600 MB); 7500 tokens, 8 heads of 96 15.5 / 24.7 (17 / 31: 69 and 104 MB).
+template <typename T, bool BWD, bool ATT, int NV> constexpr int layer_pre_waves() { return NV > 3 || std::is_same<T, float>::value ? 1 : BWD && ATT ? 3 : 4; }
 template <typename T, bool BWD, bool ATT, int G, int NV>
-__global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
+__global__ __launch_bounds__(256, (layer_pre_waves<T, BWD, ATT, NV>())) void k_layer_pre(const LayerPreParams p) {
   prefetch_args<sizeof(p)>();
   using RL = RowLanes<G, NV>;
   const int wave = threadIdx.x >> 6, grp = RL::group();
   const int hd = p.g.hd, h = blockIdx.x % p.g.H;
   const size_t dim = (size_t)p.g.H * hd;
-  float sc[2][NV][4], off[2][NV][4];           // ATT: this lane's channels of the rescaling
+  float sc[2][NV][4], off[2][NV][4];           // ATT: this lane's channels of the rescaling; backward: in LDS, [q, k][channels of a row]
+  __shared__ __attribute__((aligned(16))) float scl[BWD && ATT ? 2 * NV * 4 * G : 1];
   float acc[4][NV][4];                         // ATT && BWD: this lane's share of the parameter gradients
   if (ATT) {
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int c = min(RL::col(i), hd - 4);
-      const float* ps = p.qk_scale + ((size_t)h * hd + c) * 2;
-      const float4 s0 = *reinterpret_cast<const float4*>(ps), s1 = *reinterpret_cast<const float4*>(ps + 4);
-      sc[0][i][0] = s0.x; sc[1][i][0] = s0.y; sc[0][i][1] = s0.z; sc[1][i][1] = s0.w;
-      sc[0][i][2] = s1.x; sc[1][i][2] = s1.y; sc[0][i][3] = s1.z; sc[1][i][3] = s1.w;
-      if (!BWD) {
-        const float* po = p.qk_offset + ((size_t)h * hd + c) * 2;
-        const float4 o0 = *reinterpret_cast<const float4*>(po), o1 = *reinterpret_cast<const float4*>(po + 4);
-        off[0][i][0] = o0.x; off[1][i][0] = o0.y; off[0][i][1] = o0.z; off[1][i][1] = o0.w;
-        off[0][i][2] = o1.x; off[1][i][2] = o1.y; off[0][i][3] = o1.z; off[1][i][3] = o1.w;
-      } else {
+      if (BWD) {
+        if (threadIdx.x < G)
+          for (int j = 0; j < 4; ++j)
+            for (int a = 0; a < 2; ++a) scl[a * NV * 4 * G + RL::col(i) + j] = p.qk_scale[((size_t)h * hd + c + j) * 2 + a];
 #pragma unroll
         for (int a = 0; a < 4; ++a)
 #pragma unroll
           for (int j = 0; j < 4; ++j) acc[a][i][j] = 0.f;
+        continue;
       }
+      const float* ps = p.qk_scale + ((size_t)h * hd + c) * 2;
+      const float4 s0 = *reinterpret_cast<const float4*>(ps), s1 = *reinterpret_cast<const float4*>(ps + 4);
+      sc[0][i][0] = s0.x; sc[1][i][0] = s0.y; sc[0][i][1] = s0.z; sc[1][i][1] = s0.w;
+      sc[0][i][2] = s1.x; sc[1][i][2] = s1.y; sc[0][i][3] = s1.z; sc[1][i][3] = s1.w;
+      const float* po = p.qk_offset + ((size_t)h * hd + c) * 2;
+      const float4 o0 = *reinterpret_cast<const float4*>(po), o1 = *reinterpret_cast<const float4*>(po + 4);
+      off[0][i][0] = o0.x; off[1][i][0] = o0.y; off[0][i][1] = o0.z; off[1][i][1] = o0.w;
+      off[0][i][2] = o1.x; off[1][i][2] = o1.y; off[0][i][3] = o1.z; off[1][i][3] = o1.w;
     }
+    if (BWD) __syncthreads();
   }
   for (long long bl = ((long long)(blockIdx.x / p.g.H) * 4 + wave) * RL::ROWS + grp; bl < (long long)p.g.B * p.g.L; bl += p.tokens_per_pass) {
     const int l = (int)(bl % p.g.L);
     const long long b = bl / p.g.L;
     const size_t oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd, ai = (size_t)bl * dim + (size_t)h * hd;
-    float xs[3][NV][4], gs[3][NV][4], as[3][NV][4];
-#pragma unroll
-    for (int which = 0; which < 3; ++which)
+    using Raw = typename Elem<T>::Raw4;
+    Raw xs[3][NV], gs[3][NV], as[3][NV];       // unpacked where they are used: half the registers
+    auto load = [&](int which) {
 #pragma unroll
       for (int i = 0; i < NV; ++i) {
         const int c = RL::col(i);
+        xs[which][i] = gs[which][i] = as[which][i] = Raw{};
         if (c < hd) {
-          Elem<T>::load4(reinterpret_cast<const T*>(p.qkv) + ((size_t)(bl * 3 + which) * p.g.H + h) * hd + c, xs[which][i]);
-          if (BWD) Elem<T>::load4(reinterpret_cast<const T*>(p.dout[which]) + oi + c, gs[which][i]);
-          if (BWD && ATT) Elem<T>::load4(reinterpret_cast<const T*>(p.datt[which]) + ai + c, as[which][i]);
-        } else {
-#pragma unroll
-          for (int j = 0; j < 4; ++j) xs[which][i][j] = gs[which][i][j] = as[which][i][j] = 0.f;
+          xs[which][i] = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(p.qkv) + ((size_t)(bl * 3 + which) * p.g.H + h) * hd + c);
+          if (BWD) gs[which][i] = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(p.dout[which]) + oi + c);
+          if (BWD && ATT) as[which][i] = *reinterpret_cast<const Raw*>(reinterpret_cast<const T*>(p.datt[which]) + ai + c);
         }
       }
+    };
+    constexpr int FIRST = BWD && ATT ? 2 : 3;  // (the third's registers are those of the first)
+#pragma unroll
+    for (int which = 0; which < FIRST; ++which) load(which);
 #pragma unroll
     for (int which = 0; which < 3; ++which) {
       const bool norm = p.l2norm && which < 2;
-      float (&x)[NV][4] = xs[which];
-      float (&g)[NV][4] = gs[which];
-      float y[NV][4];
+      float x[NV][4], g[NV][4], y[NV][4];
+#pragma unroll
+      for (int i = 0; i < NV; ++i) {
+        Elem<T>::unpack4(xs[which][i], x[i]);
+        if (BWD) Elem<T>::unpack4(gs[which][i], g[i]);
+      }
 #pragma unroll
       for (int i = 0; i < NV; ++i)
 #pragma unroll
@@ -174,16 +186,23 @@ __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
             Elem<T>::store4(reinterpret_cast<T*>(p.att[which]) + ai + c, a[0], a[1], a[2], a[3]);
           }
         } else {
-          float o[4];
+          float o[4], at[4], s[4];
+          if (ATT) {
+            Elem<T>::unpack4(as[which][i], at);
+            if (which < 2) {
+              const float4 t = *reinterpret_cast<const float4*>(&scl[which * NV * 4 * G + c]);
+              s[0] = t.x; s[1] = t.y; s[2] = t.z; s[3] = t.w;
+            }
+          }
 #pragma unroll
           for (int j = 0; j < 4; ++j) {
             o[j] = (g[i][j] * inv - y[i][j] * c1) * silu_grad_f(x[i][j]);
             if (ATT) {
-              const float a = as[which][i][j];
+              const float a = at[j];
               if (which < 2) {
                 acc[2 * (which & 1)][i][j] += a * x[i][j];
                 acc[2 * (which & 1) + 1][i][j] += a;
-                o[j] += a * sc[which & 1][i][j];
+                o[j] += a * s[j];
               } else {
                 o[j] += a;
               }
@@ -192,6 +211,7 @@ __global__ __launch_bounds__(256) void k_layer_pre(const LayerPreParams p) {
           Elem<T>::store4(reinterpret_cast<T*>(p.dqkv) + ((size_t)(bl * 3 + which) * p.g.H + h) * hd + c, o[0], o[1], o[2], o[3]);
         }
       }
+      if (FIRST < 3 && which == 0) load(2);
     }
   }
   if (ATT && BWD) {      // the shares of the wave's rows, then the four waves', in a fixed order
@@ -292,10 +312,10 @@ struct LayerPostParams {
   float* dw_part;             // [gridDim.x][hd] partial sums of the weight gradient, or null
 };
 // Backward: each wave walks rows row0, row0 + stride, ... so that its partial weight gradient stays in registers.
-// HBM bound.  bf16, us forward / backward, with all 64 lanes and four chunks on a row before: 16384 tokens, 4 heads of 384 42 / 46
-// (53 / 71: 150 MB each); 7500 tokens, 8 heads of 96 9.3 / 12.6 (22 / 36).
+// HBM bound.  bf16, us forward / backward, with all 64 lanes and four chunks on a row before: 16384 tokens, 4 heads of 384 31 / 45
+// (53 / 71: 150 MB each; the forward with one row a wave and its gate asked for behind the sum 43); 7500 tokens, 8 heads of 96 8.7 / 13 (22 / 36).
 template <typename T, bool BWD, int G, int NV>
-__global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
+__global__ __launch_bounds__(256, (NV > 3 || std::is_same<T, float>::value ? 1 : 4)) void k_layer_post(const LayerPostParams p) {
   prefetch_args<sizeof(p)>();
   using RL = RowLanes<G, NV>;
   const int wave = threadIdx.x >> 6, grp = RL::group();
@@ -311,33 +331,53 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
       dwacc[i][j] = 0.f;
     }
   }
-  for (long long row = ((long long)blockIdx.x * 4 + wave) * RL::ROWS + grp; row < p.g.rows(); row += step) {
+  using Raw = typename Elem<T>::Raw4;
+  struct Row {
+    size_t oi, yi;                // in o and in y
+    long long gi;                 // its gate
+    Raw x[NV], z[NV];             // z: what is added, or the gradient
+    float gate;
+  };
+  auto load = [&](long long row, Row& r) {
     const int h = (int)(row % p.g.H);
     const long long bl = row / p.g.H;
     const int l = (int)(bl % p.g.L);
     const long long b = bl / p.g.L;
-    const size_t oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd;
-    const size_t yi = ((size_t)bl * p.g.H + h) * hd;
-    const T* src = reinterpret_cast<const T*>(p.o) + oi;
-    const T* other = BWD ? reinterpret_cast<const T*>(p.dy) + yi : p.add ? reinterpret_cast<const T*>(p.add) + yi : nullptr;
-    float x[NV][4], z[NV][4];     // z: what is added, or the gradient
+    r.oi = ((size_t)(b * p.g.H + h) * p.g.L + l) * hd;
+    r.yi = ((size_t)bl * p.g.H + h) * hd;
+    r.gi = bl * p.g.H + h;
+    const T* src = reinterpret_cast<const T*>(p.o) + r.oi;
+    const T* other = BWD ? reinterpret_cast<const T*>(p.dy) + r.yi : p.add ? reinterpret_cast<const T*>(p.add) + r.yi : nullptr;
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
       const int c = RL::col(i);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) x[i][j] = z[i][j] = 0.f;
+      r.x[i] = r.z[i] = Raw{};
       if (c < hd) {
-        Elem<T>::load4(src + c, x[i]);
-        if (other) Elem<T>::load4(other + c, z[i]);
+        r.x[i] = *reinterpret_cast<const Raw*>(src + c);
+        if (other) r.z[i] = *reinterpret_cast<const Raw*>(other + c);
       }
+    }
+    r.gate = p.gate_raw ? Elem<T>::load(reinterpret_cast<const T*>(p.gate_raw) + r.gi) : 0.f;
+  };
+  // Forward: a row ahead, so that the loads of the next one are on their way while this one is summed.  (The backward has too few
+  // registers left for it: 45 -> 47 us.)
+  Row cur, next;
+  long long row = ((long long)blockIdx.x * 4 + wave) * RL::ROWS + grp;
+  if (!BWD && row < p.g.rows()) load(row, cur);
+  for (; row < p.g.rows(); row += step) {
+    if (BWD) load(row, cur);
+    else if (row + step < p.g.rows()) load(row + step, next);
+    const size_t oi = cur.oi, yi = cur.yi;
+    const float graw = cur.gate;
+    float x[NV][4], z[NV][4];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      Elem<T>::unpack4(cur.x[i], x[i]);
+      Elem<T>::unpack4(cur.z[i], z[i]);
     }
     float rstd = 1.f;
     if (p.use_norm) rstd = rsqrtf(RL::sum([&](int i, int j, float s) { return s + x[i][j] * x[i][j]; }) / (float)hd + p.eps);
-    float graw = 0.f, gate = 1.f;
-    if (p.gate_raw) {
-      graw = Elem<T>::load(reinterpret_cast<const T*>(p.gate_raw) + bl * p.g.H + h);
-      gate = Elem<T>::rnd(silu_f(graw));
-    }
+    const float gate = p.gate_raw ? Elem<T>::rnd(silu_f(graw)) : 1.f;
     if (!BWD) {
       T* dst = reinterpret_cast<T*>(p.y) + yi;
 #pragma unroll
@@ -373,7 +413,7 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
           const float n = x[i][j] * rstd;
           return s + z[i][j] * (p.use_norm ? n * wv[i][j] : n);
         });
-        if ((threadIdx.x & (G - 1)) == 0) Elem<T>::store(reinterpret_cast<T*>(p.dgate_raw) + bl * p.g.H + h, dg * silu_grad_f(graw));
+        if ((threadIdx.x & (G - 1)) == 0) Elem<T>::store(reinterpret_cast<T*>(p.dgate_raw) + cur.gi, dg * silu_grad_f(graw));
       }
       T* dx = reinterpret_cast<T*>(p.d_o) + oi;
 #pragma unroll
@@ -387,6 +427,7 @@ __global__ __launch_bounds__(256) void k_layer_post(const LayerPostParams p) {
         }
       }
     }
+    if (!BWD) cur = next;
   }
   if (BWD && p.dw_part) {      // the shares of the wave's rows, then the four waves', in a fixed order
     __shared__ float red[NV * 4 * G];

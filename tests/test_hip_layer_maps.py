@@ -289,3 +289,30 @@ def test_rows_of_every_head_size_against_float64(hd, dtype):
         exact = torch.autograd.grad(want, list(d.values()), [t.double() for t in go], allow_unused=True)
         for n, x, y in zip(inp, got, exact):
             assert y is None or not y.any() or rel_l2(x, y) < tol, n
+
+
+# more rows than the blocks of one pass take (2048 blocks of 4 waves forward, 1024 backward), ending inside a wave's rows: four, eight and
+# two rows a wave, fp32
+@pytest.mark.parametrize("L,H,hd,dtype", [(16390, 2, 64, torch.bfloat16), (32773, 2, 96, torch.bfloat16), (16411, 1, 384, torch.bfloat16), (16399, 2, 36, torch.float32)])
+def test_rows_beyond_one_pass_of_the_waves(L, H, hd, dtype):
+    """RMSNorm, gate and sum over many rows: every row's result and gradients are those of a call on a part of the rows (the same
+    arithmetic per row, hence the same bits; the weight's gradient, a sum over all rows, against float64)."""
+    print("[gpu-test] many rows", L, H, hd, dtype, flush=True)
+    g = torch.Generator().manual_seed(hd)
+    r = lambda *s, t=dtype: torch.randn(*s, generator=g).to(t).to(DEV)
+    o, w, gate, add, dy = r(H, L, hd), r(hd, t=torch.float32), r(1, L, H), r(1, L, H * hd), r(1, L, H * hd)
+    host = _lib.host()
+
+    def run(rows):
+        x = [o[:, rows].contiguous().requires_grad_(True), w.clone().requires_grad_(True), gate[:, rows].contiguous().requires_grad_(True),
+             add[:, rows].contiguous().requires_grad_(True)]
+        y = host.layer_post(*x[:3], 1, H, True, 1e-5, x[3])
+        return [y.detach(), *torch.autograd.grad(y, x, dy[:, rows].contiguous())]
+
+    whole, parts = run(slice(0, L)), [run(slice(a, min(a + 4000, L))) for a in range(0, L, 4000)]
+    for i in (0, 1, 3, 4):     # y, do, dgate, dadd
+        assert torch.equal(whole[i], torch.cat([p[i] for p in parts], dim=1)), i
+    n = o.double() * torch.rsqrt(o.double().square().mean(-1, keepdim=True) + 1e-5)
+    dt = (dy.double().view(L, H, hd) * F.silu(gate.double()).to(dtype).double().view(L, H, 1)).transpose(0, 1)
+    # fp32 sums (some thousand roundings of 2^-24 that mostly cancel); a bf16 gate that rounds the other way here is 2^-9 of one addend
+    assert rel_l2(whole[2], (dt * n).sum((0, 1))) < (1e-5 if dtype == torch.float32 else 1e-4)

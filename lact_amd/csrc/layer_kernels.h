@@ -478,8 +478,8 @@ __global__ __launch_bounds__(1024) void k_layer_sum_rows(const float* part, int 
 // Output n of the launch: n < NL * 4: rate row n (valid below n1), from the fp32 input and weights; behind them the rows of the
 // two bf16 maps, from input and weights rounded to bf16, the sum in fp32, the result rounded: what the GEMMs of autocast do.
 // Bound by HBM and vector-ALU issue alike.  16384 tokens of 1536 channels, 12 + 8 outputs, us: forward 28 (the two products and four
-// casts 85), gradient of the input 50, of the parameters 45 + 8 (six products with a dozen rows or columns each, two bias sums and
-// seven additions and casts: 520).  7500 tokens of 768 channels, 24 outputs: 20 and 19 + 5 (85).
+// casts 85), gradient of the input 37 (51 with a token's row asked for behind the one before it), of the parameters 37 + 8 (six products with a dozen rows or columns each, two bias sums and
+// seven additions and casts: 520).  7500 tokens of 768 channels, 24 outputs: 15.5 and 18 + 5 (85).
 struct LayerInMap {
   const float* w;      // [n][dim] fp32
   const float* bias;   // [n] or null (forward)
@@ -525,15 +525,31 @@ __device__ __forceinline__ float4 layer_in_weight(const LayerInParams& p, int n,
   if (m > 0) v = make_float4(round_bf16(v.x), round_bf16(v.y), round_bf16(v.z), round_bf16(v.w));
   return v;
 }
-// gradient that arrives at output n of token t
+// The gradients that arrive at the outputs of `toks` tokens from t0 on, to g[token][output] in LDS by `threads` threads.  Each map's lie
+// one after the other in memory: four loads of a thread at a time (one by one, each behind the last
+// one's latency, k_layer_in_dw took 44 us instead of 37).
 template <int NL, int NB>
-__device__ __forceinline__ float layer_in_grad(const LayerInParams& p, int n, long long t) {
-  int r;
-  const int m = layer_in_row<NL, NB>(p, n, r);
-  if (m < 0 || t >= p.rows) return 0.f;
-  if (m == 0) return p.dlr ? p.dlr[t * p.lr.n + r] : 0.f;
-  if (m == 1) return p.dmom ? round_bf16(p.dmom[t * p.mom.n + r]) : 0.f;
-  return p.dgate ? bf16_to_f32(p.dgate[t * p.gate.n + r]) : 0.f;
+__device__ __forceinline__ void layer_in_grads(const LayerInParams& p, float* g, long long t0, int toks, int tid, int threads) {
+  constexpr int NO = 4 * (NL + NB);
+  for (int i = tid; i < toks * NO; i += threads) g[i] = 0.f;
+  __syncthreads();
+  auto map = [&](int n, int first, auto load) {
+    const int total = toks * n;
+    const long long from = t0 * n;
+    for (int i0 = tid; i0 < total; i0 += 4 * threads) {
+      float v[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = load(from + min(i0 + j * threads, total - 1));
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int i = i0 + j * threads, k = i / n;
+        if (i < total) g[k * NO + first + i - k * n] = v[j];
+      }
+    }
+  };
+  if (NL > 0 && p.dlr) map(p.lr.n, 0, [&](long long e) { return p.dlr[e]; });
+  if (NB > 0 && p.dmom) map(p.mom.n, 4 * NL, [&](long long e) { return round_bf16(p.dmom[e]); });
+  if (NB > 0 && p.dgate) map(p.gate.n, 4 * NL + p.mom.n, [&](long long e) { return bf16_to_f32(p.dgate[e]); });
 }
 
 // Forward: the bf16 copy and the bf16 maps.  (The rates stay a library product: they decide the roundings of everything that
@@ -620,24 +636,38 @@ __global__ __launch_bounds__(256) void k_layer_in_dx(const LayerInParams p) {
   constexpr int NO = 4 * (NL + NB), TOK = LAYER_IN_DXTOK;
   __shared__ float gs[TOK][NO];
   const long long t0 = (long long)blockIdx.x * TOK;
-  for (int i = threadIdx.x; i < TOK * NO; i += blockDim.x) gs[i / NO][i % NO] = layer_in_grad<NL, NB>(p, i % NO, t0 + i / NO);
+  const int toks = (int)min((long long)TOK, p.rows - t0);
   const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
+  constexpr int AHEAD = 8;                   // tokens whose rows are asked for together
+  uint2 in[AHEAD];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) in[k] = *reinterpret_cast<const uint2*>(p.dxq + (t0 + min(k0 + k, toks - 1)) * p.dim + min(c, p.dim - 4));
+  };
+  fetch(0);
   float4 w[NO];
 #pragma unroll
   for (int n = 0; n < NO; ++n) w[n] = layer_in_weight<NL, NB>(p, n, c);
+  layer_in_grads<NL, NB>(p, &gs[0][0], t0, toks, threadIdx.x, blockDim.x);
   __syncthreads();
   if (c >= p.dim) return;
-  const int toks = (int)min((long long)TOK, p.rows - t0);
-#pragma unroll 8
-  for (int k = 0; k < toks; ++k) {
-    float o[4];
-    Elem<uint16_t>::load4(p.dxq + (t0 + k) * p.dim + c, o);
+  for (int k0 = 0; k0 < toks; k0 += AHEAD) {
+    uint2 now[AHEAD];
 #pragma unroll
-    for (int n = 0; n < NO; ++n) {
-      const float g = gs[k][n];
-      o[0] = fmaf(g, w[n].x, o[0]); o[1] = fmaf(g, w[n].y, o[1]); o[2] = fmaf(g, w[n].z, o[2]); o[3] = fmaf(g, w[n].w, o[3]);
+    for (int k = 0; k < AHEAD; ++k) now[k] = in[k];
+    if (k0 + AHEAD < toks) fetch(k0 + AHEAD);
+#pragma unroll
+    for (int k = 0; k < AHEAD; ++k) {
+      if (k0 + k >= toks) break;
+      float o[4];
+      Elem<uint16_t>::unpack4(now[k], o);
+#pragma unroll
+      for (int n = 0; n < NO; ++n) {
+        const float g = gs[k0 + k][n];
+        o[0] = fmaf(g, w[n].x, o[0]); o[1] = fmaf(g, w[n].y, o[1]); o[2] = fmaf(g, w[n].z, o[2]); o[3] = fmaf(g, w[n].w, o[3]);
+      }
+      *reinterpret_cast<float4*>(p.dx + (t0 + k0 + k) * p.dim + c) = make_float4(o[0], o[1], o[2], o[3]);
     }
-    *reinterpret_cast<float4*>(p.dx + (t0 + k) * p.dim + c) = make_float4(o[0], o[1], o[2], o[3]);
   }
 }
 
@@ -651,18 +681,18 @@ __global__ __launch_bounds__(256) void k_layer_in_dw(const LayerInParams p) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, tok = p.dw_tok;
   const long long t0 = ((long long)blockIdx.x * 4 + wave) * tok;
   float* gs = lds + wave * TOK * NO;
-  for (int i = lane; i < tok * NO; i += 64) gs[i] = layer_in_grad<NL, NB>(p, i % NO, t0 + i / NO);
+  const int toks = (int)max(0LL, min((long long)tok, p.rows - t0));
+  layer_in_grads<NL, NB>(p, gs, t0, toks, lane, 64);
   __syncthreads();
   const int c = blockIdx.y * 256 + lane * 4;
   if (blockIdx.y == 0 && lane < NO) {
     float s = 0.f;
-    for (int k = 0; k < tok; ++k) s += gs[k * NO + lane];
+    for (int k = 0; k < toks; ++k) s += gs[k * NO + lane];
     p.bpart[((size_t)blockIdx.x * 4 + wave) * NO + lane] = s;
   }
   float4 acc[NO];
 #pragma unroll
   for (int n = 0; n < NO; ++n) acc[n] = make_float4(0.f, 0.f, 0.f, 0.f);
-  const int toks = (int)max(0LL, min((long long)tok, p.rows - t0));
   if (c < p.dim) {
 #pragma unroll 8
     for (int k = 0; k < toks; ++k) {

@@ -121,7 +121,6 @@ template <> const char* tname<float>() { return "f32"; }
 // pool per device, created on first use and kept until the process ends.
 struct SideCtx {
   hipStream_t stream = nullptr;
-  hipStream_t tail = nullptr;        // second side stream: what depends on the inputs of a forward only (k * lr0, k * lr2)
   std::vector<hipEvent_t> ev;
   size_t next = 0;
   // Fused Newton-Schulz kernels of this process must not overlap each other (each needs its groups resident as a whole).
@@ -173,7 +172,6 @@ SideCtx* side_ctx() {
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return nullptr;
   SideCtx& c = ctx[dev];
   if (!c.stream && hipStreamCreateWithFlags(&c.stream, hipStreamNonBlocking) != hipSuccess) return nullptr;
-  if (!c.tail && hipStreamCreateWithFlags(&c.tail, hipStreamNonBlocking) != hipSuccess) return nullptr;
   if (c.cus == 0) {
     int n = 0;
     c.cus = (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && n > 0) ? n : -1;
@@ -329,14 +327,13 @@ struct Runner {
   char* sc;   // scratch
   const lact_desc_t& d;
   hipStream_t s_main, s_side;   // caller's stream; stream of the apply steps (= s_main when overlap is off)
-  hipStream_t s_tail;           // stream of k * lr0 and k * lr2 at the start of a forward (= s_main when overlap is off)
   SideCtx* side = nullptr;
   const size_t* hsel;           // token-major intermediates of the chain being enqueued
   size_t partial_sel;
   Runner(const Plan& p, void* saved, void* scratch, hipStream_t st)
-      : P(p), s(st), sv(align256(saved)), sc(align256(scratch)), d(p.d), s_main(st), s_side(st), s_tail(st), hsel(p.t_h), partial_sel(p.t_partial) {
+      : P(p), s(st), sv(align256(saved)), sc(align256(scratch)), d(p.d), s_main(st), s_side(st), hsel(p.t_h), partial_sel(p.t_partial) {
     side = side_ctx();
-    if (side && g_overlap && !P.groups.empty()) { s_side = side->stream; s_tail = side->tail; }
+    if (side && g_overlap && !P.groups.empty()) s_side = side->stream;
   }
   // ---- fused Newton-Schulz: launches of at most 256 resident blocks
   static bool tiles_fit(int r, int c, int bm, int bn) {
@@ -952,12 +949,6 @@ struct Runner {
               const float* lr1, const float* lr2, const float* mom, T* out, float* const w_out[3], float* const m_out[3],
               const float* const m_in[3]) {
     const dim3 rowgrid(ceil_div(P.g.maxrows(), 4), 3 * d.b);
-    // what depends on the inputs only may start on the tail stream right here, beside the first kernels of the call
-    hipEvent_t entry = nullptr;
-    if (s_tail != s_main && side && P.nupd > 0) {
-      entry = side->event();
-      (void)hipEventRecord(entry, s_main);
-    }
     // carried momentum state: read where it lies (three copies took 18 us at 3 matrices of 768 x 1536 and two batch entries), but for one
     // that 16-byte loads do not reach (a device-to-device copy node when captured)
     if (P.state_in && P.nupd > 0)
@@ -1002,25 +993,15 @@ struct Runner {
     T* upd_z[3] = {nullptr, nullptr, nullptr};   // lr-scaled operands of the current update's gradient GEMMs
     long long upd_zbs = 0;
     bool side_used = false;
-    // k * lr0, k * lr2 depend on the inputs only and are first read by the first token reduction: one launch, on the tail stream
-    // beside the first kernels of the call where there is one
-    hipEvent_t kl_ready = nullptr;
+    // k * lr0, k * lr2 of all updates in one launch, in line: on a stream of its own, beside the first kernels of the call, the launch
+    // itself costs nothing but the two events 7 us on either side and as much host time (us of a training step: eight fp32 heads of
+    // 128, 2048 tokens 421 / 411 in line, 6 heads of 256 x 512, 5003 tokens 822 / 809; 16 heads of 384, 4096 tokens 1141 either way).
     const long long klbs = (long long)(P.kl_end - P.kl_begin) * d.d;
     const bool fused = updates_fused();
-    if (klbs > 0 && !fused) {
-      if (entry) {
-        (void)hipStreamWaitEvent(s_tail, entry, 0);
-        s = s_tail;
-      }
+    if (klbs > 0 && !fused)
       LACT_LAUNCH("k_lr_scale_rows", "update_lr_k", 0.0, (k_lr_scale_rows<T>), dim3((unsigned)((klbs / 4 + 255) / 256), d.b), dim3(256), s,
                   k + (size_t)P.kl_begin * d.k_ld, d.k_ld, d.k_bs, lr0 + P.kl_begin, lr2 + P.kl_begin, (long long)d.kv_len, P.kl_end - P.kl_begin, d.d,
                   scr<T>(P.t_kl[0]), scr<T>(P.t_kl[1]), klbs);
-      if (entry) {
-        kl_ready = side->event();
-        (void)hipEventRecord(kl_ready, s_tail);
-        s = s_main;
-      }
-    }
     // Apply steps only need their weight version.  A group of them is enqueued when its last version is final, on the side stream
     // and at the point of the following update where the chip is least busy -- in front of its Newton-Schulz kernels, which leave
     // a quarter of the compute units idle; the newest version's at the end, on the caller's stream.
@@ -1083,8 +1064,6 @@ struct Runner {
       // the pre-Muon gradient (= the momentum state) of the last update: read by nothing when Newton-Schulz output is
       // what enters the weights (the next update and its backward would read it; the caller gets its own copy)
       const bool d_unread = P.muon && !d.muon_replaces_weight && u + 1 == P.nupd;
-      if (kl_ready) (void)hipStreamWaitEvent(s_main, kl_ready, 0);
-      kl_ready = nullptr;
       if (!fused) {
         TokenReduceJob jobs[3];
         memset(jobs, 0, sizeof(jobs));

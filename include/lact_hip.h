@@ -252,10 +252,11 @@ int lact_window_attention_backward(int32_t B, int32_t L, int32_t H, int32_t D, i
 /* Execution options (process-wide; no counterpart in the reference, where PyTorch enqueues the whole layer on one
  * stream as separate kernels).  The switches are on by default and change no result bit.
  *   LACT_OPT_STREAM_OVERLAP: the apply steps of a program do not depend on the update chain that runs beside
- *     them, and k times the learning rates depends on the inputs only; where a program has apply steps on a
- *     version that is not its newest, lact_forward / lact_backward enqueue them on two library-owned streams
- *     (default priority, per device, created on first use) that are forked from and joined back into the caller's
- *     stream with events, so the call as a whole stays asynchronous and ordered on the caller's stream.
+ *     them; where a program has apply steps on a version that is not its newest, lact_forward / lact_backward
+ *     enqueue them on a library-owned stream (default priority, per device, created on first use) that is forked
+ *     from and joined back into the caller's stream with events, so the call as a whole stays asynchronous and
+ *     ordered on the caller's stream.  1 (the default): where these steps are long enough to pay for the events, or
+ *     the call is being captured; 2: always; 0: never.
  *   LACT_OPT_FUSED_NEWTON_SCHULZ: all Newton-Schulz iterations of an update (and of its backward) run as one
  *     kernel whose blocks meet at per-matrix barriers (bf16; rows and columns multiples of 192, of 128, or rows of
  *     128 and columns of 64; at most 8 iterations); otherwise three GEMM launches per iteration.

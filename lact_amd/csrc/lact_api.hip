@@ -159,7 +159,7 @@ struct SideCtx {
 // lact_check_async_error (each GPU holds its own copy; host code reaches it through hipGetSymbolAddress only).
 static __device__ unsigned g_async_errors;
 namespace {
-bool g_overlap = true;
+int g_overlap = 1;          // LACT_OPT_STREAM_OVERLAP: 0 never, 1 where it pays, 2 wherever there is something to overlap
 bool g_fused_ns = true;
 int g_persist = 1;          // hidden-stage kernels on the persistent engine (LACT_OPT_PERSISTENT_TILES): bit 0 apply, 1 update, 2 apply backward
                             // (the one-tile-per-block kernels of the update and the apply backward, whose pointwise epilogues run on all
@@ -333,7 +333,21 @@ struct Runner {
   Runner(const Plan& p, void* saved, void* scratch, hipStream_t st)
       : P(p), s(st), sv(align256(saved)), sc(align256(scratch)), d(p.d), s_main(st), s_side(st), hsel(p.t_h), partial_sel(p.t_partial) {
     side = side_ctx();
-    if (side && g_overlap && !P.groups.empty()) s_side = side->stream;
+    if (side && !P.groups.empty() && overlap_pays(p, st)) s_side = side->stream;
+  }
+  // Apply steps beside the update chain: what is hidden against the events of the forks and joins, 60 to 100 us of host time a training step
+  // and 6 us on the GPU each.  us of a training step, overlapped / in line, by 1e9 operations of the apply steps (Plan::side_work): 0.13
+  // (1 fp32 head of 64, 700 tokens) 350 / 256; 1.1 (4 x 3000 tokens, d = dh = 128) 318 / 256; 2.8 (6 x 3000, 128 x 256) 295 / 270; 4.4 (2 x 3000,
+  // 256 x 512) 424 / 432; 4.7 (4 x 4000, 256) 331 / 336; 10.6 (16 x 4000, 192) 535 / 587; 24 784 / 888; 108 2600 / 2850; fp32 11 410 / 405 and 33
+  // 795 / 847.  With Newton-Schulz the GPU is the longer side earlier: 0.2 (3 x 1500, 96) 641 / 572; 1.3 (16 x 1200, 128) 361 / 366; beyond
+  // 128 features, where its matrices take several blocks each, always: 1.2 (2 x 1400, 384) 318 / 349.  A captured call pays no host time.
+  static bool overlap_pays(const Plan& P, hipStream_t st) {
+    if (g_overlap != 1) return g_overlap > 1;
+    if (P.side_work >= (!P.muon ? 4e9 : P.d.d <= 128 ? 1e9 : 0.)) return true;
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
+    (void)hipGetLastError();      // (the legacy stream beside another one's capture: the launches will say so)
+    return false;
   }
   // ---- fused Newton-Schulz: launches of at most 256 resident blocks
   static bool tiles_fit(int r, int c, int bm, int bn) {
@@ -2004,7 +2018,12 @@ int lact_set_option(int32_t option, int32_t value) {
     g_persist = value;
     return was;
   }
-  bool* flag = option == LACT_OPT_STREAM_OVERLAP ? &g_overlap : (option == LACT_OPT_FUSED_NEWTON_SCHULZ ? &g_fused_ns : nullptr);
+  if (option == LACT_OPT_STREAM_OVERLAP) {
+    const int was = g_overlap;
+    g_overlap = value > 1 ? 2 : (value != 0);
+    return was;
+  }
+  bool* flag = option == LACT_OPT_FUSED_NEWTON_SCHULZ ? &g_fused_ns : nullptr;
   if (!flag) return fail("lact_set_option: unknown option");
   const int was = *flag ? 1 : 0;
   *flag = value != 0;

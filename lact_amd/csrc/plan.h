@@ -115,6 +115,7 @@ struct Plan {
   std::vector<float> coeffs;
   MatGeom g;
   int nupd = 0, Tcap = 0, Tupd = 1, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 1024, kl_begin = 0, kl_end = 0, side_slots = 1;
+  double side_work = 0;   // of the grouped apply steps' forward, in operations of bf16
   int nw = 0;       // initial weights and their gradients: matrices of each kind, batch entry i uses i % nw
   bool muon = false, bf16 = true, momentum = false, state_in = false;
   size_t mat3 = 0;  // 3*b*elems
@@ -335,12 +336,14 @@ struct Plan {
     gw_slot.assign(nupd + 1, -1);
     gw_slots = 0;
     Tnew = 0;
+    side_work = 0;
     int ver = 0;
     for (const auto& st : live) {
       if (st.kind == LACT_UPDATE) { ++ver; continue; }
       const int T = st.end - st.start;
       if (ver == nupd) { Tnew = std::max(Tnew, T); continue; }
       if (gw_slot[ver] < 0) gw_slot[ver] = gw_slots++;
+      side_work += 6.0 * T * d.d * d.dh * d.b * (bf16 ? 1 : 9);      // (fp32 products run at a ninth of the rate)
       const long long tiles1 = (long long)ceil_div(T, 128) * ceil_div(d.dh, 128) * d.b;
       const int limit = (int)std::max(1LL, std::min(std::min(65535LL / (3 * d.b), 64LL), (256 + tiles1 - 1) / tiles1));
       if (!groups.empty()) {

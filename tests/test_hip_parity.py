@@ -1126,6 +1126,38 @@ def test_stream_overlap_is_bit_identical(prenorm):
     assert torch.equal(on[0][0], on[2][0]) and all(torch.equal(on[0][1][n], on[2][1][n]) for n in on[0][1])
 
 
+@pytest.mark.parametrize("body", ["identical", "streams", "threads", "captured"])
+def test_stream_overlap_of_small_programs(body):
+    """Apply steps too short to pay for the second stream's events run in line by default: forced onto it, the same bits, and so
+    from two streams and two threads; on either side of the line the default gives the bits of one stream."""
+    say("stream overlap forced", body)
+    from lact_amd import _lib
+    L_ = _lib.lib()
+    prev = L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, 2)
+    try:
+        if body == "streams":
+            return test_calls_on_two_caller_streams()
+        if body == "threads":
+            return test_calls_from_two_host_threads()
+        if body == "captured":
+            return test_graph_capture_replays_match_eager()
+        for dtype, b, d, L, C in ((torch.bfloat16, 2, 128, 700, 100), (torch.float32, 2, 64, 300, 90), (torch.bfloat16, 8, 256, 4 * 512, 512),
+                                  (torch.bfloat16, 12, 256, 5 * 512, 512)):      # 0.06 to 9.7 thousand million operations; the line is at 4
+            inp = problem(b, L, d, d, seed=78, act=dtype)
+            go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(5)).to(dtype).to(DEV)
+            res = []
+            for mode in (2, 1, 0):
+                L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, mode)
+                t = clone_to(inp, DEV)
+                out = T.block_causal_lact_swiglu(*args9(t), C, False, t["momentum"])
+                res.append([out, *grads_of(out, t, go).values()])
+            for other in res[1:]:
+                assert all(torch.equal(a, r) for a, r in zip(res[0], other))
+    finally:
+        L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, prev)
+
+
+
 @pytest.mark.parametrize("b,L,d,dh,C,muon", [
     (2, 3 * 128 + 40, 128, 128, 128, False),      # ragged last token tile, one hidden tile
     (3, 2 * 300 + 50, 64, 192, 300, True),        # dh = 128 + 64: a half-valid hidden tile; chunk not a multiple of 128

@@ -21,8 +21,13 @@
 // that: its two accumulators and its own rows fill 192 of 256, and with half the waves and 512 registers each the vector
 // work on accumulators in the second register file and the bare barriers cost more than the order gained (434 us against 394).
 //
-// Measured at B = 4, L = 4096, window 2048, 12 heads of 128, before / now: forward 226 / 178 us (50 % of the matrix pipes' time), dq 292 / 247
-// (54 %), dk and dv 460 / 394.  Of that a tenth is the order of the blocks (locate).  Tried: the waves of a SIMD taking turns at the
+// Heads of 64 have as much vector work for half the products, and without a second tile's scores (119 and 128 registers instead of 186
+// and 180) two blocks of eight waves fit a compute unit, which overlap better than one that forms them ahead: 4 x 24 heads, 4096 tokens, window
+// 2048 / 512, forward 197 / 89 us against 214 / 108, dq 241 / 106 against 280 / 139.
+//
+// Measured at B = 4, L = 4096, window 2048, 12 heads of 128, before / now: forward 205 / 170 us (50 % of the matrix pipes' time), dq 260 / 238
+// (54 %), dk and dv 402 / 350.  Of that a tenth is the order of the blocks (locate); the copies of dk/dv are two tiles ahead (three, or
+// past the last tile without a branch, cost up to 3 % where a block has few).  Tried: the waves of a SIMD taking turns at the
 // matrix pipe behind barriers (forward 208, dq 333); wave priorities that alternate from tile to tile (nothing); torch's masked
 // attention over window-sized blocks: 930 and 3400 us, plus building its masks and copying around it.  A single
 // backward pass over the keys with atomic adds into dq would save two of the seven products and is not deterministic.
@@ -181,6 +186,9 @@ __device__ __forceinline__ void attn_store_rows(char* lds, const f32x16 (&acc)[D
   wave_lds_fence();
 }
 
+// Heads of 128 form scores a tile ahead (forward and dq); of 64, where two blocks of eight waves share a compute unit, tile after tile.
+template <int D> constexpr bool attn_ahead() { return D == 128; }
+template <int D> constexpr int attn_waves() { return attn_ahead<D>() ? 2 : 4; }     // a SIMD's, forward and dq
 constexpr float ATTN_LOG2E = 1.4426950408889634f;
 constexpr int ATTN_RING = 4;   // slots of two tiles
 template <int D, int NW>
@@ -208,8 +216,22 @@ __device__ __forceinline__ void attn_walk(int n, Odd odd, Even even) {
   wait_vmcnt<0>();
 }
 
+// Walks the tiles [0, n) one after the other: issue(t) starts the copies of tile t, COPIES of a wave, two tiles ahead; body(t) uses it.
+template <int COPIES, typename Issue, typename Body>
+__device__ __forceinline__ void attn_walk_in_order(int n, Issue issue, Body body) {
+  issue(0);
+  if (n > 1) issue(1);
+  for (int t = 0; t < n; ++t) {
+    if (t + 1 < n) wait_vmcnt<COPIES>();
+    else wait_vmcnt<0>();
+    __syncthreads();      // tile t is there for every wave, and all are through with t - 1
+    if (t + 2 < n) issue(t + 2);
+    body(t);
+  }
+}
+
 template <int D, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_fwd(const WindowAttnParams p) {
+__global__ __launch_bounds__(64 * NW, NW == 8 ? attn_waves<D>() : 1) void k_window_attn_fwd(const WindowAttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using T = AttnTile<D>;
   using Copy = AttnCopy<D, NW>;
@@ -242,111 +264,8 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_fwd(co
   const int ta = max(0, row0 - p.window + 1 - first) / 64, tb = (min(row0 + 31, last - 1) - first) / 64 + 1;   // the tiles in the wave's windows
   auto in_reach = [&](int t) { return t >= ta && t < tb; };
   constexpr int COPIES = 2 * Copy::NC;
-  // Step t brings the keys of tile t + 3 and the values of t + 2, which the next two steps do not use yet: one barrier for every two
-  auto issue = [&](int t, int i) LACT_INLINE_LAMBDA {
-    if (i < Copy::NC) ck.issue(t + 3, i, lds0 + (t + 3) % ATTN_RING * STAGE, wave);
-    else cv.issue(t + 2, i - Copy::NC, lds0 + (t + 2) % ATTN_RING * STAGE + T::BYTES, wave);
-  };
-  // Step t: the exponentials of tile t between the matrix instructions that form the scores of t + 1, then the product with them,
-  // the maximum of the new scores between its instructions.
-  auto step = [&](int t, f32x16 (&cur)[2], f32x16 (&nxt)[2]) LACT_INLINE_LAMBDA {
-    const bool here = in_reach(t), ahead = in_reach(t + 1);
-    if (!here) {
-#pragma unroll
-      for (int i = 0; i < COPIES; ++i) issue(t, i);
-      if (!ahead) return;
-    }
-    const char* kt = smem + (t + 1) % ATTN_RING * STAGE;
-    const char* vt = smem + t % ATTN_RING * STAGE + T::BYTES;
-    bf16x8 vb[4];
-    uint32_t pw[16];
-    bf16x8 kb[3][2];
-    auto keys = [&](int ks) LACT_INLINE_LAMBDA {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) kb[ks % 3][i] = fr.rows(kt, i, ks);
-    };
-    constexpr int KS = D / 16;
-    keys(0);
-    keys(1);
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 16; ++j) nxt[i][j] = 0.f;
-    if (here) {
-#pragma unroll
-      for (int i = 0; i < 3; ++i) vb[i] = fr.cols(vt, i % (D / 32), i / (D / 32));
-      float part[4] = {0.f, 0.f, 0.f, 0.f};
-      // two scores a step and instruction: product and offset, exponential, sum and conversion one step behind each other
-      constexpr int PER = 16 / (2 * KS);      // pairs per matrix instruction
-      auto soft = [&](int e) LACT_INLINE_LAMBDA {
-#pragma unroll
-        for (int x = 2 * e; x < 2 * e + 2; ++x)
-          if (x < 32) cur[x / 16][x % 16] = fmaf(cur[x / 16][x % 16], c, -mc);
-#pragma unroll
-        for (int x = 2 * e - 2; x < 2 * e; ++x)
-          if (x >= 0 && x < 32) cur[x / 16][x % 16] = __builtin_amdgcn_exp2f(cur[x / 16][x % 16]);
-        const int x = 2 * e - 4;
-        if (x >= 0) {
-          part[(e & 1) * 2] += cur[x / 16][x % 16];
-          part[(e & 1) * 2 + 1] += cur[x / 16][x % 16 + 1];
-          pw[x / 2] = pack_bf16(cur[x / 16][x % 16], cur[x / 16][x % 16 + 1]);
-        }
-      };
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 2 < KS) keys(ks + 2);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) {
-          nxt[i] = mma32(kb[ks % 3][i], qf[ks], nxt[i]);
-          if ((ks * 2 + i) % (2 * KS / COPIES) == 1 % (2 * KS / COPIES)) issue(t, (ks * 2 + i) / (2 * KS / COPIES));
-#pragma unroll
-          for (int e = 0; e < PER; ++e) soft((ks * 2 + i) * PER + e);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      }
-      soft(16);
-      soft(17);
-      sum += (part[0] + part[1]) + (part[2] + part[3]);
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 2 < KS) keys(ks + 2);
-#pragma unroll
-        for (int i = 0; i < 2; ++i) nxt[i] = mma32(kb[ks % 3][i], qf[ks], nxt[i]);
-      }
-    }
-    const int k0 = first + (t + 1) * 64;
-    if (ahead && (k0 + 63 > row0 || k0 < row0 + 31 - p.window + 1)) {
-      const int lo = row - p.window - k0 - 4 * (lane >> 5), hi = row - k0 - 4 * (lane >> 5);
-#pragma unroll
-      for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 16; ++j) {
-          const int key = i * 32 + 8 * (j / 4) + j % 4;
-          nxt[i][j] = (key <= hi && key > lo) ? nxt[i][j] : -__builtin_inff();
-        }
-    }
-    float m4[4] = {nxt[0][0], nxt[1][0], nxt[0][1], nxt[1][1]};
-    auto larger = [](float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); };   // one instruction; fmaxf quiets its operands first
-    if (here) {
-      constexpr int DT = D / 32, MM = 4 * DT;
-#pragma unroll
-      for (int e = 0; e < MM; ++e) {
-        if (e + 3 < MM) vb[(e + 3) % 4] = fr.cols(vt, (e + 3) % DT, (e + 3) / DT);
-        const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[4 * (e / DT)], pw[4 * (e / DT) + 1], pw[4 * (e / DT) + 2], pw[4 * (e / DT) + 3]));
-        o[e % DT] = mma32(vb[e % 4], pf, o[e % DT]);
-#pragma unroll
-        for (int j = e * 16 / MM; j < (e + 1) * 16 / MM; ++j)
-          if (j >= 2) { m4[2 * (j & 1)] = larger(m4[2 * (j & 1)], nxt[0][j]); m4[2 * (j & 1) + 1] = larger(m4[2 * (j & 1) + 1], nxt[1][j]); }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    } else {
-#pragma unroll
-      for (int j = 2; j < 16; ++j) { m4[2 * (j & 1)] = larger(m4[2 * (j & 1)], nxt[0][j]); m4[2 * (j & 1) + 1] = larger(m4[2 * (j & 1) + 1], nxt[1][j]); }
-    }
-    if (!ahead) return;
-    float mx = larger(larger(m4[0], m4[1]), larger(m4[2], m4[3])) * c;   // of this lane's half of the row
-    // The maximum only has to keep exp2 in range: it follows the row when it is exceeded by more than 2^8.
+  // The maximum only has to keep exp2 in range: it follows the row when it is exceeded by more than 2^8.
+  auto follow = [&](float mx) LACT_INLINE_LAMBDA {     // of this lane's half of the row
     if (__any(mx > mc + 8.f)) {
       mx = fmaxf(mx, __shfl_xor(mx, 32, 64));
       const float nm = fmaxf(mc, mx), f = __builtin_amdgcn_exp2f(mc - nm);
@@ -358,15 +277,168 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_fwd(co
         for (int j = 0; j < 16; ++j) o[i][j] *= f;
     }
   };
-  f32x16 s[2][2];
+  auto mask = [&](int k0, f32x16 (&s)[2]) LACT_INLINE_LAMBDA {
+    if (k0 + 63 > row0 || k0 < row0 + 31 - p.window + 1) {
+      const int lo = row - p.window - k0 - 4 * (lane >> 5), hi = row - k0 - 4 * (lane >> 5);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const int key = i * 32 + 8 * (j / 4) + j % 4;
+          s[i][j] = (key <= hi && key > lo) ? s[i][j] : -__builtin_inff();
+        }
+    }
+  };
+  auto larger = [](float a, float b) { return __builtin_amdgcn_fmed3f(a, b, __builtin_inff()); };   // one instruction; fmaxf quiets its operands first
   attn_arrived(qf);
+  if constexpr (!attn_ahead<D>()) {
+    attn_walk_in_order<COPIES>(tiles,
+      [&](int t) LACT_INLINE_LAMBDA {
+        const uint32_t slot = lds0 + t % ATTN_RING * STAGE;
 #pragma unroll
-  for (int t = -3; t < -1; ++t)
+        for (int i = 0; i < Copy::NC; ++i) {
+          ck.issue(t, i, slot, wave);
+          cv.issue(t, i, slot + T::BYTES, wave);
+        }
+      },
+      [&](int t) LACT_INLINE_LAMBDA {
+        if (!in_reach(t)) return;
+        const char* kt = smem + t % ATTN_RING * STAGE;
+        const char* vt = kt + T::BYTES;
+        f32x16 s[2];
 #pragma unroll
-    for (int i = 0; i < COPIES; ++i)
-      if (t == -2 || i < Copy::NC) issue(t, i);
-  attn_walk<COPIES, false>(tiles,
-    [&](int t) LACT_INLINE_LAMBDA { step(t, s[1], s[0]); }, [&](int t) LACT_INLINE_LAMBDA { step(t, s[0], s[1]); });
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) s[i][j] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < D / 16; ++ks)
+#pragma unroll
+          for (int i = 0; i < 2; ++i) s[i] = mma32(fr.rows(kt, i, ks), qf[ks], s[i]);
+        mask(first + t * 64, s);
+        float mx = larger(s[0][0], s[1][0]);
+#pragma unroll
+        for (int j = 1; j < 16; ++j) mx = larger(mx, larger(s[0][j], s[1][j]));
+        follow(mx * c);
+        float part[2] = {0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 16; ++j) {
+            s[i][j] = __builtin_amdgcn_exp2f(fmaf(s[i][j], c, -mc));
+            part[i] += s[i][j];
+          }
+        sum += part[0] + part[1];
+#pragma unroll
+        for (int st = 0; st < 4; ++st) {
+          const bf16x8 pf = attn_pack(s[st >> 1], st & 1);
+#pragma unroll
+          for (int dt = 0; dt < D / 32; ++dt) o[dt] = mma32(fr.cols(vt, dt, st), pf, o[dt]);
+        }
+      });
+  } else {
+    // Step t brings the keys of tile t + 3 and the values of t + 2, which the next two steps do not use yet: one barrier for every two
+    auto issue = [&](int t, int i) LACT_INLINE_LAMBDA {
+      if (i < Copy::NC) ck.issue(t + 3, i, lds0 + (t + 3) % ATTN_RING * STAGE, wave);
+      else cv.issue(t + 2, i - Copy::NC, lds0 + (t + 2) % ATTN_RING * STAGE + T::BYTES, wave);
+    };
+    // Step t: the exponentials of tile t between the matrix instructions that form the scores of t + 1, then the product with them,
+    // the maximum of the new scores between its instructions.
+    auto step = [&](int t, f32x16 (&cur)[2], f32x16 (&nxt)[2]) LACT_INLINE_LAMBDA {
+      const bool here = in_reach(t), ahead = in_reach(t + 1);
+      if (!here) {
+#pragma unroll
+        for (int i = 0; i < COPIES; ++i) issue(t, i);
+        if (!ahead) return;
+      }
+      const char* kt = smem + (t + 1) % ATTN_RING * STAGE;
+      const char* vt = smem + t % ATTN_RING * STAGE + T::BYTES;
+      bf16x8 vb[4];
+      uint32_t pw[16];
+      bf16x8 kb[3][2];
+      auto keys = [&](int ks) LACT_INLINE_LAMBDA {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) kb[ks % 3][i] = fr.rows(kt, i, ks);
+      };
+      constexpr int KS = D / 16;
+      keys(0);
+      keys(1);
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) nxt[i][j] = 0.f;
+      if (here) {
+#pragma unroll
+        for (int i = 0; i < 3; ++i) vb[i] = fr.cols(vt, i % (D / 32), i / (D / 32));
+        float part[4] = {0.f, 0.f, 0.f, 0.f};
+        // two scores a step and instruction: product and offset, exponential, sum and conversion one step behind each other
+        constexpr int PER = 16 / (2 * KS);      // pairs per matrix instruction
+        auto soft = [&](int e) LACT_INLINE_LAMBDA {
+#pragma unroll
+          for (int x = 2 * e; x < 2 * e + 2; ++x)
+            if (x < 32) cur[x / 16][x % 16] = fmaf(cur[x / 16][x % 16], c, -mc);
+#pragma unroll
+          for (int x = 2 * e - 2; x < 2 * e; ++x)
+            if (x >= 0 && x < 32) cur[x / 16][x % 16] = __builtin_amdgcn_exp2f(cur[x / 16][x % 16]);
+          const int x = 2 * e - 4;
+          if (x >= 0) {
+            part[(e & 1) * 2] += cur[x / 16][x % 16];
+            part[(e & 1) * 2 + 1] += cur[x / 16][x % 16 + 1];
+            pw[x / 2] = pack_bf16(cur[x / 16][x % 16], cur[x / 16][x % 16 + 1]);
+          }
+        };
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          if (ks + 2 < KS) keys(ks + 2);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) {
+            nxt[i] = mma32(kb[ks % 3][i], qf[ks], nxt[i]);
+            if ((ks * 2 + i) % (2 * KS / COPIES) == 1 % (2 * KS / COPIES)) issue(t, (ks * 2 + i) / (2 * KS / COPIES));
+#pragma unroll
+            for (int e = 0; e < PER; ++e) soft((ks * 2 + i) * PER + e);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        soft(16);
+        soft(17);
+        sum += (part[0] + part[1]) + (part[2] + part[3]);
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          if (ks + 2 < KS) keys(ks + 2);
+#pragma unroll
+          for (int i = 0; i < 2; ++i) nxt[i] = mma32(kb[ks % 3][i], qf[ks], nxt[i]);
+        }
+      }
+      if (ahead) mask(first + (t + 1) * 64, nxt);
+      float m4[4] = {nxt[0][0], nxt[1][0], nxt[0][1], nxt[1][1]};
+      if (here) {
+        constexpr int DT = D / 32, MM = 4 * DT;
+#pragma unroll
+        for (int e = 0; e < MM; ++e) {
+          if (e + 3 < MM) vb[(e + 3) % 4] = fr.cols(vt, (e + 3) % DT, (e + 3) / DT);
+          const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[4 * (e / DT)], pw[4 * (e / DT) + 1], pw[4 * (e / DT) + 2], pw[4 * (e / DT) + 3]));
+          o[e % DT] = mma32(vb[e % 4], pf, o[e % DT]);
+#pragma unroll
+          for (int j = e * 16 / MM; j < (e + 1) * 16 / MM; ++j)
+            if (j >= 2) { m4[2 * (j & 1)] = larger(m4[2 * (j & 1)], nxt[0][j]); m4[2 * (j & 1) + 1] = larger(m4[2 * (j & 1) + 1], nxt[1][j]); }
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int j = 2; j < 16; ++j) { m4[2 * (j & 1)] = larger(m4[2 * (j & 1)], nxt[0][j]); m4[2 * (j & 1) + 1] = larger(m4[2 * (j & 1) + 1], nxt[1][j]); }
+      }
+      if (!ahead) return;
+      follow(larger(larger(m4[0], m4[1]), larger(m4[2], m4[3])) * c);
+    };
+    f32x16 s[2][2];
+#pragma unroll
+    for (int t = -3; t < -1; ++t)
+#pragma unroll
+      for (int i = 0; i < COPIES; ++i)
+        if (t == -2 || i < Copy::NC) issue(t, i);
+    attn_walk<COPIES, false>(tiles,
+      [&](int t) LACT_INLINE_LAMBDA { step(t, s[1], s[0]); }, [&](int t) LACT_INLINE_LAMBDA { step(t, s[0], s[1]); });
+  }
   sum += __shfl_xor(sum, 32, 64);
   if (lane < 32 && row < L) p.lse[(size_t)z * L + row] = mc + __builtin_amdgcn_logf(sum);   // v_log_f32 is base 2
   __syncthreads();
@@ -375,7 +447,7 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_fwd(co
 
 // dq = scale * sum_keys p (dp - delta) k, and delta itself.
 template <int D, int NW>
-__global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_dq(const WindowAttnParams p) {
+__global__ __launch_bounds__(64 * NW, NW == 8 ? attn_waves<D>() : 1) void k_window_attn_dq(const WindowAttnParams p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   using T = AttnTile<D>;
   using Copy = AttnCopy<D, NW>;
@@ -426,88 +498,123 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_dq(con
     if (i < Copy::NC) ck.issue(t, i, slot, wave);
     else cv.issue(t, i - Copy::NC, slot + T::BYTES, wave);
   };
-  // Half tile u: its probabilities and their gradients between the matrix instructions that form the two products of u + 1, then the product with them.
-  auto step = [&](int u, Scores& cur, Scores& nxt) LACT_INLINE_LAMBDA {
-    const bool here = in_reach(u), ahead = in_reach(u + 1);
-    const int t = (u + 2) / 2 - 1, part0 = (u & 1) * HALF;    // the half tile's share of its tile's copies
-    if (!here) {
-#pragma unroll
-      for (int i = 0; i < HALF; ++i) issue(t + 3, part0 + i);
-      if (!ahead) return;
-    }
-    const char* kn = smem + (u + 1) / 2 % ATTN_RING * STAGE;
-    const int in = (u + 1) & 1, iu = u & 1;
-    constexpr int KS = D / 16, DT = D / 32;
-    bf16x8 kb[2], vb[2], cb[3];
-    kb[0] = fr.rows(kn, in, 0);
-    vb[0] = fr.rows(kn + T::BYTES, in, 0);
-#pragma unroll
-    for (int j = 0; j < 16; ++j) nxt.s[j] = nxt.dp[j] = 0.f;
-    uint32_t pw[8];
-    constexpr int PER = 16 / (2 * KS);
-    auto soft = [&](int j) LACT_INLINE_LAMBDA {     // one score a step: product and offset, exponential, gradient one step behind each other
-      if (j < 16) cur.s[j] = fmaf(cur.s[j], c, -lse);
-      if (j >= 1 && j < 17) { cur.s[j - 1] = __builtin_amdgcn_exp2f(cur.s[j - 1]); cur.dp[j - 1] -= delta; }
-      if (j >= 2 && j < 18) cur.s[j - 2] *= cur.dp[j - 2];
-      if (j >= 3 && (j & 1)) pw[(j - 3) / 2] = pack_bf16(cur.s[j - 3], cur.s[j - 2]);
-    };
-    if (here) {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 1 < KS) { kb[(ks + 1) % 2] = fr.rows(kn, in, ks + 1); vb[(ks + 1) % 2] = fr.rows(kn + T::BYTES, in, ks + 1); }
-        nxt.s = mma32(kb[ks % 2], qf[ks], nxt.s);
-        if (ks % (KS / HALF) == 0) issue(t + 3, part0 + ks / (KS / HALF));
-#pragma unroll
-        for (int e = 0; e < PER; ++e) soft(2 * ks * PER + e);
-        __builtin_amdgcn_sched_barrier(0);
-        nxt.dp = mma32(vb[ks % 2], gf[ks], nxt.dp);
-#pragma unroll
-        for (int e = 0; e < PER; ++e) soft((2 * ks + 1) * PER + e);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      const char* kt = smem + u / 2 % ATTN_RING * STAGE;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) cb[i] = fr.cols(kt, i % DT, 2 * iu + i / DT);
-      soft(16);
-      soft(17);
-#pragma unroll
-      for (int e = 0; e < 2 * DT; ++e) {
-        if (e + 2 < 2 * DT) cb[(e + 2) % 3] = fr.cols(kt, (e + 2) % DT, 2 * iu + (e + 2) / DT);
-        const int st = e / DT;
-        const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]));
-        o[e % DT] = mma32(cb[e % 3], pf, o[e % DT]);
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < KS; ++ks) {
-        if (ks + 1 < KS) { kb[(ks + 1) % 2] = fr.rows(kn, in, ks + 1); vb[(ks + 1) % 2] = fr.rows(kn + T::BYTES, in, ks + 1); }
-        nxt.s = mma32(kb[ks % 2], qf[ks], nxt.s);
-        nxt.dp = mma32(vb[ks % 2], gf[ks], nxt.dp);
-      }
-    }
-    const int k0 = first + (u + 1) * 32;
-    if (ahead && (k0 + 31 > row0 || k0 < row0 + 31 - p.window + 1)) {
+  auto mask = [&](int k0, f32x16& s) LACT_INLINE_LAMBDA {
+    if (k0 + 31 > row0 || k0 < row0 + 31 - p.window + 1) {
       const int lo = row - p.window - k0 - 4 * (lane >> 5), hi = row - k0 - 4 * (lane >> 5);
 #pragma unroll
       for (int j = 0; j < 16; ++j) {
         const int key = 8 * (j / 4) + j % 4;
-        nxt.s[j] = (key <= hi && key > lo) ? nxt.s[j] : -__builtin_inff();
+        s[j] = (key <= hi && key > lo) ? s[j] : -__builtin_inff();
       }
     }
-  };
-  Scores sc[2];
-  auto tile = [&](int t) LACT_INLINE_LAMBDA {
-    step(2 * t, sc[0], sc[1]);
-    step(2 * t + 1, sc[1], sc[0]);
   };
   attn_arrived(qf);
   attn_arrived(gf);
   asm volatile("" : "+v"(lse), "+v"(delta));
+  if constexpr (!attn_ahead<D>()) {
+    attn_walk_in_order<COPIES>(tiles,
+      [&](int t) LACT_INLINE_LAMBDA {
 #pragma unroll
-  for (int t = 0; t < 2; ++t)
+        for (int i = 0; i < COPIES; ++i) issue(t, i);
+      },
+      [&](int t) LACT_INLINE_LAMBDA {
+        const char* kt = smem + t % ATTN_RING * STAGE;
+        const char* vt = kt + T::BYTES;
 #pragma unroll
-    for (int i = 0; i < COPIES; ++i) issue(t, i);
-  attn_walk<COPIES, true>(tiles, tile, tile);
+        for (int i = 0; i < 2; ++i) {
+          if (!in_reach(2 * t + i)) continue;
+          f32x16 s, dp;
+#pragma unroll
+          for (int j = 0; j < 16; ++j) s[j] = dp[j] = 0.f;
+#pragma unroll
+          for (int ks = 0; ks < D / 16; ++ks) {
+            s = mma32(fr.rows(kt, i, ks), qf[ks], s);
+            dp = mma32(fr.rows(vt, i, ks), gf[ks], dp);
+          }
+          mask(first + t * 64 + i * 32, s);
+#pragma unroll
+          for (int j = 0; j < 16; ++j) s[j] = __builtin_amdgcn_exp2f(fmaf(s[j], c, -lse)) * (dp[j] - delta);
+#pragma unroll
+          for (int st = 0; st < 2; ++st) {
+            const bf16x8 pf = attn_pack(s, st);
+#pragma unroll
+            for (int dt = 0; dt < D / 32; ++dt) o[dt] = mma32(fr.cols(kt, dt, 2 * i + st), pf, o[dt]);
+          }
+        }
+      });
+  } else {
+    // Half tile u: its probabilities and their gradients between the matrix instructions that form the two products of u + 1, then the product with them.
+    auto step = [&](int u, Scores& cur, Scores& nxt) LACT_INLINE_LAMBDA {
+      const bool here = in_reach(u), ahead = in_reach(u + 1);
+      const int t = (u + 2) / 2 - 1, part0 = (u & 1) * HALF;    // the half tile's share of its tile's copies
+      if (!here) {
+#pragma unroll
+        for (int i = 0; i < HALF; ++i) issue(t + 3, part0 + i);
+        if (!ahead) return;
+      }
+      const char* kn = smem + (u + 1) / 2 % ATTN_RING * STAGE;
+      const int in = (u + 1) & 1, iu = u & 1;
+      constexpr int KS = D / 16, DT = D / 32;
+      bf16x8 kb[2], vb[2], cb[3];
+      kb[0] = fr.rows(kn, in, 0);
+      vb[0] = fr.rows(kn + T::BYTES, in, 0);
+#pragma unroll
+      for (int j = 0; j < 16; ++j) nxt.s[j] = nxt.dp[j] = 0.f;
+      uint32_t pw[8];
+      constexpr int PER = 16 / (2 * KS);
+      auto soft = [&](int j) LACT_INLINE_LAMBDA {     // one score a step: product and offset, exponential, gradient one step behind each other
+        if (j < 16) cur.s[j] = fmaf(cur.s[j], c, -lse);
+        if (j >= 1 && j < 17) { cur.s[j - 1] = __builtin_amdgcn_exp2f(cur.s[j - 1]); cur.dp[j - 1] -= delta; }
+        if (j >= 2 && j < 18) cur.s[j - 2] *= cur.dp[j - 2];
+        if (j >= 3 && (j & 1)) pw[(j - 3) / 2] = pack_bf16(cur.s[j - 3], cur.s[j - 2]);
+      };
+      if (here) {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          if (ks + 1 < KS) { kb[(ks + 1) % 2] = fr.rows(kn, in, ks + 1); vb[(ks + 1) % 2] = fr.rows(kn + T::BYTES, in, ks + 1); }
+          nxt.s = mma32(kb[ks % 2], qf[ks], nxt.s);
+          if (ks % (KS / HALF) == 0) issue(t + 3, part0 + ks / (KS / HALF));
+#pragma unroll
+          for (int e = 0; e < PER; ++e) soft(2 * ks * PER + e);
+          __builtin_amdgcn_sched_barrier(0);
+          nxt.dp = mma32(vb[ks % 2], gf[ks], nxt.dp);
+#pragma unroll
+          for (int e = 0; e < PER; ++e) soft((2 * ks + 1) * PER + e);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        const char* kt = smem + u / 2 % ATTN_RING * STAGE;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) cb[i] = fr.cols(kt, i % DT, 2 * iu + i / DT);
+        soft(16);
+        soft(17);
+#pragma unroll
+        for (int e = 0; e < 2 * DT; ++e) {
+          if (e + 2 < 2 * DT) cb[(e + 2) % 3] = fr.cols(kt, (e + 2) % DT, 2 * iu + (e + 2) / DT);
+          const int st = e / DT;
+          const bf16x8 pf = __builtin_bit_cast(bf16x8, make_uint4(pw[4 * st], pw[4 * st + 1], pw[4 * st + 2], pw[4 * st + 3]));
+          o[e % DT] = mma32(cb[e % 3], pf, o[e % DT]);
+        }
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          if (ks + 1 < KS) { kb[(ks + 1) % 2] = fr.rows(kn, in, ks + 1); vb[(ks + 1) % 2] = fr.rows(kn + T::BYTES, in, ks + 1); }
+          nxt.s = mma32(kb[ks % 2], qf[ks], nxt.s);
+          nxt.dp = mma32(vb[ks % 2], gf[ks], nxt.dp);
+        }
+      }
+      if (ahead) mask(first + (u + 1) * 32, nxt.s);
+    };
+    Scores sc[2];
+    auto tile = [&](int t) LACT_INLINE_LAMBDA {
+      step(2 * t, sc[0], sc[1]);
+      step(2 * t + 1, sc[1], sc[0]);
+    };
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int i = 0; i < COPIES; ++i) issue(t, i);
+    attn_walk<COPIES, true>(tiles, tile, tile);
+  }
   __syncthreads();
   attn_store_rows<D>(smem + wave * 32 * (D + 8) * 2, o, p.scale, p.dq + ((size_t)b * L * p.H + h) * D, (size_t)p.H * D, row0, L);
 }
@@ -556,12 +663,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_dkv(co
       cq.issue(t, i, lds0 + slot * STAGE, wave);
       cg.issue(t, i, lds0 + slot * STAGE + T::BYTES, wave);
     }
-    const int q0 = first + min(t, tiles - 1) * 64;
+    const int q0 = first + t * 64;
     dma4(st_src + q0, (uint32_t)min(lane, L - 1 - q0) * 4, lds0 + ATTN_RING * STAGE + slot * 512 + (wave & 1) * 256);
   };
   auto tile = [&](int t) LACT_INLINE_LAMBDA {
-    issue_all(t + 3);
-    if (t < 0 || t >= tiles) return;
     const int slot = t % ATTN_RING;
     const char* qt = smem + slot * STAGE;
     const char* gt = qt + T::BYTES;
@@ -608,12 +713,10 @@ __global__ __launch_bounds__(64 * NW, NW == 8 ? 2 : 1) void k_window_attn_dkv(co
         }
       }
     }
-    };
+  };
   attn_arrived(kf);
   attn_arrived(vf);
-  issue_all(0);
-  issue_all(1);
-  attn_walk<COPIES, true>(tiles, tile, tile);
+  attn_walk_in_order<COPIES>(tiles, issue_all, tile);
   __syncthreads();
   const size_t o = ((size_t)b * L * p.H + h) * D;
   attn_store_rows<D>(smem + wave * 32 * (D + 8) * 2, ok, p.scale, p.dk + o, (size_t)p.H * D, row0, L);

@@ -33,7 +33,10 @@ def test_window_attention_against_oracle(b, l, h, d, window):
     (1, 70, 2, 128, 1, 1.0),        # every query sees itself alone
     (2, 300, 64, 64, 64, 1.0),      # 256-row blocks of heads of 64, the window one tile
     (1, 515, 3, 128, 190, 40.0),    # scores that grow along the sequence: the rows' maxima follow them from tile to tile
-    (2, 600, 70, 128, 600, 300.0)])
+    (2, 600, 70, 128, 600, 300.0),
+    (1, 70, 2, 64, 1, 1.0),         # heads of 64 walk their tiles one after the other
+    (1, 515, 3, 64, 190, 40.0),
+    (2, 600, 70, 64, 600, 300.0)])
 def test_window_attention_scores_and_window_edges(b, l, h, d, window, growth):
     """The scores of a tile are formed one step ahead of their exponentials: window edges inside and on the tiles, and maxima that grow
     from tile to tile by far more than exp2 reaches.  Grown scores leave a handful of probabilities per row, which bf16 rounds to 2^-9

@@ -77,12 +77,15 @@ struct NsFusedParams {
 
 struct GroupBarrier {
   unsigned* ctr;
-  unsigned* sticky;          // per-device count of timed-out waits, never cleared by a kernel (lact_check_async_error reads it)
+  unsigned* sticky;          // per-device count of blocks' timed-out waits, never cleared by a kernel (lact_check_async_error reads it)
+  unsigned* counted;         // in LDS: the last of this block's waits that was counted there, which several waves may have waited
   unsigned members, epoch;
   long long limit;
   bool split;                // group spread over several XCDs: fence at device scope
   __device__ __forceinline__ void init(unsigned* line, unsigned nmembers, unsigned* error, long long spin_limit, unsigned* sticky_count) {
-    ctr = line; members = nmembers; epoch = 0; split = false; limit = spin_limit; sticky = sticky_count;
+    __shared__ unsigned last_counted;
+    ctr = line; members = nmembers; epoch = 0; split = false; limit = spin_limit; sticky = sticky_count; counted = &last_counted;
+    if (threadIdx.x == 0) last_counted = 0;
     unsigned xcc = 0;
     asm volatile("s_getreg_b32 %0, hwreg(HW_REG_XCC_ID)" : "=s"(xcc));
     if (threadIdx.x == 0) __hip_atomic_fetch_or(line + 1, 1u << (xcc & 0xf), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -111,7 +114,7 @@ struct GroupBarrier {
       __builtin_amdgcn_s_sleep(1);
       if (++spins >= limit) {
         __hip_atomic_store(error, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (sticky) __hip_atomic_fetch_add(sticky, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (sticky && atomicMax(counted, epoch) < epoch) __hip_atomic_fetch_add(sticky, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         break;
       }
     }

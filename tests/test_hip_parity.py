@@ -17,6 +17,7 @@ Tolerances (relative L2, written where they are used):
 """
 import math
 import os
+import re
 import sys
 
 import numpy as np
@@ -695,6 +696,35 @@ def test_video_model_shape_full_size_equals_its_inference_rollout():
         e_w = max(O.rel_l2(a.cpu(), c.detach().cpu()) for a, c in zip(w, res[1:4]))
     say("   rollout vs program: out", e_out, "final weights", e_w)
     assert e_out < 1e-2 and e_w < 2e-3
+
+
+def test_block_that_gives_up_at_a_barrier_is_counted_once():
+    """A block may wait at a barrier with several waves: the count of time-outs is of blocks' waits, whatever their waves.  Two updates of
+    six 512 x 512 matrices, many blocks to each, most of whose waits time out; a block waits at the first barrier, three times an iteration,
+    and in the backward once more."""
+    from lact_amd import _lib
+    say("fused Newton-Schulz: time-outs are counted per block")
+    inp = problem(2, 3 * 128, 512, 512, 41, torch.bfloat16, momentum=True, lr_shift=-1.0)
+    hip, _ = block_causal_pair(128, True)
+
+    def run():
+        g = clone_to(inp, DEV)
+        out = hip(g)
+        grads_of(out, g, torch.ones_like(out))
+        torch.cuda.synchronize()
+    L = _lib.lib()
+    assert L.lact_check_async_error() == 0
+    L.lact_set_option(_lib.OPT_NS_BARRIER_SPIN_LIMIT, 1)
+    try:
+        names = {n for n in kernels(run)[1] if n.startswith("k_ns_fused")}
+        n = L.lact_check_async_error()
+    finally:
+        L.lact_set_option(_lib.OPT_NS_BARRIER_SPIN_LIMIT, 0)
+        L.lact_set_option(_lib.OPT_FUSED_NEWTON_SCHULZ, 1)
+    assert len(names) == 2
+    waits = sum(2 * 6 * (512 // int(m[0])) * (512 // int(m[1])) * (1 + 3 * 5 + (m[2] == "bwd"))
+                for m in (re.match(r"k_ns_fused<(\d+)x(\d+).*,(fwd|bwd)>", name).groups() for name in names))
+    assert 0 < n <= waits
 
 
 def test_fused_newton_schulz_barrier_timeout_ends_every_kernel_and_poisons_the_step():

@@ -1220,6 +1220,15 @@ struct Runner {
     return 0;
   }
 
+  // Threads to a quad of an initial weight's gradient (k_finish_weight_grads): one where every entry has its own, or while the launch has
+  // four blocks to a compute unit; else twice as many until it has, up to the entries of a matrix.
+  int finish_lanes() const {
+    const long long blocks = (P.g.elems / 4 + 255) / 256 * 3 * P.nw;
+    int n = 1;
+    while (n < 16 && n < d.b / P.nw && blocks * n < 1024) n *= 2;
+    return n;
+  }
+
   // ------------------------------------------------------------------------------------------
   // Gradient rows of a token range are stored on first touch and accumulated on a repeat.  `force` (set when two
   // ranges of the program overlap without being equal) pre-zeroes the whole buffer and accumulates everywhere.
@@ -1776,8 +1785,8 @@ struct Runner {
       p.carry = (d.prenorm && carry_main >= 0) ? scr<float>(P.t_gwhat[carry_main]) : nullptr;
       p.gn0 = gn0; p.n0 = n0(); p.w_init = wf(0);
       p.through_norms = d.detach_norms ? 0 : 1;
-      p.out[0] = dw0; p.out[1] = dw1; p.out[2] = dw2; p.nw = P.nw;
-      LACT_LAUNCH("k_finish_weight_grads", "k_finish_weight_grads", 0.0, k_finish_weight_grads, dim3(eg.x, 3 * P.nw), dim3(256), s, p);
+      p.out[0] = dw0; p.out[1] = dw1; p.out[2] = dw2; p.nw = P.nw; p.lanes = finish_lanes();
+      LACT_LAUNCH("k_finish_weight_grads", "k_finish_weight_grads", 0.0, k_finish_weight_grads, dim3((unsigned)((P.g.elems / 4 * p.lanes + 255) / 256), 3 * P.nw), dim3(256), s, p);
     }
     LACT_CHECK_LAUNCH();
     return 0;

@@ -768,16 +768,22 @@ struct FinishParams {
   int through_norms;
   float* out[3];          // [nw, rows, cols] each
   int nw;                 // matrices: where fewer than batch entries, a gradient is the sum over the entries i, i + nw, ...
+  int lanes;              // threads that share a quad of it, each every lanes-th of these entries: a power of two, 1 .. 16
 };
-__global__ void k_finish_weight_grads(const FinishParams p) {
+// A quad's entries one after the other are a chain of memory latencies, which few matrices of many entries do not hide.  us on one thread a
+// quad / now: one matrix of 64 x 64 for 32 entries 34 / 7.3, of 128 x 128 for 64 65 / 10, of 384 x 384 for 16 and 48 21.5 / 13.9 and 78 / 38;
+// four of 384 x 384 for 4, whose 1728 blocks are enough, 13.8 on one and 15.5 on two threads.
+__global__ __launch_bounds__(256) void k_finish_weight_grads(const FinishParams p) {
   prefetch_args<sizeof(p)>();
+  __shared__ float4 part[256];
   // flat over a matrix, 4 consecutive elements per thread (a row holds a multiple of 4): every lane works
   const int j = blockIdx.y / p.nw, iw = blockIdx.y % p.nw;
-  const long long e = ((long long)blockIdx.x * blockDim.x + threadIdx.x) * 4;
-  if (e >= p.g.elems) return;
-  const int cols = p.g.cols(j), row = (int)(e / cols);
+  const int quads = 256 / p.lanes, share = threadIdx.x / quads;
+  const long long e = ((long long)blockIdx.x * quads + threadIdx.x % quads) * 4;
+  const bool there = e < p.g.elems;
+  const int cols = p.g.cols(j), row = there ? (int)(e / cols) : 0;
   float4 sum = f4(0.f, 0.f, 0.f, 0.f);
-  for (int ib = iw; ib < p.g.nb; ib += p.nw) {
+  for (int ib = there ? iw + share * p.nw : p.g.nb; ib < p.g.nb; ib += p.lanes * p.nw) {
     const int z = j * p.g.nb + ib;
     const size_t o = (size_t)z * p.g.elems + e;
     float4 v = p.gw ? ld4(p.gw + o) : f4(0.f, 0.f, 0.f, 0.f);
@@ -796,10 +802,20 @@ __global__ void k_finish_weight_grads(const FinishParams p) {
       const float4 w = ld4(p.w_init + o);
       v.x += c * w.x; v.y += c * w.y; v.z += c * w.z; v.w += c * w.w;
     }
-    if (ib == iw) sum = v;
+    if (ib == iw + share * p.nw) sum = v;
     else { sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w; }
   }
-  st4(p.out[j] + (size_t)iw * p.g.elems + e, sum);
+  if (p.lanes > 1) {      // the shares, in a fixed order (those without an entry are zero and left out: -0 + 0 is 0)
+    part[threadIdx.x] = sum;
+    __syncthreads();
+    if (share > 0) return;
+    const int shares = min(p.lanes, p.g.nb / p.nw);
+    for (int i = 1; i < shares; ++i) {
+      const float4 v = part[i * quads + threadIdx.x];
+      sum.x += v.x; sum.y += v.y; sum.z += v.z; sum.w += v.w;
+    }
+  }
+  if (there) st4(p.out[j] + (size_t)iw * p.g.elems + e, sum);
 }
 
 // the three caller tensors (null: zeros) -> [3b][elems], 4 elements per thread

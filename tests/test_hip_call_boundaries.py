@@ -192,7 +192,9 @@ def test_rows_further_apart_than_the_kernels_reach_are_copied():
 
 @pytest.mark.parametrize("dtype,nw,b,d,dh,L,C,muon,momentum", [
     (torch.bfloat16, 3, 6, 64, 96, 300, 130, True, True), (torch.bfloat16, 1, 5, 128, 40, 250, 200, False, False),
-    (torch.float32, 2, 2, 40, 72, 150, 60, False, True), (torch.float32, 4, 12, 128, 32, 90, 40, True, False)])
+    (torch.float32, 2, 2, 40, 72, 150, 60, False, True), (torch.float32, 4, 12, 128, 32, 90, 40, True, False),
+    # 16 and 8 threads to a quad of a gradient: 33 entries and 5; quads that end inside a block
+    (torch.float32, 1, 33, 40, 24, 50, 30, False, False), (torch.bfloat16, 2, 10, 72, 104, 130, 70, False, True)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_shared_weights_are_repeated_ones(dtype, nw, b, d, dh, L, C, muon, momentum, transposed):
     """Batch entries that share initial weights: the bits of a call with the weights repeated, its weight gradients summed over the

@@ -108,8 +108,10 @@ struct AsyncRing {
   using TS = typename AT::TS;
   static constexpr int EPG = 16 / sizeof(T), BK = 8 * EPG, WAVES = AT::THREADS / 64;
   static constexpr int A_BYTES = TS::BM * 128, B_BYTES = TS::BN * 128, STAGE = A_BYTES + NB * B_BYTES;
-  // two blocks to a compute unit: with a third stage of four whole B tiles (120 KiB, one block) launches of 512 blocks and more were slower
-  static constexpr int STAGES = NB > 2 && !HALF ? 2 : NB > 1 ? 3 : AT::STAGES, BYTES = STAGE * STAGES;
+  // Two blocks to a compute unit: with a third stage of four whole B tiles (120 KiB, one block) launches of 512 blocks and more were slower.
+  // bf16, whose K-steps have half the matrix instructions of fp32, three: with a third stage of two B tiles (72 KiB, two blocks) the apply and
+  // update hidden stages and the apply backward of 16 x 1024 tokens, d = 200, dh = 392 took 109, 141 and 184 us instead of 97, 125 and 168.
+  static constexpr int STAGES = NB == 1 ? AT::STAGES : sizeof(T) == 2 || (NB > 2 && !HALF) ? 2 : 3, BYTES = STAGE * STAGES;
   static constexpr int NA = TS::BM / 8 / WAVES, NBC = TS::BN / 8 / WAVES, COPIES = NA + NBC;   // per wave and stage, with one B operand
   static_assert(TS::BM / 8 % WAVES == 0 && TS::BN / 8 % WAVES == 0, "copies must split evenly over the waves");
   static_assert(BYTES <= 160 * 1024, "ring does not fit the 160 KiB LDS");

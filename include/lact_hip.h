@@ -255,7 +255,7 @@ int lact_window_attention_backward(int32_t B, int32_t L, int32_t H, int32_t D, i
  *     them; where a program has apply steps on a version that is not its newest, lact_forward / lact_backward
  *     enqueue them on a library-owned stream (default priority, per device, created on first use) that is forked
  *     from and joined back into the caller's stream with events, so the call as a whole stays asynchronous and
- *     ordered on the caller's stream.  1 (the default): where these steps are long enough to pay for the events, or
+ *     ordered on the caller's stream.  1 (the default): where these steps are measured to pay for the events, or
  *     the call is being captured; 2: always; 0: never.
  *   LACT_OPT_FUSED_NEWTON_SCHULZ: all Newton-Schulz iterations of an update (and of its backward) run as one
  *     kernel whose blocks meet at per-matrix barriers (bf16; rows and columns multiples of 192, of 128, or rows of
@@ -298,8 +298,8 @@ int lact_check_async_error(void);
 /* Per-launch timing with HIP events on the caller's stream (no counterpart in the reference, which
  * times with wall-clock prints, lact_ar_video/minVid/train.py:458-460).  While enabled every kernel
  * launch of lact_forward / lact_backward is bracketed by two events; lact_profile_report synchronises
- * the device, writes a JSON array of {kernel, site, launches, ms, flops} into buf and resets the
- * records.  Not thread-safe; meant for benchmarking. */
+ * the device, writes a JSON array of {kernel, site, stream, launches, ms, flops} into buf (stream: streams in the
+ * order of their first launch, from 0) and resets the records.  Not thread-safe; meant for benchmarking. */
 int lact_profile_enable(int on);
 /* Calibration kernel for matrix-pipe counters (`rocprofv3 --pmc SQ_VALU_MFMA_BUSY_CYCLES ...`): `blocks` workgroups of
  * four waves that issue nothing but bf16 matrix instructions, `iters` x 8 each; out: blocks * 256 floats.  What the

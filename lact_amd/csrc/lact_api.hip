@@ -36,6 +36,7 @@ struct ProfRec {
   const char* kernel;
   const char* site;
   double flops;
+  hipStream_t stream;
   hipEvent_t e0, e1;
 };
 struct Profiler {
@@ -66,7 +67,7 @@ struct ProfScope {
   hipEvent_t e1 = nullptr;
   ProfScope(const char* kernel, const char* site, double flops, hipStream_t st) : s(st) {
     if (!g_prof.on) return;
-    ProfRec r{kernel, site, flops, g_prof.get(), g_prof.get()};
+    ProfRec r{kernel, site, flops, st, g_prof.get(), g_prof.get()};
     (void)hipEventRecord(r.e0, s);
     e1 = r.e1;
     g_prof.recs.push_back(r);
@@ -335,15 +336,32 @@ struct Runner {
     side = side_ctx();
     if (side && !P.groups.empty() && overlap_pays(p, st)) s_side = side->stream;
   }
-  // Apply steps beside the update chain: what is hidden against the events of the forks and joins, 60 to 100 us of host time a training step
-  // and 6 us on the GPU each.  us of a training step, overlapped / in line, by 1e9 operations of the apply steps (Plan::side_work): 0.13
-  // (1 fp32 head of 64, 700 tokens) 350 / 256; 1.1 (4 x 3000 tokens, d = dh = 128) 318 / 256; 2.8 (6 x 3000, 128 x 256) 295 / 270; 4.4 (2 x 3000,
-  // 256 x 512) 424 / 432; 4.7 (4 x 4000, 256) 331 / 336; 10.6 (16 x 4000, 192) 535 / 587; 24 784 / 888; 108 2600 / 2850; fp32 11 410 / 405 and 33
-  // 795 / 847.  With Newton-Schulz the GPU is the longer side earlier: 0.2 (3 x 1500, 96) 641 / 572; 1.3 (16 x 1200, 128) 361 / 366; beyond
-  // 128 features, where its matrices take several blocks each, always: 1.2 (2 x 1400, 384) 318 / 349.  A captured call pays no host time.
+  // Whether the apply steps on earlier versions run beside the update chain.  What is hidden, against the events of the forks and joins, 60 to
+  // 100 us of host time a training step (two forks and a wait for every group) and 6 us on the GPU each, and against the compute units that
+  // a group takes from the chain's small launches.  us, overlapped / in line, by 1e9 operations of the apply steps (Plan::side_work), updates
+  // and groups:
+  //   training, no Newton-Schulz.  2.5, 1, 1 (1024 features) 286 / 345; 2.4, 1, 1 (fp32 384) 252 / 292; 0.23, 1, 1 (768) 200 / 222; 1.0, 5, 1
+  //     (512) 487 / 507, but 0.3, 1, 1 (512) 197 / 188: chains of wide matrices are long whatever the tokens.  Up to 256 features 3.5, 1, 1
+  //     (192) 238 / 231, 4.0, 4, 2 (96) 395 / 336, 4.4, 5, 2 (128) 417 / 405, but 5.4, 3, 1 (192 x 384) 361 / 384, 5.9, 1, 1 (64) 452 / 474,
+  //     7.1, 2, 2 (128) 342 / 385, and with more groups 3.6, 9, 5 (64) 522 / 538.  Long chains of small links lose at any sum: 2.5, 199, 4
+  //     (128) 7683 / 7034; 3.9, 39, 1 (256) 2526 / 2388; 11.9, 59, 4 (128 x 256) 2976 / 3042.
+  //   training with Newton-Schulz.  Matrices of one block (ns_local.h): 2.4, 1, 1 (128) 289 / 278, 2.7, 1, 1 (96) 362 / 336, 4.7, 1, 1 (128)
+  //     331 / 363, 5.4, 3, 3 (96) 734 / 745, 4.8, 2, 2 (128 x 256) 584 / 636.  Larger ones of fewer than 128 rows, three launches an iteration:
+  //     1.2, 2, 1 (64 x 512) 949 / 852, 4.8, 3, 3 1011 / 996.  The fused kernel of the others leaves units free: 0.27, 1, 1 (192 x 384) 368 / 381,
+  //     but 0.2, 1, 1 (256) 319 / 264; long chains 2.9, 29, 1 (256) 6283 / 6187.
+  //   forward only.  Half as much to hide, and the host further behind: 7.3, 9, 9 (64) 242 / 214; 11.0, 1, 1 (128 x 256) 112 / 102; 15, 1, 1 (256)
+  //     173 / 170, but 10.6, 2, 2 (192) 156 / 167; 33, 9, 3 (384) 485 / 512; 29, 9, 5 (256 x 512) 401 / 408; 2.5, 1, 1 (1024) 100 / 107.  With
+  //     Newton-Schulz 5.4, 3, 3 (96) 175 / 171; 2.9, 29, 1 (256) 2761 / 2702; 4.8, 2, 2 (128 x 256) 221 / 224; 7.3, 2, 2 (128 x 384) 284 / 294.
+  // A captured call pays no host time.
   static bool overlap_pays(const Plan& P, hipStream_t st) {
     if (g_overlap != 1) return g_overlap > 1;
-    if (P.side_work >= (!P.muon ? 4e9 : P.d.d <= 128 ? 1e9 : 0.)) return true;
+    const double work = P.side_work, group = work / (double)P.groups.size(), wide = work * P.d.d * P.d.dh;
+    const bool many = P.groups.size() >= 4, block_each = P.r <= 128 && P.c <= 256;
+    const bool pays = P.d.forward_only ? (P.muon ? work >= 4.5e9 && group >= 2.4e9 : (P.groups.size() >= 2 && group >= 5e9) || wide >= 2.5e15)
+                      : work < 1.5e8 * P.nupd ? false
+                      : P.muon ? work >= (block_each ? 3e9 : P.r < 128 ? 5e9 : 2.5e8)
+                               : work >= 5.35e9 || (many && work >= 3e9) || wide >= 1.32e14;
+    if (pays) return true;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;
     (void)hipGetLastError();      // (the legacy stream beside another one's capture: the launches will say so)
@@ -2570,16 +2588,19 @@ int lact_profile_report(char* buf, size_t cap) {
   if (!buf || cap == 0) return fail("null report buffer");
   hipError_t e = hipDeviceSynchronize();
   if (e != hipSuccess) return fail(std::string("synchronize failed: ") + hipGetErrorString(e));
-  struct Agg { std::string kernel, site; long n = 0; double ms = 0, flops = 0; };
+  struct Agg { std::string kernel, site; int stream; long n = 0; double ms = 0, flops = 0; };
   std::vector<Agg> aggs;
+  std::vector<hipStream_t> streams;
   for (auto& r : g_prof.recs) {
     float ms = 0.f;
     if (hipEventElapsedTime(&ms, r.e0, r.e1) != hipSuccess) continue;
+    const int stream = (int)(std::find(streams.begin(), streams.end(), r.stream) - streams.begin());
+    if (stream == (int)streams.size()) streams.push_back(r.stream);
     Agg* a = nullptr;
     for (auto& x : aggs)
-      if (x.kernel == r.kernel && x.site == r.site) a = &x;
+      if (x.kernel == r.kernel && x.site == r.site && x.stream == stream) a = &x;
     if (!a) {
-      aggs.push_back(Agg{r.kernel, r.site});
+      aggs.push_back(Agg{r.kernel, r.site, stream});
       a = &aggs.back();
     }
     a->n += 1;
@@ -2589,8 +2610,8 @@ int lact_profile_report(char* buf, size_t cap) {
   std::string out = "[";
   for (size_t i = 0; i < aggs.size(); ++i) {
     char line[512];
-    snprintf(line, sizeof(line), "%s{\"kernel\": \"%s\", \"site\": \"%s\", \"launches\": %ld, \"ms\": %.6f, \"flops\": %.6e}",
-             i ? ", " : "", aggs[i].kernel.c_str(), aggs[i].site.c_str(), aggs[i].n, aggs[i].ms, aggs[i].flops);
+    snprintf(line, sizeof(line), "%s{\"kernel\": \"%s\", \"site\": \"%s\", \"stream\": %d, \"launches\": %ld, \"ms\": %.6f, \"flops\": %.6e}",
+             i ? ", " : "", aggs[i].kernel.c_str(), aggs[i].site.c_str(), aggs[i].stream, aggs[i].n, aggs[i].ms, aggs[i].flops);
     out += line;
   }
   out += "]";

@@ -23,7 +23,7 @@ import sys
 import numpy as np
 import pytest
 import torch
-from launches import kernels
+from launches import kernels, streams
 
 from lact_amd import ar_video, minimal, nvs, ops
 from lact_amd import ttt_operation as T
@@ -1156,6 +1156,30 @@ def test_stream_overlap_is_bit_identical(prenorm):
     assert torch.equal(on[0][0], on[2][0]) and all(torch.equal(on[0][1][n], on[2][1][n]) for n in on[0][1])
 
 
+@pytest.mark.parametrize("act,b,chunks,C,d,dh,muon,grad,expected", [
+    # training: wide matrices from few tokens on, others from more work on, less of it in many groups; not chains of many small links
+    (torch.bfloat16, 1, 2, 64, 768, 768, False, True, 2), (torch.float32, 1, 2, 300, 384, 384, False, True, 2),
+    (torch.bfloat16, 4, 2, 512, 128, 128, False, True, 1), (torch.bfloat16, 8, 4, 512, 192, 384, False, True, 2),
+    (torch.bfloat16, 16, 10, 1024, 64, 64, False, True, 2), (torch.bfloat16, 1, 40, 256, 256, 256, False, True, 1),
+    # with Newton-Schulz: matrices of one block, of several launches an iteration, of the fused kernel
+    (torch.bfloat16, 8, 2, 3000, 128, 128, True, True, 1), (torch.bfloat16, 4, 3, 512, 64, 512, True, True, 1),
+    (torch.bfloat16, 2, 2, 300, 192, 384, True, True, 2), (torch.bfloat16, 2, 2, 256, 256, 256, True, True, 1),
+    # forward only
+    (torch.bfloat16, 16, 10, 1024, 64, 64, False, False, 1), (torch.bfloat16, 8, 4, 512, 192, 384, False, False, 1),
+    (torch.bfloat16, 16, 3, 1500, 192, 192, False, False, 2), (torch.bfloat16, 2, 2, 200, 1024, 1024, False, False, 2),
+    (torch.bfloat16, 2, 2, 300, 192, 384, True, False, 1), (torch.bfloat16, 4, 4, 2048, 128, 384, True, False, 2)])
+def test_apply_steps_run_beside_the_chain_where_that_was_measured_to_pay(act, b, chunks, C, d, dh, muon, grad, expected):
+    """The second stream by default: on the side of each line on which it was the faster one."""
+    say("stream overlap by default", b, chunks, C, d, dh, muon, grad)
+    t = clone_to(problem(b, chunks * C, d, dh, seed=79, act=act), DEV, grad=grad)
+
+    def run():
+        with torch.set_grad_enabled(grad):
+            out = T.block_causal_lact_swiglu(*args9(t), C, muon, None)
+            return grads_of(out, {n: x for n, x in t.items() if n != "momentum"}, torch.ones_like(out)) if grad else out
+    assert streams(run)[1] == expected
+
+
 @pytest.mark.parametrize("body", ["identical", "streams", "threads", "captured"])
 def test_stream_overlap_of_small_programs(body):
     """Apply steps too short to pay for the second stream's events run in line by default: forced onto it, the same bits, and so
@@ -1172,7 +1196,7 @@ def test_stream_overlap_of_small_programs(body):
         if body == "captured":
             return test_graph_capture_replays_match_eager()
         for dtype, b, d, L, C in ((torch.bfloat16, 2, 128, 700, 100), (torch.float32, 2, 64, 300, 90), (torch.bfloat16, 8, 256, 4 * 512, 512),
-                                  (torch.bfloat16, 12, 256, 5 * 512, 512)):      # 0.06 to 9.7 thousand million operations; the line is at 4
+                                  (torch.bfloat16, 12, 256, 5 * 512, 512)):      # 0.12, 0.12, 4.8 and 9.7 thousand million operations; the line is at 5.35
             inp = problem(b, L, d, d, seed=78, act=dtype)
             go = torch.randn(b, L, d, generator=torch.Generator().manual_seed(5)).to(dtype).to(DEV)
             res = []

@@ -1158,7 +1158,7 @@ def test_stream_overlap_is_bit_identical(prenorm):
 
 @pytest.mark.parametrize("act,b,chunks,C,d,dh,muon,grad,expected", [
     # training: wide matrices from few tokens on, others from more work on, less of it in many groups; not chains of many small links
-    (torch.bfloat16, 1, 2, 64, 768, 768, False, True, 2), (torch.float32, 1, 2, 300, 384, 384, False, True, 2),
+    (torch.bfloat16, 2, 2, 200, 1024, 1024, False, True, 2), (torch.bfloat16, 1, 2, 64, 768, 768, False, True, 1), (torch.float32, 1, 2, 300, 384, 384, False, True, 2),
     (torch.bfloat16, 4, 2, 512, 128, 128, False, True, 1), (torch.bfloat16, 8, 4, 512, 192, 384, False, True, 2),
     (torch.bfloat16, 16, 10, 1024, 64, 64, False, True, 2), (torch.bfloat16, 1, 40, 256, 256, 256, False, True, 1),
     # with Newton-Schulz: matrices of one block, of several launches an iteration, of the fused kernel

@@ -645,7 +645,6 @@ struct GradPrepParams {
 };
 template <typename T, typename TN>
 __global__ __launch_bounds__(256) void k_grad_prep(const GradPrepParams p) {
-  prefetch_args<sizeof(p)>();
   __shared__ float red[16];
   __shared__ __attribute__((aligned(16))) float tx[TallTile<float>::C * TallTile<float>::LD];
   __shared__ __attribute__((aligned(16))) TN tg[TallTile<TN>::C * TallTile<TN>::LD];

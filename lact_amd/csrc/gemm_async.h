@@ -108,10 +108,12 @@ struct AsyncRing {
   using TS = typename AT::TS;
   static constexpr int EPG = 16 / sizeof(T), BK = 8 * EPG, WAVES = AT::THREADS / 64;
   static constexpr int A_BYTES = TS::BM * 128, B_BYTES = TS::BN * 128, STAGE = A_BYTES + NB * B_BYTES;
-  // Two blocks to a compute unit: with a third stage of four whole B tiles (120 KiB, one block) launches of 512 blocks and more were slower.
-  // bf16, whose K-steps have half the matrix instructions of fp32, three: with a third stage of two B tiles (72 KiB, two blocks) the apply and
-  // update hidden stages and the apply backward of 16 x 1024 tokens, d = 200, dh = 392 took 109, 141 and 184 us instead of 97, 125 and 168.
-  static constexpr int STAGES = NB == 1 ? AT::STAGES : sizeof(T) == 2 || (NB > 2 && !HALF) ? 2 : 3, BYTES = STAGE * STAGES;
+  // Where several B operands share a stage two of them, for three blocks to a compute unit (two with four B operands: a third stage of those
+  // would leave one).  us with a third stage of 24 KiB and two blocks, with two and three, at 768 blocks of fp32: update hidden stage at d = dh =
+  // 64 33.2 / 27.6, 128 39.9 / 35.4, 384 82.7 / 74.0, apply 35.7 / 31.3, 50.5 / 44.7, 105 / 97, apply backward 56.1 / 55.9, 81 / 74, 166 / 150; at
+  // 1024 blocks, whose last round is a third full, 189 / 194, 116 / 110, 183 / 180; bf16 (16 x 1024 tokens, d = 200, dh = 392) update 141 / 125,
+  // apply 109 / 97, apply backward 184 / 168.  Half tiles, launched where there are fewer blocks than compute units, have three.
+  static constexpr int STAGES = NB == 1 ? AT::STAGES : HALF ? 3 : 2, BYTES = STAGE * STAGES;
   static constexpr int NA = TS::BM / 8 / WAVES, NBC = TS::BN / 8 / WAVES, COPIES = NA + NBC;   // per wave and stage, with one B operand
   static_assert(TS::BM / 8 % WAVES == 0 && TS::BN / 8 % WAVES == 0, "copies must split evenly over the waves");
   static_assert(BYTES <= 160 * 1024, "ring does not fit the 160 KiB LDS");

@@ -2129,9 +2129,18 @@ int layer_token_blocks(int act_dtype, const LayerGeom& g) {   // one pass of eve
   const long long n = 4LL * layer_rows_per_wave(act_dtype, g.hd);
   return (int)(((long long)g.B * g.L + n - 1) / n);
 }
-// blocks per head of the backward with parameter gradients: as many as are resident at once (three waves a SIMD), few enough
-// that the partial sums stay small beside the activations
-int layer_pre_attn_blocks(const LayerGeom& g) { return (int)std::max(1LL, std::min(((long long)g.B * g.L + 3) / 4, 768LL / g.H)); }
+// Rows of partial sums that a caller provides for the backward with parameter gradients, whatever its type and hd: few enough that they
+// stay small beside the activations
+int layer_pre_attn_rows(const LayerGeom& g) { return (int)std::max(1LL, std::min(((long long)g.B * g.L + 3) / 4, 1024LL / g.H)); }
+// Its blocks per head, one row each: as many as are resident at once, by the waves a SIMD that the registers of one, two or three, and four
+// chunks a lane leave.  With three waves' worth for all, us at 16384 tokens (fp32 4096): heads of 64 157 / 144, 1024 109 / 90, fp32 384 67.5 / 61.5.
+int layer_pre_attn_blocks(int act_dtype, const LayerGeom& g) {
+  int waves = 1;
+  auto resident = [&](auto, auto nv) { waves = decltype(nv)::value == 1 ? 4 : decltype(nv)::value < 4 ? 3 : 2; };
+  if (act_dtype == LACT_BF16) layer_lanes<uint16_t>(g.hd, resident);
+  else layer_lanes<float>(g.hd, resident);
+  return std::min(layer_pre_attn_rows(g), std::max(1, 256 * waves / g.H));
+}
 }  // namespace
 extern "C" {
 
@@ -2176,7 +2185,7 @@ int lact_layer_pre_attn_forward(int32_t act_dtype, int32_t B, int32_t L, int32_t
 int32_t lact_layer_pre_attn_part_rows(int32_t B, int32_t L, int32_t H) {
   LayerGeom g;
   if (layer_geom(B, L, H, 4, &g)) return -1;
-  return layer_pre_attn_blocks(g);
+  return layer_pre_attn_rows(g);
 }
 
 int lact_layer_pre_attn_backward(int32_t act_dtype, int32_t B, int32_t L, int32_t H, int32_t hd, int32_t l2norm, const void* qkv,
@@ -2189,7 +2198,7 @@ int lact_layer_pre_attn_backward(int32_t act_dtype, int32_t B, int32_t L, int32_
   p.l2norm = l2norm; p.qkv = qkv; p.dout[0] = dq; p.dout[1] = dk; p.dout[2] = dv; p.dqkv = dqkv;
   p.datt[0] = daq; p.datt[1] = dak; p.datt[2] = dav; p.qk_scale = qk_scale; p.part = part;
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-  const int rows = layer_pre_attn_blocks(p.g), dim = H * hd;
+  const int rows = layer_pre_attn_blocks(act_dtype, p.g), dim = H * hd;
   if (launch_layer_pre<true>(act_dtype, p, rows, s)) return -1;
   LACT_LAUNCH("k_layer_qk_reduce", "layer_pre_bwd", 0.0, k_layer_qk_reduce, dim3((dim + 63) / 64, 4), dim3(256), s, part, rows, dim, dqk_scale, dqk_offset);
   LACT_CHECK_LAUNCH();

@@ -60,7 +60,9 @@ def test_window_attention_scores_and_window_edges(b, l, h, d, window, growth):
             assert rel_l2(a, r) < 2e-2, i
 
 
-@pytest.mark.parametrize("dtype,B,L,H,hd", [(torch.float32, 2, 37, 3, 16), (torch.float32, 1, 5, 2, 520), (torch.bfloat16, 1, 4099, 2, 384)])
+@pytest.mark.parametrize("dtype,B,L,H,hd", [(torch.float32, 2, 37, 3, 16), (torch.float32, 1, 5, 2, 520), (torch.bfloat16, 1, 4099, 2, 384),
+                                             # blocks of the backward by the chunks a lane holds: one and four of bf16, more heads than blocks
+                                             (torch.bfloat16, 2, 700, 24, 64), (torch.bfloat16, 1, 2100, 1, 1024), (torch.float32, 1, 9, 600, 136)])
 def test_pre_attention_kernel_against_torch(dtype, B, L, H, hd):
     """The layer's pre-processing with the attention's inputs: outputs, and the gradients of the projection and of the rescaling."""
     print("[gpu-test] layer pre with attention", dtype, B, L, H, hd, flush=True)

@@ -1142,11 +1142,13 @@ def test_stream_overlap_is_bit_identical(prenorm):
         torch.cuda.synchronize()
         return res
     L_ = _lib.lib()
-    prev = L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, 1)
+    prev = L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, 2)
     try:
         on = run()
+        assert streams(run)[1] == 2
         L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, 0)
         off = run()
+        assert streams(run)[1] == 1
     finally:
         L_.lact_set_option(_lib.OPT_STREAM_OVERLAP, prev)
     for (o1, g1), (o0, g0) in zip(on, off):

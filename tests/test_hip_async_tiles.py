@@ -345,3 +345,58 @@ def test_momentum_step_of_matrices_held_transposed(b, d, dh, T, carried):
     # gradient's direction at the norm of one
     for a, r in zip([out, *ws, *ms], [ref, *wr, *mr]):
         assert O.rel_l2(a, r) < 1e-2
+
+
+@pytest.mark.parametrize("dtype,muon,kernel", [(torch.bfloat16, True, None), (torch.float32, True, "k_momentum_prep"), (torch.bfloat16, False, None)])
+@pytest.mark.parametrize("where", ["aligned", "unaligned", "in place"])
+def test_carried_momentum_states_anywhere_in_memory(dtype, muon, kernel, where):
+    """The library reads a carried state where it lies, or, where 16-byte loads do not reach it, a copy; a caller may have the new state
+    written over it.  The bits of a call on aligned states of its own: in the epilogue of the token reduction, in the momentum kernel, and
+    in the row norm's."""
+    print("[gpu-test] carried states in memory", dtype, muon, where, flush=True)
+    import ctypes
+    from lact_amd import _lib, ops
+    from lact_amd._lib import LACT_APPLY, LACT_UPDATE
+    b, L, d, dh = 2, 100, 64, 128
+    inp = O.make_inputs(b, L, d, dh, seed=62, act_dtype=dtype)
+    dev = [inp[n].to("cuda").contiguous() for n in ORDER]
+    g = torch.Generator().manual_seed(8)
+    state = [1e-3 * torch.randn(b, *s, generator=g).to("cuda") for s in ((dh, d), (d, dh), (dh, d))]
+    steps = ((LACT_UPDATE, 0, L, 0), (LACT_APPLY, 0, L, 0))
+    prog = ops.Program(steps=steps, out_len=L, ns_coeffs=ops.NS5_COEFFS if muon else None)
+    with torch.no_grad():
+        out, ws, ms = ops.run_program(prog, *dev, momentum_state=[m.clone() for m in state])
+
+    lib, keep = _lib.lib(), []
+    D = _lib.Desc()
+    D.b, D.d, D.dh, D.q_len, D.kv_len, D.out_len, D.act_dtype = b, d, dh, L, L, L, _lib.LACT_BF16 if dtype == torch.bfloat16 else _lib.LACT_F32
+    arr, coeffs = (_lib.Step * 2)(*[_lib.Step(*s) for s in steps]), (ctypes.c_float * 15)(*[x for t in ops.NS5_COEFFS for x in t])
+    D.n_steps, D.steps, D.ns_steps, D.weight_norm = 2, ctypes.cast(arr, ctypes.POINTER(_lib.Step)), 5 if muon else -1, 1
+    if muon:
+        D.ns_coeffs = ctypes.cast(coeffs, ctypes.POINTER(ctypes.c_float))
+    D.use_momentum = D.forward_only = D.momentum_state_in = 1
+    for n in ("q", "k", "v", "o", "do"):
+        setattr(D, n + "_ld", d)
+        setattr(D, n + "_bs", L * d)
+    saved, scratch = ctypes.c_size_t(), ctypes.c_size_t()
+    _lib.check(lib.lact_query_sizes(ctypes.byref(D), ctypes.byref(saved), ctypes.byref(scratch)))
+    buffers = [torch.empty(n.value, dtype=torch.uint8, device="cuda") for n in (saved, scratch)]
+
+    def lies(t):
+        room = torch.zeros(t.numel() + 4, device="cuda")
+        keep.append(room)
+        at = room[where == "unaligned":][:t.numel()].view(t.shape)
+        assert (at.data_ptr() % 16 != 0) == (where == "unaligned")
+        return at.copy_(t)
+    m_in = [lies(m) for m in state]
+    m_out = m_in if where == "in place" else [torch.empty_like(m) for m in state]
+    w_out, o = [torch.empty_like(w) for w in state], torch.empty_like(dev[3])
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())
+    three = lambda ts: (ctypes.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    stream = ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
+    call = lambda: _lib.check(lib.lact_forward_from_state(ctypes.byref(D), *[ptr(t) for t in dev], three(m_in), ptr(o), three(w_out), three(m_out),
+                                                          *[ptr(t) for t in buffers], stream))
+    _, names = kernels(call)
+    assert kernel is None or kernel in names
+    for a, r in zip([o, *w_out, *m_out], [out, *ws, *ms]):
+        assert torch.equal(a, r)

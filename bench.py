@@ -52,9 +52,10 @@ def _library_label(profile_name):
     n = profile_name.strip()
     n = re.sub(r"^void\s+", "", n).split("(")[0].replace("lact::", "")
     n = re.sub(r"TileShape<(\d+), (\d+), \d+, \d+>\s*", r"\1x\2", n).replace(" ", "")
-    m = re.match(r"k_ns_fused<(\d+x\d+),(true|false)(?:,\d+x\d+)?>", n)
+    m = re.match(r"k_ns_fused<(\d+x\d+),(true|false)(?:,(\d+x\d+))?>", n)
     if m:
-        return f"k_ns_fused<{m.group(1)},{'bwd' if m.group(2) == 'true' else 'fwd'}>"
+        square = "" if m.group(3) in (None, m.group(1)) else "+" + m.group(3)
+        return f"k_ns_fused<{m.group(1)}{square},{'bwd' if m.group(2) == 'true' else 'fwd'}>"
     m = re.match(r"k_row_gemm_dma<(\d+x\d+),(\d+),(\d+),(true|false)>", n)
     if m:
         epi = {"0": "store", "1": "axpby", "2": "axpby_dual"}[m.group(3)]

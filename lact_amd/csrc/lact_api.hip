@@ -502,7 +502,8 @@ struct Runner {
     p.sticky = side->sticky;
     p.spin_limit = g_ns_spin_limit;
     const double terms = BWD ? 6.0 : 3.0;
-    static const std::string name = std::string("k_ns_fused<") + std::to_string(TS::BM) + "x" + std::to_string(TS::BN) + (BWD ? ",bwd>" : ",fwd>");
+    auto tile = [](int bm, int bn) { return std::to_string(bm) + "x" + std::to_string(bn); };     // + that of the square stages, where it is another
+    static const std::string name = "k_ns_fused<" + tile(TS::BM, TS::BN) + (std::is_same<TS, TSQ>::value ? "" : "+" + tile(TSQ::BM, TSQ::BN)) + (BWD ? ",bwd>" : ",fwd>");
     for (int z0 = 0; z0 < B.n; z0 += per) {
       p.z0 = z0; p.n = std::min(per, B.n - z0); p.sync = sync + (size_t)z0 * 32;
       const int grid = 8 * ((p.n + 7) / 8) * nbm;

@@ -44,8 +44,8 @@ __device__ __forceinline__ void row_gemm_phases(const RowGemmParams<NT>& p, int 
 }
 
 // EPI_STORE / EPI_AXPBY: the tile staged in LDS as bf16 (StageTile<TS, 2>, = round(acc)) goes out in whole rows; all
-// threads of the block take part.  GRP: passes whose loads are in flight together (fewer where the caller is short of registers).
-template <class TS, int NT, int EPI, int GRP = 64>
+// threads of the block take part.
+template <class TS, int NT, int EPI>
 __device__ __forceinline__ void row_gemm_copy_out_b16(const RowGemmParams<NT>& p, int m0, int n0, int z, const char* smem) {
   using ST = StageTile<TS, 2>;
   const int r0 = ST::row0(), c0 = ST::col0();
@@ -59,55 +59,50 @@ __device__ __forceinline__ void row_gemm_copy_out_b16(const RowGemmParams<NT>& p
     const size_t ast = EPI == EPI_STORE ? dstep : astep;
     const float al = EPI == EPI_STORE ? 1.f : p.alpha, be = EPI == EPI_STORE ? 1.f : p.beta;
     uint16_t* dst2 = (EPI == EPI_STORE && p.out2) ? reinterpret_cast<uint16_t*>(p.out2) + (dst - reinterpret_cast<uint16_t*>(p.out)) : nullptr;
-    constexpr int G = GRP < ST::PASSES ? GRP : ST::PASSES, LG = G < 8 ? G : 8;
+    constexpr int G = ST::PASSES < 8 ? ST::PASSES : 8;
+    // the auxiliary loads first (no store in between may alias them), then blend and store
+    uint4 w[ST::PASSES];
+    if (blend) {
 #pragma unroll
-    for (int p0 = 0; p0 < ST::PASSES; p0 += G) {
-      // the group's auxiliary loads first (no store in between may alias them), then blend and store
-      uint4 w[G];
-      if (blend) {
-#pragma unroll
-        for (int i = 0; i < G; ++i) {
-          const int ps = p0 + i, r = r0 + ps * ST::RPP;
-          w[i] = (ps < ST::PASSES && r < TS::BM && m0 + r < p.M) ? *reinterpret_cast<const uint4*>(ap + ps * ast) : make_uint4(0, 0, 0, 0);
-        }
-      }
-      // LDS reads in unconditional groups of up to 8 (a branch per row would put every read's latency in line)
-      uint4 ug[LG];
-#pragma unroll
-      for (int i = 0; i < G; ++i) {
-        const int ps = p0 + i;
-        if (ps >= ST::PASSES) break;
-        if (i % LG == 0) {
-#pragma unroll
-          for (int g = 0; g < LG; ++g)
-            if (i + g < G && ps + g < ST::PASSES) ug[g] = ST::read16(src, r0, ps + g);
-        }
+      for (int ps = 0; ps < ST::PASSES; ++ps) {
         const int r = r0 + ps * ST::RPP;
-        if (r < TS::BM && m0 + r < p.M) {
-          uint4 u = ug[i % LG];
-          if (blend) {
-            // the staged values are round(acc); each product and the sum are tensors of their own in the reference
-            uint32_t uu[4] = {u.x, u.y, u.z, u.w}, ww[4] = {w[i].x, w[i].y, w[i].z, w[i].w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-              const float lo = round_bf16(al * __uint_as_float(uu[j] << 16)) + round_bf16(be * __uint_as_float(ww[j] << 16));
-              const float hi = round_bf16(al * __uint_as_float(uu[j] & 0xffff0000u)) + round_bf16(be * __uint_as_float(ww[j] & 0xffff0000u));
-              uu[j] = pack_bf16(lo, hi);
-            }
-            u = make_uint4(uu[0], uu[1], uu[2], uu[3]);
-          }
-          *reinterpret_cast<uint4*>(dst) = u;
-          if (dst2) {
-            uint32_t uu[4] = {u.x, u.y, u.z, u.w};
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
-              uu[j] = pack_bf16(p.alpha2 * bf16_lo(uu[j]), p.alpha2 * bf16_hi(uu[j]));
-            *reinterpret_cast<uint4*>(dst2) = make_uint4(uu[0], uu[1], uu[2], uu[3]);
-          }
-        }
-        dst += dstep;
-        if (dst2) dst2 += dstep;
+        w[ps] = (r < TS::BM && m0 + r < p.M) ? *reinterpret_cast<const uint4*>(ap + ps * ast) : make_uint4(0, 0, 0, 0);
       }
+    }
+    // LDS reads in unconditional groups of up to 8 (a branch per row would put every read's latency in line)
+    uint4 ug[G];
+#pragma unroll
+    for (int ps = 0; ps < ST::PASSES; ++ps) {
+      if (ps % G == 0) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          if (ps + g < ST::PASSES) ug[g] = ST::read16(src, r0, ps + g);
+      }
+      const int r = r0 + ps * ST::RPP;
+      if (r < TS::BM && m0 + r < p.M) {
+        uint4 u = ug[ps % G];
+        if (blend) {
+          // the staged values are round(acc); each product and the sum are tensors of their own in the reference
+          uint32_t uu[4] = {u.x, u.y, u.z, u.w}, ww[4] = {w[ps].x, w[ps].y, w[ps].z, w[ps].w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            const float lo = round_bf16(al * __uint_as_float(uu[j] << 16)) + round_bf16(be * __uint_as_float(ww[j] << 16));
+            const float hi = round_bf16(al * __uint_as_float(uu[j] & 0xffff0000u)) + round_bf16(be * __uint_as_float(ww[j] & 0xffff0000u));
+            uu[j] = pack_bf16(lo, hi);
+          }
+          u = make_uint4(uu[0], uu[1], uu[2], uu[3]);
+        }
+        *reinterpret_cast<uint4*>(dst) = u;
+        if (dst2) {
+          uint32_t uu[4] = {u.x, u.y, u.z, u.w};
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            uu[j] = pack_bf16(p.alpha2 * bf16_lo(uu[j]), p.alpha2 * bf16_hi(uu[j]));
+          *reinterpret_cast<uint4*>(dst2) = make_uint4(uu[0], uu[1], uu[2], uu[3]);
+        }
+      }
+      dst += dstep;
+      if (dst2) dst2 += dstep;
     }
   }
 }

@@ -23,8 +23,8 @@ namespace lact {
 // partial sums) -> 17.  With one A tile for the B operands that share it and one small piece of code for the copies of all contractions,
 // instead of a fully unrolled one for each, whose instructions a launch waited for: update backward 31 -> 24.5, apply hidden 14 -> 9.
 // HALF, for launches whose 64 x 64 tiles leave compute units without a block: 64 x 32 tiles, two waves to each 32 x 32 of
-// them, which take half of the k of every K-step each and add their halves of the sums at the end: twice the blocks, half the serial chain of matrix instructions in each (update backward 24.5 ->
-// 18.9 us, apply hidden 9.0 -> 7.4).
+// them, which take half of the k of every K-step each and add their halves of the sums at the end: twice the blocks, half the
+// serial chain of matrix instructions in each (update backward 24.5 -> 18.9 us, apply hidden 9.0 -> 7.4).
 template <typename T, bool HALF = false> struct AsyncTile {
   static_assert(!HALF || sizeof(T) == 4, "half tiles: fp32");
   using TS = TileShape<64, HALF ? 32 : 64, 2, HALF ? 1 : 2>;

@@ -478,8 +478,8 @@ __global__ __launch_bounds__(1024) void k_layer_sum_rows(const float* part, int 
 // Output n of the launch: n < NL * 4: rate row n (valid below n1), from the fp32 input and weights; behind them the rows of the
 // two bf16 maps, from input and weights rounded to bf16, the sum in fp32, the result rounded: what the GEMMs of autocast do.
 // Bound by HBM and vector-ALU issue alike.  16384 tokens of 1536 channels, 12 + 8 outputs, us: forward 28 (the two products and four
-// casts 85), gradient of the input 37 (51 with a token's row asked for behind the one before it), of the parameters 37 + 8 (six products with a dozen rows or columns each, two bias sums and
-// seven additions and casts: 520).  7500 tokens of 768 channels, 24 outputs: 15.5 and 18 + 5 (85).
+// casts 85), gradient of the input 37 (51 with a token's row asked for behind the one before it), of the parameters 37 + 8 (six
+// products with a dozen rows or columns each, two bias sums and seven additions and casts: 520).  7500 tokens of 768 channels, 24 outputs: 15.5 and 18 + 5 (85).
 struct LayerInMap {
   const float* w;      // [n][dim] fp32
   const float* bias;   // [n] or null (forward)
@@ -629,7 +629,7 @@ __global__ __launch_bounds__(256) void k_layer_in(const LayerInParams p) {
 
 // Gradient of the input: dx = dxq + sum over the outputs of gradient times weight row.  A lane owns four columns and keeps their
 // weights, the block's tokens have their output gradients in LDS.  Grid (token blocks, column blocks of blockDim.x * 4).  All 40 outputs take
-// 256 registers and seven accumulation registers, one wave a SIMD; more outputs would need a second pass.
+// 216 registers, two waves a SIMD; more outputs would need a second pass.
 template <int NL, int NB>
 __global__ __launch_bounds__(256) void k_layer_in_dx(const LayerInParams p) {
   prefetch_args<sizeof(p)>();

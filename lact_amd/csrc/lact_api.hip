@@ -342,8 +342,8 @@ struct Runner {
   // and groups:
   //   training, no Newton-Schulz.  2.5, 1, 1 (1024 features) 286 / 345; 2.4, 1, 1 (fp32 384) 252 / 292; 1.0, 5, 1 (512) 487 / 507, but 0.3, 1, 1
   //     (512) 197 / 188 and 0.23, 1, 1 (768) 200 or, on a slower host, 257 / 223: chains of wide matrices are long whatever the tokens.  Up to
-  //     256 features 3.5, 1, 1 (192) 238 / 231, 4.0, 4, 2 (96) 395 / 336, 4.4, 5, 2 (128) 417 / 405, but 5.4, 3, 1 (192 x 384) 361 / 384, 5.9, 1, 1
-  //     (64) 452 / 474, 7.1, 2, 2 (128) 342 / 385, and with more groups 3.6, 9, 5 (64) 522 / 538.  Long chains of small links lose at any sum:
+  //     256 features 3.5, 1, 1 (192) 238 / 231, 4.0, 4, 2 (96) 395 / 336, 4.4, 5, 2 (128) 417 / 405, but 4.7, 5, 3 (96) 403 / 432, 5.4, 3, 1 (192 x
+  //     384) 361 / 384, 7.1, 2, 2 (128) 342 / 385; fp32 5.3, 3, 1 (64) 350 / 311, but 5.6, 2, 1 (96) 321 / 329; and with more groups 3.6, 9, 5 (64) 522 / 538.  Long chains of small links lose at any sum:
   //     2.5, 199, 4 (128) 7683 / 7034; 3.9, 39, 1 (256) 2526 / 2388, but 11.9, 59, 4 (128 x 256) 2976 / 3042.
   //   training with Newton-Schulz.  Matrices of one block (ns_local.h): 2.4, 1, 1 (128) 289 / 278, 2.7, 1, 1 (96) 362 / 336, 4.7, 1, 1 (128)
   //     331 / 363, 5.4, 3, 3 (96) 734 / 745, 4.8, 2, 2 (128 x 256) 584 / 636.  Larger ones of fewer than 128 rows, three launches an iteration:
@@ -360,7 +360,7 @@ struct Runner {
     const bool pays = P.d.forward_only ? (P.muon ? work >= 4.5e9 && group >= 2.4e9 : (P.groups.size() >= 2 && group >= 5e9) || wide >= 2.5e15)
                       : work < 1.5e8 * P.nupd ? false
                       : P.muon ? work >= (block_each ? 3e9 : P.r < 128 ? 5e9 : 2.5e8)
-                               : work >= 5.35e9 || (many && work >= 3e9) || wide >= 2e14;
+                               : work >= (P.bf16 ? 4.6e9 : 5.35e9) || (many && work >= 3e9) || wide >= 2e14;
     if (pays) return true;
     hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(st, &cap) == hipSuccess) return cap != hipStreamCaptureStatusNone;

@@ -17,8 +17,8 @@
 // What bounds it: a stage is a main loop of six K-steps (twelve backwards), the staging of its tile and the exchange.  48 matrices
 // of 384 x 384 on 192 compute units, forward / backward: a stage 11 / 16.5 us, of which the matrix instructions take 3.6 / 7.2; 6.5 /
 // 13 main loop (8 matrices, whose operands stay in the L2s, 5.1 / 8.5: the rest is misses), 2.7 epilogue, 1.5 stores, barrier and set-up.
-// Launch: 214 -> 166 and 260 -> 249 us against epilogues that chose their case element by element, read the auxiliary tile behind
-// the staging and had every wave wait at the barrier; six matrices of 768 x 1536, three iterations: 195 -> 173.
+// Launch: 221 -> 190 and 271 -> 262 us in a training step (alone, by a probe's events, 214 -> 166 and 260 -> 249) against epilogues that
+// chose their case element by element, read the auxiliary tile behind the staging and had every wave wait at the barrier; six matrices of 768 x 1536, three iterations: 195 -> 173.
 // Matrices with c >= 2 r take half tiles in the r x r stages (NsHalfTile), where whole ones leave half of the blocks waiting: forward /
 // backward us, six of 768 x 1536, three iterations 190 / 267 -> 175 / 248; 24 of 384 x 768, five 197 / 257 -> 178 / 224; 30 of 256 x 512
 // 96 / 115 -> 81 / 97; 18 of 384 x 1152, where a third of the blocks still waits, 200 / 273 -> 180 / 235.

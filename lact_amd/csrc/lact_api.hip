@@ -1028,12 +1028,13 @@ struct Runner {
     bool side_used = false;
     // k * lr0, k * lr2 of all updates in one launch, in line: on a stream of its own, beside the first kernels of the call, the launch
     // itself costs nothing but the two events 7 us on either side and as much host time (us of a training step: eight fp32 heads of
-    // 128, 2048 tokens 421 / 411 in line, 6 heads of 256 x 512, 5003 tokens 822 / 809; 16 heads of 384, 4096 tokens 1141 either way).
+    // 128, 2048 tokens 421 / 411 in line, 6 heads of 256 x 512, 5003 tokens 822 / 809; 16 heads of 384, 4096 tokens 1141 either way; two of 768 x
+    // 1536, 60840 tokens 7052 / 7078, which the tokens that updates do not read, left out, more than make up for: 6971).
     const long long klbs = (long long)(P.kl_end - P.kl_begin) * d.d;
     const bool fused = updates_fused();
     if (klbs > 0 && !fused)
-      LACT_LAUNCH("k_lr_scale_rows", "update_lr_k", 0.0, (k_lr_scale_rows<T>), dim3((unsigned)((klbs / 4 + 255) / 256), d.b), dim3(256), s,
-                  k + (size_t)P.kl_begin * d.k_ld, d.k_ld, d.k_bs, lr0 + P.kl_begin, lr2 + P.kl_begin, (long long)d.kv_len, P.kl_end - P.kl_begin, d.d,
+      LACT_LAUNCH("k_lr_scale_rows", "update_lr_k", 0.0, (k_lr_scale_rows<T>), dim3((unsigned)(((long long)P.kl_len * d.d / 4 + 255) / 256), d.b, P.kl_ranges), dim3(256), s,
+                  k + (size_t)P.kl_begin * d.k_ld, d.k_ld, d.k_bs, lr0 + P.kl_begin, lr2 + P.kl_begin, (long long)d.kv_len, P.kl_end - P.kl_begin, P.kl_period, P.kl_len, d.d,
                   scr<T>(P.t_kl[0]), scr<T>(P.t_kl[1]), klbs);
     // Apply steps only need their weight version.  A group of them is enqueued when its last version is final, on the side stream
     // and at the point of the following update where the chip is least busy -- in front of its Newton-Schulz kernels, which leave

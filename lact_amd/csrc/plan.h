@@ -115,6 +115,7 @@ struct Plan {
   std::vector<float> coeffs;
   MatGeom g;
   int nupd = 0, Tcap = 0, Tupd = 1, S = -1, esz = 2, nsz = 2, r = 0, c = 0, nblk = 1, lr_slots = 1, tiles = 1, nsplit_max = 1, mdot_parts = 1, split_min = 1024, kl_begin = 0, kl_end = 0, side_slots = 1;
+  int kl_period = 0, kl_len = 0, kl_ranges = 1;   // of [kl_begin, kl_end) updates read the first kl_len tokens of every kl_period
   double side_work = 0;   // of the grouped apply steps' forward, in operations of bf16
   int nw = 0;       // initial weights and their gradients: matrices of each kind, batch entry i uses i % nw
   bool muon = false, bf16 = true, momentum = false, state_in = false;
@@ -312,6 +313,7 @@ struct Plan {
     kl_begin = d.kv_len; kl_end = 0;
     for (const auto& st : steps)
       if (st.kind == LACT_UPDATE) { kl_begin = std::min(kl_begin, st.start); kl_end = std::max(kl_end, st.end); }
+    scale_ranges();
     for (int i = 0; i < 2; ++i) t_kl[i] = sc.take((size_t)d.b * std::max(0, kl_end - kl_begin) * d.d * esz);
     t_ca = muon ? sc.take(sq3 * nsz) : 0;                   // c * A of the current Newton-Schulz iteration
     scratch_bytes = sc.off + 256;
@@ -327,6 +329,22 @@ struct Plan {
   }
   // Most splits that launch may have: what the partial-sum buffer of its chain holds (every split writes `steps` slots of mat3 elements).
   int max_splits(bool on_side, int steps) const { return std::min(MAX_SPLITS, (on_side ? side_slots : nsplit_max) / steps); }
+  // Updates with tokens between them, their starts equally far apart: k is scaled for theirs only.  Everything else is one range.
+  void scale_ranges() {
+    kl_ranges = 1;
+    kl_period = kl_len = std::max(0, kl_end - kl_begin);
+    int last = -1, apart = 0, longest = 0, n = 0;
+    for (const auto& st : live) {
+      if (st.kind != LACT_UPDATE) continue;
+      if (n == 1) apart = st.start - last;
+      if (n > 0 && (st.start - last != apart || apart <= 0)) return;
+      last = st.start;
+      longest = std::max(longest, st.end - st.start);
+      ++n;
+    }
+    if (n < 2 || n > 65535 || longest >= apart) return;
+    kl_ranges = n; kl_period = apart; kl_len = longest;
+  }
   // Groups of as many steps as it takes to give every compute unit a 128 x 128 tile of the hidden stage.  Fewer, fuller launches,
   // and fewer event waits at 12 us of host time each: 8 chunks of 64 rows in fp32 526 -> 480 us, 15 of 192 tiles
   // 2.83 -> 2.79 ms; twice the size gains nothing more and delays the chain, which waits for whole groups (many small chunks with

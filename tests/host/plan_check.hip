@@ -1,7 +1,7 @@
 // Host-side check of the buffer plan (no GPU needed): a token reduction never writes more partial-sum slots than the buffer of its
 // chain holds, whatever the lengths of the program's steps, and none of them is held below what its own length asks for on the side
 // chain, whose buffer is sized for exactly its launches; and the partial sums of squares of a reduction that folds the momentum step
-// in have a place per tile.
+// in have a place per tile; and the ranges of k that are scaled by the rates hold every token that an update reads.
 #include <cstdio>
 #include <cstring>
 #include <vector>
@@ -60,8 +60,51 @@ static int check(bool bf16, int b, int d, int dh, int rounds, int T_update, int 
   return bad;
 }
 
+// Updates of `len` tokens (the last one of `last`), their starts `apart` from one another but for the third, which is `shift` later.
+static int check_ranges(int n, int first, int apart, int len, int last, int shift) {
+  std::vector<lact_step_t> steps;
+  int kv = 0, read = 0;
+  for (int i = 0; i < n; ++i) {
+    const int start = first + i * apart + (i == 2 ? shift : 0), end = start + (i + 1 == n ? last : len);
+    steps.push_back(lact_step_t{LACT_UPDATE, start, end, 0});
+    kv = std::max(kv, end);
+  }
+  steps.push_back(lact_step_t{LACT_APPLY, 0, 8, 0});
+  lact_desc_t D;
+  memset(&D, 0, sizeof(D));
+  D.b = 2; D.d = D.dh = 192; D.q_len = 8; D.kv_len = kv + 5; D.out_len = 8; D.act_dtype = LACT_BF16;
+  D.n_steps = (int)steps.size(); D.steps = steps.data(); D.ns_steps = -1; D.weight_norm = 1;
+  D.q_ld = D.k_ld = D.v_ld = D.o_ld = D.do_ld = 192;
+  Plan P;
+  if (P.build(&D)) { printf("plan refused: %s\n", g_err.c_str()); return 1; }
+  std::vector<char> scaled(P.kl_end - P.kl_begin, 0);
+  for (int z = 0; z < P.kl_ranges; ++z)
+    for (int t = z * P.kl_period; t < z * P.kl_period + P.kl_len && t < (int)scaled.size(); ++t) scaled[t] += 1;
+  bool ok = true, twice = false;
+  for (size_t i = 0; i + 1 < steps.size(); ++i)
+    for (int t = steps[i].start; t < steps[i].end; ++t, ++read) ok = ok && scaled[t - P.kl_begin];
+  int all = 0;
+  for (char c : scaled) { twice = twice || c > 1; all += c; }
+  // equally far apart with room between them: no more than each update's, as long as the longest
+  const bool spaced = apart > 0 && apart > std::max(len, last) && (shift == 0 || n < 3) && n > 1;
+  if (ok && !twice && (P.kl_ranges > 1) == spaced && (!spaced || all <= read + std::max(0, len - last) + (n - 1) * std::max(0, last - len))) return 0;
+  printf("scaled ranges: %d updates of %d and %d tokens, %d apart from %d on, the third %d later: %d ranges of %d every %d, %d of %d tokens\n", n, len, last, apart, first, shift,
+         P.kl_ranges, P.kl_len, P.kl_period, all, read);
+  return 1;
+}
+
 int main() {
   int bad = 0, n = 0;
+  for (int count : {1, 2, 3, 7})
+    for (int first : {0, 16})
+      for (int apart : {0, 40, 64, 81})
+        for (int len : {40, 64, 100})
+          for (int last : {24, 40, 64})
+            for (int shift : {0, 8}) {
+              if (count == 1 && apart) continue;
+              bad += check_ranges(count, first, apart, len, count == 1 ? len : last, shift);
+              ++n;
+            }
   for (bool bf16 : {false, true})
     for (int b : {1, 2, 5})
       for (int d : {8, 64, 128, 192})

@@ -528,6 +528,23 @@ def test_ar_video_interleaved(use_momentum, weight_norm, use_moun, repeat, L, up
         assert max(errs.values()) < 1e-2
 
 
+@pytest.mark.parametrize("act,d,dh,mb,L", [(torch.float32, 64, 64, 40, 5 * 40 + 16), (torch.bfloat16, 192, 64, 100, 700), (torch.bfloat16, 200, 104, 72, 6 * 72)])
+def test_rates_scale_k_where_updates_read_it(act, d, dh, mb, L):
+    """Updates on every other chunk, the last window cut or not: k is scaled by the rates for their tokens only, and what lies between them,
+    not a number here, reaches nothing."""
+    say("scaled ranges of k", act, d, dh, mb, L)
+    inp = problem(2, L, d, dh, 17, act, momentum=False, lr_shift=-1.0)
+    between = [t for t in range(L) if t // mb % 2 == 0]
+    for n in ("k", "v"):
+        inp[n][:, between] = float("nan")
+    call = lambda fn, t, **kw: fn(*args9(t), 0.5, 1, mb, -1, 2 * mb, False, 3, True, None, False, **kw)[0]
+    with torch.no_grad():
+        out, names = kernels(lambda: call(ar_video.ar_fast_weight_swish_glu_weight_norm_mini_batch_with_momentum, clone_to(inp, DEV, grad=False)))
+        ref = call(O.ar_fast_weight_swish_glu_weight_norm_mini_batch, clone_to(inp, "cpu", grad=False), num=PLAIN if act == torch.float32 else AC)
+    assert "k_lr_scale_rows" in names and bool(torch.isfinite(out.float()).all())
+    assert O.rel_l2(out, ref) < (1e-4 if act == torch.float32 else 1e-2)
+
+
 @pytest.mark.parametrize("act,d,dh,L,mb", [(torch.float32, 64, 64, 96, 64), (torch.bfloat16, 128, 128, 200, 128),
                                            (torch.bfloat16, 384, 384, 300, 256)])
 def test_ar_video_inference_repeat_accumulates_kv_grads(act, d, dh, L, mb):
